@@ -51,16 +51,9 @@ def main():
     for N, M, K, label in SHAPES:
         x = torch.randn(N, K, dtype=torch.bfloat16, device=dev) * 0.3
         w = torch.randn(M, K, dtype=torch.bfloat16, device=dev) * 0.05
-        # interleaved A/B (v1, v2, hipBLASLt)
-        def v1(a, b):
-            import ctypes as _ct
-            N2, K2 = a.shape
-            M2 = b.shape[0]
-            o = torch.empty(N2, M2, dtype=a.dtype, device=a.device)
-            ops._lib.ll_decode_gemm(
-                ops._ptr(o), ops._ptr(a), ops._ptr(b), _ct.c_int(N2),
-                _ct.c_int(M2), _ct.c_int(K2), ops._stream())
-            return o
+        # interleaved A/B against hipBLASLt
+        def rows(a, b):
+            return ops._row_gemm(a, b)
 
         def v2(a, b):
             return ops.decode_gemm_v2(a, b, ver="2")
@@ -92,7 +85,7 @@ def main():
                "hipblaslt_us": round(t_blas * 1e6, 1)}
         wbytes = M * K * 2
         res["hipblaslt_tbps"] = round(wbytes / t_blas / 1e12, 2)
-        for name, fn, wb in (("v2", v2, wbytes), ("v3", v3, wbytes),
+        for name, fn, wb in (("rows", rows, wbytes), ("v2", v2, wbytes), ("v3", v3, wbytes),
                              ("v3_fp8", v3_fp8, wbytes // 2),
                              ("w8a8", w8a8, wbytes // 2),
                              ("w4a8", w4a8, wbytes // 4)):

@@ -375,9 +375,6 @@ class Engine:
                             self.model.lm_head.data)
                 except Exception:
                     pass
-        if self.ragged and self.device.type == "cuda":
-            ops.tune_decode_shapes(
-                [p for p in self.model.parameters() if p.dim() == 2])
         m = cfg.model
         self.max_rows = cfg.max_batch
         self._init_cache(dtype)

@@ -454,4 +454,6 @@ class LlamaForCausalLM(nn.Module):
                         pass
         normed, _ = ops.rmsnorm(h, self.final_norm_w, self.cfg.norm_eps,
                                 residual)
+        if normed.dim() == 2:
+            return ops.linear_decode(normed, self.lm_head)
         return torch.nn.functional.linear(normed, self.lm_head)

@@ -52,7 +52,6 @@ def _try_load() -> None:
     _lib.ll_paged_attn_decode.restype = ctypes.c_int
     _lib.ll_paged_attn_decode_fp8.restype = ctypes.c_int
     _lib.ll_kv_append_fp8.restype = ctypes.c_int
-    _lib.ll_decode_gemm.restype = ctypes.c_int
     _lib.ll_decode_gemm_v2.restype = ctypes.c_int
     _lib.ll_decode_gemm_v3.restype = ctypes.c_int
     _lib.ll_decode_gemm_v3_ws_floats.restype = ctypes.c_longlong
@@ -678,96 +677,62 @@ def quantize_fp8_weight(w: torch.Tensor):
     return q.view(torch.uint8).contiguous(), scale.squeeze(1).contiguous()
 
 
-# shapes (M, K) whose products with 17..128 rows take the staged decode
-# GEMM because the library's pick was measured far behind it
-_DECODE_CHOICE: dict[tuple[int, int], bool] = {}
-
-
-def tune_decode_shapes(weights) -> int:
-    """Time hipBLASLt against the staged decode GEMM at 64 rows for each
-    [M, K] weight the latter can take, and keep the staged kernel where
-    it is at least a third faster (split-K down-projections of uncommon
-    depth, where the library runs a handful of workgroups).  Called once
-    at engine init; returns the number of shapes switched."""
-    if _lib is None:
-        return 0
-    flush = None
-    for w in weights:
-        M, K = w.shape
-        if ((M, K) in _DECODE_CHOICE or w.dtype != torch.bfloat16
-                or K % 256 or M % 128 or K < 4096):
-            continue
-        x = torch.randn(64, K, dtype=w.dtype, device=w.device)
-        if flush is None:      # weights must come from HBM, not the cache
-            flush = torch.empty(320 << 20, dtype=torch.uint8,
-                                device=w.device)
-
-        def timed(fn):
-            best = float("inf")
-            for i in range(5):
-                flush.fill_(i)
-                a = torch.cuda.Event(enable_timing=True)
-                b = torch.cuda.Event(enable_timing=True)
-                a.record()
-                fn()
-                b.record()
-                torch.cuda.synchronize()
-                best = min(best, a.elapsed_time(b)) if i else best
-            return best
-
-        try:
-            staged = timed(lambda: decode_gemm_v2(x, w))
-        except ValueError:
-            _DECODE_CHOICE[(M, K)] = False
-            continue
-        library = timed(lambda: torch.nn.functional.linear(x, w))
-        _DECODE_CHOICE[(M, K)] = staged < library / 1.5
-    return sum(_DECODE_CHOICE.values())
+def _row_gemm(x: torch.Tensor, weight: torch.Tensor
+              ) -> torch.Tensor | None:
+    """x @ W^T by row_gemm.hip, or None where it does not take the
+    operands (depth or rows no multiple of 8, unaligned views)."""
+    N, K = x.shape
+    M = weight.shape[0]
+    if (weight.dtype != x.dtype or x.stride(1) != 1
+            or not weight.is_contiguous()):
+        return None
+    out = torch.empty(N, M, dtype=x.dtype, device=x.device)
+    rc = _require_native().ll_row_gemm(
+        _ptr(out), _ptr(x), _ptr(weight), ctypes.c_int(N), ctypes.c_int(M),
+        ctypes.c_int(K), ctypes.c_int(x.stride(0)), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "ll_row_gemm")
+    return out
 
 
 def linear_decode(x: torch.Tensor, weight: torch.Tensor,
                   w8: tuple | None = None) -> torch.Tensor:
-    """out = x @ W^T.
+    """out = x @ W^T for up to 128 rows.
 
-    Dispatch policy (measured IN-ENGINE, profiles/r01_attn_lds_and_
-    gemm_policy.md): isolated microbenches had v2 winning the
-    down-projection, but inside the captured decode step hipBLASLt is
-    ~3% faster end-to-end at bs64 (cache interactions differ), so auto
-    keeps v2 only for tiny batches (N <= 16) where its advantage held.
-    LLMLB_CUSTOM_DECODE_GEMM: "auto" (default) = this policy,
-    "1"/"on" = v2 everywhere it is legal, "0"/"off" = hipBLASLt only."""
+    bf16 products take row_gemm.hip at every size it accepts: with
+    weights from HBM it was faster than hipBLASLt at each of 16 shapes
+    from 1024 x 1024 to 32000 x 4096 and 1 to 64 rows (by 2% at the
+    largest with 64 rows, up to 3.8 times where the library runs a
+    handful of workgroups).  LLMLB_CUSTOM_DECODE_GEMM: "auto" (default)
+    = this, "1"/"on" = the staged kernels of decode_gemm.hip wherever
+    they are legal, "0"/"off" = hipBLASLt only."""
     mode = _USE_CUSTOM_DECODE_GEMM
     if (mode in ("0", "false", "off") or not x.is_cuda or _lib is None
-            or x.dtype != torch.bfloat16 or x.dim() != 2):
+            or x.dtype != torch.bfloat16 or x.dim() != 2
+            or not 0 < x.shape[0] <= 128
+            or (torch.is_grad_enabled()
+                and (x.requires_grad or weight.requires_grad))):
         return torch.nn.functional.linear(x, weight)
     N, K = x.shape
     M = weight.shape[0]
-    shape_ok = N <= 128 and K % 256 == 0 and M % 128 == 0 and K >= 4096
+    shape_ok = K % 256 == 0 and M % 128 == 0 and K >= 4096
     if w8 is not None and shape_ok and _DECODE_PHASE:
         # fp8 weights halve the dominant traffic: always take them
         try:
             return decode_gemm_v2(x, w8[0], w_scale=w8[1])
         except ValueError:
             pass
-    # measured policy (profiles/r02_decode_gemm_v3_ab.md): the
-    # pipelined v3 beats hipBLASLt 15-20% in ISOLATED probes on
-    # o_proj/down, and the rocprof trace shows its kernels ~4% faster
-    # in-engine too — but every split-K reduction scheme tried (fp32
-    # atomics + convert pass, last-arriver slab, every-slice spin)
-    # costs more than that margin inside the captured decode step
-    # (best custom arm 5.32 vs blas 5.25 ms/step at bs64).  auto
-    # therefore keeps hipBLASLt at N>16 and the v1-style fragment
-    # kernel at tiny N where it wins outright; explicit modes force
-    # the staged kernels for experiments.
-    if shape_ok:
-        try:
-            if N <= 16:
-                return decode_gemm_v2(x, weight, ver="2")
-            if mode != "auto" or _DECODE_CHOICE.get((M, K)):
-                return decode_gemm_v2(x, weight)
-        except ValueError:
-            pass
-    return torch.nn.functional.linear(x, weight)
+    if mode != "auto":
+        if shape_ok:
+            try:
+                return decode_gemm_v2(x, weight,
+                                      ver="2" if N <= 16 else None)
+            except ValueError:
+                pass
+        return torch.nn.functional.linear(x, weight)
+    out = _row_gemm(x, weight)
+    return torch.nn.functional.linear(x, weight) if out is None else out
 
 
 # fusing swiglu into the staging measured ~4% SLOWER end-to-end (the

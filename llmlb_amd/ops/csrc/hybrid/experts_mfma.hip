@@ -10,29 +10,8 @@
 // Both compute (w in^T) tiles: a lane holds outputs 4g..4g+3 (g = lane/16)
 // of pair n = lane % 16.
 #include "experts.h"
+#include "lds_copy.h"
 #include "mfma.h"
-
-__device__ __align__(16) unsigned zero_piece[4];
-
-// 64 lanes copy 16 bytes each from their own addresses to 1 KB of LDS from
-// byte ``to`` on.  The copy counts as a load of the wave; nothing but
-// wait_barrier waits for it.
-__device__ __forceinline__ void copy_to_lds(const bf16_t* src, unsigned to) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
-               : "memory");
-}
-__device__ __forceinline__ unsigned lds_byte(const unsigned short* p) {
-  return (unsigned)(uintptr_t)(
-      (const __attribute__((address_space(3))) unsigned short*)p);
-}
-// All but the newest N copies and loads of the wave are done, and its LDS
-// reads; then the workgroup's barrier.
-template <int N>
-__device__ __forceinline__ void wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N)
-               : "memory");
-}
 
 // LDS rows are P pieces of 16 bytes; piece c of row r lies at
 // c ^ swizzle(r), so that lanes reading one piece of the rows of an

@@ -1,0 +1,38 @@
+// Copies from global memory straight to LDS: a wave moves 1 KB per
+// instruction without registers, and waits for them by count.
+#pragma once
+#include "common.h"
+
+// where lanes read that have nothing to copy
+static __device__ __align__(16) unsigned zero_piece[4];
+
+// 64 lanes copy 16 bytes each from their own addresses to 1 KB of LDS from
+// byte ``to`` on.  The copy counts as a load of the wave; nothing but
+// an explicit wait waits for it.
+__device__ __forceinline__ void copy_to_lds(const bf16_t* src, unsigned to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
+               : "memory");
+}
+// the same for data that nobody reads again
+__device__ __forceinline__ void stream_to_lds(const bf16_t* src,
+                                              unsigned to) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+      ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
+      : "memory");
+}
+__device__ __forceinline__ unsigned lds_byte(const void* p) {
+  return (unsigned)(uintptr_t)((const __attribute__((address_space(3))) char*)p);
+}
+// All but the newest N copies and loads of the wave are done.
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// ... and its LDS reads; then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N)
+               : "memory");
+}
