@@ -177,14 +177,10 @@ class _DecodeGraph:
             n_parts *= 2
         self.n_parts = n_parts
         nq, D = engine.n_q_local, engine.cfg.model.head_dim
-        group = nq // engine.n_kv_local
-        use_v2 = ops._PAGED_ATTN_V2 and D == 128 and group <= 16
-        slices = n_parts * 4 if use_v2 else n_parts
         if n_parts > 1:
-            self.ws = (torch.empty(S, nq, slices, D, dtype=torch.float32,
-                                   device=dev),
-                       torch.empty(S, nq, slices, 2, dtype=torch.float32,
-                                   device=dev))
+            self.ws = tuple(torch.empty(S, nq, n_parts, width,
+                                        dtype=torch.float32, device=dev)
+                            for width in (D, 2))
         else:
             self.ws = None
         self.graph: torch.cuda.CUDAGraph | None = None

@@ -50,7 +50,6 @@ def _try_load() -> None:
     _lib.ll_decode_gemm_w4a8.restype = ctypes.c_int
     _lib.ll_decode_gemm_w8a8_ws_floats.restype = ctypes.c_longlong
     _lib.ll_paged_attn_decode.restype = ctypes.c_int
-    _lib.ll_paged_attn_decode_fp8.restype = ctypes.c_int
     _lib.ll_kv_append_fp8.restype = ctypes.c_int
     _lib.ll_decode_gemm_v2.restype = ctypes.c_int
     _lib.ll_decode_gemm_v3.restype = ctypes.c_int
@@ -785,6 +784,13 @@ _PAGED_ATTN_V2 = os.environ.get("LLMLB_PAGED_ATTN_V2",
                                 "1").lower() not in ("0", "false", "off")
 
 
+def paged_attn_tiled(head_dim: int) -> bool:
+    """Whether decode attention runs on the matrix cores
+    (page_attention.hip); other head sizes, and all with
+    LLMLB_PAGED_ATTN_V2=0, take a wave per query head."""
+    return _PAGED_ATTN_V2 and head_dim in (64, 128)
+
+
 def paged_attn_decode(q: torch.Tensor, kcache: torch.Tensor,
                       vcache: torch.Tensor, block_tables: torch.Tensor,
                       seq_lens: torch.Tensor, scale: float,
@@ -819,43 +825,35 @@ def paged_attn_decode(q: torch.Tensor, kcache: torch.Tensor,
             n_parts *= 2
     assert q.stride(-1) == 1 and q.stride(1) == D
     out = torch.empty(S, n_q, D, dtype=q.dtype, device=q.device)
-    group = n_q // n_kv
-    # v2 (GQA-amortized) always reduces through the slice workspace
-    use_v2 = _PAGED_ATTN_V2 and D == 128 and group <= 16
-    slices = n_parts * 4 if use_v2 else n_parts
+    fp8 = kcache.dtype == torch.uint8
+    tiled = paged_attn_tiled(D)
+    assert not fp8 or (tiled and D == 128 and n_q // n_kv <= 16), \
+        "FP8 KV requires D=128 and a GQA group <= 16"
+    acc_p = ml_p = None
     if n_parts > 1:
-        if workspace is not None:
-            ws_acc, ws_ml = workspace
-        else:
-            ws_acc = torch.empty(S, n_q, slices, D, dtype=torch.float32,
-                                 device=q.device)
-            ws_ml = torch.empty(S, n_q, slices, 2, dtype=torch.float32,
-                                device=q.device)
+        ws_acc, ws_ml = workspace if workspace is not None else (
+            torch.empty(S, n_q, n_parts, width, dtype=torch.float32,
+                        device=q.device) for width in (D, 2))
         acc_p, ml_p = _ptr(ws_acc), _ptr(ws_ml)
-    else:
-        acc_p = ml_p = None
     bt = block_tables if block_tables.dtype == torch.int32 \
         else block_tables.to(torch.int32)
     sl = seq_lens if seq_lens.dtype == torch.int32 \
         else seq_lens.to(torch.int32)
-    if kcache.dtype == torch.uint8:
-        assert use_v2, "FP8 KV requires the v2 attention shape " \
-            "(D=128, GQA group <= 16)"
-        rc = lib.ll_paged_attn_decode_fp8(
-            _ptr(out), acc_p, ml_p, _ptr(q), _ptr(kcache), _ptr(vcache),
-            _ptr(k_scale), _ptr(v_scale), _ptr(bt), _ptr(sl),
-            ctypes.c_int(S), ctypes.c_int(bt.shape[1]),
-            ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(D),
-            ctypes.c_int(block_size), ctypes.c_int(n_parts),
-            ctypes.c_float(scale), ctypes.c_int(q.stride(0)), _stream())
-        _check(rc, "ll_paged_attn_decode_fp8")
+    if tiled:
+        rc = lib.ll_page_attn(
+            _ptr(out), acc_p, ml_p, _ptr(q), ctypes.c_int(q.stride(0)),
+            _ptr(kcache), _ptr(vcache), _ptr(k_scale) if fp8 else None,
+            _ptr(v_scale) if fp8 else None, _ptr(bt), _ptr(sl),
+            ctypes.c_int(S), ctypes.c_int(bt.shape[1]), ctypes.c_int(n_q),
+            ctypes.c_int(n_kv), ctypes.c_int(D), ctypes.c_int(block_size),
+            ctypes.c_int(n_parts), ctypes.c_float(scale), _stream())
+        _check(rc, "ll_page_attn")
         return out
     rc = lib.ll_paged_attn_decode(
         _ptr(out), acc_p, ml_p, _ptr(q), _ptr(kcache), _ptr(vcache),
         _ptr(bt), _ptr(sl), ctypes.c_int(S), ctypes.c_int(bt.shape[1]),
         ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(D),
         ctypes.c_int(block_size), ctypes.c_int(n_parts),
-        ctypes.c_float(scale), ctypes.c_int(1 if use_v2 else 0),
-        ctypes.c_int(q.stride(0)), _stream())
+        ctypes.c_float(scale), ctypes.c_int(q.stride(0)), _stream())
     _check(rc, "ll_paged_attn_decode")
     return out

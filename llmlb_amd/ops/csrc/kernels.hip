@@ -574,270 +574,6 @@ void paged_attn_decode_kernel(
 }
 
 
-// ---------------------------------------------------------------------------
-// Paged decode attention v2 — GQA-amortized (any group <= 16 via
-// greedy 4/2/1 sub-group passes, D == 128).
-//
-// v1 gives each wave ONE query head, so the 4 waves of a workgroup
-// each stream the same K/V pages (4x redundant L1/L2 traffic — the
-// measured ceiling at ctx >= 1k).  v2 gives each wave ALL `group`
-// query heads of its kv-head and splits the PAGES across the 4 waves
-// instead: every page is read once per workgroup.  Layout: 8 lanes per
-// token x 16-element slices (D=128 -> p = lane&7, DS=16); per token
-// the lane computes `group` partial dots from one K slice load.  The
-// per-wave online-softmax state (m shared, l/acc lane-partial) is
-// combined across the 4 waves through LDS at the end (flash-decode
-// within the workgroup), then across grid partitions by the shared
-// paged_attn_reduce_kernel.
-// ---------------------------------------------------------------------------
-// GROUP <= 4 uses 8 lanes/token x 16-dim slices; GROUP 5..8 switches
-// to 16 lanes/token x 8-dim slices so qf+acc stay ~128 VGPRs and the
-// whole group runs in ONE pass over the pages (the r1 fallback ran
-// group 8 as two GROUP=4 launches and paid the page reads twice).
-template <int GROUP, bool KV8 = false>
-__global__ __launch_bounds__(PA_WAVES * WAVE)
-void paged_attn_decode_v2_kernel(
-    bf16* __restrict__ out,              // [num_seqs, n_q, D]
-    float* __restrict__ ws_acc,          // [num_seqs, n_q, n_parts, D]
-    float* __restrict__ ws_ml,           // [num_seqs, n_q, n_parts, 2]
-    const bf16* __restrict__ q,
-    const bf16* __restrict__ kcache,     // e4m3 bytes when KV8
-    const bf16* __restrict__ vcache,
-    const float* __restrict__ k_scale,   // per (page, head, token); KV8
-    const float* __restrict__ v_scale,
-    const int* __restrict__ block_tables,
-    const int* __restrict__ seq_lens,
-    int n_q, int n_kv, int max_blocks, int n_parts, float scale,
-    int q_rstride, int group_stride, int g_base) {
-  constexpr int D = 128;
-  constexpr int LPT = (GROUP > 4) ? 16 : 8;  // lanes per token
-  constexpr int DS = D / LPT;            // dims per lane (16 or 8)
-  constexpr int TPP = WAVE / LPT;        // tokens per pass (8 or 4)
-  const int seq = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int part = blockIdx.z;
-  const int seq_len = seq_lens[seq];
-  const int n_blocks = (seq_len + PA_BLOCK - 1) / PA_BLOCK;
-  // page range of this (partition, wave): partition -> waves
-  const int slices = n_parts * PA_WAVES;
-  const int wid = threadIdx.x / WAVE;
-  const int lane = threadIdx.x % WAVE;
-  const int slice = part * PA_WAVES + wid;
-  const int per_slice = (n_blocks + slices - 1) / slices;
-  const int blk_begin = slice * per_slice;
-  const int blk_end = min(blk_begin + per_slice, n_blocks);
-  const int t_local = lane / LPT;        // token within the pass
-  const int p = lane % LPT;              // dim slice
-  const int* btab = block_tables + (size_t)seq * max_blocks;
-
-  // q fragments for every head of the group, pre-scaled
-  float qf[GROUP][DS];
-#pragma unroll
-  for (int g = 0; g < GROUP; ++g) {
-    const uint4* qv = reinterpret_cast<const uint4*>(
-        q + (size_t)seq * q_rstride
-        + (size_t)(kvh * group_stride + g_base + g) * D + p * DS);
-#pragma unroll
-    for (int i = 0; i < DS / 8; ++i) {
-      float f[8];
-      unpack8(qv[i], f);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) qf[g][i * 8 + j] = f[j] * scale;
-    }
-  }
-  float m[GROUP], l[GROUP], acc[GROUP][DS];
-#pragma unroll
-  for (int g = 0; g < GROUP; ++g) {
-    m[g] = -INFINITY;
-    l[g] = 0.f;
-#pragma unroll
-    for (int i = 0; i < DS; ++i) acc[g][i] = 0.f;
-  }
-
-  for (int b = blk_begin; b < blk_end; ++b) {
-    const int blk_id = btab[b];
-#pragma unroll
-    for (int half = 0; half < PA_BLOCK / TPP; ++half) {
-      const int trow = half * TPP + t_local;
-      const int tok = b * PA_BLOCK + trow;
-      const bool valid = tok < seq_len;
-      const size_t row = ((size_t)blk_id * n_kv + kvh) * PA_BLOCK + trow;
-      float kf[DS];
-      if (KV8) {
-        const float sc = k_scale[row];
-        const unsigned char* kb =
-            reinterpret_cast<const unsigned char*>(kcache) + row * D +
-            p * DS;
-        if (DS == 16) {
-          const uint4 raw = *reinterpret_cast<const uint4*>(kb);
-          fp8x4_to_f32(raw.x, kf + 0);
-          fp8x4_to_f32(raw.y, kf + 4);
-          fp8x4_to_f32(raw.z, kf + 8);
-          fp8x4_to_f32(raw.w, kf + 12);
-        } else {
-          const uint2 raw = *reinterpret_cast<const uint2*>(kb);
-          fp8x4_to_f32(raw.x, kf + 0);
-          fp8x4_to_f32(raw.y, kf + 4);
-        }
-#pragma unroll
-        for (int j = 0; j < DS; ++j) kf[j] *= sc;
-      } else {
-        const uint4* kv4 = reinterpret_cast<const uint4*>(
-            kcache + row * D + p * DS);
-#pragma unroll
-        for (int i = 0; i < DS / 8; ++i) {
-          float f[8];
-          unpack8(kv4[i], f);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) kf[i * 8 + j] = f[j];
-        }
-      }
-      float s[GROUP];
-#pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-        float acc_s = 0.f;
-#pragma unroll
-        for (int j = 0; j < DS; ++j) acc_s += qf[g][j] * kf[j];
-        // reduce over the LPT-lane dim group
-        acc_s += __shfl_xor(acc_s, 1, WAVE);
-        acc_s += __shfl_xor(acc_s, 2, WAVE);
-        acc_s += __shfl_xor(acc_s, 4, WAVE);
-        if (LPT == 16) acc_s += __shfl_xor(acc_s, 8, WAVE);
-        s[g] = valid ? acc_s : -INFINITY;
-      }
-      // block max over the 8 tokens of this pass (lane bits 3..5)
-      float vf[DS];
-      if (KV8) {
-        const float sc = v_scale[row];
-        const unsigned char* vb =
-            reinterpret_cast<const unsigned char*>(vcache) + row * D +
-            p * DS;
-        if (DS == 16) {
-          const uint4 raw = *reinterpret_cast<const uint4*>(vb);
-          fp8x4_to_f32(raw.x, vf + 0);
-          fp8x4_to_f32(raw.y, vf + 4);
-          fp8x4_to_f32(raw.z, vf + 8);
-          fp8x4_to_f32(raw.w, vf + 12);
-        } else {
-          const uint2 raw = *reinterpret_cast<const uint2*>(vb);
-          fp8x4_to_f32(raw.x, vf + 0);
-          fp8x4_to_f32(raw.y, vf + 4);
-        }
-#pragma unroll
-        for (int j = 0; j < DS; ++j) vf[j] *= sc;
-      } else {
-        const uint4* vv4 = reinterpret_cast<const uint4*>(
-            vcache + row * D + p * DS);
-#pragma unroll
-        for (int i = 0; i < DS / 8; ++i) {
-          float f[8];
-          unpack8(vv4[i], f);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) vf[i * 8 + j] = f[j];
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-        float bm = s[g];
-        if (LPT == 8) bm = fmaxf(bm, __shfl_xor(bm, 8, WAVE));
-        bm = fmaxf(bm, __shfl_xor(bm, 16, WAVE));
-        bm = fmaxf(bm, __shfl_xor(bm, 32, WAVE));
-        const float m_new = fmaxf(m[g], bm);
-        if (m_new != -INFINITY) {
-          const float rescale =
-              (m[g] == -INFINITY) ? 0.f : __expf(m[g] - m_new);
-          const float wgt = valid ? __expf(s[g] - m_new) : 0.f;
-          l[g] = l[g] * rescale + wgt;
-#pragma unroll
-          for (int i = 0; i < DS; ++i)
-            acc[g][i] = acc[g][i] * rescale + wgt * vf[i];
-          m[g] = m_new;
-        }
-      }
-    }
-  }
-  // reduce l and acc across the token groups (butterfly)
-#pragma unroll
-  for (int off = LPT; off <= 32; off <<= 1) {
-#pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      l[g] += __shfl_xor(l[g], off, WAVE);
-#pragma unroll
-      for (int i = 0; i < DS; ++i)
-        acc[g][i] += __shfl_xor(acc[g][i], off, WAVE);
-    }
-  }
-  if (gridDim.z == 1) {
-    // single grid partition: the 4 wave-slices live in THIS workgroup,
-    // so combine through LDS and write bf16 directly — no global f32
-    // slice round trip, no reduce kernel (saves ~8 MB/layer of ws
-    // traffic + one launch at the common short-context sizes)
-    __shared__ float s_acc[PA_WAVES][GROUP][D];
-    __shared__ float s_ml[PA_WAVES][GROUP][2];
-    if (t_local == 0) {
-#pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-#pragma unroll
-        for (int i = 0; i < DS; ++i) s_acc[wid][g][p * DS + i] = acc[g][i];
-        if (p == 0) {
-          s_ml[wid][g][0] = m[g];
-          s_ml[wid][g][1] = l[g];
-        }
-      }
-    }
-    __syncthreads();
-    if (wid == 0 && t_local == 0) {
-#pragma unroll
-      for (int g = 0; g < GROUP; ++g) {
-        float m_tot = -INFINITY;
-#pragma unroll
-        for (int w2 = 0; w2 < PA_WAVES; ++w2)
-          m_tot = fmaxf(m_tot, s_ml[w2][g][0]);
-        float l_tot = 0.f, o[DS];
-#pragma unroll
-        for (int i = 0; i < DS; ++i) o[i] = 0.f;
-#pragma unroll
-        for (int w2 = 0; w2 < PA_WAVES; ++w2) {
-          const float mw = s_ml[w2][g][0];
-          const float sc = (mw == -INFINITY) ? 0.f : __expf(mw - m_tot);
-          l_tot += s_ml[w2][g][1] * sc;
-#pragma unroll
-          for (int i = 0; i < DS; ++i)
-            o[i] += s_acc[w2][g][p * DS + i] * sc;
-        }
-        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        const int qh = kvh * group_stride + g_base + g;
-        bf16* ob = out + ((size_t)seq * n_q + qh) * D + p * DS;
-#pragma unroll
-        for (int i = 0; i < DS; ++i) {
-          union { unsigned short u; __hip_bfloat16 b; } cv;
-          cv.u = f2bf(o[i] * inv);
-          ob[i] = cv.b;
-        }
-      }
-    }
-    return;
-  }
-  // multi-partition: each wave is its own flash-decode slice — write
-  // (m, l, acc) to the grid workspace; the reduce kernel combines.
-  if (t_local == 0) {
-#pragma unroll
-    for (int g = 0; g < GROUP; ++g) {
-      const int qh = kvh * group_stride + g_base + g;
-      float* wa = ws_acc +
-          (((size_t)seq * n_q + qh) * slices + slice) * D + p * DS;
-#pragma unroll
-      for (int i = 0; i < DS; ++i) wa[i] = acc[g][i];
-      if (p == 0) {
-        float* wm =
-            ws_ml + (((size_t)seq * n_q + qh) * slices + slice) * 2;
-        wm[0] = m[g];
-        wm[1] = l[g];
-      }
-    }
-  }
-}
-
 // combine partial (m, l, acc) across partitions: one wave per (seq, q-head)
 __global__ __launch_bounds__(WAVE)
 void paged_attn_reduce_kernel(bf16* __restrict__ out,
@@ -845,8 +581,6 @@ void paged_attn_reduce_kernel(bf16* __restrict__ out,
                               const float* __restrict__ ws_ml,
                               const int* __restrict__ seq_lens,
                               int n_q, int D, int n_parts) {
-  // n_parts here = total slices in the workspace (grid parts, or
-  // grid parts x PA_WAVES for the v2 kernel)
   const int seq = blockIdx.x;
   const int qh = blockIdx.y;
   const int lane = threadIdx.x;
@@ -1009,61 +743,10 @@ int ll_paged_attn_decode(void* out, void* ws_acc, void* ws_ml, const void* q,
                          const void* block_tables, const void* seq_lens,
                          int num_seqs, int max_blocks, int n_q, int n_kv,
                          int D, int block_size, int n_parts, float scale,
-                         int want_v2, int q_rstride, void* stream) {
+                         int q_rstride, void* stream) {
   if (block_size != PA_BLOCK || D > 128 || D % 32 != 0) return -2;
   if (n_q % n_kv != 0) return -2;
   hipStream_t s = (hipStream_t)stream;
-  const int group = n_q / n_kv;
-  // v2 (GQA-amortized, pages split across waves): caller must size the
-  // workspace for n_parts*PA_WAVES slices and pass want_v2 explicitly
-  const bool v2 = (want_v2 && D == 128 && group <= 16 &&
-                   (n_parts == 1 || ws_acc != nullptr));
-  if (v2) {
-    dim3 grid(num_seqs, n_kv, n_parts), block(PA_WAVES * WAVE);
-    const int slices = n_parts * PA_WAVES;
-#define LAUNCH_PA_V2(G, GS, GB)                                             \
-  hipLaunchKernelGGL((paged_attn_decode_v2_kernel<G>), grid, block, 0, s,   \
-                     (bf16*)out, (float*)ws_acc, (float*)ws_ml,             \
-                     (const bf16*)q, (const bf16*)kcache,                   \
-                     (const bf16*)vcache, nullptr, nullptr,                 \
-                     (const int*)block_tables, (const int*)seq_lens, n_q,   \
-                     n_kv, max_blocks, n_parts, scale, q_rstride, GS, GB)
-    // any GQA group: greedy 8/4/2/1 passes at the same group_stride.
-    // GROUP=8 runs SINGLE-PASS (16-lane/token layout) so the 70B
-    // shape reads each page once instead of twice (r2; the r1 +16%
-    // A/B left that amortization on the table)
-    // Default two-pass (max_g 4): the single-pass GROUP=8 kernel
-    // measured 40.08 vs 39.63 ms/step on llama-3-70b bs32 ctx1024 —
-    // the second pass's K/V re-reads are L2-hot while the 16-lane
-    // layout pays ~3x the cross-lane shuffles (profiles/
-    // r02_group8_single_pass_ab.md).  LLMLB_PA_MAX_G=8 enables it.
-    static const char* mgenv = getenv("LLMLB_PA_MAX_G");
-    const int max_g = mgenv ? atoi(mgenv) : 4;
-    for (int gb = 0, rem = group; rem > 0;) {
-      int g = rem >= 8 ? 8 : (rem >= 4 ? 4 : (rem >= 2 ? 2 : 1));
-      if (g > max_g) g = max_g;
-      switch (g) {
-        case 8: LAUNCH_PA_V2(8, group, gb); break;
-        case 4: LAUNCH_PA_V2(4, group, gb); break;
-        case 2: LAUNCH_PA_V2(2, group, gb); break;
-        default: LAUNCH_PA_V2(1, group, gb); break;
-      }
-      gb += g;
-      rem -= g;
-    }
-#undef LAUNCH_PA_V2
-    LL_CHECK(hipGetLastError());
-    if (n_parts > 1) {   // single partition combined in-workgroup
-      dim3 rgrid(num_seqs, n_q), rblock(WAVE);
-      hipLaunchKernelGGL(paged_attn_reduce_kernel, rgrid, rblock, 0, s,
-                         (bf16*)out, (const float*)ws_acc,
-                         (const float*)ws_ml, (const int*)seq_lens, n_q,
-                         D, slices);
-      LL_CHECK(hipGetLastError());
-    }
-    return 0;
-  }
-v1_path:
   dim3 grid(num_seqs, n_kv, n_parts), block(PA_WAVES * WAVE);
   hipLaunchKernelGGL(paged_attn_decode_kernel, grid, block, 0, s, (bf16*)out,
                      (float*)ws_acc, (float*)ws_ml, (const bf16*)q,
@@ -1076,57 +759,6 @@ v1_path:
     hipLaunchKernelGGL(paged_attn_reduce_kernel, rgrid, rblock, 0, s,
                        (bf16*)out, (const float*)ws_acc, (const float*)ws_ml,
                        (const int*)seq_lens, n_q, D, n_parts);
-    LL_CHECK(hipGetLastError());
-  }
-  return 0;
-}
-
-// FP8-KV decode attention: v2 kernel only (D=128, group<=16); same
-// workspace/reduce and single-partition LDS-combine semantics as bf16
-int ll_paged_attn_decode_fp8(void* out, void* ws_acc, void* ws_ml,
-                             const void* q, const void* kcache,
-                             const void* vcache, const void* k_scale,
-                             const void* v_scale,
-                             const void* block_tables,
-                             const void* seq_lens, int num_seqs,
-                             int max_blocks, int n_q, int n_kv, int D,
-                             int block_size, int n_parts, float scale,
-                             int q_rstride, void* stream) {
-  if (block_size != PA_BLOCK || D != 128) return -2;
-  if (n_q % n_kv != 0) return -2;
-  const int group = n_q / n_kv;
-  if (group > 16) return -2;
-  if (n_parts > 1 && ws_acc == nullptr) return -2;
-  hipStream_t s = (hipStream_t)stream;
-  dim3 grid(num_seqs, n_kv, n_parts), block(PA_WAVES * WAVE);
-  const int slices = n_parts * PA_WAVES;
-#define LAUNCH_V2_FP8(G, GS, GB)                                            \
-  hipLaunchKernelGGL((paged_attn_decode_v2_kernel<G, true>), grid, block,   \
-                     0, s, (bf16*)out, (float*)ws_acc, (float*)ws_ml,       \
-                     (const bf16*)q, (const bf16*)kcache,                   \
-                     (const bf16*)vcache, (const float*)k_scale,            \
-                     (const float*)v_scale, (const int*)block_tables,       \
-                     (const int*)seq_lens, n_q, n_kv, max_blocks,           \
-                     n_parts, scale, q_rstride, GS, GB)
-  for (int gb = 0, rem = group; rem > 0;) {
-    const int g = rem >= 8 ? 8 : (rem >= 4 ? 4 : (rem >= 2 ? 2 : 1));
-    switch (g) {
-      case 8: LAUNCH_V2_FP8(8, group, gb); break;
-      case 4: LAUNCH_V2_FP8(4, group, gb); break;
-      case 2: LAUNCH_V2_FP8(2, group, gb); break;
-      default: LAUNCH_V2_FP8(1, group, gb); break;
-    }
-    gb += g;
-    rem -= g;
-  }
-#undef LAUNCH_V2_FP8
-  LL_CHECK(hipGetLastError());
-  if (n_parts > 1) {
-    dim3 rgrid(num_seqs, n_q), rblock(WAVE);
-    hipLaunchKernelGGL(paged_attn_reduce_kernel, rgrid, rblock, 0, s,
-                       (bf16*)out, (const float*)ws_acc,
-                       (const float*)ws_ml, (const int*)seq_lens, n_q, D,
-                       slices);
     LL_CHECK(hipGetLastError());
   }
   return 0;

@@ -1,0 +1,400 @@
+// Attention of single tokens over a paged cache (Llama family): bf16 pages
+// of 64 or 128 numbers a head, or e4m3 pages of 128 with a scale per row.
+//
+//   out[s] = softmax(q[s] K^T scale) V,  K and V in pages of 16 rows
+//
+// What bounds it is reading the pages once.  One workgroup per sequence,
+// key/value head, up to 16 of its query heads and part of the pages: the
+// heads are the columns of the matrix cores' tiles, so a page is read from
+// LDS once for all of them.  Its four waves work on pages of their own, two
+// at a time, without a barrier: pages are whole runs of memory, copied to
+// LDS and waited for by the wave that asked.  What hides the wait is other
+// workgroups, two or more to a compute unit; a second stage of LDS in their
+// place was no faster.  Weights and sums stay floats: a weight enters its
+// product as the sum of two bf16 numbers, so products are exact to 2^-17.
+//
+// Sequences use as many parts as their length fills (16 pages each), which
+// the host does not know: the rest of the grid ends at once, and where one
+// part is all, it writes the result itself.
+//
+// Against a lane per part of a row, us (sequences, heads, tokens):
+//   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 41 (5.8 TB/s),
+//     64 x 3600 255 -> 156 (6.2 TB/s), 1 x 4000 47 -> 16
+//   e4m3, the same heads: 32 x 1800 79 -> 29, 64 x 900 70 -> 26; bound
+//     by widening to bf16 beside the reads
+//   bf16, 16 on 4 heads of 64: 64 x 900 61 -> 15, 1 x 100 12.3 -> 5.5
+#include "hybrid/lds_copy.h"
+#include "hybrid/mfma.h"
+
+#define PARTS_PAGES 16  // pages that are worth a part
+
+// 64 lanes copy 4 bytes each to 256 bytes of LDS
+__device__ __forceinline__ void copy4_to_lds(const void* src, unsigned to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
+               : "memory");
+}
+
+__device__ __forceinline__ int parts_used(int len, int parts) {
+  const int n = ((len + PAGE - 1) / PAGE + PARTS_PAGES - 1) / PARTS_PAGES;
+  return n < 1 ? 1 : (n < parts ? n : parts);
+}
+
+// e4m3 to bf16, exactly
+__device__ __forceinline__ u32x4 widen8(uint2 v) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const unsigned x = i ? v.y : v.x;
+    r[2 * i] = __builtin_bit_cast(
+        unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, false));
+    r[2 * i + 1] = __builtin_bit_cast(
+        unsigned, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, true));
+  }
+  return r;
+}
+
+// A wave's place in LDS: two pages of keys, two of values
+template <int D, bool FP8>
+struct PageAttn {
+  static constexpr int ROW = D * (FP8 ? 1 : 2), BYTES = PAGE * ROW;
+  static constexpr int PR = ROW / 16, CP = BYTES / 1024;  // pieces, copies
+  static constexpr int STAGE = 4 * BYTES + (FP8 ? 256 : 0);  // and scales
+  static constexpr int OP = D + 4;  // row of the waves' results
+  static constexpr int RESULTS = 4 * 16 * OP * 4;
+  static constexpr int LDS = 4 * STAGE > RESULTS ? 4 * STAGE : RESULTS;
+};
+
+// Piece c of row r lies at c ^ turn(r): lanes reading one piece of 16 rows
+// meet every bank once.
+template <int ROW>
+__device__ __forceinline__ int turn(int r) {
+  return ROW == 256 ? r & 15 : (r >> 1) & 7;
+}
+
+// acc [n][heads][parts][D], ml [n][heads][parts] (maximum, sum)
+template <int D, bool FP8>
+__global__ __launch_bounds__(256, 3) void page_attn_kernel(
+    bf16_t* __restrict__ out, float* __restrict__ ws_acc,
+    float* __restrict__ ws_ml, const bf16_t* __restrict__ q, int ldq,
+    const char* __restrict__ kc, const char* __restrict__ vc,
+    const float* __restrict__ k_scale, const float* __restrict__ v_scale,
+    const int* __restrict__ bt, const int* __restrict__ lens, int max_blocks,
+    int H, int G, int parts, float scale) {
+  using A = PageAttn<D, FP8>;
+  constexpr int KD = D / 32, VT = D / 16;
+  extern __shared__ __align__(1024) char lds[];
+  __shared__ float lm[4][16], ll[4][16];
+  const int R = H / G, ht = (R + 15) / 16;
+  const int seq = blockIdx.x, part = blockIdx.z;
+  const int kv = blockIdx.y / ht, h0 = blockIdx.y % ht * 16;
+  const int len = lens[seq];
+  const int used = parts_used(len, parts);
+  if (part >= used) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int n = lane & 15, g = lane >> 4;
+  const int heads = R - h0 < 16 ? R - h0 : 16;
+
+  // pairs of pages of this part, every fourth of this wave
+  const int pages = (len + PAGE - 1) / PAGE, pairs = (pages + 1) / 2;
+  const int per = (pairs + used - 1) / used;
+  const int first = part * per + wave;
+  const int stop = part * per + per < pairs ? part * per + per : pairs;
+  const int count = first < stop ? (stop - first + 3) / 4 : 0;
+  char* const st = lds + wave * A::STAGE;
+  const unsigned to = lds_byte(st);
+  const int* const row = bt + (size_t)seq * max_blocks;
+
+  // pages of 32 pairs, in lanes
+  int ids = 0;
+  auto look_up = [&](int i) {
+    const int p = 2 * (first + (i + lane / 2) * 4) + (lane & 1);
+    ids = row[p < pages ? p : pages - 1];
+  };
+  // source of lane's piece in copy j of a page
+  int off[A::CP];
+#pragma unroll
+  for (int j = 0; j < A::CP; ++j) {
+    const int r = j * (1024 / A::ROW) + lane / A::PR;
+    off[j] = r * A::ROW + (((lane % A::PR) ^ turn<A::ROW>(r)) * 16);
+  }
+  auto copy = [&](int i) {
+    if (i % 32 == 0) look_up(i);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int page = __builtin_amdgcn_readlane(ids, 2 * (i % 32) + t);
+      const size_t at = ((size_t)page * G + kv) * A::BYTES;
+#pragma unroll
+      for (int j = 0; j < A::CP; ++j) {
+        stream_to_lds(reinterpret_cast<const bf16_t*>(kc + at + off[j]),
+                      to + t * A::BYTES + j * 1024);
+        stream_to_lds(reinterpret_cast<const bf16_t*>(vc + at + off[j]),
+                      to + (2 + t) * A::BYTES + j * 1024);
+      }
+    }
+    if (FP8) {  // scales: 16 of each page's keys, then of the values
+      const int page =
+          g & 1 ? __builtin_amdgcn_readlane(ids, 2 * (i % 32) + 1)
+                : __builtin_amdgcn_readlane(ids, 2 * (i % 32));
+      const float* s = g < 2 ? k_scale : v_scale;
+      copy4_to_lds(s + ((size_t)page * G + kv) * PAGE + n,
+                   to + 4 * A::BYTES);
+    }
+  };
+
+  f32x4 o[VT];
+  float m = -1e30f, l = 0.f;
+#pragma unroll
+  for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (count) copy(0);
+  u32x4 qf[KD];
+#pragma unroll
+  for (int k = 0; k < KD; ++k) {
+    qf[k] = u32x4{0, 0, 0, 0};
+    if (n < heads)
+      qf[k] = *reinterpret_cast<const u32x4*>(
+          q + (size_t)seq * ldq + (size_t)(kv * R + h0 + n) * D + k * 32 +
+          g * 8);
+  }
+
+  for (int i = 0; i < count; ++i) {
+    wait_copies<0>();
+    const int j0 = (first + i * 4) * 32;  // the pair's first key
+    if (j0 + 32 > len) {
+      // rows past the end: an earlier sequence may have left anything there
+      const int r = lane / 2;
+      if (j0 + r >= len)
+#pragma unroll
+        for (int c = 0; c < A::ROW / 32; ++c)
+          *reinterpret_cast<uint4*>(st + 2 * A::BYTES + r * A::ROW +
+                                    (lane & 1) * (A::ROW / 2) + c * 16) =
+              make_uint4(0, 0, 0, 0);
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const char* k_row = st + t * A::BYTES + n * A::ROW;
+#pragma unroll
+      for (int k = 0; k < KD; ++k) {
+        u32x4 kf;
+        if (FP8) {
+          const int c = 2 * k + (g >> 1);
+          kf = widen8(*reinterpret_cast<const uint2*>(
+              k_row + (c ^ turn<A::ROW>(n)) * 16 + (g & 1) * 8));
+        } else {
+          kf = *reinterpret_cast<const u32x4*>(
+              k_row + ((k * 4 + g) ^ turn<A::ROW>(n)) * 16);
+        }
+        s[t] = mfma(kf, qf[k], s[t]);
+      }
+      f32x4 by = {scale, scale, scale, scale};
+      if (FP8)
+        by *= *reinterpret_cast<const f32x4*>(st + 4 * A::BYTES + t * 64 +
+                                              g * 16);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        s[t][r] = j0 + t * 16 + g * 4 + r < len ? s[t][r] * by[r] : -INFINITY;
+    }
+    float mx = m;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[t][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    if (__any(mx > m)) {  // seldom after the first pages
+      const float keep = __builtin_amdgcn_exp2f(m - mx);
+      m = mx;
+      l *= keep;
+#pragma unroll
+      for (int v = 0; v < VT; ++v) o[v] *= keep;
+    }
+    u32x4 hi, lo;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 p;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[r] = __builtin_amdgcn_exp2f(s[t][r] - m);
+        l += p[r];
+      }
+      if (FP8) {
+        const f32x4 by = *reinterpret_cast<const f32x4*>(
+            st + 4 * A::BYTES + 128 + t * 64 + g * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          p[r] = j0 + t * 16 + g * 4 + r < len ? p[r] * by[r] : 0.f;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        const unsigned h = to_bf16x2(p[r], p[r + 1]);
+        hi[2 * t + r / 2] = h;
+        lo[2 * t + r / 2] =
+            to_bf16x2(p[r] - __uint_as_float(h << 16),
+                      p[r + 1] - __uint_as_float(h & 0xffff0000u));
+      }
+    }
+    const char* values = st + 2 * A::BYTES;
+    if (FP8) {  // to bf16, in rows of 256 bytes over the stage's pages
+      const int r = lane / 2, c0 = (lane & 1) * 4;
+      uint4 x[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        x[c] = *reinterpret_cast<const uint4*>(
+            values + r * A::ROW + ((c0 + c) ^ turn<A::ROW>(r & 15)) * 16);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        char* const to = st + r * 256;
+        const int p = 2 * (c0 + c);
+        *reinterpret_cast<u32x4*>(to + (p ^ (r & 15)) * 16) =
+            widen8(make_uint2(x[c].x, x[c].y));
+        *reinterpret_cast<u32x4*>(to + ((p + 1) ^ (r & 15)) * 16) =
+            widen8(make_uint2(x[c].z, x[c].w));
+      }
+      values = st;
+    }
+    constexpr int VROW = 2 * D;
+    const int r = g * 4 + (n >> 2);
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const int c = 2 * v + ((n >> 1) & 1);
+      const u32x4 vf = load_columns(
+          reinterpret_cast<const unsigned short*>(
+              values + r * VROW + (c ^ turn<VROW>(r)) * 16 + (n & 1) * 8),
+          PAGE * D);
+      o[v] = mfma(vf, hi, o[v]);
+      o[v] = mfma(vf, lo, o[v]);
+    }
+    // all has been read before the next copy starts
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + 1 < count) copy(i + 1);
+  }
+
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+  if (g == 0) {
+    lm[wave][n] = m;
+    ll[wave][n] = l;
+  }
+  __syncthreads();  // the results lie where the stages were
+  float* const res = reinterpret_cast<float*>(lds);
+  if (n < heads) {
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
+      *reinterpret_cast<f32x4*>(
+          &res[(wave * 16 + n) * A::OP + v * 16 + g * 4]) = o[v];
+  }
+  __syncthreads();
+  for (int i = tid; i < heads * (D / 4); i += 256) {
+    const int h = i / (D / 4), c = i % (D / 4) * 4;
+    float top = lm[0][h], sum = 0.f;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) top = fmaxf(top, lm[w][h]);
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = __builtin_amdgcn_exp2f(lm[w][h] - top);
+      sum += f * ll[w][h];
+      x += *reinterpret_cast<const f32x4*>(&res[(w * 16 + h) * A::OP + c]) * f;
+    }
+    const size_t at = (size_t)seq * H + kv * R + h0 + h;
+    if (used == 1) {
+      const float f = sum > 0.f ? 1.f / sum : 0.f;
+      *reinterpret_cast<uint2*>(out + at * D + c) =
+          make_uint2(to_bf16x2(x[0] * f, x[1] * f),
+                     to_bf16x2(x[2] * f, x[3] * f));
+    } else {
+      *reinterpret_cast<f32x4*>(ws_acc + (at * parts + part) * D + c) = x;
+      if (c == 0) {
+        ws_ml[(at * parts + part) * 2] = top;
+        ws_ml[(at * parts + part) * 2 + 1] = sum;
+      }
+    }
+  }
+}
+
+// Joins the parts of sequences that used several; D / 4 lanes a head.
+template <int D>
+__global__ __launch_bounds__(256) void page_join_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ ws_acc,
+    const float* __restrict__ ws_ml, const int* __restrict__ lens, int n_rows,
+    int H, int parts) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const size_t at = i / D;
+  if (at >= (size_t)n_rows * H) return;
+  const int used = parts_used(lens[at / H], parts);
+  if (used == 1) return;
+  const float* ml = ws_ml + at * parts * 2;
+  const float* acc = ws_acc + at * parts * D + i % D;
+  float top = -1e30f, sum = 0.f;
+  for (int p = 0; p < used; ++p) top = fmaxf(top, ml[2 * p]);
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < used; ++p) {
+    const float f = __builtin_amdgcn_exp2f(ml[2 * p] - top);
+    sum += f * ml[2 * p + 1];
+    x += *reinterpret_cast<const f32x4*>(acc + (size_t)p * D) * f;
+  }
+  const float f = sum > 0.f ? 1.f / sum : 0.f;
+  *reinterpret_cast<uint2*>(out + i) = make_uint2(
+      to_bf16x2(x[0] * f, x[1] * f), to_bf16x2(x[2] * f, x[3] * f));
+}
+
+template <int D, bool FP8>
+static int page_attn_launch(void* out, void* acc, void* ml, const void* q,
+                            int ldq, const void* kc, const void* vc,
+                            const void* ks, const void* vs, const void* bt,
+                            const void* lens, int n, int max_blocks, int H,
+                            int G, int parts, float scale, hipStream_t st) {
+  constexpr int lds = PageAttn<D, FP8>::LDS;
+  static_assert(lds + 512 <= 160 * 1024, "LDS of a compute unit");
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(page_attn_kernel<D, FP8>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const int tiles = G * ((H / G + 15) / 16);
+  hipLaunchKernelGGL((page_attn_kernel<D, FP8>), dim3(n, tiles, parts),
+                     dim3(256), lds, st, (bf16_t*)out, (float*)acc,
+                     (float*)ml, (const bf16_t*)q, ldq, (const char*)kc,
+                     (const char*)vc, (const float*)ks, (const float*)vs,
+                     (const int*)bt, (const int*)lens, max_blocks, H, G,
+                     parts, scale * LOG2E);
+  HY_CHECK();
+  if (parts == 1) return 0;
+  const size_t threads = (size_t)n * H * (D / 4);
+  hipLaunchKernelGGL(page_join_kernel<D>,
+                     dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                     st, (bf16_t*)out, (const float*)acc, (const float*)ml,
+                     (const int*)lens, n, H, parts);
+  HY_CHECK();
+  return 0;
+}
+
+// q [n, H, D] with rows ldq apart; caches [pages, G, 16, D], e4m3 where
+// scales are given; acc and ml for ``parts`` parts, unused by one.
+// -2: not for this kernel.
+extern "C" int ll_page_attn(void* out, void* acc, void* ml, const void* q,
+                            int ldq, const void* kc, const void* vc,
+                            const void* ks, const void* vs, const void* bt,
+                            const void* lens, int n, int max_blocks, int H,
+                            int G, int D, int block_size, int parts,
+                            float scale, void* stream) {
+  if (n < 0 || G <= 0 || H <= 0 || H % G || block_size != PAGE || parts < 1 ||
+      parts > 65535 || (parts > 1 && (!acc || !ml)) || ldq % 8 ||
+      (uintptr_t)q % 16 || G * ((H / G + 15) / 16) > 65535)
+    return -2;
+  if ((ks != nullptr) != (vs != nullptr) || (ks && D != 128)) return -2;
+  if (n == 0) return 0;
+  hipStream_t st = (hipStream_t)stream;
+#define PAGE_ATTN(D, FP8)                                                   \
+  return page_attn_launch<D, FP8>(out, acc, ml, q, ldq, kc, vc, ks, vs, \
+                                     bt, lens, n, max_blocks, H, G, parts, \
+                                     scale, st)
+  if (ks) PAGE_ATTN(128, true);
+  if (D == 128) PAGE_ATTN(128, false);
+  if (D == 64) PAGE_ATTN(64, false);
+#undef PAGE_ATTN
+  return -2;
+}

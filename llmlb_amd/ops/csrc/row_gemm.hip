@@ -31,7 +31,7 @@
 // Tile: 16 MT rows of W, 16 NT rows of x.  KW waves; each has S stages of
 // LDS, one piece of 64 of the depth of all the tile's rows a stage.
 template <int NT, int MT, int KW, int S>
-__global__ __launch_bounds__(KW * 64) void row_gemm_kernel(
+__global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
     const bf16_t* __restrict__ w, int N, int M, int K, int ldx) {
   constexpr int ROWS = 16 * (NT + MT), C = ROWS / 8, STAGE = ROWS * 128;

@@ -1,0 +1,95 @@
+"""Decode attention over pages on the matrix cores (page_attention.hip)
+against the same attention in 64 bits, at the edges of pages, pairs of
+pages, parts and tiles of heads."""
+import pytest
+import torch
+
+import llmlb_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+LENS = [1, 2, 15, 16, 17, 31, 32, 33, 127, 128, 129, 255, 257, 512, 513, 1100]
+
+
+def _exact(q, k, v, bt, lens, scale):
+    """(result, error that float sums and one rounding to bf16 may add)"""
+    out, bound = [], []
+    for s, n in enumerate(lens.tolist()):
+        pages = bt[s, :-(-n // 16)].long()
+        ks, vs = (t[pages].double().transpose(0, 1).flatten(1, 2)[:, :n]
+                  for t in (k, v))                      # [G, n, D]
+        qs = q[s].double().view(ks.shape[0], -1, q.shape[-1])
+        p = torch.softmax(qs @ ks.transpose(1, 2) * scale, -1)
+        out.append((p @ vs).flatten(0, 1))
+        # scores are off by about 2^-24 of the sum of magnitudes, weights
+        # by as much and by 2^-17 where they enter the product
+        off = (qs.abs() @ ks.abs().transpose(1, 2)).amax(-1, keepdim=True) \
+            * scale * 2.0 ** -22 + 2.0 ** -16
+        bound.append(((p @ vs.abs()) * off).flatten(0, 1))
+    out, bound = torch.stack(out), torch.stack(bound)
+    return out, bound + out.abs() * 2.0 ** -8
+
+
+def _case(heads, kv, D, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    lens = torch.tensor(LENS, dtype=torch.int32, device=DEV)
+    per = [-(-n // 16) for n in LENS]
+    ids = torch.randperm(sum(per), generator=g, device=DEV).int() + 1
+    bt = torch.zeros(len(LENS), 80, dtype=torch.int32, device=DEV)
+    at = 0
+    for s, n in enumerate(per):
+        bt[s, :n] = ids[at:at + n]
+        at += n
+    wide = torch.randn(len(LENS), heads * D + 64, generator=g,
+                       device=DEV).bfloat16()
+    q = wide[:, 64:].unflatten(1, (heads, D))     # rows of a wider matrix
+    k, v = torch.randn(2, sum(per) + 1, kv, 16, D, generator=g, device=DEV)
+    return q, k, v, bt, lens, per
+
+
+@pytest.mark.parametrize("parts", [None, 1, 3, 16])
+@pytest.mark.parametrize("heads,kv,D", [(4, 4, 128), (32, 8, 128),
+                                        (14, 2, 64), (16, 1, 64),
+                                        (34, 2, 128)])
+def test_page_attention(heads, kv, D, parts):
+    q, k, v, bt, lens, per = _case(heads, kv, D, heads + D)
+    k, v = k.bfloat16(), v.bfloat16()
+    ref, bound = _exact(q, k, v, bt, lens, D ** -0.5)
+    # what an earlier sequence left behind a sequence's end is not read
+    for s, n in enumerate(LENS):
+        if n % 16:
+            k[bt[s, per[s] - 1].long(), :, n % 16:] = float("nan")
+            v[bt[s, per[s] - 1].long(), :, n % 16:] = float("nan")
+    out = ops.paged_attn_decode(q, k, v, bt, lens, D ** -0.5, n_parts=parts)
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("parts", [1, 4])
+@pytest.mark.parametrize("heads,kv", [(32, 8), (16, 1)])
+def test_page_attention_fp8(heads, kv, parts):
+    q, k, v, bt, lens, per = _case(heads, kv, 128, heads)
+    caches, scales, wide = [], [], []
+    for t in (k, v):
+        s = torch.rand(t.shape[:3], device=DEV) * 0.01 + 0.001
+        b = (t / s[..., None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+        wide.append(b.double() * s[..., None].double())
+        caches.append(b.view(torch.uint8))
+        scales.append(s)
+    ref, bound = _exact(q, *wide, bt, lens, 128 ** -0.5)
+    for s, n in enumerate(LENS):
+        if n % 16:
+            page = bt[s, per[s] - 1].long()
+            for c, sc in zip(caches, scales):
+                c[page, :, n % 16:] = 0x7F              # not a number
+                sc[page, :, n % 16:] = float("nan")
+    out = ops.paged_attn_decode(q, *caches, bt, lens, 128 ** -0.5,
+                                n_parts=parts, k_scale=scales[0],
+                                v_scale=scales[1])
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+def test_no_tokens_give_zeros():
+    q, k, v, bt, lens, _ = _case(8, 2, 128, 3)
+    out = ops.paged_attn_decode(q, k.bfloat16(), v.bfloat16(), bt,
+                                torch.zeros_like(lens), 0.1)
+    assert (out == 0).all()
