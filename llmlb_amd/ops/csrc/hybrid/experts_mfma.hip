@@ -10,8 +10,7 @@
 // Both compute (w in^T) tiles: a lane holds outputs 4g..4g+3 (g = lane/16)
 // of pair n = lane % 16.
 #include "experts.h"
-#include "lds_copy.h"
-#include "mfma.h"
+#include "row_tile.h"
 
 // LDS rows are P pieces of 16 bytes; piece c of row r lies at
 // c ^ swizzle(r), so that lanes reading one piece of the rows of an
@@ -176,123 +175,70 @@ void expert_tile_kernel(
   }
 }
 
-// Few pairs: workgroup (expert, 16 NT outputs), the depth split over its
-// four waves.
+// Few pairs: workgroup (expert, 32 outputs), tiles of up to 64 of the
+// expert's pairs as in row_tile.h.  Bound by reading the matrices: both
+// products of 16 experts of 4096 x 1280 took 105 us for 64 tokens with
+// operands loaded straight into registers, 67 (5.0 TB/s) this way; 8 tokens
+// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  32 outputs: 16 read the
+// inputs twice as often (89 us), 64 are too few workgroups where few
+// experts are chosen (one token 26 -> 31).
 #define FEW_PAIRS 2048  // most that fit a workgroup's list
-template <int MT, int NT>
-__device__ __forceinline__ void expert_few_rows(
-    bf16_t* __restrict__ out, const bf16_t* __restrict__ in,
-    const bf16_t* (&wp)[NT], const unsigned short* list, int first, int count,
-    float* red, int n0, int N, int K, int div, int act) {
-  constexpr int RP = 16 * NT + 4;
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & 63;
-  const int n = lane & 15, g = lane >> 4;
-  const bf16_t* ip[MT];
-#pragma unroll
-  for (int a = 0; a < MT; ++a) {
-    const int r = first + a * 16 + n;
-    ip[a] = in + (size_t)(list[r < count ? r : count - 1] / div) * K;
-  }
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int a = 0; a < MT; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // CH pieces of 64 of the depth are in flight; past its end inputs count
-  // as zero
-  constexpr int CH = 2;
-  for (int k0 = wave * 64; k0 < K; k0 += CH * 256) {
-    u32x4 wf[CH][2][NT], xf[CH][2][MT];
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int k = k0 + c * 256 + s * 32 + g * 8;
-        const int kk = k < K ? k : 0;
-#pragma unroll
-        for (int b = 0; b < NT; ++b)
-          wf[c][s][b] = *reinterpret_cast<const u32x4*>(wp[b] + kk);
-#pragma unroll
-        for (int a = 0; a < MT; ++a)
-          xf[c][s][a] = *reinterpret_cast<const u32x4*>(ip[a] + kk);
-      }
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const bool inside = k0 + c * 256 + s * 32 + g * 8 < K;
-#pragma unroll
-        for (int a = 0; a < MT; ++a) {
-          if (!inside) xf[c][s][a] = u32x4{0, 0, 0, 0};
-#pragma unroll
-          for (int b = 0; b < NT; ++b)
-            acc[a][b] = mfma(wf[c][s][b], xf[c][s][a], acc[a][b]);
-        }
-      }
-  }
-#pragma unroll
-  for (int a = 0; a < MT; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b)
-      *reinterpret_cast<f32x4*>(
-          &red[(wave * 16 * MT + a * 16 + n) * RP + b * 16 + g * 4]) =
-          acc[a][b];
-  __syncthreads();
-  for (int i = tid; i < 16 * MT * 4 * NT; i += 256) {
-    const int r = i / (4 * NT), c = i % (4 * NT) * 4;
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      x += *reinterpret_cast<const f32x4*>(
-          &red[(v * 16 * MT + r) * RP + c]);
-    if (act) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[j] = fmaxf(x[j], 0.f);
-        x[j] *= x[j];
-      }
-    }
-    if (first + r < count && n0 + c < N)
-      *reinterpret_cast<uint2*>(out + (size_t)list[first + r] * N + n0 + c) =
-          make_uint2(to_bf16x2(x[0], x[1]), to_bf16x2(x[2], x[3]));
-  }
-  __syncthreads();
-}
-
+// NT and S for the tile that the pairs need: about the same LDS for each,
+// so that two workgroups share a compute unit
+#define FEW_MT 2
+#define FEW_KW 4
 template <int NT>
-__global__ __launch_bounds__(256) void expert_few_kernel(
+using FewTile = RowTile<NT, FEW_MT, FEW_KW, NT == 1 ? 3 : (NT == 2 ? 2 : 1)>;
+#define FEW_LDS FewTile<1>::LDS
+static_assert(FewTile<2>::LDS <= FEW_LDS && FewTile<4>::LDS <= FEW_LDS,
+              "one size of LDS for all tiles");
+
+__global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ in,
     const bf16_t* __restrict__ w, const int* __restrict__ index, int N, int K,
     int div, int act, int n_pairs) {
-  constexpr int MT = 4;
-  __shared__ float red[4 * 16 * MT * (16 * NT + 4)];
+  extern __shared__ __align__(1024) char lds[];
   __shared__ unsigned short list[FEW_PAIRS];
   __shared__ int len;
-  const int e = blockIdx.y, n0 = blockIdx.x * 16 * NT;
+  const int e = blockIdx.y, n0 = blockIdx.x * 16 * FEW_MT;
   const int tid = threadIdx.x;
   if (tid == 0) len = 0;
   __syncthreads();
-  for (int p = tid; p < n_pairs; p += 256)
+  for (int p = tid; p < n_pairs; p += FEW_KW * 64)
     if (index[p] == e) list[atomicAdd(&len, 1)] = (unsigned short)p;
   __syncthreads();
   const int count = len;
-  if (count == 0) return;
-  const bf16_t* wp[NT];
+  auto tile = [&](auto t, int first) {
+    using Tile = decltype(t);
+    Tile::run(
+        lds, K, blockIdx.x + e,
+        [&](int r) {
+          const int p = first + r < count ? first + r : count - 1;
+          return in + (size_t)(list[p] / div) * K;
+        },
+        [&](int r) {
+          return w + ((size_t)e * N + (n0 + r < N ? n0 + r : N - 1)) * K;
+        });
+    Tile::each(lds, [&](int r, int c, f32x4 v) {
+      if (act) {
 #pragma unroll
-  for (int b = 0; b < NT; ++b) {
-    const int r = n0 + b * 16 + (tid & 15);
-    wp[b] = w + ((size_t)e * N + (r < N ? r : N - 1)) * K;
-  }
-#define ROWS(M)                                                             \
-  expert_few_rows<M, NT>(out, in, wp, list, first, count, red, n0, N, K, div, \
-                         act)
-  for (int first = 0; first < count; first += 16 * MT) {
+        for (int j = 0; j < 4; ++j) {
+          v[j] = fmaxf(v[j], 0.f);
+          v[j] *= v[j];
+        }
+      }
+      if (first + r < count && n0 + c < N)
+        *reinterpret_cast<uint2*>(out + (size_t)list[first + r] * N + n0 + c) =
+            make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+    });
+    __syncthreads();
+  };
+  for (int first = 0; first < count; first += 64) {
     const int left = count - first;
-    if (left <= 16) ROWS(1);
-    else if (left <= 32) ROWS(2);
-    else ROWS(MT);
+    if (left <= 16) tile(FewTile<1>{}, first);
+    else if (left <= 32) tile(FewTile<2>{}, first);
+    else tile(FewTile<4>{}, first);
   }
-#undef ROWS
 }
 
 extern "C" {
@@ -337,8 +283,13 @@ int hy_expert_few(void* out, const void* in, const void* w, const void* index,
       E > 65535 || n_pairs > FEW_PAIRS)
     return -2;
   if (n_pairs <= 0) return 0;
-  hipLaunchKernelGGL((expert_few_kernel<2>), dim3((N + 31) / 32, E),
-                     dim3(256), 0, (hipStream_t)stream, (bf16_t*)out,
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(expert_few_kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS);
+  if (sized != hipSuccess) return -1;
+  hipLaunchKernelGGL(expert_few_kernel,
+                     dim3((N + 16 * FEW_MT - 1) / (16 * FEW_MT), E),
+                     dim3(FEW_KW * 64), FEW_LDS, (hipStream_t)stream, (bf16_t*)out,
                      (const bf16_t*)in, (const bf16_t*)w, (const int*)index,
                      N, K, div, act, n_pairs);
   HY_CHECK();
