@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
-from ..ops import linear_decode
+from ..ops import linear_act, linear_decode
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
@@ -264,6 +264,9 @@ class DenseFF(nn.Module):
         self.w_down = _param(F.pad(w["down"], (0, gap)).to(**to))
 
     def forward(self, x):
+        u = linear_act(x, self.w_up, self.act)
+        if u is not None:
+            return _linear(u, self.w_down)
         u = _linear(x, self.w_up)
         if self.act == "gelu":
             hy.gelu_tanh_(u)
@@ -440,6 +443,9 @@ class ClampedSwiGLU(nn.Module):
         self.w_in = _param(stacked.to(dtype=self.dtype, device=self.device))
 
     def inner(self, x, out) -> None:
+        if linear_act(x, self.w_in, "clamped", out, self.u_off, self.limit,
+                      self.sharpness) is not None:
+            return
         hy.clamped_swiglu(out, _linear(x, self.w_in), self.u_off, self.limit,
                           self.sharpness)
 

@@ -22,6 +22,7 @@ import torch.nn as nn
 from ..backend.kv_cache import BLOCK_SIZE, HybridCache
 from ..backend.ragged import RaggedBatch
 from ..ops import hybrid as hy
+from ..ops import linear_act
 from ..parallel.tp import TPContext, get_tp_context
 from .mixers import _linear, _param
 
@@ -172,8 +173,9 @@ class PackedCausalLM(nn.Module):
 
     def logits(self, x: torch.Tensor, index=None) -> torch.Tensor:
         """float32 logits of the rows ``index`` (int32; None: all)."""
-        return hy.soft_cap(_linear(self.final_rows(x, index), self.head),
-                           self.cfg.logit_softcap)
+        rows, cap = self.final_rows(x, index), self.cfg.logit_softcap
+        z = linear_act(rows, self.head, "capped", a=cap or 0.0)
+        return hy.soft_cap(_linear(rows, self.head), cap) if z is None else z
 
     @torch.inference_mode()
     def forward_dense(self, input_ids: torch.Tensor) -> torch.Tensor:

@@ -676,23 +676,62 @@ def quantize_fp8_weight(w: torch.Tensor):
     return q.view(torch.uint8).contiguous(), scale.squeeze(1).contiguous()
 
 
-def _row_gemm(x: torch.Tensor, weight: torch.Tensor
-              ) -> torch.Tensor | None:
+_ROW_ACTS = {"plain": 0, "relu2": 1, "gelu": 2, "swiglu": 3, "clamped": 4,
+             "capped": 5}
+
+
+def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
+              out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
+              b: float = 0.0) -> torch.Tensor | None:
     """x @ W^T by row_gemm.hip, or None where it does not take the
     operands (depth or rows no multiple of 8, unaligned views)."""
     N, K = x.shape
     M = weight.shape[0]
+    gated = act in ("swiglu", "clamped")
     if (weight.dtype != x.dtype or x.stride(1) != 1
             or not weight.is_contiguous()):
         return None
-    out = torch.empty(N, M, dtype=x.dtype, device=x.device)
+    if gated:
+        M -= up                       # rows of gate and of up
+        if up < M:
+            return None
+    if out is None:
+        out = torch.empty(N, M, device=x.device, dtype=torch.float32
+                          if act == "capped" else x.dtype)
+    elif out.stride(1) != 1 or out.shape != (N, M):
+        return None
     rc = _require_native().ll_row_gemm(
-        _ptr(out), _ptr(x), _ptr(weight), ctypes.c_int(N), ctypes.c_int(M),
-        ctypes.c_int(K), ctypes.c_int(x.stride(0)), _stream())
+        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
+        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K),
+        ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
+        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b), _stream())
     if rc == -2:
         return None
     _check(rc, "ll_row_gemm")
     return out
+
+
+def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
+            and x.dim() == 2 and 0 < x.shape[0] <= 128
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or weight.requires_grad)))
+
+
+def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
+               out: torch.Tensor | None = None, up: int = 0,
+               a: float = 0.0, b: float = 0.0) -> torch.Tensor | None:
+    """act(x @ W^T) of up to 128 bf16 rows in one launch, into ``out``
+    (columns of wider rows) if given; None where row_gemm.hip does not
+    take it.
+
+    act: "relu2", "gelu" (its tanh form), "capped" (float32,
+    a tanh(z / a); a = 0: a widening); with gate in the first rows of
+    ``weight`` and up from row ``up`` on "swiglu", and "clamped" with
+    limit a and sharpness b (see hybrid.clamped_swiglu)."""
+    if _USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight):
+        return None
+    return _row_gemm(x, weight, act, out, up, a, b)
 
 
 def linear_decode(x: torch.Tensor, weight: torch.Tensor,
@@ -707,11 +746,7 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor,
     = this, "1"/"on" = the staged kernels of decode_gemm.hip wherever
     they are legal, "0"/"off" = hipBLASLt only."""
     mode = _USE_CUSTOM_DECODE_GEMM
-    if (mode in ("0", "false", "off") or not x.is_cuda or _lib is None
-            or x.dtype != torch.bfloat16 or x.dim() != 2
-            or not 0 < x.shape[0] <= 128
-            or (torch.is_grad_enabled()
-                and (x.requires_grad or weight.requires_grad))):
+    if mode in ("0", "false", "off") or not _takes_row_gemm(x, weight):
         return torch.nn.functional.linear(x, weight)
     N, K = x.shape
     M = weight.shape[0]

@@ -143,6 +143,17 @@ __device__ __forceinline__ float softplus_f(float x) {
   return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x)));
 }
 
+__device__ __forceinline__ float gelu_tanh_f(float z) {
+  const float k = 0.7978845608028654f;  // sqrt(2 / pi)
+  return 0.5f * z * (1.f + tanhf(k * (z + 0.044715f * z * z * z)));
+}
+// the same through one exponential, for 16-bit results
+__device__ __forceinline__ float gelu_tanh_fast(float z) {
+  const float k = 0.7978845608028654f;
+  const float t = k * (z + 0.044715f * z * z * z);
+  return z / (1.f + __expf(-2.f * t));
+}
+
 // flat token slot of position ``pos`` of the sequence in table row ``row``
 __device__ __forceinline__ size_t page_slot(const int* bt, int max_blocks,
                                             int row, int pos) {

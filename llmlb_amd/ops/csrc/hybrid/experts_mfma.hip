@@ -219,7 +219,8 @@ __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
         [&](int r) {
           return w + ((size_t)e * N + (n0 + r < N ? n0 + r : N - 1)) * K;
         });
-    Tile::each(lds, [&](int r, int c, f32x4 v) {
+    Tile::each(4 * FEW_MT, [&](int r, int c) {
+      f32x4 v = Tile::sum(lds, r, c);
       if (act) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {

@@ -117,18 +117,20 @@ struct RowTile {
     __syncthreads();
   }
 
-  // put(r, c, v): outputs c .. c + 3 of the tile's row r of x
-  template <class F>
-  static __device__ __forceinline__ void each(const char* lds, F put) {
+  // outputs c .. c + 3 of the tile's row r of x
+  static __device__ __forceinline__ f32x4 sum(const char* lds, int r, int c) {
     const float* const sums = reinterpret_cast<const float*>(lds);
-    for (int i = threadIdx.x; i < 64 * NT * MT; i += KW * 64) {
-      const int r = i / (4 * MT), c = i % (4 * MT) * 4;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < KW; ++w)
-        v += *reinterpret_cast<const f32x4*>(
-            &sums[(w * 16 * NT + r) * RP + c]);
-      put(r, c, v);
-    }
+    for (int w = 0; w < KW; ++w)
+      v += *reinterpret_cast<const f32x4*>(
+          &sums[(w * 16 * NT + r) * RP + c]);
+    return v;
+  }
+  // put(r, c) for every four of the first 4 * quads outputs of all rows
+  template <class F>
+  static __device__ __forceinline__ void each(int quads, F put) {
+    for (int i = threadIdx.x; i < 16 * NT * quads; i += KW * 64)
+      put(i / quads, i % quads * 4);
   }
 };

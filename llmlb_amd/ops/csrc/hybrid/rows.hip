@@ -442,17 +442,6 @@ __global__ __launch_bounds__(256) void post_pre_norm_kernel(
   }
 }
 
-__device__ __forceinline__ float gelu_tanh_f(float z) {
-  const float k = 0.7978845608028654f;  // sqrt(2 / pi)
-  return 0.5f * z * (1.f + tanhf(k * (z + 0.044715f * z * z * z)));
-}
-// the same through one exponential, for 16-bit results
-__device__ __forceinline__ float gelu_tanh_fast(float z) {
-  const float k = 0.7978845608028654f;
-  const float t = k * (z + 0.044715f * z * z * z);
-  return z / (1.f + __expf(-2.f * t));
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_tanh_kernel(T* __restrict__ y,
                                                         long long n) {

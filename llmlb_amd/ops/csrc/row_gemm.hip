@@ -17,86 +17,159 @@
 // every tile reads all of its x and W.
 #include "hybrid/row_tile.h"
 
-template <int NT, int MT, int KW, int S>
+// What becomes of a sum before it is stored: a launch less than a kernel of
+// its own, 3 us to 5 in decoding, and no rounding in between.  With two
+// matrices, gate and up, a tile's rows are half of the one and half of the
+// other, at the same outputs.
+enum { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };
+struct RowAct {
+  int kind;
+  int up;      // SWIGLU, CLAMPED: the first row of up
+  float a, b;  // CLAMPED: limit, sharpness; CAPPED: cap (0: none)
+};
+__device__ __forceinline__ float row_act(const RowAct& act, float z) {
+  if (act.kind == RELU2) {
+    z = fmaxf(z, 0.f);
+    return z * z;
+  }
+  if (act.kind == GELU) return gelu_tanh_fast(z);
+  if (act.kind == CAPPED && act.a > 0.f) return act.a * tanhf(z / act.a);
+  return z;
+}
+__device__ __forceinline__ float row_gate(const RowAct& act, float g,
+                                          float u) {
+  if (act.kind == SWIGLU) return g / (1.f + __expf(-g)) * u;
+  g = fminf(g, act.a);
+  u = fminf(fmaxf(u, -act.a), act.a);
+  return g / (1.f + __expf(-act.b * g)) * (u + 1.f);
+}
+
+// M outputs; CAPPED results are floats, all others bf16
+template <int NT, int MT, int KW, int S, bool GATED>
 __global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(
-    bf16_t* __restrict__ out, const bf16_t* __restrict__ x,
-    const bf16_t* __restrict__ w, int N, int M, int K, int ldx) {
+    void* __restrict__ out_, int ld_out, const bf16_t* __restrict__ x,
+    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, RowAct act) {
   using Tile = RowTile<NT, MT, KW, S>;
+  constexpr int OUT = GATED ? 8 * MT : 16 * MT;  // outputs a tile
   extern __shared__ __align__(1024) char lds[];
   // tiles of the same rows of W are 8 apart: on one XCD
   const int across = (N + 16 * NT - 1) / (16 * NT);
   const int in = blockIdx.x % (8 * across);
   const int tile = blockIdx.x / (8 * across) * 8 + in % 8;
-  const int m0 = tile * 16 * MT, n0 = in / 8 * 16 * NT;
+  const int m0 = tile * OUT, n0 = in / 8 * 16 * NT;
   if (m0 >= M) return;
   Tile::run(
       lds, K, tile >> 3,
       [&](int r) {
         return x + (size_t)(n0 + r < N ? n0 + r : N - 1) * ldx;
       },
-      [&](int r) { return w + (size_t)(m0 + r < M ? m0 + r : M - 1) * K; });
-  Tile::each(lds, [&](int r, int c, f32x4 v) {
-    if (n0 + r < N && m0 + c < M)
-      *reinterpret_cast<uint2*>(out + (size_t)(n0 + r) * M + m0 + c) =
+      [&](int r) {
+        const bool up = GATED && r >= OUT;
+        const int m = m0 + (up ? r - OUT : r);
+        return w + (size_t)((up ? act.up : 0) + (m < M ? m : M - 1)) * K;
+      });
+  Tile::each(OUT / 4, [&](int r, int c) {
+    f32x4 v = Tile::sum(lds, r, c);
+    if (GATED) {
+      const f32x4 u = Tile::sum(lds, r, c + OUT);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = row_gate(act, v[i], u[i]);
+    } else if (act.kind != PLAIN) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = row_act(act, v[i]);
+    }
+    if (n0 + r >= N || m0 + c >= M) return;
+    const size_t at = (size_t)(n0 + r) * ld_out + m0 + c;
+    if (!GATED && act.kind == CAPPED)
+      *reinterpret_cast<f32x4*>(static_cast<float*>(out_) + at) = v;
+    else
+      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out_) + at) =
           make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
   });
 }
 
-template <int NT, int MT, int KW, int S>
-static int row_gemm_launch(void* out, const void* x, const void* w, int N,
-                           int M, int K, int ldx, hipStream_t stream) {
+struct RowGemm {
+  void* out;
+  int ld_out;
+  const bf16_t *x, *w;
+  int N, M, K, ldx;
+  RowAct act;
+  hipStream_t stream;
+};
+
+template <int NT, int MT, int KW, int S, bool GATED>
+static int row_gemm_launch(const RowGemm& p) {
   constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(row_gemm_kernel<NT, MT, KW, S>),
+      reinterpret_cast<const void*>(row_gemm_kernel<NT, MT, KW, S, GATED>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (sized != hipSuccess) return -1;
-  const int down = (M + 16 * MT - 1) / (16 * MT);
-  const int across = (N + 16 * NT - 1) / (16 * NT);
-  hipLaunchKernelGGL((row_gemm_kernel<NT, MT, KW, S>),
+  constexpr int OUT = GATED ? 8 * MT : 16 * MT;
+  const int down = (p.M + OUT - 1) / OUT;
+  const int across = (p.N + 16 * NT - 1) / (16 * NT);
+  hipLaunchKernelGGL((row_gemm_kernel<NT, MT, KW, S, GATED>),
                      dim3((down + 7) / 8 * 8 * across), dim3(KW * 64), lds,
-                     stream, (bf16_t*)out, (const bf16_t*)x, (const bf16_t*)w,
-                     N, M, K, ldx);
+                     p.stream, p.out, p.ld_out, p.x, p.w, p.N, p.M, p.K,
+                     p.ldx, p.act);
   HY_CHECK();
   return 0;
 }
 
-// 0: done, -2: not for this kernel.  Rows of x start ldx numbers apart.
-extern "C" int ll_row_gemm(void* out, const void* x, const void* w, int N,
-                           int M, int K, int ldx, void* stream) {
-  if (N <= 0 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
-      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 8)
-    return -2;
-  // The largest tile of which there are enough for the chip: a larger one
-  // reads less (64 x 64 half of what 32 x 32 does), but under about 176 of
-  // them, two thirds of the compute units, idle ones cost more than that
-  // (64 rows against 6144 x 4096: 96 tiles of 64 x 64 17.0 us, 192 of
-  // 32 x 64 15.9; against 11264 x 2048: 176 of 64 x 64 13.8, 352 of 32 x 64
-  // 18).  Rows of x go in equal shares of up to 4 x 16.
-  const int tiles = (N + 15) / 16, shares = (tiles + 3) / 4;
+// The largest tile of which there are enough for the chip: a larger one
+// reads less (64 x 64 half of what 32 x 32 does), but under about 176 of
+// them, two thirds of the compute units, idle ones cost more than that (64
+// rows against 6144 x 4096: 96 tiles of 64 x 64 17.0 us, 192 of 32 x 64
+// 15.9; against 11264 x 2048: 176 of 64 x 64 13.8, 352 of 32 x 64 18).
+// Rows of x go in equal shares of up to 4 x 16.
+template <bool GATED>
+static int row_gemm_pick(const RowGemm& p) {
+  const int tiles = (p.N + 15) / 16, shares = (tiles + 3) / 4;
   const int nt = (tiles + shares - 1) / shares;
+  const int rows = GATED ? 2 * p.M : p.M;
   auto enough = [&](int n, int m) {
-    return (size_t)((M + 16 * m - 1) / (16 * m)) * ((tiles + n - 1) / n) >=
+    return (size_t)((rows + 16 * m - 1) / (16 * m)) * ((tiles + n - 1) / n) >=
            176;
   };
-  hipStream_t st = (hipStream_t)stream;
 #define ROW_GEMM(NT, MT, KW, S) \
-  return row_gemm_launch<NT, MT, KW, S>(out, x, w, N, M, K, ldx, st)
+  return row_gemm_launch<NT, MT, KW, S, GATED>(p)
   if (nt == 4) {
     if (enough(4, 4)) ROW_GEMM(4, 4, 4, 2);
     if (enough(4, 2)) ROW_GEMM(4, 2, 4, 2);
   } else if (nt == 3) {
     if (enough(3, 4)) ROW_GEMM(3, 4, 4, 2);
     if (enough(3, 2)) ROW_GEMM(3, 2, 4, 2);
-    if (enough(3, 1)) ROW_GEMM(3, 1, 4, 3);
+    if constexpr (!GATED)
+      if (enough(3, 1)) ROW_GEMM(3, 1, 4, 3);
   }
   if (nt >= 2) {
     if (enough(2, 4)) ROW_GEMM(2, 4, 4, 2);
     if (enough(2, 2)) ROW_GEMM(2, 2, 4, 2);
-    if (enough(2, 1)) ROW_GEMM(2, 1, 4, 3);
+    if constexpr (!GATED)
+      if (enough(2, 1)) ROW_GEMM(2, 1, 4, 3);
   }
   // few rows, or a small matrix: all of a tile's depth is on its way at once
-  if (enough(1, 2)) ROW_GEMM(1, 2, 4, 3);
-  ROW_GEMM(1, 1, 8, 2);
+  if constexpr (GATED) {
+    ROW_GEMM(1, 2, 4, 3);
+  } else {
+    if (enough(1, 2)) ROW_GEMM(1, 2, 4, 3);
+    ROW_GEMM(1, 1, 8, 2);
+  }
 #undef ROW_GEMM
+}
+
+// Rows of x start ldx numbers apart, those of out ld_out.  0: done, -2: not
+// for this kernel.
+extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
+                           const void* w, int N, int M, int K, int ldx,
+                           int kind, int up, float a, float b, void* stream) {
+  if (N <= 0 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
+      ld_out % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
+      (uintptr_t)out % (kind == CAPPED ? 16 : 8) || kind < PLAIN ||
+      kind > CAPPED)
+    return -2;
+  const RowGemm p{out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K,
+                  ldx, RowAct{kind, up, a, b}, (hipStream_t)stream};
+  return kind == SWIGLU || kind == CLAMPED ? row_gemm_pick<true>(p)
+                                           : row_gemm_pick<false>(p);
 }

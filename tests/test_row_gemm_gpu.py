@@ -52,3 +52,46 @@ def test_gradients_keep_the_library():
     w = torch.randn(32, 64, device=DEV, dtype=torch.bfloat16)
     ops.linear_decode(x, w).float().sum().backward()
     assert x.grad is not None
+
+
+def _act(act, z, up, a, b):
+    if act == "relu2":
+        return z.clamp(min=0.0).square()
+    if act == "gelu":
+        return torch.nn.functional.gelu(z, approximate="tanh")
+    if act == "capped":
+        return a * torch.tanh(z / a) if a else z
+    g, u = z[:, :up], z[:, up:]
+    if act == "swiglu":
+        return torch.nn.functional.silu(g) * u
+    g, u = g.clamp(max=a), u.clamp(-a, a)
+    return g * torch.sigmoid(b * g) * (u + 1.0)
+
+
+@pytest.mark.parametrize("act,a,b", [("relu2", 0, 0), ("gelu", 0, 0),
+                                     ("capped", 0, 0), ("capped", 3.0, 0),
+                                     ("swiglu", 0, 0), ("clamped", 1.5, 1.7)])
+@pytest.mark.parametrize("M,K", [(8, 72), (2180, 1024), (6148, 328)])
+@pytest.mark.parametrize("N", [1, 23, 40, 64, 97])
+def test_row_gemm_with_activation(N, M, K, act, a, b):
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    up = M if act in ("swiglu", "clamped") else 0
+    w = torch.randn(M + up, K, generator=g, device=DEV).mul_(
+        K ** -0.5).bfloat16()
+    z = x.double() @ w.double().T
+    ref = _act(act, z, up, a, b)
+    wide = torch.full((N, M + 16), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = None if act == "capped" else wide[:, 8:8 + M]
+    out = ops.linear_act(x, w, act, out, up, a, b)
+    # sums are K float roundings off; activations of numbers of size 1 to 30
+    # (K ** -0.5 rows) change by at most 60 times as much, and their own
+    # functions are good to 2^-20
+    off = (x.double().abs() @ w.double().abs().T).amax() * K * 2.0 ** -24
+    bound = 60 * off + ref.abs() * 2.0 ** -20
+    if act == "capped":
+        assert out.dtype == torch.float32
+    else:
+        bound = bound + ref.abs() * 2.0 ** -8
+        assert (wide[:, :8] == 7).all() and (wide[:, 8 + M:] == 7).all()
+    assert ((out.double() - ref).abs() <= bound).all()
