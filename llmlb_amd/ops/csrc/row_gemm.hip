@@ -18,9 +18,11 @@
 #include "hybrid/row_tile.h"
 
 // What becomes of a sum before it is stored: a launch less than a kernel of
-// its own, 3 us to 5 in decoding, and no rounding in between.  With two
-// matrices, gate and up, a tile's rows are half of the one and half of the
-// other, at the same outputs.
+// its own, 3 us to 5 in decoding.  The sum is rounded to bf16 first, as it
+// is where that kernel reads it (more than 128 rows): a token's numbers are
+// the same whichever way it comes.  With two matrices, gate and up, a
+// tile's rows are half of the one and half of the other, at the same
+// outputs.
 enum { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };
 struct RowAct {
   int kind;
@@ -73,10 +75,13 @@ __global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(
     if (GATED) {
       const f32x4 u = Tile::sum(lds, r, c + OUT);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = row_gate(act, v[i], u[i]);
+      for (int i = 0; i < 4; ++i)
+        v[i] = row_gate(act, to_f(from_f<bf16_t>(v[i])),
+                        to_f(from_f<bf16_t>(u[i])));
     } else if (act.kind != PLAIN) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = row_act(act, v[i]);
+      for (int i = 0; i < 4; ++i)
+        v[i] = row_act(act, to_f(from_f<bf16_t>(v[i])));
     }
     if (n0 + r >= N || m0 + c >= M) return;
     const size_t at = (size_t)(n0 + r) * ld_out + m0 + c;
