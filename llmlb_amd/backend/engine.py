@@ -4,7 +4,7 @@ One engine per GPU (one process per GPU at node scale; TP replicas span
 a process group over RCCL/xGMI).  Each ``step()``:
 
   1. admits queued prompts while KV pages are available and runs their
-     prefill BATCHED (grouped by prompt length; one SDPA + one set of
+     prefill BATCHED (grouped by prompt length; one attention + one set of
      GEMMs per group instead of per sequence),
   2. runs one decode iteration for every running sequence through the
      paged-attention kernel — decode state (block tables, lengths, last
@@ -13,9 +13,9 @@ a process group over RCCL/xGMI).  Each ``step()``:
   3. samples, streams tokens to per-request sinks, retires finished
      sequences and releases their pages.
 
-Prefill attention uses torch SDPA on the prompt's own K/V (flash path
-on ROCm); decode attention is the hand-written gfx950 paged kernel
-(llmlb_amd/ops/csrc/kernels.hip).
+Prefill attention runs on the prompt's own K/V
+(llmlb_amd/ops/csrc/flash_attention.hip), decode attention on the paged
+cache (page_attention.hip there).
 
 Optional serving features (all measured in profiles/):
   * automatic prefix caching (kv_cache.PrefixCache) — default on,
@@ -692,7 +692,7 @@ class Engine:
     def _prefill_batch(self, seqs: list[_Sequence]) -> None:
         """Batched prefill, grouped by (prompt length, cached prefix):
         same-shape groups share one packed forward (GEMMs batched, one
-        SDPA per group).  A group longer than ``prefill_chunk`` runs in
+        attention per group).  A group longer than ``prefill_chunk`` runs in
         chunks — every chunk after the first behaves exactly like a
         cached-prefix suffix (its keys are already in the paged cache),
         which bounds activation memory for long prompts and keeps
@@ -766,9 +766,9 @@ class Engine:
         Returns the final (h, residual) of the chunk's tokens."""
         dev = self.device
         Ls = L - P
-        # fp8 prefill GEMMs only on P==0 chunks: continuation chunks
-        # run the mask-path SDPA (fp32 math fallback) whose ~13 GB
-        # buffers lose 30%+ wall time with the fp8 path interleaved
+        # fp8 prefill GEMMs only on P==0 chunks: measured while
+        # continuation chunks ran masked SDPA (as head sizes other than
+        # 64 and 128 still do), whose ~13 GB buffers lose 30%+ wall time with the fp8 path interleaved
         # (profiles/r02_fp8_prefill_ab.md, same-box 8x6144 A/B)
         ops.set_prefill_fp8_ok(P == 0)
         ids = torch.tensor([s.prompt_ids[P:L] for s in group],
@@ -783,9 +783,6 @@ class Engine:
                 [sl for s in group for sl in self._slots_for(s, 0, P)],
                 dtype=torch.long, device=dev)
             pblks, poffs = pslots // BLOCK_SIZE, pslots % BLOCK_SIZE
-            # rectangular causal mask: chunk query i sees keys 0..P+i
-            mask = (torch.arange(L, device=dev)[None, :]
-                    <= torch.arange(P, L, device=dev)[:, None])
         h = self.model.embed_tokens(ids)
         residual = None
         nq, nkv, D = self.n_q_local, self.n_kv_local, \
@@ -794,7 +791,6 @@ class Engine:
             q, k, v, residual = self.model.layer_attn_prelude(
                 li, h, residual, positions)
             self._kv_append(li, k, v, slots)
-            qh = q.view(B, Ls, nq, D).transpose(1, 2)
             kh = k.view(B, Ls, nkv, D)
             vh = v.view(B, Ls, nkv, D)
             if P:
@@ -804,25 +800,8 @@ class Engine:
                                dim=1)
                 vh = torch.cat([vpre.view(B, P, nkv, D).to(vh.dtype), vh],
                                dim=1)
-            kh, vh = kh.transpose(1, 2), vh.transpose(1, 2)
-            if P:
-                # masked SDPA + enable_gqa has no fused kernel on ROCm
-                # (the head-count mismatch forces torch's fp32 math
-                # path: 35.4 ms/layer and ~13 GB of transient fp32 at
-                # the 8x6144 shape).  Repeating KV to the full head
-                # count keeps the efficient kernel: 6.1 ms/layer
-                # measured (benchmarks/gqa_mask_probe.py); the ~50 us
-                # copy is noise against the 29 ms saved.
-                G = nq // nkv
-                if G > 1:
-                    kh = kh.repeat_interleave(G, dim=1)
-                    vh = vh.repeat_interleave(G, dim=1)
-                o = torch.nn.functional.scaled_dot_product_attention(
-                    qh, kh, vh, attn_mask=mask)
-            else:
-                o = torch.nn.functional.scaled_dot_product_attention(
-                    qh, kh, vh, is_causal=Ls > 1, enable_gqa=True)
-            attn = o.transpose(1, 2).reshape(B * Ls, nq, D).contiguous()
+            attn = ops.prompt_attention(q.view(B, Ls, nq, D), kh, vh,
+                                        self.scale)
             h, residual = self.model.layer_attn_epilogue(li, attn,
                                                          residual)
         return h, residual

@@ -205,12 +205,9 @@ class LlamaForCausalLM(nn.Module):
         for li in range(self.cfg.layers):
             q, k, v, residual = self.layer_attn_prelude(
                 li, h, residual, positions)
-            qh = q.view(B, L, nq, D).transpose(1, 2)
-            kh = k.view(B, L, nkv, D).transpose(1, 2)
-            vh = v.view(B, L, nkv, D).transpose(1, 2)
-            o = torch.nn.functional.scaled_dot_product_attention(
-                qh, kh, vh, is_causal=L > 1, enable_gqa=True)
-            attn = o.transpose(1, 2).reshape(B * L, nq, D).contiguous()
+            attn = ops.prompt_attention(
+                q.view(B, L, nq, D), k.view(B, L, nkv, D),
+                v.view(B, L, nkv, D), D ** -0.5)
             h, residual = self.layer_attn_epilogue(li, attn, residual)
         final = ops.rmsnorm(h + residual if residual is not None else h,
                             self.final_norm_w, self.cfg.norm_eps, None)[0]

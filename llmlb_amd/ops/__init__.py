@@ -892,3 +892,53 @@ def paged_attn_decode(q: torch.Tensor, kcache: torch.Tensor,
         ctypes.c_float(scale), ctypes.c_int(q.stride(0)), _stream())
     _check(rc, "ll_paged_attn_decode")
     return out
+
+
+def prompt_attn_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
+                      ) -> bool:
+    """Whether ``prompt_attention`` runs flash_attention.hip: bf16 heads
+    of 64 or 128 on the GPU, rows of a wider matrix or their own."""
+    B, Lq, nq, D = q.shape
+    return (q.is_cuda and _lib is not None and q.dtype == torch.bfloat16
+            and k.dtype == v.dtype == q.dtype and D in (64, 128)
+            and nq // k.shape[2] <= 128 and k.stride() == v.stride()
+            and all(t.stride(3) == 1 and t.stride(2) == D
+                    and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
+                    and t.data_ptr() % 16 == 0 for t in (q, k, v))
+            and not (torch.is_grad_enabled()
+                     and (q.requires_grad or k.requires_grad
+                          or v.requires_grad)))
+
+
+def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                     scale: float) -> torch.Tensor:
+    """Causal attention of prompts: q [B, Lq, nq, D] asks k, v
+    [B, Lk, nkv, D], of whose Lk tokens the queries are the last Lq.
+    Returns [B * Lq, nq, D], contiguous."""
+    B, Lq, nq, D = q.shape
+    Lk, nkv = k.shape[1], k.shape[2]
+    if prompt_attn_tiled(q, k, v):
+        out = torch.empty(B * Lq, nq, D, dtype=q.dtype, device=q.device)
+        rc = _require_native().ll_prompt_attn(
+            _ptr(out), _ptr(q), _ptr(k), _ptr(v),
+            ctypes.c_longlong(q.stride(0)), ctypes.c_longlong(k.stride(0)),
+            ctypes.c_int(q.stride(1)), ctypes.c_int(k.stride(1)),
+            ctypes.c_int(B), ctypes.c_int(nq), ctypes.c_int(nkv),
+            ctypes.c_int(Lq), ctypes.c_int(Lk), ctypes.c_int(D),
+            ctypes.c_float(scale), _stream())
+        _check(rc, "ll_prompt_attn")
+        return out
+    kw = dict(is_causal=Lq > 1, enable_gqa=True)
+    if Lk > Lq:
+        # masked SDPA + enable_gqa has no fused kernel on ROCm (the
+        # head-count mismatch forces torch's fp32 math path: 35.4
+        # ms/layer and ~13 GB of transient fp32 at the 8x6144 shape);
+        # repeating KV to the full head count keeps the efficient kernel
+        G = nq // nkv
+        if G > 1:
+            k, v = (t.repeat_interleave(G, dim=2) for t in (k, v))
+        kw = dict(attn_mask=torch.arange(Lk, device=q.device)[None]
+                  <= torch.arange(Lk - Lq, Lk, device=q.device)[:, None])
+    o = torch.nn.functional.scaled_dot_product_attention(
+        *(t.transpose(1, 2) for t in (q, k, v)), scale=scale, **kw)
+    return o.transpose(1, 2).reshape(B * Lq, nq, D).contiguous()

@@ -14,6 +14,19 @@ __device__ __forceinline__ void copy_to_lds(const bf16_t* src, unsigned to) {
                ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
                : "memory");
 }
+// the same from ``at`` bytes behind one address of the wave's
+__device__ __forceinline__ void copy_to_lds(const bf16_t* base, unsigned at,
+                                            unsigned to) {
+  const unsigned long long b = (unsigned long long)base;
+  const unsigned long long wave_base =
+      (unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(b >> 32))
+          << 32 |
+      (unsigned)__builtin_amdgcn_readfirstlane((unsigned)b);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(at),
+                 "s"(wave_base)
+               : "memory");
+}
 // the same for data that nobody reads again
 __device__ __forceinline__ void stream_to_lds(const bf16_t* src,
                                               unsigned to) {
