@@ -312,11 +312,11 @@ __global__ __launch_bounds__(64) void memory_gates_kernel(
   if (lane == 0) ex[extra_row(D) - 4] = m;
 }
 
-// g = sigmoid(dec + bias)^rate per channel
+// g = sigmoid(dec + bias)^rate per channel; logs: its logarithm (of two)
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void gla_decay_kernel(
     float* __restrict__ g, const T* __restrict__ dec,
-    const float* __restrict__ bias, int n_tok, int C, float rate) {
+    const float* __restrict__ bias, int n_tok, int C, float rate, bool logs) {
   constexpr int N = VEC ? 8 : 1;
   const int c = (blockIdx.y * 256 + threadIdx.x) * N;
   if (c >= C) return;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(
     float f[N];
     load_run<N, VEC>(dec + (size_t)t * C + c, f);
 #pragma unroll
-    for (int i = 0; i < N; ++i) f[i] = decay_t<T>(-(f[i] + b[i]), rate);
+    for (int i = 0; i < N; ++i) f[i] = decay_t<T>(-(f[i] + b[i]), rate, logs);
     store_run<N, VEC>(g + (size_t)t * C + c, f);
   }
 }
@@ -378,7 +378,8 @@ __global__ __launch_bounds__(256) void ssm_conv_run_kernel(
   }
 }
 
-// steps [2][T][H]: decay and dt.  per_head [3][H]: bias, rate, skip.
+// steps [2][T][H]: decay and dt (null: not wanted).  per_head [3][H]: bias,
+// rate, skip.
 template <typename T>
 __global__ __launch_bounds__(256) void ssm_times_kernel(
     float* __restrict__ steps, const T* __restrict__ proj, int ld, int dt_off,
@@ -674,7 +675,8 @@ int hy_linear_scan(void* o, void* state, const void* in, int ld, int q_off,
 }
 
 int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
-                 float rate, int dtype, void* stream) {
+                 float rate, int logs, int dtype, void* stream) {
+  if (logs && dtype != 0) return -2;
   if (n_tok <= 0 || C <= 0) return 0;
   const bool vec = C % 8 == 0;
   const int cols = vec ? 2048 : 256;
@@ -683,7 +685,7 @@ int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                    \
       (gla_decay_kernel<T, VEC>), grid, dim3(256), 0,                    \
       (hipStream_t)stream, (float*)g, (const T*)dec, (const float*)bias, \
-      n_tok, C, rate))
+      n_tok, C, rate, logs != 0))
   if (vec) GO(true);
   else GO(false);
 #undef GO
@@ -775,6 +777,7 @@ int hy_ssm_prep(void* xbc, void* steps, const void* proj, int ld, int dt_off,
         (const int*)tstart, C, taps));
   }
   HY_CHECK();
+  if (!steps) return 0;
   HY_DTYPE(dtype, hipLaunchKernelGGL(
       ssm_times_kernel<T>, dim3((n_tok * H + 255) / 256), dim3(256), 0, st,
       (float*)steps, (const T*)proj, ld, dt_off, (const float*)per_head,

@@ -1,6 +1,7 @@
-// Matrix memory (see linear_scan.hip) of prompt portions on the matrix
-// cores, 64 tokens at a time, bf16 storage.
+// Matrix memory and Mamba-2 (see linear_scan.hip) of prompt portions on the
+// matrix cores, 64 tokens at a time, bf16 storage.
 //
+// Matrix memory.
 // With F_t the sum of the chunk's log forget gates up to token t and m_in
 // the running maximum before the chunk, m_t = max(F_t + m_in, b_t), b_t
 // being the maximum of i_s + F_t - F_s over the chunk's s <= t.  Then
@@ -11,6 +12,15 @@
 //           last token's),
 // and the normaliser is the same with v = 1: no exponent is above zero, and
 // nothing is divided by a decay.
+//
+// Mamba-2: the same without m, b and the normaliser, F_t being the sum of
+// -rate dt and i_s the logarithm of dt_s.  Its gates are not bounded as the
+// memory's are: F is kept as two floats, so that the difference of two of
+// them is as good as one float, and a step's decay is no less than 2^-160,
+// which as a float is zero all the same.
+// Scanned token by token, a head's 64 tokens wait for each other: 8 x 2048
+// tokens of 32 heads, 128 x 128 each, took 1173 us, in chunks
+// 202.
 //
 // q, k and v are bf16 as projected.  What is float, the weights of s and the
 // state, enters a product as the sum of two bf16 numbers (relative error
@@ -78,12 +88,45 @@ __global__ __launch_bounds__(1024) void memory_chunk_gates_kernel(
   }
 }
 
-// two floats as sums of bf16 numbers, hi + lo
-__device__ __forceinline__ void split2(float a, float b, unsigned& hi,
-                                       unsigned& lo) {
-  hi = to_bf16x2(a, b);
-  lo = to_bf16x2(a - __uint_as_float(hi << 16),
-                 b - __uint_as_float(hi & 0xffff0000u));
+// The same of Mamba-2: F, c = log dt - F' and F', F + F' being the sum.
+// per_head [3][H]: bias, rate, skip.
+__global__ __launch_bounds__(1024) void ssm_chunk_gates_kernel(
+    float* __restrict__ gates, const bf16_t* __restrict__ proj, int ld,
+    int dt_off, const float* __restrict__ per_head,
+    const int* __restrict__ e_start, const int* __restrict__ e_len, int n_tok,
+    int H) {
+  __shared__ float z[CHUNK][17];
+  const int e = blockIdx.y, t0 = blockIdx.x * CHUNK, h0 = blockIdx.z * 16;
+  const int len = e_len[e];
+  if (t0 >= len) return;
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
+  const size_t first = (size_t)e_start[e];
+  {
+    const int i = threadIdx.x / 16, t = t0 + i, h = threadIdx.x % 16;
+    if (h0 + h < H)
+      z[i][h] = to_f(proj[(first + (t < len ? t : len - 1)) * ld + dt_off +
+                          h0 + h]);
+  }
+  __syncthreads();
+  const int h = h0 + wave;
+  if (h >= H) return;
+  const float dt = softplus_f(z[lane][wave] + per_head[h]);
+  float f = -per_head[H + h] * dt * LOG2E;
+  f = f < -160.f ? -160.f : f;
+  double F = f;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const double f1 = __shfl_up(F, o, WAVE);
+    if (lane >= o) F += f1;
+  }
+  if (t0 + lane < len) {
+    float* to = gates + (size_t)h * n_tok + first + t0 + lane;
+    const size_t plane = (size_t)H * n_tok;
+    const float high = (float)F, low = (float)(F - high);
+    to[0] = high;
+    to[plane] = log2f(dt) - low;
+    to[2 * plane] = low;
+  }
 }
 
 // One workgroup: VB value columns of one head of one entry, chunk after
@@ -92,25 +135,28 @@ __device__ __forceinline__ void split2(float a, float b, unsigned& hi,
 // all waves the state goes through LDS.  The next chunk is in flight
 // meanwhile.
 //   o [n_tok][H V]; state [slots][H][V][D]
-template <int DQ, int VB>
+//   MEM: matrix memory, not Mamba-2.  G groups of heads share q and k.
+//   skip [H]: Mamba-2's
+template <int DQ, int VB, bool MEM>
 __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1)
 void memory_chunk_kernel(
     float* __restrict__ o, float* __restrict__ state,
     float* __restrict__ extra, const bf16_t* __restrict__ proj, int ld,
-    int k_off, int v_off, const float* __restrict__ gates,
-    const float* __restrict__ carry, const int* __restrict__ e_start,
-    const int* __restrict__ e_len, const int* __restrict__ e_pos,
-    const int* __restrict__ e_row, int n_tok, int H, int D, int V,
-    float q_scale) {
+    int q_off, int k_off, int v_off, const float* __restrict__ gates,
+    const float* __restrict__ carry, const float* __restrict__ skip_,
+    const int* __restrict__ e_start, const int* __restrict__ e_len,
+    const int* __restrict__ e_pos, const int* __restrict__ e_row, int n_tok,
+    int G, int H, int D, int V, float q_scale) {
   constexpr int KD = DQ / 32, VT = VB / 16, DT = DQ < 64 ? 1 : DQ / 64;
   constexpr int KP = DQ + 8, VP = VB + 8;       // LDS pitches
   constexpr int KL = DQ / 32, VL = VB / 32;     // pieces of a tile a thread
   __shared__ unsigned short lk[CHUNK * KP];
   __shared__ unsigned short lv[CHUNK * VP];
-  // [2][VB + 1][KP]: the columns of S and n, high and low parts
+  // [2][VB (+ 1)][KP]: the columns of S (and n), high and low parts
   extern __shared__ __attribute__((aligned(16))) unsigned short ls[];
   __shared__ __attribute__((aligned(16))) float lc[CHUNK], lw[CHUNK];
-  constexpr int LO = (VB + 1) * KP;
+  __shared__ __attribute__((aligned(16))) float lf[MEM ? 1 : CHUNK];
+  constexpr int LO = (VB + MEM) * KP;
   const int e = blockIdx.y;
   const int head = blockIdx.x % H, c0 = blockIdx.x / H * VB;
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
@@ -124,7 +170,10 @@ void memory_chunk_kernel(
   const int d0 = wave * DT * 16;      // the wave's key channels
   const bool holds = DQ >= 64 || d0 < DQ;  // 32 channels are two waves'
   float* sp = state + ((size_t)e_row[e] * H + head) * V * D;
-  const float* cr = carry + ((size_t)e * H + head) * extra_row(D);
+  const float* cr =
+      MEM ? carry + ((size_t)e * H + head) * extra_row(D) : nullptr;
+  q_off += head / (H / G) * D;
+  k_off += head / (H / G) * D;
 
   // the state: S[dt][v] holds key channels d0 + 16 dt + 4 g .. + 3 of
   // column 16 v + n, N[dt] the normaliser's
@@ -134,7 +183,7 @@ void memory_chunk_kernel(
     const int d = d0 + a * 16 + g * 4;
     const bool real = holds && d < D;
     N[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (real) {
+    if (MEM && real) {
       const float4 x = *reinterpret_cast<const float4*>(cr + d);
       N[a] = f32x4{x.x, x.y, x.z, x.w};
     }
@@ -149,7 +198,8 @@ void memory_chunk_kernel(
       }
     }
   }
-  float m = cr[extra_row(D) - 4] * LOG2E;
+  float m = MEM ? cr[extra_row(D) - 4] * LOG2E : 0.f;
+  const float skip = MEM ? 0.f : skip_[head];
 
   auto share = [&]() {  // the state for all waves' queries
     if (!holds) return;
@@ -165,7 +215,7 @@ void memory_chunk_kernel(
         *reinterpret_cast<uint2*>(to) = hi;
         *reinterpret_cast<uint2*>(to + LO) = lo;
       }
-      if (n == 0) {
+      if (MEM && n == 0) {
         uint2 hi, lo;
         split2(N[a][0], N[a][1], hi.x, lo.x);
         split2(N[a][2], N[a][3], hi.y, lo.y);
@@ -187,8 +237,7 @@ void memory_chunk_kernel(
     for (int i = 0; i < KL; ++i) {
       const int p = tid + i * 256, t = p / (DQ / 8), d = p % (DQ / 8) * 8;
       pk[i] = *reinterpret_cast<const u32x4*>(
-          at + (unsigned)((t < end ? t : end) * ld + k_off + head * D +
-                          (d < D ? d : 0)));
+          at + (unsigned)((t < end ? t : end) * ld + k_off + (d < D ? d : 0)));
     }
 #pragma unroll
     for (int i = 0; i < VL; ++i) {
@@ -202,8 +251,7 @@ void memory_chunk_kernel(
     for (int k = 0; k < KD; ++k) {
       const int d = k * 32 + g * 8;
       qn[k] = *reinterpret_cast<const u32x4*>(
-          at + (unsigned)((tq < end ? tq : end) * ld + head * D +
-                          (d < D ? d : 0)));
+          at + (unsigned)((tq < end ? tq : end) * ld + q_off + (d < D ? d : 0)));
     }
     const float* x = gate + t0 + (lane < end ? lane : end);
     gf = x[0];
@@ -231,19 +279,32 @@ void memory_chunk_kernel(
       qf[k] = k * 32 + g * 8 < D ? qn[k] : u32x4{0, 0, 0, 0};
     // past the entry's end nothing is forgotten and nothing comes in
     if (t0 + lane >= len) gc = -INFINITY;
-    const float mt = fmaxf(gf + m, gb);
-    const float f_end = __shfl(gf, 63, WAVE), m_end = __shfl(mt, 63, WAVE);
-    const float decay = __builtin_amdgcn_exp2f(f_end + m - m_end);
-    if (wave == 0) {
-      lc[lane] = gc;
-      lw[lane] = __builtin_amdgcn_exp2f(f_end + gc - m_end);
+    const float f_end = __shfl(gf, 63, WAVE);
+    const float f_q = __shfl(gf, wave * 16 + n, WAVE);  // this lane's query
+    float decay, from, least, q_exp;  // q_exp: of the query's weights
+    if constexpr (MEM) {
+      const float mt = fmaxf(gf + m, gb), m_end = __shfl(mt, 63, WAVE);
+      const float m_q = __shfl(mt, wave * 16 + n, WAVE);
+      decay = __builtin_amdgcn_exp2f(f_end + m - m_end);
+      if (wave == 0) {
+        lc[lane] = gc;
+        lw[lane] = __builtin_amdgcn_exp2f(f_end + gc - m_end);
+      }
+      from = __builtin_amdgcn_exp2f(f_q + m - m_q);
+      least = __builtin_amdgcn_exp2f(-m_q);
+      q_exp = f_q - m_q;
+      m = m_end;
+    } else {
+      const float low_end = __shfl(gb, 63, WAVE);
+      q_exp = __shfl(gb, wave * 16 + n, WAVE);
+      decay = __builtin_amdgcn_exp2f(f_end);
+      from = __builtin_amdgcn_exp2f(f_q);
+      if (wave == 0) {
+        lc[lane] = gc;
+        lf[lane] = gf;
+        lw[lane] = __builtin_amdgcn_exp2f(f_end - gf + (low_end + gc));
+      }
     }
-    // of this lane's query
-    const float f_q = __shfl(gf, wave * 16 + n, WAVE);
-    const float m_q = __shfl(mt, wave * 16 + n, WAVE);
-    const float from = __builtin_amdgcn_exp2f(f_q + m - m_q);
-    const float least = __builtin_amdgcn_exp2f(-m_q);
-    m = m_end;
     __syncthreads();
     if (t0 + CHUNK < len) fetch(t0 + CHUNK);
 
@@ -264,13 +325,20 @@ void memory_chunk_kernel(
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const float4 c = *reinterpret_cast<const float4*>(&lc[t * 16 + g * 4]);
-      const float cs[4] = {c.x, c.y, c.z, c.w};
+      float cs[4] = {c.x, c.y, c.z, c.w};
+      if constexpr (!MEM) {
+        const float4 x = *reinterpret_cast<const float4*>(&lf[t * 16 + g * 4]);
+        cs[0] += f_q - x.x;
+        cs[1] += f_q - x.y;
+        cs[2] += f_q - x.z;
+        cs[3] += f_q - x.w;
+      }
       const int age = (wave - t) * 16 + n - g * 4;  // of key (t, 0)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float w = s[t][i] * __builtin_amdgcn_exp2f(f_q - m_q + cs[i]);
+        const float w = s[t][i] * __builtin_amdgcn_exp2f(q_exp + cs[i]);
         s[t][i] = age >= i ? w : 0.f;
-        den += s[t][i];
+        if (MEM) den += s[t][i];
       }
       unsigned h0, h1, l0, l1;
       split2(s[t][0], s[t][1], h0, l0);
@@ -280,8 +348,10 @@ void memory_chunk_kernel(
       lo[t / 2][t % 2 * 2] = l0;
       lo[t / 2][t % 2 * 2 + 1] = l1;
     }
-    den += __shfl_xor(den, 16, WAVE);
-    den += __shfl_xor(den, 32, WAVE);
+    if (MEM) {
+      den += __shfl_xor(den, 16, WAVE);
+      den += __shfl_xor(den, 32, WAVE);
+    }
 
     // what the state before the chunk gives
     f32x4 acc[VT], nq = {0.f, 0.f, 0.f, 0.f};
@@ -296,15 +366,17 @@ void memory_chunk_kernel(
         acc[v] = mfma(*reinterpret_cast<const u32x4*>(x), qf[k], acc[v]);
         acc[v] = mfma(*reinterpret_cast<const u32x4*>(x + LO), qf[k], acc[v]);
       }
-      const unsigned short* x = r + VB * KP;  // the same for every row
-      nq = mfma(*reinterpret_cast<const u32x4*>(x), qf[k], nq);
-      nq = mfma(*reinterpret_cast<const u32x4*>(x + LO), qf[k], nq);
+      if constexpr (MEM) {
+        const unsigned short* x = r + VB * KP;  // the same for every row
+        nq = mfma(*reinterpret_cast<const u32x4*>(x), qf[k], nq);
+        nq = mfma(*reinterpret_cast<const u32x4*>(x + LO), qf[k], nq);
+      }
     }
 #pragma unroll
     for (int v = 0; v < VT; ++v) acc[v] *= from;
 #pragma unroll
     for (int a = 0; a < DT; ++a) {
-      N[a] *= decay;
+      if (MEM) N[a] *= decay;
 #pragma unroll
       for (int v = 0; v < VT; ++v) S[a][v] *= decay;
     }
@@ -348,16 +420,31 @@ void memory_chunk_kernel(
             S[a][v] = mfma(kh, vf[v], S[a][v]);
             S[a][v] = mfma(kl, vf[v], S[a][v]);
           }
-          N[a] = mfma(kh, one, N[a]);
-          N[a] = mfma(kl, one, N[a]);
+          if constexpr (MEM) {
+            N[a] = mfma(kh, one, N[a]);
+            N[a] = mfma(kl, one, N[a]);
+          }
         }
       }
     }
 
     const int t = t0 + wave * 16 + n;
     if (t < len) {
-      den = fabsf((den + nq[0] * from) * q_scale);
-      const float f = q_scale / (fmaxf(den, least) + MEMORY_EPS);
+      float f = 1.f;
+      if constexpr (MEM) {
+        den = fabsf((den + nq[0] * from) * q_scale);
+        f = q_scale / (fmaxf(den, least) + MEMORY_EPS);
+      } else {  // the token's own values
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+          const uint2 x = *reinterpret_cast<const uint2*>(
+              &lv[(wave * 16 + n) * VP + v * 16 + g * 4]);
+          acc[v][0] += skip * __uint_as_float(x.x << 16);
+          acc[v][1] += skip * __uint_as_float(x.x & 0xffff0000u);
+          acc[v][2] += skip * __uint_as_float(x.y << 16);
+          acc[v][3] += skip * __uint_as_float(x.y & 0xffff0000u);
+        }
+      }
       float* dst = o + ((first + t) * H + head) * V + c0;
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
@@ -373,7 +460,8 @@ void memory_chunk_kernel(
   }
 
   if (!holds) return;
-  float* ex = extra + ((size_t)e_row[e] * H + head) * extra_row(D);
+  float* ex =
+      MEM ? extra + ((size_t)e_row[e] * H + head) * extra_row(D) : nullptr;
 #pragma unroll
   for (int a = 0; a < DT; ++a) {
     const int d = d0 + a * 16 + g * 4;
@@ -385,11 +473,53 @@ void memory_chunk_kernel(
         *reinterpret_cast<float4*>(sp + (size_t)col * D + d) = make_float4(
             S[a][v][0], S[a][v][1], S[a][v][2], S[a][v][3]);
     }
-    if (c0 == 0 && n == 0)
+    if (MEM && c0 == 0 && n == 0)
       *reinterpret_cast<float4*>(ex + d) =
           make_float4(N[a][0], N[a][1], N[a][2], N[a][3]);
   }
-  if (c0 == 0 && tid == 0) ex[extra_row(D) - 4] = m / LOG2E;
+  if (MEM && c0 == 0 && tid == 0) ex[extra_row(D) - 4] = m / LOG2E;
+}
+
+// the columns of a workgroup and the launch, for both
+template <bool MEM>
+static int launch_chunks(void* o, void* state, void* extra, const void* in,
+                         int ld, int q_off, int k_off, int v_off,
+                         const void* gates, const void* carry,
+                         const void* skip, const void* e_start,
+                         const void* e_len, const void* e_pos,
+                         const void* e_row, int n_entries, int n_tok, int G,
+                         int H, int D, int V, float q_scale, hipStream_t s) {
+#define GO(DQ, VB)                                                           \
+  do {                                                                       \
+    constexpr int lds = 2 * (VB + MEM) * (DQ + 8) * 2;                       \
+    static const hipError_t ready = hipFuncSetAttribute(                     \
+        reinterpret_cast<const void*>(memory_chunk_kernel<DQ, VB, MEM>),     \
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \
+    if (ready != hipSuccess) return -3;                                      \
+    hipLaunchKernelGGL((memory_chunk_kernel<DQ, VB, MEM>),                   \
+                       dim3(H * ((V + VB - 1) / VB), n_entries), dim3(256),  \
+                       lds, s, (float*)o, (float*)state, (float*)extra,      \
+                       (const bf16_t*)in, ld, q_off, k_off, v_off,           \
+                       (const float*)gates, (const float*)carry,             \
+                       (const float*)skip, (const int*)e_start,              \
+                       (const int*)e_len, (const int*)e_pos,                 \
+                       (const int*)e_row, n_tok, G, H, D, V, q_scale);       \
+  } while (0)
+#define PICK(DQ)                \
+  do {                          \
+    if (wide) GO(DQ, 64);       \
+    else GO(DQ, 32);            \
+  } while (0)
+  // 64 columns a workgroup where that still fills the chip
+  const bool wide = (long long)n_entries * H * ((V + 63) / 64) >= 256;
+  if (D <= 32) PICK(32);
+  else if (D <= 64) PICK(64);
+  else if (D <= 128) PICK(128);
+  else PICK(256);
+#undef PICK
+#undef GO
+  HY_CHECK();
+  return 0;
 }
 
 extern "C" {
@@ -414,37 +544,36 @@ int hy_memory_chunk(void* o, void* gates, void* carry, void* state,
       (const int*)e_start, (const int*)e_len, (const int*)e_pos,
       (const int*)e_row, n_tok, H, D, cap);
   HY_CHECK();
-#define GO(DQ, VB)                                                           \
-  do {                                                                       \
-    constexpr int lds = 2 * (VB + 1) * (DQ + 8) * 2;                         \
-    static const hipError_t ready = hipFuncSetAttribute(                     \
-        reinterpret_cast<const void*>(memory_chunk_kernel<DQ, VB>),          \
-        hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \
-    if (ready != hipSuccess) return -3;                                      \
-    hipLaunchKernelGGL((memory_chunk_kernel<DQ, VB>),                        \
-                       dim3(H * ((V + VB - 1) / VB), n_entries), dim3(256),  \
-                       lds, s, (float*)o, (float*)state, (float*)extra,      \
-                       (const bf16_t*)proj, ld, k_off, v_off,                \
-                       (const float*)gates, (const float*)carry,             \
-                       (const int*)e_start, (const int*)e_len,               \
-                       (const int*)e_pos, (const int*)e_row, n_tok, H, D, V, \
-                       q_scale);                                             \
-  } while (0)
-#define PICK(DQ)                \
-  do {                          \
-    if (wide) GO(DQ, 64);       \
-    else GO(DQ, 32);            \
-  } while (0)
-  // 64 columns a workgroup where that still fills the chip
-  const bool wide = (long long)n_entries * H * ((V + 63) / 64) >= 256;
-  if (D <= 32) PICK(32);
-  else if (D <= 64) PICK(64);
-  else if (D <= 128) PICK(128);
-  else PICK(256);
-#undef PICK
-#undef GO
+  return launch_chunks<true>(o, state, extra, proj, ld, 0, k_off, v_off,
+                             gates, carry, nullptr, e_start, e_len, e_pos,
+                             e_row, n_entries, n_tok, H, H, D, V, q_scale, s);
+}
+
+// in [n_tok][ld]: the convolved x, k and q; dt's projection and per_head as
+// for hy_ssm_prep; gates [3][H][n_tok] of scratch
+int hy_ssm_chunk(void* o, void* gates, void* state, const void* in, int ld,
+                 int q_off, int k_off, const void* proj, int ld_proj,
+                 int dt_off, const void* per_head, const void* e_start,
+                 const void* e_len, const void* e_pos, const void* e_row,
+                 int n_entries, int max_len, int n_tok, int G, int H, int D,
+                 int V, void* stream) {
+  if (G <= 0 || H <= 0 || H % G || D <= 0 || V <= 0 || D % 8 || V % 8 ||
+      D > 256 || V > 4096 || ld % 8 || q_off % 8 || k_off % 8 ||
+      n_entries > 65535)
+    return -2;
+  if (n_entries <= 0 || n_tok <= 0) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(
+      ssm_chunk_gates_kernel,
+      dim3((max_len + CHUNK - 1) / CHUNK, n_entries, (H + 15) / 16),
+      dim3(1024), 0, s, (float*)gates, (const bf16_t*)proj, ld_proj, dt_off,
+      (const float*)per_head, (const int*)e_start, (const int*)e_len, n_tok,
+      H);
   HY_CHECK();
-  return 0;
+  return launch_chunks<false>(o, state, nullptr, in, ld, q_off, k_off, 0,
+                              gates, nullptr, (const float*)per_head + 2 * H,
+                              e_start, e_len, e_pos, e_row, n_entries, n_tok,
+                              G, H, D, V, 1.f, s);
 }
 
 }  // extern "C"

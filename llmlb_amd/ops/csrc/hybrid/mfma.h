@@ -34,4 +34,12 @@ __device__ __forceinline__ unsigned to_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
 }
 
+// two floats as sums of bf16 numbers, hi + lo
+__device__ __forceinline__ void split2(float a, float b, unsigned& hi,
+                                       unsigned& lo) {
+  hi = to_bf16x2(a, b);
+  lo = to_bf16x2(a - __uint_as_float(hi << 16),
+                 b - __uint_as_float(hi & 0xffff0000u));
+}
+
 #define LOG2E 1.4426950408889634f

@@ -327,6 +327,27 @@ def latent_flash(out, proj, heads, dim, rot, w_uk, w_uv, cache, b, window,
         _i(-1 if g_off is None else g_off), st), "hy_latent_flash")
 
 
+def _runs(b):
+    return (_ptr(b.e_start), _ptr(b.e_len), _ptr(b.e_pos), _ptr(b.e_row),
+            _i(len(b.entries)))
+
+
+def by_chunks(b) -> bool:
+    """Whether recurrences of the batch go by chunks of tokens on the
+    matrix cores (bf16 models): a chunk costs about what a dozen tokens
+    cost one by one.  32 heads of 128 x 128, us, gated linear attention:
+    64 portions of 1 token 63 (one by one 45), of 4 66 (55), of 16 71
+    (90), 8 portions of 2048 395 (1025); Mamba-2: 76 (44), 75 (51), 78
+    (87) and 215 (1119)."""
+    longest = max((n for _, n, _, _ in b.entries), default=0)
+    return longest >= 64 or b.n_tok >= 12 * len(b.entries)
+
+
+def can_chunk_scan(dtype, dim) -> bool:
+    """Sizes that chunk_scan.hip takes."""
+    return dtype == torch.bfloat16 and dim % 8 == 0 and dim <= 128
+
+
 # -- gated delta rule ------------------------------------------------------
 
 def gated_delta(proj, b_off, dec, gate, state, ring, b, wconv, a_log,
@@ -359,15 +380,23 @@ def gated_delta(proj, b_off, dec, gate, state, ring, b, wconv, a_log,
     ws = torch.empty(T, int(lib.hy_delta_ws_floats(*sizes)),
                      dtype=torch.float32, device=proj.device)
     o = torch.empty(T, H * V, dtype=torch.float32, device=proj.device)
+    chunks = by_chunks(b) and taps <= 4 and can_chunk_scan(proj.dtype, D)
     _check(lib.hy_delta_prep(
         _ptr(ws), _ptr(proj), ld, _i(b_off), _ptr(dec), _ptr(ring),
         _ptr(wconv), _ptr(a_log), _ptr(dt_bias), _ptr(b.pos), _ptr(b.row),
-        _ptr(b.tstart), _i(T), *sizes, _i(taps), q_scale, dt, st),
-        "hy_delta_prep")
-    _check(lib.hy_delta_scan(
-        _ptr(o), _ptr(state), _ptr(ws), _ptr(b.e_start), _ptr(b.e_len),
-        _ptr(b.e_pos), _ptr(b.e_row), _i(len(b.entries)), *sizes, st),
-        "hy_delta_scan")
+        _ptr(b.tstart), _i(T), *sizes, _i(taps), q_scale, _i(chunks), dt,
+        st), "hy_delta_prep")
+    if chunks:
+        g, v, size = 2 * KH * D, 2 * KH * D + H * D, ws.shape[1]
+        beta = v + H * V + KH
+        _check(lib.hy_chunk_scan(
+            _ptr(o), _ptr(state), _ptr(ws), _i(size), _i(0), _i(KH * D),
+            _i(v), _ptr(ws[:, g:]), _i(size), _ptr(ws[:, beta:]), *_runs(b),
+            *sizes, _f(1.0), _i(1), st), "hy_chunk_scan")
+    else:
+        _check(lib.hy_delta_scan(
+            _ptr(o), _ptr(state), _ptr(ws), *_runs(b), *sizes, st),
+            "hy_delta_scan")
     _check(lib.hy_delta_out(
         _ptr(out), _ptr(o), _ptr(gate), _ptr(w_norm), _f(eps), _ptr(proj),
         ld, _ptr(ring), _ptr(b.pos), _ptr(b.row), _ptr(b.tend), _i(T),
@@ -485,14 +514,22 @@ def gated_linear(out, proj, k_off, v_off, g_off, dec, dec_bias, state, b,
         return
     g = torch.empty(T, H * D, dtype=torch.float32, device=proj.device)
     o = torch.empty(T, H * V, dtype=torch.float32, device=proj.device)
+    chunks = by_chunks(b) and can_chunk_scan(proj.dtype, D) \
+        and proj.stride(0) % 8 == 0 and k_off % 8 == 0 \
+        and proj.data_ptr() % 16 == 0
     _check(lib.hy_gla_decay(
-        _ptr(g), _ptr(dec), _ptr(dec_bias), _i(T), _i(H * D), rate, dt, st),
-        "hy_gla_decay")
-    _check(lib.hy_linear_scan(
-        _ptr(o), _ptr(state), _ptr(proj), ld, _i(0), _i(k_off), _i(v_off),
-        _ptr(g), None, None, _ptr(b.e_start), _ptr(b.e_len), _ptr(b.e_pos),
-        _ptr(b.e_row), _i(len(b.entries)), _i(H), _i(H), _i(D), _i(V),
-        q_scale, None, None, dt, st), "hy_linear_scan")
+        _ptr(g), _ptr(dec), _ptr(dec_bias), _i(T), _i(H * D), rate,
+        _i(chunks), dt, st), "hy_gla_decay")
+    if chunks:
+        _check(lib.hy_chunk_scan(
+            _ptr(o), _ptr(state), _ptr(proj), ld, _i(0), _i(k_off),
+            _i(v_off), _ptr(g), _i(H * D), None, *_runs(b), _i(H), _i(H),
+            _i(D), _i(V), q_scale, _i(0), st), "hy_chunk_scan")
+    else:
+        _check(lib.hy_linear_scan(
+            _ptr(o), _ptr(state), _ptr(proj), ld, _i(0), _i(k_off),
+            _i(v_off), _ptr(g), None, None, *_runs(b), _i(H), _i(H), _i(D),
+            _i(V), q_scale, None, None, dt, st), "hy_linear_scan")
     _gated_norm(out, o, proj, g_off, w_norm, H, False, eps)
 
 
@@ -522,22 +559,30 @@ def state_space(out, proj, z_off, dt_off, state, ring, b, wconv, bconv,
             _i(taps), dt, st), "hy_ssm_step")
     else:
         xbc = torch.empty(T, C, dtype=proj.dtype, device=proj.device)
-        steps = torch.empty(2, T, H, dtype=torch.float32,
+        chunks = by_chunks(b) and can_memory_mfma(proj.dtype, N, V)
+        steps = torch.empty(3 if chunks else 2, T, H, dtype=torch.float32,
                             device=proj.device)
         _check(lib.hy_ssm_prep(
-            _ptr(xbc), _ptr(steps), _ptr(proj), ld, _i(dt_off), *conv,
-            _ptr(b.pos), _ptr(b.row), _ptr(b.tstart), _i(T), _i(C), _i(H),
-            _i(taps), dt, st), "hy_ssm_prep")
+            _ptr(xbc), None if chunks else _ptr(steps), _ptr(proj), ld,
+            _i(dt_off), *conv, _ptr(b.pos), _ptr(b.row), _ptr(b.tstart),
+            _i(T), _i(C), _i(H), _i(taps), dt, st), "hy_ssm_prep")
+        runs = _runs(b)
         _check(lib.hy_ring_store(
-            _ptr(ring), _ptr(proj), ld, _ptr(b.e_start), _ptr(b.e_len),
-            _ptr(b.e_pos), _ptr(b.e_row), _i(len(b.entries)), _i(C),
+            _ptr(ring), _ptr(proj), ld, *runs[:4], _i(len(b.entries)), _i(C),
             _i(taps), dt, st), "hy_ring_store")
-        _check(lib.hy_linear_scan(
-            _ptr(o), _ptr(state), _ptr(xbc), _i(C), _i(H * V + G * N),
-            _i(H * V), _i(0), _ptr(steps[0]), _ptr(steps[1]),
-            _ptr(per_head[2]), _ptr(b.e_start), _ptr(b.e_len),
-            _ptr(b.e_pos), _ptr(b.e_row), _i(len(b.entries)), _i(G), _i(H),
-            _i(N), _i(V), _f(1.0), None, None, dt, st), "hy_linear_scan")
+        if chunks:
+            _check(lib.hy_ssm_chunk(
+                _ptr(o), _ptr(steps), _ptr(state), _ptr(xbc), _i(C),
+                _i(H * V + G * N), _i(H * V), _ptr(proj), ld, _i(dt_off),
+                _ptr(per_head), *runs,
+                _i(max(n for _, n, _, _ in b.entries)), _i(T), _i(G), _i(H),
+                _i(N), _i(V), st), "hy_ssm_chunk")
+        else:
+            _check(lib.hy_linear_scan(
+                _ptr(o), _ptr(state), _ptr(xbc), _i(C), _i(H * V + G * N),
+                _i(H * V), _i(0), _ptr(steps[0]), _ptr(steps[1]),
+                _ptr(per_head[2]), *runs, _i(G), _i(H), _i(N), _i(V),
+                _f(1.0), None, None, dt, st), "hy_linear_scan")
     _gated_norm(out, o, proj, z_off, w_norm, norm_groups, True, eps)
 
 
@@ -585,8 +630,7 @@ def matrix_memory(out, proj, k_off, v_off, g_off, i_off, gate_bias, cap,
     f32 = dict(dtype=torch.float32, device=proj.device)
     steps = torch.empty(3, T, H, **f32)
     o = torch.empty(T, H * V, **f32)
-    runs = (_ptr(b.e_start), _ptr(b.e_len), _ptr(b.e_pos), _ptr(b.e_row),
-            _i(E))
+    runs = _runs(b)
     if can_memory_mfma(proj.dtype, D, V) and proj.stride(0) % 8 == 0 \
             and k_off % 8 == 0 and v_off % 8 == 0:
         carry = torch.empty(E, H, memory_extra(D), **f32)
