@@ -32,6 +32,7 @@ HybridCache whose state slots are the decode rows.
 """
 from __future__ import annotations
 
+import array
 import contextlib
 import gc
 import logging
@@ -50,7 +51,7 @@ from .. import ops
 from ..models.llama import LlamaConfig
 from ..models.registry import model_class
 from .kv_cache import BLOCK_SIZE, HybridCache, KVCache, PrefixCache
-from .ragged import RaggedBatch
+from .ragged import RaggedBatch, staged, to_device
 from .sampler import SamplingParams, sample
 
 
@@ -248,6 +249,17 @@ class _DecodeGraph:
         return self.logits[:n]
 
 
+def _token_array(toks) -> np.ndarray:
+    """Token ids as int64.  (numpy looks at every element of a list for its
+    type first: 391 us for 16384 ids, 263 this way.)"""
+    if type(toks) is list:
+        try:
+            return np.array(array.array("q", toks))
+        except (TypeError, OverflowError):
+            pass
+    return np.asarray(toks, dtype=np.int64)
+
+
 class _RaggedGraph:
     """A hipGraph of one decode forward of a ``ragged`` model at a padded
     batch size.  A step fills one int buffer and replays.  Padded rows
@@ -265,7 +277,8 @@ class _RaggedGraph:
     def _fill(self, runs) -> None:
         runs = runs + [(self._engine.max_rows, 0, [0])] \
             * (self.S - len(runs))
-        self.flat.copy_(torch.from_numpy(RaggedBatch.pack(runs)))
+        self.flat.copy_(staged(RaggedBatch.pack(runs), self.flat.device),
+                        non_blocking=True)
         if self.batch is None:
             eng = self._engine
             self.batch = RaggedBatch.over(
@@ -967,12 +980,15 @@ class Engine:
 
     def _write_tables(self, new) -> None:
         """Append page lists to sequences and to the device table."""
-        cells = []
+        rows, cols, vals = [], [], []
         for seq, blocks in new:
             at = len(seq.block_table)
             seq.block_table = seq.block_table + blocks
-            cells += [(seq.row, at + i, blk) for i, blk in enumerate(blocks)]
-        rows, cols, vals = torch.tensor(cells, device=self.device).unbind(1)
+            rows += [seq.row] * len(blocks)
+            cols += range(at, at + len(blocks))
+            vals += blocks
+        rows, cols, vals = to_device([rows, cols, vals], self.device,
+                                     np.int64)
         self._bt_dev[rows, cols] = vals.to(torch.int32)
 
     @torch.inference_mode()
@@ -986,7 +1002,7 @@ class Engine:
         vocab = self.cfg.model.vocab
         cap = min(self.cfg.model.max_pos,
                   self.max_blocks_per_seq * BLOCK_SIZE)
-        work = [(seq, np.asarray(toks, dtype=np.int64), want)
+        work = [(seq, _token_array(toks), want)
                 for seq, toks, want in work]
         for seq, toks, want in work:
             if not len(toks) or toks.min() < 0 or toks.max() >= vocab:
@@ -1013,13 +1029,12 @@ class Engine:
         if graph is not None:
             logits = graph.run(runs)
             if index != list(range(len(runs))):
-                logits = logits[torch.tensor(index, dtype=torch.long,
-                                             device=self.device)]
+                logits = logits[to_device(index, self.device, np.int64)]
         else:
-            x = self.model.forward(RaggedBatch.build(runs, self._bt_dev),
-                                   self.kv)
-            logits = self.model.logits(x, torch.tensor(
-                index, dtype=torch.int32, device=self.device)) \
+            batch = RaggedBatch.build(runs, self._bt_dev)
+            wanted = to_device(index, self.device)
+            x = self.model.forward(batch, self.kv)
+            logits = self.model.logits(x, wanted) \
                 if index else torch.empty(0, vocab, device=self.device)
         for seq, toks, _ in work:
             seq.length += len(toks)

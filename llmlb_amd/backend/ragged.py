@@ -19,6 +19,24 @@ import torch
 SHORT_ENTRY = 8
 
 
+def staged(numbers, device, dtype=np.int32) -> torch.Tensor:
+    """Integers in host memory that a copy to ``device`` need not wait
+    for.  A copy from pageable memory waits for all the stream has to do
+    before, and the GPU then for the host: a step of 24 tokens and three
+    prompts took 2.56 ms with six such copies for 2.05 ms of kernels,
+    2.18 now.  Pinned memory comes from torch's pool, which keeps the
+    block until the copy is done."""
+    a = np.asarray(numbers, dtype=dtype)
+    out = torch.empty(a.shape, dtype=torch.from_numpy(np.empty(0, dtype)).dtype,
+                      pin_memory=torch.device(device).type == "cuda")
+    out.numpy()[...] = a
+    return out
+
+
+def to_device(numbers, device, dtype=np.int32) -> torch.Tensor:
+    return staged(numbers, device, dtype).to(device, non_blocking=True)
+
+
 @dataclass
 class RaggedBatch:
     ids: torch.Tensor        # [T] token ids (all int32)
@@ -60,8 +78,7 @@ class RaggedBatch:
                 # last queries first: they see the most keys
                 for q in reversed(range(0, n, 128)):
                     items += (start + q, pos + q, min(128, n - q), at, first)
-            flat = torch.tensor(blocks + items, dtype=torch.int32,
-                                device=self.pos.device)
+            flat = to_device(blocks + items, self.pos.device)
             plan = (flat[:len(blocks)], flat[len(blocks):],
                     len(blocks) // 3, len(items) // 5)
             self.plans[window] = plan
@@ -74,14 +91,16 @@ class RaggedBatch:
         first."""
         plan = self.plans.get(("tiles", size))
         if plan is None:
-            items = []
+            tiles = []
             for start, n, pos, row in self.entries:
                 if n > SHORT_ENTRY:
-                    items += [(start + q, pos + q, min(size, n - q), row)
-                              for q in range(0, n, size)]
-            items.sort(key=lambda it: -it[1])
-            plan = (torch.tensor(items, dtype=torch.int32,
-                                 device=self.pos.device), len(items))
+                    q = np.arange(0, n, size)
+                    tiles.append(np.stack(
+                        [start + q, pos + q, np.minimum(size, n - q),
+                         np.full_like(q, row)], 1))
+            items = np.concatenate(tiles) if tiles else np.empty((0, 4))
+            items = items[np.argsort(-items[:, 1], kind="stable")]
+            plan = to_device(items, self.pos.device), len(items)
             self.plans["tiles", size] = plan
         return plan
 
@@ -126,6 +145,5 @@ class RaggedBatch:
 
     @classmethod
     def build(cls, runs, block_tables) -> "RaggedBatch":
-        dev = block_tables.device
-        flat = torch.from_numpy(cls.pack(runs)).to(dev)
+        flat = to_device(cls.pack(runs), block_tables.device)
         return cls.over(flat, runs, block_tables)
