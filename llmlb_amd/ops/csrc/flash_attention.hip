@@ -59,11 +59,13 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttn a,
   const int w_hi = before + (wave * 32 + 31) / R;
   f.template run<true>(
       lds,
-      [&](int j) {
-        const size_t at = (size_t)j * a.ldk;
-        return KeyRows{k0 + at, v0 + at};
-      },
-      a.ldk, 0, last, pos, span, w_lo, w_hi, 0, 0, a.scale);
+      paged_rows<D>(
+          [&](int j) {
+            const size_t at = (size_t)j * a.ldk;
+            return KeyRows{k0 + at, v0 + at};
+          },
+          a.ldk, last),
+      0, last, pos, span, w_lo, w_hi, 0, 0, a.scale);
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     if (wave * 32 + s * 16 + n >= n_rows) continue;

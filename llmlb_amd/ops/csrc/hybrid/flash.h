@@ -1,14 +1,15 @@
 // The loop of prompt attention that its kernels share: 128 rows a workgroup
 // of four waves, 32 a wave, a row being one head of one query; keys and
-// values of one head in tiles of 64, D numbers each, bf16.
+// values of one head in tiles of 64, bf16.
 //
 // S^T = K Q^T with 16x16x32 MFMAs: a lane holds, for ONE row n = lane % 16
 // of each of its two sets, the scores of keys 4g .. 4g + 3 of each 16-key
 // tile (g = lane / 16), so that sums and maxima are its own, and P^T is
 // already the operand of O^T = V^T P^T.
 //
-// The matrix cores need 1024 cycles for a wave's tile and LDS as many for
-// the two waves of a SIMD, so what costs is all that comes on top.
+// With 128 numbers a key the matrix cores need 1024 cycles for a wave's tile
+// and LDS as many for the two waves of a SIMD, so what costs is all that
+// comes on top.
 //  * Tiles are copied to LDS by the memory path itself, one ahead, with one
 //    barrier a tile; V is read transposed.
 //  * A row's first tile with keys sets what its scores are taken relative
@@ -24,93 +25,130 @@
 #include "lds_copy.h"
 #include "mfma.h"
 
+// A tile's 64 rows of D numbers in LDS.
+template <int D>
+struct TileRows {
+  static_assert(D == 64 || D == 96 || D == 128 || D == 192,
+                "what turn() knows, in whole copies");
+  static constexpr int ROW = 2 * D, PR = ROW / 16;  // bytes, pieces of 16
+  static constexpr int BYTES = 64 * ROW;
+  static constexpr int COPIES = 16 * PR / 64;  // of a wave, its 16 rows
+
+  // Piece c of row r lies at c ^ turn(r): lanes reading one piece of 16
+  // rows meet every bank once.
+  static __device__ __forceinline__ int turn(int r) {
+    return D == 128 ? r & 15 : D == 96 ? (r >> 2) & 3 : (r >> 1) & 7;
+  }
+  // row among the wave's 16 and its piece that a lane copies in copy c
+  static __device__ __forceinline__ int row(int c, int lane) {
+    return (c * 64 + lane) / PR;
+  }
+  static __device__ __forceinline__ int piece(int c, int lane) {
+    return (c * 64 + lane) % PR ^ turn(row(c, lane));
+  }
+};
+
 // where 16 neighbouring rows of keys and values begin
 struct KeyRows {
   const bf16_t *k, *v;
 };
 
-template <int D>
+// Rows of as many numbers for keys and values, ld apart among 16
+// neighbours.  find(j): KeyRows of keys j .. j + 15, j a multiple of 16.
+template <int D, class Find>
+struct PagedRows {
+  using Tile = TileRows<D>;
+  Find find;
+  int ld, last, lane;
+  unsigned off[Tile::COPIES];
+
+  __device__ __forceinline__ PagedRows(Find f, int ld_, int last_)
+      : find(f), ld(ld_), last(last_), lane(threadIdx.x & 63) {
+#pragma unroll
+    for (int c = 0; c < Tile::COPIES; ++c) off[c] = place(c, 15);
+  }
+  __device__ __forceinline__ unsigned place(int c, int most) {
+    const int r = Tile::row(c, lane);
+    return (unsigned)((r < most ? r : most) * ld + Tile::piece(c, lane) * 8) *
+           2;
+  }
+  // the wave's rows, from key j on; looked up a tile before they are copied
+  __device__ __forceinline__ KeyRows look_up(int j) {
+    return find((j < last ? j : last) & ~15);
+  }
+  __device__ __forceinline__ void copy(const KeyRows& s, int j, unsigned k_to,
+                                       unsigned v_to) {
+    if (j + 15 <= last) {
+#pragma unroll
+      for (int c = 0; c < Tile::COPIES; ++c) {
+        copy_to_lds(s.k, off[c], k_to + c * 1024);
+        copy_to_lds(s.v, off[c], v_to + c * 1024);
+      }
+    } else {
+      // rows past the last one repeat it: their weights are zero, and
+      // what they are multiplied with has to be a number
+#pragma unroll
+      for (int c = 0; c < Tile::COPIES; ++c) {
+        const unsigned from = place(c, last & 15);
+        copy_to_lds(s.k, from, k_to + c * 1024);
+        copy_to_lds(s.v, from, v_to + c * 1024);
+      }
+    }
+  }
+};
+template <int D, class Find>
+__device__ __forceinline__ PagedRows<D, Find> paged_rows(Find f, int ld,
+                                                         int last) {
+  return PagedRows<D, Find>(f, ld, last);
+}
+
+// keys of DK numbers, values of DV
+template <int DK, int DV = DK>
 struct Flash {
-  static_assert(D == 64 || D == 128, "whole rows of a copy");
-  static constexpr int KD = D / 32, VT = D / 16;
-  static constexpr int ROW = 2 * D, PR = ROW / 16;  // bytes, pieces of 16
-  static constexpr int RC = 64 / PR;                // rows of a copy
-  static constexpr int HALF = 64 * ROW, TILE = 2 * HALF;
-  static constexpr int LDS = 2 * TILE;
+  using K = TileRows<DK>;
+  using V = TileRows<DV>;
+  static constexpr int KD = DK / 32, VT = DV / 16;
+  static constexpr int TILE = K::BYTES + V::BYTES, LDS = 2 * TILE;
 
   u32x4 qf[2][KD];
   f32x4 o[2][VT];
   float l[2];
 
-  // Piece c of row r lies at c ^ turn(r): lanes reading one piece of 16
-  // rows meet every bank once.
-  static __device__ __forceinline__ int turn(int r) {
-    return D == 128 ? r & 15 : (r >> 1) & 7;
-  }
-
   // Attention of the rows over keys lo .. last (lo a multiple of 16).
-  //   rows(j): KeyRows of keys j .. j + 15, ld numbers apart, j a multiple
-  //     of 16
+  //   rows: what brings a tile's rows, by wave (see PagedRows)
   //   pos, span: a row's position, and how far back it sees
   //   w_lo, w_hi: positions of the wave's first and last row; w_lo_key,
   //     w_hi_key: the first keys they see
   // scale: of scores, in powers of two; SCALED: it is not one
+  // sink: a score (in powers of two) without key and value, if has_sink
   template <bool SCALED, class R>
-  __device__ __forceinline__ void run(char* lds, R rows, int ld, int lo, int last,
+  __device__ __forceinline__ void run(char* lds, R rows, int lo, int last,
                                       const int (&pos)[2],
                                       const int (&span)[2], int w_lo,
                                       int w_hi, int w_lo_key, int w_hi_key,
-                                      float scale) {
+                                      float scale, float sink = 0.f,
+                                      bool has_sink = false) {
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const unsigned at = lds_byte(lds) + wave * 16 * ROW;
-    // the wave's rows of the tile at j0; looked up a tile before they are
-    // copied
-    auto look_up = [&](int j0) {
-      const int j = j0 + wave * 16;
-      return rows((j < last ? j : last) & ~15);
-    };
-    auto place = [&](int c, int most) {  // a lane's in copy c
-      int r = c * RC + lane / PR;
-      const int p = ((lane % PR) ^ turn(r)) * 8;
-      r = r < most ? r : most;
-      return (unsigned)(r * ld + p) * 2;
-    };
-    unsigned off[16 / RC];
-#pragma unroll
-    for (int c = 0; c < 16 / RC; ++c) off[c] = place(c, 15);
-    auto copy = [&](const KeyRows& s, int j0, int buf) {
-      const int j = j0 + wave * 16;
-      const unsigned to = at + buf * TILE;
-      if (j + 15 <= last) {
-#pragma unroll
-        for (int c = 0; c < 16 / RC; ++c) {
-          copy_to_lds(s.k, off[c], to + c * 1024);
-          copy_to_lds(s.v, off[c], to + HALF + c * 1024);
-        }
-      } else {
-        // rows past the last one repeat it: their weights are zero, and
-        // what they are multiplied with has to be a number
-#pragma unroll
-        for (int c = 0; c < 16 / RC; ++c) {
-          const unsigned from = place(c, last & 15);
-          copy_to_lds(s.k, from, to + c * 1024);
-          copy_to_lds(s.v, from, to + HALF + c * 1024);
-        }
-      }
+    const unsigned at = lds_byte(lds) + wave * 16 * K::ROW;
+    const unsigned at_v = lds_byte(lds) + K::BYTES + wave * 16 * V::ROW;
+    auto look_up = [&](int j0) { return rows.look_up(j0 + wave * 16); };
+    auto copy = [&](const auto& s, int j0, int buf) {
+      rows.copy(s, j0 + wave * 16, at + buf * TILE, at_v + buf * TILE);
     };
     float m[2];
     bool seen[2];  // whether the row has met a key
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
-      m[a] = l[a] = 0.f;
-      seen[a] = false;
+      m[a] = sink;
+      l[a] = has_sink && g == 0 ? 1.f : 0.f;
+      seen[a] = has_sink;
 #pragma unroll
       for (int v = 0; v < VT; ++v) o[a][v] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
     copy(look_up(lo), lo, 0);
-    KeyRows ahead = look_up(lo + 64);
+    auto ahead = look_up(lo + 64);
     int buf = 0, j0 = lo;
     auto next = [&]() {  // the tile at j0 is there, the one after it comes
       wait_barrier<0>();
@@ -123,7 +161,7 @@ struct Flash {
     for (; j0 <= w_hi && j0 <= last; j0 += 64, buf ^= 1) {
       next();
       const char* kt = lds + buf * TILE;
-      const char* vt = kt + HALF;
+      const char* vt = kt + K::BYTES;
       f32x4 s[2][4];
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -136,7 +174,7 @@ struct Flash {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const u32x4 kf = *reinterpret_cast<const u32x4*>(
-              kt + (t * 16 + n) * ROW + ((k * 4 + g) ^ turn(n)) * 16);
+              kt + (t * 16 + n) * K::ROW + ((k * 4 + g) ^ K::turn(n)) * 16);
           s[0][t] = mfma(kf, qf[0][k], s[0][t]);
           s[1][t] = mfma(kf, qf[1][k], s[1][t]);
         }
@@ -219,8 +257,8 @@ struct Flash {
           const int c = 2 * v + ((n >> 1) & 1);
           const u32x4 vf = load_columns(
               reinterpret_cast<const unsigned short*>(
-                  vt + r * ROW + (c ^ turn(r)) * 16 + (n & 1) * 8),
-              16 * D);
+                  vt + r * V::ROW + (c ^ V::turn(r)) * 16 + (n & 1) * 8),
+              16 * DV);
           o[0][v] = mfma(vf, pf[0][p], o[0][v]);
           o[1][v] = mfma(vf, pf[1][p], o[1][v]);
         }

@@ -11,7 +11,7 @@
 // and its three partners, rescaling factors are one scalar a lane, and in
 // the prompt kernel the probabilities are already laid out as the B
 // operand of O^T = V^T P^T (keys 4g+i of two tiles make one operand).
-#include "mfma.h"
+#include "flash.h"
 
 // ---------------------------------------------------------------------------
 // Copy the latents that a portion's queries can see out of the pages, 16
@@ -264,6 +264,106 @@ void latent_flash_kernel(
         for (int i = 0; i < 4; ++i)
           if (d + i < V) dst[d + i] = from_f<bf16_t>(o[a][v][i] * inv);
       }
+    }
+  }
+}
+
+// The same for key and value rows that lie in LDS as they are, by the loop
+// of flash.h; values [keys][H V], not transposed.  8 x 2048 tokens, 16 heads
+// of 128 + 64 and 128, a window of 1024: 314 us transposed
+// and through registers, now 192.
+template <int DK, int DV>
+struct LatentRows {
+  using K = TileRows<DK>;
+  using V = TileRows<DV>;
+  const bf16_t* k[K::COPIES];  // the lane's pieces of the wave's first row
+  int step[K::COPIES];         // and numbers to the next row
+  const bf16_t* v;
+  int ld_v;
+  unsigned off[V::COPIES];
+
+  __device__ __forceinline__ int look_up(int j) { return j; }
+  __device__ __forceinline__ void copy(int j, int, unsigned k_to,
+                                       unsigned v_to) {
+#pragma unroll
+    for (int c = 0; c < K::COPIES; ++c)
+      copy_to_lds(k[c] + (size_t)j * step[c], k_to + c * 1024);
+#pragma unroll
+    for (int c = 0; c < V::COPIES; ++c)
+      copy_to_lds(v + (size_t)j * ld_v, off[c], v_to + c * 1024);
+  }
+};
+
+template <int DK, int DV>
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(
+    bf16_t* __restrict__ out, const bf16_t* __restrict__ proj, int ld,
+    const bf16_t* __restrict__ kx, const bf16_t* __restrict__ kr,
+    const bf16_t* __restrict__ vx, const int* __restrict__ items, int H,
+    int D, int window, float scale_log2, const float* __restrict__ sink,
+    int g_off) {
+  using F = Flash<DK, DV>;
+  extern __shared__ __align__(1024) char lds[];
+  const int h = blockIdx.x % H, R = DK - D;
+  const int* it = items + (blockIdx.x / H) * 5;
+  const int q_row = it[0], q_pos = it[1], n_q = it[2], k_row = it[3],
+            k_pos = it[4];
+  const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  F f;
+  int row[2], pos[2];
+  const int span[2] = {window - 1, window - 1};
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    int r = wave * 32 + a * 16 + n;
+    r = r < n_q ? r : n_q - 1;
+    row[a] = q_row + r;
+    pos[a] = q_pos + r - k_pos;
+    const bf16_t* q = proj + (size_t)row[a] * ld + (size_t)h * DK + g * 8;
+#pragma unroll
+    for (int k = 0; k < F::KD; ++k)
+      f.qf[a][k] = *reinterpret_cast<const u32x4*>(q + k * 32);
+  }
+  LatentRows<DK, DV> rows;
+#pragma unroll
+  for (int c = 0; c < F::K::COPIES; ++c) {
+    const int d = F::K::piece(c, lane) * 8;
+    const size_t key = (size_t)k_row + F::K::row(c, lane);
+    rows.k[c] = d >= D ? kr + key * R + (d - D)
+                       : kx + key * H * D + (size_t)h * D + d;
+    rows.step[c] = d >= D ? R : H * D;
+  }
+  rows.v = vx + ((size_t)k_row * H + h) * DV;
+  rows.ld_v = H * DV;
+#pragma unroll
+  for (int c = 0; c < F::V::COPIES; ++c)
+    rows.off[c] = (unsigned)(F::V::row(c, lane) * rows.ld_v +
+                             F::V::piece(c, lane) * 8) * 2;
+
+  // keys as places in the item's key rows, which come in whole 64s
+  const int seen_lo = q_pos - window + 1 - k_pos;
+  const int w_lo = q_pos + wave * 32 - k_pos, w_hi = w_lo + 31;
+  f.template run<true>(lds, rows, (seen_lo > 0 ? seen_lo : 0) & ~63,
+                       q_pos + n_q - k_pos - 1, pos, span, w_lo, w_hi,
+                       w_lo - window + 1, w_hi - window + 1, scale_log2,
+                       sink ? sink[h] * LOG2E : 0.f, sink != nullptr);
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    if (wave * 32 + a * 16 + n >= n_q) continue;
+    const float inv = 1.f / f.l[a];
+    bf16_t* dst = out + ((size_t)row[a] * H + h) * DV + g * 4;
+    const bf16_t* gate = proj + (size_t)row[a] * ld + g_off +
+                         (size_t)h * DV + g * 4;
+#pragma unroll
+    for (int v = 0; v < F::VT; ++v) {
+      float x[4], z[4] = {0.f, 0.f, 0.f, 0.f};
+      if (g_off >= 0) load4(gate + v * 16, z);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[i] = f.o[a][v][i] * inv;
+        if (g_off >= 0) x[i] /= 1.f + __expf(-z[i]);
+      }
+      *reinterpret_cast<uint2*>(dst + v * 16) =
+          make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
     }
   }
 }
@@ -603,6 +703,38 @@ int hy_latent_flash(void* out, const void* proj, int ld, const void* kx,
   } else {
     GO(256, 256);
   }
+#undef GO
+  HY_CHECK();
+  return 0;
+}
+
+// v [keys][H V] here; -2: not for this kernel
+int hy_latent_prompt(void* out, const void* proj, int ld, const void* kx,
+                     const void* kr, const void* v, const void* items,
+                     int n_items, int H, int D, int R, int V, int window,
+                     float scale, const void* sink, int g_off, void* stream) {
+  if (H <= 0 || D <= 0 || D % 8 || R < 0 || R % 8 || ld % 8 || (g_off >= 0 && g_off % 4) ||
+      window < 1 || !(scale > 0.f))
+    return -2;
+#define GO(DK, DV)                                                          \
+  do {                                                                      \
+    constexpr int lds = Flash<DK, DV>::LDS;                                 \
+    static const hipError_t ready = hipFuncSetAttribute(                    \
+        reinterpret_cast<const void*>(latent_prompt_kernel<DK, DV>),        \
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);                   \
+    if (ready != hipSuccess) return -3;                                     \
+    if (n_items <= 0) return 0;                                             \
+    hipLaunchKernelGGL((latent_prompt_kernel<DK, DV>),                      \
+                       dim3((unsigned)n_items * H), dim3(256), lds,         \
+                       (hipStream_t)stream, (bf16_t*)out,                   \
+                       (const bf16_t*)proj, ld, (const bf16_t*)kx,          \
+                       (const bf16_t*)kr, (const bf16_t*)v,                 \
+                       (const int*)items, H, D, window, scale * LOG2E,      \
+                       (const float*)sink, g_off);                          \
+  } while (0)
+  if (D + R == 96 && V == 64) GO(96, 64);
+  else if (D + R == 192 && V == 128) GO(192, 128);
+  else return -2;
 #undef GO
   HY_CHECK();
   return 0;

@@ -215,15 +215,17 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(
   const int w_lo = q_pos + wave * 32 / R;
   const int w_hi = q_pos + (wave * 32 + 31) / R;
   const int* pages = bt + (size_t)it[3] * max_blocks;
+  const int last = q_pos + it[2] - 1;
   f.template run<false>(
       lds,
-      [&](int j) {
-        const bf16_t* k =
-            cache + ((size_t)pages[j / PAGE] * G + kv) * PAGE * (2 * D);
-        return KeyRows{k, k + D};
-      },
-      2 * D, mask.first(q_pos) & ~(PAGE - 1), q_pos + it[2] - 1, pos, span,
-      w_lo, w_hi, w_lo - mask.span(w_lo), w_hi - mask.span(w_hi), 1.f);
+      paged_rows<D>(
+          [&](int j) {
+            const bf16_t* k =
+                cache + ((size_t)pages[j / PAGE] * G + kv) * PAGE * (2 * D);
+            return KeyRows{k, k + D};
+          },
+          2 * D, last),
+      mask.first(q_pos) & ~(PAGE - 1), last, pos, span, w_lo, w_hi, w_lo - mask.span(w_lo), w_hi - mask.span(w_hi), 1.f);
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     if (wave * 32 + a * 16 + n >= n_rows) continue;
