@@ -702,11 +702,20 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
                           if act == "capped" else x.dtype)
     elif out.stride(1) != 1 or out.shape != (N, M):
         return None
-    rc = _require_native().ll_row_gemm(
-        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
-        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K),
-        ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
-        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b), _stream())
+    lib = _require_native()
+    src = (_ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight))
+    sizes = (ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
+    shares = lib.ll_row_gemm_shares(*sizes) if act == "plain" else 1
+    if shares > 1:
+        ws = torch.empty(shares, N, M, device=x.device, dtype=torch.float32)
+        rc = lib.ll_row_gemm_split(
+            *src, _ptr(ws), ctypes.c_int(shares), *sizes,
+            ctypes.c_int(x.stride(0)), _stream())
+    else:
+        rc = lib.ll_row_gemm(
+            *src, *sizes, ctypes.c_int(x.stride(0)),
+            ctypes.c_int(_ROW_ACTS[act]), ctypes.c_int(up),
+            ctypes.c_float(a), ctypes.c_float(b), _stream())
     if rc == -2:
         return None
     _check(rc, "ll_row_gemm")

@@ -93,6 +93,50 @@ __global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(
   });
 }
 
+// A share of the depth, ``depth`` numbers from blockIdx.y * depth on, into
+// ws [shares][N][M] floats.
+template <int NT, int MT, int KW, int S>
+__global__ __launch_bounds__(KW * 64, 2) void row_gemm_share_kernel(
+    float* __restrict__ ws, const bf16_t* __restrict__ x,
+    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, int depth) {
+  using Tile = RowTile<NT, MT, KW, S>;
+  extern __shared__ __align__(1024) char lds[];
+  const int across = (N + 16 * NT - 1) / (16 * NT);
+  const int in = blockIdx.x % (8 * across);
+  const int tile = blockIdx.x / (8 * across) * 8 + in % 8;
+  const int m0 = tile * 16 * MT, n0 = in / 8 * 16 * NT;
+  if (m0 >= M) return;
+  const int k0 = blockIdx.y * depth;
+  Tile::run(
+      lds, K - k0 < depth ? K - k0 : depth, tile >> 3,
+      [&](int r) {
+        return x + (size_t)(n0 + r < N ? n0 + r : N - 1) * ldx + k0;
+      },
+      [&](int r) {
+        return w + (size_t)(m0 + r < M ? m0 + r : M - 1) * K + k0;
+      });
+  Tile::each(4 * MT, [&](int r, int c) {
+    if (n0 + r >= N || m0 + c >= M) return;
+    *reinterpret_cast<f32x4*>(
+        ws + ((size_t)blockIdx.y * N + n0 + r) * M + m0 + c) =
+        Tile::sum(lds, r, c);
+  });
+}
+
+// out = the sum of the shares, four outputs a thread
+__global__ __launch_bounds__(256) void row_gemm_join_kernel(
+    bf16_t* __restrict__ out, int ld_out, const float* __restrict__ ws, int N,
+    int M, int shares) {
+  const int i = blockIdx.x * 256 + threadIdx.x, n = i / (M / 4);
+  if (n >= N) return;
+  const int m = (i - n * (M / 4)) * 4;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < shares; ++s)
+    v += *reinterpret_cast<const f32x4*>(ws + ((size_t)s * N + n) * M + m);
+  *reinterpret_cast<uint2*>(out + (size_t)n * ld_out + m) =
+      make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+}
+
 struct RowGemm {
   void* out;
   int ld_out;
@@ -161,6 +205,66 @@ static int row_gemm_pick(const RowGemm& p) {
     ROW_GEMM(1, 1, 8, 2);
   }
 #undef ROW_GEMM
+}
+
+// In how many shares the depth is taken.  A deep matrix of so few rows that
+// only small tiles fill the chip is bound by what these read of x, not by
+// its own size: larger tiles of a part of the depth read half, for a second
+// launch that adds the parts up.  us, weights from HBM, in one -> in shares:
+//   64 rows: 4096 x 14336 40.2 -> 30.0, 4096 x 19456 54.2 -> 38.6,
+//       4096 x 8192 22.8 -> 20.3, 6144 x 8192 32.2 -> 29.2
+//   32 rows: 4096 x 14336 33.9 -> 25.9, 4096 x 8192 18.2 -> 17.6
+//   128 rows: 4096 x 14336 50.7 -> 45.8, 2048 x 8192 18.8 -> 17.8
+// Not gained by it: 17 rows (4096 x 8192 15.2 -> 16.9), 128 rows of 4096 x
+// 4096 (15.5 -> 16.8), 64 of 2048 x 8192 in shares of 1024 (14.8 -> 16.9 at
+// best).
+extern "C" int ll_row_gemm_shares(int N, int M, int K) {
+  if (N < 32 || N > 128 || K < 8192 || M <= 0 || M % 4) return 1;
+  const int tiles = (N + 15) / 16, across = (tiles + 3) / 4;
+  const int large = (M + 63) / 64 * across;
+  if (large >= 176) return 1;
+  const int most = K / 2048, shares = 256 / large < most ? 256 / large : most;
+  return shares >= 2 && large * shares >= 176 ? shares : 1;
+}
+
+// The same in shares (see above), ws [shares][N][M] floats.
+extern "C" int ll_row_gemm_split(void* out, int ld_out, const void* x,
+                                 const void* w, void* ws, int shares, int N,
+                                 int M, int K, int ldx, void* stream) {
+  if (N <= 16 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
+      ld_out % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
+      (uintptr_t)out % 8 || (uintptr_t)ws % 16 || shares < 1 ||
+      shares > 256)
+    return -2;
+  const int tiles = (N + 15) / 16, across = (tiles + 3) / 4;
+  const int depth = ((K + shares - 1) / shares + 63) / 64 * 64;
+  const int parts = (K + depth - 1) / depth;
+  hipStream_t st = (hipStream_t)stream;
+#define GO(NT)                                                               \
+  do {                                                                       \
+    constexpr int lds = RowTile<NT, 4, 4, 2>::LDS;                           \
+    static const hipError_t sized = hipFuncSetAttribute(                     \
+        reinterpret_cast<const void*>(row_gemm_share_kernel<NT, 4, 4, 2>),   \
+        hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \
+    if (sized != hipSuccess) return -1;                                      \
+    hipLaunchKernelGGL((row_gemm_share_kernel<NT, 4, 4, 2>),                 \
+                       dim3(((M + 63) / 64 + 7) / 8 * 8 * across, parts),    \
+                       dim3(256), lds, st, (float*)ws, (const bf16_t*)x,     \
+                       (const bf16_t*)w, N, M, K, ldx, depth);               \
+  } while (0)
+  switch ((tiles + across - 1) / across) {
+    case 2: GO(2); break;
+    case 3: GO(3); break;
+    default: GO(4); break;
+  }
+#undef GO
+  HY_CHECK();
+  hipLaunchKernelGGL(row_gemm_join_kernel,
+                     dim3((unsigned)(((size_t)N * (M / 4) + 255) / 256)),
+                     dim3(256), 0, st, (bf16_t*)out, ld_out, (const float*)ws,
+                     N, M, parts);
+  HY_CHECK();
+  return 0;
 }
 
 // Rows of x start ldx numbers apart, those of out ld_out.  0: done, -2: not

@@ -35,6 +35,20 @@ def test_row_gemm(N, M, K):
     assert torch.equal(out, ops.linear_decode(x, w))
 
 
+# two to six shares, depths and rows that are no whole pieces or tiles
+@pytest.mark.parametrize("M,K", [(4096, 8200), (2564, 12296), (1348, 17000)])
+@pytest.mark.parametrize("N", [32, 41, 64, 100, 128])
+def test_row_gemm_in_shares(N, M, K):
+    assert ops._require_native().ll_row_gemm_shares(N, M, K) > 1
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    wide = torch.full((N, M + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = ops._row_gemm(x, w, out=wide[:, 4:4 + M])
+    _close(out, x, w)
+    assert (wide[:, :4] == 7).all() and (wide[:, 4 + M:] == 7).all()
+
+
 @pytest.mark.parametrize("N,M,K,shift", [(3, 6, 64, 0), (3, 64, 60, 0),
                                          (3, 64, 64, 1), (3, 64, 64, 4)])
 def test_other_operands_go_to_the_library(N, M, K, shift):
