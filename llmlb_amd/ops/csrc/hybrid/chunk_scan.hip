@@ -297,7 +297,8 @@ void chunk_scan_kernel(ChunkScan p) {
   using C = Chunks<T, DB, CH>;
   constexpr bool DELTA = C::DELTA;
   extern __shared__ __attribute__((aligned(1024))) char lds[];
-  const int e = blockIdx.y, len = p.e_len[e];
+  // long portions come last in a batch and take longest: they go first
+  const int e = gridDim.y - 1 - blockIdx.y, len = p.e_len[e];
   if (len <= 0) return;
   const int head = blockIdx.x % p.H, D = p.D;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);

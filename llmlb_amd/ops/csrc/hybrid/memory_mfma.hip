@@ -157,7 +157,8 @@ void memory_chunk_kernel(
   __shared__ __attribute__((aligned(16))) float lc[CHUNK], lw[CHUNK];
   __shared__ __attribute__((aligned(16))) float lf[MEM ? 1 : CHUNK];
   constexpr int LO = (VB + MEM) * KP;
-  const int e = blockIdx.y;
+  // long portions come last in a batch and take longest: they go first
+  const int e = gridDim.y - 1 - blockIdx.y;
   const int head = blockIdx.x % H, c0 = blockIdx.x / H * VB;
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
   const int n = lane & 15, g = lane >> 4;
