@@ -29,7 +29,13 @@ __device__ __forceinline__ int swizzle_w(int r) {
 // Within 32 outputs of a wave, row g * 8 + t * 4 + i of the matrix is row
 // 4 g + i of MFMA tile t: a lane then holds 8 consecutive outputs of each
 // of its pairs.
-template <int BM, int BN, int WM, int WN, int BK, int ST>
+// WHOLE: the depth is whole steps, and all rows lie within 4 GB of each
+// other: copies are at one scalar address and a lane's own offset, which
+// takes no vector instruction a step (63 a wave before, a quarter of the
+// time).  16384 tokens with 4 of 16 experts, us: 4096 to 1280 wide 668 ->
+// 612, back 752 -> 687; 2048 to 512 169 -> 153, back 174 -> 166.  What a
+// compute unit takes in bounds it then, 42 GB/s of about 50.
+template <int BM, int BN, int WM, int WN, int BK, int ST, bool WHOLE>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 void expert_tile_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ in,
@@ -60,33 +66,59 @@ void expert_tile_kernel(
   const int* list = pairs + (size_t)t.expert * n_tok + t.first;
   const bf16_t* we = w + (size_t)t.expert * N * K;
 
-  const bf16_t *ap[CA], *bp[CB];
-  int ac[CA], bc[CB];  // the lane's column within a row
+  const bf16_t *ap[WHOLE ? 1 : CA], *bp[WHOLE ? 1 : CB];
+  int ac[WHOLE ? 1 : CA], bc[WHOLE ? 1 : CB];  // the lane's column in a row
+  unsigned ao[WHOLE ? CA : 1], bo[WHOLE ? CB : 1];
 #pragma unroll
   for (int i = 0; i < CA; ++i) {
     const int r = (wave * CA + i) * RC + lane / P;
-    ac[i] = ((lane % P) ^ swizzle_in<P>(r)) * 8;
-    ap[i] = in + (size_t)(list[r < t.n ? r : t.n - 1] / div) * K + ac[i];
+    const int c = ((lane % P) ^ swizzle_in<P>(r)) * 8;
+    const size_t at =
+        (size_t)(list[r < t.n ? r : t.n - 1] / div) * K + c;
+    if constexpr (WHOLE) {
+      ao[i] = (unsigned)at * 2;
+    } else {
+      ac[i] = c;
+      ap[i] = in + at;
+    }
   }
 #pragma unroll
   for (int i = 0; i < CB; ++i) {
     const int r = (wave * CB + i) * RC + lane / P;
-    bc[i] = ((lane % P) ^ swizzle_w<P>(r)) * 8;
-    bp[i] = we + (size_t)(n0 + r < N ? n0 + r : N - 1) * K + bc[i];
+    const int c = ((lane % P) ^ swizzle_w<P>(r)) * 8;
+    const size_t at = (size_t)(n0 + r < N ? n0 + r : N - 1) * K + c;
+    if constexpr (WHOLE) {
+      bo[i] = (unsigned)at * 2;
+    } else {
+      bc[i] = c;
+      bp[i] = we + at;
+    }
   }
   const unsigned base = lds_byte(lds);
   const bf16_t* zero = reinterpret_cast<const bf16_t*>(zero_piece);
-  // past the depth zeros are copied: every step has as many copies
+  // past the depth something is copied as well: every step has as many
+  // copies
   auto fetch = [&](int k0, int place) {
     const unsigned to = base + place * SIZE * 2;
+    if constexpr (WHOLE) {
+      const int k = k0 < K ? k0 : 0;
 #pragma unroll
-    for (int i = 0; i < CA; ++i)
-      copy_to_lds(k0 + ac[i] < K ? ap[i] + k0 : zero,
-                  to + (wave * CA + i) * 1024);
+      for (int i = 0; i < CA; ++i)
+        copy_to_lds(in + k, ao[i], to + (wave * CA + i) * 1024);
 #pragma unroll
-    for (int i = 0; i < CB; ++i)
-      copy_to_lds(k0 + bc[i] < K ? bp[i] + k0 : zero,
-                  to + BM * BK * 2 + (wave * CB + i) * 1024);
+      for (int i = 0; i < CB; ++i)
+        copy_to_lds(we + k, bo[i],
+                    to + BM * BK * 2 + (wave * CB + i) * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < CA; ++i)
+        copy_to_lds(k0 + ac[i] < K ? ap[i] + k0 : zero,
+                    to + (wave * CA + i) * 1024);
+#pragma unroll
+      for (int i = 0; i < CB; ++i)
+        copy_to_lds(k0 + bc[i] < K ? bp[i] + k0 : zero,
+                    to + BM * BK * 2 + (wave * CB + i) * 1024);
+    }
   };
   const int wm = wave / WN * (BM / WM), wn = wave % WN * (BN / WN);
   f32x4 acc[TM][TN][4];
@@ -253,25 +285,30 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
       div <= 0)
     return -2;
   if (n_tok <= 0 || n_pairs <= 0) return 0;
-#define GO(BM, BN, WM, WN, BK, ST)                                                 \
+#define RUN(BM, BN, WM, WN, BK, ST, WHOLE)                                   \
+  hipLaunchKernelGGL((expert_tile_kernel<BM, BN, WM, WN, BK, ST, WHOLE>),    \
+                     dim3((unsigned)groups * 8), dim3(WM * WN * 64), 0,      \
+                     (hipStream_t)stream, (bf16_t*)out, (const bf16_t*)in,   \
+                     (const bf16_t*)w, (const int*)counts,                   \
+                     (const int*)pairs, E, N, K, div, act, n_tok, (int)nb)
+#define GO(BM, BN, WM, WN, BK, ST)                                           \
   do {                                                                       \
     const long long nb = (N + BN - 1) / BN;                                  \
     const long long groups = (n_pairs / BM * nb + 7) / 8 +                   \
                              ((E < n_pairs ? E : n_pairs) * nb + 7) / 8;     \
     if (groups >= (1ll << 27)) return -2;                                    \
-    hipLaunchKernelGGL((expert_tile_kernel<BM, BN, WM, WN, BK, ST>),                 \
-                       dim3((unsigned)groups * 8),                           \
-                       dim3(WM * WN * 64), 0, (hipStream_t)stream,           \
-                       (bf16_t*)out, (const bf16_t*)in, (const bf16_t*)w,    \
-                       (const int*)counts, (const int*)pairs, E, N, K, div,  \
-                       act, n_tok, (int)nb);                                 \
+    if (K % BK == 0 && near) RUN(BM, BN, WM, WN, BK, ST, true);              \
+    else RUN(BM, BN, WM, WN, BK, ST, false);                                 \
   } while (0)
+  const long long rows = n_pairs / div + 1 > N ? n_pairs / div + 1 : N;
+  const bool near = rows * K * 2 < (1ll << 32);
   switch (tile) {
     case 0: GO(128, 128, 2, 2, 64, 2); break;
     case 1: GO(256, 256, 4, 4, 64, 2); break;
     case 2: GO(128, 256, 2, 4, 32, 3); break;
     default: return -2;
   }
+#undef RUN
 #undef GO
   HY_CHECK();
   return 0;
