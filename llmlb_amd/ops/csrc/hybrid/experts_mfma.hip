@@ -35,6 +35,9 @@ __device__ __forceinline__ int swizzle_w(int r) {
 // time).  16384 tokens with 4 of 16 experts, us: 4096 to 1280 wide 668 ->
 // 612, back 752 -> 687; 2048 to 512 169 -> 153, back 174 -> 166.  What a
 // compute unit takes in bounds it then, 42 GB/s of about 50.
+// Results are stored by way of the caches: the next kernel reads them, and
+// past the caches (nontemporal) they wait for what these write back (2048
+// wide in a model: back 222 -> 193).
 template <int BM, int BN, int WM, int WN, int BK, int ST, bool WHOLE>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN == 4 ? 2 : 1)
 void expert_tile_kernel(
@@ -200,9 +203,8 @@ void expert_tile_kernel(
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         if (c + i * 32 < N)
-          __builtin_nontemporal_store(
-              u32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]},
-              reinterpret_cast<u32x4*>(dst + c + i * 32));
+          *reinterpret_cast<u32x4*>(dst + c + i * 32) =
+              u32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
     }
   }
 }
