@@ -11,6 +11,7 @@ backend.ragged.RaggedBatch.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -853,12 +854,20 @@ def route(h, w, top, groups, keep, scale, lists: bool = True):
 
 def expert_tile(pairs: int, experts: int, n: int, k: int) -> int:
     """Tile of ``hy_expert_tiles`` for products of depth k with n
-    outputs: 128 x 128 where experts have few pairs or outputs, 256 x 256
-    for deep products, 128 x 256 (two a compute unit, so that one stores
-    while the other multiplies) for shallow ones."""
-    if pairs < 192 * experts or n <= 256:
+    outputs: 128 x 128 where experts have few pairs or outputs, 128 x 256
+    (two a compute unit, so that one stores while the other multiplies)
+    for shallow products.  Deep ones take 256 x 256, a round of one tile a
+    compute unit, unless the last round is too empty: by output 128 x 128
+    takes 1.35 times as long, but in rounds of an eighth.  2048 to 512
+    wide, us (256 x 256, 128 x 128): 0.76 rounds 53, 63; 1.06 98, 83;
+    1.55 105, 114; 2.06 151, 143; 4096 to 1280: 1.42 200, 185; 2.65 325,
+    349; 5.15 619, 720."""
+    if pairs < 192 * experts or n < 256:
         return 0
-    return 1 if k > 1024 else 2
+    if k < 1024:
+        return 2 if n > 256 else 0
+    rounds = (pairs / 256 + experts / 2) * -(-n // 256) / 256
+    return 1 if math.ceil(rounds) <= 1.35 * rounds else 0
 
 
 def experts(h, index, lists, w_up, w_down):
