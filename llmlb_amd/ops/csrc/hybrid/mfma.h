@@ -42,4 +42,12 @@ __device__ __forceinline__ void split2(float a, float b, unsigned& hi,
                  b - __uint_as_float(hi & 0xffff0000u));
 }
 
+// ... and of three, which hold all of a float's 24 bits
+__device__ __forceinline__ void split3(float a, float b, unsigned& hi,
+                                       unsigned& mid, unsigned& lo) {
+  hi = to_bf16x2(a, b);
+  split2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u),
+         mid, lo);
+}
+
 #define LOG2E 1.4426950408889634f

@@ -11,7 +11,7 @@
 // LDS and waited for by the wave that asked.  What hides the wait is other
 // workgroups, two or more to a compute unit; a second stage of LDS in their
 // place was no faster.  Weights and sums stay floats: a weight enters its
-// product as the sum of two bf16 numbers, so products are exact to 2^-17.
+// product as the sum of three bf16 numbers, which are all of its 24 bits.
 //
 // Sequences use as many parts as their length fills (16 pages each), which
 // the host does not know: the rest of the grid ends at once, and where one
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
 #pragma unroll
       for (int v = 0; v < VT; ++v) o[v] *= keep;
     }
-    u32x4 hi, lo;
+    u32x4 hi, mid, lo;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       f32x4 p;
@@ -229,11 +229,11 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
       }
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
-        const unsigned h = to_bf16x2(p[r], p[r + 1]);
+        unsigned h, m2, l2;
+        split3(p[r], p[r + 1], h, m2, l2);
         hi[2 * t + r / 2] = h;
-        lo[2 * t + r / 2] =
-            to_bf16x2(p[r] - __uint_as_float(h << 16),
-                      p[r + 1] - __uint_as_float(h & 0xffff0000u));
+        mid[2 * t + r / 2] = m2;
+        lo[2 * t + r / 2] = l2;
       }
     }
     const char* values = st + 2 * A::BYTES;
@@ -265,8 +265,9 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
           reinterpret_cast<const unsigned short*>(
               values + r * VROW + (c ^ turn<VROW>(r)) * 16 + (n & 1) * 8),
           PAGE * D);
-      o[v] = mfma(vf, hi, o[v]);
       o[v] = mfma(vf, lo, o[v]);
+      o[v] = mfma(vf, mid, o[v]);
+      o[v] = mfma(vf, hi, o[v]);
     }
     // all has been read before the next copy starts
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -93,3 +93,37 @@ def test_no_tokens_give_zeros():
     out = ops.paged_attn_decode(q, k.bfloat16(), v.bfloat16(), bt,
                                 torch.zeros_like(lens), 0.1)
     assert (out == 0).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True], ids=["bf16", "fp8"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_weights_are_floats(D, fp8):
+    """Pairs of keys whose weights differ by 2^-12 and whose values cancel,
+    beside one that takes the rest: what is left shows the weights' last
+    bits.  exp2, the scores, two scalings and the sums are good to about
+    2^-24 each, eight such together; weights of 16 bits would be off by
+    2^-18."""
+    if fp8 and D == 64:
+        pytest.skip("8-bit caches have heads of 128")
+    S, lo = 64, 2.0 ** -12
+    lens = torch.full((S,), 3, dtype=torch.int32, device=DEV)
+    bt = torch.arange(S, dtype=torch.int32, device=DEV)[:, None]
+    q = torch.zeros(S, 16, D, device=DEV)
+    q[..., 0] = torch.linspace(-1.5, -0.1, S, device=DEV)[:, None]
+    q[..., 1], q[..., 2] = 1.0, lo
+    k, v = torch.zeros(2, S, 1, 16, D, device=DEV)
+    k[:, :, :2, 0], k[:, :, 1, 2] = 1.0, 1.0
+    v[:, :, 0], v[:, :, 1] = 1.0, -1.0
+    q = q.bfloat16()
+    scales = {}
+    if fp8:
+        ones = torch.ones(S, 1, 16, device=DEV)
+        scales = dict(k_scale=ones, v_scale=ones)
+        caches = [t.to(torch.float8_e4m3fn).view(torch.uint8)
+                  for t in (k, v)]
+    else:
+        caches = [t.bfloat16() for t in (k, v)]
+    out = ops.paged_attn_decode(q, *caches, bt, lens, 1.0, **scales)
+    ref, _ = _exact(q, k, v, bt, lens, 1.0)
+    bound = ref.abs() * 2.0 ** -8 + 8 * 2.0 ** -24
+    assert ((out.double() - ref).abs() <= bound).all()
