@@ -23,8 +23,9 @@
 // 202.
 //
 // q, k and v are bf16 as projected.  What is float, the weights of s and the
-// state, enters a product as the sum of two bf16 numbers (relative error
-// 2^-17); sums, the state and everything about the gates are float.
+// state, enters a product as a sum of bf16 numbers: of two in the matrix
+// memory (relative error 2^-17), of three in Mamba-2, which hold a float's
+// bits.  Sums, the state and everything about the gates are float.
 // Exponents are of two: F, c and b below carry log2(e).
 #include "memory.h"
 #include "mfma.h"
@@ -152,7 +153,8 @@ void memory_chunk_kernel(
   constexpr int KL = DQ / 32, VL = VB / 32;     // pieces of a tile a thread
   __shared__ unsigned short lk[CHUNK * KP];
   __shared__ unsigned short lv[CHUNK * VP];
-  // [2][VB (+ 1)][KP]: the columns of S (and n), high and low parts
+  constexpr int PARTS = MEM ? 2 : 3;
+  // [PARTS][VB (+ 1)][KP]: the columns of S (and n), high parts first
   extern __shared__ __attribute__((aligned(16))) unsigned short ls[];
   __shared__ __attribute__((aligned(16))) float lc[CHUNK], lw[CHUNK];
   __shared__ __attribute__((aligned(16))) float lf[MEM ? 1 : CHUNK];
@@ -209,12 +211,13 @@ void memory_chunk_kernel(
       const int d = d0 + a * 16 + g * 4;
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
-        uint2 hi, lo;
-        split2(S[a][v][0], S[a][v][1], hi.x, lo.x);
-        split2(S[a][v][2], S[a][v][3], hi.y, lo.y);
+        unsigned x[PARTS], y[PARTS];
+        split_into(S[a][v][0], S[a][v][1], x);
+        split_into(S[a][v][2], S[a][v][3], y);
         unsigned short* to = ls + (v * 16 + n) * KP + d;
-        *reinterpret_cast<uint2*>(to) = hi;
-        *reinterpret_cast<uint2*>(to + LO) = lo;
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+          *reinterpret_cast<uint2*>(to + i * LO) = make_uint2(x[i], y[i]);
       }
       if (MEM && n == 0) {
         uint2 hi, lo;
@@ -321,7 +324,7 @@ void memory_chunk_kernel(
         s[t] = mfma(*reinterpret_cast<const u32x4*>(
                         &lk[(t * 16 + n) * KP + k * 32 + g * 8]),
                     qf[k], s[t]);
-    u32x4 hi[2], lo[2];
+    u32x4 w[2][PARTS];
     float den = 0.f;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -337,17 +340,18 @@ void memory_chunk_kernel(
       const int age = (wave - t) * 16 + n - g * 4;  // of key (t, 0)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float w = s[t][i] * __builtin_amdgcn_exp2f(q_exp + cs[i]);
-        s[t][i] = age >= i ? w : 0.f;
+        const float x = s[t][i] * __builtin_amdgcn_exp2f(q_exp + cs[i]);
+        s[t][i] = age >= i ? x : 0.f;
         if (MEM) den += s[t][i];
       }
-      unsigned h0, h1, l0, l1;
-      split2(s[t][0], s[t][1], h0, l0);
-      split2(s[t][2], s[t][3], h1, l1);
-      hi[t / 2][t % 2 * 2] = h0;
-      hi[t / 2][t % 2 * 2 + 1] = h1;
-      lo[t / 2][t % 2 * 2] = l0;
-      lo[t / 2][t % 2 * 2 + 1] = l1;
+      unsigned x[PARTS], y[PARTS];
+      split_into(s[t][0], s[t][1], x);
+      split_into(s[t][2], s[t][3], y);
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i) {
+        w[t / 2][i][t % 2 * 2] = x[i];
+        w[t / 2][i][t % 2 * 2 + 1] = y[i];
+      }
     }
     if (MEM) {
       den += __shfl_xor(den, 16, WAVE);
@@ -364,8 +368,10 @@ void memory_chunk_kernel(
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
         const unsigned short* x = r + (v * 16 + n) * KP;
-        acc[v] = mfma(*reinterpret_cast<const u32x4*>(x), qf[k], acc[v]);
-        acc[v] = mfma(*reinterpret_cast<const u32x4*>(x + LO), qf[k], acc[v]);
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+          acc[v] = mfma(*reinterpret_cast<const u32x4*>(x + i * LO), qf[k],
+                        acc[v]);
       }
       if constexpr (MEM) {
         const unsigned short* x = r + VB * KP;  // the same for every row
@@ -393,8 +399,8 @@ void memory_chunk_kernel(
             &lv[(r + (n >> 2)) * VP + v * 16 + (n & 3) * 4], 16 * VP);
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
-        acc[v] = mfma(vf[v], hi[p], acc[v]);
-        acc[v] = mfma(vf[v], lo[p], acc[v]);
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i) acc[v] = mfma(vf[v], w[p][i], acc[v]);
       }
       if (holds) {
         const float4 wa = *reinterpret_cast<const float4*>(&lw[r]);
@@ -406,24 +412,24 @@ void memory_chunk_kernel(
         for (int a = 0; a < DT; ++a) {
           const u32x4 kf = load_columns(
               &lk[(r + (n >> 2)) * KP + d0 + a * 16 + (n & 3) * 4], 16 * KP);
-          u32x4 kh, kl;
+          u32x4 kw[PARTS];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            unsigned h, l;
-            split2(__uint_as_float(kf[i] << 16) * ws[2 * i],
-                   __uint_as_float(kf[i] & 0xffff0000u) * ws[2 * i + 1], h,
-                   l);
-            kh[i] = h;
-            kl[i] = l;
+            unsigned x[PARTS];
+            split_into(__uint_as_float(kf[i] << 16) * ws[2 * i],
+                       __uint_as_float(kf[i] & 0xffff0000u) * ws[2 * i + 1],
+                       x);
+#pragma unroll
+            for (int j = 0; j < PARTS; ++j) kw[j][i] = x[j];
           }
 #pragma unroll
-          for (int v = 0; v < VT; ++v) {
-            S[a][v] = mfma(kh, vf[v], S[a][v]);
-            S[a][v] = mfma(kl, vf[v], S[a][v]);
-          }
+          for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int j = 0; j < PARTS; ++j)
+              S[a][v] = mfma(kw[j], vf[v], S[a][v]);
           if constexpr (MEM) {
-            N[a] = mfma(kh, one, N[a]);
-            N[a] = mfma(kl, one, N[a]);
+#pragma unroll
+            for (int j = 0; j < PARTS; ++j) N[a] = mfma(kw[j], one, N[a]);
           }
         }
       }
@@ -492,7 +498,7 @@ static int launch_chunks(void* o, void* state, void* extra, const void* in,
                          int H, int D, int V, float q_scale, hipStream_t s) {
 #define GO(DQ, VB)                                                           \
   do {                                                                       \
-    constexpr int lds = 2 * (VB + MEM) * (DQ + 8) * 2;                       \
+    constexpr int lds = (MEM ? 2 : 3) * (VB + MEM) * (DQ + 8) * 2;           \
     static const hipError_t ready = hipFuncSetAttribute(                     \
         reinterpret_cast<const void*>(memory_chunk_kernel<DQ, VB, MEM>),     \
         hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \

@@ -50,4 +50,13 @@ __device__ __forceinline__ void split3(float a, float b, unsigned& hi,
          mid, lo);
 }
 
+__device__ __forceinline__ void split_into(float a, float b,
+                                           unsigned (&parts)[2]) {
+  split2(a, b, parts[0], parts[1]);
+}
+__device__ __forceinline__ void split_into(float a, float b,
+                                           unsigned (&parts)[3]) {
+  split3(a, b, parts[0], parts[1], parts[2]);
+}
+
 #define LOG2E 1.4426950408889634f

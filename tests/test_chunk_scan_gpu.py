@@ -14,6 +14,9 @@ F64 = torch.float64
 # on each side; the delta rule's products follow each other three deep and
 # pass through the state.  Errors of that size add up like noise.
 TOL = 2.0 ** -14
+# The state-space part's floats enter as three, good to 2^-24: sums of up to
+# 256 products, two such behind each other and through the state.
+FLOATS = 2.0 ** -19
 
 
 def entries(lens, resume):
@@ -28,9 +31,9 @@ def entries(lens, resume):
         for x in (start, lens, pos, row)]
 
 
-def close(got, want):
+def close(got, want, tol=TOL):
     err = (got.double() - want).abs().max() / want.abs().max()
-    assert err < TOL, float(err)
+    assert err < tol, float(err)
 
 
 def run(delta, lens, G, H, D, V, logs, resume=True):
@@ -145,5 +148,5 @@ def test_state_space(D, V, rate):
         _i(H * V + G * D), _i(H * V), _ptr(dt_in), _i(H), _i(0), _ptr(head),
         *(_ptr(t) for t in e), _i(len(lens)), _i(max(lens)), _i(T), _i(G),
         _i(H), _i(D), _i(V), _stream()), "hy_ssm_chunk")
-    close(o.view(T, H, V), want)
-    close(state, want_S)
+    close(o.view(T, H, V), want, FLOATS)
+    close(state, want_S, FLOATS)
