@@ -32,8 +32,7 @@ __device__ __forceinline__ float decay_of(float z, float a_log) {
 // Everything that enters the recurrence, in float.  One wave per unit:
 // units [0, KH) a q/k head, units [KH, KH + H) a value head.
 // ws layout per token: q [KH D] | k [KH D] | g [H D] | v [H V] |
-// qk [KH] | beta [H], padded to whole 16-byte vectors.  g: the decays, or
-// their logarithms (of two).
+// qk [KH] | beta [H], padded to whole 16-byte vectors.
 struct WsLayout {
   int g, v, qk, beta, size;
   __host__ __device__ WsLayout(int KH, int H, int D, int V)
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     const float* __restrict__ dt_bias, const int* __restrict__ pos_,
     const int* __restrict__ row_, const int* __restrict__ tstart_, int n_tok,
     int KH, int H, int D, int V, int taps, float q_scale, int qk_blocks,
-    int v_blocks, bool logs) {
+    int v_blocks) {
   const int t0 = blockIdx.x * PREP_TOK;
   const int t1 = t0 + PREP_TOK < n_tok ? t0 + PREP_TOK : n_tok;
   const int C = 2 * KH * D + H * V;
@@ -199,7 +198,7 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     float f[8];
     load_some<8, VEC>(dec + (size_t)t * H * D + j, valid, f);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = decay_t<T>(f[i] + bias[i], rate[i], logs);
+    for (int i = 0; i < 8; ++i) f[i] = decay_t<T>(f[i] + bias[i], rate[i]);
     store_some<8, VEC>(ws + (size_t)t * at.size + at.g + j, valid, f);
   }
 }
@@ -524,10 +523,9 @@ int hy_delta_prep(void* ws, const void* proj, int ld, int b_off,
                   const void* dec, const void* ring, const void* wconv,
                   const void* a_log, const void* dt_bias, const void* pos,
                   const void* row, const void* tstart, int n_tok, int KH,
-                  int H, int D, int V, int taps, float q_scale, int logs,
-                  int dtype, void* stream) {
+                  int H, int D, int V, int taps, float q_scale, int dtype,
+                  void* stream) {
   if (!delta_ok(KH, H, D, V, taps)) return -2;
-  if (logs && (dtype != 0 || taps > TAPS_MAX || D > 256)) return -2;
   if (n_tok <= 0) return 0;
   if (taps <= TAPS_MAX && D <= 256) {
     const int qk_blocks = (KH + 15) / 16;
@@ -544,7 +542,7 @@ int hy_delta_prep(void* ws, const void* proj, int ld, int b_off,
       (const T*)dec, (const T*)ring, (const float*)wconv,                    \
       (const float*)a_log, (const float*)dt_bias, (const int*)pos,           \
       (const int*)row, (const int*)tstart, n_tok, KH, H, D, V, taps,         \
-      q_scale, qk_blocks, v_blocks, logs != 0))
+      q_scale, qk_blocks, v_blocks))
 #define PICK(RPL)            \
   do {                       \
     if (whole) RUN(RPL, true); \

@@ -2,48 +2,91 @@
 // linear attention, see linear_scan.hip; gated delta rule, see
 // channel_delta.hip) on the matrix cores, 16 tokens at a time.
 //
-// With F_t the sum of the chunk's log decays up to token t and S the state
-// before it, both are
-//   o_t = S^T (q_t e^F_t) + sum over s <= t of Q_ts u_s,
-//   S  <- e^F_15 S + sum over s of (k_s e^(F_15 - F_s)) u_s^T,
-//   Q_ts = sum over channels of q_t k_s e^(F_t - F_s),
+// With F(s, t) the product of the decays after token s up to token t, of a
+// chunk's tokens 0 .. 15, and S the state before it, both are
+//   o_t = S^T (q_t F(-1, t)) + sum over s <= t of Q_ts u_s,
+//   S  <- F(-1, 15) S + sum over s of (k_s F(s, 15)) u_s^T,
+//   Q_ts = sum over channels of q_t k_s F(s, t),
 // with u = v for gated linear attention, and for the delta rule
-//   u = (I + L)^-1 beta (v - S^T (k e^F)),   L_ts = beta_t K_ts (s < t),
+//   u = (I + L)^-1 beta (v - S^T (k F(-1, .))),   L_ts = beta_t K_ts (s < t),
 // K being Q with k_t for q_t.  The inverse is made by substitution.
 //
-// Q and K are products of the matrix cores if e^(F_t - F_s) is taken apart:
-// within eight tokens as e^(F_t - R) e^(R - F_s), R being F after the first
-// four of them, from the second eight to the first as e^(F_t - R) and
-// e^(R - F_s), R of the second.  A step's log decay is taken as no less than
-// 2^-24, which beside what comes in is what a float keeps, so no factor is
-// above 2^96.
+// Q and K are products of factors if F(s, t) is taken apart at a token
+// between the two: of every 2 B tokens, B = 8, 4, 2, 1, the second half asks
+// the first, with the decays of the one from its start on and of the other up
+// to its end.  Those are products of decays as they come, by halves that
+// double: nothing is divided by a decay, and one may be as small as it likes.
+// B = 8 and 4 go to the matrix cores; 2 and 1 are a few pairs within lanes
+// next to each other, and are summed where the factors are made.
 //
-// Everything enters a product as the sum of two bf16 numbers (relative error
-// 2^-17); sums, the state, decays and the substitution are float.
+// All is float, as token by token: the products are those of the matrix cores
+// for floats (16x16x4).  (As sums of two bf16 numbers their results were off
+// by 5e-6 and 7e-6 of their size; now 2e-7, token by token 3e-7.)
 //
 // Bound by the chain from chunk to chunk.  Waves carry the state, 16 value
-// columns each, and work on one chunk while one or two others make Q and the
-// inverse of the next one and the rest the factors of the one after it; they
-// meet once a chunk, and a chunk takes about as long as what the waves of
-// one SIMD issue for it.  8 x 2048 tokens, heads of 128 x 128, us, token by
-// token -> now: delta rule, 16 heads, 1179 -> 340; gated linear attention,
-// 32 heads, 1030 -> 395.
+// columns each, and work on one chunk while others make what it takes of the
+// next ones: the factors, Q and K of them, the inverse.  They meet once a
+// chunk, and a chunk takes about as long as what the waves of one SIMD issue
+// for it.  8 x 2048 tokens, heads of 128 x 128, us, token by token -> now:
+// delta rule, 16 heads, 965 -> 508; gated linear attention, 32 heads, 895
+// -> 490.
 #include "common.h"
 #include "mfma.h"
 #include <type_traits>
 
 #define CHUNK 16
 
-// lane x of every 16 for all of them; the lane n before, or zero
-template <int LANE>
-__device__ __forceinline__ float row_lane(float x) {
+template <int A, int B, int C, int D>
+__device__ __forceinline__ float quad_lanes(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(
-      0, __float_as_int(x), 0x150 + LANE, 0xf, 0xf, true));
+      0, __float_as_int(x), A | B << 2 | C << 4 | D << 6, 0xf, 0xf, true));
 }
+// x *= by of lane LANE of every 16, in the fours of lanes that BANKS names
+template <int LANE, int BANKS>
+__device__ __forceinline__ void times_lane(f32x4& x, f32x4 by) {
+  float a = x[0], b = x[1], c = x[2], d = x[3];
+  // (a number is read from another lane two instructions after it is made)
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %4, %0 row_newbcast:%8 row_mask:0xf bank_mask:%9\n\t"
+      "v_mul_f32_dpp %1, %5, %1 row_newbcast:%8 row_mask:0xf bank_mask:%9\n\t"
+      "v_mul_f32_dpp %2, %6, %2 row_newbcast:%8 row_mask:0xf bank_mask:%9\n\t"
+      "v_mul_f32_dpp %3, %7, %3 row_newbcast:%8 row_mask:0xf bank_mask:%9"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d)
+      : "v"(by[0]), "v"(by[1]), "v"(by[2]), "v"(by[3]), "n"(LANE),
+        "n"(BANKS));
+  x = f32x4{a, b, c, d};
+}
+// four sums over the 16-lane rows, row i with the i-th
+__device__ __forceinline__ float by_rows(const float (&x)[4]) {
+  auto halves = [](float a, float b) {  // rows a0 + a1, b0 + b1, a2 + a3, ..
+    const auto r = __builtin_amdgcn_permlane16_swap(
+        __float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(halves(x[0], x[1])),
+      __float_as_uint(halves(x[2], x[3])), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// c += a^T b for 16 x 16 results and four numbers a lane of the contraction
+__device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 c) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+  return c;
+}
+
+// c[0 .. 3]: parts of the sum of N products
 template <int N>
-__device__ __forceinline__ float row_before(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(
-      0, __float_as_int(x), 0x110 + N, 0xf, 0xf, true));
+__device__ __forceinline__ void products(const f32x4* a, const f32x4* b,
+                                         f32x4 (&c)[4]) {
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      c[j & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+          a[j][i], b[j][i], i == 0 && j < 4 ? zero : c[j & 3], 0, 0, 0);
 }
 
 template <int BYTES, typename To>
@@ -70,43 +113,60 @@ struct ChunkScan {
   float scale;     // of the output
 };
 
-// T: bf16 (gated linear attention) or float (delta rule); g: logs of two
+// T: bf16 (gated linear attention) or float (delta rule)
 // CH: channels of a lane that prepares
 template <typename T, int DB, int CH>
 struct Chunks {
   static constexpr bool DELTA = sizeof(T) == 4;
-  static constexpr int KJ = DB / 32, ROW = 2 * DB, PART = CHUNK * ROW;
-  // waves that prepare, and that make Q and the inverse
-  static constexpr int PREPARE = DB / (4 * CH), SOLVE = DELTA ? 2 : 1;
-  // arrays of hi and lo rows: for the waves with the state, of three chunks
-  static constexpr int QT = 0, KH = 2 * PART, KT = 4 * PART;
-  static constexpr int OWN = DELTA ? 6 * PART : 4 * PART;
-  // and of two chunks left factors, right ones, right ones of the first
-  // eight tokens for the second
-  static constexpr int LQ = 0, RK = 2 * PART, RB = 4 * PART, LK = 5 * PART;
-  static constexpr int PAIR = DELTA ? 7 * PART : 5 * PART;
-  static constexpr int PAIRS = 3 * OWN;                  // [2][PAIR]
-  static constexpr int MT = PAIRS + 2 * PAIR;            // [2][Q, T][1024]
-  static constexpr int END = MT + 4 * 1024;              // [3][DB] floats
-  static constexpr int BETA = END + 3 * DB * 4;               // [2][16]
-  static constexpr int SUB = BETA + 2 * 64;  // [16][16] floats
-  static constexpr int LDS = SUB + (DELTA ? 1024 : 0);
+  static constexpr int ROW = 4 * DB, PART = CHUNK * ROW;
+  // waves that prepare, that make Q, K and the inverse; chunks from the
+  // first of these to the state
+  static constexpr int PREPARE = DB / (4 * CH), SOLVE = DELTA ? 3 : 1;
+  static constexpr int LAG = DELTA ? 3 : 2;
+  // for the waves with the state, of LAG + 1 chunks: q F(-1, t), k F(s, 15)
+  // transposed, k F(-1, t)
+  static constexpr int QT = 0, KH = PART, KT = 2 * PART;
+  static constexpr int OWN = DELTA ? 3 * PART : 2 * PART;
+  // and of two chunks the factors of B = 8 and 4, 8 rows each: q of tokens
+  // that ask, k of those asked, k of those that ask
+  static constexpr int LQ = 0, RK = PART, LK = 2 * PART;
+  static constexpr int PAIR = DELTA ? 3 * PART : 2 * PART;
+  static constexpr int PAIRS = (LAG + 1) * OWN;          // [2][PAIR]
+  static constexpr int Q = PAIRS + 2 * PAIR;             // [LAG][1024]
+  static constexpr int INV = Q + LAG * 1024;             // [2][1024]
+  static constexpr int SUB = INV + (DELTA ? 2048 : 0);   // [2][16][16] floats
+  static constexpr int END = SUB + (DELTA ? 2048 : 0);   // [LAG + 1][DB]
+  static constexpr int SUMS = END + (LAG + 1) * DB * 4;  // [2][PREPARE][64]
+  static constexpr int BETA = SUMS + 2 * PREPARE * 256;  // [4][16]
+  static constexpr int LDS = BETA + 256;
+  static_assert(LDS <= 160 * 1024, "LDS of a compute unit");
 
-  // 16-byte piece p of row r lies at p ^ turn(r)
-  static __device__ __forceinline__ int turn(int r) {
-    return DB == 128 ? r & 15 : (r >> 1) & 7;
+  // 16-byte piece p of row r lies at p ^ r: lanes reading one piece of 16
+  // rows meet every bank once
+  static __device__ __forceinline__ f32x4 piece(const char* a, int r, int p) {
+    return *reinterpret_cast<const f32x4*>(a + r * ROW + (p ^ r) * 16);
   }
-  static __device__ __forceinline__ u32x4 piece(const char* a, int r, int j,
-                                                int g) {
-    return *reinterpret_cast<const u32x4*>(
-        a + r * ROW + ((j * 4 + g) ^ turn(r)) * 16);
+  // where channel ch of the transposed rows is, a row of 16 tokens, and
+  // tokens 4 p .. 4 p + 3 in it: writing lanes differ in ch / 4, reading
+  // ones in ch
+  static __device__ __forceinline__ int column(int ch, int p) {
+    return ((ch & ~15) + (ch & 3) * 4 + (ch >> 2 & 3)) * 64 +
+           (p ^ (ch & 3)) * 16;
   }
-  // sum of the products of hi + lo numbers, but for lo * lo
-  static __device__ __forceinline__ f32x4 both(u32x4 ah, u32x4 al, u32x4 bh,
-                                               u32x4 bl, f32x4 c) {
-    c = mfma(ah, bh, c);
-    c = mfma(ah, bl, c);
-    return mfma(al, bh, c);
+  // element (t, s) of a 16 x 16 matrix in bytes
+  static __device__ __forceinline__ int element(int t, int s) {
+    return t * 64 + ((s >> 2) ^ (t >> 2)) * 16 + (s & 3) * 4;
+  }
+
+  // Where token t's sum g is among a wave's 64 (which: 0 Q, 1 K): with
+  // itself (Q), with the token before it (t odd), with the first two of its
+  // four (t % 4 = 2 or 3); and whether there is one.
+  static __device__ __forceinline__ int sum_at(int which, int g, int t) {
+    const int j = g == 1 ? t >> 1 : (t >> 2) * 2 + (t & 1);
+    return g == 0 ? t : which * 24 + 8 + g * 8 + j;
+  }
+  static __device__ __forceinline__ bool sum_is(int which, int g, int t) {
+    return g == 0 ? which == 0 : g == 1 ? t & 1 : t & 2;
   }
 
   // -- waves that prepare: lane t = lane % 16 is a token, with CH of the
@@ -115,152 +175,184 @@ struct Chunks {
     float g[CH], beta;
     typename std::conditional<DELTA, float[CH], unsigned[CH / 2]>::type q, k;
   };
-
-  // x e into row t of an array, from channel c on; part: its bytes
-  static __device__ __forceinline__ void write(char* a, int c, int t,
-                                               const float (&x)[CH],
-                                               const float (&e)[CH],
-                                               int part = PART) {
-    // quads of channels 0 to 3 of every 32 are the first halves of the
-    // pieces, 4 to 7 the second: as the state's lanes hold them
+  // Products of decays, by token: since the first of its B tokens, and
+  // after it to the last of them.
+  struct Decays {
+    f32x4 pre, suf;
+    // B is doubled
+    __device__ __forceinline__ void pairs(bool second) {
 #pragma unroll
-    for (int h = 0; h < CH; h += 4) {
-      uint2 hi, lo;
-      split2(x[h] * e[h], x[h + 1] * e[h + 1], hi.x, lo.x);
-      split2(x[h + 2] * e[h + 2], x[h + 3] * e[h + 3], hi.y, lo.y);
-      const int quad = (c + h) / 4;
-      char* to = a + t * ROW +
-                 ((quad / 8 * 4 + (quad & 3)) ^ turn(t)) * 16 +
-                 (quad >> 2 & 1) * 8;
-      *reinterpret_cast<uint2*>(to) = hi;
-      *reinterpret_cast<uint2*>(to + part) = lo;
-    }
-  }
-
-  // chunk i, the j-th of three, channels c .. of token t = lane % 16;
-  // real: whether there are such
-  static __device__ __forceinline__ void prepare(char* lds, int i, int j,
-                                                 int c, int t,
-                                                 const Loads& in, bool real,
-                                                 bool all_real) {
-    float F[CH], q[CH], k[CH], e[CH], first[CH], mid[CH], mid2[CH];
-#pragma unroll
-    for (int x = 0; x < CH; ++x) {
-      const float f = in.g[x];
-      F[x] = f < -24.f ? -24.f : f;
-      if constexpr (DELTA) {
-        q[x] = in.q[x];
-        k[x] = in.k[x];
-      } else {
-        const unsigned a = in.q[x / 2], b = in.k[x / 2];
-        q[x] = __uint_as_float(x & 1 ? a & 0xffff0000u : a << 16);
-        k[x] = __uint_as_float(x & 1 ? b & 0xffff0000u : b << 16);
+      for (int x = 0; x < 4; ++x) {
+        const float next = quad_lanes<1, 1, 3, 3>(pre[x]);
+        const float both = pre[x] * quad_lanes<0, 0, 2, 2>(pre[x]);
+        suf[x] = second ? 1.f : next;
+        pre[x] = second ? both : pre[x];
       }
     }
-    if (!all_real && !real) {
+    __device__ __forceinline__ void fours(bool second) {
 #pragma unroll
-      for (int x = 0; x < CH; ++x) F[x] = q[x] = k[x] = 0.f;
+      for (int x = 0; x < 4; ++x) {
+        const float behind = suf[x] * quad_lanes<3, 3, 3, 3>(pre[x]);
+        const float both = pre[x] * quad_lanes<1, 1, 1, 1>(pre[x]);
+        suf[x] = second ? suf[x] : behind;
+        pre[x] = second ? both : pre[x];
+      }
     }
-    // sums over the tokens, of the second eight without the first
-    const bool second = t >= 8;
-#pragma unroll
-    for (int x = 0; x < CH; ++x) {
-      F[x] += row_before<1>(F[x]);
-      F[x] += row_before<2>(F[x]);
-      F[x] += row_before<4>(F[x]);
-      F[x] += row_before<8>(F[x]);
-      first[x] = row_lane<7>(F[x]);
-      if (second) F[x] -= first[x];
-      mid2[x] = row_lane<11>(F[x]);
-      mid[x] = second ? mid2[x] : row_lane<3>(F[x]);
+    __device__ __forceinline__ void eights() {
+      times_lane<7, 1>(suf, pre);
+      times_lane<15, 4>(suf, pre);
+      times_lane<3, 2>(pre, pre);
+      times_lane<11, 8>(pre, pre);
     }
-    char* own = lds + j * OWN;
+    __device__ __forceinline__ void sixteen() {
+      times_lane<15, 3>(suf, pre);
+      times_lane<7, 12>(pre, pre);
+    }
+  };
+
+  // factors of channels c .. c + 3 for the matrix cores
+  template <int B>
+  static __device__ __forceinline__ void factors(char* pair, int c, int t,
+                                                 f32x4 q, f32x4 k,
+                                                 const Decays& f) {
+    const bool asks = t & B;
+    // of B = 8 the rows are 0 to 7 where tokens ask and 8 to 15 where they
+    // are asked, of 4 the other way round: a write's lanes meet every bank
+    // once
+    const int row = t / (2 * B) * B + t % B + (asks == (B == 8) ? 0 : 8);
+    char* to = pair + row * ROW + ((c >> 2) ^ row) * 16;
+    const f32x4 by = asks ? f.pre : f.suf;
+    *reinterpret_cast<f32x4*>(to + (asks ? LQ : RK)) = (asks ? q : k) * by;
+    if (DELTA && asks) *reinterpret_cast<f32x4*>(to + LK) = k * by;
+  }
+
+  // chunk i, channels c .. of token t = lane % 16; real: whether there are
+  // such
+  static __device__ __forceinline__ void prepare(char* lds, int i, int c,
+                                                 int t, const Loads& in,
+                                                 bool real, bool all_real) {
+    char* own = lds + (LAG == 3 ? i & 3 : i % 3) * OWN;
     char* pair = lds + PAIRS + (i & 1) * PAIR;
-    auto exps = [&](auto&& of) {
+    float sum[2][4] = {};
 #pragma unroll
-      for (int x = 0; x < CH; ++x) e[x] = __builtin_amdgcn_exp2f(of(x));
-    };
-    exps([&](int x) { return F[x] - mid[x]; });
-    write(pair + LQ, c, t, q, e);
-    if constexpr (DELTA) write(pair + LK, c, t, k, e);
-    exps([&](int x) { return mid[x] - F[x]; });
-    write(pair + RK, c, t, k, e);
-    exps([&](int x) { return first[x] - F[x] + mid2[x]; });
-    if (!second) write(pair + RB, c, t, k, e, PART / 2);
-    exps([&](int x) {
-      const float last = row_lane<15>(F[x]);
-      return second ? last - F[x] : first[x] - F[x] + last;
-    });
-    write(own + KH, c, t, k, e);
-    exps([&](int x) { return second ? first[x] + F[x] : F[x]; });
-    write(own + QT, c, t, q, e);
-    if constexpr (DELTA) write(own + KT, c, t, k, e);
-    if (t == 15) {
-      float* end = reinterpret_cast<float*>(lds + END) + j * DB + c;
+    for (int h = 0; h < CH / 4; ++h) {
+      const int ch = c + h * 4;
+      f32x4 q, k;
+      Decays f;
 #pragma unroll
-      for (int x = 0; x < CH; x += 4)
-        *reinterpret_cast<float4*>(end + x) =
-            make_float4(e[x], e[x + 1], e[x + 2], e[x + 3]);
+      for (int x = 0; x < 4; ++x) {
+        const int j = h * 4 + x;
+        f.pre[x] = in.g[j];
+        if constexpr (DELTA) {
+          q[x] = in.q[j];
+          k[x] = in.k[j];
+        } else {
+          const unsigned a = in.q[j / 2], b = in.k[j / 2];
+          q[x] = __uint_as_float(j & 1 ? a & 0xffff0000u : a << 16);
+          k[x] = __uint_as_float(j & 1 ? b & 0xffff0000u : b << 16);
+        }
+      }
+      if (!all_real && !real) {
+        q = k = f32x4{0.f, 0.f, 0.f, 0.f};
+        f.pre = f32x4{1.f, 1.f, 1.f, 1.f};
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float before = quad_lanes<0, 0, 2, 2>(k[x]);
+        sum[0][0] += q[x] * k[x];
+        sum[0][1] += q[x] * f.pre[x] * before;
+        if (DELTA) sum[1][1] += k[x] * f.pre[x] * before;
+      }
+      f.pairs(t & 1);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const float asked = k[x] * f.suf[x];
+        const float s0 = quad_lanes<0, 0, 0, 0>(asked);
+        const float s1 = quad_lanes<1, 1, 1, 1>(asked);
+        const float qf = q[x] * f.pre[x], kf = k[x] * f.pre[x];
+        sum[0][2] += qf * s0;
+        sum[0][3] += qf * s1;
+        if (DELTA) {
+          sum[1][2] += kf * s0;
+          sum[1][3] += kf * s1;
+        }
+      }
+      f.fours(t & 2);
+      factors<4>(pair, ch, t, q, k, f);
+      f.eights();
+      factors<8>(pair, ch, t, q, k, f);
+      f.sixteen();
+      const int at = t * ROW + ((ch >> 2) ^ t) * 16;
+      *reinterpret_cast<f32x4*>(own + QT + at) = q * f.pre;
+      if constexpr (DELTA) *reinterpret_cast<f32x4*>(own + KT + at) = k * f.pre;
+      const f32x4 kh = k * f.suf;
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        *reinterpret_cast<float*>(own + KH + column(ch + x, t >> 2) +
+                                  (t & 3) * 4) = kh[x];
+      if (t == 15)
+        *reinterpret_cast<f32x4*>(
+            lds + END + ((LAG == 3 ? i & 3 : i % 3) * DB + ch) * 4) = f.pre;
+    }
+    float* sums = reinterpret_cast<float*>(lds + SUMS) +
+                  ((i & 1) * PREPARE + c / (4 * CH)) * 64;
+    const int g = threadIdx.x >> 4 & 3;
+#pragma unroll
+    for (int which = 0; which <= DELTA; ++which) {
+      const float x = by_rows(sum[which]);
+      if (sum_is(which, g, t)) sums[sum_at(which, g, t)] = x;
     }
     if (DELTA && c == 0)
-      reinterpret_cast<float*>(lds + BETA)[(i & 1) * 16 + t] =
+      reinterpret_cast<float*>(lds + BETA)[(i & 3) * 16 + t] =
           real ? in.beta : 0.f;
   }
 
-  // row t = 4 g + i, column s = n of the left factors' product with the
-  // right ones; what is above the diagonal is anything
-  static __device__ __forceinline__ f32x4 pairs(const char* pair, int left,
-                                                int n, int g) {
+  // put(t, s, x) with the products of tokens t and s: those of B = 8 and 4
+  // of the factors at ``left`` with those asked, and of the sums made above
+  // (which: 0 Q, 1 K)
+  template <class F>
+  static __device__ __forceinline__ void products(const char* lds, int buf,
+                                                  int left, int which,
+                                                  int lane, F put) {
+    const int n = lane & 15, g = lane >> 4;
+    const char* pair = lds + PAIRS + buf * PAIR;
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
 #pragma unroll
-    for (int j = 0; j < KJ; ++j) {
-      const u32x4 lh = piece(pair + left, n, j, g);
-      const u32x4 ll = piece(pair + left + PART, n, j, g);
-      a = both(lh, ll, piece(pair + RK, n, j, g),
-               piece(pair + RK + PART, n, j, g), a);
-      b = both(lh, ll, piece(pair + RB, n & 7, j, g),
-               piece(pair + RB + PART / 2, n & 7, j, g), b);
+    for (int j = 0; j < DB / 16; j += 2) {
+      a = mfma4(piece(pair + left, n, 4 * j + g),
+                piece(pair + RK, n, 4 * j + g), a);
+      b = mfma4(piece(pair + left, n, 4 * j + 4 + g),
+                piece(pair + RK, n, 4 * j + 4 + g), b);
     }
-    return g >= 2 && n < 8 ? b : a;
-  }
-
-  // a 16 x 16 matrix as the left operand of a product with u: a row's
-  // columns 4 g .. + 3, hi and then lo
-  static __device__ __forceinline__ void put(char* m, int t, int s, float x) {
-    unsigned hi, lo;
-    split2(x, 0.f, hi, lo);
-    unsigned short* to =
-        reinterpret_cast<unsigned short*>(m + t * 64 + (s >> 2) * 16) +
-        (s & 3);
-    to[0] = hi;
-    to[4] = lo;
-  }
-
-  static __device__ __forceinline__ void outputs_of_values(char* lds, int buf,
-                                                           int lane) {
-    const int n = lane & 15, g = lane >> 4;
-    const f32x4 m = pairs(lds + PAIRS + buf * PAIR, LQ, n, g);
+    a += b;
+    const float* sums = reinterpret_cast<const float*>(lds + SUMS) +
+                        buf * PREPARE * 64 + sum_at(which, g, n);
+    float x = sums[0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      put(lds + MT + buf * 2048, 4 * g + i, n, n <= 4 * g + i ? m[i] : 0.f);
+    for (int p = 1; p < PREPARE; ++p) x += sums[p * 64];
+    // rows 0 to 7 of a with columns 8 to 15 are of B = 8, rows 8 to 15 with
+    // columns 0 to 7 of B = 4, where both are of the same eight tokens
+    if ((g < 2) == (n >= 8)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = (4 * g + i) & 7, s = n & 7;
+        if (g < 2)
+          put(8 + t, s, a[i]);
+        else if (t >> 2 == s >> 2)
+          put(8 * (t >> 2) + 4 + (t & 3), 8 * (s >> 2) + (s & 3), a[i]);
+      }
+    }
+    if (sum_is(which, g, n))
+      put(n, g == 0 ? n : g == 1 ? n - 1 : (n & ~3) + g - 2, x);
   }
 
   // (I + L)^-1 beta by substitution, four rows at a time: of these lane g
   // makes row g of column n as far as the rows before go, then every lane
   // has all four
-  static __device__ __forceinline__ void inverse(char* lds, int buf,
+  static __device__ __forceinline__ void inverse(const float* L,
+                                                 const float* beta, char* m,
                                                  int lane) {
     const int n = lane & 15, g = lane >> 4;
-    const float* beta =
-        reinterpret_cast<const float*>(lds + BETA) + buf * 16;
-    const float bn = beta[n];
-    const float4 bt = *reinterpret_cast<const float4*>(beta + 4 * g);
-    const f32x4 m = pairs(lds + PAIRS + buf * PAIR, LK, n, g);
-    const f32x4 l = m * f32x4{bt.x, bt.y, bt.z, bt.w};
-    float* L = reinterpret_cast<float*>(lds + SUB);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) L[(4 * g + i) * 16 + n] = l[i];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     float x[16];
 #pragma unroll
     for (int r = 0; r < 16; r += 4) {
@@ -279,17 +371,19 @@ struct Chunks {
           x[r + i] -= L[(r + i) * 16 + r + s] * x[r + s];
       }
     }
+    const float bn = beta[n];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float y =
           g < 2 ? (g == 0 ? x[i] : x[4 + i]) : (g == 2 ? x[8 + i] : x[12 + i]);
-      put(lds + MT + buf * 2048 + 1024, 4 * g + i, n, y * bn);
+      *reinterpret_cast<float*>(m + element(4 * g + i, n)) = y * bn;
     }
   }
 };
 
 // One workgroup: 16 NC value columns of one head of one entry.  In step i
-// the waves with the state are at chunk i - 2.
+// waves prepare chunk i, make Q and K of chunk i - 1, the inverse of chunk
+// i - 2, and those with the state are at chunk i - LAG.
 template <typename T, int DB, int CH, int NC>
 __global__ __launch_bounds__(64 * (NC + Chunks<T, DB, CH>::PREPARE +
                                    Chunks<T, DB, CH>::SOLVE))
@@ -308,15 +402,35 @@ void chunk_scan_kernel(ChunkScan p) {
   const int chunks = (len + CHUNK - 1) / CHUNK;
 
   if (wave >= NC + C::PREPARE) {
+    const int part = wave - NC - C::PREPARE;
+    if (part == 0)  // what Q has above its diagonal stays zero
+      for (int i = lane; i < C::LAG * 64; i += 64)
+        *reinterpret_cast<uint4*>(lds + C::Q + i * 16) =
+            make_uint4(0, 0, 0, 0);
+    float* const beta = reinterpret_cast<float*>(lds + C::BETA);
+    float* const sub = reinterpret_cast<float*>(lds + C::SUB);
     __syncthreads();
-    for (int i = 0; i < chunks; ++i) {
-      if (wave == NC + C::PREPARE)
-        C::outputs_of_values(lds, i & 1, lane);
-      else if constexpr (DELTA)
-        C::inverse(lds, i & 1, lane);
+    for (int i = 0; i < chunks + C::LAG - 2; ++i) {
+      if (part == 0) {
+        char* m = lds + C::Q + i % C::LAG * 1024;
+        if (i < chunks)
+          C::products(lds, i & 1, C::LQ, 0, lane,
+                      [&](int t, int s, float x) {
+                        *reinterpret_cast<float*>(m + C::element(t, s)) = x;
+                      });
+      } else if (DELTA && part == 1) {
+        float* L = sub + (i & 1) * 256;
+        const float* b = beta + (i & 3) * 16;
+        if (i < chunks)
+          C::products(lds, i & 1, C::LK, 1, lane, [&](int t, int s, float x) {
+            L[t * 16 + s] = x * b[t];
+          });
+      } else if (DELTA && i > 0 && i <= chunks) {
+        C::inverse(sub + (~i & 1) * 256, beta + ((i - 1) & 3) * 16,
+                   lds + C::INV + (~i & 1) * 1024, lane);
+      }
       __syncthreads();
     }
-    __syncthreads();
     return;
   }
   if (wave >= NC) {
@@ -324,46 +438,43 @@ void chunk_scan_kernel(ChunkScan p) {
     const bool real = c < D;
     const int ch = real ? c : 0;
     const int kv = head / (p.H / p.G) * D + ch;
-    typename C::Loads next;
+    typename C::Loads x;
     auto fetch = [&](int t) {
       t = t < len ? t : len - 1;
       const T* row = in + (size_t)t * p.ld + kv;
       const float* gr = p.g + (first + t) * p.ld_g + (size_t)head * D + ch;
       constexpr int B = CH * sizeof(T);
-      load_bytes<B>(row + p.q_off, next.q);
-      load_bytes<B>(row + p.k_off, next.k);
-      load_bytes<CH * 4>(gr, next.g);
-      if (DELTA) next.beta = p.beta[(first + t) * p.ld + head];
+      load_bytes<B>(row + p.q_off, x.q);
+      load_bytes<B>(row + p.k_off, x.k);
+      load_bytes<CH * 4>(gr, x.g);
+      if (DELTA) x.beta = p.beta[(first + t) * p.ld + head];
     };
     fetch(n);
-    for (int i = 0, j = 0; i < chunks; ++i, j = j == 2 ? 0 : j + 1) {
-      const typename C::Loads now = next;
-      if (i + 1 < chunks) fetch((i + 1) * CHUNK + n);
-      C::prepare(lds, i, j, c, n, now, real && i * CHUNK + n < len,
-                 D == DB && (i + 1) * CHUNK <= len);
+    for (int i = 0; i < chunks + C::LAG - 1; ++i) {
+      if (i < chunks) {
+        const typename C::Loads now = x;
+        if (i + 1 < chunks) fetch((i + 1) * CHUNK + n);
+        C::prepare(lds, i, c, n, now, real && i * CHUNK + n < len,
+                   D == DB && (i + 1) * CHUNK <= len);
+      }
       __syncthreads();
     }
-    __syncthreads();
-    __syncthreads();
     return;
   }
 
-  // S[tile] holds key channels 16 tile + 4 g .. + 3 of the lane's column
+  // S[a] holds key channels 16 a + 4 g .. + 3 of the lane's column
   const int col = blockIdx.x / p.H * (16 * NC) + wave * 16 + n;
   const bool real = col < p.V;
   const int cv = real ? col : p.V - 1;
-  f32x4 S[2 * C::KJ];
+  f32x4 S[DB / 16];
   float* sp =
       p.state + (((size_t)p.e_row[e] * p.H + head) * p.V + cv) * (size_t)D;
   const bool resume = p.e_pos[e] > 0;
 #pragma unroll
-  for (int a = 0; a < 2 * C::KJ; ++a) {
+  for (int a = 0; a < DB / 16; ++a) {
     const int d = a * 16 + g * 4;
     S[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (resume && d < D) {
-      const float4 x = *reinterpret_cast<const float4*>(sp + d);
-      S[a] = f32x4{x.x, x.y, x.z, x.w};
-    }
+    if (resume && d < D) S[a] = *reinterpret_cast<const f32x4*>(sp + d);
   }
   T vn[4];
   auto fetch = [&](int t0) {
@@ -377,89 +488,78 @@ void chunk_scan_kernel(ChunkScan p) {
   fetch(0);
   float* out = p.o + (first * p.H + head) * p.V + cv;
   const size_t step = (size_t)p.H * p.V;
-  __syncthreads();
-  __syncthreads();
-  for (int i = 0, third = 0; i < chunks;
-       ++i, third = third == 2 ? 0 : third + 1) {
-    const char* own = lds + third * C::OWN;
-    const char* mats = lds + C::MT + (i & 1) * 2048 + n * 64 + g * 16;
-    T v[4];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) v[x] = vn[x];
-    if (i + 1 < chunks) fetch((i + 1) * CHUNK);
+  for (int i = 0; i < C::LAG; ++i) __syncthreads();
+  for (int i = 0; i < chunks; ++i) {
+    const int place = C::LAG == 3 ? i & 3 : i % 3;
+    const char* own = lds + place * C::OWN;
+    const char* q = lds + C::Q + i % C::LAG * 1024 + C::element(n, 4 * g);
+    f32x4 u;  // of tokens 4 g .. + 3
+#pragma unroll
+    for (int x = 0; x < 4; ++x) u[x] = to_f(vn[x]);
+    fetch((i + 1) * CHUNK);
 
-    f32x4 w = {0.f, 0.f, 0.f, 0.f}, o = w;
-#pragma unroll
-    for (int j = 0; j < C::KJ; ++j) {
-      u32x4 sh, sl;
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        unsigned a, b;
-        split2(S[2 * j + h / 2][h % 2 * 2], S[2 * j + h / 2][h % 2 * 2 + 1],
-               a, b);
-        sh[h] = a;
-        sl[h] = b;
-      }
-      if constexpr (DELTA)
-        w = C::both(C::piece(own + C::KT, n, j, g),
-                    C::piece(own + C::KT + C::PART, n, j, g), sh, sl, w);
-      o = C::both(C::piece(own + C::QT, n, j, g),
-                  C::piece(own + C::QT + C::PART, n, j, g), sh, sl, o);
-    }
-    // hi and lo of u, tokens 4 g .. + 3 twice
-    u32x4 uh, ul;
-    auto parts = [&](f32x4 x) {
-      unsigned h0, h1, l0, l1;
-      split2(x[0], x[1], h0, l0);
-      split2(x[2], x[3], h1, l1);
-      uh = u32x4{h0, h1, h0, h1};
-      ul = u32x4{l0, l1, l0, l1};
-    };
+    // sums in four parts, so that no product waits for the one before
+    constexpr int N = DB / 16;
+    f32x4 x[N], o[4];
     if constexpr (DELTA) {
-      parts(f32x4{v[0] - w[0], v[1] - w[1], v[2] - w[2], v[3] - w[3]});
-      const u32x4 m = *reinterpret_cast<const u32x4*>(mats + 1024);
-      f32x4 u = {0.f, 0.f, 0.f, 0.f};
-      u = mfma(m, uh, u);
-      parts(mfma(m, ul, u));
-    } else {
-      parts(f32x4{to_f(v[0]), to_f(v[1]), to_f(v[2]), to_f(v[3])});
+      f32x4 w[4];
+#pragma unroll
+      for (int a = 0; a < N; ++a) x[a] = C::piece(own + C::KT, n, 4 * a + g);
+      products<N>(x, S, w);
+      u = mfma4(*reinterpret_cast<const f32x4*>(
+                    lds + C::INV + (i & 1) * 1024 + C::element(n, 4 * g)),
+                u - ((w[0] + w[1]) + (w[2] + w[3])),
+                f32x4{0.f, 0.f, 0.f, 0.f});
     }
-    const u32x4 m = *reinterpret_cast<const u32x4*>(mats);
-    o = mfma(m, uh, o);
-    if constexpr (DELTA) o = mfma(m, ul, o);
+#pragma unroll
+    for (int a = 0; a < N; ++a) x[a] = C::piece(own + C::QT, n, 4 * a + g);
+    products<N>(x, S, o);
+    const f32x4 m = *reinterpret_cast<const f32x4*>(q);
     const float* end =
-        reinterpret_cast<const float*>(lds + C::END) + third * DB;
-    const int r = 4 * g + (n >> 2);
+        reinterpret_cast<const float*>(lds + C::END) + place * DB;
 #pragma unroll
-    for (int a = 0; a < 2 * C::KJ; ++a) {
-      const float4 f = *reinterpret_cast<const float4*>(end + a * 16 + g * 4);
-      const char* at = own + C::KH + r * C::ROW +
-                       ((a / 2 * 4 + (n & 3)) ^ C::turn(r)) * 16 + a % 2 * 8;
-      const u32x4 k = load_columns(
-          reinterpret_cast<const unsigned short*>(at), C::PART / 2);
-      S[a] *= f32x4{f.x, f.y, f.z, f.w};
-      S[a] = mfma(k, uh, S[a]);
-      if constexpr (DELTA) S[a] = mfma(k, ul, S[a]);
+    for (int a = 0; a < N; ++a)
+      x[a] = *reinterpret_cast<const f32x4*>(own + C::KH +
+                                             C::column(16 * a + n, g));
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      o[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], u[r], o[r], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+      S[a] *= *reinterpret_cast<const f32x4*>(end + a * 16 + g * 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int a = 0; a < N; ++a)
+        S[a] =
+            __builtin_amdgcn_mfma_f32_16x16x4f32(x[a][r], u[r], S[a], 0, 0, 0);
+    const f32x4 sum = (o[0] + o[1]) + (o[2] + o[3]);
+    // Lanes without a column of their own repeat the last one and store the
+    // same.  Only the last chunk asks which tokens there are: what may or
+    // may not be stored would be waited for with the next chunk's values.
+    if (i + 1 < chunks) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        out[(i * CHUNK + 4 * g + x) * step] = sum[x] * p.scale;
+      __syncthreads();
+      continue;
     }
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int t = i * CHUNK + 4 * g + x;
-      if (real && t < len) out[t * step] = o[x] * p.scale;
-    }
-    __syncthreads();
+    for (int x = 0; x < 4; ++x)
+      if (i * CHUNK + 4 * g + x < len)
+        out[(i * CHUNK + 4 * g + x) * step] = sum[x] * p.scale;
   }
   if (!real) return;
 #pragma unroll
-  for (int a = 0; a < 2 * C::KJ; ++a) {
+  for (int a = 0; a < DB / 16; ++a) {
     const int d = a * 16 + g * 4;
-    if (d < D)
-      *reinterpret_cast<float4*>(sp + d) =
-          make_float4(S[a][0], S[a][1], S[a][2], S[a][3]);
+    if (d < D) *reinterpret_cast<f32x4*>(sp + d) = S[a];
   }
 }
 
 // dtype 0: in bf16 (gated linear attention, G = H), 1: in float (delta rule,
-// beta [n_tok][ld]); g: logarithms (of two) of the decays
+// beta [n_tok][ld]); g: the decays
 extern "C" int hy_chunk_scan(void* o, void* state, const void* in, int ld,
                              int q_off, int k_off, int v_off, const void* g,
                              int ld_g, const void* beta, const void* e_start,

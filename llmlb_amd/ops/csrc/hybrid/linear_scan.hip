@@ -312,11 +312,11 @@ __global__ __launch_bounds__(64) void memory_gates_kernel(
   if (lane == 0) ex[extra_row(D) - 4] = m;
 }
 
-// g = sigmoid(dec + bias)^rate per channel; logs: its logarithm (of two)
+// g = sigmoid(dec + bias)^rate per channel
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void gla_decay_kernel(
     float* __restrict__ g, const T* __restrict__ dec,
-    const float* __restrict__ bias, int n_tok, int C, float rate, bool logs) {
+    const float* __restrict__ bias, int n_tok, int C, float rate) {
   constexpr int N = VEC ? 8 : 1;
   const int c = (blockIdx.y * 256 + threadIdx.x) * N;
   if (c >= C) return;
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(
     float f[N];
     load_run<N, VEC>(dec + (size_t)t * C + c, f);
 #pragma unroll
-    for (int i = 0; i < N; ++i) f[i] = decay_t<T>(-(f[i] + b[i]), rate, logs);
+    for (int i = 0; i < N; ++i) f[i] = decay_t<T>(-(f[i] + b[i]), rate);
     store_run<N, VEC>(g + (size_t)t * C + c, f);
   }
 }
@@ -675,8 +675,7 @@ int hy_linear_scan(void* o, void* state, const void* in, int ld, int q_off,
 }
 
 int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
-                 float rate, int logs, int dtype, void* stream) {
-  if (logs && dtype != 0) return -2;
+                 float rate, int dtype, void* stream) {
   if (n_tok <= 0 || C <= 0) return 0;
   const bool vec = C % 8 == 0;
   const int cols = vec ? 2048 : 256;
@@ -685,7 +684,7 @@ int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                    \
       (gla_decay_kernel<T, VEC>), grid, dim3(256), 0,                    \
       (hipStream_t)stream, (float*)g, (const T*)dec, (const float*)bias, \
-      n_tok, C, rate, logs != 0))
+      n_tok, C, rate))
   if (vec) GO(true);
   else GO(false);
 #undef GO

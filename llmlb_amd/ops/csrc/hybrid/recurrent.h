@@ -102,16 +102,13 @@ template <typename T>
 __device__ __forceinline__ float sigmoid_t(float x) {
   return sizeof(T) == 2 ? 1.f / (1.f + __expf(-x)) : sigmoid_f(x);
 }
-// logs: the logarithm (of two) instead
 template <typename T>
-__device__ __forceinline__ float decay_t(float z, float rate,
-                                         bool logs = false) {
+__device__ __forceinline__ float decay_t(float z, float rate) {
   if (sizeof(T) == 2) {
     const float e = __expf(-fabsf(z));
     // log(1 + e) by its series where 1 + e would lose e
     const float lp = e < 1e-3f ? e * (1.f - 0.5f * e) : __logf(1.f + e);
-    const float f = -rate * (fmaxf(z, 0.f) + lp);
-    return logs ? f * 1.4426950408889634f : __expf(f);
+    return __expf(-rate * (fmaxf(z, 0.f) + lp));
   }
   return expf(-rate * softplus_f(z));
 }

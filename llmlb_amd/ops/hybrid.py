@@ -343,15 +343,22 @@ def _runs(b):
             _i(len(b.entries)))
 
 
-def by_chunks(b) -> bool:
+def by_chunks(b, tokens=12, heads=48) -> bool:
     """Whether recurrences of the batch go by chunks of tokens on the
-    matrix cores (bf16 models): a chunk costs about what a dozen tokens
-    cost one by one.  32 heads of 128 x 128, us, gated linear attention:
-    64 portions of 1 token 63 (one by one 45), of 4 66 (55), of 16 71
-    (90), 8 portions of 2048 395 (1025); Mamba-2: 76 (44), 75 (51), 78
-    (87) and 215 (1119)."""
-    longest = max((n for _, n, _, _ in b.entries), default=0)
-    return longest >= 64 or b.n_tok >= 12 * len(b.entries)
+    matrix cores (bf16 models): a chunk costs about what ``tokens`` tokens
+    cost one by one.  32 heads of 128 x 128, us, Mamba-2 (12): 64 portions
+    of 1 token 76 (one by one 44), of 4 75 (51), of 16 78 (87), 8 portions
+    of 2048 215 (1119); gated linear attention (16): 64 portions of 8
+    tokens 65 (53), of 16 67 (78), 8 of 2048 490 (895); delta rule (32): 64
+    of 16 87 (93), of 32 148 (196), 8 of 2048 710 (1259).
+
+    The delta rule's chunks are also a longer chain than its tokens, and
+    gain only where those share compute units, from about 48 ``heads`` of
+    portions on: 1 x 300 tokens, 16 heads 65 (50), 2 x 300, 16 heads 66
+    (61), 3 x 517, 16 heads 111 (163), 2 x 300, 32 heads 66 (80)."""
+    lens = [n for _, n, _, _ in b.entries]
+    return (max(lens, default=0) >= 64 or b.n_tok >= tokens * len(lens)) \
+        and heads * sum(n >= tokens for n in lens) >= 48
 
 
 def can_chunk_scan(dtype, dim) -> bool:
@@ -391,12 +398,13 @@ def gated_delta(proj, b_off, dec, gate, state, ring, b, wconv, a_log,
     ws = torch.empty(T, int(lib.hy_delta_ws_floats(*sizes)),
                      dtype=torch.float32, device=proj.device)
     o = torch.empty(T, H * V, dtype=torch.float32, device=proj.device)
-    chunks = by_chunks(b) and taps <= 4 and can_chunk_scan(proj.dtype, D)
+    chunks = by_chunks(b, 32, H) and taps <= 4 \
+        and can_chunk_scan(proj.dtype, D)
     _check(lib.hy_delta_prep(
         _ptr(ws), _ptr(proj), ld, _i(b_off), _ptr(dec), _ptr(ring),
         _ptr(wconv), _ptr(a_log), _ptr(dt_bias), _ptr(b.pos), _ptr(b.row),
-        _ptr(b.tstart), _i(T), *sizes, _i(taps), q_scale, _i(chunks), dt,
-        st), "hy_delta_prep")
+        _ptr(b.tstart), _i(T), *sizes, _i(taps), q_scale, dt, st),
+        "hy_delta_prep")
     if chunks:
         g, v, size = 2 * KH * D, 2 * KH * D + H * D, ws.shape[1]
         beta = v + H * V + KH
@@ -525,12 +533,12 @@ def gated_linear(out, proj, k_off, v_off, g_off, dec, dec_bias, state, b,
         return
     g = torch.empty(T, H * D, dtype=torch.float32, device=proj.device)
     o = torch.empty(T, H * V, dtype=torch.float32, device=proj.device)
-    chunks = by_chunks(b) and can_chunk_scan(proj.dtype, D) \
+    chunks = by_chunks(b, 16) and can_chunk_scan(proj.dtype, D) \
         and proj.stride(0) % 8 == 0 and k_off % 8 == 0 \
         and proj.data_ptr() % 16 == 0
     _check(lib.hy_gla_decay(
-        _ptr(g), _ptr(dec), _ptr(dec_bias), _i(T), _i(H * D), rate,
-        _i(chunks), dt, st), "hy_gla_decay")
+        _ptr(g), _ptr(dec), _ptr(dec_bias), _i(T), _i(H * D), rate, dt, st),
+        "hy_gla_decay")
     if chunks:
         _check(lib.hy_chunk_scan(
             _ptr(o), _ptr(state), _ptr(proj), ld, _i(0), _i(k_off),

@@ -10,13 +10,11 @@ from llmlb_amd.ops.hybrid import _check, _f, _i, _ptr, _stream
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 F64 = torch.float64
-# What is no bf16 number enters a product as two of them, good to 2^-17, one
-# on each side; the delta rule's products follow each other three deep and
-# pass through the state.  Errors of that size add up like noise.
-TOL = 2.0 ** -14
-# The state-space part's floats enter as three, good to 2^-24: sums of up to
-# 256 products, two such behind each other and through the state.
-FLOATS = 2.0 ** -19
+# All is float (the state-space part's weights and state take three bf16
+# numbers each): numbers good to 2^-24, sums of up to 256 products, products
+# of up to 16 decays, three such products behind each other and through the
+# state.  Errors of that size add up like noise.
+TOL = 2.0 ** -19
 
 
 def entries(lens, resume):
@@ -31,13 +29,15 @@ def entries(lens, resume):
         for x in (start, lens, pos, row)]
 
 
-def close(got, want, tol=TOL):
+def close(got, want):
     err = (got.double() - want).abs().max() / want.abs().max()
-    assert err < tol, float(err)
+    assert err < TOL, float(err)
 
 
-def run(delta, lens, G, H, D, V, logs, resume=True):
-    """logs: (lowest, highest) logarithm of two of a decay."""
+def run(delta, lens, G, H, D, V, logs, resume=True, reset=None):
+    """logs: (lowest, highest) logarithm of two of a decay; reset: tokens
+    whose decays are 2^-90 and after which inputs are 2^-20 of those before,
+    for 2 tokens."""
     g = torch.Generator(device=DEV).manual_seed(sum(lens) + D + V)
     T, start, pos, row, e = entries(lens, resume)
     kind = torch.float32 if delta else torch.bfloat16
@@ -48,10 +48,13 @@ def run(delta, lens, G, H, D, V, logs, resume=True):
         x[:, :2 * G * D] = torch.nn.functional.normalize(
             x[:, :2 * G * D].unflatten(1, (2 * G, D)), dim=2).flatten(1)
         x[:, vo + H * V:] = x[:, vo + H * V:].sigmoid()
-    x = x.to(kind)
     lo, hi = logs
     f = (torch.rand(T, H, D, generator=g, device=DEV) * (hi - lo) + lo).neg_()
     f[:, :, ::3] *= 2.0 ** -6      # channels that remember
+    for t in reset or ():
+        f[t] = -90.0
+        x[t:t + 3, G * D:vo + H * V] *= 2.0 ** -20      # k and v
+    x = x.to(kind)
     state = torch.randn(len(lens), H, V, D, generator=g, device=DEV)
     want_S = state.double()
     o = torch.full((T, H * V), 7.0, device=DEV)
@@ -63,7 +66,7 @@ def run(delta, lens, G, H, D, V, logs, resume=True):
     for s, n, p, r in zip(start, lens, pos, row):
         S = want_S[r] if p else torch.zeros_like(want_S[r])
         for t in range(s, s + n):
-            S = S * torch.exp2(f[t].double())[:, None]
+            S = S * f[t].exp2().double()[:, None]
             u = v[t]
             if delta:
                 b = beta[t, :H].double()[:, None]
@@ -73,11 +76,14 @@ def run(delta, lens, G, H, D, V, logs, resume=True):
         want_S[r] = S
     _check(hy.native().hy_chunk_scan(
         _ptr(o), _ptr(state), _ptr(x), _i(width), _i(qo), _i(ko), _i(vo),
-        _ptr(f), _i(H * D), None if beta is None else _ptr(beta),
+        _ptr(f.exp2()), _i(H * D), None if beta is None else _ptr(beta),
         *(_ptr(t) for t in e), _i(len(lens)), _i(G), _i(H), _i(D), _i(V),
         _f(0.5), _i(int(delta)), _stream()), "hy_chunk_scan")
     close(o.view(T, H, V), want)
     close(state, want_S)
+    for t in reset or ():          # tokens of their own size
+        for n in range(t, t + 3):
+            close(o.view(T, H, V)[n], want[n])
 
 
 @pytest.mark.parametrize("D,V", [(8, 1), (40, 24), (64, 64), (72, 70),
@@ -94,6 +100,15 @@ def test_decays(delta, logs):
     run(delta, [70, 64], 2, 2, 128, 64, logs)
 
 
+@pytest.mark.parametrize("delta", [False, True], ids=["linear", "delta"])
+def test_resets(delta):
+    """What a reset leaves of the state is nothing beside inputs however
+    small: places in a chunk, in a half, quarter and pair of tokens, and the
+    last of one chunk."""
+    run(delta, [70, 64], 2, 2, 128, 64, (0.0, 0.1),
+        reset=[5, 12, 24, 31, 47, 70 + 19, 70 + 40])
+
+
 def test_repeated_keys():
     """Steps that undo each other: L is far from small."""
     D = V = 64
@@ -102,7 +117,7 @@ def test_repeated_keys():
                     generator=torch.Generator(device=DEV).manual_seed(1))
     x[:, :2 * D] = torch.nn.functional.normalize(x[0, :D], dim=0).repeat(2)
     x[:, 2 * D + V] = 1.0
-    f = torch.zeros(T, D, device=DEV)
+    f = torch.ones(T, D, device=DEV)
     o = torch.empty(T, V, device=DEV)
     state = torch.zeros(1, 1, V, D, device=DEV)
     _check(hy.native().hy_chunk_scan(
@@ -148,5 +163,5 @@ def test_state_space(D, V, rate):
         _i(H * V + G * D), _i(H * V), _ptr(dt_in), _i(H), _i(0), _ptr(head),
         *(_ptr(t) for t in e), _i(len(lens)), _i(max(lens)), _i(T), _i(G),
         _i(H), _i(D), _i(V), _stream()), "hy_ssm_chunk")
-    close(o.view(T, H, V), want, FLOATS)
-    close(state, want_S, FLOATS)
+    close(o.view(T, H, V), want)
+    close(state, want_S)
