@@ -16,9 +16,14 @@
 #define ROWS_KEYS 16
 
 // Numbers a row: W of them meet the query's, V from v_off on are values.
-template <int VT, int NW>
+// E: weights are powers of e, not of two (a factor of log2(e) on the queries
+// or the scores would cost their last bits).
+template <int VT, int NW, bool E>
 struct FloatRows {
   static_assert(VT % 4 == 0, "64 columns at a time");
+  static __device__ __forceinline__ float power(float x) {
+    return E ? expf(x) : exp2f(x);
+  }
   // floats of LDS
   static constexpr int maxima = 2 * 16 * NW;
   static __host__ __device__ int pitch(int W) { return (W + 15) / 16 * 16 + 4; }
@@ -27,8 +32,7 @@ struct FloatRows {
     return maxima + (q > o ? q : o);
   }
 
-  // lds: at ``maxima`` the queries [16][pitch], scaled to powers of two,
-  // zeros past W and past the real heads (the caller has waited for them).
+  // lds: at ``maxima`` the queries [16][pitch], scaled, zeros past W and past the real heads (the caller has waited for them).
   //   row(j): where key j's row begins
   // Leaves there the sums of values [16][16 VT + 4] and returns the sum of
   // weights of head n, both relative to the returned maximum; all threads
@@ -48,15 +52,25 @@ struct FloatRows {
     for (int j0 = first + wave * ROWS_KEYS; j0 <= last;
          j0 += NW * ROWS_KEYS) {
       const float* key = row(j0 + n < last ? j0 + n : last);
+      // 128 numbers at a time, in four parts: long sums lose digits
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-      for (int b = 0; b < blocks; ++b) {
-        const int d = b * 16 + g * 4;
-        const f32x4 k = *reinterpret_cast<const f32x4*>(key + (d < W ? d : 0));
-        const f32x4 q = *reinterpret_cast<const f32x4*>(lq + n * KP + d);
+      for (int b0 = 0; b0 < blocks; b0 += 8) {
+        f32x4 part[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], q[i], s, 0, 0, 0);
+        for (int i = 0; i < 4; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int end = b0 + 8 < blocks ? b0 + 8 : blocks;
+#pragma unroll 4
+        for (int b = b0; b < end; ++b) {
+          const int d = b * 16 + g * 4;
+          const f32x4 k =
+              *reinterpret_cast<const f32x4*>(key + (d < W ? d : 0));
+          const f32x4 q = *reinterpret_cast<const f32x4*>(lq + n * KP + d);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i], q[i], part[i],
+                                                           0, 0, 0);
+        }
+        s += (part[0] + part[1]) + (part[2] + part[3]);
       }
       const float* value[4];
       float mx = m;
@@ -69,12 +83,12 @@ struct FloatRows {
       }
       mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
       mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-      const float keep = __builtin_amdgcn_exp2f(m - mx);
+      const float keep = power(m - mx);
       m = mx;
       l *= keep;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        s[i] = __builtin_amdgcn_exp2f(s[i] - m);
+        s[i] = power(s[i] - m);
         l += s[i];
       }
 #pragma unroll
@@ -106,9 +120,8 @@ struct FloatRows {
     float sum = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w)
-      sum += __builtin_amdgcn_exp2f(lds[n * NW + w] - mx) *
-             lds[(16 + n) * NW + w];
-    const float mine = __builtin_amdgcn_exp2f(m - mx);
+      sum += power(lds[n * NW + w] - mx) * lds[(16 + n) * NW + w];
+    const float mine = power(m - mx);
     // register i of products v .. v + 3: columns 16 v + 16 g + 4 i .. + 3
     float* to = lq + n * (16 * VT + 4) + g * 16;
     for (int w = 0; w < NW; ++w) {

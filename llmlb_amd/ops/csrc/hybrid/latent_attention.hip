@@ -198,13 +198,12 @@ void latent_float_kernel(
     const float* __restrict__ cache, const int* __restrict__ pos_,
     const int* __restrict__ row_, const int* __restrict__ bt, int max_blocks,
     int window, float scale, const float* __restrict__ sink, int N) {
-  using F = FloatRows<VT, NW>;
+  using F = FloatRows<VT, NW, true>;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int t = blockIdx.x, h0 = blockIdx.y * 16;
   const int heads = H - h0 < 16 ? H - h0 : 16;
   const int W = rank + R, KP = F::pitch(W), pos = pos_[t];
   const int* pages = bt + (size_t)row_[t] * max_blocks;
-  scale *= LOG2E;
   for (int i = threadIdx.x; i < 16 * KP; i += 64 * NW) {
     const int h = i / KP, d = i - h * KP;
     float x = 0.f;
@@ -227,9 +226,9 @@ void latent_float_kernel(
   if (threadIdx.x < 16) {
     float s = l, f = 1.f;
     if (sink && (int)threadIdx.x < heads) {
-      const float z = sink[h0 + threadIdx.x] * LOG2E, mx = fmaxf(m, z);
-      f = __builtin_amdgcn_exp2f(m - mx);
-      s = s * f + __builtin_amdgcn_exp2f(z - mx);
+      const float z = sink[h0 + threadIdx.x], mx = fmaxf(m, z);
+      f = F::power(m - mx);
+      s = s * f + F::power(z - mx);
     }
     lds[threadIdx.x] = f / s;
   }
@@ -334,7 +333,7 @@ int hy_latent_rows(void* out, const void* qa, const void* proj, int ld, int H,
 #define GO(VT, NW)                                                         \
   hipLaunchKernelGGL(                                                      \
       (latent_float_kernel<VT, NW>), grid, dim3(64 * NW),                  \
-      (FloatRows<VT, NW>::floats(rank + R)) * sizeof(float),               \
+      (FloatRows<VT, NW, true>::floats(rank + R)) * sizeof(float),         \
       (hipStream_t)stream, (float*)out, (const float*)qa,                  \
       (const float*)proj, ld, H, D, R, rank, (const float*)cache,          \
       (const int*)pos, (const int*)row, (const int*)bt, max_blocks,        \

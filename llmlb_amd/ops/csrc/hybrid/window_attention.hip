@@ -72,7 +72,7 @@ void window_float_kernel(
     const int* __restrict__ pos_, const int* __restrict__ row_,
     const int* __restrict__ bt, int max_blocks, int H, int G, int D, int V,
     Mask mask) {
-  using F = FloatRows<VT, NW>;
+  using F = FloatRows<VT, NW, false>;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int t = blockIdx.x, R = H / G, per = (R + 15) / 16;
   const int g = blockIdx.y / per, r0 = blockIdx.y % per * 16;
@@ -249,7 +249,7 @@ int hy_window_rows(void* out, int ld_out, const void* proj, int ld, int g_off,
     const dim3 grid(n_rows, G * per);
 #define GO(VT, NW)                                                           \
   hipLaunchKernelGGL((window_float_kernel<VT, NW>), grid, dim3(64 * NW),     \
-                     (FloatRows<VT, NW>::floats(D)) * sizeof(float),         \
+                     (FloatRows<VT, NW, false>::floats(D)) * sizeof(float),  \
                      (hipStream_t)stream, (float*)out, ld_out,               \
                      (const float*)proj, ld, g_off, (const float*)cache,     \
                      (const int*)pos, (const int*)row, (const int*)bt,       \

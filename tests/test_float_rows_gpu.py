@@ -11,12 +11,19 @@ DEV = "cuda:0"
 F64 = torch.float64
 # rows of up to 1000 keys: sums in float and one exponential's rounding
 TOL = 5e-6
+# All in all: a number passes about sixteen roundings (parts of a score and
+# their sum, scaling, exponential, weights' and values' sums, quotient), each
+# 2^-24 / sqrt(3) off.  That makes 4 / sqrt(3) * 2^-24; not more than 3.
+RMS = 3 * 2.0 ** -24
 PAGES, BLOCKS = 70, 64
 
 
 def close(got, want):
-    err = (got.double() - want).abs().max() / want.abs().max()
+    off = got.double() - want
+    err = off.abs().max() / want.abs().max()
     assert err < TOL, float(err)
+    rms = off.norm() / want.norm()
+    assert rms < RMS, float(rms)
 
 
 def tokens(N, g):
