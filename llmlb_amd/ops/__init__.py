@@ -682,25 +682,34 @@ _ROW_ACTS = {"plain": 0, "relu2": 1, "gelu": 2, "swiglu": 3, "clamped": 4,
              "capped": 5}
 
 
+def _fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether x @ W^T is a product of two matrices.  Kernels see addresses
+    only; what does not fit goes to the library, which says so."""
+    return (x.dim() == weight.dim() == 2 and x.device == weight.device
+            and x.shape[1] == weight.shape[1])
+
+
 def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
               out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
               b: float = 0.0) -> torch.Tensor | None:
     """x @ W^T by row_gemm.hip, or None where it does not take the
-    operands (depth or rows no multiple of 8, unaligned views)."""
+    operands (depth or rows no multiple of 8, unaligned views, what does
+    not fit together)."""
+    if (not _fit(x, weight) or weight.dtype != x.dtype or x.stride(1) != 1
+            or not weight.is_contiguous()):
+        return None
     N, K = x.shape
     M = weight.shape[0]
     gated = act in ("swiglu", "clamped")
-    if (weight.dtype != x.dtype or x.stride(1) != 1
-            or not weight.is_contiguous()):
-        return None
+    kind = torch.float32 if act == "capped" else x.dtype
     if gated:
         M -= up                       # rows of gate and of up
         if up < M:
             return None
     if out is None:
-        out = torch.empty(N, M, device=x.device, dtype=torch.float32
-                          if act == "capped" else x.dtype)
-    elif out.stride(1) != 1 or out.shape != (N, M):
+        out = torch.empty(N, M, device=x.device, dtype=kind)
+    elif (out.shape != (N, M) or out.stride(1) != 1 or out.dtype != kind
+          or out.device != x.device):
         return None
     lib = _require_native()
     src = (_ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight))
@@ -724,7 +733,7 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
 
 def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
-            and x.dim() == 2 and 0 < x.shape[0] <= 128
+            and _fit(x, weight) and 0 < x.shape[0] <= 128
             and not (torch.is_grad_enabled()
                      and (x.requires_grad or weight.requires_grad)))
 

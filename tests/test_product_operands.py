@@ -1,0 +1,59 @@
+"""What products of few rows refuse, and what they leave to the library,
+before a kernel sees an address (no GPU needed: nothing is launched)."""
+import pytest
+import torch
+
+import llmlb_amd.ops as ops
+
+BF16 = torch.bfloat16
+
+
+@pytest.fixture
+def no_launch(monkeypatch):
+    def launched():
+        raise AssertionError("a kernel was about to run")
+    monkeypatch.setattr(ops, "_require_native", launched)
+
+
+def _operands(N=4, M=8, K=64):
+    return torch.ones(N, K, dtype=BF16), torch.ones(M, K, dtype=BF16)
+
+
+@pytest.mark.parametrize("weight", [
+    torch.ones(8, 32, dtype=BF16),                  # less deep than x
+    torch.ones(8, 128, dtype=BF16),                 # deeper
+    torch.ones(64, dtype=BF16),                     # a vector
+    torch.ones(2, 4, 64, dtype=BF16),               # matrices
+    torch.ones(8, 64, dtype=torch.float32),
+    torch.ones(8, 64, dtype=BF16, device="meta"),   # another device
+], ids=["shallow", "deep", "vector", "batch", "type", "device"])
+@pytest.mark.parametrize("act", ["plain", "relu2", "capped"])
+def test_weight_has_to_fit(no_launch, weight, act):
+    x, _ = _operands()
+    assert ops._row_gemm(x, weight, act) is None
+
+
+@pytest.mark.parametrize("act,out", [
+    ("plain", torch.empty(4, 8)),
+    ("relu2", torch.empty(4, 8)),
+    ("capped", torch.empty(4, 8, dtype=BF16)),
+    ("plain", torch.empty(4, 16, dtype=BF16)),
+    ("plain", torch.empty(8, 4, dtype=BF16).T),
+    ("plain", torch.empty(4, 8, dtype=BF16, device="meta")),
+])
+def test_result_has_to_fit(no_launch, act, out):
+    assert ops._row_gemm(*_operands(), act, out) is None
+
+
+@pytest.mark.parametrize("shape", [(8, 32), (8, 128)])
+@pytest.mark.parametrize("mode", ["auto", "1"])
+def test_misfits_raise(no_launch, monkeypatch, shape, mode):
+    """The whole call, for tensors that pass as the GPU's: the library's
+    product refuses them."""
+    x, _ = _operands()
+    monkeypatch.setattr(ops, "_lib", object())
+    monkeypatch.setattr(ops, "_USE_CUSTOM_DECODE_GEMM", mode)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    with pytest.raises(RuntimeError, match="mat1 and mat2|shapes"):
+        ops.linear_decode(x, torch.ones(*shape, dtype=BF16))
+    assert ops.linear_act(x, torch.ones(*shape, dtype=BF16), "gelu") is None
