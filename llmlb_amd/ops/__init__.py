@@ -16,6 +16,7 @@ import os
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 from . import reference
 
@@ -682,6 +683,25 @@ _ROW_ACTS = {"plain": 0, "relu2": 1, "gelu": 2, "swiglu": 3, "clamped": 4,
              "capped": 5}
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _only_numbers(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel that sees the numbers sees all that the library's
+    operation would: nobody asks for gradients or carries tangents, and the
+    tensors are not those of vmap, of a trace or of a subclass."""
+    if (forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (grad and t.requires_grad) or type(t) not in _PLAIN:
+            return False
+    return True
+
+
 def _fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether x @ W^T is a product of two matrices.  Kernels see addresses
     only; what does not fit goes to the library, which says so."""
@@ -732,10 +752,9 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
 
 
 def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
-            and _fit(x, weight) and 0 < x.shape[0] <= 128
-            and not (torch.is_grad_enabled()
-                     and (x.requires_grad or weight.requires_grad)))
+    return (x.is_cuda and _lib is not None and _only_numbers(x, weight)
+            and x.dtype == torch.bfloat16 and _fit(x, weight)
+            and 0 < x.shape[0] <= 128)
 
 
 def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
@@ -919,15 +938,13 @@ def prompt_attn_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     """Whether ``prompt_attention`` runs flash_attention.hip: bf16 heads
     of 64 or 128 on the GPU, rows of a wider matrix or their own."""
     B, Lq, nq, D = q.shape
-    return (q.is_cuda and _lib is not None and q.dtype == torch.bfloat16
-            and k.dtype == v.dtype == q.dtype and D in (64, 128)
+    return (q.is_cuda and _lib is not None and _only_numbers(q, k, v)
+            and q.dtype == torch.bfloat16 and k.dtype == v.dtype == q.dtype
+            and D in (64, 128)
             and nq // k.shape[2] <= 128 and k.stride() == v.stride()
             and all(t.stride(3) == 1 and t.stride(2) == D
                     and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
-                    and t.data_ptr() % 16 == 0 for t in (q, k, v))
-            and not (torch.is_grad_enabled()
-                     and (q.requires_grad or k.requires_grad
-                          or v.requires_grad)))
+                    and t.data_ptr() % 16 == 0 for t in (q, k, v)))
 
 
 def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

@@ -57,3 +57,67 @@ def test_misfits_raise(no_launch, monkeypatch, shape, mode):
     with pytest.raises(RuntimeError, match="mat1 and mat2|shapes"):
         ops.linear_decode(x, torch.ones(*shape, dtype=BF16))
     assert ops.linear_act(x, torch.ones(*shape, dtype=BF16), "gelu") is None
+
+
+def _seen(monkeypatch, call):
+    """Whether the kernels would take what ``call(check)`` hands to check,
+    for tensors that pass as the GPU's."""
+    found = []
+    monkeypatch.setattr(ops, "_lib", object())
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+
+    def check(x, w):
+        h = x.view(-1, 4, 1, 64)
+        found.append((ops._takes_row_gemm(x, w),
+                      ops.prompt_attn_tiled(h, h, h)))
+        return torch.nn.functional.linear(x, w)
+
+    call(check)
+    assert found
+    return {taken for pair in found for taken in pair}
+
+
+X, W = torch.ones(4, 64, dtype=BF16), torch.ones(64, 64, dtype=BF16)
+
+
+def _forward_mode(check):
+    with torch.autograd.forward_ad.dual_level():
+        check(torch.autograd.forward_ad.make_dual(X, X), W)
+
+
+def _fake(check):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode() as mode:
+        check(mode.from_tensor(X), mode.from_tensor(W))
+
+
+def _proxies(check):
+    from torch.fx.experimental.proxy_tensor import make_fx
+    make_fx(check)(X, W)
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("call", [
+    lambda f: torch.vmap(f, (0, None))(X.expand(3, 4, 64), W),
+    lambda f: torch.func.jvp(f, (X, W), (X, W)),
+    lambda f: torch.func.grad(lambda x: f(x, W).float().sum())(X),
+    lambda f: torch.jit.trace(f, (X, W), check_trace=False), _forward_mode, _fake, _proxies,
+    lambda f: f(X.as_subclass(_Sub), W),
+    lambda f: f(X.clone().requires_grad_(), W)],
+    ids=["vmap", "jvp", "grad", "trace", "forward", "fake", "proxies",
+         "subclass", "requires_grad"])
+def test_more_than_numbers_goes_to_the_library(monkeypatch, call):
+    assert _seen(monkeypatch, call) == {False}
+
+
+def test_numbers_go_to_the_kernels(monkeypatch):
+    p = torch.nn.Parameter(W, requires_grad=False)
+    assert _seen(monkeypatch, lambda f: f(X, p)) == {True}
+    with torch.no_grad():
+        assert _seen(monkeypatch, lambda f: f(X, p.requires_grad_())) \
+            == {True}
+    with torch.inference_mode():
+        assert _seen(monkeypatch, lambda f: f(X.clone(), W)) == {True}
