@@ -936,12 +936,17 @@ def paged_attn_decode(q: torch.Tensor, kcache: torch.Tensor,
 def prompt_attn_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
                       ) -> bool:
     """Whether ``prompt_attention`` runs flash_attention.hip: bf16 heads
-    of 64 or 128 on the GPU, rows of a wider matrix or their own."""
+    of 64 or 128 on the GPU, rows of a wider matrix or their own.  What does
+    not fit together goes to the library, which says so."""
     B, Lq, nq, D = q.shape
     return (q.is_cuda and _lib is not None and _only_numbers(q, k, v)
-            and q.dtype == torch.bfloat16 and k.dtype == v.dtype == q.dtype
-            and D in (64, 128)
-            and nq // k.shape[2] <= 128 and k.stride() == v.stride()
+            and q.dtype == k.dtype == v.dtype == torch.bfloat16
+            and q.device == k.device == v.device
+            and k.dim() == 4 and k.shape == v.shape
+            and k.stride() == v.stride()
+            and k.shape[0] == B and k.shape[3] == D and D in (64, 128)
+            and k.shape[1] >= Lq and 0 < k.shape[2] <= nq
+            and nq % k.shape[2] == 0 and nq // k.shape[2] <= 128
             and all(t.stride(3) == 1 and t.stride(2) == D
                     and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
                     and t.data_ptr() % 16 == 0 for t in (q, k, v)))
@@ -954,7 +959,7 @@ def prompt_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     Returns [B * Lq, nq, D], contiguous."""
     B, Lq, nq, D = q.shape
     Lk, nkv = k.shape[1], k.shape[2]
-    if prompt_attn_tiled(q, k, v):
+    if scale > 0 and prompt_attn_tiled(q, k, v):
         out = torch.empty(B * Lq, nq, D, dtype=q.dtype, device=q.device)
         rc = _require_native().ll_prompt_attn(
             _ptr(out), _ptr(q), _ptr(k), _ptr(v),

@@ -121,3 +121,31 @@ def test_numbers_go_to_the_kernels(monkeypatch):
             == {True}
     with torch.inference_mode():
         assert _seen(monkeypatch, lambda f: f(X.clone(), W)) == {True}
+
+
+def _heads(B=2, L=16, n=4, D=64, dtype=BF16, device="cpu"):
+    return torch.ones(B, L, n, D, dtype=dtype, device=device)
+
+
+@pytest.mark.parametrize("k,v", [
+    (_heads(B=1), _heads(B=1)), (_heads(), _heads()[:, :8]),
+    (_heads(), _heads()[:1]), (_heads(D=128), _heads(D=128)),
+    (_heads(n=3), _heads(n=3)), (_heads(n=8), _heads(n=8)),
+    (_heads(L=8), _heads(L=8)), (_heads(dtype=torch.float32),) * 2,
+    (_heads(device="meta"),) * 2],
+    ids=["batch", "tokens of v", "batch of v", "head size", "heads",
+         "more heads", "fewer keys than queries", "type", "device"])
+def test_keys_have_to_fit(no_launch, monkeypatch, k, v):
+    monkeypatch.setattr(ops, "_lib", object())
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    assert ops.prompt_attn_tiled(_heads(), _heads(n=2), _heads(n=2))
+    assert not ops.prompt_attn_tiled(_heads(), k, v)
+
+
+def test_negative_scales_go_to_the_library(no_launch, monkeypatch):
+    q = torch.randn(1, 8, 2, 64).bfloat16()
+    want = ops.prompt_attention(q, q, q, -0.1)
+    monkeypatch.setattr(ops, "_lib", object())
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    assert ops.prompt_attn_tiled(q, q, q)
+    assert torch.equal(ops.prompt_attention(q, q, q, -0.1), want)
