@@ -342,10 +342,15 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(
   // keys as places in the item's key rows, which come in whole 64s
   const int seen_lo = q_pos - window + 1 - k_pos;
   const int w_lo = q_pos + wave * 32 - k_pos, w_hi = w_lo + 31;
+  // a sink as low as numbers go weighs nothing; the loop's arithmetic needs
+  // one that is finite
+  float low = sink ? sink[h] * LOG2E : 0.f;
+  const bool has_sink = sink && !(low < -1e30f);
+  if (!has_sink) low = 0.f;
   f.template run<true>(lds, rows, (seen_lo > 0 ? seen_lo : 0) & ~63,
                        q_pos + n_q - k_pos - 1, pos, span, w_lo, w_hi,
-                       w_lo - window + 1, w_hi - window + 1, scale_log2,
-                       sink ? sink[h] * LOG2E : 0.f, sink != nullptr);
+                       w_lo - window + 1, w_hi - window + 1, scale_log2, low,
+                       has_sink);
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     if (wave * 32 + a * 16 + n >= n_q) continue;

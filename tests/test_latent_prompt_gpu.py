@@ -15,7 +15,7 @@ TOL = 2.0 ** -7
 
 # portions at the start and behind others, edges of 16, 64 and 128 queries
 @pytest.mark.parametrize("window", [1, 50, 200, 2 ** 30])
-@pytest.mark.parametrize("sink", [None, -3.0, 40.0])
+@pytest.mark.parametrize("sink", [None, -3.0, 40.0, -3e38, float("-inf")])
 @pytest.mark.parametrize("H,D,R,V", [(3, 64, 32, 64), (2, 128, 64, 128),
                                      (5, 96, 0, 64), (1, 136, 56, 128)])
 def test_latent_prompt(H, D, R, V, sink, window):
