@@ -901,6 +901,8 @@ def paged_attn_decode(q: torch.Tensor, kcache: torch.Tensor,
     out = torch.empty(S, n_q, D, dtype=q.dtype, device=q.device)
     fp8 = kcache.dtype == torch.uint8
     tiled = paged_attn_tiled(D)
+    if tiled and (q.stride(0) % 8 or q.data_ptr() % 16):
+        q = q.clone(memory_format=torch.contiguous_format)
     assert not fp8 or (tiled and D == 128 and n_q // n_kv <= 16), \
         "FP8 KV requires D=128 and a GQA group <= 16"
     acc_p = ml_p = None

@@ -64,6 +64,21 @@ def test_page_attention(heads, kv, D, parts):
     assert ((out.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("shift,gap", [(4, 0), (0, 4), (1, 3)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_queries_of_any_alignment(D, shift, gap):
+    q, k, v, bt, lens, _ = _case(8, 2, D, 5)
+    k, v = k.bfloat16(), v.bfloat16()
+    n = 8 * D
+    rows = torch.zeros(len(LENS), shift + n + gap, device=DEV).bfloat16()
+    rows[:, shift:shift + n] = q.flatten(1)
+    loose = rows[:, shift:shift + n].unflatten(1, (8, D))
+    assert loose.stride(0) % 8 or loose.data_ptr() % 16
+    want = ops.paged_attn_decode(q, k, v, bt, lens, D ** -0.5)
+    assert torch.equal(
+        ops.paged_attn_decode(loose, k, v, bt, lens, D ** -0.5), want)
+
+
 @pytest.mark.parametrize("parts", [1, 4])
 @pytest.mark.parametrize("heads,kv", [(32, 8), (16, 1)])
 def test_page_attention_fp8(heads, kv, parts):
