@@ -409,13 +409,11 @@ class LlamaForCausalLM(nn.Module):
                 return layer.down.forward(ops.swiglu(gateup)), residual
         normed, residual = ops.rmsnorm(o, layer.post_norm_w,
                                        self.cfg.norm_eps, residual)
-        gate_up = layer.gate_up
-        if not ops._FP8_WEIGHTS and not ops._FUSED_SWIGLU:
-            act = ops.linear_act(normed, gate_up.weight, "swiglu",
-                                 up=gate_up.out_local // 2)
-            if act is not None:
-                return layer.down(act), residual
-        gateup = gate_up(normed)
+        fused = getattr(layer.gate_up, "forward_swiglu", None)
+        act = fused(normed) if fused else None
+        if act is not None:
+            return layer.down.forward(act), residual
+        gateup = layer.gate_up(normed)
         h = layer.down.forward_swiglu(gateup)
         return h, residual
 

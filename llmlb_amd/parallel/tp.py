@@ -126,6 +126,16 @@ class _Fp8WeightMixin:
             return None
 
 
+def _watched(module: nn.Module) -> bool:
+    """Whether calling the module runs hooks."""
+    every = nn.modules.module
+    return bool(
+        module._forward_hooks or module._forward_pre_hooks
+        or module._backward_hooks or module._backward_pre_hooks
+        or every._global_forward_hooks or every._global_forward_pre_hooks
+        or every._global_backward_hooks or every._global_backward_pre_hooks)
+
+
 class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
     """Y = X W^T with W split along the output dim; no communication.
 
@@ -159,6 +169,19 @@ class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
             if y is not None:
                 return y + self.bias if self.bias is not None else y
         return torch.nn.functional.linear(x, self.weight, self.bias)
+
+    def forward_swiglu(self, x: torch.Tensor) -> torch.Tensor | None:
+        """swiglu of the shard's [gate | up] outputs in the product's own
+        launch, or None where calling the module and then swiglu would do
+        something else or more: a bias, hooks, another forward."""
+        from .. import ops as _ops
+        if (self.bias is not None or _ops._FP8_WEIGHTS or _ops._FUSED_SWIGLU
+                or _watched(self)
+                or getattr(self.forward, "__func__", None)
+                is not ColumnParallelLinear.forward):
+            return None
+        return _ops.linear_act(x, self.weight, "swiglu",
+                               up=self.out_local // 2)
 
 
 class RowParallelLinear(nn.Module, _Fp8WeightMixin):
