@@ -267,6 +267,16 @@ extern "C" int ll_row_gemm_split(void* out, int ld_out, const void* x,
   return 0;
 }
 
+// Whether the library's product is the faster one: more than 64 rows read W
+// twice, and of the largest matrices the second time from memory.  us, here
+// and the library, 72, 96, 128 rows: 32000 x 4096 77, 78, 86 and 103, 101,
+// 101; 128256 x 2048 159, 165, 184 and 185, 186, 189; 96000 x 4096 227, 224,
+// 245 and 230, 221, 234; 128256 x 4096 304, 298, 325 and 285, 280, 289; 57344
+// x 8192 298, 256, 274 and 228, 228, 233.
+static bool read_twice(int N, size_t rows, int K) {
+  return N > 64 && rows * K > (384u << 20);
+}
+
 // Rows of x start ldx numbers apart, those of out ld_out.  0: done, -2: not
 // for this kernel.
 extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
@@ -277,8 +287,9 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
       (uintptr_t)out % (kind == CAPPED ? 16 : 8) || kind < PLAIN ||
       kind > CAPPED)
     return -2;
+  const bool gated = kind == SWIGLU || kind == CLAMPED;
+  if (read_twice(N, (size_t)M * (gated ? 2 : 1), K)) return -2;
   const RowGemm p{out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K,
                   ldx, RowAct{kind, up, a, b}, (hipStream_t)stream};
-  return kind == SWIGLU || kind == CLAMPED ? row_gemm_pick<true>(p)
-                                           : row_gemm_pick<false>(p);
+  return gated ? row_gemm_pick<true>(p) : row_gemm_pick<false>(p);
 }

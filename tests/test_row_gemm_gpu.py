@@ -60,6 +60,17 @@ def test_other_operands_go_to_the_library(N, M, K, shift):
     _close(ops.linear_decode(x, w), x, w)
 
 
+def test_largest_matrices_of_many_rows_go_to_the_library():
+    w = torch.randn(98336, 4096, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(65, 4096, device=DEV, dtype=torch.bfloat16)
+    assert ops._row_gemm(x, w) is None
+    assert ops._row_gemm(x, w, "swiglu", up=49168) is None
+    assert ops._row_gemm(x[:64], w) is not None
+    assert ops._row_gemm(x, w[:98304]) is not None
+    assert torch.equal(ops.linear_decode(x, w),
+                       torch.nn.functional.linear(x, w))
+
+
 def test_gradients_keep_the_library():
     x = torch.randn(5, 64, device=DEV, dtype=torch.bfloat16,
                     requires_grad=True)
