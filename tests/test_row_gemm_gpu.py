@@ -23,7 +23,7 @@ def _close(out, x, w):
 # remainder, more pieces than waves; outputs: a remainder of every tile
 @pytest.mark.parametrize("M,K", [(4, 8), (20, 72), (1036, 1024),
                                  (5644, 200), (12300, 1096), (520, 4160)])
-@pytest.mark.parametrize("N", [1, 16, 17, 33, 48, 49, 64, 80, 96, 113, 128])
+@pytest.mark.parametrize("N", [1, 16, 17, 33, 48, 49, 64, 80, 96, 97, 113, 128])
 def test_row_gemm(N, M, K):
     g = torch.Generator(device=DEV).manual_seed(N * 7 + M + K)
     wide = torch.randn(N, K + 16, generator=g, device=DEV).bfloat16()
