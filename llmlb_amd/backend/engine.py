@@ -779,10 +779,11 @@ class Engine:
         Returns the final (h, residual) of the chunk's tokens."""
         dev = self.device
         Ls = L - P
-        # fp8 prefill GEMMs only on P==0 chunks: measured while
-        # continuation chunks ran masked SDPA (as head sizes other than
-        # 64 and 128 still do), whose ~13 GB buffers lose 30%+ wall time with the fp8 path interleaved
-        # (profiles/r02_fp8_prefill_ab.md, same-box 8x6144 A/B)
+        # fp8 prefill GEMMs only on P==0 chunks: continuation chunks lost
+        # 30%+ of their time to the fp8 path beside masked SDPA and its
+        # ~13 GB of buffers (profiles/r02_fp8_prefill_ab.md, same-box
+        # 8x6144 A/B).  Head sizes other than 64 and 128 still take that
+        # SDPA; for those two, which do not, it has not been measured again.
         ops.set_prefill_fp8_ok(P == 0)
         ids = torch.tensor([s.prompt_ids[P:L] for s in group],
                            dtype=torch.long, device=dev).reshape(-1)

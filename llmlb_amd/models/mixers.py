@@ -257,8 +257,11 @@ class DenseFF(nn.Module):
 
     def load(self, w: dict[str, torch.Tensor]) -> None:
         to = dict(dtype=self.dtype, device=self.device)
-        # an uneven depth would keep the staged decode GEMM from the
-        # product down; what is added is zero in both matrices
+        # Rows that do not begin on whole lines of memory cost the product
+        # down up to twice its time (16 rows, 7100 deep 24.8 us, 7168 14.5;
+        # 18312 46.2, 18432 31.8), and prompts' product up gains by whole
+        # 256s (16384 rows, 6784 408 us, 6912 365).  What is added is zero
+        # in both matrices.
         gap = -self.ff % 256 if self.ff >= 4096 else 0
         self.w_up = _param(F.pad(w["up"], (0, 0, 0, gap)).to(**to))
         self.w_down = _param(F.pad(w["down"], (0, gap)).to(**to))

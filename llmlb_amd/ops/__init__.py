@@ -777,11 +777,10 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor,
                   w8: tuple | None = None) -> torch.Tensor:
     """out = x @ W^T for up to 128 rows.
 
-    bf16 products take row_gemm.hip at every size it accepts: with
-    weights from HBM it was faster than hipBLASLt at each of 16 shapes
-    from 1024 x 1024 to 32000 x 4096 and 1 to 64 rows (by 2% at the
-    largest with 64 rows, up to 3.8 times where the library runs a
-    handful of workgroups).  LLMLB_CUSTOM_DECODE_GEMM: "auto" (default)
+    bf16 products take row_gemm.hip at every size it accepts: it is
+    faster than hipBLASLt there (profiles/row_products.md, 1024 x 1024 to
+    128256 x 4096 and 1 to 128 rows: 1.01 to 4.4 times, but 0.94 times
+    for 128 rows of 32000 x 1024).  LLMLB_CUSTOM_DECODE_GEMM: "auto" (default)
     = this, "1"/"on" = the staged kernels of decode_gemm.hip wherever
     they are legal, "0"/"off" = hipBLASLt only."""
     mode = _USE_CUSTOM_DECODE_GEMM

@@ -335,16 +335,6 @@ __global__ void kv_append_kernel(bf16* __restrict__ kcache,
 // fnuz variant is gone), so bytes round-trip exactly with torch's
 // float8_e4m3fn.
 // ---------------------------------------------------------------------------
-typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-
-// one dword of packed e4m3 -> 4 floats (gfx950 native converts)
-__device__ __forceinline__ void fp8x4_to_f32(unsigned int d, float* o) {
-  f32x2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8(d, false);
-  f32x2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8(d, true);
-  o[0] = lo.x; o[1] = lo.y; o[2] = hi.x; o[3] = hi.y;
-}
-
-
 // round-to-nearest-even f32 -> e4m3 byte (input pre-scaled to +-448)
 __device__ __forceinline__ unsigned char f32_to_e4m3(float f) {
   __hip_fp8_e4m3 q(f);

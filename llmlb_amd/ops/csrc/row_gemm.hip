@@ -4,13 +4,15 @@
 //
 // W is read once and nothing else is large, so the bound is memory for big
 // matrices and latency for small ones; hybrid/row_tile.h says how a tile is
-// computed.  Its result needs no second kernel.
+// computed.  Deep matrices of more than 31 rows take the depth in shares, and
+// a second kernel that adds them up.
 //
 // Sizes of a tile are ll_row_gemm's choice.  Against the library's
 // products, us, weights from HBM (N rows: M x K, before -> now):
 //   64: 1024 x 1024 8.8 -> 3.7,  1024 x 2816 9.7 -> 4.7, 2048 x 5632
 //       18.5 -> 11.8, 4096 x 4096 15.5 -> 11.9, 6144 x 4096 17.4 -> 15.9,
-//       4096 x 14336 40.7 -> 36.4, 28672 x 4096 48.9 -> 45.8 (5.1 TB/s)
+//       4096 x 14336 40.7 -> 30.0 (in shares; 36.4 in one), 28672 x 4096
+//       48.9 -> 45.8 (5.1 TB/s)
 //   16: 1024 x 1024 6.1 -> 3.5, 4096 x 4096 15.9 -> 8.2, 28672 x 4096
 //       60.9 -> 37.0 (6.3 TB/s)
 // With more rows the bound is what a compute unit takes in, about 50 GB/s:
@@ -18,9 +20,10 @@
 #include "hybrid/row_tile.h"
 
 // What becomes of a sum before it is stored: a launch less than a kernel of
-// its own, 3 us to 5 in decoding.  The sum is rounded to bf16 first, as it
-// is where that kernel reads it (more than 128 rows): a token's numbers are
-// the same whichever way it comes.  With two matrices, gate and up, a
+// its own, 3 us to 5 in decoding.  The sum is rounded to bf16 first, where it
+// is rounded for that kernel (more than 128 rows).  The order in which it is
+// made differs with the number of rows, as with any product: tiles, waves and
+// shares follow from it.  With two matrices, gate and up, a
 // tile's rows are half of the one and half of the other, at the same
 // outputs.
 enum { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };

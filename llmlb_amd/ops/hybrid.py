@@ -320,7 +320,9 @@ def latent_flash(out, proj, heads, dim, rot, w_uk, w_uv, cache, b, window,
         _ptr(c), _ptr(kr), _ptr(cache), _ptr(blocks), _i(n_blocks), _ptr(bt),
         _i(bt.shape[1]), _i(rank), _i(rot), st), "hy_latent_gather")
     kx = torch.nn.functional.linear(c, w_uk.view(H * dim, rank))
-    # rows of 64 + 32 and 64, 128 + 64 and 128: values as they are expanded
+    # Rows of 64 + 32 and 64, 128 + 64 and 128 (a rotated part of half a
+    # head), values as they are expanded.  The loop would take others whose
+    # rows are 64, 96, 128 or 192 numbers; they have not been measured there.
     if (dim + rot, V) in ((96, 64), (192, 128)) and scale > 0 \
             and (g_off or 0) % 4 == 0:
         vx = torch.nn.functional.linear(c, w_uv.view(H * V, rank))
