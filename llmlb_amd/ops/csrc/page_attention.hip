@@ -265,9 +265,9 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
           reinterpret_cast<const unsigned short*>(
               values + r * VROW + (c ^ turn<VROW>(r)) * 16 + (n & 1) * 8),
           PAGE * D);
-      o[v] = mfma(vf, lo, o[v]);
-      o[v] = mfma(vf, mid, o[v]);
       o[v] = mfma(vf, hi, o[v]);
+      o[v] = mfma(vf, mid, o[v]);
+      o[v] = mfma(vf, lo, o[v]);
     }
     // all has been read before the next copy starts
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
