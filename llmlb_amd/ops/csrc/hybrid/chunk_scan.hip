@@ -28,7 +28,7 @@
 // next ones: the factors, Q and K of them, the inverse.  They meet once a
 // chunk, and a chunk takes about as long as what the waves of one SIMD issue
 // for it.  8 x 2048 tokens, heads of 128 x 128, us, token by token -> now:
-// delta rule, 16 heads, 965 -> 508; gated linear attention, 32 heads, 895
+// delta rule, 16 heads, 973 -> 497; gated linear attention, 32 heads, 889
 // -> 490.
 #include "common.h"
 #include "mfma.h"
@@ -76,17 +76,15 @@ __device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 c) {
   return c;
 }
 
-// c[0 .. 3]: parts of the sum of N products
-template <int N>
-__device__ __forceinline__ void products(const f32x4* a, const f32x4* b,
+// c[0 .. 3] += parts of the sum of four products
+__device__ __forceinline__ void products(const f32x4 (&a)[4], const f32x4* b,
                                          f32x4 (&c)[4]) {
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < N; ++j)
-      c[j & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-          a[j][i], b[j][i], i == 0 && j < 4 ? zero : c[j & 3], 0, 0, 0);
+    for (int j = 0; j < 4; ++j)
+      c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][i], b[j][i], c[j], 0,
+                                                  0, 0);
 }
 
 template <int BYTES, typename To>
@@ -452,10 +450,9 @@ void chunk_scan_kernel(ChunkScan p) {
     fetch(n);
     for (int i = 0; i < chunks + C::LAG - 1; ++i) {
       if (i < chunks) {
-        const typename C::Loads now = x;
-        if (i + 1 < chunks) fetch((i + 1) * CHUNK + n);
-        C::prepare(lds, i, c, n, now, real && i * CHUNK + n < len,
+        C::prepare(lds, i, c, n, x, real && i * CHUNK + n < len,
                    D == DB && (i + 1) * CHUNK <= len);
+        fetch((i + 1) * CHUNK + n);
       }
       __syncthreads();
     }
@@ -499,41 +496,51 @@ void chunk_scan_kernel(ChunkScan p) {
     for (int x = 0; x < 4; ++x) u[x] = to_f(vn[x]);
     fetch((i + 1) * CHUNK);
 
-    // sums in four parts, so that no product waits for the one before
+    // Sums in four parts, so that no product waits for the one before;
+    // operands of four products at a time, as more of them do not fit the
+    // registers (and what is spilled waits for all loads on their way).
     constexpr int N = DB / 16;
-    f32x4 x[N], o[4];
-    if constexpr (DELTA) {
-      f32x4 w[4];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 x[4], o[4];
+    auto with_state = [&](const char* rows) {
 #pragma unroll
-      for (int a = 0; a < N; ++a) x[a] = C::piece(own + C::KT, n, 4 * a + g);
-      products<N>(x, S, w);
+      for (int j = 0; j < 4; ++j) o[j] = zero;
+#pragma unroll
+      for (int a = 0; a < N; a += 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = C::piece(rows, n, 4 * (a + j) + g);
+        products(x, S + a, o);
+      }
+    };
+    if constexpr (DELTA) {
+      with_state(own + C::KT);
       u = mfma4(*reinterpret_cast<const f32x4*>(
                     lds + C::INV + (i & 1) * 1024 + C::element(n, 4 * g)),
-                u - ((w[0] + w[1]) + (w[2] + w[3])),
-                f32x4{0.f, 0.f, 0.f, 0.f});
+                u - ((o[0] + o[1]) + (o[2] + o[3])), zero);
     }
-#pragma unroll
-    for (int a = 0; a < N; ++a) x[a] = C::piece(own + C::QT, n, 4 * a + g);
-    products<N>(x, S, o);
+    with_state(own + C::QT);
     const f32x4 m = *reinterpret_cast<const f32x4*>(q);
     const float* end =
         reinterpret_cast<const float*>(lds + C::END) + place * DB;
 #pragma unroll
-    for (int a = 0; a < N; ++a)
-      x[a] = *reinterpret_cast<const f32x4*>(own + C::KH +
-                                             C::column(16 * a + n, g));
-#pragma unroll
     for (int r = 0; r < 4; ++r)
       o[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], u[r], o[r], 0, 0, 0);
 #pragma unroll
-    for (int a = 0; a < N; ++a)
-      S[a] *= *reinterpret_cast<const f32x4*>(end + a * 16 + g * 4);
+    for (int a = 0; a < N; a += 4) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int j = 0; j < 4; ++j) {
+        x[j] = *reinterpret_cast<const f32x4*>(
+            own + C::KH + C::column(16 * (a + j) + n, g));
+        S[a + j] *=
+            *reinterpret_cast<const f32x4*>(end + (a + j) * 16 + g * 4);
+      }
 #pragma unroll
-      for (int a = 0; a < N; ++a)
-        S[a] =
-            __builtin_amdgcn_mfma_f32_16x16x4f32(x[a][r], u[r], S[a], 0, 0, 0);
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          S[a + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j][r], u[r],
+                                                          S[a + j], 0, 0, 0);
+    }
     const f32x4 sum = (o[0] + o[1]) + (o[2] + o[3]);
     // Lanes without a column of their own repeat the last one and store the
     // same.  Only the last chunk asks which tokens there are: what may or

@@ -351,13 +351,14 @@ def by_chunks(b, tokens=12, heads=48) -> bool:
     cost one by one.  32 heads of 128 x 128, us, Mamba-2 (12): 64 portions
     of 1 token 76 (one by one 44), of 4 75 (51), of 16 78 (87), 8 portions
     of 2048 215 (1119); gated linear attention (16): 64 portions of 8
-    tokens 65 (53), of 16 67 (78), 8 of 2048 490 (895); delta rule (32): 64
-    of 16 87 (93), of 32 148 (196), 8 of 2048 710 (1259).
+    tokens 63 (53), of 16 65 (77), 8 of 2048 490 (889); delta rule (32): 64
+    of 16 85 (95; with heads of 64 45, 30), of 32 129 (197), 8 of 2048 663
+    (1273).
 
     The delta rule's chunks are also a longer chain than its tokens, and
     gain only where those share compute units, from about 48 ``heads`` of
-    portions on: 1 x 300 tokens, 16 heads 65 (50), 2 x 300, 16 heads 66
-    (61), 3 x 517, 16 heads 111 (163), 2 x 300, 32 heads 66 (80)."""
+    portions on: 1 x 300 tokens, 16 heads 64 (50), 2 x 300, 16 heads 64
+    (60), 3 x 517, 16 heads 108 (162), 2 x 300, 32 heads 65 (80)."""
     lens = [n for _, n, _, _ in b.entries]
     return (max(lens, default=0) >= 64 or b.n_tok >= tokens * len(lens)) \
         and heads * sum(n >= tokens for n in lens) >= 48
