@@ -19,8 +19,8 @@
 // them is as good as one float, and a step's decay is no less than 2^-160,
 // which as a float is zero all the same.
 // Scanned token by token, a head's 64 tokens wait for each other: 8 x 2048
-// tokens of 32 heads, 128 x 128 each, took 1173 us, in chunks
-// 202.
+// tokens of 32 heads, 128 x 128 each, took 1173 us, in chunks 245 (200 with
+// two parts of each float, see below).
 //
 // q, k and v are bf16 as projected.  What is float, the weights of s and the
 // state, enters a product as a sum of bf16 numbers: of two in the matrix

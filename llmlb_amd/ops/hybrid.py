@@ -345,15 +345,14 @@ def _runs(b):
             _i(len(b.entries)))
 
 
-def by_chunks(b, tokens=12, heads=48) -> bool:
+def by_chunks(b, tokens=16, heads=48) -> bool:
     """Whether recurrences of the batch go by chunks of tokens on the
     matrix cores (bf16 models): a chunk costs about what ``tokens`` tokens
-    cost one by one.  32 heads of 128 x 128, us, Mamba-2 (12): 64 portions
-    of 1 token 76 (one by one 44), of 4 75 (51), of 16 78 (87), 8 portions
-    of 2048 215 (1119); gated linear attention (16): 64 portions of 8
-    tokens 63 (53), of 16 65 (77), 8 of 2048 490 (889); delta rule (32): 64
-    of 16 85 (95; with heads of 64 45, 30), of 32 129 (197), 8 of 2048 663
-    (1273).
+    cost one by one.  32 heads of 128 x 128, us, Mamba-2: 64 portions of 8
+    tokens 71 (one by one 57), of 16 72 (88), 8 portions of 2048 243 (1058);
+    gated linear attention: 64 portions of 8 tokens 63 (53), of 16 65 (77),
+    8 of 2048 490 (889); delta rule (32): 64 of 16 85 (95; with heads of 64
+    45, 30), of 32 129 (197), 8 of 2048 663 (1273).
 
     The delta rule's chunks are also a longer chain than its tokens, and
     gain only where those share compute units, from about 48 ``heads`` of
@@ -536,7 +535,7 @@ def gated_linear(out, proj, k_off, v_off, g_off, dec, dec_bias, state, b,
         return
     g = torch.empty(T, H * D, dtype=torch.float32, device=proj.device)
     o = torch.empty(T, H * V, dtype=torch.float32, device=proj.device)
-    chunks = by_chunks(b, 16) and can_chunk_scan(proj.dtype, D) \
+    chunks = by_chunks(b) and can_chunk_scan(proj.dtype, D) \
         and proj.stride(0) % 8 == 0 and k_off % 8 == 0 \
         and proj.data_ptr() % 16 == 0
     _check(lib.hy_gla_decay(
