@@ -119,8 +119,9 @@ def test_forward_dense_embeddings_gpu():
 
 def test_multichunk_prefill_and_cached_prefix_gpu():
     """Exercise the P>0 prefill branch on GPU: (a) a prompt longer
-    than prefill_chunk runs in chunks (chunk 2+ takes the
-    repeated-KV fused masked SDPA — engine.py _prefill_chunk), and
+    than prefill_chunk runs in chunks (chunk 2+ takes, at this model's
+    heads of 32, the repeated-KV fused masked SDPA — engine.py
+    _prefill_chunk; heads of 64 and 128: test_prefill_chunks_gpu.py), and
     (b) a re-submitted prompt reuses cached prefix pages (cached_len
     > 0, same branch).  Determinism across identical runs is also
     asserted (greedy, fixed seed)."""

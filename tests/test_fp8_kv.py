@@ -88,7 +88,7 @@ def test_fp8_append_and_attention_gpu():
 def test_fp8_engine_gpu_decode():
     """End-to-end fp8-KV engine on GPU: greedy decode runs through the
     fp8 kernels (graphs on) and stays close to the bf16-KV engine."""
-    # fp8 KV needs D=128 / group<=4 on GPU (the v2 attention shape)
+    # fp8 KV needs heads of 128 on GPU, up to 16 to a key/value head
     cfg = LlamaConfig(hidden=512, layers=4, q_heads=4, kv_heads=2,
                       head_dim=128, inter=1024, vocab=4096, max_pos=1024,
                       name="fp8-test")
@@ -182,8 +182,8 @@ def test_fp8_with_prefix_and_spec_cpu():
 
 @pytest.mark.gpu
 def test_fp8_group8_engine_gpu():
-    """fp8 KV with GQA group 8 (the 70B shape): exercises the two-pass
-    v2 fp8 attention end to end."""
+    """fp8 KV with GQA group 8 (the 70B shape): the tiled attention's
+    8-bit pages end to end."""
     from llmlb_amd.backend.engine import Engine, EngineConfig
     from llmlb_amd.backend.sampler import SamplingParams
     from llmlb_amd.models.llama import LlamaConfig

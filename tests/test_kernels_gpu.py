@@ -243,8 +243,8 @@ def test_swiglu_linear_fused():
 
 @pytest.mark.gpu
 def test_paged_attn_v2_group8():
-    """GQA group 8 (the 70B shape) runs through the v2 kernel as two
-    offset GROUP=4 passes; must match the fp32 reference."""
+    """GQA group 8 (the 70B shape): half of a tile's 16 heads; must match
+    the fp32 reference."""
     torch.manual_seed(6)
     dev = "cuda:0"
     S, nq, nkv, D, BS, nb = 4, 16, 2, 128, 16, 12
