@@ -709,20 +709,16 @@ def _fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and x.shape[1] == weight.shape[1])
 
 
-def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
-              out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
-              b: float = 0.0) -> torch.Tensor | None:
-    """x @ W^T by row_gemm.hip, or None where it does not take the
-    operands (depth or rows no multiple of 8, unaligned views, what does
-    not fit together)."""
+def _product_of(x: torch.Tensor, weight: torch.Tensor, act: str,
+                out: torch.Tensor | None, up: int):
+    """(outputs a row, result) of a product with an activation, or None
+    where the operands or ``out`` do not fit."""
     if (not _fit(x, weight) or weight.dtype != x.dtype or x.stride(1) != 1
             or not weight.is_contiguous()):
         return None
-    N, K = x.shape
-    M = weight.shape[0]
-    gated = act in ("swiglu", "clamped")
+    N, M = x.shape[0], weight.shape[0]
     kind = torch.float32 if act == "capped" else x.dtype
-    if gated:
+    if act in ("swiglu", "clamped"):
         M -= up                       # rows of gate and of up
         if up < M:
             return None
@@ -731,6 +727,19 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     elif (out.shape != (N, M) or out.stride(1) != 1 or out.dtype != kind
           or out.device != x.device):
         return None
+    return M, out
+
+
+def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
+              out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
+              b: float = 0.0) -> torch.Tensor | None:
+    """x @ W^T by row_gemm.hip, or None where it does not take the
+    operands (depth or rows no multiple of 8, unaligned views, what does
+    not fit together)."""
+    found = _product_of(x, weight, act, out, up)
+    if found is None:
+        return None
+    (M, out), (N, K) = found, x.shape
     lib = _require_native()
     src = (_ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight))
     sizes = (ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
@@ -751,26 +760,55 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     return out
 
 
-def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str,
+               out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
+               b: float = 0.0) -> torch.Tensor | None:
+    """act(x @ W^T) by tile_gemm.hip, or None where it does not take the
+    operands or the library's product and a kernel of the activation's own
+    are the faster."""
+    if not _require_native().ll_tile_gemm_gains(
+            ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0])):
+        return None
+    found = _product_of(x, weight, act, out, up)
+    if found is None:
+        return None
+    M, out = found
+    rc = _require_native().ll_tile_gemm(
+        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
+        ctypes.c_int(x.shape[0]), ctypes.c_int(M), ctypes.c_int(x.shape[1]),
+        ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
+        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "ll_tile_gemm")
+    return out
+
+
+def _takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return (x.is_cuda and _lib is not None and _only_numbers(x, weight)
             and x.dtype == torch.bfloat16 and _fit(x, weight)
-            and 0 < x.shape[0] <= 128)
+            and x.shape[0] > 0)
+
+
+def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return _takes_product(x, weight) and x.shape[0] <= 128
 
 
 def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
                out: torch.Tensor | None = None, up: int = 0,
                a: float = 0.0, b: float = 0.0) -> torch.Tensor | None:
-    """act(x @ W^T) of up to 128 bf16 rows in one launch, into ``out``
-    (columns of wider rows) if given; None where row_gemm.hip does not
-    take it.
+    """act(x @ W^T) of bf16 rows in one launch, into ``out`` (columns of
+    wider rows) if given; None where neither row_gemm.hip (up to 128 rows)
+    nor tile_gemm.hip takes it.
 
     act: "relu2", "gelu" (its tanh form), "capped" (float32,
     a tanh(z / a); a = 0: a widening); with gate in the first rows of
     ``weight`` and up from row ``up`` on "swiglu", and "clamped" with
     limit a and sharpness b (see hybrid.clamped_swiglu)."""
-    if _USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight):
+    if _USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_product(x, weight):
         return None
-    return _row_gemm(x, weight, act, out, up, a, b)
+    product = _row_gemm if x.shape[0] <= 128 else _tile_gemm
+    return product(x, weight, act, out, up, a, b)
 
 
 def linear_decode(x: torch.Tensor, weight: torch.Tensor,

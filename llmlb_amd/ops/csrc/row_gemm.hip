@@ -18,37 +18,12 @@
 // With more rows the bound is what a compute unit takes in, about 50 GB/s:
 // every tile reads all of its x and W.
 #include "hybrid/row_tile.h"
+#include "row_act.h"
 
-// What becomes of a sum before it is stored: a launch less than a kernel of
-// its own, 3 us to 5 in decoding.  The sum is rounded to bf16 first, where it
-// is rounded for that kernel (more than 128 rows).  The order in which it is
-// made differs with the number of rows, as with any product: tiles, waves and
-// shares follow from it.  With two matrices, gate and up, a
+// The order in which a sum is made differs with the number of rows, as with
+// any product: tiles, waves and shares follow from it.  With gate and up, a
 // tile's rows are half of the one and half of the other, at the same
 // outputs.
-enum { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };
-struct RowAct {
-  int kind;
-  int up;      // SWIGLU, CLAMPED: the first row of up
-  float a, b;  // CLAMPED: limit, sharpness; CAPPED: cap (0: none)
-};
-__device__ __forceinline__ float row_act(const RowAct& act, float z) {
-  if (act.kind == RELU2) {
-    z = fmaxf(z, 0.f);
-    return z * z;
-  }
-  if (act.kind == GELU) return gelu_tanh_fast(z);
-  if (act.kind == CAPPED && act.a > 0.f) return act.a * tanhf(z / act.a);
-  return z;
-}
-__device__ __forceinline__ float row_gate(const RowAct& act, float g,
-                                          float u) {
-  if (act.kind == SWIGLU) return g / (1.f + __expf(-g)) * u;
-  g = fminf(g, act.a);
-  u = fminf(fmaxf(u, -act.a), act.a);
-  return g / (1.f + __expf(-act.b * g)) * (u + 1.f);
-}
-
 // M outputs; CAPPED results are floats, all others bf16
 template <int NT, int MT, int KW, int S, bool GATED>
 __global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(

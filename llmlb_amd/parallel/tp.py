@@ -173,9 +173,11 @@ class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
     def forward_swiglu(self, x: torch.Tensor) -> torch.Tensor | None:
         """swiglu of the shard's [gate | up] outputs in the product's own
         launch, or None where calling the module and then swiglu would do
-        something else or more: a bias, hooks, another forward."""
+        something else or more: a bias, hooks, another forward, prompts
+        with 8-bit weights."""
         from .. import ops as _ops
         if (self.bias is not None or _ops._FP8_WEIGHTS or _ops._FUSED_SWIGLU
+                or (x.shape[0] > 128 and _ops.fp8_prefill_active())
                 or _watched(self)
                 or getattr(self.forward, "__func__", None)
                 is not ColumnParallelLinear.forward):

@@ -1,0 +1,92 @@
+"""Products of many rows with an activation (tile_gemm.hip) against float
+products of the same numbers, at the edges of its tiles."""
+import pytest
+import torch
+
+import llmlb_amd.ops as ops
+from test_row_gemm_gpu import DEV, _act
+
+pytestmark = pytest.mark.gpu
+
+
+def _tiled(x, w, act, out, up, a, b, monkeypatch):
+    """The kernel at sizes at which the library would be the faster."""
+    monkeypatch.setattr(ops._lib, "ll_tile_gemm_gains", lambda n, m: 1)
+    return ops.linear_act(x, w, act, out, up, a, b)
+
+
+# one tile, edges of rows and outputs, several tiles a workgroup (2100 rows
+# of 9000 outputs are 324 to 639 tiles); depths of one step to three
+@pytest.mark.parametrize("act,a,b", [("relu2", 0, 0), ("gelu", 0, 0),
+                                     ("swiglu", 0, 0), ("clamped", 1.5, 1.7)])
+@pytest.mark.parametrize("N,M,K", [(129, 8, 64), (256, 256, 128),
+                                   (300, 1160, 192), (513, 520, 1024),
+                                   (2100, 9000, 64), (2100, 9000, 192),
+                                   (1000, 16392, 128)])
+def test_tile_gemm(N, M, K, act, a, b, monkeypatch):
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(N, K + 16, generator=g, device=DEV).bfloat16()[:, 8:8 + K]
+    up = M if act in ("swiglu", "clamped") else 0
+    w = torch.randn(M + up, K, generator=g, device=DEV).mul_(
+        K ** -0.5).bfloat16()
+    z = x.double() @ w.double().T
+    ref = _act(act, z.bfloat16().double(), up, a, b)
+    wide = torch.full((N, M + 16), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = _tiled(x, w, act, wide[:, 8:8 + M], up, a, b, monkeypatch)
+    # as for few rows: sums near the middle of two bf16 numbers may take
+    # the other one, which an activation makes at most 60 times larger
+    off = (x.double().abs() @ w.double().abs().T).amax() * K * 2.0 ** -24
+    apart = (z - off).bfloat16() != (z + off).bfloat16()
+    if up:
+        apart = apart[:, :up] | apart[:, up:]
+    bound = ref.abs() * (2.0 ** -20 + 2.0 ** -8) + 1e-30 \
+        + apart * 60 * z.abs().amax() * 2.0 ** -8
+    assert ((out.double() - ref).abs() <= bound).all()
+    assert (wide[:, :8] == 7).all() and (wide[:, 8 + M:] == 7).all()
+
+
+@pytest.mark.parametrize("act", ["gelu", "swiglu"])
+def test_infinities_and_nan(act, monkeypatch):
+    """What the activation of the library's product makes of them."""
+    x = torch.zeros(256, 64, device=DEV, dtype=torch.bfloat16)
+    x[:, 0] = 1.0
+    special = torch.tensor([float("inf"), -float("inf"), float("nan"), 3e38,
+                            -3e38, -90.0, 90.0, 0.0], device=DEV)
+    w = torch.zeros(16, 64, device=DEV, dtype=torch.bfloat16)
+    w[:, 0] = torch.cat([special, torch.ones_like(special)])
+    up = 8 if act == "swiglu" else 0
+    out = _tiled(x, w, act, None, up, 0, 0, monkeypatch)
+    # zeros times the special numbers are in no sum: the column has one
+    z = (x.float()[:, :1] * w.float()[:, 0]).bfloat16()
+    ref = _act(act, z.double(), up, 0, 0)
+    mine = out.double()
+    assert torch.equal(mine.isnan(), ref.isnan())
+    seen = ~ref.isnan()
+    torch.testing.assert_close(mine[seen], ref[seen], rtol=2 ** -7,
+                               atol=1e-30)
+
+
+@pytest.mark.parametrize("N,M,K,shift", [(300, 12, 64, 0), (300, 64, 72, 0),
+                                         (300, 64, 64, 4)])
+def test_other_operands_go_to_the_library(N, M, K, shift, monkeypatch):
+    x = torch.randn(N, K + 8, device=DEV).bfloat16()[:, shift:shift + K]
+    w = torch.randn(M, K, device=DEV).bfloat16()
+    assert _tiled(x, w, "gelu", None, 0, 0, 0, monkeypatch) is None
+
+
+def test_capture():
+    """Replays give what an eager call gives."""
+    x = torch.randn(2048, 256, device=DEV).bfloat16()
+    w = torch.randn(8192, 256, device=DEV).mul_(0.06).bfloat16()
+    want = ops.linear_act(x, w, "gelu")
+    assert want is not None
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = ops.linear_act(x, w, "gelu")
+    for i in range(3):
+        x.add_(1.0)
+        want = ops.linear_act(x, w, "gelu")
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i
