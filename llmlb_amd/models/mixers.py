@@ -22,13 +22,13 @@ import torch.nn.functional as F
 
 from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
-from ..ops import linear_act, linear_decode
+from ..ops import linear_act, linear_decode, linear_rows
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
 
 def _linear(x, w):
-    return linear_decode(x, w) if x.shape[0] <= 128 else F.linear(x, w)
+    return linear_decode(x, w) if x.shape[0] <= 128 else linear_rows(x, w)
 
 
 def _param(t):

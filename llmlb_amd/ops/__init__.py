@@ -760,14 +760,15 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     return out
 
 
-def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str,
+def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
                out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
-               b: float = 0.0) -> torch.Tensor | None:
+               b: float = 0.0, tile: int = -1) -> torch.Tensor | None:
     """act(x @ W^T) by tile_gemm.hip, or None where it does not take the
-    operands or the library's product and a kernel of the activation's own
-    are the faster."""
-    if not _require_native().ll_tile_gemm_gains(
-            ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0])):
+    operands, or the library's product and a kernel of the activation's own
+    are the faster.  ``tile``: one of the kernel's, -1: its choice."""
+    if act == "capped" or not _require_native().ll_tile_gemm_gains(
+            ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0]),
+            ctypes.c_int(x.shape[1]), ctypes.c_int(_ROW_ACTS[act])):
         return None
     found = _product_of(x, weight, act, out, up)
     if found is None:
@@ -777,7 +778,8 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str,
         _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
         ctypes.c_int(x.shape[0]), ctypes.c_int(M), ctypes.c_int(x.shape[1]),
         ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
-        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b), _stream())
+        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b),
+        ctypes.c_int(tile), _stream())
     if rc == -2:
         return None
     _check(rc, "ll_tile_gemm")
@@ -842,6 +844,15 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor,
                 pass
         return torch.nn.functional.linear(x, weight)
     out = _row_gemm(x, weight)
+    return torch.nn.functional.linear(x, weight) if out is None else out
+
+
+def linear_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """out = x @ W^T for more rows than a decode step has: prompts."""
+    out = None
+    if (_USE_CUSTOM_DECODE_GEMM == "auto" and _takes_product(x, weight)
+            and x.shape[0] > 128):
+        out = _tile_gemm(x, weight)
     return torch.nn.functional.linear(x, weight) if out is None else out
 
 

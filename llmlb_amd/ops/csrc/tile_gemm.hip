@@ -28,22 +28,23 @@ constexpr int DEPTH = 64;  // of a step: a row's part is a line of memory
 // Workgroup: tiles of BM rows of x and BN rows of W, by WM x WN waves, one
 // after the other.
 //
-// LDS is a ring of five units, in turn a step's rows of x and of W.  A step
-// is computed in two halves of 32 of its depth; while one is multiplied, the
-// operands of the next are read, each into the registers of one that is no
-// longer needed (W's, which all of a wave's rows need, have two sets).  The
-// step's only barrier stands BP groups of products into its second half:
-// past it every wave has read all of the step, whose place the next copies
-// take, and the step after is there.  Rows of x are on their way for one and
-// a half steps then, those of W for one; a tile's first steps are fetched
-// while the last of the one before is computed, and its results are stored
-// while the next one is.
+// LDS holds D steps of W's rows and D + 1 of x's.  A step is computed in two
+// halves of 32 of its depth; while one is multiplied, the operands of the
+// next are read, each into the registers of one that is no longer needed
+// (W's, which all of a wave's rows need, have two sets).  The step's only
+// barrier stands BP groups of products into its second half: past it every
+// wave has read all of the step, whose places the next copies take, and the
+// step after is there.  Rows of x are on their way for D - 1/2 steps then,
+// those of W for D - 1: small tiles, whose steps are short, need more (48
+// tiles of 128 x 128: 0.74 us a step with D = 2, 0.43 with 4).  A tile's first
+// steps are fetched while the last of the one before are computed, and its
+// results are stored while the next one is.
 //
 // LDS rows are 8 pieces of 16 bytes; piece c of row r lies at c ^ swizzle(r),
 // so that lanes reading one piece of the rows of an operand meet different
 // banks.  W's rows enter the matrix cores in an order in which a lane gets 8
 // consecutive outputs of each of its rows.
-template <int BM, int BN, int WM, int WN, int KIND>
+template <int BM, int BN, int WM, int WN, int D, int KIND>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
 void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
                       const bf16_t* __restrict__ x,
@@ -56,9 +57,10 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
   constexpr int OUT = GATED ? BN / 2 : BN;             // outputs a tile
   constexpr int GROUPS = GATED ? TW / 4 : TW / 2;      // of 32 outputs
   constexpr int STORES = GROUPS * TX;
-  constexpr int UNIT = (BM > BN ? BM : BN) * DEPTH;
-  constexpr int BP = TX / 4;
-  static_assert(GROUPS >= 1, "a wave's outputs");
+  constexpr int UX = BM * DEPTH, UW = BN * DEPTH;      // a step's rows
+  constexpr int BP = TX < 8 ? 1 : 2;
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole copies");
+  static_assert(GROUPS >= 1 && D >= 2, "a wave's outputs, steps ahead");
   extern __shared__ __align__(1024) unsigned short lds[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -84,7 +86,7 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
   // -- copies: tile and depth they are at, the lane's offsets in bytes
   unsigned xo[CX], wo[CW];
   const bf16_t* xt;
-  int xk = 0, wk = 0, x_tile = tile, w_tile = tile, to = 0;
+  int xk = 0, wk = 0, x_tile = tile, w_tile = tile, to_x = 0, to_w = 0;
   auto aim_x = [&] {
     int n0, m0;
     place(x_tile, n0, m0);
@@ -111,18 +113,21 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
       wo[i] = ((unsigned)row * (unsigned)K + c) * 2;
     }
   };
-  auto next = [](int unit) { return unit == 4 ? 0 : unit + 1; };
+  auto next_x = [](int u) { return u == D ? 0 : u + 1; };
+  auto next_w = [](int u) { return u == D - 1 ? 0 : u + 1; };
   const unsigned base = lds_byte(lds);
   auto copy_x = [&](int i) {
-    copy_to_lds(xt + xk, xo[i], base + to * UNIT * 2 + (wave * CX + i) * 1024);
+    copy_to_lds(xt + xk, xo[i], base + to_x * UX * 2 + (wave * CX + i) * 1024);
   };
   auto copy_w = [&](int i) {
-    copy_to_lds(w + wk, wo[i], base + to * UNIT * 2 + (wave * CW + i) * 1024);
+    copy_to_lds(w + wk, wo[i],
+                base + ((D + 1) * UX + to_w * UW) * 2 +
+                    (wave * CW + i) * 1024);
   };
   // past the last tile its beginning is copied again: every step has as
   // many copies
   auto step_x = [&] {
-    to = next(to);
+    to_x = next_x(to_x);
     if ((xk += DEPTH) < K) return;
     xk = 0;
     if (x_tile + slots < end) {
@@ -131,7 +136,7 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
     }
   };
   auto step_w = [&] {
-    to = next(to);
+    to_w = next_w(to_w);
     if ((wk += DEPTH) < K) return;
     wk = 0;
     if (w_tile + slots < end) {
@@ -142,7 +147,7 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
   aim_x();
   aim_w();
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
+  for (int s = 0; s < D; ++s) {
 #pragma unroll
     for (int i = 0; i < CX; ++i) copy_x(i);
     step_x();
@@ -158,12 +163,13 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
   const int sx = swizzle_x(rx), sw = swizzle_w(rw);
   u32x4 fx[TX], fw[2][TW];
   f32x4 acc[TX][TW];
-  int ux = 0, uw = 1;  // the step's units
+  int ux = 0, uw = 0;  // where the step lies
   auto at_x = [&](int half) {
-    return lds + ux * UNIT + rx * DEPTH + ((half * 4 + g) ^ sx) * 8;
+    return lds + ux * UX + rx * DEPTH + ((half * 4 + g) ^ sx) * 8;
   };
   auto at_w = [&](int half) {
-    return lds + uw * UNIT + rw * DEPTH + ((half * 4 + g) ^ sw) * 8;
+    return lds + (D + 1) * UX + uw * UW + rw * DEPTH +
+           ((half * 4 + g) ^ sw) * 8;
   };
   auto read_x = [&](const unsigned short* p, int i) {
     fx[i] = *reinterpret_cast<const u32x4*>(p + i * 16 * DEPTH);
@@ -187,12 +193,16 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
       }
       times<TW>([&](auto IB) {
         constexpr int i = IB, b = a % 2 ? TW - 1 - i : i;
+        // W's reads: every second product, or where groups are few all
+        constexpr int LEFT = (TW + TX - first - 1) / (TX - first);
+        constexpr int RW = LEFT > TW / 2 ? LEFT : TW / 2;
+        constexpr int IS = RW > TW / 2 ? i : (i % 2 ? i / 2 : RW);
         acc[a][b] = mfma(fw[h][b], fx[a], acc[a][b]);
         if constexpr (i == 0 && a == 0) read_x(px, TX - 1);
         if constexpr (i == 0 && a > first) read_x(nx, a - 1);
         if constexpr (h && a == BP && i < BP) read_x(nx, i);
-        if constexpr (a >= first && a < first + 2 && i % 2 == 1)
-          read_w(h ^ 1, nw, (a - first) * (TW / 2) + i / 2);
+        if constexpr (a >= first && IS < RW && (a - first) * RW + IS < TW)
+          read_w(h ^ 1, nw, (a - first) * RW + IS);
         if constexpr (a >= first && i == 2 % TW)
           times<PER>([&](auto IC) {
             constexpr int c = (a - first) * PER + IC;
@@ -209,7 +219,7 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
   constexpr std::integral_constant<int, 1> H1{};
 
   bool stored = false;  // STORES of each wave's may be under way
-  wait_barrier<CX + CW>();
+  wait_barrier<(D - 1) * (CX + CW)>();
 #pragma unroll
   for (int b = 0; b < TW; ++b) read_w(0, at_w(0), b);
 #pragma unroll
@@ -224,12 +234,13 @@ void tile_gemm_kernel(bf16_t* __restrict__ out, int ld_out,
       half(H0, [] {});
       step_x();
       half(H1, [&] {
-        // all but the copies of this step's first half, and what a tile
-        // before its first step has stored
-        if (s == 0 && stored) wait_barrier<CX + STORES>();
-        else wait_barrier<CX>();
-        ux = next(uw);
-        uw = next(ux);
+        // all but the copies of the steps past the next one, and what the
+        // tile before stored behind the next one's
+        constexpr int COPIES = (D - 2) * (CX + CW) + CX;
+        if (s < (D - 1) * DEPTH && stored) wait_barrier<COPIES + STORES>();
+        else wait_barrier<COPIES>();
+        ux = next_x(ux);
+        uw = next_w(uw);
       });
       step_w();
     } while ((s += DEPTH) < K);
@@ -283,10 +294,10 @@ struct TileGemm {
   hipStream_t stream;
 };
 
-template <int BM, int BN, int WM, int WN, int KIND>
+template <int BM, int BN, int WM, int WN, int D, int KIND>
 static int tile_gemm_launch(const TileGemm& p) {
-  auto* kernel = &tile_gemm_kernel<BM, BN, WM, WN, KIND>;
-  constexpr int lds = 5 * (BM > BN ? BM : BN) * DEPTH * 2;
+  auto* kernel = &tile_gemm_kernel<BM, BN, WM, WN, D, KIND>;
+  constexpr int lds = ((D + 1) * BM + D * BN) * DEPTH * 2;
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
@@ -304,29 +315,98 @@ static int tile_gemm_launch(const TileGemm& p) {
   return 0;
 }
 
-// Whether this is faster than the library's product and a kernel of the
-// activation's own: where there are tiles for half of the compute units or
-// more.  us, before -> now, rows: outputs x depth:
-//   swiglu 2048: 2816 x 1024 45 -> 30, 14336 x 4096 398 -> 365; 4096: 5632 x
-//       2048 191 -> 149; 16384: 2816 x 1024 233 -> 160, 5632 x 2048 650 ->
-//       551, 14336 x 4096 2891 -> 2691 (1430 TFLOP/s)
-//   gelu 2048: 3584 x 1024 32 -> 29; 16384: 3584 x 1024 155 -> 119, 7168 x
-//       2048 440 -> 374, 19456 x 4096 2025 -> 1902
-//   clamped 2048: 2176 x 1024 35 -> 29; 16384: 4352 x 2048 547 -> 449, 11904
-//       x 4096 2405 -> 2267
-//   squared relu 2048: 3328 x 1024 27.3 -> 26.1; 16384: 6912 x 2048 433 ->
-//       352, 18432 x 4096 1875 -> 1756
-// Not gained by it: gelu 777: 19456 x 4096 138 -> 170; 1355: 7168 x 2048 48
-// -> 50.
-extern "C" int ll_tile_gemm_gains(int N, int rows) {
-  return N >= 2048 && ((long long)N + 255) / 256 * ((rows + 255) / 256) >= 128;
+// Tiles that there are: us of a step with all compute units at work and with
+// half of them or fewer (then L2 and the clock give more), and of a tile's
+// beginning and end, fitted to products 1024 and 8192 deep.
+struct Tile {
+  int rows, cols;
+  float all, half, ends;
+};
+static const Tile TILES[] = {
+    {256, 256, 1.38f, 0.98f, 11.f}, {192, 256, 1.14f, 0.89f, 7.f},
+    {128, 256, 0.85f, 0.70f, 5.f},  {256, 128, 0.80f, 0.53f, 6.f},
+    {192, 128, 0.69f, 0.48f, 5.5f}, {160, 128, 0.61f, 0.41f, 5.f},
+    {128, 128, 0.55f, 0.37f, 4.5f}, {96, 128, 0.46f, 0.31f, 4.5f},
+    {64, 128, 0.39f, 0.27f, 4.f}};
+
+template <int KIND>
+static int tile_gemm_go(const TileGemm& p, int tile) {
+  switch (tile) {
+    case 0: return tile_gemm_launch<256, 256, 2, 4, 2, KIND>(p);
+    case 1: return tile_gemm_launch<192, 256, 2, 4, 2, KIND>(p);
+    case 2: return tile_gemm_launch<128, 256, 2, 4, 3, KIND>(p);
+    case 3: return tile_gemm_launch<256, 128, 4, 2, 2, KIND>(p);
+    case 4: return tile_gemm_launch<192, 128, 2, 2, 3, KIND>(p);
+    case 5: return tile_gemm_launch<160, 128, 2, 2, 3, KIND>(p);
+    case 6: return tile_gemm_launch<128, 128, 2, 2, 4, KIND>(p);
+    case 7: return tile_gemm_launch<96, 128, 2, 2, 5, KIND>(p);
+    case 8: return tile_gemm_launch<64, 128, 2, 2, 5, KIND>(p);
+  }
+  return -2;
 }
 
-// Rows of x start ldx numbers apart, those of out ld_out.  0: done, -2: not
-// for this kernel.
+// The tile that is estimated to take least: a compute unit's time is that of
+// its rounds, the last of which may be of few tiles.  (1355 rows of 6912 x
+// 2048 are 162 tiles of 256 x 256, 42 us, 216 of 192 x 256, 39, or 297 of 128 x
+// 256, 51.)
+static int best_tile(int N, int rows, int K) {
+  int best = 0;
+  float least = 0.f;
+  for (int t = 0; t < (int)(sizeof(TILES) / sizeof(Tile)); ++t) {
+    const Tile& at = TILES[t];
+    const long long n = ((long long)N + at.rows - 1) / at.rows *
+                        ((rows + at.cols - 1) / at.cols);
+    const float steps = (float)K / DEPTH;
+    float us = (float)(n / 256) * (at.all * steps + at.ends);
+    if (const int rest = (int)(n % 256)) {
+      const float more = rest > 128 ? (rest - 128) / 128.f : 0.f;
+      us += (at.half + (at.all - at.half) * more) * steps + at.ends;
+    }
+    if (t == 0 || us < least) least = us, best = t;
+  }
+  return best;
+}
+
+// Whether this is faster than the library's product and, with an activation,
+// a kernel of its own.  us, the library -> here, rows: outputs x depth:
+//  * always with an activation, but for few tiles of some depth.  swiglu 333:
+//    2816 x 1024 18 -> 11; 1355: 5632 x 2048 79 -> 65, 14336 x 4096 291 -> 275;
+//    16384: 2816 x 1024 233 -> 160, 14336 x 4096 2891 -> 2691 (1430 TFLOP/s).
+//    gelu 16384: 7168 x 2048 440 -> 374, 19456 x 4096 2025 -> 1902.  clamped
+//    16384: 4352 x 2048 547 -> 449, 11904 x 4096 2405 -> 2267.  squared relu
+//    333: 6912 x 2048 29 -> 20; 1355: 50 -> 44, 18432 x 4096 193 -> 183
+//  * not for few tiles of some depth, which the library takes in shares: 333:
+//    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18
+//  * outputs that are no whole tiles of 256: 333: 8224 x 2048 25 -> 21; 1355:
+//    3216 x 1024 17.5 -> 13.2, 8224 x 2048 56 -> 52; 8200: 1808 x 1024 53 -> 34,
+//    16448 x 4096 922 -> 834; 16384: 3600 x 2048 236 -> 200, 6416 x 2048 378 ->
+//    338, but 16512 x 4096 1557 -> 1604
+//  * shallow ones, or of medium depth and not too many rows: 1355: 1024 x 1024
+//    10.8 -> 9.0, 2048 x 2048 18.6 -> 18.1, 3072 x 2048 24.6 -> 22.2; 12288:
+//    1024 x 1024 28.4 -> 26.0, but 16384: 2048 x 2048 101 -> 104
+//  * deep ones have the library's best rate (16384: 4096 x 14336 1250 -> 1296,
+//    1355: 2048 x 7168 55 -> 59), but where its tiles of 256 x 256 leave a last
+//    round of few (8200: 2048 x 7168 322 -> 216, 4096 x 4096 302 -> 216; 4100:
+//    4096 x 18432 906 -> 614), and the deepest of medium rows (1355: 4096 x
+//    18432 308 -> 227)
+extern "C" int ll_tile_gemm_gains(int N, int rows, int K, int kind) {
+  if (N <= 0 || rows <= 0 || K <= 0) return 0;
+  const long long few = ((long long)N + 63) / 64 * ((rows + 127) / 128);
+  if (K > 1024 && few < (kind == PLAIN ? 200 : 150)) return 0;
+  if (kind != PLAIN || K <= 1024) return 1;
+  if (rows % 256) return K < 3072 || N < 12288;
+  if (K < 3072) return N < 4096;
+  const long long large = ((long long)N + 255) / 256 * (rows / 256);
+  const int last = (int)(large % 256);
+  return (large > 256 && last > 0 && last <= 64) ||
+         (K >= 16384 && N >= 256 && N <= 2048);
+}
+
+// Rows of x start ldx numbers apart, those of out ld_out.  tile: -1, or the one
+// to take.  0: done, -2: not for this kernel.
 extern "C" int ll_tile_gemm(void* out, int ld_out, const void* x,
                             const void* w, int N, int M, int K, int ldx,
-                            int kind, int up, float a, float b,
+                            int kind, int up, float a, float b, int tile,
                             void* stream) {
   if (N <= 0 || M <= 0 || K <= 0 || M % 8 || K % DEPTH || ldx < K ||
       ldx % 8 || ld_out < M || ld_out % 8 || up < 0 || (uintptr_t)x % 16 ||
@@ -338,11 +418,14 @@ extern "C" int ll_tile_gemm(void* out, int ld_out, const void* x,
   const TileGemm p{(bf16_t*)out, ld_out,           (const bf16_t*)x,
                    (const bf16_t*)w, N, M, K, ldx, RowAct{kind, up, a, b},
                    (hipStream_t)stream};
+  const bool gated = kind == SWIGLU || kind == CLAMPED;
+  if (tile < 0) tile = best_tile(N, gated ? 2 * M : M, K);
   switch (kind) {
-    case RELU2: return tile_gemm_launch<256, 256, 2, 4, RELU2>(p);
-    case GELU: return tile_gemm_launch<256, 256, 2, 4, GELU>(p);
-    case SWIGLU: return tile_gemm_launch<256, 256, 2, 4, SWIGLU>(p);
-    case CLAMPED: return tile_gemm_launch<256, 256, 2, 4, CLAMPED>(p);
+    case PLAIN: return tile_gemm_go<PLAIN>(p, tile);
+    case RELU2: return tile_gemm_go<RELU2>(p, tile);
+    case GELU: return tile_gemm_go<GELU>(p, tile);
+    case SWIGLU: return tile_gemm_go<SWIGLU>(p, tile);
+    case CLAMPED: return tile_gemm_go<CLAMPED>(p, tile);
   }
   return -2;
 }

@@ -168,6 +168,8 @@ class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
             y = _ops.scaled_mm_prefill(x, self._w8, self.weight)
             if y is not None:
                 return y + self.bias if self.bias is not None else y
+        if self.bias is None:
+            return _ops.linear_rows(x, self.weight)
         return torch.nn.functional.linear(x, self.weight, self.bias)
 
     def forward_swiglu(self, x: torch.Tensor) -> torch.Tensor | None:
@@ -213,7 +215,7 @@ class RowParallelLinear(nn.Module, _Fp8WeightMixin):
                 y = _ops.scaled_mm_prefill(x, self._w8,
                                            self.weight)
             if y is None:
-                y = torch.nn.functional.linear(x, self.weight)
+                y = _ops.linear_rows(x, self.weight)
         return self.tp.all_reduce(y)
 
     def forward_swiglu_w8a8(self, gateup: torch.Tensor):

@@ -1,5 +1,5 @@
-"""Products of many rows with an activation (tile_gemm.hip) against float
-products of the same numbers, at the edges of its tiles."""
+"""Products of many rows (tile_gemm.hip) against float products of the same
+numbers, at the edges of its tiles."""
 import pytest
 import torch
 
@@ -9,30 +9,32 @@ from test_row_gemm_gpu import DEV, _act
 pytestmark = pytest.mark.gpu
 
 
-def _tiled(x, w, act, out, up, a, b, monkeypatch):
+def _tiled(x, w, act, out, up, a, b, monkeypatch, tile=-1):
     """The kernel at sizes at which the library would be the faster."""
-    monkeypatch.setattr(ops._lib, "ll_tile_gemm_gains", lambda n, m: 1)
-    return ops.linear_act(x, w, act, out, up, a, b)
+    monkeypatch.setattr(ops._lib, "ll_tile_gemm_gains", lambda *sizes: 1)
+    return ops._tile_gemm(x, w, act, out, up, a, b, tile)
 
 
 # one tile, edges of rows and outputs, several tiles a workgroup (2100 rows
-# of 9000 outputs are 324 to 639 tiles); depths of one step to three
-@pytest.mark.parametrize("act,a,b", [("relu2", 0, 0), ("gelu", 0, 0),
-                                     ("swiglu", 0, 0), ("clamped", 1.5, 1.7)])
+# of 9000 outputs are 324 to 2343 tiles); depths of one step, fewer than are
+# fetched ahead and more; tile -1: the kernel's choice
+@pytest.mark.parametrize("tile,act,a,b", [
+    (0, "relu2", 0, 0), (0, "gelu", 0, 0), (0, "clamped", 1.5, 1.7),
+    (-1, "gelu", 0, 0), (-1, "plain", 0, 0),
+    *((t, act, 0, 0) for t in range(9) for act in ("plain", "swiglu"))])
 @pytest.mark.parametrize("N,M,K", [(129, 8, 64), (256, 256, 128),
                                    (300, 1160, 192), (513, 520, 1024),
-                                   (2100, 9000, 64), (2100, 9000, 192),
-                                   (1000, 16392, 128)])
-def test_tile_gemm(N, M, K, act, a, b, monkeypatch):
+                                   (2100, 9000, 64), (2100, 9000, 448)])
+def test_tile_gemm(N, M, K, tile, act, a, b, monkeypatch):
     g = torch.Generator(device=DEV).manual_seed(N + M)
     x = torch.randn(N, K + 16, generator=g, device=DEV).bfloat16()[:, 8:8 + K]
     up = M if act in ("swiglu", "clamped") else 0
     w = torch.randn(M + up, K, generator=g, device=DEV).mul_(
         K ** -0.5).bfloat16()
     z = x.double() @ w.double().T
-    ref = _act(act, z.bfloat16().double(), up, a, b)
+    ref = z if act == "plain" else _act(act, z.bfloat16().double(), up, a, b)
     wide = torch.full((N, M + 16), 7.0, device=DEV, dtype=torch.bfloat16)
-    out = _tiled(x, w, act, wide[:, 8:8 + M], up, a, b, monkeypatch)
+    out = _tiled(x, w, act, wide[:, 8:8 + M], up, a, b, monkeypatch, tile)
     # as for few rows: sums near the middle of two bf16 numbers may take
     # the other one, which an activation makes at most 60 times larger
     off = (x.double().abs() @ w.double().abs().T).amax() * K * 2.0 ** -24
@@ -74,6 +76,7 @@ def test_other_operands_go_to_the_library(N, M, K, shift, monkeypatch):
     assert _tiled(x, w, "gelu", None, 0, 0, 0, monkeypatch) is None
 
 
+@torch.inference_mode()
 def test_capture():
     """Replays give what an eager call gives."""
     x = torch.randn(2048, 256, device=DEV).bfloat16()
@@ -90,3 +93,24 @@ def test_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
+
+
+def test_prompt_products():
+    """The whole call, on both sides of the choice."""
+    for N, M, K, taken in ((1355, 3216, 1024, True),
+                           (1355, 2048, 7168, False)):
+        x = torch.randn(N, K, device=DEV).bfloat16()
+        w = torch.randn(M, K, device=DEV).mul_(K ** -0.5).bfloat16()
+        assert (ops._tile_gemm(x, w) is not None) == taken
+        z = x.double() @ w.double().T
+        bound = z.abs() * 2.0 ** -8 + (
+            x.double().abs() @ w.double().abs().T) * K * 2.0 ** -24
+        assert ((ops.linear_rows(x, w).double() - z).abs() <= bound).all()
+
+
+def test_gradients_keep_the_library():
+    x = torch.randn(300, 64, device=DEV, dtype=torch.bfloat16,
+                    requires_grad=True)
+    w = torch.randn(512, 64, device=DEV, dtype=torch.bfloat16)
+    ops.linear_rows(x, w).float().sum().backward()
+    assert x.grad is not None
