@@ -4,6 +4,8 @@
 //
 //  * expert_tile_kernel  prompts: tiles of an expert's list (experts.h)
 //    against tiles of its matrix, both copied to LDS directly
+//  * expert_product_kernel  the same by tile_product.h, where there are tiles
+//    of 192 x 256 for the compute units
 //  * expert_few_kernel   few pairs: a workgroup finds its expert's pairs
 //    among all choices and streams some rows of its matrix once
 //
@@ -11,6 +13,7 @@
 // of pair n = lane % 16.
 #include "experts.h"
 #include "row_tile.h"
+#include "tile_product.h"
 
 // LDS rows are P pieces of 16 bytes; piece c of row r lies at
 // c ^ swizzle(r), so that lanes reading one piece of the rows of an
@@ -209,6 +212,93 @@ void expert_tile_kernel(
   }
 }
 
+// The rows of experts' lists, for tile_product
+template <int BM, int BN>
+struct ListRows {
+  const bf16_t *in, *w_;
+  const int *counts, *pairs;
+  int E, N, K, div, n_tok, n_blocks;
+  const ExpertTiles<BM>* found;
+  struct At {
+    ExpertTile t;
+    const int* list;
+    int m0;
+  };
+  __device__ __forceinline__ long long tiles() const {
+    return (long long)(found->whole[E - 1] + found->rest[E - 1]) * n_blocks;
+  }
+  __device__ __forceinline__ At at(int i) const {
+    const int whole = found->whole[E - 1], j = i / n_blocks;
+    At a;
+    a.t = found->get(counts, E, j < whole ? j : j - whole, j >= whole);
+    a.list = pairs + (size_t)a.t.expert * n_tok + a.t.first;
+    a.m0 = i % n_blocks * BN;
+    return a;
+  }
+  __device__ __forceinline__ const bf16_t* x(const At&) const { return in; }
+  __device__ __forceinline__ const bf16_t* w(const At& a) const {
+    return w_ + (size_t)a.t.expert * N * K;
+  }
+  __device__ __forceinline__ unsigned x_offset(const At& a, int r) const {
+    return (unsigned)(a.list[r < a.t.n ? r : a.t.n - 1] / div) * (unsigned)K;
+  }
+  __device__ __forceinline__ long long row(const At& a, int r) const {
+    return r < a.t.n ? a.list[r] : -1;
+  }
+  __device__ __forceinline__ bool whole(const At& a) const {
+    return a.t.n == BM;
+  }
+};
+
+// Bound by the matrix cores' power and, for shallow products, by what they
+// write: 16384 tokens with 4 of 16 experts, us, the best of the tiles above
+// -> here: 1024 to 256 wide 60 -> 46, back 61 -> 58; 2048 to 512 162 -> 135,
+// back 211 -> 187; 4096 to 1280 629 -> 573 (1200 TFLOP/s), back 720 -> 695.
+// 256 x 256 leaves no LDS for the tiles' numbers; 256 x 128 and 128 x 256
+// read more (2048 to 512: 146, 156).
+template <int BM, int BN, int WM, int WN, int D, int KIND>
+__global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
+void expert_product_kernel(bf16_t* __restrict__ out,
+                           ListRows<BM, BN> rows) {
+  __shared__ ExpertTiles<BM> tiles;
+  if (threadIdx.x < WAVE) tiles.count(rows.counts, rows.E);
+  __syncthreads();
+  rows.found = &tiles;
+  tile_product<BM, BN, WM, WN, D, KIND, false>(rows, out, rows.N, rows.N, rows.K,
+                                        RowAct{KIND, 0, 0.f, 0.f});
+}
+
+struct ExpertProduct {
+  bf16_t* out;
+  const bf16_t *in, *w;
+  const int *counts, *pairs;
+  int E, N, K, div, n_tok, n_pairs;
+  hipStream_t stream;
+};
+template <int BM, int BN, int WM, int WN, int D, int KIND>
+static int expert_product(const ExpertProduct& p) {
+  auto* kernel = &expert_product_kernel<BM, BN, WM, WN, D, KIND>;
+  constexpr int lds = ((D + 1) * BM + D * BN) * DEPTH * 2;
+  static_assert(lds + sizeof(ExpertTiles<BM>) <= 160 * 1024,
+                "LDS of a compute unit");
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const int nb = (p.N + BN - 1) / BN;
+  // as many tiles as there can be, and a workgroup a compute unit at most
+  const long long most =
+      ((long long)p.n_pairs / BM + (p.E < p.n_pairs ? p.E : p.n_pairs)) * nb;
+  if (most >= 1ll << 27) return -2;
+  const long long per = (most + 7) / 8;
+  const ListRows<BM, BN> rows{p.in, p.w, p.counts, p.pairs, p.E, p.N,
+                              p.K,  p.div, p.n_tok, nb, nullptr};
+  hipLaunchKernelGGL(kernel, dim3(8 * (unsigned)(per < 32 ? per : 32)),
+                     dim3(WM * WN * 64), lds, p.stream, p.out, rows);
+  HY_CHECK();
+  return 0;
+}
+
 // Few pairs: workgroup (expert, 32 outputs), tiles of up to 64 of the
 // expert's pairs as in row_tile.h.  Bound by reading the matrices: both
 // products of 16 experts of 4096 x 1280 took 105 us for 64 tokens with
@@ -278,7 +368,8 @@ __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
 
 extern "C" {
 
-// tile: 0 128 x 128, 1 256 x 256, 2 128 x 256 (pairs x outputs)
+// tile: 0 128 x 128, 1 256 x 256, 2 128 x 256, 3 192 x 256 by tile_product
+// (pairs x outputs)
 int hy_expert_tiles(void* out, const void* in, const void* w,
                     const void* counts, const void* pairs, int E, int N,
                     int K, int div, int act, int n_tok, int n_pairs,
@@ -308,6 +399,17 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
     case 0: GO(128, 128, 2, 2, 64, 2); break;
     case 1: GO(256, 256, 4, 4, 64, 2); break;
     case 2: GO(128, 256, 2, 4, 32, 3); break;
+    case 3:
+      if (K % DEPTH == 0 && near) {
+        const ExpertProduct p{(bf16_t*)out, (const bf16_t*)in,
+                              (const bf16_t*)w, (const int*)counts,
+                              (const int*)pairs, E, N, K, div, n_tok,
+                              n_pairs, (hipStream_t)stream};
+        return act ? expert_product<192, 256, 2, 4, 2, RELU2>(p)
+                   : expert_product<192, 256, 2, 4, 2, PLAIN>(p);
+      }
+      GO(256, 256, 4, 4, 64, 2);
+      break;
     default: return -2;
   }
 #undef RUN

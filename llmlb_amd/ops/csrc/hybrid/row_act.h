@@ -3,9 +3,9 @@
 // to bf16 first, as where it is stored for that kernel.  With two matrices,
 // gate and up, the rows of up begin at row ``up`` of the weight.
 #pragma once
-#include "hybrid/mfma.h"
+#include "mfma.h"
 
-enum { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };
+enum RowKind { PLAIN, RELU2, GELU, SWIGLU, CLAMPED, CAPPED };
 struct RowAct {
   int kind;
   int up;      // SWIGLU, CLAMPED: the first row of up

@@ -17,8 +17,8 @@
 //       60.9 -> 37.0 (6.3 TB/s)
 // With more rows the bound is what a compute unit takes in, about 50 GB/s:
 // every tile reads all of its x and W.
+#include "hybrid/row_act.h"
 #include "hybrid/row_tile.h"
-#include "row_act.h"
 
 // The order in which a sum is made differs with the number of rows, as with
 // any product: tiles, waves and shares follow from it.  With gate and up, a

@@ -864,16 +864,20 @@ def route(h, w, top, groups, keep, scale, lists: bool = True):
 
 def expert_tile(pairs: int, experts: int, n: int, k: int) -> int:
     """Tile of ``hy_expert_tiles`` for products of depth k with n
-    outputs: 128 x 128 where experts have few pairs or outputs, 128 x 256
-    (two a compute unit, so that one stores while the other multiplies)
-    for shallow products.  Deep ones take 256 x 256, a round of one tile a
-    compute unit, unless the last round is too empty: by output 128 x 128
-    takes 1.35 times as long, but in rounds of an eighth.  2048 to 512
-    wide, us (256 x 256, 128 x 128): 0.76 rounds 53, 63; 1.06 98, 83;
-    1.55 105, 114; 2.06 151, 143; 4096 to 1280: 1.42 200, 185; 2.65 325,
-    349; 5.15 619, 720."""
+    outputs: 128 x 128 where experts have few pairs or outputs, 192 x 256
+    where rounds of a tile a compute unit are full enough (an expert's last
+    tile counted as half of one).  2048 to 512 wide, us (128 x 128, 192 x
+    256): 0.39 rounds 32, 41; 0.73 58, 43; 1.4 92, 75; 2.73 162, 135; 4096 to
+    1280: 0.44 65, 87; 0.97 139, 97.  Else 128 x 256 (two a compute unit, so
+    that one stores while the other multiplies) for shallow products, and for
+    deep ones 256 x 256, a round of one tile a compute unit, unless the last
+    round is too empty: by output 128 x 128 takes 1.35 times as long, but in
+    rounds of an eighth."""
     if pairs < 192 * experts or n < 256:
         return 0
+    rounds = (pairs / 192 + experts / 2) * -(-n // 256) / 256
+    if math.ceil(rounds) <= 1.6 * rounds:
+        return 3
     if k < 1024:
         return 2 if n > 256 else 0
     rounds = (pairs / 256 + experts / 2) * -(-n // 256) / 256

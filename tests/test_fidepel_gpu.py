@@ -328,6 +328,32 @@ def test_experts(case, form, monkeypatch):
     close(got[sure], want[sure], dtype)
 
 
+# whole steps of the depth (64): experts with no pair, one, an edge and
+# several tiles of 192, several tiles a workgroup
+@pytest.mark.parametrize("case", [(4, 2, 64, 64, 1), (14, 5, 256, 320, 60),
+                                  (16, 4, 128, 192, 700), (3, 1, 64, 8, 900),
+                                  (40, 3, 64, 128, 33),
+                                  (60, 4, 2048, 64, 2500)], ids=str)
+def test_experts_by_products(case, monkeypatch):
+    E, top, W, ff, T = case
+    mlp = U.moe(E, top, ff)
+    w = U.experts_case(mlp, W, E)
+    h = U.inputs(T, W, 5)
+    w["router"][:top] += 0.5 * h[: T // 2 + 1].mean(0)
+    h[: T // 2] = h[0]
+    w["router"] = w["router"].bfloat16().double()
+    monkeypatch.setattr(hy, "FEW_PAIRS", 0)
+    monkeypatch.setattr(hy, "expert_tile", lambda *a: 3)
+    module = U.experts_module(mlp, w, W, DEV, B16)
+    got = U.run_experts(module, h)
+    want = O.mixture(h, w, "", mlp)
+    sure = O.margins(h, w["router"], mlp["router"]) > 1e-4
+    close(got[sure], want[sure], B16)
+    # the sums are made in the order of the other tiles
+    monkeypatch.setattr(hy, "expert_tile", lambda *a: 0)
+    assert torch.equal(U.run_experts(module, h), got)
+
+
 @pytest.mark.parametrize("W,ff", [(50, 12), (64, 15), (31, 33)])
 @DTYPES
 def test_experts_of_odd_sizes(W, ff, dtype):
