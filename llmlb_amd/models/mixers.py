@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
-from ..ops import linear_act, linear_decode, linear_rows
+from ..ops import linear_act, linear_decode, linear_heads, linear_rows
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
@@ -123,6 +123,7 @@ class LatentAttention(nn.Module):
             if self.sink else None
         self.w_uk = _param(w["uk"].reshape(
             self.heads, self.dim, self.rank).to(**to).contiguous())
+        self.w_uk_t = _param(self.w_uk.transpose(1, 2).contiguous())
         uv = w["uv"].reshape(self.heads, self.vdim, self.rank).to(**to)
         self.w_uv = _param(uv.contiguous())
         self.w_uv_t = _param(uv.transpose(1, 2).contiguous())
@@ -157,23 +158,28 @@ class LatentAttention(nn.Module):
 
     def _absorbed(self, proj, b, pages, n, out=None):
         """The first n tokens of the batch -> [n, heads * vdim]."""
-        H, D = self.heads, self.dim
+        H, D, V = self.heads, self.dim, self.vdim
         q = proj[:n, :H * (D + self.rot)].unflatten(
             1, (H, D + self.rot))[..., :D].transpose(0, 1)
-        qa = torch.bmm(q, self.w_uk)
+        qa = torch.empty(H, n, self.rank, dtype=proj.dtype,
+                         device=proj.device)
+        if not linear_heads(q, self.w_uk_t, qa):
+            qa = torch.bmm(q, self.w_uk)
         attend = hy.latent_decode if self.tiled and proj.is_cuda \
             else hy.latent_rows
         lat = attend(qa, proj, D, self.rot, pages, b, self.window,
                      self.scale, self.w_sink)
+        if out is None:
+            out = torch.empty(n, H * V, dtype=proj.dtype, device=proj.device)
+        gate = proj[:n, self.g_off:self.g_off + H * V] if self.gate else None
+        if linear_heads(lat, self.w_uv, out.view(n, H, V).transpose(0, 1),
+                        gate):
+            return out
         o = torch.bmm(lat, self.w_uv_t)                 # [H, n, vdim]
         if self.gate:
-            if out is None:
-                out = torch.empty(n, H * self.vdim, dtype=o.dtype,
-                                  device=o.device)
             hy.join_heads(out, o, proj, self.g_off)
             return out
-        o = o.transpose(0, 1).reshape(n, H * self.vdim)
-        return o if out is None else out.copy_(o)
+        return out.copy_(o.transpose(0, 1).reshape(n, H * V))
 
 
 class ChannelDelta(nn.Module):

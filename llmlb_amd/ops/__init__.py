@@ -856,6 +856,41 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, weight) if out is None else out
 
 
+def linear_heads(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
+                 gate: torch.Tensor | None = None) -> bool:
+    """out[h] = x[h] @ weight[h]^T of up to 128 bf16 rows for all heads in
+    one launch, times the sigmoid of ``gate``; False where row_gemm.hip does
+    not take it.  x [H, N, K] and out [H, N, M] may be views whose last
+    dimension is dense, weight [H, M, K], gate [N, H * M]."""
+    if not (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
+            and x.dim() == weight.dim() == out.dim() == 3
+            and _only_numbers(x, weight, out)):
+        return False
+    (H, N, K), M = x.shape, weight.shape[1]
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or not 0 < N <= 128
+            or weight.shape != (H, M, K) or out.shape != (H, N, M)
+            or weight.dtype != x.dtype or out.dtype != x.dtype
+            or not weight.is_contiguous() or x.stride(2) != 1
+            or out.stride(2) != 1
+            or not x.device == weight.device == out.device):
+        return False
+    if gate is not None and (
+            gate.shape != (N, H * M) or gate.stride(1) != 1
+            or gate.dtype != x.dtype or gate.device != x.device
+            or not _only_numbers(gate)):
+        return False
+    rc = _lib.ll_head_gemm(
+        _ptr(out), ctypes.c_int(out.stride(1)), ctypes.c_int(out.stride(0)),
+        _ptr(x), ctypes.c_int(x.stride(1)), ctypes.c_int(x.stride(0)),
+        _ptr(weight), None if gate is None else _ptr(gate),
+        ctypes.c_int(0 if gate is None else gate.stride(0)), ctypes.c_int(H),
+        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K), _stream())
+    if rc == -2:
+        return False
+    _check(rc, "ll_head_gemm")
+    return True
+
+
 # fusing swiglu into the staging measured ~4% SLOWER end-to-end (the
 # per-M-block silu recompute sits on the single-buffered staging
 # critical path; profiles/r01_fused_swiglu_ab.md) — default OFF

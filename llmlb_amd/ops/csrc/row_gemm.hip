@@ -271,3 +271,108 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
                   ldx, RowAct{kind, up, a, b}, (hipStream_t)stream};
   return gated ? row_gemm_pick<true>(p) : row_gemm_pick<false>(p);
 }
+
+// The same for H pairs of rows and matrices at once, as latent attention needs
+// for its heads: out[h] = x[h] W[h]^T, W [H][M][K].  x's and out's heads lie
+// xs and os numbers apart.  With a gate, out = bf16(sum) sigmoid(gate), the
+// gate of output m of head h being column h M + m of the row.
+// A launch and two dependent loads; us, the library's batched product -> here,
+// captured, weights from HBM (the second joins the heads in one row, which
+// was a copy of torch's):
+//   64 rows: 32 heads of 512 x 128 5.3 -> 4.3, of 128 x 512 13.5 -> 3.9;
+//       16 heads of 256 x 64 5.0 -> 2.7, of 64 x 256 9.0 -> 2.9
+//   128 rows: 32 heads of 512 x 128 6.2 -> 5.3, of 128 x 512 15.4 -> 4.7
+//   4 rows: 16 heads of 512 x 128 4.2 -> 2.8, of 128 x 512 14.0 -> 3.3
+template <int NT, int MT, int KW, int S, bool GATED>
+__global__ __launch_bounds__(KW * 64, 2) void head_gemm_kernel(
+    bf16_t* __restrict__ out, int ld_out, int os,
+    const bf16_t* __restrict__ x, int ldx, int xs,
+    const bf16_t* __restrict__ w, const bf16_t* __restrict__ gate,
+    int ld_gate, int N, int M, int K) {
+  using Tile = RowTile<NT, MT, KW, S>;
+  constexpr int OUT = 16 * MT;
+  extern __shared__ __align__(1024) char lds[];
+  const int h = blockIdx.y, n0 = blockIdx.z * 16 * NT;
+  const int m0 = blockIdx.x * OUT;
+  const bf16_t* wh = w + (size_t)h * M * K;
+  const bf16_t* xh = x + (size_t)h * xs;
+  Tile::run(
+      lds, K, blockIdx.x + h,
+      [&](int r) {
+        return xh + (size_t)(n0 + r < N ? n0 + r : N - 1) * ldx;
+      },
+      [&](int r) {
+        return wh + (size_t)(m0 + r < M ? m0 + r : M - 1) * K;
+      });
+  Tile::each(OUT / 4, [&](int r, int c) {
+    if (n0 + r >= N || m0 + c >= M) return;
+    f32x4 v = Tile::sum(lds, r, c);
+    if (GATED) {
+      const uint2 z = *reinterpret_cast<const uint2*>(
+          gate + (size_t)(n0 + r) * ld_gate + (size_t)h * M + m0 + c);
+      const float g[4] = {
+          __uint_as_float(z.x << 16), __uint_as_float(z.x & 0xffff0000u),
+          __uint_as_float(z.y << 16), __uint_as_float(z.y & 0xffff0000u)};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = to_f(from_f<bf16_t>(v[i])) * sigmoid_f(g[i]);
+    }
+    *reinterpret_cast<uint2*>(out + (size_t)h * os +
+                              (size_t)(n0 + r) * ld_out + m0 + c) =
+        make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+  });
+}
+
+struct HeadGemm {
+  bf16_t* out;
+  int ld_out, os;
+  const bf16_t* x;
+  int ldx, xs;
+  const bf16_t *w, *gate;
+  int ld_gate, H, N, M, K;
+  hipStream_t stream;
+};
+template <int NT, int MT, int KW, int S, bool GATED>
+static int head_gemm_launch(const HeadGemm& p) {
+  constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
+  static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(head_gemm_kernel<NT, MT, KW, S, GATED>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  hipLaunchKernelGGL((head_gemm_kernel<NT, MT, KW, S, GATED>),
+                     dim3((p.M + 16 * MT - 1) / (16 * MT), p.H,
+                          (p.N + 16 * NT - 1) / (16 * NT)),
+                     dim3(KW * 64), lds, p.stream, p.out, p.ld_out, p.os, p.x,
+                     p.ldx, p.xs, p.w, p.gate, p.ld_gate, p.N, p.M, p.K);
+  HY_CHECK();
+  return 0;
+}
+// Waves for the pieces of 64 of the depth that there are; 16 rows a tile, from
+// 49 rows on 32 (us, 16 and 32: 64 rows, 32 heads of 128 x 512 4.1 and 3.9, 128
+// rows 6.3 and 4.7; 16 heads of 64 x 256 2.9 and 3.1).  64 rows or outputs a
+// tile are too few workgroups (4.5).
+template <bool GATED>
+static int head_gemm_pick(const HeadGemm& p) {
+  if (p.K <= 128)
+    return p.N <= 48 ? head_gemm_launch<1, 2, 2, 1, GATED>(p)
+                     : head_gemm_launch<2, 2, 2, 1, GATED>(p);
+  return p.N <= 48 ? head_gemm_launch<1, 2, 4, 2, GATED>(p)
+                   : head_gemm_launch<2, 2, 4, 2, GATED>(p);
+}
+
+// 0: done, -2: not for this kernel
+extern "C" int ll_head_gemm(void* out, int ld_out, int os, const void* x,
+                            int ldx, int xs, const void* w, const void* gate,
+                            int ld_gate, int H, int N, int M, int K,
+                            void* stream) {
+  if (H <= 0 || H > 65535 || N <= 0 || N > 128 || M <= 0 || K <= 0 || M % 4 ||
+      K % 8 || ldx % 8 || xs % 8 || ld_out % 4 || os % 4 ||
+      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 8 ||
+      (gate && (ld_gate % 4 || (uintptr_t)gate % 8)))
+    return -2;
+  const HeadGemm p{(bf16_t*)out,     ld_out,  os, (const bf16_t*)x, ldx, xs,
+                   (const bf16_t*)w, (const bf16_t*)gate, ld_gate, H, N, M, K,
+                   (hipStream_t)stream};
+  return gate ? head_gemm_pick<true>(p) : head_gemm_pick<false>(p);
+}

@@ -125,3 +125,47 @@ def test_row_gemm_with_activation(N, M, K, act, a, b):
         bound = bound + ref.abs() * 2.0 ** -8
         assert (wide[:, :8] == 7).all() and (wide[:, 8 + M:] == 7).all()
     assert ((out.double() - ref).abs() <= bound).all()
+
+
+# heads, outputs, depth: one and two pieces of the depth, remainders of both
+@pytest.mark.parametrize("H,M,K", [(4, 512, 128), (3, 68, 72), (5, 128, 512),
+                                   (2, 36, 264)])
+@pytest.mark.parametrize("N", [1, 16, 48, 49, 65, 128])
+@pytest.mark.parametrize("gated", [False, True])
+def test_heads(N, H, M, K, gated):
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    wide = torch.randn(N, H * (K + 8) + 24, generator=g, device=DEV).bfloat16()
+    x = wide[:, 16:16 + H * (K + 8)].unflatten(1, (H, K + 8))[..., :K] \
+        .transpose(0, 1)
+    w = torch.randn(H, M, K, generator=g, device=DEV).mul_(
+        K ** -0.5).bfloat16()
+    rows = torch.full((N, H * M + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    gate = torch.randn(N, H * M + 4, generator=g, device=DEV).bfloat16()
+    gate = gate[:, 4:] if gated else None
+    out = rows[:, 4:4 + H * M].unflatten(1, (H, M)).transpose(0, 1)
+    assert ops.linear_heads(x, w, out, gate)
+    assert (rows[:, :4] == 7).all() and (rows[:, 4 + H * M:] == 7).all()
+    if not gated:
+        for h in range(H):
+            _close(out[h], x[h], w[h])
+        return
+    # a sum that may round either way, then the gate, then a rounding
+    z = x.double() @ w.double().transpose(1, 2)
+    ref = z * gate.double().sigmoid().view(N, H, M).transpose(0, 1)
+    bound = z.abs() * 2.0 ** -7 \
+        + (x.double().abs() @ w.double().abs().transpose(1, 2)) * K * 2.0 ** -24
+    assert ((out.double() - ref).abs() <= bound).all()
+
+
+def test_heads_that_do_not_fit():
+    x = torch.randn(4, 129, 64, device=DEV).bfloat16()
+    w = torch.randn(4, 32, 64, device=DEV).bfloat16()
+    out = torch.empty(4, 129, 32, device=DEV, dtype=torch.bfloat16)
+    assert not ops.linear_heads(x, w, out)                # rows
+    x, out = x[:, :8], out[:, :8]
+    assert ops.linear_heads(x, w, out)
+    assert not ops.linear_heads(x, w[:3], out)            # heads
+    assert not ops.linear_heads(x, w.transpose(1, 2), out)
+    assert not ops.linear_heads(x, w, out.float())
+    assert not ops.linear_heads(x[..., 4:36], w[..., :32].contiguous(), out)
+    assert not ops.linear_heads(x, w, out, out[0])        # gate's shape
