@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
   const int pos = pos_[s], slot = row_[s];
   const int C = 2 * KH * D + H * V;
-  const int r0 = (lane & 15) * RPL;
+  const int l16 = lane & 15;
   const int col0 = wave * 4 + lane / 16;
   float* sp = state + ((size_t)slot * H + h) * (size_t)V * D;
 
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
     for (int n = 0; n < NU; ++n) {
       const int col = base + n * 16 + col0;
       if (pos > 0 && col < V) {
-        load_rows<RPL, EXACT>(sp + (size_t)col * D, r0, D, S[n]);
+        load_spread<RPL, EXACT>(sp + (size_t)col * D, l16, D, S[n]);
       } else {
 #pragma unroll
         for (int i = 0; i < RPL; ++i) S[n][i] = 0.f;
@@ -463,9 +463,10 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
   float q[RPL], k[RPL], g[RPL];
 #pragma unroll
   for (int i = 0; i < RPL; ++i) {
-    q[i] = lq[r0 + i] * qs;
-    k[i] = lk[r0 + i] * ks;
-    g[i] = lg[r0 + i];
+    const int at = spread_at<RPL, EXACT>(l16, i);
+    q[i] = lq[at] * qs;
+    k[i] = lk[at] * ks;
+    g[i] = lg[at];
   }
   float ssq = 0.f;
   for (int base = 0; base < V; base += NU * 16) {
@@ -486,7 +487,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
         const float u = beta * (lv[col] - x);
 #pragma unroll
         for (int i = 0; i < RPL; ++i) S[n][i] += k[i] * u;
-        store_rows<RPL, EXACT>(sp + (size_t)col * D, r0, D, S[n]);
+        store_spread<RPL, EXACT>(sp + (size_t)col * D, l16, D, S[n]);
         const float r = y + qk * u;
         if ((lane & 15) == 0) {
           lo[col] = r;

@@ -445,7 +445,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
   const int group = h / (H / G);
   const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & (WAVE - 1);
   const int pos = pos_[s], slot = row_[s];
-  const int r0 = (lane & 15) * RPL;
+  const int l16 = lane & 15;
   const int col0 = wave * 4 + lane / 16;
   float* sp = state + ((size_t)slot * H + h) * (size_t)V * D;
 
@@ -455,7 +455,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
     for (int n = 0; n < NU; ++n) {
       const int col = base + n * 16 + col0;
       if (pos > 0 && col < V) {
-        load_rows<RPL, EXACT>(sp + (size_t)col * D, r0, D, S[n]);
+        load_spread<RPL, EXACT>(sp + (size_t)col * D, l16, D, S[n]);
       } else {
 #pragma unroll
         for (int i = 0; i < RPL; ++i) S[n][i] = 0.f;
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
     dt = expf(li - m);
 #pragma unroll
     for (int i = 0; i < RPL; ++i) N[i] = 0.f;
-    if (pos > 0) load_rows<RPL, EXACT>(ex, r0, D, N);
+    if (pos > 0) load_spread<RPL, EXACT>(ex, l16, D, N);
   } else {
     for (int d = tid; d < DP; d += 256) {
       const bool ok = d < D;
@@ -519,9 +519,10 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
   float q[RPL], k[RPL], g[RPL];
 #pragma unroll
   for (int i = 0; i < RPL; ++i) {
-    q[i] = lq[r0 + i];
-    k[i] = lk[r0 + i] * dt;
-    g[i] = KIND == CHANNEL ? lg[r0 + i] : gh;
+    const int at = spread_at<RPL, EXACT>(l16, i);
+    q[i] = lq[at];
+    k[i] = lk[at] * dt;
+    g[i] = KIND == CHANNEL ? lg[at] : gh;
   }
   if constexpr (KIND == MEMORY) {
     // every 16 lanes make the normaliser; what it was has been read
@@ -532,7 +533,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
       a += q[i] * N[i];
     }
     inv = 1.f / (fmaxf(fabsf(row16_sum(a)), expf(-m)) + MEMORY_EPS);
-    if (tid < 16) store_rows<RPL, EXACT>(ex, r0, D, N);
+    if (tid < 16) store_spread<RPL, EXACT>(ex, l16, D, N);
     if (tid == 0) ex[extra_row(D) - 4] = m;
   }
   float ssq = 0.f;
@@ -551,7 +552,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
       r = row16_sum(r);
       if (KIND == MEMORY) r *= inv;
       if (col < V) {
-        store_rows<RPL, EXACT>(sp + (size_t)col * D, r0, D, S[n]);
+        store_spread<RPL, EXACT>(sp + (size_t)col * D, l16, D, S[n]);
         if ((lane & 15) == 0) {
           lo[col] = r + skip * v;
           ssq += r * r;

@@ -201,6 +201,51 @@ __device__ __forceinline__ void store_rows(float* __restrict__ p, int r0,
   }
 }
 
+// The same with a lane's numbers spread over the column by fours: number i is
+// channel spread_at<RPL, EXACT>(lane, i).  16 lanes then read and write 256
+// bytes in a row with each instruction, where every lane's own run leaves
+// gaps that a later instruction fills.  They go past the caches: a step
+// reads and writes every state once, and what it leaves dirty in them is
+// written back under the products that follow.  64 sequences at 32 heads of
+// 128 x 128, us a step of the model: Dibelix 1634 with runs by way of the
+// caches, 1630 spread, 1617 with stores past the caches, 1615 with loads, 1540
+// with both; Taletar 1596, 1592, 1564, 1570, 1526.
+template <int RPL, bool EXACT>
+__device__ __forceinline__ int spread_at(int lane, int i) {
+  return EXACT && RPL % 4 == 0 ? i / 4 * 64 + lane * 4 + i % 4
+                               : lane * RPL + i;
+}
+typedef __attribute__((ext_vector_type(4))) float fvec4;
+template <int RPL, bool EXACT>
+__device__ __forceinline__ void load_spread(const float* __restrict__ p,
+                                            int lane, int D, float* f) {
+  if (EXACT && RPL % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < RPL / 4; ++i) {
+      const fvec4 v = __builtin_nontemporal_load(
+          reinterpret_cast<const fvec4*>(p) + i * 16 + lane);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[i * 4 + j] = v[j];
+    }
+  } else {
+    load_rows<RPL, EXACT>(p, lane * RPL, D, f);
+  }
+}
+template <int RPL, bool EXACT>
+__device__ __forceinline__ void store_spread(float* __restrict__ p, int lane,
+                                             int D, const float* f) {
+  if (EXACT && RPL % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < RPL / 4; ++i) {
+      const fvec4 v = {f[i * 4], f[i * 4 + 1], f[i * 4 + 2], f[i * 4 + 3]};
+      __builtin_nontemporal_store(
+          v, reinterpret_cast<fvec4*>(p) + i * 16 + lane);
+    }
+  } else {
+    store_rows<RPL, EXACT>(p, lane * RPL, D, f);
+  }
+}
+
 // key channels a lane holds when 16 lanes share a column of D
 static int rows_per_lane(int D) {
   int r = 1;
