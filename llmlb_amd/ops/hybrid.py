@@ -15,7 +15,7 @@ import math
 
 import torch
 
-from . import NativeKernelsMissing, _check, _ptr, _stream
+from . import NativeKernelsMissing, _check, _ptr, _stream, linear_rows
 from . import reference_hybrid as ref
 from .build import library_path
 
@@ -319,20 +319,20 @@ def latent_flash(out, proj, heads, dim, rot, w_uk, w_uv, cache, b, window,
     _check(lib.hy_latent_gather(
         _ptr(c), _ptr(kr), _ptr(cache), _ptr(blocks), _i(n_blocks), _ptr(bt),
         _i(bt.shape[1]), _i(rank), _i(rot), st), "hy_latent_gather")
-    kx = torch.nn.functional.linear(c, w_uk.view(H * dim, rank))
+    kx = linear_rows(c, w_uk.view(H * dim, rank))
     # Rows of 64 + 32 and 64, 128 + 64 and 128 (a rotated part of half a
     # head), values as they are expanded.  The loop would take others whose
     # rows are 64, 96, 128 or 192 numbers; they have not been measured there.
     if (dim + rot, V) in ((96, 64), (192, 128)) and scale > 0 \
             and (g_off or 0) % 4 == 0:
-        vx = torch.nn.functional.linear(c, w_uv.view(H * V, rank))
+        vx = linear_rows(c, w_uv.view(H * V, rank))
         _check(lib.hy_latent_prompt(
             _ptr(out), _ptr(proj), _i(proj.stride(0)), _ptr(kx), _ptr(kr),
             _ptr(vx), _ptr(items), _i(n_items), _i(H), _i(dim), _i(rot),
             _i(V), _i(window), _f(scale), _p(sink),
             _i(-1 if g_off is None else g_off), st), "hy_latent_prompt")
         return
-    vt = torch.nn.functional.linear(w_uv.view(H * V, rank), c)
+    vt = linear_rows(w_uv.view(H * V, rank), c)
     _check(lib.hy_latent_flash(
         _ptr(out), _ptr(proj), _i(proj.stride(0)), _ptr(kx), _ptr(kr),
         _ptr(vt), _i(n), _ptr(items), _i(n_items), _i(H), _i(dim), _i(rot),
