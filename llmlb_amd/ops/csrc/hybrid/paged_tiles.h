@@ -44,6 +44,13 @@ struct Stage {
     return cache + (size_t)__builtin_amdgcn_readfirstlane(p) * page_size +
            head_off + (r % PAGE) * width;
   }
+  // ONCE: nobody reads the tile again, it goes past the caches
+  template <bool ONCE = false>
+  static __device__ __forceinline__ u32x4 load(const bf16_t* p) {
+    const u32x4* at = reinterpret_cast<const u32x4*>(p);
+    return ONCE ? __builtin_nontemporal_load(at) : *at;
+  }
+  template <bool ONCE = false>
   __device__ __forceinline__ void fetch(int j0, const int (&pg)[4],
                                         u32x4 (&pk)[KL],
                                         u32x4 (&pv)[VL]) const {
@@ -52,15 +59,14 @@ struct Stage {
       const int p = threadIdx.x + i * 256;
       const int c = p % KR, d = c % (DQ / 8) * 8;
       // columns past D meet zeros of the query
-      pk[i] = *reinterpret_cast<const u32x4*>(
-          row(p / KR, pg) + c / (DQ / 8) * D + (d < D ? d : 0));
+      pk[i] = load<ONCE>(row(p / KR, pg) + c / (DQ / 8) * D +
+                         (d < D ? d : 0));
     }
 #pragma unroll
     for (int i = 0; i < VL; ++i) {
       const int p = threadIdx.x + i * 256;
       const int r = p / VR, d = p % VR * 8;
-      pv[i] = *reinterpret_cast<const u32x4*>(row(r, pg) + MAPS * D +
-                                              (d < V ? d : 0));
+      pv[i] = load<ONCE>(row(r, pg) + MAPS * D + (d < V ? d : 0));
       // columns past V are zeros; rows past the last key meet zero weights
       // and must be finite
       if (j0 + r > last_key || d >= V) pv[i] = u32x4{0, 0, 0, 0};
