@@ -787,8 +787,8 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
 
 
 def _takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return (x.is_cuda and _lib is not None and _only_numbers(x, weight)
-            and x.dtype == torch.bfloat16 and _fit(x, weight)
+    return (x.dtype == torch.bfloat16 and x.is_cuda and _lib is not None
+            and _only_numbers(x, weight) and _fit(x, weight)
             and x.shape[0] > 0)
 
 
