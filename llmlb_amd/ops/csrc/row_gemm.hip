@@ -143,46 +143,67 @@ static int row_gemm_launch(const RowGemm& p) {
   return 0;
 }
 
-// The largest tile of which there are enough for the chip: a larger one
-// reads less (64 x 64 half of what 32 x 32 does), but under about 176 of
-// them, two thirds of the compute units, idle ones cost more than that (64
-// rows against 6144 x 4096: 96 tiles of 64 x 64 17.0 us, 192 of 32 x 64
-// 15.9; against 11264 x 2048: 176 of 64 x 64 13.8, 352 of 32 x 64 18).
-// Rows of x go in equal shares of up to 4 x 16.
+// The tile of which a compute unit takes in least.  What bounds all but the
+// fewest rows is the busiest compute unit's intake, about 50 GB/s: the tiles
+// that it gets, of 256 at a time, times the rows of a tile, of x and of W.  So
+// what counts is that a last round is full, or that there is none.  64 rows,
+// us, the largest tile with 176 of its kind before -> now: 19456 x 4096 43.4 (64
+// outputs a tile, two rounds) -> 30.1 (80, one), 16512 x 4096 42.3 -> 28.0,
+// 10272 x 4096 30.3 -> 21.2 (48), gate and up of 11904 x 4096 45.2 -> 35.3 (96),
+// 8224 x 2048 16.4 -> 11.7; 16 rows: 12576 x 4096 21.0 -> 17.5; 128 rows: 10272 x
+// 4096 38.3 -> 27.6, gate and up of 5632 x 2048 23.2 -> 16.5.
 template <bool GATED>
 static int row_gemm_pick(const RowGemm& p) {
-  const int tiles = (p.N + 15) / 16, shares = (tiles + 3) / 4;
-  const int nt = (tiles + shares - 1) / shares;
-  const int rows = GATED ? 2 * p.M : p.M;
-  auto enough = [&](int n, int m) {
-    return (size_t)((rows + 16 * m - 1) / (16 * m)) * ((tiles + n - 1) / n) >=
-           176;
+  const int tiles = (p.N + 15) / 16;
+  const long long rows = GATED ? 2ll * p.M : p.M;
+  // what memory takes for W, in the same unit: 16 rows at 50 GB/s
+  const float floor = rows / 2500.f;
+  int nt = 0, mt = 0;
+  float least = 0.f;
+  auto look = [&](int n, int m) {
+    // tiles of the same rows of W are on one of eight XCDs of 32 units
+    const long long down = (rows + 16 * m - 1) / (16 * m);
+    const long long count = (down + 7) / 8 * ((tiles + n - 1) / n);
+    const float takes =
+        fmaxf((float)((count + 31) / 32 * (n + m)), floor);
+    if (!nt || takes < 0.95f * least) least = takes, nt = n, mt = m;
   };
-#define ROW_GEMM(NT, MT, KW, S) \
-  return row_gemm_launch<NT, MT, KW, S, GATED>(p)
-  if (nt == 4) {
-    if (enough(4, 4)) ROW_GEMM(4, 4, 4, 2);
-    if (enough(4, 2)) ROW_GEMM(4, 2, 4, 2);
-  } else if (nt == 3) {
-    if (enough(3, 4)) ROW_GEMM(3, 4, 4, 2);
-    if (enough(3, 2)) ROW_GEMM(3, 2, 4, 2);
-    if constexpr (!GATED)
-      if (enough(3, 1)) ROW_GEMM(3, 1, 4, 3);
+  // what is as good: more rows of x, which read W less often, then the sizes
+  // that memory likes best
+  static const int OF_MANY[] = {4, 5, 6, 3, 2, 1}, OF_ONE[] = {2, 4, 3, 1, 5, 5};
+  for (int n = tiles < 4 ? tiles : 4; n >= 1; --n)
+    for (int i = 0; i < 6; ++i) {
+      const int m = n == 1 ? OF_ONE[i] : OF_MANY[i];
+      if (n < 3 || m > 1) look(n, m);  // (3, 1) and (4, 1) take in no less
+    }
+  // waves that share the depth, and pieces of it on their way, fit LDS
+#define TILE(NT, MT, KW, S) \
+  case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S, GATED>(p);
+  switch (nt * 8 + mt) {
+    TILE(1, 1, 8, 2)
+    TILE(1, 2, 4, 3)
+    TILE(1, 3, 4, 3)
+    TILE(1, 4, 4, 3)
+    TILE(1, 5, 4, 3)
+    TILE(2, 1, 4, 3)
+    TILE(2, 2, 4, 2)
+    TILE(2, 3, 4, 2)
+    TILE(2, 4, 4, 2)
+    TILE(2, 5, 4, 2)
+    TILE(2, 6, 4, 2)
+    TILE(3, 2, 4, 2)
+    TILE(3, 3, 4, 2)
+    TILE(3, 4, 4, 2)
+    TILE(3, 5, 4, 2)
+    TILE(3, 6, 4, 2)
+    TILE(4, 2, 4, 2)
+    TILE(4, 3, 4, 2)
+    TILE(4, 4, 4, 2)
+    TILE(4, 5, 4, 2)
+    TILE(4, 6, 4, 2)
   }
-  if (nt >= 2) {
-    if (enough(2, 4)) ROW_GEMM(2, 4, 4, 2);
-    if (enough(2, 2)) ROW_GEMM(2, 2, 4, 2);
-    if constexpr (!GATED)
-      if (enough(2, 1)) ROW_GEMM(2, 1, 4, 3);
-  }
-  // few rows, or a small matrix: all of a tile's depth is on its way at once
-  if constexpr (GATED) {
-    ROW_GEMM(1, 2, 4, 3);
-  } else {
-    if (enough(1, 2)) ROW_GEMM(1, 2, 4, 3);
-    ROW_GEMM(1, 1, 8, 2);
-  }
-#undef ROW_GEMM
+#undef TILE
+  return -2;
 }
 
 // In how many shares the depth is taken.  A deep matrix of so few rows that

@@ -35,6 +35,24 @@ def test_row_gemm(N, M, K):
     assert torch.equal(out, ops.linear_decode(x, w))
 
 
+# rows and outputs at which each tile is taken (of 16 to 64 rows of x and 16
+# to 96 of W), with remainders
+@pytest.mark.parametrize("N,M", [
+    (1, 4), (76, 1284), (1, 8196), (1, 11924), (1, 16412), (106, 516),
+    (106, 1028), (106, 2564), (31, 12332), (31, 16412), (31, 20492),
+    (106, 2052), (76, 4100), (76, 6148), (76, 8196), (76, 10292),
+    (106, 3076), (106, 4100), (106, 6148), (106, 8196), (106, 10292)])
+@pytest.mark.parametrize("K", [72, 520])
+def test_tiles(N, M, K):
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    _close(ops._row_gemm(x, w), x, w)
+    # gate and up are half as many outputs of as many rows
+    if M > 4:
+        test_row_gemm_with_activation(N, (M + 4) // 8 * 4, K, "swiglu", 0, 0)
+
+
 # two to six shares, depths and rows that are no whole pieces or tiles
 @pytest.mark.parametrize("M,K", [(4096, 8200), (2564, 12296), (1348, 17000)])
 @pytest.mark.parametrize("N", [32, 41, 64, 100, 128])
