@@ -299,32 +299,34 @@ static int expert_product(const ExpertProduct& p) {
   return 0;
 }
 
-// Few pairs: workgroup (expert, 32 outputs), tiles of up to 64 of the
+// Few pairs: workgroup (expert, 16 MT outputs), tiles of up to 64 of the
 // expert's pairs as in row_tile.h.  Bound by reading the matrices: both
 // products of 16 experts of 4096 x 1280 took 105 us for 64 tokens with
 // operands loaded straight into registers, 67 (5.0 TB/s) this way; 8 tokens
-// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  32 outputs: 16 read the
-// inputs twice as often (89 us), 64 are too few workgroups where few
-// experts are chosen (one token 26 -> 31).
+// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  hy_expert_few has the
+// outputs a tile.
 #define FEW_PAIRS 2048  // most that fit a workgroup's list
-// NT and S for the tile that the pairs need: about the same LDS for each,
-// so that two workgroups share a compute unit
-#define FEW_MT 2
+// 16 NT pairs by 16 MT outputs; pieces of the depth on their way so that every
+// NT fits the LDS of the first
 #define FEW_KW 4
-template <int NT>
-using FewTile = RowTile<NT, FEW_MT, FEW_KW, NT == 1 ? 3 : (NT == 2 ? 2 : 1)>;
-#define FEW_LDS FewTile<1>::LDS
-static_assert(FewTile<2>::LDS <= FEW_LDS && FewTile<4>::LDS <= FEW_LDS,
-              "one size of LDS for all tiles");
+template <int NT, int MT>
+using FewTile =
+    RowTile<NT, MT, FEW_KW, NT == 1 ? 3 : (NT == 2 ? 2 : 1)>;
+template <int MT>
+constexpr int FEW_LDS = FewTile<1, MT>::LDS;
 
+template <int MT>
 __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ in,
     const bf16_t* __restrict__ w, const int* __restrict__ index, int N, int K,
     int div, int act, int n_pairs) {
+  static_assert(FewTile<2, MT>::LDS <= FEW_LDS<MT> &&
+                    FewTile<4, MT>::LDS <= FEW_LDS<MT>,
+                "one size of LDS for all tiles");
   extern __shared__ __align__(1024) char lds[];
   __shared__ unsigned short list[FEW_PAIRS];
   __shared__ int len;
-  const int e = blockIdx.y, n0 = blockIdx.x * 16 * FEW_MT;
+  const int e = blockIdx.y, n0 = blockIdx.x * 16 * MT;
   const int tid = threadIdx.x;
   if (tid == 0) len = 0;
   __syncthreads();
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
         [&](int r) {
           return w + ((size_t)e * N + (n0 + r < N ? n0 + r : N - 1)) * K;
         });
-    Tile::each(4 * FEW_MT, [&](int r, int c) {
+    Tile::each(4 * MT, [&](int r, int c) {
       f32x4 v = Tile::sum(lds, r, c);
       if (act) {
 #pragma unroll
@@ -360,9 +362,9 @@ __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
   };
   for (int first = 0; first < count; first += 64) {
     const int left = count - first;
-    if (left <= 16) tile(FewTile<1>{}, first);
-    else if (left <= 32) tile(FewTile<2>{}, first);
-    else tile(FewTile<4>{}, first);
+    if (left <= 16) tile(FewTile<1, MT>{}, first);
+    else if (left <= 32) tile(FewTile<2, MT>{}, first);
+    else tile(FewTile<4, MT>{}, first);
   }
 }
 
@@ -425,15 +427,36 @@ int hy_expert_few(void* out, const void* in, const void* w, const void* index,
       E > 65535 || n_pairs > FEW_PAIRS)
     return -2;
   if (n_pairs <= 0) return 0;
-  static const hipError_t sized = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(expert_few_kernel),
-      hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS);
-  if (sized != hipSuccess) return -1;
-  hipLaunchKernelGGL(expert_few_kernel,
-                     dim3((N + 16 * FEW_MT - 1) / (16 * FEW_MT), E),
-                     dim3(FEW_KW * 64), FEW_LDS, (hipStream_t)stream, (bf16_t*)out,
-                     (const bf16_t*)in, (const bf16_t*)w, (const int*)index,
-                     N, K, div, act, n_pairs);
+  // Outputs a tile, by what a compute unit takes in as for other products of
+  // few rows: rounds of 256 tiles of the experts that are likely used, times
+  // a tile's rows.  32, but 16 for small matrices and 80 for deep ones.  us, 32
+  // outputs -> these, 61 tokens: 1024 to 256 wide 5.4 -> 4.9, 4096 to 1280 32.2
+  // -> 29.4, 300 tokens 90 -> 62; 1280 deep 80 outputs lost (81.6 -> 90.4).
+  const float used = E * (1.f - powf(1.f - 1.f / E, (float)n_pairs));
+  const int each = (int)(n_pairs / used + 15.f) / 16;
+  auto takes = [&](int mt) {
+    const float tiles = (float)((N + 16 * mt - 1) / (16 * mt)) * used;
+    return ceilf(tiles / 256.f) * ((each < 4 ? each : 4) + mt);
+  };
+  int mt = 2;
+  if (K >= 1024 && takes(1) < 0.95f * takes(2)) mt = 1;
+  if (K >= 2048 && takes(5) < 0.95f * takes(mt)) mt = 5;
+#define GO(MT)                                                               \
+  do {                                                                       \
+    static const hipError_t sized = hipFuncSetAttribute(                     \
+        reinterpret_cast<const void*>(expert_few_kernel<MT>),                \
+        hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS<MT>);            \
+    if (sized != hipSuccess) return -1;                                      \
+    hipLaunchKernelGGL(expert_few_kernel<MT>,                                \
+                       dim3((N + 16 * MT - 1) / (16 * MT), E),               \
+                       dim3(FEW_KW * 64), FEW_LDS<MT>, (hipStream_t)stream,  \
+                       (bf16_t*)out, (const bf16_t*)in, (const bf16_t*)w,    \
+                       (const int*)index, N, K, div, act, n_pairs);          \
+  } while (0)
+  if (mt == 1) GO(1);
+  else if (mt == 5) GO(5);
+  else GO(2);
+#undef GO
   HY_CHECK();
   return 0;
 }
