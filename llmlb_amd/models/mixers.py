@@ -218,6 +218,11 @@ class ChannelDelta(nn.Module):
         self.w_in = _param(stacked.to(**to))
         self.w_a2 = _param(w["a2"].to(**to))
         self.w_g2 = _param(w["g2"].to(**to))
+        # alike, they are one launch in decoding
+        self.w_low = None
+        if w["a2"].shape == w["g2"].shape:
+            self.w_low = _param(torch.stack([self.w_a2, self.w_g2]))
+            self.w_a2, self.w_g2 = (_param(t) for t in self.w_low)
         self.w_o = _param(w["o"].to(**to))
 
         def wide(t):
@@ -234,16 +239,28 @@ class ChannelDelta(nn.Module):
 
     def forward(self, x, b, cache, index: int):
         proj = _linear(x, self.w_in)
-        dec = _linear(proj[:, self.a_off:self.a_off + self.decay_rank],
-                      self.w_a2)
-        gate = _linear(proj[:, self.g_off:self.g_off + self.gate_rank],
-                       self.w_g2)
+        dec, gate = self._low_rank(proj)
         o = hy.gated_delta(
             proj, self.b_off, dec, gate, cache.state[index],
             cache.ring[index], b, self.w_conv, self.a_log, self.dt_bias,
             self.w_norm, self.kv_heads, self.heads, self.dim, self.vdim,
             self.taps, self.eps)
         return _linear(o, self.w_o)
+
+    def _low_rank(self, proj):
+        """The second projections of decays and gates."""
+        N, K = proj.shape[0], self.decay_rank
+        if self.w_low is not None and N <= 128:
+            both = torch.empty(2, N, self.w_low.shape[1], dtype=proj.dtype,
+                               device=proj.device)
+            x = proj.as_strided((2, N, K), (self.g_off - self.a_off,
+                                            proj.stride(0), 1),
+                                proj.storage_offset() + self.a_off)
+            if linear_heads(x, self.w_low, both):
+                return both[0], both[1]
+        return (_linear(proj[:, self.a_off:self.a_off + K], self.w_a2),
+                _linear(proj[:, self.g_off:self.g_off + self.gate_rank],
+                        self.w_g2))
 
 
 class DenseFF(nn.Module):
