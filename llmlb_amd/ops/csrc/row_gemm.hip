@@ -12,7 +12,7 @@
 //   64: 1024 x 1024 8.8 -> 3.7,  1024 x 2816 9.7 -> 4.7, 2048 x 5632
 //       18.5 -> 11.8, 4096 x 4096 15.5 -> 11.9, 6144 x 4096 17.4 -> 15.9,
 //       4096 x 14336 40.7 -> 30.0 (in shares; 36.4 in one), 28672 x 4096
-//       48.9 -> 45.8 (5.1 TB/s)
+//       48.9 -> 40.0 (5.9 TB/s)
 //   16: 1024 x 1024 6.1 -> 3.5, 4096 x 4096 15.9 -> 8.2, 28672 x 4096
 //       60.9 -> 37.0 (6.3 TB/s)
 // With more rows the bound is what a compute unit takes in, about 50 GB/s:
@@ -26,7 +26,8 @@
 // outputs.
 // M outputs; CAPPED results are floats, all others bf16
 template <int NT, int MT, int KW, int S, bool GATED>
-__global__ __launch_bounds__(KW * 64, 2) void row_gemm_kernel(
+__global__ __launch_bounds__(KW * 64, NT * MT > 24 ? 1 : 2)
+void row_gemm_kernel(
     void* __restrict__ out_, int ld_out, const bf16_t* __restrict__ x,
     const bf16_t* __restrict__ w, int N, int M, int K, int ldx, RowAct act) {
   using Tile = RowTile<NT, MT, KW, S>;
@@ -151,7 +152,11 @@ static int row_gemm_launch(const RowGemm& p) {
 // outputs a tile, two rounds) -> 30.1 (80, one), 16512 x 4096 42.3 -> 28.0,
 // 10272 x 4096 30.3 -> 21.2 (48), gate and up of 11904 x 4096 45.2 -> 35.3 (96),
 // 8224 x 2048 16.4 -> 11.7; 16 rows: 12576 x 4096 21.0 -> 17.5; 128 rows: 10272 x
-// 4096 38.3 -> 27.6, gate and up of 5632 x 2048 23.2 -> 16.5.
+// 4096 38.3 -> 27.6, gate and up of 5632 x 2048 23.2 -> 16.5.  112 outputs a
+// tile are for what they fit into one round, or two: 64 rows, from tiles of 64
+// on, gate and up of 14336 x 4096 47.6 -> 39.8, 26000 x 2048 27.8 -> 22.1,
+// 57344 x 1024 (two) 31.5 -> 29.9; with five rounds they lose (40 rows, 128256
+// x 4096 170 -> 178: the card's memory is the bound).
 template <bool GATED>
 static int row_gemm_pick(const RowGemm& p) {
   const int tiles = (p.N + 15) / 16;
@@ -164,15 +169,17 @@ static int row_gemm_pick(const RowGemm& p) {
     // tiles of the same rows of W are on one of eight XCDs of 32 units
     const long long down = (rows + 16 * m - 1) / (16 * m);
     const long long count = (down + 7) / 8 * ((tiles + n - 1) / n);
-    const float takes =
-        fmaxf((float)((count + 31) / 32 * (n + m)), floor);
+    const long long rounds = (count + 31) / 32;
+    if (m == 7 && rounds > 2) return;  // memory bounds these, of any tile
+    const float takes = fmaxf((float)(rounds * (n + m)), floor);
     if (!nt || takes < 0.95f * least) least = takes, nt = n, mt = m;
   };
   // what is as good: more rows of x, which read W less often, then the sizes
   // that memory likes best
-  static const int OF_MANY[] = {4, 5, 6, 3, 2, 1}, OF_ONE[] = {2, 4, 3, 1, 5, 5};
+  static const int OF_MANY[] = {4, 5, 6, 3, 2, 1, 7};
+  static const int OF_ONE[] = {2, 4, 3, 1, 5, 5, 5};
   for (int n = tiles < 4 ? tiles : 4; n >= 1; --n)
-    for (int i = 0; i < 6; ++i) {
+    for (int i = 0; i < 7; ++i) {
       const int m = n == 1 ? OF_ONE[i] : OF_MANY[i];
       if (n < 3 || m > 1) look(n, m);  // (3, 1) and (4, 1) take in no less
     }
@@ -191,16 +198,19 @@ static int row_gemm_pick(const RowGemm& p) {
     TILE(2, 4, 4, 2)
     TILE(2, 5, 4, 2)
     TILE(2, 6, 4, 2)
+    TILE(2, 7, 4, 2)
     TILE(3, 2, 4, 2)
     TILE(3, 3, 4, 2)
     TILE(3, 4, 4, 2)
     TILE(3, 5, 4, 2)
     TILE(3, 6, 4, 2)
+    TILE(3, 7, 4, 2)
     TILE(4, 2, 4, 2)
     TILE(4, 3, 4, 2)
     TILE(4, 4, 4, 2)
     TILE(4, 5, 4, 2)
     TILE(4, 6, 4, 2)
+    TILE(4, 7, 3, 2)
   }
 #undef TILE
   return -2;
