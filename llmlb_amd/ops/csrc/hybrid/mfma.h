@@ -26,6 +26,15 @@ __device__ __forceinline__ u32x4 load_columns(const unsigned short* p,
   return u32x4{a.x, a.y, b.x, b.y};
 }
 
+// The same of bytes: lane i addresses 8 of row i / 2 (columns 8 (i % 2) ..) of
+// 8 rows of 16, and gets its column of all of them.
+typedef __attribute__((ext_vector_type(2))) int s32x2;
+typedef __attribute__((address_space(3))) s32x2 lds_s32x2;
+__device__ __forceinline__ uint2 load_byte_columns(const char* p) {
+  return __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_s32x2*)p));
+}
+
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 // two floats to bf16, nearest even

@@ -20,8 +20,10 @@
 // Against a lane per part of a row, us (sequences, heads, tokens):
 //   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 41 (5.8 TB/s),
 //     64 x 3600 255 -> 156 (6.2 TB/s), 1 x 4000 47 -> 16
-//   e4m3, the same heads: 32 x 1800 79 -> 29, 64 x 900 70 -> 26; bound
-//     by widening to bf16 beside the reads
+//   e4m3, the same heads: 32 x 2048 79 -> 28 (5.0 TB/s), 64 x 900 70 -> 21,
+//     128 x 1500 71 -> 56; values leave LDS as columns of bytes and are
+//     widened in registers.  Widened on a way back through LDS, 29, 24 and
+//     71; by two conversions to float and a permutation, 28.5, 22 and 58
 //   bf16, 16 on 4 heads of 64: 64 x 900 61 -> 15, 1 x 100 12.3 -> 5.5
 #include "hybrid/lds_copy.h"
 #include "hybrid/mfma.h"
@@ -129,7 +131,8 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
       for (int j = 0; j < A::CP; ++j) {
         stream_to_lds(reinterpret_cast<const bf16_t*>(kc + at + off[j]),
                       to + t * A::BYTES + j * 1024);
-        stream_to_lds(reinterpret_cast<const bf16_t*>(vc + at + off[j]),
+        stream_to_lds(reinterpret_cast<const bf16_t*>(
+                          vc + at + (FP8 && t ? off[j] ^ 64 : off[j])),
                       to + (2 + t) * A::BYTES + j * 1024);
       }
     }
@@ -236,35 +239,25 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
         lo[2 * t + r / 2] = l2;
       }
     }
-    const char* values = st + 2 * A::BYTES;
-    if (FP8) {  // to bf16, in rows of 256 bytes over the stage's pages
-      const int r = lane / 2, c0 = (lane & 1) * 4;
-      uint4 x[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        x[c] = *reinterpret_cast<const uint4*>(
-            values + r * A::ROW + ((c0 + c) ^ turn<A::ROW>(r & 15)) * 16);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        char* const to = st + r * 256;
-        const int p = 2 * (c0 + c);
-        *reinterpret_cast<u32x4*>(to + (p ^ (r & 15)) * 16) =
-            widen8(make_uint2(x[c].x, x[c].y));
-        *reinterpret_cast<u32x4*>(to + ((p + 1) ^ (r & 15)) * 16) =
-            widen8(make_uint2(x[c].z, x[c].w));
-      }
-      values = st;
-    }
-    constexpr int VROW = 2 * D;
-    const int r = g * 4 + (n >> 2);
+    const char* const values = st + 2 * A::BYTES;
+    // columns of four keys of either page: of e4m3 at once, and those of the
+    // second page lie turned by four pieces more, in the other banks
+    const int t = FP8 ? n >> 3 : 0;
+    const int r = g * 4 + (FP8 ? n >> 1 & 3 : n >> 2);
+    const char* const v_row = values + t * A::BYTES + r * A::ROW;
 #pragma unroll
     for (int v = 0; v < VT; ++v) {
-      const int c = 2 * v + ((n >> 1) & 1);
-      const u32x4 vf = load_columns(
-          reinterpret_cast<const unsigned short*>(
-              values + r * VROW + (c ^ turn<VROW>(r)) * 16 + (n & 1) * 8),
-          PAGE * D);
+      u32x4 vf;
+      if (FP8) {
+        vf = widen8(load_byte_columns(
+            v_row + (v ^ turn<A::ROW>(r) ^ t * 4) * 16 + (n & 1) * 8));
+      } else {
+        const int c = 2 * v + ((n >> 1) & 1);
+        vf = load_columns(
+            reinterpret_cast<const unsigned short*>(
+                v_row + (c ^ turn<A::ROW>(r)) * 16 + (n & 1) * 8),
+            PAGE * D);
+      }
       o[v] = mfma(vf, hi, o[v]);
       o[v] = mfma(vf, mid, o[v]);
       o[v] = mfma(vf, lo, o[v]);
