@@ -6,10 +6,10 @@
 // What bounds it is reading the pages once.  One workgroup per sequence,
 // key/value head, up to 16 of its query heads and part of the pages: the
 // heads are the columns of the matrix cores' tiles, so a page is read from
-// LDS once for all of them.  Its four waves work on pages of their own, two
-// at a time, without a barrier: pages are whole runs of memory, copied to
-// LDS and waited for by the wave that asked.  What hides the wait is other
-// workgroups, two or more to a compute unit; a second stage of LDS in their
+// LDS once for all of them.  Its four or eight waves work on pages of their
+// own, two at a time, without a barrier: pages are whole runs of memory,
+// copied to LDS and waited for by the wave that asked.  What hides the wait is
+// other waves, eight or more to a compute unit; a second stage of LDS in their
 // place was no faster.  Weights and sums stay floats: a weight enters its
 // product as the sum of three bf16 numbers, which are all of its 24 bits.
 //
@@ -20,10 +20,11 @@
 // Against a lane per part of a row, us (sequences, heads, tokens):
 //   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 41 (5.8 TB/s),
 //     64 x 3600 255 -> 156 (6.2 TB/s), 1 x 4000 47 -> 16
-//   e4m3, the same heads: 32 x 2048 79 -> 28 (5.0 TB/s), 64 x 900 70 -> 21,
-//     128 x 1500 71 -> 56; values leave LDS as columns of bytes and are
-//     widened in registers.  Widened on a way back through LDS, 29, 24 and
-//     71; by two conversions to float and a permutation, 28.5, 22 and 58
+//   e4m3, the same heads: 64 x 900 70 -> 21; 32 x 2048 in two parts 28, in
+//     one of eight waves 25 (5.6 TB/s), 128 x 1500 56.  Values leave LDS as
+//     columns of bytes and are widened in registers; widened on a way back
+//     through LDS 24, 29 (two parts) and 71, by two conversions to float and
+//     a permutation 22, 28.5 and 58
 //   bf16, 16 on 4 heads of 64: 64 x 900 61 -> 15, 1 x 100 12.3 -> 5.5
 #include "hybrid/lds_copy.h"
 #include "hybrid/mfma.h"
@@ -57,14 +58,14 @@ __device__ __forceinline__ u32x4 widen8(uint2 v) {
 }
 
 // A wave's place in LDS: two pages of keys, two of values
-template <int D, bool FP8>
+template <int D, bool FP8, int W>
 struct PageAttn {
   static constexpr int ROW = D * (FP8 ? 1 : 2), BYTES = PAGE * ROW;
   static constexpr int PR = ROW / 16, CP = BYTES / 1024;  // pieces, copies
   static constexpr int STAGE = 4 * BYTES + (FP8 ? 256 : 0);  // and scales
   static constexpr int OP = D + 4;  // row of the waves' results
-  static constexpr int RESULTS = 4 * 16 * OP * 4;
-  static constexpr int LDS = 4 * STAGE > RESULTS ? 4 * STAGE : RESULTS;
+  static constexpr int RESULTS = W * 16 * OP * 4;
+  static constexpr int LDS = W * STAGE > RESULTS ? W * STAGE : RESULTS;
 };
 
 // Piece c of row r lies at c ^ turn(r): lanes reading one piece of 16 rows
@@ -75,18 +76,18 @@ __device__ __forceinline__ int turn(int r) {
 }
 
 // acc [n][heads][parts][D], ml [n][heads][parts] (maximum, sum)
-template <int D, bool FP8>
-__global__ __launch_bounds__(256, 3) void page_attn_kernel(
+template <int D, bool FP8, int W>
+__global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
     bf16_t* __restrict__ out, float* __restrict__ ws_acc,
     float* __restrict__ ws_ml, const bf16_t* __restrict__ q, int ldq,
     const char* __restrict__ kc, const char* __restrict__ vc,
     const float* __restrict__ k_scale, const float* __restrict__ v_scale,
     const int* __restrict__ bt, const int* __restrict__ lens, int max_blocks,
     int H, int G, int parts, float scale) {
-  using A = PageAttn<D, FP8>;
+  using A = PageAttn<D, FP8, W>;
   constexpr int KD = D / 32, VT = D / 16;
   extern __shared__ __align__(1024) char lds[];
-  __shared__ float lm[4][16], ll[4][16];
+  __shared__ float lm[W][16], ll[W][16];
   const int R = H / G, ht = (R + 15) / 16;
   const int seq = blockIdx.x, part = blockIdx.z;
   const int kv = blockIdx.y / ht, h0 = blockIdx.y % ht * 16;
@@ -98,12 +99,12 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
   const int n = lane & 15, g = lane >> 4;
   const int heads = R - h0 < 16 ? R - h0 : 16;
 
-  // pairs of pages of this part, every fourth of this wave
+  // pairs of pages of this part, every W-th of this wave
   const int pages = (len + PAGE - 1) / PAGE, pairs = (pages + 1) / 2;
   const int per = (pairs + used - 1) / used;
   const int first = part * per + wave;
   const int stop = part * per + per < pairs ? part * per + per : pairs;
-  const int count = first < stop ? (stop - first + 3) / 4 : 0;
+  const int count = first < stop ? (stop - first + W - 1) / W : 0;
   char* const st = lds + wave * A::STAGE;
   const unsigned to = lds_byte(st);
   const int* const row = bt + (size_t)seq * max_blocks;
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
   // pages of 32 pairs, in lanes
   int ids = 0;
   auto look_up = [&](int i) {
-    const int p = 2 * (first + (i + lane / 2) * 4) + (lane & 1);
+    const int p = 2 * (first + (i + lane / 2) * W) + (lane & 1);
     ids = row[p < pages ? p : pages - 1];
   };
   // source of lane's piece in copy j of a page
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
 
   for (int i = 0; i < count; ++i) {
     wait_copies<0>();
-    const int j0 = (first + i * 4) * 32;  // the pair's first key
+    const int j0 = (first + i * W) * 32;  // the pair's first key
     if (j0 + 32 > len) {
       // rows past the end: an earlier sequence may have left anything there
       const int r = lane / 2;
@@ -282,14 +283,14 @@ __global__ __launch_bounds__(256, 3) void page_attn_kernel(
           &res[(wave * 16 + n) * A::OP + v * 16 + g * 4]) = o[v];
   }
   __syncthreads();
-  for (int i = tid; i < heads * (D / 4); i += 256) {
+  for (int i = tid; i < heads * (D / 4); i += W * 64) {
     const int h = i / (D / 4), c = i % (D / 4) * 4;
     float top = lm[0][h], sum = 0.f;
 #pragma unroll
-    for (int w = 1; w < 4; ++w) top = fmaxf(top, lm[w][h]);
+    for (int w = 1; w < W; ++w) top = fmaxf(top, lm[w][h]);
     f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < W; ++w) {
       const float f = __builtin_amdgcn_exp2f(lm[w][h] - top);
       sum += f * ll[w][h];
       x += *reinterpret_cast<const f32x4*>(&res[(w * 16 + h) * A::OP + c]) * f;
@@ -336,21 +337,21 @@ __global__ __launch_bounds__(256) void page_join_kernel(
       to_bf16x2(x[0] * f, x[1] * f), to_bf16x2(x[2] * f, x[3] * f));
 }
 
-template <int D, bool FP8>
+template <int D, bool FP8, int W>
 static int page_attn_launch(void* out, void* acc, void* ml, const void* q,
                             int ldq, const void* kc, const void* vc,
                             const void* ks, const void* vs, const void* bt,
                             const void* lens, int n, int max_blocks, int H,
                             int G, int parts, float scale, hipStream_t st) {
-  constexpr int lds = PageAttn<D, FP8>::LDS;
+  constexpr int lds = PageAttn<D, FP8, W>::LDS;
   static_assert(lds + 512 <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(page_attn_kernel<D, FP8>),
+      reinterpret_cast<const void*>(page_attn_kernel<D, FP8, W>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (sized != hipSuccess) return -1;
   const int tiles = G * ((H / G + 15) / 16);
-  hipLaunchKernelGGL((page_attn_kernel<D, FP8>), dim3(n, tiles, parts),
-                     dim3(256), lds, st, (bf16_t*)out, (float*)acc,
+  hipLaunchKernelGGL((page_attn_kernel<D, FP8, W>), dim3(n, tiles, parts),
+                     dim3(W * 64), lds, st, (bf16_t*)out, (float*)acc,
                      (float*)ml, (const bf16_t*)q, ldq, (const char*)kc,
                      (const char*)vc, (const float*)ks, (const float*)vs,
                      (const int*)bt, (const int*)lens, max_blocks, H, G,
@@ -382,10 +383,24 @@ extern "C" int ll_page_attn(void* out, void* acc, void* ml, const void* q,
   if ((ks != nullptr) != (vs != nullptr) || (ks && D != 128)) return -2;
   if (n == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-#define PAGE_ATTN(D, FP8)                                                   \
-  return page_attn_launch<D, FP8>(out, acc, ml, q, ldq, kc, vc, ks, vs, \
-                                     bt, lens, n, max_blocks, H, G, parts, \
-                                     scale, st)
+  // Two parts of four waves are one of eight, with no results to join, where
+  // whole ones leave compute units idle no longer than halves do.  Two parts
+  // -> one, us, 32 sequences of 2048 and of up to 300 tokens, 32 heads on 8 of
+  // 128: bf16 46.2 -> 43.5, 12.6 -> 9.1; e4m3 27.8 -> 24.9, 9.0 -> 6.6; 64 of
+  // 3000, 16 on 4 of 64: 29.9 -> 27.8.
+  const long long count = (long long)n * G * ((H / G + 15) / 16);
+  const bool whole = parts == 2 && (count + 255) / 256 * 2 <=
+                                       (2 * count + 255) / 256;
+#define PAGE_ATTN(D, FP8)                                                    \
+  do {                                                                       \
+    if (whole)                                                               \
+      return page_attn_launch<D, FP8, 8>(out, acc, ml, q, ldq, kc, vc, ks,   \
+                                         vs, bt, lens, n, max_blocks, H, G,  \
+                                         1, scale, st);                      \
+    return page_attn_launch<D, FP8, 4>(out, acc, ml, q, ldq, kc, vc, ks, vs, \
+                                       bt, lens, n, max_blocks, H, G, parts, \
+                                       scale, st);                           \
+  } while (0)
   if (ks) PAGE_ATTN(128, true);
   if (D == 128) PAGE_ATTN(128, false);
   if (D == 64) PAGE_ATTN(64, false);

@@ -142,3 +142,17 @@ def test_weights_are_floats(D, fp8):
     ref, _ = _exact(q, k, v, bt, lens, 1.0)
     bound = ref.abs() * 2.0 ** -8 + 8 * 2.0 ** -24
     assert ((out.double() - ref).abs() <= bound).all()
+
+
+# one part of eight waves (144 and 256 workgroups) or two of four (128 and
+# 320), of sequences with fewer pages than waves and with more
+@pytest.mark.parametrize("kv", [8, 9, 16, 20])
+@pytest.mark.parametrize("D", [64, 128])
+def test_two_parts(kv, D):
+    q, k, v, bt, lens, _ = _case(2 * kv, kv, D, kv + D)
+    k, v = k.bfloat16(), v.bfloat16()
+    ref, bound = _exact(q, k, v, bt, lens, D ** -0.5)
+    out = ops.paged_attn_decode(q, k, v, bt, lens, D ** -0.5, n_parts=2)
+    assert ((out.double() - ref).abs() <= bound).all()
+    if D == 128:
+        test_page_attention_fp8(2 * kv, kv, 2)
