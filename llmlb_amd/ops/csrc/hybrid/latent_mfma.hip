@@ -612,25 +612,43 @@ void latent_decode_kernel(
   }
 }
 
-__global__ __launch_bounds__(256) void latent_merge_kernel(
+// Joins a head's parts, four columns a thread.  Each lane has one part's
+// weight, and the parts' sums are asked for four at a time: what bounds this
+// is a chain of loads.  us, loads one after the other -> now: 10 parts of 24
+// sequences 8.4 -> 5.4, four of 64 6.3 -> 5.2.
+__global__ __launch_bounds__(128) void latent_merge_kernel(
     bf16_t* __restrict__ out, const float* __restrict__ ws_acc,
     const float* __restrict__ ws_ml, int rank, int H, int N, int parts) {
-  const int q = blockIdx.x, h = blockIdx.y;
+  const int q = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
   const size_t at = ((size_t)q * H + h) * parts;
+  const float2* const ml = reinterpret_cast<const float2*>(ws_ml) + at;
   float mx = -1e30f;
-  for (int p = 0; p < parts; ++p) mx = fmaxf(mx, ws_ml[(at + p) * 2]);
+  for (int p = lane; p < parts; p += 64) mx = fmaxf(mx, ml[p].x);
+#pragma unroll
+  for (int i = 32; i; i >>= 1) mx = fmaxf(mx, __shfl_xor(mx, i, WAVE));
+  const int d = threadIdx.x * 4;  // rank <= 512, a multiple of 8
+  const float* const acc = ws_acc + at * rank + (d < rank ? d : 0);
   float sum = 0.f;
-  for (int p = 0; p < parts; ++p)
-    sum += ws_ml[(at + p) * 2 + 1] *
-           __builtin_amdgcn_exp2f(ws_ml[(at + p) * 2] - mx);
-  const float inv = 1.f / sum;
-  for (int d = threadIdx.x; d < rank; d += 256) {
-    float v = 0.f;
-    for (int p = 0; p < parts; ++p)
-      v += ws_acc[(at + p) * rank + d] *
-           __builtin_amdgcn_exp2f(ws_ml[(at + p) * 2] - mx);
-    out[((size_t)h * N + q) * rank + d] = from_f<bf16_t>(v * inv);
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < parts; p0 += 64) {
+    float f = 0.f;
+    if (p0 + lane < parts) {
+      const float2 x = ml[p0 + lane];
+      f = __builtin_amdgcn_exp2f(x.x - mx);
+      sum += x.y * f;
+    }
+    const int n = parts - p0 < 64 ? parts - p0 : 64;
+#pragma unroll 4
+    for (int i = 0; i < n; ++i)
+      v += *reinterpret_cast<const f32x4*>(acc + (size_t)(p0 + i) * rank) *
+           __shfl(f, i, WAVE);
   }
+#pragma unroll
+  for (int i = 32; i; i >>= 1) sum += __shfl_xor(sum, i, WAVE);
+  if (d >= rank) return;
+  const float inv = 1.f / sum;
+  *reinterpret_cast<uint2*>(out + ((size_t)h * N + q) * rank + d) =
+      make_uint2(pack2(v[0] * inv, v[1] * inv), pack2(v[2] * inv, v[3] * inv));
 }
 
 template <int NT, int HT>
@@ -654,7 +672,7 @@ static int launch_decode(void* out, void* acc, void* ml, const void* qa,
                      scale * LOG2E, (const float*)sink, N, parts);
   HY_CHECK();
   if (parts > 1) {
-    hipLaunchKernelGGL(latent_merge_kernel, dim3(N, H), block, 0, s,
+    hipLaunchKernelGGL(latent_merge_kernel, dim3(N, H), dim3(128), 0, s,
                        (bf16_t*)out, (const float*)acc, (const float*)ml,
                        rank, H, N, parts);
     HY_CHECK();

@@ -198,6 +198,12 @@ def test_decode_parts(parts, heads, monkeypatch):
         close(got[i][0], want[-1], B16)
 
 
+# fewer parts than a wave has lanes, as many, more
+@pytest.mark.parametrize("parts", [4, 63, 64, 65, 130])
+def test_many_parts(parts, monkeypatch):
+    test_decode_parts(parts, 7, monkeypatch)
+
+
 # -- gated delta rule alone ------------------------------------------------
 
 def delta_case(heads, kv_heads, dim, vdim, taps, width, seed):
