@@ -281,3 +281,28 @@ def test_planted_scores(window):
         other = dict(spec, mask={"size": window + off})
         wrong = O.latent_attention(h, w, "", other, 1e-5)[0]
         assert (wrong - want).abs().amax(-1)[[T - 1, T - 3]].max() > 0.05
+
+
+def test_copies_of_weights_are_no_part_of_a_saved_state():
+    """A state holds weights and what was always in it; copies that decoding
+    reads follow a loaded one, in the memory that a graph may have seen."""
+    layers = [U.latent(2, 16, 8, 16, 24, 19),
+              U.delta(4, 4, 16, 16, 2, low=(16, 16))]
+    cfg = U.config(layers, vocab=97, width=64, ff=96)
+
+    def mixers(seed):
+        w = U.weights(cfg, seed=seed)
+        return [make(ly["mixer"], {k[len(f"l{i}.mix."):]: t
+                                   for k, t in w.items()
+                                   if k.startswith(f"l{i}.mix.")}, 1e-5, 64)
+                for i, (ly, make) in enumerate(zip(
+                    layers, [U.latent_mixer, U.delta_mixer]))]
+
+    for one, two, name in zip(mixers(1), mixers(2), ["w_uk_t", "w_low"]):
+        copy = getattr(one, name)
+        place, saved = copy.data_ptr(), two.state_dict()
+        assert name not in saved and name not in dict(one.named_parameters())
+        assert not torch.equal(copy, getattr(two, name))
+        one.load_state_dict(saved)
+        assert torch.equal(getattr(one, name), getattr(two, name))
+        assert getattr(one, name).data_ptr() == place
