@@ -311,26 +311,56 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
   }
 }
 
-// Joins the parts of sequences that used several; D / 4 lanes a head.
+// Joins the parts of sequences that used several; D / 4 lanes a head, each
+// with one part's weight.  Four parts are asked for at a time, the first before
+// the weights are there: what bounds this is a chain of loads.  us of attention
+// with parts, loads one after the other -> now: 32 heads on 8 of 128, 8
+// sequences of 1000 tokens 11.7 -> 10.8, 16 of 2048 25.2 -> 24.4; 16 on 4 of 64,
+// 4 of 3000 11.5 -> 8.8.
 template <int D>
 __global__ __launch_bounds__(256) void page_join_kernel(
     bf16_t* __restrict__ out, const float* __restrict__ ws_acc,
     const float* __restrict__ ws_ml, const int* __restrict__ lens, int n_rows,
     int H, int parts) {
+  constexpr int LANES = D / 4;
+  const int lane = threadIdx.x % LANES;
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const size_t at = i / D;
   if (at >= (size_t)n_rows * H) return;
   const int used = parts_used(lens[at / H], parts);
   if (used == 1) return;
-  const float* ml = ws_ml + at * parts * 2;
+  const float2* ml = reinterpret_cast<const float2*>(ws_ml) + at * parts;
   const float* acc = ws_acc + at * parts * D + i % D;
+  f32x4 part[4];
+  auto ask = [&](int p0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int p = p0 + j < used ? p0 + j : used - 1;
+      part[j] = *reinterpret_cast<const f32x4*>(acc + (size_t)p * D);
+    }
+  };
+  ask(0);
   float top = -1e30f, sum = 0.f;
-  for (int p = 0; p < used; ++p) top = fmaxf(top, ml[2 * p]);
+  for (int p = lane; p < used; p += LANES) top = fmaxf(top, ml[p].x);
+#pragma unroll
+  for (int k = LANES / 2; k; k >>= 1)
+    top = fmaxf(top, __shfl_xor(top, k, LANES));
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < used; ++p) {
-    const float f = __builtin_amdgcn_exp2f(ml[2 * p] - top);
-    sum += f * ml[2 * p + 1];
-    x += *reinterpret_cast<const f32x4*>(acc + (size_t)p * D) * f;
+  float w = 0.f, l = 0.f;
+  for (int p0 = 0; p0 < used; p0 += 4) {
+    if (p0 % LANES == 0) {
+      const float2 v = ml[p0 + lane < used ? p0 + lane : used - 1];
+      w = __builtin_amdgcn_exp2f(v.x - top);
+      l = v.y;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (p0 + j >= used) break;
+      const float f = __shfl(w, (p0 + j) % LANES, LANES);
+      sum += f * __shfl(l, (p0 + j) % LANES, LANES);
+      x += part[j] * f;
+    }
+    if (p0 + 4 < used) ask(p0 + 4);
   }
   const float f = sum > 0.f ? 1.f / sum : 0.f;
   *reinterpret_cast<uint2*>(out + i) = make_uint2(
