@@ -102,7 +102,9 @@ __global__ __launch_bounds__(KW * 64, 2) void row_gemm_share_kernel(
   });
 }
 
-// out = the sum of the shares, four outputs a thread
+// out = the sum of the shares, four outputs a thread.  Four shares are asked
+// for at a time: what bounds this is a chain of loads.  us with the product, one
+// after the other -> now: 64 rows of 4096 x 14336 28.5 -> 28.1, 32 25.1 -> 24.4.
 __global__ __launch_bounds__(256) void row_gemm_join_kernel(
     bf16_t* __restrict__ out, int ld_out, const float* __restrict__ ws, int N,
     int M, int shares) {
@@ -110,8 +112,18 @@ __global__ __launch_bounds__(256) void row_gemm_join_kernel(
   if (n >= N) return;
   const int m = (i - n * (M / 4)) * 4;
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < shares; ++s)
-    v += *reinterpret_cast<const f32x4*>(ws + ((size_t)s * N + n) * M + m);
+  for (int s0 = 0; s0 < shares; s0 += 4) {
+    f32x4 part[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = s0 + i < shares ? s0 + i : shares - 1;
+      part[i] =
+          *reinterpret_cast<const f32x4*>(ws + ((size_t)s * N + n) * M + m);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s0 + i < shares) v += part[i];
+  }
   *reinterpret_cast<uint2*>(out + (size_t)n * ld_out + m) =
       make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
 }
