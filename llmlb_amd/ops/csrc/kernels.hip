@@ -67,13 +67,18 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
 //   if residual != nullptr:  residual += x;  x' = residual  (updated in place)
 //   out = x' * rsqrt(mean(x'^2) + eps) * weight
 // One 256-thread block per token row; fp32 accumulation; bf16x8 loads.
+// Decoding has a row for every fourth compute unit, and its time is a chain
+// of loads: up to RMS_KEEP vectors a thread and their weights are asked for at
+// once, and stay in registers for the second pass.  A decoding step of 64
+// sequences of 1024 tokens, with 8 norms of 4096 columns: 654.6 -> 648.1 us;
+// 16384 rows, as before: 83 us (4.8 TB/s).
 // ---------------------------------------------------------------------------
+#define RMS_KEEP 2
 template <bool FUSE_RESIDUAL>
-__global__ void rmsnorm_kernel(bf16* __restrict__ out,
-                               const bf16* __restrict__ in,
-                               const bf16* __restrict__ weight,
-                               bf16* __restrict__ residual,
-                               int hidden, float eps) {
+__global__ __launch_bounds__(256) void rmsnorm_kernel(
+    bf16* __restrict__ out, const bf16* __restrict__ in,
+    const bf16* __restrict__ weight, bf16* __restrict__ residual, int hidden,
+    float eps) {
   const int row = blockIdx.x;
   const uint4* inv = reinterpret_cast<const uint4*>(in + (size_t)row * hidden);
   uint4* resv = FUSE_RESIDUAL
@@ -83,28 +88,41 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
   const int nvec = hidden >> 3;  // uint4 = 8 bf16
 
   float ssq = 0.f;
-  // pass 1: (residual add +) sum of squares.  Rows are at most a few K
-  // elements (hidden 4096..16384) so keep the row in registers when it
-  // fits one iteration, else re-read (L1/L2-resident on pass 2).
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-    uint4 v = inv[i];
+  // (residual add +) sum of squares of a vector
+  auto first = [&](int i, uint4 v, uint4 res) {
     float f[8];
     unpack8(v, f);
     if (FUSE_RESIDUAL) {
       float r[8];
-      unpack8(resv[i], r);
+      unpack8(res, r);
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] += r[j];
-      uint4 packed = pack8(f);
-      resv[i] = packed;  // residual stream carries the sum forward
+      v = pack8(f);
+      resv[i] = v;  // residual stream carries the sum forward
       // the norm consumes the STORED (bf16-rounded) residual, so the
-      // sum of squares must use the rounded values too (pass 2 re-reads
-      // resv) — otherwise rrms is computed against different data
-      unpack8(packed, f);
+      // sum of squares must use the rounded values too
+      unpack8(v, f);
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) ssq += f[j] * f[j];
+    return v;
+  };
+  uint4 keep[RMS_KEEP], res[RMS_KEEP], w[RMS_KEEP];
+#pragma unroll
+  for (int n = 0; n < RMS_KEEP; ++n)
+    if (n * 256 < nvec) {
+      const int i = threadIdx.x + n * 256, at = i < nvec ? i : nvec - 1;
+      keep[n] = inv[at];
+      if (FUSE_RESIDUAL) res[n] = resv[at];
+      w[n] = wv[at];
+    }
+#pragma unroll
+  for (int n = 0; n < RMS_KEEP; ++n) {
+    const int i = threadIdx.x + n * 256;
+    if (i < nvec) keep[n] = first(i, keep[n], res[n]);
   }
+  for (int i = threadIdx.x + RMS_KEEP * 256; i < nvec; i += 256)
+    first(i, inv[i], FUSE_RESIDUAL ? resv[i] : uint4{});
   // wave reduce then cross-wave via LDS
   for (int off = 32; off > 0; off >>= 1) ssq += __shfl_xor(ssq, off, WAVE);
   __shared__ float warp_ssq[4];
@@ -117,15 +135,22 @@ __global__ void rmsnorm_kernel(bf16* __restrict__ out,
   for (int w = 0; w < 4; ++w) total += (w < nw) ? warp_ssq[w] : 0.f;
   const float rrms = rsqrtf(total / hidden + eps);
 
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-    uint4 v = FUSE_RESIDUAL ? resv[i] : inv[i];
-    float f[8], w[8];
+  auto second = [&](int i, uint4 v, uint4 weights) {
+    float f[8], g[8];
     unpack8(v, f);
-    unpack8(wv[i], w);
+    unpack8(weights, g);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = f[j] * rrms * w[j];
+    for (int j = 0; j < 8; ++j) f[j] = f[j] * rrms * g[j];
     outv[i] = pack8(f);
+  };
+#pragma unroll
+  for (int n = 0; n < RMS_KEEP; ++n) {
+    const int i = threadIdx.x + n * 256;
+    if (i < nvec) second(i, keep[n], w[n]);
   }
+  // beyond them a thread reads back what it wrote itself
+  for (int i = threadIdx.x + RMS_KEEP * 256; i < nvec; i += 256)
+    second(i, FUSE_RESIDUAL ? resv[i] : inv[i], wv[i]);
 }
 
 // ---------------------------------------------------------------------------

@@ -45,6 +45,25 @@ def test_rmsnorm_fused_residual():
     assert _mx(r_out.cpu(), exp_r) < 2e-2
 
 
+@pytest.mark.parametrize("hidden", [8, 2040, 2056, 4096, 4104, 6152])
+@pytest.mark.parametrize("fused", [False, True])
+def test_rmsnorm_at_the_edges_of_what_threads_keep(hidden, fused):
+    torch.manual_seed(hidden)
+    x, r = torch.randn(2, 3, hidden, device=DEV).bfloat16()
+    w = torch.randn(hidden, device=DEV).bfloat16()
+    out, stream = ops.rmsnorm(x, w, 1e-5, residual=r.clone() if fused
+                              else None)
+    norm = x + r if fused else x
+    if fused:
+        assert torch.equal(stream, norm)
+    n = norm.double()
+    want = n * (n.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    # bf16 has 8 bits of a number: rounding moves it by up to 2^-8 of its
+    # size; float sums add up to 1e-5
+    assert ((out.double() - want).abs() <= want.abs() * (2 ** -8 + 1e-5)
+            + 1e-30).all()
+
+
 @pytest.mark.parametrize("tokens,nq,nkv,D", [(5, 32, 8, 128), (64, 16, 4, 64),
                                              (3, 8, 8, 128)])
 def test_rope(tokens, nq, nkv, D):
