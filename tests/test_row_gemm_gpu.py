@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import llmlb_amd.ops as ops
+from llmlb_amd.ops import hybrid as hy
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -144,6 +145,38 @@ def test_row_gemm_with_activation(N, M, K, act, a, b):
         bound = bound + ref.abs() * 2.0 ** -8
         assert (wide[:, :8] == 7).all() and (wide[:, 8 + M:] == 7).all()
     assert ((out.double() - ref).abs() <= bound).all()
+
+
+# of few rows and of many
+@pytest.mark.parametrize("act", ["gelu", "swiglu", "clamped"])
+@pytest.mark.parametrize("N", [16, 130])
+def test_activations_are_those_of_their_own_kernels(N, act):
+    """To the bit, of every finite gate beside N numbers: divisions are a
+    float's, and what underflows is what does there."""
+    z = torch.arange(65536, device=DEV, dtype=torch.int32).to(
+        torch.uint16).view(torch.bfloat16)
+    z = z[z.isfinite()]
+    M = z.numel()
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.zeros(N, 64, device=DEV, dtype=torch.bfloat16)
+    x[:, 5] = 1.0
+    x[:, 6] = torch.randn(N, generator=g, device=DEV).mul_(3.0)
+    w = torch.zeros(M if act == "gelu" else 2 * M, 64, device=DEV,
+                    dtype=torch.bfloat16)
+    w[:M, 5] = z
+    w[M:, 6] = 1.0
+    if act == "gelu":
+        want = hy.gelu_tanh_(z.repeat(N, 1))
+    else:
+        both = torch.cat([z.repeat(N, 1), x[:, 6:7].expand(N, M)], 1)
+        want = torch.empty(N, M, device=DEV, dtype=torch.bfloat16)
+        if act == "swiglu":
+            want = ops.swiglu(both)
+        else:
+            hy.clamped_swiglu(want, both, M, 7.0, 1.702)
+    out = ops.linear_act(x, w, act, None, 0 if act == "gelu" else M, 7.0,
+                         1.702)
+    assert torch.equal(out, want)
 
 
 # heads, outputs, depth: one and two pieces of the depth, remainders of both
