@@ -31,20 +31,6 @@ def _linear(x, w):
     return linear_decode(x, w) if x.shape[0] <= 128 else linear_rows(x, w)
 
 
-def _derive(module, *_):
-    """Copies of weights in another layout: no part of a saved state, and
-    made again, where they lie, after one has been loaded."""
-    if not hasattr(module, "w_in"):
-        return                         # without weights so far
-    for name, t in module.derived().items():
-        held = getattr(module, name, None)
-        if (held is not None and t is not None and held.shape == t.shape
-                and held.dtype == t.dtype and held.device == t.device):
-            held.copy_(t)
-        else:
-            module.register_buffer(name, t, persistent=False)
-
-
 def _param(t):
     return nn.Parameter(t, requires_grad=False)
 
@@ -97,7 +83,6 @@ class LatentAttention(nn.Module):
         self.tiled = hy.can_decode_tiled(dtype, dim, rot_dim, kv_rank)
         self.flash = hy.can_flash(dtype, dim, rot_dim, kv_rank, vdim)
         self.cos_sin = None            # set by the model, [max_pos, rot]
-        self.register_load_state_dict_post_hook(_derive)
 
     def weight_shapes(self) -> dict[str, tuple]:
         H, R = self.heads, self.rank
@@ -138,16 +123,12 @@ class LatentAttention(nn.Module):
             if self.sink else None
         self.w_uk = _param(w["uk"].reshape(
             self.heads, self.dim, self.rank).to(**to).contiguous())
-        _derive(self)
         uv = w["uv"].reshape(self.heads, self.vdim, self.rank).to(**to)
         self.w_uv = _param(uv.contiguous())
         self.w_uv_t = _param(uv.transpose(1, 2).contiguous())
         self.w_o = _param(w["o"].to(**to))
         self.w_norm = _param(w["dkv.norm"].float().to(self.device)) \
             if own else None
-
-    def derived(self) -> dict[str, torch.Tensor]:
-        return {"w_uk_t": self.w_uk.transpose(1, 2).contiguous()}
 
     def cache_spec(self):
         return PageSpec(self.rank + self.rot) \
@@ -181,7 +162,7 @@ class LatentAttention(nn.Module):
             1, (H, D + self.rot))[..., :D].transpose(0, 1)
         qa = torch.empty(H, n, self.rank, dtype=proj.dtype,
                          device=proj.device)
-        if not linear_heads(q, self.w_uk_t, qa):
+        if not linear_heads(q, self.w_uk, qa, down=True):
             qa = torch.bmm(q, self.w_uk)
         attend = hy.latent_decode if self.tiled and proj.is_cuda \
             else hy.latent_rows
@@ -215,7 +196,6 @@ class ChannelDelta(nn.Module):
         self.taps, self.eps, self.width = taps, eps, width
         self.decay_rank, self.gate_rank = decay_rank, gate_rank
         self.dtype, self.device = dtype, device
-        self.register_load_state_dict_post_hook(_derive)
 
     def weight_shapes(self) -> dict[str, tuple]:
         W, qk, v = self.width, self.kv_heads * self.dim, \
@@ -237,7 +217,6 @@ class ChannelDelta(nn.Module):
         self.w_in = _param(stacked.to(**to))
         self.w_a2 = _param(w["a2"].to(**to))
         self.w_g2 = _param(w["g2"].to(**to))
-        _derive(self)
         self.w_o = _param(w["o"].to(**to))
 
         def wide(t):
@@ -247,12 +226,6 @@ class ChannelDelta(nn.Module):
             [w["q.conv"], w["k.conv"], w["v.conv"]]).t())   # [taps, C]
         self.a_log, self.dt_bias = wide(w["A_log"]), wide(w["dt_bias"])
         self.w_norm = wide(w["norm"])
-
-    def derived(self) -> dict[str, torch.Tensor | None]:
-        # alike, they are one launch in decoding
-        alike = self.w_a2.shape == self.w_g2.shape
-        return {"w_low": torch.stack([self.w_a2, self.w_g2])
-                if alike else None}
 
     def cache_spec(self):
         C = 2 * self.kv_heads * self.dim + self.heads * self.vdim
@@ -269,15 +242,16 @@ class ChannelDelta(nn.Module):
         return _linear(o, self.w_o)
 
     def _low_rank(self, proj):
-        """The second projections of decays and gates."""
+        """The second projections of decays and gates; alike, they are one
+        launch in decoding."""
         N, K = proj.shape[0], self.decay_rank
-        if self.w_low is not None and N <= 128:
-            both = torch.empty(2, N, self.w_low.shape[1], dtype=proj.dtype,
+        if N <= 128 and self.w_a2.shape == self.w_g2.shape:
+            both = torch.empty(2, N, self.w_a2.shape[0], dtype=proj.dtype,
                                device=proj.device)
             x = proj.as_strided((2, N, K), (self.g_off - self.a_off,
                                             proj.stride(0), 1),
                                 proj.storage_offset() + self.a_off)
-            if linear_heads(x, self.w_low, both):
+            if linear_heads(x, (self.w_a2, self.w_g2), both):
                 return both[0], both[1]
         return (_linear(proj[:, self.a_off:self.a_off + K], self.w_a2),
                 _linear(proj[:, self.g_off:self.g_off + self.gate_rank],

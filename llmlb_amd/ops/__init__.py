@@ -856,23 +856,31 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, weight) if out is None else out
 
 
-def linear_heads(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
-                 gate: torch.Tensor | None = None) -> bool:
+def linear_heads(x: torch.Tensor, weight, out: torch.Tensor,
+                 gate: torch.Tensor | None = None,
+                 down: bool = False) -> bool:
     """out[h] = x[h] @ weight[h]^T of up to 128 bf16 rows for all heads in
     one launch, times the sigmoid of ``gate``; False where row_gemm.hip does
     not take it.  x [H, N, K] and out [H, N, M] may be views whose last
-    dimension is dense, weight [H, M, K], gate [N, H * M]."""
+    dimension is dense, weight [H, M, K] or the matrices of two heads, gate
+    [N, H * M].  ``down``: weight [H, K, M], out[h] = x[h] @ weight[h]."""
+    pair = weight if isinstance(weight, tuple) else (weight,)
     if not (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
-            and x.dim() == weight.dim() == out.dim() == 3
-            and _only_numbers(x, weight, out)):
+            and x.dim() == out.dim() == 3
+            and all(w.dim() == 4 - len(pair) for w in pair)
+            and _only_numbers(x, out, *pair)):
         return False
-    (H, N, K), M = x.shape, weight.shape[1]
+    (H, N, K), M = x.shape, out.shape[2]
+    shape = (K, M) if down else (M, K)
     if (_USE_CUSTOM_DECODE_GEMM != "auto" or not 0 < N <= 128
-            or weight.shape != (H, M, K) or out.shape != (H, N, M)
-            or weight.dtype != x.dtype or out.dtype != x.dtype
-            or not weight.is_contiguous() or x.stride(2) != 1
-            or out.stride(2) != 1
-            or not x.device == weight.device == out.device):
+            or out.shape != (H, N, M) or out.dtype != x.dtype
+            or len(pair) == 2 and H != 2
+            or any(w.shape[-2:] != shape or w.dtype != x.dtype
+                   or w.dim() == 3 and w.shape[0] != H
+                   or not w.is_contiguous() or w.device != x.device
+                   for w in pair)
+            or x.stride(2) != 1 or out.stride(2) != 1
+            or x.device != out.device):
         return False
     if gate is not None and (
             gate.shape != (N, H * M) or gate.stride(1) != 1
@@ -882,7 +890,8 @@ def linear_heads(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor,
     rc = _lib.ll_head_gemm(
         _ptr(out), ctypes.c_int(out.stride(1)), ctypes.c_int(out.stride(0)),
         _ptr(x), ctypes.c_int(x.stride(1)), ctypes.c_int(x.stride(0)),
-        _ptr(weight), None if gate is None else _ptr(gate),
+        _ptr(pair[0]), _ptr(pair[1]) if len(pair) == 2 else None,
+        ctypes.c_int(down), None if gate is None else _ptr(gate),
         ctypes.c_int(0 if gate is None else gate.stride(0)), ctypes.c_int(H),
         ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K), _stream())
     if rc == -2:

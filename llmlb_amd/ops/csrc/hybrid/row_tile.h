@@ -25,9 +25,12 @@ struct RowTile {
 
   // x_row(r), w_row(r): where the tile's row r of x, of W begins; ``step``:
   // any number, workgroups' differ.  The waves' sums are in LDS after it.
-  template <class X, class W>
+  // DOWN: W's depth goes down, w_row(r) is where r's column begins, r a
+  // multiple of 8, and its next number lies ld numbers further.
+  template <bool DOWN = false, class X, class W>
   static __device__ __forceinline__ void run(char* lds, int K, int step,
-                                             X x_row, W w_row) {
+                                             X x_row, W w_row, int ld = 0) {
+    static_assert(!DOWN || MT % 2 == 0, "pieces that turn in twos");
     const int tid = threadIdx.x, lane = tid & 63;
     const int lo = lane & 15, hi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
@@ -35,11 +38,19 @@ struct RowTile {
     const unsigned own_byte = lds_byte(own);
     // Copy j of a stage fills rows 8 j .. 8 j + 7, 8 lanes a row.  Piece c
     // of 16 bytes of row r lies at c ^ (r / 2 % 8): lanes reading one piece
-    // of 16 rows meet every bank once.
+    // of 16 rows meet every bank once.  DOWN: of W, 2 MT lanes a number of
+    // the depth; pieces turn by two, so that two of the four blocks of eight
+    // that are read at once meet other banks.
     const bf16_t* src[C];
     int piece[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) {
+      if (DOWN && j >= 2 * NT) {
+        const int at = (j - 2 * NT) * 64 + lane, k = at / (2 * MT);
+        piece[j] = k;
+        src[j] = w_row((at % (2 * MT) ^ (k >> 2 & 2)) * 8) + (size_t)k * ld;
+        continue;
+      }
       const int r = 8 * j + lane / 8;
       piece[j] = ((lane & 7) ^ ((r >> 1) & 7)) * 8;
       src[j] = (j < 2 * NT ? x_row(r) : w_row(r - 16 * NT)) + piece[j];
@@ -54,10 +65,12 @@ struct RowTile {
 #pragma unroll
       for (int j = 0; j < C; ++j) {
         // past the depth both sides are zero
+        const size_t along = DOWN && j >= 2 * NT ? (size_t)k0 * ld : k0;
         const bf16_t* p = k0 + piece[j] < K
-                              ? src[j] + k0
+                              ? src[j] + along
                               : reinterpret_cast<const bf16_t*>(zero_piece);
-        if (j < 2 * NT)
+        // (several tiles read columns' lines)
+        if (j < 2 * NT || DOWN)
           copy_to_lds(p, to + j * 1024);
         else
           stream_to_lds(p, to + j * 1024);
@@ -88,10 +101,18 @@ struct RowTile {
 #pragma unroll
         for (int b = 0; b < NT; ++b)
           xf[s][b] = *reinterpret_cast<const u32x4*>(st + b * 2048 + at);
+        const char* const down = st + NT * 2048 +
+                                 (s * 32 + hi * 8 + lo / 4) * (32 * MT) +
+                                 (lo & 1) * 8;
 #pragma unroll
         for (int a = 0; a < MT; ++a)
           wf[s][a] =
-              *reinterpret_cast<const u32x4*>(st + (NT + a) * 2048 + at);
+              DOWN ? load_columns(
+                         reinterpret_cast<const unsigned short*>(
+                             down + ((2 * a + (lo >> 1 & 1)) ^ (hi & 1) * 2) *
+                                        16),
+                         4 * 16 * MT)
+                   : *reinterpret_cast<const u32x4*>(st + (NT + a) * 2048 + at);
       }
 #pragma unroll
       for (int s = 0; s < 2; ++s)

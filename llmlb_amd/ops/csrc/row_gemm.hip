@@ -316,37 +316,41 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
 }
 
 // The same for H pairs of rows and matrices at once, as latent attention needs
-// for its heads: out[h] = x[h] W[h]^T, W [H][M][K].  x's and out's heads lie
-// xs and os numbers apart.  With a gate, out = bf16(sum) sigmoid(gate), the
+// for its heads: out[h] = x[h] W[h]^T, W [H][M][K], or out[h] = x[h] W[h], W
+// [H][K][M] (DOWN).  x's and out's heads lie xs and os numbers apart; with w2
+// there are two matrices, which lie anywhere.  With a gate, out = bf16(sum) sigmoid(gate), the
 // gate of output m of head h being column h M + m of the row.
 // A launch and two dependent loads; us, the library's batched product -> here,
-// captured, weights from HBM (the second joins the heads in one row, which
+// captured, weights from HBM (the first is DOWN, the second joins the heads in one row, which
 // was a copy of torch's):
-//   64 rows: 32 heads of 512 x 128 5.3 -> 4.3, of 128 x 512 13.5 -> 3.9;
-//       16 heads of 256 x 64 5.0 -> 2.7, of 64 x 256 9.0 -> 2.9
-//   128 rows: 32 heads of 512 x 128 6.2 -> 5.3, of 128 x 512 15.4 -> 4.7
-//   4 rows: 16 heads of 512 x 128 4.2 -> 2.8, of 128 x 512 14.0 -> 3.3
-template <int NT, int MT, int KW, int S, bool GATED>
+//   64 rows: 32 heads, 128 deep to 512 6.2 -> 4.3, 512 to 128 13.5 -> 3.9;
+//       16 heads, 64 to 256 5.2 -> 2.7, 256 to 64 9.0 -> 2.9
+//   128 rows: 32 heads, 128 to 512 6.9 -> 5.2, 512 to 128 15.4 -> 4.7
+//   4 rows: 16 heads, 128 to 512 4.1 -> 2.9, 512 to 128 14.0 -> 3.3
+template <int NT, int MT, int KW, int S, bool GATED, bool DOWN>
 __global__ __launch_bounds__(KW * 64, 2) void head_gemm_kernel(
     bf16_t* __restrict__ out, int ld_out, int os,
     const bf16_t* __restrict__ x, int ldx, int xs,
-    const bf16_t* __restrict__ w, const bf16_t* __restrict__ gate,
-    int ld_gate, int N, int M, int K) {
+    const bf16_t* __restrict__ w, const bf16_t* __restrict__ w2,
+    const bf16_t* __restrict__ gate, int ld_gate, int N, int M, int K) {
   using Tile = RowTile<NT, MT, KW, S>;
   constexpr int OUT = 16 * MT;
   extern __shared__ __align__(1024) char lds[];
   const int h = blockIdx.y, n0 = blockIdx.z * 16 * NT;
   const int m0 = blockIdx.x * OUT;
-  const bf16_t* wh = w + (size_t)h * M * K;
+  const bf16_t* wh = w2 && h ? w2 : w + (size_t)h * M * K;
   const bf16_t* xh = x + (size_t)h * xs;
-  Tile::run(
+  // DOWN: M is a multiple of 8, and so are columns
+  Tile::template run<DOWN>(
       lds, K, blockIdx.x + h,
       [&](int r) {
         return xh + (size_t)(n0 + r < N ? n0 + r : N - 1) * ldx;
       },
       [&](int r) {
-        return wh + (size_t)(m0 + r < M ? m0 + r : M - 1) * K;
-      });
+        return DOWN ? wh + (m0 + r < M ? m0 + r : M - 8)
+                    : wh + (size_t)(m0 + r < M ? m0 + r : M - 1) * K;
+      },
+      M);
   Tile::each(OUT / 4, [&](int r, int c) {
     if (n0 + r >= N || m0 + c >= M) return;
     f32x4 v = Tile::sum(lds, r, c);
@@ -371,23 +375,24 @@ struct HeadGemm {
   int ld_out, os;
   const bf16_t* x;
   int ldx, xs;
-  const bf16_t *w, *gate;
+  const bf16_t *w, *w2, *gate;
   int ld_gate, H, N, M, K;
   hipStream_t stream;
 };
-template <int NT, int MT, int KW, int S, bool GATED>
+template <int NT, int MT, int KW, int S, bool GATED, bool DOWN>
 static int head_gemm_launch(const HeadGemm& p) {
+  auto* kernel = &head_gemm_kernel<NT, MT, KW, S, GATED, DOWN>;
   constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(head_gemm_kernel<NT, MT, KW, S, GATED>),
+      reinterpret_cast<const void*>(kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (sized != hipSuccess) return -1;
-  hipLaunchKernelGGL((head_gemm_kernel<NT, MT, KW, S, GATED>),
+  hipLaunchKernelGGL(kernel,
                      dim3((p.M + 16 * MT - 1) / (16 * MT), p.H,
                           (p.N + 16 * NT - 1) / (16 * NT)),
                      dim3(KW * 64), lds, p.stream, p.out, p.ld_out, p.os, p.x,
-                     p.ldx, p.xs, p.w, p.gate, p.ld_gate, p.N, p.M, p.K);
+                     p.ldx, p.xs, p.w, p.w2, p.gate, p.ld_gate, p.N, p.M, p.K);
   HY_CHECK();
   return 0;
 }
@@ -398,24 +403,38 @@ static int head_gemm_launch(const HeadGemm& p) {
 template <bool GATED>
 static int head_gemm_pick(const HeadGemm& p) {
   if (p.K <= 128)
-    return p.N <= 48 ? head_gemm_launch<1, 2, 2, 1, GATED>(p)
-                     : head_gemm_launch<2, 2, 2, 1, GATED>(p);
-  return p.N <= 48 ? head_gemm_launch<1, 2, 4, 2, GATED>(p)
-                   : head_gemm_launch<2, 2, 4, 2, GATED>(p);
+    return p.N <= 48 ? head_gemm_launch<1, 2, 2, 1, GATED, false>(p)
+                     : head_gemm_launch<2, 2, 2, 1, GATED, false>(p);
+  return p.N <= 48 ? head_gemm_launch<1, 2, 4, 2, GATED, false>(p)
+                   : head_gemm_launch<2, 2, 4, 2, GATED, false>(p);
+}
+// Columns of W: 64 outputs are whole lines of memory (us, 32 and 64: 64 rows, 32
+// heads of 128 x 512 5.0 and 4.3, one row 3.8 and 3.4), but too few workgroups
+// for small matrices (one row, 16 heads of 64 x 256 2.5 and 2.6); 32 rows a tile
+// only past 1024 workgroups (128 rows, 32 heads 5.5 and 5.2; 64 rows 4.3 and 4.4).
+template <int KW, int S>
+static int head_gemm_down(const HeadGemm& p) {
+  if (p.H * (long long)p.M < 8192)
+    return head_gemm_launch<1, 2, KW, S, false, true>(p);
+  if ((p.N + 15) / 16 * (long long)p.H * ((p.M + 63) / 64) <= 1024)
+    return head_gemm_launch<1, 4, KW, S, false, true>(p);
+  return head_gemm_launch<2, 4, KW, S, false, true>(p);
 }
 
-// 0: done, -2: not for this kernel
+// w2: null, or the second of two matrices.  0: done, -2: not for this kernel
 extern "C" int ll_head_gemm(void* out, int ld_out, int os, const void* x,
-                            int ldx, int xs, const void* w, const void* gate,
-                            int ld_gate, int H, int N, int M, int K,
-                            void* stream) {
+                            int ldx, int xs, const void* w, const void* w2,
+                            int down, const void* gate, int ld_gate, int H,
+                            int N, int M, int K, void* stream) {
   if (H <= 0 || H > 65535 || N <= 0 || N > 128 || M <= 0 || K <= 0 || M % 4 ||
       K % 8 || ldx % 8 || xs % 8 || ld_out % 4 || os % 4 ||
       (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 8 ||
+      (w2 && (H != 2 || (uintptr_t)w2 % 16)) || (down && (M % 8 || gate)) ||
       (gate && (ld_gate % 4 || (uintptr_t)gate % 8)))
     return -2;
   const HeadGemm p{(bf16_t*)out,     ld_out,  os, (const bf16_t*)x, ldx, xs,
-                   (const bf16_t*)w, (const bf16_t*)gate, ld_gate, H, N, M, K,
-                   (hipStream_t)stream};
+                   (const bf16_t*)w, (const bf16_t*)w2, (const bf16_t*)gate,
+                   ld_gate, H, N, M, K, (hipStream_t)stream};
+  if (down) return K <= 128 ? head_gemm_down<2, 1>(p) : head_gemm_down<4, 2>(p);
   return gate ? head_gemm_pick<true>(p) : head_gemm_pick<false>(p);
 }

@@ -284,8 +284,8 @@ def test_planted_scores(window):
 
 
 def test_copies_of_weights_are_no_part_of_a_saved_state():
-    """A state holds weights and what was always in it; copies that decoding
-    reads follow a loaded one, in the memory that a graph may have seen."""
+    """A mixer holds weights and no copies beside them, and a loaded state
+    goes where they lie, which a graph may have seen."""
     layers = [U.latent(2, 16, 8, 16, 24, 19),
               U.delta(4, 4, 16, 16, 2, low=(16, 16))]
     cfg = U.config(layers, vocab=97, width=64, ff=96)
@@ -298,11 +298,12 @@ def test_copies_of_weights_are_no_part_of_a_saved_state():
                 for i, (ly, make) in enumerate(zip(
                     layers, [U.latent_mixer, U.delta_mixer]))]
 
-    for one, two, name in zip(mixers(1), mixers(2), ["w_uk_t", "w_low"]):
-        copy = getattr(one, name)
-        place, saved = copy.data_ptr(), two.state_dict()
-        assert name not in saved and name not in dict(one.named_parameters())
-        assert not torch.equal(copy, getattr(two, name))
+    for one, two, names in zip(mixers(1), mixers(2),
+                               [["w_uk"], ["w_a2", "w_g2"]]):
+        places = [getattr(one, n).data_ptr() for n in names]
+        saved = two.state_dict()
+        assert set(saved) == set(dict(one.named_parameters()))
+        assert not list(one.buffers())
         one.load_state_dict(saved)
-        assert torch.equal(getattr(one, name), getattr(two, name))
-        assert getattr(one, name).data_ptr() == place
+        assert all(torch.equal(getattr(one, n), saved[n]) for n in names)
+        assert places == [getattr(one, n).data_ptr() for n in names]

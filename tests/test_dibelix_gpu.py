@@ -259,6 +259,40 @@ def test_delta_rule_full_chip(rows):
         close(got, want[:len(got)], F32)
 
 
+@pytest.mark.parametrize("other", [False, True])
+@pytest.mark.parametrize("kind", ["latent", "delta"])
+def test_weights_that_change(kind, other):
+    """Prompts and single tokens see the weights that a mixer has now,
+    changed in place or replaced."""
+    width, T = 64, 30
+    layer = U.latent(4, 16, 8, 16, 24, 19) if kind == "latent" \
+        else U.delta(4, 4, 16, 16, 2, low=(16, 16))
+    w = {k[len("l0.mix."):]: t.double() for k, t in U.weights(
+        U.config([layer], 8, width, 8), 5).items()
+        if k.startswith("l0.mix.")}
+    make, oracle = (U.latent_mixer, O.latent_attention) \
+        if kind == "latent" else (U.delta_mixer, O.channel_delta)
+    mix = make(layer["mixer"], w, 1e-5, width, DEV, B16)
+    run = U.MixerRun(mix, 1, T)
+    g = torch.Generator().manual_seed(4)
+    h = torch.randn(T, width, generator=g).bfloat16().double()
+    run.cuts(0, h, [20])
+    for name in ("uk",) if kind == "latent" else ("a2", "g2"):
+        w[name] = w[name] * -2.0
+        held = getattr(mix, "w_" + name)
+        new = (held * -2.0).detach()
+        if other:
+            setattr(mix, "w_" + name,
+                    torch.nn.Parameter(new, requires_grad=False))
+        else:
+            held.data.copy_(new)
+    want = oracle(h, w, "", layer["mixer"], 1e-5)
+    want = want[0] if kind == "latent" else want
+    for cuts in ([], range(1, T)):
+        run.restart(0)
+        close(run.cuts(0, h, cuts), want, B16, rel=3e-2)
+
+
 def test_slots_start_empty():
     """A slot's next sequence sees nothing of the last one, also when it
     is shorter than the convolution."""

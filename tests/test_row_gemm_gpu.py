@@ -209,6 +209,36 @@ def test_heads(N, H, M, K, gated):
     assert ((out.double() - ref).abs() <= bound).all()
 
 
+# columns of W: one and two pieces of the depth, remainders of both
+@pytest.mark.parametrize("H,K,M", [(4, 128, 512), (3, 72, 72), (5, 512, 136),
+                                   (2, 8, 8), (2, 264, 40)])
+@pytest.mark.parametrize("N", [1, 16, 48, 49, 65, 128])
+def test_heads_against_columns(N, H, K, M):
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(N, H, K + 8, generator=g, device=DEV).bfloat16()[
+        ..., 8:].transpose(0, 1)
+    w = torch.randn(H, K, M, generator=g, device=DEV).bfloat16()
+    rows = torch.full((H, N, M + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+    assert ops.linear_heads(x, w, rows[..., 4:4 + M], down=True)
+    assert (rows[..., :4] == 7).all() and (rows[..., 4 + M:] == 7).all()
+    for h in range(H):
+        _close(rows[h, :, 4:4 + M], x[h], w[h].T)
+
+
+@pytest.mark.parametrize("N", [1, 64])
+def test_two_matrices(N):
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(2, N, 136, generator=g, device=DEV).bfloat16()
+    w = torch.randn(3, 68, 136, generator=g, device=DEV).bfloat16()
+    out = torch.empty(2, N, 68, device=DEV, dtype=torch.bfloat16)
+    for one, two in ((w[0], w[2]), (w[2], w[1])):
+        assert ops.linear_heads(x, (one, two), out)
+        _close(out[0], x[0], one)
+        _close(out[1], x[1], two)
+    assert not ops.linear_heads(x, (w[0], w[1, :60]), out)
+    assert not ops.linear_heads(x[:1], (w[0], w[1]), out[:1])
+
+
 def test_heads_that_do_not_fit():
     x = torch.randn(4, 129, 64, device=DEV).bfloat16()
     w = torch.randn(4, 32, 64, device=DEV).bfloat16()
@@ -221,3 +251,8 @@ def test_heads_that_do_not_fit():
     assert not ops.linear_heads(x, w, out.float())
     assert not ops.linear_heads(x[..., 4:36], w[..., :32].contiguous(), out)
     assert not ops.linear_heads(x, w, out, out[0])        # gate's shape
+    w = torch.randn(4, 64, 36, device=DEV).bfloat16()
+    assert not ops.linear_heads(x, w[..., :32], out, down=True)
+    out = torch.empty(4, 8, 36, device=DEV, dtype=torch.bfloat16)
+    assert not ops.linear_heads(x, w, out, down=True)     # 36 outputs
+    assert not ops.linear_heads(x, w, out)
