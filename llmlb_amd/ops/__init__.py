@@ -760,15 +760,23 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     return out
 
 
+def _as_it_is(x: torch.Tensor) -> bool:
+    """Whether the library would keep x's type and the current device's
+    stream: kernels know of neither autocast nor another device."""
+    return (not torch.is_autocast_enabled(x.device.type)
+            and x.device.index == torch.cuda.current_device())
+
+
 def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
                out: torch.Tensor | None = None, up: int = 0, a: float = 0.0,
                b: float = 0.0, tile: int = -1) -> torch.Tensor | None:
     """act(x @ W^T) by tile_gemm.hip, or None where it does not take the
     operands, or the library's product and a kernel of the activation's own
     are the faster.  ``tile``: one of the kernel's, -1: its choice."""
-    if act == "capped" or not _require_native().ll_tile_gemm_gains(
-            ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0]),
-            ctypes.c_int(x.shape[1]), ctypes.c_int(_ROW_ACTS[act])):
+    if act == "capped" or not _as_it_is(x) \
+            or not _require_native().ll_tile_gemm_gains(
+                ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0]),
+                ctypes.c_int(x.shape[1]), ctypes.c_int(_ROW_ACTS[act])):
         return None
     found = _product_of(x, weight, act, out, up)
     if found is None:
@@ -868,7 +876,7 @@ def linear_heads(x: torch.Tensor, weight, out: torch.Tensor,
     if not (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
             and x.dim() == out.dim() == 3
             and all(w.dim() == 4 - len(pair) for w in pair)
-            and _only_numbers(x, out, *pair)):
+            and _only_numbers(x, out, *pair) and _as_it_is(x)):
         return False
     (H, N, K), M = x.shape, out.shape[2]
     shape = (K, M) if down else (M, K)

@@ -114,3 +114,32 @@ def test_gradients_keep_the_library():
     w = torch.randn(512, 64, device=DEV, dtype=torch.bfloat16)
     ops.linear_rows(x, w).float().sum().backward()
     assert x.grad is not None
+
+
+def _operands():
+    x = torch.randn(300, 64, device=DEV).bfloat16()
+    return x, torch.randn(4096, 64, device=DEV).bfloat16()
+
+
+@torch.inference_mode()
+def test_autocast_keeps_the_library():
+    x, w = _operands()
+    assert ops.linear_act(x, w, "gelu") is not None
+    heads = x[:100].view(2, 50, 64), w.view(2, 2048, 64)
+    with torch.autocast("cuda", torch.float16):
+        assert ops.linear_rows(x, w).dtype == torch.float16
+        assert ops.linear_act(x, w, "gelu") is None
+        assert not ops.linear_heads(*heads, x.new_empty(2, 50, 2048))
+    assert ops.linear_heads(*heads, x.new_empty(2, 50, 2048))
+
+
+@torch.inference_mode()
+def test_operands_of_another_device_keep_the_library(monkeypatch):
+    """Kernels are launched on the current device's stream."""
+    x, w = _operands()
+    want = torch.nn.functional.linear(x, w)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert torch.equal(ops.linear_rows(x, w), want)
+    assert ops.linear_act(x, w, "gelu") is None
+    assert not ops.linear_heads(x[:100].view(2, 50, 64), w.view(2, 2048, 64),
+                                x.new_empty(2, 50, 2048))
