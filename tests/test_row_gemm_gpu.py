@@ -209,9 +209,11 @@ def test_heads(N, H, M, K, gated):
     assert ((out.double() - ref).abs() <= bound).all()
 
 
-# columns of W: one and two pieces of the depth, remainders of both
+# columns of W: one and two pieces of the depth, remainders of both; from
+# 8192 outputs of all heads on 64 a tile, past 1024 workgroups of 32 rows
 @pytest.mark.parametrize("H,K,M", [(4, 128, 512), (3, 72, 72), (5, 512, 136),
-                                   (2, 8, 8), (2, 264, 40)])
+                                   (2, 8, 8), (2, 264, 40), (16, 72, 520),
+                                   (17, 264, 520)])
 @pytest.mark.parametrize("N", [1, 16, 48, 49, 65, 128])
 def test_heads_against_columns(N, H, K, M):
     g = torch.Generator(device=DEV).manual_seed(N + M)
