@@ -862,26 +862,34 @@ def route(h, w, top, groups, keep, scale, lists: bool = True):
     return index, weight, (counts, pairs) if lists else None
 
 
-def expert_tile(pairs: int, experts: int, n: int, k: int) -> int:
+def expert_tile(pairs: int, experts: int, n: int, k: int,
+                inputs: int = 0) -> int:
     """Tile of ``hy_expert_tiles`` for products of depth k with n
-    outputs: 128 x 128 where experts have few pairs or outputs, 192 x 256
-    where rounds of a tile a compute unit are full enough (an expert's last
-    tile counted as half of one).  2048 to 512 wide, us (128 x 128, 192 x
-    256): 0.39 rounds 32, 41; 0.73 58, 43; 1.4 92, 75; 2.73 162, 135; 4096 to
-    1280: 0.44 65, 87; 0.97 139, 97.  Else 128 x 256 (two a compute unit, so
-    that one stores while the other multiplies) for shallow products, and for
-    deep ones 256 x 256, a round of one tile a compute unit, unless the last
-    round is too empty: by output 128 x 128 takes 1.35 times as long, but in
-    rounds of an eighth."""
+    outputs, ``inputs`` rows of inputs: 128 x 128 where experts have few
+    pairs or outputs, 192 x 256 where its copies take the operands (whole
+    steps of 64 of the depth, offsets of 32 bits) and rounds of a tile a
+    compute unit are full enough (an expert's last tile counted as half of
+    one).  2048 to 512 wide, us (128 x 128, 192 x 256): 0.39 rounds 32, 41;
+    0.73 58, 43; 1.4 92, 75; 2.73 162, 135; 4096 to 1280: 0.44 65, 87; 0.97
+    139, 97.  Else 128 x 256 (two a compute unit, so that one stores while
+    the other multiplies) for shallow products, and for deep ones 256 x 256,
+    a round of one tile a compute unit, unless the last round is too empty:
+    by output 128 x 128 takes 1.35 times as long, but in rounds of an
+    eighth.  Where the depth is no whole steps, whose edges are checked, both
+    of the smaller take longer (65536 pairs, 2048 outputs, us in order 128 x
+    128, 256 x 256, 128 x 256: 520 deep 288, 233, 265; 264 deep 1024 outputs
+    78, 81, 69; 16384 pairs, 1.41 rounds, 1032 deep 67, 62, 63)."""
     if pairs < 192 * experts or n < 256:
         return 0
     rounds = (pairs / 192 + experts / 2) * -(-n // 256) / 256
-    if math.ceil(rounds) <= 1.6 * rounds:
+    near = (max(inputs, n) + 1) * k * 2 < 2 ** 32
+    if math.ceil(rounds) <= 1.6 * rounds and k % 64 == 0 and near:
         return 3
-    if k < 1024:
+    shallow, empty = (512, 1.8) if k % 64 else (1024, 1.35)
+    if k < shallow:
         return 2 if n > 256 else 0
     rounds = (pairs / 256 + experts / 2) * -(-n // 256) / 256
-    return 1 if math.ceil(rounds) <= 1.35 * rounds else 0
+    return 1 if math.ceil(rounds) <= empty * rounds else 0
 
 
 def experts(h, index, lists, w_up, w_down):
@@ -909,11 +917,12 @@ def experts(h, index, lists, w_up, w_down):
         return z
     where = (_ptr(lists[0]), _ptr(lists[1]))
     tiles = can_expert_mfma(h.dtype, W, F)
-    for data, size, n, k in ((up, up_size, F, W), (down, down_size, W, F)):
+    for data, size, n, k, rows in ((up, up_size, F, W, T),
+                                   (down, down_size, W, F, T * top)):
         args = (*data, *where, *size, _i(T), _i(T * top))
         if tiles:
             _check(lib.hy_expert_tiles(
-                *args, _i(expert_tile(T * top, E, n, k)), st),
+                *args, _i(expert_tile(T * top, E, n, k, rows)), st),
                 "hy_expert_tiles")
         else:
             _check(lib.hy_expert_rows(*args, _dt(h.dtype), st),

@@ -298,3 +298,16 @@ def test_routing_details():
     assert index.tolist() == [[0, 4, 1]]        # not 2 and 3
     index, _, _ = hy.route(z, eye, 3, 1, 1, 1.0)
     assert index.tolist() == [[0, 4, 2]]
+
+
+def test_expert_tiles_of_depths_and_offsets():
+    """192 x 256 only where its copies take the operands; other depths and
+    operands past 32 bits keep the tiles of a product of their depth."""
+    from llmlb_amd.ops import hybrid as hy
+    assert hy.expert_tile(65536, 16, 1024, 512, 65536) == 3
+    for k, tile in ((8, 2), (264, 2), (416, 2), (520, 1), (1032, 1)):
+        assert hy.expert_tile(65536, 16, 1024, k, 65536) == tile
+        assert hy.expert_tile(65536, 16, 256, k, 65536) == 0
+    assert hy.expert_tile(1 << 20, 16, 1024, 2048, 1 << 20) == 1
+    assert hy.expert_tile(1 << 20, 16, 1024, 2048, 1 << 18) == 3
+    assert hy.expert_tile(1 << 22, 16, 1024, 512, 1 << 22) == 2
