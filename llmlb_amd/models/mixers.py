@@ -160,9 +160,9 @@ class LatentAttention(nn.Module):
         H, D, V = self.heads, self.dim, self.vdim
         q = proj[:n, :H * (D + self.rot)].unflatten(
             1, (H, D + self.rot))[..., :D].transpose(0, 1)
-        qa = torch.empty(H, n, self.rank, dtype=proj.dtype,
-                         device=proj.device)
-        if not linear_heads(q, self.w_uk, qa, down=True):
+        fits = proj.is_cuda and proj.dtype == torch.bfloat16 and n <= 128
+        qa = q.new_empty(H, n, self.rank) if fits else None
+        if not fits or not linear_heads(q, self.w_uk, qa, down=True):
             qa = torch.bmm(q, self.w_uk)
         attend = hy.latent_decode if self.tiled and proj.is_cuda \
             else hy.latent_rows
@@ -171,14 +171,15 @@ class LatentAttention(nn.Module):
         if out is None:
             out = torch.empty(n, H * V, dtype=proj.dtype, device=proj.device)
         gate = proj[:n, self.g_off:self.g_off + H * V] if self.gate else None
-        if linear_heads(lat, self.w_uv, out.view(n, H, V).transpose(0, 1),
-                        gate):
+        to = out.unflatten(1, (H, V)).transpose(0, 1)
+        if fits and linear_heads(lat, self.w_uv, to, gate):
             return out
         o = torch.bmm(lat, self.w_uv_t)                 # [H, n, vdim]
         if self.gate:
             hy.join_heads(out, o, proj, self.g_off)
-            return out
-        return out.copy_(o.transpose(0, 1).reshape(n, H * V))
+        else:
+            to.copy_(o)
+        return out
 
 
 class ChannelDelta(nn.Module):

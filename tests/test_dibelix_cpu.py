@@ -307,3 +307,27 @@ def test_copies_of_weights_are_no_part_of_a_saved_state():
         one.load_state_dict(saved)
         assert all(torch.equal(getattr(one, n), saved[n]) for n in names)
         assert places == [getattr(one, n).data_ptr() for n in names]
+
+
+def test_heads_are_joined_by_one_copy():
+    """Where the kernel of heads takes no operands, outputs are copied to
+    their rows once."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Copies(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            name = func.overloadpacket.__name__
+            if name in ("clone", "copy_") and args[0].shape[-1] in (16, 32) \
+                    and args[0].numel() == 5 * 2 * 16:
+                self.seen += 1
+            return func(*args, **(kwargs or {}))
+
+    layer = U.latent(2, 16, 8, 16, 24, 19)
+    w = {k[len("l0.mix."):]: t for k, t in U.weights(
+        U.config([layer], 8, 40, 8), 1).items() if k.startswith("l0.mix.")}
+    run = U.MixerRun(U.latent_mixer(layer["mixer"], w, 1e-5, 40), 1, 16)
+    with Copies() as mode:
+        run.step([(0, torch.randn(5, 40).double())])
+    assert mode.seen == 1
