@@ -144,11 +144,19 @@ static int best_tile(int N, int rows, int K) {
 //    16384: 4352 x 2048 547 -> 449, 11904 x 4096 2405 -> 2267.  squared relu
 //    333: 6912 x 2048 29 -> 20; 1355: 50 -> 44, 18432 x 4096 193 -> 183
 //  * not for few tiles of some depth, which the library takes in shares: 333:
-//    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18
+//    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18; 129:
+//    1024 x 1024 8.1 -> 8.4, 512 x 640 (gain 0.87), but with a depth up to 512
+//    256 x 512 (2.1), 4096 x 512 7.5 -> 6.4
+//  * not for the widest that are not shallow, which memory bounds: 320: 32768 x
+//    2048 50 -> 55, 57344 x 2048 90 -> 98; 2048: 349 -> 365
 //  * outputs that are no whole tiles of 256: 333: 8224 x 2048 25 -> 21; 1355:
 //    3216 x 1024 17.5 -> 13.2, 8224 x 2048 56 -> 52; 8200: 1808 x 1024 53 -> 34,
 //    16448 x 4096 922 -> 834; 16384: 3600 x 2048 236 -> 200, 6416 x 2048 378 ->
-//    338, but 16512 x 4096 1557 -> 1604
+//    338, but 16512 x 4096 1557 -> 1604.  From 129 to 1024 rows the library's
+//    times go up and down by a fifth, and so do the gains: 129, 200, 256, 320,
+//    400, 512, 700, 1024 rows of 8224 x 2048 0.94 (not taken), 1.24, 1.22, 1.04,
+//    1.30, 0.95, 1.11, 1.04; of 10272 x 4096 0.95, 0.90, 1.16, 0.92, 1.18, 0.93,
+//    1.03, 1.01
 //  * shallow ones, or of medium depth and not too many rows: 1355: 1024 x 1024
 //    10.8 -> 9.0, 2048 x 2048 18.6 -> 18.1, 3072 x 2048 24.6 -> 22.2; 12288:
 //    1024 x 1024 28.4 -> 26.0, but 16384: 2048 x 2048 101 -> 104
@@ -161,9 +169,10 @@ extern "C" int ll_tile_gemm_gains(int N, int rows, int K, int kind) {
   if (N <= 0 || rows <= 0 || K <= 0) return 0;
   const long long few = ((long long)N + 63) / 64 * ((rows + 127) / 128);
   if (K > 1024 && few < (kind == PLAIN ? 200 : 150)) return 0;
-  if (kind != PLAIN || K <= 1024) return 1;
+  if (kind != PLAIN) return 1;
+  if (K <= 1024) return K <= 512 || few >= 64;
   if (rows % 256) return K < 3072 || N < 12288;
-  if (K < 3072) return N < 4096;
+  if (K < 3072) return N < 4096 && rows < 32768;
   const long long large = ((long long)N + 255) / 256 * (rows / 256);
   const int last = (int)(large % 256);
   return (large > 256 && last > 0 && last <= 64) ||

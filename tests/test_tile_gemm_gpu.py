@@ -108,6 +108,15 @@ def test_prompt_products():
         assert ((ops.linear_rows(x, w).double() - z).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("N,M,K,taken", [
+    (129, 1024, 1024, 0), (320, 512, 640, 0), (129, 256, 512, 1),
+    (129, 3216, 1024, 1), (320, 32768, 2048, 0), (320, 32000, 2048, 1)])
+def test_plain_products_taken(N, M, K, taken):
+    """Small products of some depth and the widest are the library's."""
+    assert ops._lib.ll_tile_gemm_gains(N, M, K, ops._ROW_ACTS["plain"]) \
+        == taken
+
+
 def test_gradients_keep_the_library():
     x = torch.randn(300, 64, device=DEV, dtype=torch.bfloat16,
                     requires_grad=True)
