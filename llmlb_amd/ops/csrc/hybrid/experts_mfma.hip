@@ -303,8 +303,8 @@ static int expert_product(const ExpertProduct& p) {
 // expert's pairs as in row_tile.h.  Bound by reading the matrices: both
 // products of 16 experts of 4096 x 1280 took 105 us for 64 tokens with
 // operands loaded straight into registers, 67 (5.0 TB/s) this way; 8 tokens
-// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  hy_expert_few has the
-// outputs a tile.
+// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  hy_expert_few_tile
+// has the outputs a tile.
 #define FEW_PAIRS 2048  // most that fit a workgroup's list
 // 16 NT pairs by 16 MT outputs; pieces of the depth on their way so that every
 // NT fits the LDS of the first
@@ -420,18 +420,13 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
   return 0;
 }
 
-int hy_expert_few(void* out, const void* in, const void* w, const void* index,
-                  int E, int N, int K, int div, int act, int n_pairs,
-                  void* stream) {
-  if (E <= 0 || N <= 0 || K <= 0 || N % 8 || K % 8 || div <= 0 ||
-      E > 65535 || n_pairs > FEW_PAIRS)
-    return -2;
-  if (n_pairs <= 0) return 0;
-  // Outputs a tile, by what a compute unit takes in as for other products of
-  // few rows: rounds of 256 tiles of the experts that are likely used, times
-  // a tile's rows.  32, but 16 for small matrices and 80 for deep ones.  us, 32
-  // outputs -> these, 61 tokens: 1024 to 256 wide 5.4 -> 4.9, 4096 to 1280 32.2
-  // -> 29.4, 300 tokens 90 -> 62; 1280 deep 80 outputs lost (81.6 -> 90.4).
+// Outputs a tile of hy_expert_few over 16, by what a compute unit takes in as
+// for other products of few rows: rounds of 256 tiles of the experts that are
+// likely used, times a tile's rows.  32, but 16 for small matrices and 80 for
+// deep ones.  us, 32 outputs -> these, 61 tokens: 1024 to 256 wide 5.4 -> 4.9,
+// 4096 to 1280 32.2 -> 29.4, 300 tokens 90 -> 62; 1280 deep 80 outputs lost (81.6
+// -> 90.4).
+int hy_expert_few_tile(int E, int N, int K, int n_pairs) {
   const float used = E * (1.f - powf(1.f - 1.f / E, (float)n_pairs));
   const int each = (int)(n_pairs / used + 15.f) / 16;
   auto takes = [&](int mt) {
@@ -441,8 +436,21 @@ int hy_expert_few(void* out, const void* in, const void* w, const void* index,
   int mt = 2;
   if (K >= 1024 && takes(1) < 0.95f * takes(2)) mt = 1;
   if (K >= 2048 && takes(5) < 0.95f * takes(mt)) mt = 5;
+  return mt;
+}
+
+// tile: 1, 2 or 5 times 16 outputs; -1: the choice above
+int hy_expert_few(void* out, const void* in, const void* w, const void* index,
+                  int E, int N, int K, int div, int act, int n_pairs, int tile,
+                  void* stream) {
+  if (E <= 0 || N <= 0 || K <= 0 || N % 8 || K % 8 || div <= 0 ||
+      E > 65535 || n_pairs > FEW_PAIRS)
+    return -2;
+  if (n_pairs <= 0) return 0;
 #define GO(MT)                                                               \
   do {                                                                       \
+    static_assert(FEW_LDS<MT> + sizeof(short) * FEW_PAIRS + 64 <=            \
+                      160 * 1024, "LDS of a compute unit");                  \
     static const hipError_t sized = hipFuncSetAttribute(                     \
         reinterpret_cast<const void*>(expert_few_kernel<MT>),                \
         hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS<MT>);            \
@@ -453,9 +461,12 @@ int hy_expert_few(void* out, const void* in, const void* w, const void* index,
                        (bf16_t*)out, (const bf16_t*)in, (const bf16_t*)w,    \
                        (const int*)index, N, K, div, act, n_pairs);          \
   } while (0)
-  if (mt == 1) GO(1);
-  else if (mt == 5) GO(5);
-  else GO(2);
+  switch (tile < 0 ? hy_expert_few_tile(E, N, K, n_pairs) : tile) {
+    case 1: GO(1); break;
+    case 2: GO(2); break;
+    case 5: GO(5); break;
+    default: return -2;
+  }
 #undef GO
   HY_CHECK();
   return 0;

@@ -824,6 +824,7 @@ def window_attention(out, proj, g_off, heads, kv_heads, dim, vdim, cache, b,
 # -- mixture of experts ----------------------------------------------------
 
 FEW_PAIRS = 512      # (token, choice) pairs that need no lists of experts
+FEW_TILE = -1        # of their kernel: -1, or 1, 2, 5 times 16 outputs
 
 
 def can_expert_mfma(dtype, width, ff) -> bool:
@@ -913,7 +914,7 @@ def experts(h, index, lists, w_up, w_down):
     if lists is None:
         for data, size in ((up, up_size), (down, down_size)):
             _check(lib.hy_expert_few(*data, _ptr(index), *size, _i(T * top),
-                                     st), "hy_expert_few")
+                                     _i(FEW_TILE), st), "hy_expert_few")
         return z
     where = (_ptr(lists[0]), _ptr(lists[1]))
     tiles = can_expert_mfma(h.dtype, W, F)

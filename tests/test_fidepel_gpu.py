@@ -328,6 +328,23 @@ def test_experts(case, form, monkeypatch):
     close(got[sure], want[sure], dtype)
 
 
+# outputs that are whole tiles of 80 (240, 320) and not, by experts of up to
+# 16 pairs, 17 to 32, more, and of more than a list's tile of 64
+@pytest.mark.parametrize("case", [(4, 2, 160, 88, 6), (3, 3, 264, 240, 20),
+                                  (2, 2, 136, 320, 40), (3, 2, 240, 408, 90)],
+                         ids=str)
+@pytest.mark.parametrize("tile", [1, 2, 5])
+def test_tiles_of_few_pairs(case, tile, monkeypatch):
+    monkeypatch.setattr(hy, "FEW_TILE", tile)
+    test_experts(case, "few", monkeypatch)
+
+
+def test_choice_of_tiles_of_few_pairs():
+    choice = hy.native().hy_expert_few_tile
+    assert [choice(16, n, k, 244) for n, k in (
+        (256, 1024), (1024, 256), (1280, 4096), (4096, 1280))] == [1, 2, 5, 2]
+
+
 # whole steps of the depth (64): experts with no pair, one, an edge and
 # several tiles of 192, several tiles a workgroup
 @pytest.mark.parametrize("case", [(4, 2, 64, 64, 1), (14, 5, 256, 320, 60),
