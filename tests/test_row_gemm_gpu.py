@@ -113,6 +113,28 @@ def _act(act, z, up, a, b):
     return g * torch.sigmoid(b * g) * (u + 1.0)
 
 
+def _act_bound(act, x, w, up, a, b):
+    """(activation of the products, how far a result may be from it).  A sum
+    is K float roundings off and then a bf16 number, so it is one between two
+    that are mostly neighbours; the result is between the activations of
+    those (which are monotone where there are more), whose own functions are
+    good to 2^-20, and rounded."""
+    x, w = x.double(), w.double()
+    z = x @ w.T
+    off = (x.abs() @ w.abs().T) * x.shape[1] * 2.0 ** -24
+    if act == "plain":
+        return z, off + z.abs() * 2.0 ** -8 + 1e-30
+    ref = _act(act, z.bfloat16().double(), up, a, b)
+    ends = [(z + s * off).bfloat16().double() for s in (-1, 1)]
+    far = torch.zeros_like(ref)
+    for g in ends:
+        for u in ends if up else ends[:1]:
+            end = torch.cat([g[:, :up], u[:, up:]], 1) if up else g
+            far = torch.maximum(far, (_act(act, end, up, a, b) - ref).abs())
+    unit = 2.0 ** -20 + (0.0 if act == "capped" else 2.0 ** -8)
+    return ref, far + (ref.abs() + far) * unit + 1e-30
+
+
 @pytest.mark.parametrize("act,a,b", [("relu2", 0, 0), ("gelu", 0, 0),
                                      ("capped", 0, 0), ("capped", 3.0, 0),
                                      ("swiglu", 0, 0), ("clamped", 1.5, 1.7)])
@@ -124,25 +146,13 @@ def test_row_gemm_with_activation(N, M, K, act, a, b):
     up = M if act in ("swiglu", "clamped") else 0
     w = torch.randn(M + up, K, generator=g, device=DEV).mul_(
         K ** -0.5).bfloat16()
-    z = x.double() @ w.double().T
-    ref = _act(act, z.bfloat16().double(), up, a, b)
+    ref, bound = _act_bound(act, x, w, up, a, b)
     wide = torch.full((N, M + 16), 7.0, device=DEV, dtype=torch.bfloat16)
     out = None if act == "capped" else wide[:, 8:8 + M]
     out = ops.linear_act(x, w, act, out, up, a, b)
-    # sums are K float roundings off, which where they lie near the middle
-    # of two bf16 numbers may take the other one; activations of numbers of
-    # size 1 to 30 (K ** -0.5 rows) change by at most 60 times as much, and
-    # their own functions are good to 2^-20
-    off = (x.double().abs() @ w.double().abs().T).amax() * K * 2.0 ** -24
-    apart = (z - off).bfloat16() != (z + off).bfloat16()
-    if up:
-        apart = apart[:, :up] | apart[:, up:]
-    bound = ref.abs() * 2.0 ** -20 + 1e-30 \
-        + apart * 60 * z.abs().amax() * 2.0 ** -8
     if act == "capped":
         assert out.dtype == torch.float32
     else:
-        bound = bound + ref.abs() * 2.0 ** -8
         assert (wide[:, :8] == 7).all() and (wide[:, 8 + M:] == 7).all()
     assert ((out.double() - ref).abs() <= bound).all()
 
