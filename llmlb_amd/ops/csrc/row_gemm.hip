@@ -168,7 +168,11 @@ static int row_gemm_launch(const RowGemm& p) {
 // tile are for what they fit into one round, or two: 64 rows, from tiles of 64
 // on, gate and up of 14336 x 4096 47.6 -> 39.8, 26000 x 2048 27.8 -> 22.1,
 // 57344 x 1024 (two) 31.5 -> 29.9; with five rounds they lose (40 rows, 128256
-// x 4096 170 -> 178: the card's memory is the bound).
+// x 4096 170 -> 178: the card's memory is the bound).  One 16 of rows is mostly
+// bound by memory, and small tiles, of which a unit has two, are less uneven
+// than whole rounds say: another than 32 outputs has to take in 15% less (one
+// row of 20480 x 1024 11.0 with 48, 10.1 with 32; 16512 x 1024 9.2 with 32, 8.6
+// with 80).
 template <bool GATED>
 static int row_gemm_pick(const RowGemm& p) {
   const int tiles = (p.N + 15) / 16;
@@ -184,16 +188,20 @@ static int row_gemm_pick(const RowGemm& p) {
     const long long rounds = (count + 31) / 32;
     if (m == 7 && rounds > 2) return;  // memory bounds these, of any tile
     const float takes = fmaxf((float)(rounds * (n + m)), floor);
-    if (!nt || takes < 0.95f * least) least = takes, nt = n, mt = m;
+    const float by = n == 1 ? 0.85f : 0.95f;
+    if (!nt || takes < by * least) least = takes, nt = n, mt = m;
   };
   // what is as good: more rows of x, which read W less often, then the sizes
   // that memory likes best
   static const int OF_MANY[] = {4, 5, 6, 3, 2, 1, 7};
-  static const int OF_ONE[] = {2, 4, 3, 1, 5, 5, 5};
+  static const int OF_ONE[] = {2, 3, 4, 1, 5, 5, 5};
   for (int n = tiles < 4 ? tiles : 4; n >= 1; --n)
     for (int i = 0; i < 7; ++i) {
       const int m = n == 1 ? OF_ONE[i] : OF_MANY[i];
-      if (n < 3 || m > 1) look(n, m);  // (3, 1) and (4, 1) take in no less
+      // (3, 1) and (4, 1) take in no less; of gate and up, tiles of 8 outputs
+      // by eight waves are for what they share (1024 x 128, one row: 3.0 with
+      // them, 2.8 with 16; 1024 x 768 3.4, 3.7)
+      if ((n < 3 || m > 1) && (!GATED || m > 1 || p.K > 256)) look(n, m);
     }
   // waves that share the depth, and pieces of it on their way, fit LDS
 #define TILE(NT, MT, KW, S) \
@@ -318,11 +326,11 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
 // The same for H pairs of rows and matrices at once, as latent attention needs
 // for its heads: out[h] = x[h] W[h]^T, W [H][M][K], or out[h] = x[h] W[h], W
 // [H][K][M] (DOWN).  x's and out's heads lie xs and os numbers apart; with w2
-// there are two matrices, which lie anywhere.  With a gate, out = bf16(sum) sigmoid(gate), the
-// gate of output m of head h being column h M + m of the row.
+// there are two matrices, which lie anywhere.  With a gate, out = bf16(sum)
+// sigmoid(gate), the gate of output m of head h being column h M + m of the row.
 // A launch and two dependent loads; us, the library's batched product -> here,
-// captured, weights from HBM (the first is DOWN, the second joins the heads in one row, which
-// was a copy of torch's):
+// captured, weights from HBM (the first is DOWN, the second joins the heads in
+// one row, which was a copy of torch's):
 //   64 rows: 32 heads, 128 deep to 512 6.2 -> 4.3, 512 to 128 13.5 -> 3.9;
 //       16 heads, 64 to 256 5.2 -> 2.7, 256 to 64 9.0 -> 2.9
 //   128 rows: 32 heads, 128 to 512 6.9 -> 5.2, 512 to 128 15.4 -> 4.7

@@ -39,9 +39,9 @@ def test_row_gemm(N, M, K):
 # rows and outputs at which each tile is taken (of 16 to 64 rows of x and 16
 # to 112 of W), with remainders
 @pytest.mark.parametrize("N,M", [
-    (1, 4), (76, 1284), (1, 8196), (1, 11924), (1, 16412), (106, 516),
-    (106, 1028), (106, 2564), (31, 12332), (31, 16412), (31, 20492),
-    (106, 2052), (76, 4100), (76, 6148), (76, 8196), (76, 10292),
+    (1, 4), (1, 1028), (1, 12332), (76, 1284), (1, 8196), (1, 11924),
+    (1, 16412), (106, 516), (106, 1028), (106, 2564), (31, 12332),
+    (31, 16412), (31, 20492), (106, 2052), (76, 4100), (76, 6148), (76, 8196), (76, 10292),
     (106, 3076), (106, 4100), (106, 6148), (106, 8196), (106, 10292),
     (31, 24708), (76, 12332), (106, 12332)])
 @pytest.mark.parametrize("K", [72, 520])
