@@ -374,7 +374,7 @@ static int page_attn_launch(void* out, void* acc, void* ml, const void* q,
                             const void* lens, int n, int max_blocks, int H,
                             int G, int parts, float scale, hipStream_t st) {
   constexpr int lds = PageAttn<D, FP8, W>::LDS;
-  static_assert(lds + 512 <= 160 * 1024, "LDS of a compute unit");
+  static_assert(lds + W * 128 <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
       reinterpret_cast<const void*>(page_attn_kernel<D, FP8, W>),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -417,10 +417,14 @@ extern "C" int ll_page_attn(void* out, void* acc, void* ml, const void* q,
   // whole ones leave compute units idle no longer than halves do.  Two parts
   // -> one, us, 32 sequences of 2048 and of up to 300 tokens, 32 heads on 8 of
   // 128: bf16 46.2 -> 43.5, 12.6 -> 9.1; e4m3 27.8 -> 24.9, 9.0 -> 6.6; 64 of
-  // 3000, 16 on 4 of 64: 29.9 -> 27.8.
+  // 3000, 16 on 4 of 64: 29.9 -> 27.8.  Eight waves of bf16 heads of 128 fill a
+  // compute unit's LDS, and past one round a long sequence among short ones
+  // waits for what its halves would share (50 sequences of 100 tokens, one of
+  // 8000: 54.5 -> 74.6; all of 1000 39.2 -> 36.7): two parts there.
   const long long count = (long long)n * G * ((H / G + 15) / 16);
-  const bool whole = parts == 2 && (count + 255) / 256 * 2 <=
-                                       (2 * count + 255) / 256;
+  const bool whole =
+      parts == 2 && (count + 255) / 256 * 2 <= (2 * count + 255) / 256 &&
+      (count <= 256 || D < 128 || ks);
 #define PAGE_ATTN(D, FP8)                                                    \
   do {                                                                       \
     if (whole)                                                               \

@@ -145,8 +145,9 @@ def test_weights_are_floats(D, fp8):
 
 
 # one part of eight waves (144 and 256 workgroups) or two of four (128 and
-# 320), of sequences with fewer pages than waves and with more
-@pytest.mark.parametrize("kv", [8, 9, 16, 20])
+# 320), of sequences with fewer pages than waves and with more; 400: one, but
+# two of bf16 heads of 128
+@pytest.mark.parametrize("kv", [8, 9, 16, 20, 25])
 @pytest.mark.parametrize("D", [64, 128])
 def test_two_parts(kv, D):
     q, k, v, bt, lens, _ = _case(2 * kv, kv, D, kv + D)
