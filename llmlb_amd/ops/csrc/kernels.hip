@@ -68,13 +68,15 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
 //   out = x' * rsqrt(mean(x'^2) + eps) * weight
 // One 256-thread block per token row; fp32 accumulation; bf16x8 loads.
 // Decoding has a row for every fourth compute unit, and its time is a chain
-// of loads: up to RMS_KEEP vectors a thread and their weights are asked for at
-// once, and stay in registers for the second pass.  A decoding step of 64
-// sequences of 1024 tokens, with 8 norms of 4096 columns: 654.6 -> 648.1 us;
-// 16384 rows of them 84 -> 79 us (6.8 TB/s).
+// of loads: KEEP vectors a thread and their weights are asked for at once, and
+// stay in registers for the second pass; MORE: rows have more of them.  A
+// decoding step of 64 sequences of 1024 tokens, with 8 norms of 4096 columns:
+// 654.6 -> 648.1 us.  us, read twice -> this, with a residual: 64 rows of 1024 2.63
+// -> 2.47, of 4096 3.34 -> 3.09; 16384 of 512 17.7 -> 16.8, of 4096 98.8 -> 92.5 (5.8
+// TB/s).  Room for two where there is one costs many short rows more than the
+// second pass does (16384 of 512: 18.8).
 // ---------------------------------------------------------------------------
-#define RMS_KEEP 2
-template <bool FUSE_RESIDUAL>
+template <bool FUSE_RESIDUAL, int KEEP, bool MORE>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     bf16* __restrict__ out, const bf16* __restrict__ in,
     const bf16* __restrict__ weight, bf16* __restrict__ residual, int hidden,
@@ -107,21 +109,22 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     for (int j = 0; j < 8; ++j) ssq += f[j] * f[j];
     return v;
   };
-  uint4 keep[RMS_KEEP], res[RMS_KEEP], w[RMS_KEEP];
+  uint4 keep[KEEP + 1], res[KEEP + 1], w[KEEP + 1];
 #pragma unroll
-  for (int n = 0; n < RMS_KEEP; ++n)
-    if (n * 256 < nvec) {
-      const int i = threadIdx.x + n * 256, at = i < nvec ? i : nvec - 1;
-      keep[n] = inv[at];
-      if (FUSE_RESIDUAL) res[n] = resv[at];
-      w[n] = wv[at];
+  for (int n = 0; n < KEEP; ++n) {
+    const int i = threadIdx.x + n * 256;
+    if (i < nvec) {
+      keep[n] = inv[i];
+      if (FUSE_RESIDUAL) res[n] = resv[i];
+      w[n] = wv[i];
     }
+  }
 #pragma unroll
-  for (int n = 0; n < RMS_KEEP; ++n) {
+  for (int n = 0; n < KEEP; ++n) {
     const int i = threadIdx.x + n * 256;
     if (i < nvec) keep[n] = first(i, keep[n], res[n]);
   }
-  for (int i = threadIdx.x + RMS_KEEP * 256; i < nvec; i += 256)
+  for (int i = threadIdx.x + KEEP * 256; MORE && i < nvec; i += 256)
     first(i, inv[i], FUSE_RESIDUAL ? resv[i] : uint4{});
   // wave reduce then cross-wave via LDS
   for (int off = 32; off > 0; off >>= 1) ssq += __shfl_xor(ssq, off, WAVE);
@@ -144,12 +147,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     outv[i] = pack8(f);
   };
 #pragma unroll
-  for (int n = 0; n < RMS_KEEP; ++n) {
+  for (int n = 0; n < KEEP; ++n) {
     const int i = threadIdx.x + n * 256;
     if (i < nvec) second(i, keep[n], w[n]);
   }
   // beyond them a thread reads back what it wrote itself
-  for (int i = threadIdx.x + RMS_KEEP * 256; i < nvec; i += 256)
+  for (int i = threadIdx.x + KEEP * 256; MORE && i < nvec; i += 256)
     second(i, FUSE_RESIDUAL ? resv[i] : inv[i], wv[i]);
 }
 
@@ -650,15 +653,20 @@ int ll_rmsnorm(void* out, const void* in, const void* weight, void* residual,
   if (hidden % 8 != 0) return -2;
   dim3 grid(n_tokens), block(256);
   hipStream_t s = (hipStream_t)stream;
-  if (residual) {
-    hipLaunchKernelGGL(rmsnorm_kernel<true>, grid, block, 0, s, (bf16*)out,
-                       (const bf16*)in, (const bf16*)weight, (bf16*)residual,
-                       hidden, eps);
-  } else {
-    hipLaunchKernelGGL(rmsnorm_kernel<false>, grid, block, 0, s, (bf16*)out,
-                       (const bf16*)in, (const bf16*)weight, nullptr, hidden,
-                       eps);
-  }
+#define RMSNORM(KEEP, MORE)                                                   \
+  do {                                                                        \
+    auto* kernel = residual ? &rmsnorm_kernel<true, KEEP, MORE>               \
+                            : &rmsnorm_kernel<false, KEEP, MORE>;             \
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, (bf16*)out,                 \
+                       (const bf16*)in, (const bf16*)weight, (bf16*)residual, \
+                       hidden, eps);                                          \
+  } while (0)
+  if (hidden <= 2048) RMSNORM(1, false);
+  else if (hidden <= 4096) RMSNORM(2, false);
+  // a few of the longest rows: nothing kept (one of 16384 6.3, 6.6 us with two)
+  else if (hidden > 8192 && n_tokens < 1024) RMSNORM(0, true);
+  else RMSNORM(2, true);
+#undef RMSNORM
   LL_CHECK(hipGetLastError());
   return 0;
 }
