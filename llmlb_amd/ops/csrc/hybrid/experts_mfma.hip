@@ -425,7 +425,11 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
 // likely used, times a tile's rows.  32, but 16 for small matrices and 80 for
 // deep ones.  us, 32 outputs -> these, 61 tokens: 1024 to 256 wide 5.4 -> 4.9,
 // 4096 to 1280 32.2 -> 29.4, 300 tokens 90 -> 62; 1280 deep 80 outputs lost (81.6
-// -> 90.4).
+// -> 90.4).  16 are not for many experts, whose idle workgroups they double (one
+// token, 64 of 2048 to 512 9.0 -> 9.8); of 80 a compute unit has one workgroup,
+// which with 64 pairs a tile waits for every piece of the depth (128 tokens, 8 of
+// 2048 to 4096 53.7 -> 58.5), and the last may be mostly empty (300 tokens, 64 of
+// 2048 to 512 30.0 -> 32.9).
 int hy_expert_few_tile(int E, int N, int K, int n_pairs) {
   const float used = E * (1.f - powf(1.f - 1.f / E, (float)n_pairs));
   const int each = (int)(n_pairs / used + 15.f) / 16;
@@ -434,8 +438,11 @@ int hy_expert_few_tile(int E, int N, int K, int n_pairs) {
     return ceilf(tiles / 256.f) * ((each < 4 ? each : 4) + mt);
   };
   int mt = 2;
-  if (K >= 1024 && takes(1) < 0.95f * takes(2)) mt = 1;
-  if (K >= 2048 && takes(5) < 0.95f * takes(mt)) mt = 5;
+  if (K >= 1024 && E * (long long)N <= 8192 && takes(1) < 0.95f * takes(2))
+    mt = 1;
+  const float whole = (float)N / ((N + 79) / 80 * 80);
+  const float waits = each > 2 ? 1.4f : 1.f;
+  if (K >= 2048 && takes(5) * waits < 0.85f * whole * takes(mt)) mt = 5;
   return mt;
 }
 

@@ -343,6 +343,10 @@ def test_choice_of_tiles_of_few_pairs():
     choice = hy.native().hy_expert_few_tile
     assert [choice(16, n, k, 244) for n, k in (
         (256, 1024), (1024, 256), (1280, 4096), (4096, 1280))] == [1, 2, 5, 2]
+    # many experts, tiles of 64 pairs, a last tile that is mostly empty
+    assert choice(64, 512, 2048, 4) == 2
+    assert choice(8, 4096, 2048, 512) == 2 and choice(16, 1280, 4096, 1200) == 5
+    assert choice(64, 512, 2048, 1200) == 2
 
 
 # whole steps of the depth (64): experts with no pair, one, an edge and
