@@ -760,11 +760,14 @@ def _row_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     return out
 
 
-def _as_it_is(x: torch.Tensor) -> bool:
-    """Whether the library would keep x's type and the current device's
-    stream: kernels know of neither autocast nor another device."""
-    return (not torch.is_autocast_enabled(x.device.type)
-            and x.device.index == torch.cuda.current_device())
+def _stream_as_library(x: torch.Tensor) -> ctypes.c_void_p | None:
+    """The current device's stream where the library would keep x's type on
+    it; None under autocast and for another device's operands, of which
+    kernels know nothing."""
+    device = torch.cuda.current_device()
+    if x.get_device() != device or torch.is_autocast_enabled("cuda"):
+        return None
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device))
 
 
 def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
@@ -773,10 +776,12 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     """act(x @ W^T) by tile_gemm.hip, or None where it does not take the
     operands, or the library's product and a kernel of the activation's own
     are the faster.  ``tile``: one of the kernel's, -1: its choice."""
-    if act == "capped" or not _as_it_is(x) \
-            or not _require_native().ll_tile_gemm_gains(
-                ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0]),
-                ctypes.c_int(x.shape[1]), ctypes.c_int(_ROW_ACTS[act])):
+    if act == "capped" or not _require_native().ll_tile_gemm_gains(
+            ctypes.c_int(x.shape[0]), ctypes.c_int(weight.shape[0]),
+            ctypes.c_int(x.shape[1]), ctypes.c_int(_ROW_ACTS[act])):
+        return None
+    stream = _stream_as_library(x)
+    if stream is None:
         return None
     found = _product_of(x, weight, act, out, up)
     if found is None:
@@ -787,7 +792,7 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
         ctypes.c_int(x.shape[0]), ctypes.c_int(M), ctypes.c_int(x.shape[1]),
         ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
         ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b),
-        ctypes.c_int(tile), _stream())
+        ctypes.c_int(tile), stream)
     if rc == -2:
         return None
     _check(rc, "ll_tile_gemm")
@@ -872,23 +877,27 @@ def linear_heads(x: torch.Tensor, weight, out: torch.Tensor,
     not take it.  x [H, N, K] and out [H, N, M] may be views whose last
     dimension is dense, weight [H, M, K] or the matrices of two heads, gate
     [N, H * M].  ``down``: weight [H, K, M], out[h] = x[h] @ weight[h]."""
-    pair = weight if isinstance(weight, tuple) else (weight,)
+    first, second = weight if isinstance(weight, tuple) else (weight, None)
     if not (x.is_cuda and _lib is not None and x.dtype == torch.bfloat16
             and x.dim() == out.dim() == 3
-            and all(w.dim() == 4 - len(pair) for w in pair)
-            and _only_numbers(x, out, *pair) and _as_it_is(x)):
+            and _only_numbers(x, out, first, x if second is None else second)):
         return False
     (H, N, K), M = x.shape, out.shape[2]
     shape = (K, M) if down else (M, K)
+    if second is None:
+        shape = (H, *shape)
+    elif (H != 2 or second.shape != shape or second.dtype != x.dtype
+          or second.device != x.device or not second.is_contiguous()):
+        return False
     if (_USE_CUSTOM_DECODE_GEMM != "auto" or not 0 < N <= 128
-            or out.shape != (H, N, M) or out.dtype != x.dtype
-            or len(pair) == 2 and H != 2
-            or any(w.shape[-2:] != shape or w.dtype != x.dtype
-                   or w.dim() == 3 and w.shape[0] != H
-                   or not w.is_contiguous() or w.device != x.device
-                   for w in pair)
-            or x.stride(2) != 1 or out.stride(2) != 1
-            or x.device != out.device):
+            or first.shape != shape or out.shape != (H, N, M)
+            or first.dtype != x.dtype or out.dtype != x.dtype
+            or not first.is_contiguous() or x.stride(2) != 1
+            or out.stride(2) != 1
+            or not x.device == first.device == out.device):
+        return False
+    stream = _stream_as_library(x)
+    if stream is None:
         return False
     if gate is not None and (
             gate.shape != (N, H * M) or gate.stride(1) != 1
@@ -898,10 +907,10 @@ def linear_heads(x: torch.Tensor, weight, out: torch.Tensor,
     rc = _lib.ll_head_gemm(
         _ptr(out), ctypes.c_int(out.stride(1)), ctypes.c_int(out.stride(0)),
         _ptr(x), ctypes.c_int(x.stride(1)), ctypes.c_int(x.stride(0)),
-        _ptr(pair[0]), _ptr(pair[1]) if len(pair) == 2 else None,
+        _ptr(first), None if second is None else _ptr(second),
         ctypes.c_int(down), None if gate is None else _ptr(gate),
         ctypes.c_int(0 if gate is None else gate.stride(0)), ctypes.c_int(H),
-        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K), _stream())
+        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K), stream)
     if rc == -2:
         return False
     _check(rc, "ll_head_gemm")

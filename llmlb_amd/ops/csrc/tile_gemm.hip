@@ -144,9 +144,10 @@ static int best_tile(int N, int rows, int K) {
 //    16384: 4352 x 2048 547 -> 449, 11904 x 4096 2405 -> 2267.  squared relu
 //    333: 6912 x 2048 29 -> 20; 1355: 50 -> 44, 18432 x 4096 193 -> 183
 //  * not for few tiles of some depth, which the library takes in shares: 333:
-//    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18; 129:
-//    1024 x 1024 8.1 -> 8.4, 512 x 640 (gain 0.87), but with a depth up to 512
-//    256 x 512 (2.1), 4096 x 512 7.5 -> 6.4
+//    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18.  Of up
+//    to 1024 deep fewer than 64 lose less than half a microsecond (129: 1024 x 1024
+//    8.1 -> 8.4) or gain (129: 256 x 512 2.1 times), and the host, which prompts of
+//    a few hundred rows wait for, is done 12 us earlier than with the library
 //  * not for the widest that are not shallow, which memory bounds: 320: 32768 x
 //    2048 50 -> 55, 57344 x 2048 90 -> 98; 2048: 349 -> 365
 //  * outputs that are no whole tiles of 256: 333: 8224 x 2048 25 -> 21; 1355:
@@ -170,7 +171,7 @@ extern "C" int ll_tile_gemm_gains(int N, int rows, int K, int kind) {
   const long long few = ((long long)N + 63) / 64 * ((rows + 127) / 128);
   if (K > 1024 && few < (kind == PLAIN ? 200 : 150)) return 0;
   if (kind != PLAIN) return 1;
-  if (K <= 1024) return K <= 512 || few >= 64;
+  if (K <= 1024) return 1;
   if (rows % 256) return K < 3072 || N < 12288;
   if (K < 3072) return N < 4096 && rows < 32768;
   const long long large = ((long long)N + 255) / 256 * (rows / 256);

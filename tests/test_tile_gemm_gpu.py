@@ -101,10 +101,10 @@ def test_prompt_products():
 
 
 @pytest.mark.parametrize("N,M,K,taken", [
-    (129, 1024, 1024, 0), (320, 512, 640, 0), (129, 256, 512, 1),
-    (129, 3216, 1024, 1), (320, 32768, 2048, 0), (320, 32000, 2048, 1)])
+    (129, 1024, 1024, 1), (129, 3216, 1024, 1), (129, 2048, 2048, 0),
+    (320, 32768, 2048, 0), (320, 32000, 2048, 1)])
 def test_plain_products_taken(N, M, K, taken):
-    """Small products of some depth and the widest are the library's."""
+    """Few tiles of some depth and the widest are the library's."""
     assert ops._lib.ll_tile_gemm_gains(N, M, K, ops._ROW_ACTS["plain"]) \
         == taken
 
