@@ -3,13 +3,15 @@
 //   out[N, M] = act(x[N, K] W[M, K]^T)     bf16, summed in float
 //
 // Bound by the power of the matrix cores: at 1430 TFLOP/s they are busy 87% of
-// the cycles, and the clock is down to 1.2 to 1.7 GHz.  So what counts beside
-// the cycles is the energy of a product: 16 x 16 x 32 (registers alone: 2060
-// TFLOP/s) and not 32 x 32 x 16 (1790), LDS read without bank conflicts, each
-// number once.  16384 rows of 4096 x 14336 take 1296 us without an
-// activation; with copies all at once and two stages of 64 KB it was 1582, with
-// the ring below and 32 x 32 products 1370.  The library's product takes 1250
-// us, but a pass over its results more (swiglu of 16384 x 14336: 263 us).
+// the cycles, and the clock is down to 1.2 to 1.7 GHz (with how long the chip has
+// been at it, swiglu of 16384 rows against 28672 x 4096 takes 2.55 to 2.65 ms,
+// 1510 to 1450 TFLOP/s).  So what counts beside the cycles is the energy of a
+// product: 16 x 16 x 32 (registers alone: 2060 TFLOP/s) and not 32 x 32 x 16
+// (1790), LDS read without bank conflicts, each number once.  16384 rows of 4096 x
+// 14336 take 1290 us without an activation; with copies all at once and two
+// stages of 64 KB it was 1582, with the ring below and 32 x 32 products 1370.  The
+// library's product takes 1200 to 1250 us, but a pass over its results more
+// (swiglu of 16384 x 14336: 263 us).
 #include "hybrid/tile_product.h"
 
 struct TileGemm {
@@ -138,11 +140,12 @@ static int best_tile(int N, int rows, int K) {
 // Whether this is faster than the library's product and, with an activation,
 // a kernel of its own.  us, the library -> here, rows: outputs x depth:
 //  * always with an activation, but for few tiles of some depth.  swiglu 333:
-//    2816 x 1024 18 -> 11; 1355: 5632 x 2048 79 -> 65, 14336 x 4096 291 -> 275;
-//    16384: 2816 x 1024 233 -> 160, 14336 x 4096 2891 -> 2691 (1430 TFLOP/s).
-//    gelu 16384: 7168 x 2048 440 -> 374, 19456 x 4096 2025 -> 1902.  clamped
-//    16384: 4352 x 2048 547 -> 449, 11904 x 4096 2405 -> 2267.  squared relu
-//    333: 6912 x 2048 29 -> 20; 1355: 50 -> 44, 18432 x 4096 193 -> 183
+//    2816 x 1024 26 -> 12; 1355: 5632 x 2048 72 -> 58, 14336 x 4096 282 -> 264;
+//    16384: 2816 x 1024 228 -> 156, 14336 x 4096 2792 -> 2631.  gelu 16384: 7168 x
+//    2048 429 -> 367, 19456 x 4096 1957 -> 1820.  clamped 16384: 4352 x 2048 522 ->
+//    441, 11904 x 4096 2338 -> 2255.  squared relu 333: 6912 x 2048 25 -> 16; 1355:
+//    43 -> 37, 18432 x 4096 179 -> 170.  From 129 to 320 rows by 1.03 to 1.9, but
+//    for a last round of few tiles (320: 28672 x 4096 swiglu 86 -> 89)
 //  * not for few tiles of some depth, which the library takes in shares: 333:
 //    2048 x 2048 10.7 -> 12.9, 2048 x 7168 30 -> 43, 1024 x 3328 13 -> 18.  Of up
 //    to 1024 deep fewer than 64 lose less than half a microsecond (129: 1024 x 1024
