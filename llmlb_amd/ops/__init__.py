@@ -799,6 +799,35 @@ def _tile_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
     return out
 
 
+def _float_gemm(x: torch.Tensor, weight: torch.Tensor, act: str = "plain",
+                out: torch.Tensor | None = None, tile: int = -1
+                ) -> torch.Tensor | None:
+    """act(x @ W^T) of 32-bit rows by float_gemm.hip, or None where it does
+    not take the operands.  act: "plain", "relu2" or "gelu"; ``tile``: one of
+    the kernel's, -1: its choice."""
+    if (act not in ("plain", "relu2", "gelu") or not x.is_cuda
+            or _lib is None or _USE_CUSTOM_DECODE_GEMM != "auto"
+            or x.dtype != torch.float32 or not _only_numbers(x, weight)
+            or not _fit(x, weight) or not x.shape[0]):
+        return None
+    stream = _stream_as_library(x)
+    if stream is None:
+        return None
+    found = _product_of(x, weight, act, out, 0)
+    if found is None:
+        return None
+    M, out = found
+    rc = _lib.ll_float_gemm(
+        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
+        ctypes.c_int(x.shape[0]), ctypes.c_int(M), ctypes.c_int(x.shape[1]),
+        ctypes.c_int(x.stride(0)), ctypes.c_int(_ROW_ACTS[act]),
+        ctypes.c_int(tile), stream)
+    if rc == -2:
+        return None
+    _check(rc, "ll_float_gemm")
+    return out
+
+
 def _takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return (x.dtype == torch.bfloat16 and x.is_cuda and _lib is not None
             and _only_numbers(x, weight) and _fit(x, weight)
@@ -812,14 +841,16 @@ def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
                out: torch.Tensor | None = None, up: int = 0,
                a: float = 0.0, b: float = 0.0) -> torch.Tensor | None:
-    """act(x @ W^T) of bf16 rows in one launch, into ``out`` (columns of
-    wider rows) if given; None where neither row_gemm.hip (up to 128 rows)
-    nor tile_gemm.hip takes it.
+    """act(x @ W^T) in one launch, into ``out`` (columns of wider rows) if
+    given; None where neither row_gemm.hip (up to 128 bf16 rows), tile_gemm.hip
+    nor, for 32-bit rows, float_gemm.hip takes it.
 
     act: "relu2", "gelu" (its tanh form), "capped" (float32,
     a tanh(z / a); a = 0: a widening); with gate in the first rows of
     ``weight`` and up from row ``up`` on "swiglu", and "clamped" with
     limit a and sharpness b (see hybrid.clamped_swiglu)."""
+    if x.dtype == torch.float32:
+        return _float_gemm(x, weight, act, out)
     if _USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_product(x, weight):
         return None
     product = _row_gemm if x.shape[0] <= 128 else _tile_gemm
@@ -837,6 +868,8 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor,
     = this, "1"/"on" = the staged kernels of decode_gemm.hip wherever
     they are legal, "0"/"off" = hipBLASLt only."""
     mode = _USE_CUSTOM_DECODE_GEMM
+    if x.dtype == torch.float32:
+        return linear_rows(x, weight)
     if mode in ("0", "false", "off") or not _takes_row_gemm(x, weight):
         return torch.nn.functional.linear(x, weight)
     N, K = x.shape
@@ -861,10 +894,13 @@ def linear_decode(x: torch.Tensor, weight: torch.Tensor,
 
 
 def linear_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """out = x @ W^T for more rows than a decode step has: prompts."""
+    """out = x @ W^T for more rows than a decode step has: prompts, and all
+    32-bit products."""
     out = None
-    if (_USE_CUSTOM_DECODE_GEMM == "auto" and _takes_product(x, weight)
-            and x.shape[0] > 128):
+    if x.dtype == torch.float32:
+        out = _float_gemm(x, weight)
+    elif (_USE_CUSTOM_DECODE_GEMM == "auto" and _takes_product(x, weight)
+          and x.shape[0] > 128):
         out = _tile_gemm(x, weight)
     return torch.nn.functional.linear(x, weight) if out is None else out
 

@@ -1,0 +1,299 @@
+// Products of 32-bit matrices on the matrix cores' bf16 instructions:
+//
+//   out[N, M] = act(x[N, K] W[M, K]^T)     float, summed in float
+//
+// A float is the sum of three bf16 numbers without a remainder (8 + 8 + 8
+// bits), so a product of two is nine products of those, of which the three
+// smallest are left out: less than 2^-21 of the product, 2^-24 on average.  Six
+// times the work at sixteen times the rate of the float instructions, and the
+// sum is rounded once in 32 of the depth where theirs is in every four: errors
+// of normal numbers 1024 deep are 1.7e-7 to 2.4e-7 of the result (the library's
+// product 2.9e-7 to 5.7e-7), 3328 deep 3.2e-7 to 4.5e-7 (5.2e-7 to 1.0e-6).
+//
+// Bound by vector instructions, which take numbers apart (5.5 a number of a
+// tile's edge), beside matrix instructions: of one tile of 64 x 64 1.4 and 1.5
+// thousand cycles a SIMD for 128 of the depth, and what a compute unit takes in
+// comes on top.  So waves have one stage and no pipeline of their own, and two
+// to four of them a SIMD cover each other (two stages and a software pipeline
+// at one wave a SIMD: 600 rows, 1024 x 1024 16 us, 13.5 this way).  us, the
+// library -> here, weights from HBM:
+//   600 rows: 1024 x 1024 17.3 -> 13.8, 3328 x 1024 38 -> 34, 1024 x 3328 43 ->
+//       33; 64 rows: 8.3 -> 5.1, 12.4 -> 8.4, 11.5 -> 11.6; 16 rows of 4096 x
+//       2048 12.3 -> 9.4; 1600 rows of 4096 x 2048 264 -> 166 (162 TFLOP/s)
+#include <float.h>
+
+#include "hybrid/row_act.h"
+#include "hybrid/lds_copy.h"
+
+// Two floats as sums of three bf16 numbers each, by cutting bits off.
+__device__ __forceinline__ void cut3(unsigned a, unsigned b,
+                                     unsigned (&part)[3]) {
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    part[t] = __builtin_amdgcn_perm(b, a, 0x07060302);
+    a = __float_as_uint(__uint_as_float(a) -
+                        __uint_as_float(a & 0xffff0000u));
+    b = __float_as_uint(__uint_as_float(b) -
+                        __uint_as_float(b & 0xffff0000u));
+  }
+}
+
+// One tile, 16 NT rows of x against 16 MT of W; KW waves share it and split
+// the depth in pieces of 32 (rows of 128 bytes), as RowTile's do.
+template <int NT, int MT, int KW>
+struct FloatTile {
+  static constexpr int F = NT + MT, C = 2 * F;
+  static constexpr int STAGE = F * 2048;  // one piece of all rows
+  static constexpr int RP = 16 * MT + 4;  // row of the sums
+  static constexpr int STAGES = KW * STAGE, SUMS = KW * 16 * NT * RP * 4;
+  static constexpr int LDS = STAGES > SUMS ? STAGES : SUMS;
+
+  // x, w: the tile's first rows; last_x, last_w: the last ones there are
+  static __device__ __forceinline__ void run(char* lds, int K, int step,
+                                             const float* x, int ldx,
+                                             int last_x, const float* w,
+                                             int last_w) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int lo = lane & 15, hi = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    char* const own = lds + wave * STAGE;
+    const unsigned own_byte = lds_byte(own);
+    // rows and pieces of 16 bytes lie as RowTile's
+    unsigned at[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int r = 8 * j + lane / 8, piece = ((lane & 7) ^ ((r >> 1) & 7)) * 4;
+      const int rw = r - 16 * NT;
+      at[j] = j < 2 * NT
+                  ? (unsigned)(r < last_x ? r : last_x) * (unsigned)ldx
+                  : (unsigned)(rw < last_w ? rw : last_w) * (unsigned)K;
+      at[j] = (at[j] + piece) * 4;
+    }
+    const int pieces = K / 32;
+    const int count = pieces > wave ? (pieces - wave + KW - 1) / KW : 0;
+    const int turn = count ? step % count : 0;
+    auto copy = [&](int i) {
+      const int turned = i + turn;
+      const int k0 =
+          (wave + (turned < count ? turned : turned - count) * KW) * 32;
+#pragma unroll
+      for (int j = 0; j < C; ++j)
+        copy_to_lds(reinterpret_cast<const bf16_t*>((j < 2 * NT ? x : w) + k0),
+                    at[j], own_byte + j * 1024);
+    };
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+      for (int b = 0; b < NT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (count) copy(0);
+    for (int i = 0; i < count; ++i) {
+      wait_copies<0>();
+      u32x4 raw[F][2], part[F][3];
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          raw[f][s] = *reinterpret_cast<const u32x4*>(
+              own + f * 2048 + lo * 128 + ((s * 4 + hi) ^ (lo >> 1)) * 16);
+      // the stage has been read before its next copy starts
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (i + 1 < count) copy(i + 1);
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            unsigned cut[3];
+            cut3(raw[f][s][2 * c], raw[f][s][2 * c + 1], cut);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) part[f][t][2 * s + c] = cut[t];
+          }
+      constexpr int WP[] = {2, 0, 1, 1, 0, 0}, XP[] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+          for (int b = 0; b < NT; ++b)
+            acc[a][b] =
+                mfma(part[NT + a][WP[q]], part[b][XP[q]], acc[a][b]);
+    }
+
+    __syncthreads();  // the sums lie where the stages were
+    float* const sums = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int b = 0; b < NT; ++b)
+#pragma unroll
+      for (int a = 0; a < MT; ++a)
+        *reinterpret_cast<f32x4*>(
+            &sums[(wave * 16 * NT + b * 16 + lo) * RP + a * 16 + hi * 4]) =
+            acc[a][b];
+    __syncthreads();
+  }
+
+  static __device__ __forceinline__ f32x4 sum(const char* lds, int r, int c) {
+    const float* const sums = reinterpret_cast<const float*>(lds);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < KW; ++w)
+      v += *reinterpret_cast<const f32x4*>(
+          &sums[(w * 16 * NT + r) * RP + c]);
+    return v;
+  }
+};
+
+// One output as a loop over the depth, where the sum of parts will not do.
+// The parts of an infinite number are that and no number.  Parts of numbers
+// below 2^-102 may be too small for a bf16 number; what is lost of a depth of
+// 10^6 is 2^-24 of a result of 10^-20 at most, unless the other numbers are
+// above 10^5.
+static __device__ __noinline__ float float_dot(const float* x, const float* w,
+                                               int K) {
+  float v = 0.f;
+  for (int k = 0; k < K; ++k) v = fmaf(x[k], w[k], v);
+  return v;
+}
+
+template <int NT, int MT, int KW>
+__global__ __launch_bounds__(KW * 64, 1) void float_gemm_kernel(
+    float* __restrict__ out, int ld_out, const float* __restrict__ x,
+    const float* __restrict__ w, int N, int M, int K, int ldx, int kind,
+    bool narrow) {
+  using Tile = FloatTile<NT, MT, KW>;
+  extern __shared__ __align__(1024) char lds[];
+  // One of eight XCDs has every eighth tile of W, and goes through them by
+  // eight tiles of x at a time: what its workgroups read at once fits its L2.
+  // Where W is narrow it has every eighth tile of x.
+  const int across = (N + 16 * NT - 1) / (16 * NT);
+  const int down = (M + 16 * MT - 1) / (16 * MT);
+  const int xcd = blockIdx.x % 8, in = blockIdx.x / 8;
+  int tile_x, tile_w, turn;
+  if (narrow) {
+    tile_x = in / down * 8 + xcd, tile_w = turn = in % down;
+  } else {
+    const int each = (down + 7) / 8, first = in / (8 * each) * 8;
+    const int rest = in - first * each;
+    const int wide = across - first < 8 ? across - first : 8;
+    turn = rest / wide;
+    tile_x = first + rest % wide, tile_w = turn * 8 + xcd;
+  }
+  const int n0 = tile_x * 16 * NT, m0 = tile_w * 16 * MT;
+  if (n0 >= N || m0 >= M) return;
+  Tile::run(lds, K, turn, x + (size_t)n0 * ldx, ldx, N - 1 - n0,
+            w + (size_t)m0 * K, M - 1 - m0);
+  for (int i = threadIdx.x; i < 16 * NT * 4 * MT; i += KW * 64) {
+    const int r = i / (4 * MT), c = i % (4 * MT) * 4;
+    if (n0 + r >= N || m0 + c >= M) continue;
+    f32x4 v = Tile::sum(lds, r, c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float size = fabsf(v[j]);
+      if (!(size <= FLT_MAX) || (size < 1e-20f && size > 0.f))
+        v[j] = float_dot(x + (size_t)(n0 + r) * ldx,
+                         w + (size_t)(m0 + c + j) * K, K);
+      if (kind == RELU2) {
+        v[j] = fmaxf(v[j], 0.f);
+        v[j] *= v[j];
+      } else if (kind == GELU) {
+        v[j] = gelu_tanh_f(v[j]);
+      }
+    }
+    *reinterpret_cast<f32x4*>(out + (size_t)(n0 + r) * ld_out + m0 + c) = v;
+  }
+}
+
+struct FloatGemm {
+  float* out;
+  int ld_out;
+  const float *x, *w;
+  int N, M, K, ldx, kind;
+  hipStream_t stream;
+};
+
+template <int NT, int MT, int KW>
+static int float_gemm_launch(const FloatGemm& p) {
+  auto* kernel = &float_gemm_kernel<NT, MT, KW>;
+  constexpr int lds = FloatTile<NT, MT, KW>::LDS;
+  static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const long long down = (p.M + 16 * MT - 1) / (16 * MT);
+  const long long across = (p.N + 16 * NT - 1) / (16 * NT);
+  const bool narrow = across > down && down < 64;
+  const long long grid =
+      narrow ? (across + 7) / 8 * 8 * down : (down + 7) / 8 * 8 * across;
+  if (grid > 1 << 30) return -2;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(KW * 64), lds,
+                     p.stream, p.out, p.ld_out, p.x, p.w, p.N, p.M, p.K,
+                     p.ldx, p.kind, narrow);
+  HY_CHECK();
+  return 0;
+}
+
+// Tiles that there are: how many a compute unit has at once, us of a tile 1024
+// deep where each unit has one and where each has all of them, and of the
+// beginning and end, fitted to products 1024 and 3328 deep.
+struct FloatTileTime {
+  int rows, cols, at_once;
+  float one, all, ends;
+};
+static const FloatTileTime FLOAT_TILES[] = {
+    {16, 16, 4, 2.8f, 8.f, 2.1f},  {32, 16, 3, 3.5f, 8.3f, 2.1f},
+    {32, 32, 2, 4.8f, 9.3f, 1.9f}, {48, 32, 2, 4.7f, 11.5f, 3.7f},
+    {48, 64, 1, 8.f, 12.5f, 5.f},  {48, 48, 3, 7.5f, 22.f, 4.5f},
+    {64, 64, 2, 12.f, 21.f, 5.4f}};
+
+// The tile that is estimated to take least.  A last round takes as long as
+// the units with most of its tiles.
+static int float_tile(int N, int M, int K) {
+  int best = 0;
+  float least = 0.f;
+  for (int t = 0; t < (int)(sizeof(FLOAT_TILES) / sizeof(FloatTileTime));
+       ++t) {
+    const FloatTileTime& at = FLOAT_TILES[t];
+    const long long n = ((long long)N + at.rows - 1) / at.rows *
+                        ((M + at.cols - 1) / at.cols);
+    const int round = 256 * at.at_once, rest = (int)(n % round);
+    float tiles = (float)(n / round) * at.all;
+    if (rest)
+      tiles += at.one + (rest <= 256 ? 0.f
+                                     : (at.all - at.one) *
+                                           (float)((rest - 1) / 256) /
+                                           (float)(at.at_once - 1));
+    const float us = tiles * ((float)K / 1024.f) + at.ends;
+    if (t == 0 || us < least) least = us, best = t;
+  }
+  return best;
+}
+
+// Rows of x start ldx numbers apart, those of out ld_out.  tile: -1, or the
+// one to take.  0: done, -2: not for this kernel.
+extern "C" int ll_float_gemm(void* out, int ld_out, const void* x,
+                             const void* w, int N, int M, int K, int ldx,
+                             int kind, int tile, void* stream) {
+  // copies are at a lane's 32-bit offset in bytes
+  if (N <= 0 || M <= 0 || K <= 0 || M % 4 || K % 32 || ldx < K || ldx % 4 ||
+      ld_out < M || ld_out % 4 || K >= 1 << 24 || ldx >= 1 << 24 ||
+      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16 ||
+      (kind != PLAIN && kind != RELU2 && kind != GELU))
+    return -2;
+  // a tile's beginning and end are most of a shallow product (us, the library
+  // and here: 1600 rows, 1024 x 128 8.8 and 12.3, 1024 x 256 12.5 and 13.8)
+  if (tile < 0 && K < 256 && N > 512) return -2;
+  const FloatGemm p{(float*)out, ld_out, (const float*)x, (const float*)w,
+                    N, M, K, ldx, kind, (hipStream_t)stream};
+  switch (tile < 0 ? float_tile(N, M, K) : tile) {
+    case 0: return float_gemm_launch<1, 1, 8>(p);
+    case 1: return float_gemm_launch<2, 1, 8>(p);
+    case 2: return float_gemm_launch<2, 2, 8>(p);
+    case 3: return float_gemm_launch<3, 2, 8>(p);
+    case 4: return float_gemm_launch<3, 4, 8>(p);
+    case 5: return float_gemm_launch<3, 3, 4>(p);
+    case 6: return float_gemm_launch<4, 4, 4>(p);
+  }
+  return -2;
+}

@@ -1,0 +1,121 @@
+"""Products of 32-bit matrices (float_gemm.hip) against 64-bit products of the
+same numbers, at the edges of its tiles."""
+import pytest
+import torch
+
+import llmlb_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TILES = 7
+
+
+def _close(out, x, w):
+    """Of every product 2^-21 is left out at most, and a sum of K is rounded
+    less than K times."""
+    x, w = x.double(), w.double()
+    bound = (x.abs() @ w.abs().T) * (2.0 ** -21 + x.shape[1] * 2.0 ** -24)
+    assert ((out.double() - x @ w.T).abs() <= bound).all()
+
+
+def _rows(N, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(N, K + 8, generator=g, device=DEV)[:, 4:4 + K]
+
+
+# depths of one piece, of fewer pieces than waves and of a remainder; rows and
+# outputs that are no whole tiles; matrices narrow enough to go by rows
+@pytest.mark.parametrize("tile", range(TILES))
+@pytest.mark.parametrize("N,M,K", [
+    (1, 4, 32), (17, 36, 160), (50, 68, 288), (65, 260, 1056),
+    (1030, 100, 64), (300, 1028, 96), (700, 2052, 32)])
+def test_tiles(N, M, K, tile):
+    x, w = _rows(N, K, N + M), _rows(M, K, K).contiguous()
+    wide = torch.full((N, M + 8), 7.0, device=DEV)
+    out = ops._float_gemm(x, w, out=wide[:, 4:4 + M], tile=tile)
+    _close(out, x, w)
+    assert (wide[:, :4] == 7).all() and (wide[:, 4 + M:] == 7).all()
+
+
+@pytest.mark.parametrize("N,M,K", [(1, 1024, 1024), (300, 288, 1024),
+                                   (600, 1024, 3328)])
+def test_errors_are_not_the_librarys(N, M, K):
+    x, w = _rows(N, K, 1), _rows(M, K, 2).contiguous()
+    ref = x.double() @ w.double().T
+    ours, library = ((t.double() - ref).norm() / ref.norm() for t in
+                     (ops.linear_rows(x, w), torch.nn.functional.linear(x, w)))
+    assert ours <= library
+
+
+@pytest.mark.parametrize("act", ["relu2", "gelu"])
+@pytest.mark.parametrize("N", [5, 130])
+def test_activations_are_those_of_their_own_kernels(N, act):
+    from llmlb_amd.ops import hybrid as hy
+    x, w = _rows(N, 256, 3), _rows(512, 256, 4).contiguous()
+    z = ops._float_gemm(x, w)
+    if act == "gelu":
+        hy.gelu_tanh_(z)
+    else:
+        hy.squared_relu(z, z)
+    assert torch.equal(ops.linear_act(x, w, act), z)
+
+
+def test_numbers_that_do_not_come_apart():
+    """Infinities, no numbers, numbers that round up to infinity as bf16, and
+    ones whose parts bf16 does not hold."""
+    x, w = _rows(70, 256, 5).contiguous(), _rows(68, 256, 6).contiguous()
+    inf = float("inf")
+    x[3, 7], x[5, 9], w[11, 3] = inf, float("nan"), -inf
+    x[8], x[20, 5] = 3e38 / 256, 3.402e38
+    w[30] *= 1e-30
+    x[40] *= 1e-36
+    x[41] = 0.0
+    out, ref = ops.linear_rows(x, w), (x.double() @ w.double().T)
+    exact = ref.float()
+    assert torch.equal(out.isnan(), exact.isnan())
+    assert torch.equal(out.isinf(), exact.isinf())
+    assert torch.equal(out[out.isinf()], exact[exact.isinf()])
+    keep = [i for i in range(70) if i not in (3, 5, 20)]
+    cols = [i for i in range(68) if i != 11]
+    x, w, out = x[keep], w[cols], out[keep][:, cols]
+    # what is below the smallest normal number may be lost
+    bound = (x.double().abs() @ w.double().abs().T) \
+        * (2.0 ** -21 + 256 * 2.0 ** -24) + 256 * 2.0 ** -126
+    assert ((out.double() - x.double() @ w.double().T).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("N,M,K,shift", [(3, 6, 64, 0), (3, 64, 48, 0),
+                                         (3, 64, 64, 1), (513, 64, 224, 0)])
+def test_other_operands_go_to_the_library(N, M, K, shift):
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(N, K + 4, generator=g, device=DEV)[:, shift:shift + K]
+    w = torch.randn(M, K, generator=g, device=DEV)
+    assert ops._float_gemm(x, w) is None
+    assert torch.equal(ops.linear_rows(x, w),
+                       torch.nn.functional.linear(x, w))
+    assert torch.equal(ops.linear_decode(x, w),
+                       torch.nn.functional.linear(x, w))
+
+
+def test_gradients_and_autocast_keep_the_library():
+    x = torch.randn(5, 64, device=DEV, requires_grad=True)
+    w = torch.randn(32, 64, device=DEV)
+    ops.linear_rows(x, w).sum().backward()
+    assert x.grad is not None
+    x = x.detach()
+    with torch.autocast("cuda", torch.bfloat16):
+        assert ops.linear_rows(x, w).dtype == torch.bfloat16
+        assert ops.linear_act(x, w, "gelu") is None
+
+
+def test_captured():
+    x, w = _rows(300, 512, 8).contiguous(), _rows(640, 512, 9).contiguous()
+    graph = torch.cuda.CUDAGraph()
+    ops.linear_rows(x, w)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = ops.linear_rows(x, w)
+    for seed in range(3):
+        x.copy_(_rows(300, 512, seed))
+        graph.replay()
+        assert torch.equal(out, ops.linear_rows(x, w))
