@@ -364,6 +364,13 @@ class LlamaForCausalLM(nn.Module):
                                            self.cfg.norm_eps, residual)
             if residual is None:
                 residual = h
+            fused = getattr(layer.qkv, "forward_rotary", None)
+            if fused is not None:
+                qkv = fused(normed, layer.q_local, layer.kv_local,
+                            self.cfg.head_dim, self.cos_sin, positions,
+                            kv_sink)
+                if qkv is not None:
+                    return *layer.split_qkv(qkv), residual
             qkv = layer.qkv(normed)
         q, k, v = layer.split_qkv(qkv)
         if kv_sink is not None:

@@ -182,6 +182,50 @@ def rope_kv_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _check(rc, "ll_rope_kv_append")
 
 
+def linear_rotary(x: torch.Tensor, weight: torch.Tensor, n_q: int,
+                  n_kv: int, head_dim: int, cos_sin: torch.Tensor,
+                  positions: torch.Tensor, kv_sink: tuple | None = None
+                  ) -> torch.Tensor | None:
+    """Queries, keys and values x @ W^T of up to 128 bf16 rows, in one launch
+    with what ``rope_apply`` or, with ``kv_sink`` (kcache, vcache, slots),
+    ``rope_kv_append`` do to them.  None where row_gemm.hip does not take the
+    operands."""
+    N, M = x.shape[0], (n_q + 2 * n_kv) * head_dim
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight)
+            or weight.dtype != x.dtype or weight.shape[0] != M
+            or x.stride(1) != 1 or not weight.is_contiguous()
+            or cos_sin.dtype != torch.float32 or cos_sin.dim() != 2
+            or cos_sin.shape[1] != head_dim or not cos_sin.is_contiguous()
+            or cos_sin.device != x.device or positions.device != x.device
+            or positions.shape != (N,)):
+        return None
+    caches = (None, None, None)
+    page = 1
+    if kv_sink is not None:
+        kcache, vcache, slots = kv_sink
+        if (kcache.dtype != x.dtype or kcache.dim() != 4
+                or kcache.shape != vcache.shape or vcache.dtype != x.dtype
+                or kcache.shape[1] != n_kv or kcache.shape[3] != head_dim
+                or not kcache.is_contiguous() or not vcache.is_contiguous()
+                or not x.device == kcache.device == vcache.device
+                == slots.device or slots.shape != (N,)):
+            return None
+        slots = slots.to(torch.int32).contiguous()
+        caches, page = (_ptr(kcache), _ptr(vcache), _ptr(slots)), \
+            kcache.shape[2]
+    pos = positions.to(torch.int32).contiguous()
+    out = torch.empty(N, M, device=x.device, dtype=x.dtype)
+    rc = _lib.ll_row_gemm_rotary(
+        _ptr(out), _ptr(x), _ptr(weight), _ptr(cos_sin), _ptr(pos), *caches,
+        ctypes.c_int(N), ctypes.c_int(n_q), ctypes.c_int(n_kv),
+        ctypes.c_int(head_dim), ctypes.c_int(x.shape[1]),
+        ctypes.c_int(x.stride(0)), ctypes.c_int(page), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "ll_row_gemm_rotary")
+    return out
+
+
 def swiglu(gateup: torch.Tensor) -> torch.Tensor:
     """gateup [T, 2*inter] -> silu(gate) * up  [T, inter]."""
     if not gateup.is_cuda or gateup.dtype != torch.bfloat16:

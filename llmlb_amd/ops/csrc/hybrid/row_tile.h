@@ -15,6 +15,10 @@
 #include "lds_copy.h"
 #include "mfma.h"
 
+struct Nothing {
+  __device__ __forceinline__ void operator()() const {}
+};
+
 template <int NT, int MT, int KW, int S>
 struct RowTile {
   static constexpr int ROWS = 16 * (NT + MT), C = ROWS / 8;
@@ -26,10 +30,12 @@ struct RowTile {
   // x_row(r), w_row(r): where the tile's row r of x, of W begins; ``step``:
   // any number, workgroups' differ.  The waves' sums are in LDS after it.
   // DOWN: W's depth goes down, w_row(r) is where r's column begins, r a
-  // multiple of 8, and its next number lies ld numbers further.
-  template <bool DOWN = false, class X, class W>
+  // multiple of 8, and its next number lies ld numbers further.  ``last``:
+  // called where a wave's last piece has come, to ask for what follows.
+  template <bool DOWN = false, class X, class W, class L = Nothing>
   static __device__ __forceinline__ void run(char* lds, int K, int step,
-                                             X x_row, W w_row, int ld = 0) {
+                                             X x_row, W w_row, int ld = 0,
+                                             L last = L{}) {
     static_assert(!DOWN || MT % 2 == 0, "pieces that turn in twos");
     const int tid = threadIdx.x, lane = tid & 63;
     const int lo = lane & 15, hi = lane >> 4;
@@ -93,6 +99,7 @@ struct RowTile {
         wait_copies<(S > 2 ? C : 0)>();
       else
         wait_copies<0>();
+      if (newer == 0) last();
       const char* st = own + i % S * STAGE;
       u32x4 wf[2][MT], xf[2][NT];
 #pragma unroll
@@ -126,6 +133,7 @@ struct RowTile {
       if (i + S < count) copy(i + S);
     }
 
+    if (count == 0) last();
     __syncthreads();  // the sums lie where the stages were
     float* const sums = reinterpret_cast<float*>(lds);
 #pragma unroll

@@ -20,18 +20,144 @@
 #include "hybrid/row_act.h"
 #include "hybrid/row_tile.h"
 
+// What becomes of the sums of a tile's row n of x: put(.., n, m, ..) stores
+// those of outputs m .. m + 3.  PAIRED: a tile's rows of W are first(m) and, as
+// many, second(m) of the same outputs.  What put will need that does not depend
+// on the sums is asked for before they are made: token(n) at once, early(token,
+// m), which takes a token's position to its table, with the last piece.
+struct PlainEnd {
+  static constexpr bool PAIRED = false;
+  struct Token {};
+  struct Early {};
+  RowAct act;
+  __device__ __forceinline__ Token token(int) const { return {}; }
+  __device__ __forceinline__ Early early(Token, int) const { return {}; }
+  __device__ __forceinline__ int first(int m) const { return m; }
+  __device__ __forceinline__ int second(int m) const { return m; }
+  // CAPPED results are floats, all others bf16
+  __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
+                                      Early, f32x4 v, f32x4) const {
+    if (act.kind != PLAIN) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = row_act(act, to_f(from_f<bf16_t>(v[i])));
+    }
+    const size_t at = (size_t)n * ld_out + m;
+    if (act.kind == CAPPED)
+      *reinterpret_cast<f32x4*>(static_cast<float*>(out) + at) = v;
+    else
+      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out) + at) =
+          make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+  }
+};
+// gate and up
+struct GatedEnd {
+  static constexpr bool PAIRED = true;
+  struct Token {};
+  struct Early {};
+  RowAct act;
+  __device__ __forceinline__ Token token(int) const { return {}; }
+  __device__ __forceinline__ Early early(Token, int) const { return {}; }
+  __device__ __forceinline__ int first(int m) const { return m; }
+  __device__ __forceinline__ int second(int m) const { return act.up + m; }
+  __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
+                                      Early, f32x4 v, f32x4 u) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = row_gate(act, to_f(from_f<bf16_t>(v[i])),
+                      to_f(from_f<bf16_t>(u[i])));
+    *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out) +
+                              (size_t)n * ld_out + m) =
+        make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+  }
+};
+// Queries, keys and values: the first two are rotated (halves of a head
+// together), and with caches keys and values are copied to the page slot of
+// their token as well; a slot below 0 has no place.  What rope_kv_append does
+// in a launch of its own, to the bit: decoding pays for launches.  us a step
+// with both, with this: one sequence of a small model 135.2, 127.9; 64 of four
+// layers of an 8B model 650.1, 644.2; 32 with 8-bit caches (rotation only)
+// 551.2, 546.7.
+struct RotaryEnd {
+  static constexpr bool PAIRED = true;
+  struct Token {
+    int position, slot;
+  };
+  struct Early {
+    float4 c, s;
+    int slot;
+  };
+  const float* cos_sin;        // [position][cosines, sines]
+  const int *positions, *slots;
+  bf16_t *kcache, *vcache;     // null: no caches
+  int shift, n_q, n_kv, page;  // half a head is 1 << shift numbers
+  __device__ __forceinline__ Token token(int n) const {
+    return {positions[n], kcache ? slots[n] : -1};
+  }
+  __device__ __forceinline__ Early early(Token t, int m) const {
+    const int half = 1 << shift, head = m >> shift, j = m & (half - 1);
+    Early e{};
+    if (head < n_q + n_kv) {
+      const float* cs = cos_sin + (size_t)t.position * (2 * half) + j;
+      e.c = *reinterpret_cast<const float4*>(cs);
+      e.s = *reinterpret_cast<const float4*>(cs + half);
+    }
+    e.slot = head >= n_q ? t.slot : -1;
+    return e;
+  }
+  __device__ __forceinline__ int first(int m) const {
+    return m + (m >> shift << shift);
+  }
+  __device__ __forceinline__ int second(int m) const {
+    return first(m) + (1 << shift);
+  }
+  __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
+                                      const Early& e, f32x4 v, f32x4 u) const {
+    const int half = 1 << shift, head = m >> shift, j = m & (half - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = to_f(from_f<bf16_t>(v[i]));
+      u[i] = to_f(from_f<bf16_t>(u[i]));
+    }
+    if (head < n_q + n_kv) {
+      const float c[4] = {e.c.x, e.c.y, e.c.z, e.c.w};
+      const float s[4] = {e.s.x, e.s.y, e.s.z, e.s.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a = v[i], b = u[i];
+        v[i] = fmaf(a, c[i], -(b * s[i]));
+        u[i] = fmaf(b, c[i], a * s[i]);
+      }
+    }
+    const uint2 lo = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+    const uint2 hi = make_uint2(pack2(u[0], u[1]), pack2(u[2], u[3]));
+    bf16_t* to = static_cast<bf16_t*>(out) + (size_t)n * ld_out + first(m);
+    *reinterpret_cast<uint2*>(to) = lo;
+    *reinterpret_cast<uint2*>(to + half) = hi;
+    if (e.slot < 0) return;
+    const bool is_v = head >= n_q + n_kv;
+    to = (is_v ? vcache : kcache) +
+         (((size_t)(e.slot / page) * n_kv + head - n_q - (is_v ? n_kv : 0)) *
+              page +
+          e.slot % page) *
+             (2 * half) +
+         j;
+    *reinterpret_cast<uint2*>(to) = lo;
+    *reinterpret_cast<uint2*>(to + half) = hi;
+  }
+};
+
 // The order in which a sum is made differs with the number of rows, as with
-// any product: tiles, waves and shares follow from it.  With gate and up, a
-// tile's rows are half of the one and half of the other, at the same
-// outputs.
-// M outputs; CAPPED results are floats, all others bf16
-template <int NT, int MT, int KW, int S, bool GATED>
+// any product: tiles, waves and shares follow from it.  M outputs, of PAIRED
+// ends pairs.
+template <int NT, int MT, int KW, int S, class End>
 __global__ __launch_bounds__(KW * 64, NT * MT > 24 ? 1 : 2)
 void row_gemm_kernel(
-    void* __restrict__ out_, int ld_out, const bf16_t* __restrict__ x,
-    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, RowAct act) {
+    void* __restrict__ out, int ld_out, const bf16_t* __restrict__ x,
+    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, End end) {
   using Tile = RowTile<NT, MT, KW, S>;
-  constexpr int OUT = GATED ? 8 * MT : 16 * MT;  // outputs a tile
+  constexpr int OUT = End::PAIRED ? 8 * MT : 16 * MT;  // outputs a tile
+  constexpr int ITEMS = 16 * NT * (OUT / 4);
   extern __shared__ __align__(1024) char lds[];
   // tiles of the same rows of W are 8 apart: on one XCD
   const int across = (N + 16 * NT - 1) / (16 * NT);
@@ -39,37 +165,37 @@ void row_gemm_kernel(
   const int tile = blockIdx.x / (8 * across) * 8 + in % 8;
   const int m0 = tile * OUT, n0 = in / 8 * 16 * NT;
   if (m0 >= M) return;
+  auto here = [&](int i, int& n, int& m) {
+    n = n0 + i / (OUT / 4), m = m0 + i % (OUT / 4) * 4;
+    return i < ITEMS && n < N && m < M;
+  };
+  int n, m;
+  typename End::Token token{};
+  typename End::Early early{};
+  const bool some = here(threadIdx.x, n, m);
+  if (some) token = end.token(n);
   Tile::run(
       lds, K, tile >> 3,
       [&](int r) {
         return x + (size_t)(n0 + r < N ? n0 + r : N - 1) * ldx;
       },
       [&](int r) {
-        const bool up = GATED && r >= OUT;
-        const int m = m0 + (up ? r - OUT : r);
-        return w + (size_t)((up ? act.up : 0) + (m < M ? m : M - 1)) * K;
+        const bool other = End::PAIRED && r >= OUT;
+        int m = m0 + (other ? r - OUT : r);
+        m = m < M ? m : M - 1;
+        return w + (size_t)(other ? end.second(m) : end.first(m)) * K;
+      },
+      0,
+      [&] {
+        if (some) early = end.early(token, m);
       });
-  Tile::each(OUT / 4, [&](int r, int c) {
-    f32x4 v = Tile::sum(lds, r, c);
-    if (GATED) {
-      const f32x4 u = Tile::sum(lds, r, c + OUT);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = row_gate(act, to_f(from_f<bf16_t>(v[i])),
-                        to_f(from_f<bf16_t>(u[i])));
-    } else if (act.kind != PLAIN) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = row_act(act, to_f(from_f<bf16_t>(v[i])));
-    }
-    if (n0 + r >= N || m0 + c >= M) return;
-    const size_t at = (size_t)(n0 + r) * ld_out + m0 + c;
-    if (!GATED && act.kind == CAPPED)
-      *reinterpret_cast<f32x4*>(static_cast<float*>(out_) + at) = v;
-    else
-      *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out_) + at) =
-          make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
-  });
+  for (int i = threadIdx.x; i < ITEMS; i += KW * 64) {
+    if (!here(i, n, m)) continue;
+    if (i != (int)threadIdx.x) early = end.early(end.token(n), m);
+    const f32x4 v = Tile::sum(lds, n - n0, m - m0);
+    const f32x4 u = End::PAIRED ? Tile::sum(lds, n - n0, m - m0 + OUT) : v;
+    end.put(out, ld_out, n, m, early, v, u);
+  }
 }
 
 // A share of the depth, ``depth`` numbers from blockIdx.y * depth on, into
@@ -128,30 +254,31 @@ __global__ __launch_bounds__(256) void row_gemm_join_kernel(
       make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
 }
 
+template <class End>
 struct RowGemm {
   void* out;
   int ld_out;
   const bf16_t *x, *w;
   int N, M, K, ldx;
-  RowAct act;
+  End end;
   hipStream_t stream;
 };
 
-template <int NT, int MT, int KW, int S, bool GATED>
-static int row_gemm_launch(const RowGemm& p) {
+template <int NT, int MT, int KW, int S, class End>
+static int row_gemm_launch(const RowGemm<End>& p) {
+  auto* kernel = &row_gemm_kernel<NT, MT, KW, S, End>;
   constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(row_gemm_kernel<NT, MT, KW, S, GATED>),
+      reinterpret_cast<const void*>(kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (sized != hipSuccess) return -1;
-  constexpr int OUT = GATED ? 8 * MT : 16 * MT;
+  constexpr int OUT = End::PAIRED ? 8 * MT : 16 * MT;
   const int down = (p.M + OUT - 1) / OUT;
   const int across = (p.N + 16 * NT - 1) / (16 * NT);
-  hipLaunchKernelGGL((row_gemm_kernel<NT, MT, KW, S, GATED>),
-                     dim3((down + 7) / 8 * 8 * across), dim3(KW * 64), lds,
-                     p.stream, p.out, p.ld_out, p.x, p.w, p.N, p.M, p.K,
-                     p.ldx, p.act);
+  hipLaunchKernelGGL(kernel, dim3((down + 7) / 8 * 8 * across), dim3(KW * 64),
+                     lds, p.stream, p.out, p.ld_out, p.x, p.w, p.N, p.M, p.K,
+                     p.ldx, p.end);
   HY_CHECK();
   return 0;
 }
@@ -173,10 +300,10 @@ static int row_gemm_launch(const RowGemm& p) {
 // than whole rounds say: another than 32 outputs has to take in 15% less (one
 // row of 20480 x 1024 11.0 with 48, 10.1 with 32; 16512 x 1024 9.2 with 32, 8.6
 // with 80).
-template <bool GATED>
-static int row_gemm_pick(const RowGemm& p) {
+template <class End>
+static int row_gemm_pick(const RowGemm<End>& p) {
   const int tiles = (p.N + 15) / 16;
-  const long long rows = GATED ? 2ll * p.M : p.M;
+  const long long rows = End::PAIRED ? 2ll * p.M : p.M;
   // what memory takes for W, in the same unit: 16 rows at 50 GB/s
   const float floor = rows / 2500.f;
   int nt = 0, mt = 0;
@@ -201,11 +328,11 @@ static int row_gemm_pick(const RowGemm& p) {
       // (3, 1) and (4, 1) take in no less; of gate and up, tiles of 8 outputs
       // by eight waves are for what they share (1024 x 128, one row: 3.0 with
       // them, 2.8 with 16; 1024 x 768 3.4, 3.7)
-      if ((n < 3 || m > 1) && (!GATED || m > 1 || p.K > 256)) look(n, m);
+      if ((n < 3 || m > 1) && (!End::PAIRED || m > 1 || p.K > 256)) look(n, m);
     }
   // waves that share the depth, and pieces of it on their way, fit LDS
 #define TILE(NT, MT, KW, S) \
-  case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S, GATED>(p);
+  case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S>(p);
   switch (nt * 8 + mt) {
     TILE(1, 1, 8, 2)
     TILE(1, 2, 4, 3)
@@ -318,9 +445,40 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
     return -2;
   const bool gated = kind == SWIGLU || kind == CLAMPED;
   if (read_twice(N, (size_t)M * (gated ? 2 : 1), K)) return -2;
-  const RowGemm p{out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K,
-                  ldx, RowAct{kind, up, a, b}, (hipStream_t)stream};
-  return gated ? row_gemm_pick<true>(p) : row_gemm_pick<false>(p);
+  const RowAct act{kind, up, a, b};
+  if (gated)
+    return row_gemm_pick(RowGemm<GatedEnd>{
+        out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K, ldx,
+        GatedEnd{act}, (hipStream_t)stream});
+  return row_gemm_pick(RowGemm<PlainEnd>{
+      out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K, ldx,
+      PlainEnd{act}, (hipStream_t)stream});
+}
+
+// Queries, keys and values of N rows, rotated, and with caches appended: see
+// RotaryEnd.  W holds n_q + 2 n_kv heads of D rows, D a power of two, in that
+// order; caches are [page][head][page slot][D].
+extern "C" int ll_row_gemm_rotary(void* out, const void* x, const void* w,
+                                  const void* cos_sin, const void* positions,
+                                  void* kcache, void* vcache,
+                                  const void* slots, int N, int n_q, int n_kv,
+                                  int D, int K, int ldx, int page,
+                                  void* stream) {
+  if (N <= 0 || N > 128 || n_q <= 0 || n_kv <= 0 || D < 8 || (D & (D - 1)) ||
+      n_q > 1 << 16 || n_kv > 1 << 16 || D > 1 << 10 || K <= 0 || K % 8 ||
+      ldx % 8 || page <= 0 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
+      (uintptr_t)out % 8 || (uintptr_t)cos_sin % 16 ||
+      (uintptr_t)kcache % 8 || (uintptr_t)vcache % 8 || !cos_sin ||
+      !positions || !kcache != !vcache || (kcache && !slots))
+    return -2;
+  const int M = (n_q + 2 * n_kv) * D;
+  if (read_twice(N, M, K) || ll_row_gemm_shares(N, M, K) > 1) return -2;
+  return row_gemm_pick(RowGemm<RotaryEnd>{
+      out, M, (const bf16_t*)x, (const bf16_t*)w, N, M / 2, K, ldx,
+      RotaryEnd{(const float*)cos_sin, (const int*)positions,
+                (const int*)slots, (bf16_t*)kcache, (bf16_t*)vcache,
+                __builtin_ctz(D) - 1, n_q, n_kv, page},
+      (hipStream_t)stream});
 }
 
 // The same for H pairs of rows and matrices at once, as latent attention needs

@@ -172,17 +172,31 @@ class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
             return _ops.linear_rows(x, self.weight)
         return torch.nn.functional.linear(x, self.weight, self.bias)
 
+    def _only_product(self) -> bool:
+        """Whether calling the module is the product with its weight and no
+        more: no bias, hooks, 8-bit weights or another forward."""
+        from .. import ops as _ops
+        return not (self.bias is not None or _ops._FP8_WEIGHTS
+                    or _watched(self)
+                    or getattr(self.forward, "__func__", None)
+                    is not ColumnParallelLinear.forward)
+
+    def forward_rotary(self, x: torch.Tensor, *args) -> torch.Tensor | None:
+        """The shard's queries, keys and values with what follows in the
+        product's own launch (``ops.linear_rotary``), or None where that would
+        be something else, or more than 128 rows."""
+        from .. import ops as _ops
+        if x.dim() != 2 or x.shape[0] > 128 or not self._only_product():
+            return None
+        return _ops.linear_rotary(x, self.weight, *args)
+
     def forward_swiglu(self, x: torch.Tensor) -> torch.Tensor | None:
         """swiglu of the shard's [gate | up] outputs in the product's own
         launch, or None where calling the module and then swiglu would do
-        something else or more: a bias, hooks, another forward, prompts
-        with 8-bit weights."""
+        something else or more."""
         from .. import ops as _ops
-        if (self.bias is not None or _ops._FP8_WEIGHTS or _ops._FUSED_SWIGLU
-                or (x.shape[0] > 128 and _ops.fp8_prefill_active())
-                or _watched(self)
-                or getattr(self.forward, "__func__", None)
-                is not ColumnParallelLinear.forward):
+        if (not self._only_product() or _ops._FUSED_SWIGLU
+                or (x.shape[0] > 128 and _ops.fp8_prefill_active())):
             return None
         return _ops.linear_act(x, self.weight, "swiglu",
                                up=self.out_local // 2)
