@@ -11,15 +11,17 @@
 // product 2.9e-7 to 5.7e-7), 3328 deep 3.2e-7 to 4.5e-7 (5.2e-7 to 1.0e-6).
 //
 // Bound by vector instructions, which take numbers apart (5.5 a number of a
-// tile's edge), beside matrix instructions: of one tile of 64 x 64 1.4 and 1.5
-// thousand cycles a SIMD for 128 of the depth, and what a compute unit takes in
-// comes on top.  So waves have one stage and no pipeline of their own, and two
-// to four of them a SIMD cover each other (two stages and a software pipeline
-// at one wave a SIMD: 600 rows, 1024 x 1024 16 us, 13.5 this way).  us, the
-// library -> here, weights from HBM:
-//   600 rows: 1024 x 1024 17.3 -> 13.8, 3328 x 1024 38 -> 34, 1024 x 3328 43 ->
-//       33; 64 rows: 8.3 -> 5.1, 12.4 -> 8.4, 11.5 -> 11.6; 16 rows of 4096 x
-//       2048 12.3 -> 9.4; 1600 rows of 4096 x 2048 264 -> 166 (162 TFLOP/s)
+// tile's edge), beside matrix instructions (a tile of 64 x 64, of 128 of the
+// depth: 1630 and 1540 cycles a SIMD, 3060 in all), and by how tiles fill the
+// last round.  So waves have one stage and no pipeline of their own, and two to
+// four of them a SIMD cover each other (two stages and a software pipeline at
+// one wave a SIMD: 600 rows, 1024 x 1024 16 us, 13.5 this way); larger tiles
+// take less apart (600 rows of 4096 x 2048 74 us with 64 x 64, 61 with 80 x 64).
+// us, the library -> here, weights from HBM:
+//   600 rows: 1024 x 1024 16.5 -> 13.4, 3328 x 1024 38 -> 32, 4128 x 1024 52 ->
+//       39, 1024 x 3328 43 -> 32; 64 rows: 8.3 -> 5.1, 12.5 -> 8.4, 13.7 ->
+//       12.7, 11.5 -> 11.7; 16 rows of 4096 x 2048 12.5 -> 9.5; 1600 rows of
+//       4096 x 2048 245 -> 143 (188 TFLOP/s)
 #include <float.h>
 
 #include "hybrid/row_act.h"
@@ -45,7 +47,7 @@ struct FloatTile {
   static constexpr int F = NT + MT, C = 2 * F;
   static constexpr int STAGE = F * 2048;  // one piece of all rows
   static constexpr int RP = 16 * MT + 4;  // row of the sums
-  static constexpr int STAGES = KW * STAGE, SUMS = KW * 16 * NT * RP * 4;
+  static constexpr int STAGES = KW * STAGE, SUMS = KW / 2 * 16 * NT * RP * 4;
   static constexpr int LDS = STAGES > SUMS ? STAGES : SUMS;
 
   // x, w: the tile's first rows; last_x, last_w: the last ones there are
@@ -121,15 +123,30 @@ struct FloatTile {
                 mfma(part[NT + a][WP[q]], part[b][XP[q]], acc[a][b]);
     }
 
-    __syncthreads();  // the sums lie where the stages were
-    float* const sums = reinterpret_cast<float*>(lds);
+    // the sums lie where the stages were: first those of half of the waves,
+    // then the others' with them
+    auto at_of = [&](int w, int a, int b) {
+      return reinterpret_cast<f32x4*>(
+          reinterpret_cast<float*>(lds) + (w * 16 * NT + b * 16 + lo) * RP +
+          a * 16 + hi * 4);
+    };
+    __syncthreads();
+    if (wave >= KW / 2) {
 #pragma unroll
-    for (int b = 0; b < NT; ++b)
+      for (int b = 0; b < NT; ++b)
 #pragma unroll
-      for (int a = 0; a < MT; ++a)
-        *reinterpret_cast<f32x4*>(
-            &sums[(wave * 16 * NT + b * 16 + lo) * RP + a * 16 + hi * 4]) =
-            acc[a][b];
+        for (int a = 0; a < MT; ++a) *at_of(wave - KW / 2, a, b) = acc[a][b];
+    }
+    __syncthreads();
+    if (wave < KW / 2) {
+#pragma unroll
+      for (int b = 0; b < NT; ++b)
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+          f32x4* const at = at_of(wave, a, b);
+          *at = *at + acc[a][b];
+        }
+    }
     __syncthreads();
   }
 
@@ -137,7 +154,7 @@ struct FloatTile {
     const float* const sums = reinterpret_cast<const float*>(lds);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int w = 0; w < KW; ++w)
+    for (int w = 0; w < KW / 2; ++w)
       v += *reinterpret_cast<const f32x4*>(
           &sums[(w * 16 * NT + r) * RP + c]);
     return v;
@@ -204,6 +221,11 @@ __global__ __launch_bounds__(KW * 64, 1) void float_gemm_kernel(
   }
 }
 
+// Whether tiles of x and not those of W are dealt to the XCDs
+static bool narrow_w(long long across, long long down) {
+  return across > down && down < 64;
+}
+
 struct FloatGemm {
   float* out;
   int ld_out;
@@ -223,7 +245,7 @@ static int float_gemm_launch(const FloatGemm& p) {
   if (sized != hipSuccess) return -1;
   const long long down = (p.M + 16 * MT - 1) / (16 * MT);
   const long long across = (p.N + 16 * NT - 1) / (16 * NT);
-  const bool narrow = across > down && down < 64;
+  const bool narrow = narrow_w(across, down);
   const long long grid =
       narrow ? (across + 7) / 8 * 8 * down : (down + 7) / 8 * 8 * across;
   if (grid > 1 << 30) return -2;
@@ -242,10 +264,12 @@ struct FloatTileTime {
   float one, all, ends;
 };
 static const FloatTileTime FLOAT_TILES[] = {
-    {16, 16, 4, 2.8f, 8.f, 2.1f},  {32, 16, 3, 3.5f, 8.3f, 2.1f},
-    {32, 32, 2, 4.8f, 9.3f, 1.9f}, {48, 32, 2, 4.7f, 11.5f, 3.7f},
-    {48, 64, 1, 8.f, 12.5f, 5.f},  {48, 48, 3, 7.5f, 22.f, 4.5f},
-    {64, 64, 2, 12.f, 21.f, 5.4f}};
+    {16, 16, 4, 2.8f, 8.f, 2.1f},     {32, 16, 3, 3.5f, 8.3f, 2.1f},
+    {32, 32, 2, 4.8f, 9.3f, 1.9f},    {48, 32, 2, 4.7f, 11.f, 3.7f},
+    {48, 64, 1, 7.7f, 12.3f, 5.5f},   {48, 48, 3, 7.6f, 22.f, 5.f},
+    {48, 64, 2, 9.4f, 17.f, 6.f},     {64, 64, 2, 11.7f, 20.5f, 6.5f},
+    {80, 64, 2, 13.2f, 22.5f, 7.5f},  {64, 96, 2, 14.9f, 27.f, 8.f},
+    {80, 80, 2, 15.3f, 27.5f, 9.f}};
 
 // The tile that is estimated to take least.  A last round takes as long as
 // the units with most of its tiles.
@@ -255,8 +279,12 @@ static int float_tile(int N, int M, int K) {
   for (int t = 0; t < (int)(sizeof(FLOAT_TILES) / sizeof(FloatTileTime));
        ++t) {
     const FloatTileTime& at = FLOAT_TILES[t];
-    const long long n = ((long long)N + at.rows - 1) / at.rows *
-                        ((M + at.cols - 1) / at.cols);
+    const long long across = (N + at.rows - 1) / at.rows;
+    const long long down = (M + at.cols - 1) / at.cols;
+    // those of the XCD that has most, of 32 units
+    const long long n = 8 * (narrow_w(across, down)
+                                 ? (across + 7) / 8 * down
+                                 : (down + 7) / 8 * across);
     const int round = 256 * at.at_once, rest = (int)(n % round);
     float tiles = (float)(n / round) * at.all;
     if (rest)
@@ -293,7 +321,11 @@ extern "C" int ll_float_gemm(void* out, int ld_out, const void* x,
     case 3: return float_gemm_launch<3, 2, 8>(p);
     case 4: return float_gemm_launch<3, 4, 8>(p);
     case 5: return float_gemm_launch<3, 3, 4>(p);
-    case 6: return float_gemm_launch<4, 4, 4>(p);
+    case 6: return float_gemm_launch<3, 4, 4>(p);
+    case 7: return float_gemm_launch<4, 4, 4>(p);
+    case 8: return float_gemm_launch<5, 4, 4>(p);
+    case 9: return float_gemm_launch<4, 6, 4>(p);
+    case 10: return float_gemm_launch<5, 5, 4>(p);
   }
   return -2;
 }

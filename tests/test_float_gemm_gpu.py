@@ -7,7 +7,7 @@ import llmlb_amd.ops as ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-TILES = 7
+TILES = 11
 
 
 def _close(out, x, w):
@@ -27,7 +27,7 @@ def _rows(N, K, seed):
 # outputs that are no whole tiles; matrices narrow enough to go by rows
 @pytest.mark.parametrize("tile", range(TILES))
 @pytest.mark.parametrize("N,M,K", [
-    (1, 4, 32), (17, 36, 160), (50, 68, 288), (65, 260, 1056),
+    (1, 4, 32), (17, 36, 160), (50, 68, 288), (65, 260, 1056), (81, 100, 128),
     (1030, 100, 64), (300, 1028, 96), (700, 2052, 32)])
 def test_tiles(N, M, K, tile):
     x, w = _rows(N, K, N + M), _rows(M, K, K).contiguous()
