@@ -360,15 +360,21 @@ class LlamaForCausalLM(nn.Module):
             if qkv is not None and layer.qkv.bias is not None:
                 qkv = qkv + layer.qkv.bias
         if qkv is None:
+            fused = getattr(layer.qkv, "forward_rotary", None)
+            after = (layer.q_local, layer.kv_local, self.cfg.head_dim,
+                     self.cos_sin, positions, kv_sink)
+            if fused is not None and ops.norms_rows(h):
+                found = fused(h, *after, norm=(layer.input_norm_w,
+                                               self.cfg.norm_eps, residual))
+                if found is not None:
+                    qkv, total = found
+                    return *layer.split_qkv(qkv), h if total is None else total
             normed, residual = ops.rmsnorm(h, layer.input_norm_w,
                                            self.cfg.norm_eps, residual)
             if residual is None:
                 residual = h
-            fused = getattr(layer.qkv, "forward_rotary", None)
             if fused is not None:
-                qkv = fused(normed, layer.q_local, layer.kv_local,
-                            self.cfg.head_dim, self.cos_sin, positions,
-                            kv_sink)
+                qkv = fused(normed, *after)
                 if qkv is not None:
                     return *layer.split_qkv(qkv), residual
             qkv = layer.qkv(normed)
@@ -414,6 +420,11 @@ class LlamaForCausalLM(nn.Module):
                     return h, residual
                 # fall back mid-path: finish with bf16 swiglu+down
                 return layer.down.forward(ops.swiglu(gateup)), residual
+        fused = getattr(layer.gate_up, "forward_normed_swiglu", None)
+        found = fused(o, (layer.post_norm_w, self.cfg.norm_eps, residual)) \
+            if fused else None
+        if found is not None:
+            return layer.down.forward(found[0]), found[1]
         normed, residual = ops.rmsnorm(o, layer.post_norm_w,
                                        self.cfg.norm_eps, residual)
         fused = getattr(layer.gate_up, "forward_swiglu", None)
@@ -460,6 +471,10 @@ class LlamaForCausalLM(nn.Module):
                                                     self._lm8[1])
                     except ValueError:
                         pass
+        found = ops.linear_normed(
+            h, self.lm_head, (self.final_norm_w, self.cfg.norm_eps, residual))
+        if found is not None:
+            return found[0]
         normed, _ = ops.rmsnorm(h, self.final_norm_w, self.cfg.norm_eps,
                                 residual)
         if normed.dim() == 2:

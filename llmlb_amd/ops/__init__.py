@@ -182,14 +182,41 @@ def rope_kv_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _check(rc, "ll_rope_kv_append")
 
 
+def norms_rows(x: torch.Tensor) -> bool:
+    """Whether a product may norm rows of this shape itself
+    (linear_normed)."""
+    return x.dim() == 2 and x.shape[0] <= 4 and x.numel() <= 4096
+
+
+def _norm_operands(x: torch.Tensor, norm: tuple):
+    """(arguments, x + residual or None) of a product that norms its rows by
+    ``norm`` (weight, eps, residual or None); None where it does not."""
+    weight, eps, residual = norm
+    K = x.shape[1]
+    if (not norms_rows(x) or K % 64 or not x.is_contiguous() or weight.shape != (K,)
+            or weight.dtype != x.dtype or weight.device != x.device
+            or not weight.is_contiguous() or not _only_numbers(weight)):
+        return None
+    if residual is None:
+        return (None, None, _ptr(weight), ctypes.c_float(eps)), None
+    if (residual.shape != x.shape or residual.dtype != x.dtype
+            or residual.device != x.device or not residual.is_contiguous()
+            or not _only_numbers(residual)):
+        return None
+    total = torch.empty_like(residual)
+    return (_ptr(residual), _ptr(total), _ptr(weight),
+            ctypes.c_float(eps)), total
+
+
 def linear_rotary(x: torch.Tensor, weight: torch.Tensor, n_q: int,
                   n_kv: int, head_dim: int, cos_sin: torch.Tensor,
-                  positions: torch.Tensor, kv_sink: tuple | None = None
-                  ) -> torch.Tensor | None:
+                  positions: torch.Tensor, kv_sink: tuple | None = None,
+                  norm: tuple | None = None):
     """Queries, keys and values x @ W^T of up to 128 bf16 rows, in one launch
     with what ``rope_apply`` or, with ``kv_sink`` (kcache, vcache, slots),
-    ``rope_kv_append`` do to them.  None where row_gemm.hip does not take the
-    operands."""
+    ``rope_kv_append`` do to them.  ``norm`` (weight, eps, residual): of the
+    rows' norm, and the result is (q, k and v, x + residual).  None where
+    row_gemm.hip does not take the operands."""
     N, M = x.shape[0], (n_q + 2 * n_kv) * head_dim
     if (_USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight)
             or weight.dtype != x.dtype or weight.shape[0] != M
@@ -213,17 +240,50 @@ def linear_rotary(x: torch.Tensor, weight: torch.Tensor, n_q: int,
         slots = slots.to(torch.int32).contiguous()
         caches, page = (_ptr(kcache), _ptr(vcache), _ptr(slots)), \
             kcache.shape[2]
+    total, normed = None, (None, None, None, ctypes.c_float(0.0))
+    if norm is not None:
+        found = _norm_operands(x, norm)
+        if found is None:
+            return None
+        normed, total = found
     pos = positions.to(torch.int32).contiguous()
     out = torch.empty(N, M, device=x.device, dtype=x.dtype)
     rc = _lib.ll_row_gemm_rotary(
         _ptr(out), _ptr(x), _ptr(weight), _ptr(cos_sin), _ptr(pos), *caches,
-        ctypes.c_int(N), ctypes.c_int(n_q), ctypes.c_int(n_kv),
+        *normed, ctypes.c_int(N), ctypes.c_int(n_q), ctypes.c_int(n_kv),
         ctypes.c_int(head_dim), ctypes.c_int(x.shape[1]),
         ctypes.c_int(x.stride(0)), ctypes.c_int(page), _stream())
     if rc == -2:
         return None
     _check(rc, "ll_row_gemm_rotary")
-    return out
+    return out if norm is None else (out, total)
+
+
+def linear_normed(x: torch.Tensor, weight: torch.Tensor, norm: tuple,
+                  act: str = "plain", up: int = 0):
+    """(act(norm(x) @ W^T), x + residual) of a few bf16 rows in one launch,
+    ``norm`` as for linear_rotary, act "plain" or "swiglu" (as for
+    linear_act); None where row_gemm.hip does not take it."""
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or act not in ("plain", "swiglu")
+            or not norms_rows(x) or not _takes_row_gemm(x, weight)):
+        return None
+    found = _norm_operands(x, norm)
+    if found is None:
+        return None
+    normed, total = found
+    found = _product_of(x, weight, act, None, up)
+    if found is None:
+        return None
+    M, out = found
+    rc = _lib.ll_row_gemm_normed(
+        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x), _ptr(weight),
+        *normed, ctypes.c_int(x.shape[0]), ctypes.c_int(M),
+        ctypes.c_int(x.shape[1]), ctypes.c_int(x.stride(0)),
+        ctypes.c_int(_ROW_ACTS[act]), ctypes.c_int(up), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "ll_row_gemm_normed")
+    return out, total
 
 
 def swiglu(gateup: torch.Tensor) -> torch.Tensor:

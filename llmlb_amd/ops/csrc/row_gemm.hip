@@ -17,6 +17,7 @@
 //       60.9 -> 37.0 (6.3 TB/s)
 // With more rows the bound is what a compute unit takes in, about 50 GB/s:
 // every tile reads all of its x and W.
+#include "hybrid/norm_tile.h"
 #include "hybrid/row_act.h"
 #include "hybrid/row_tile.h"
 
@@ -198,6 +199,46 @@ void row_gemm_kernel(
   }
 }
 
+// The same of a few normed rows: out = norm(x) W^T
+template <int MT, int KW, int S, class End>
+__global__ __launch_bounds__(KW * 64, 2) void row_gemm_normed_kernel(
+    void* __restrict__ out, int ld_out, const bf16_t* __restrict__ x,
+    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, RowNorm norm,
+    End end) {
+  using Tile = NormTile<MT, KW, S>;
+  constexpr int OUT = End::PAIRED ? 8 * MT : 16 * MT;
+  constexpr int ITEMS = 16 * (OUT / 4);
+  extern __shared__ __align__(1024) char lds[];
+  const int tile = blockIdx.x, m0 = tile * OUT;
+  auto here = [&](int i, int& n, int& m) {
+    n = i / (OUT / 4), m = m0 + i % (OUT / 4) * 4;
+    return i < ITEMS && n < N && m < M;
+  };
+  int n, m;
+  typename End::Token token{};
+  typename End::Early early{};
+  const bool some = here(threadIdx.x, n, m);
+  if (some) token = end.token(n);
+  Tile::run(
+      lds, N, K, tile >> 3, x, ldx, norm, tile == 0,
+      [&](int r) {
+        const bool other = End::PAIRED && r >= OUT;
+        int m = m0 + (other ? r - OUT : r);
+        m = m < M ? m : M - 1;
+        return w + (size_t)(other ? end.second(m) : end.first(m)) * K;
+      },
+      [&] {
+        if (some) early = end.early(token, m);
+      });
+  for (int i = threadIdx.x; i < ITEMS; i += KW * 64) {
+    if (!here(i, n, m)) continue;
+    if (i != (int)threadIdx.x) early = end.early(end.token(n), m);
+    const f32x4 v = Tile::sum(lds, n, m - m0);
+    const f32x4 u = End::PAIRED ? Tile::sum(lds, n, m - m0 + OUT) : v;
+    end.put(out, ld_out, n, m, early, v, u);
+  }
+}
+
 // A share of the depth, ``depth`` numbers from blockIdx.y * depth on, into
 // ws [shares][N][M] floats.
 template <int NT, int MT, int KW, int S>
@@ -264,6 +305,24 @@ struct RowGemm {
   hipStream_t stream;
 };
 
+template <int MT, int KW, int S, class End>
+static int row_gemm_normed_launch(const RowGemm<End>& p, const RowNorm& norm) {
+  auto* kernel = &row_gemm_normed_kernel<MT, KW, S, End>;
+  using Tile = NormTile<MT, KW, S>;
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  const int lds = Tile::lds(p.N, p.K);
+  if (sized != hipSuccess) return -1;
+  if (p.K > Tile::DEEPEST || lds > 160 * 1024) return -2;
+  constexpr int OUT = End::PAIRED ? 8 * MT : 16 * MT;
+  hipLaunchKernelGGL(kernel, dim3((p.M + OUT - 1) / OUT), dim3(KW * 64), lds,
+                     p.stream, p.out, p.ld_out, p.x, p.w, p.N, p.M, p.K,
+                     p.ldx, norm, p.end);
+  HY_CHECK();
+  return 0;
+}
+
 template <int NT, int MT, int KW, int S, class End>
 static int row_gemm_launch(const RowGemm<End>& p) {
   auto* kernel = &row_gemm_kernel<NT, MT, KW, S, End>;
@@ -300,10 +359,8 @@ static int row_gemm_launch(const RowGemm<End>& p) {
 // than whole rounds say: another than 32 outputs has to take in 15% less (one
 // row of 20480 x 1024 11.0 with 48, 10.1 with 32; 16512 x 1024 9.2 with 32, 8.6
 // with 80).
-template <class End>
-static int row_gemm_pick(const RowGemm<End>& p) {
-  const int tiles = (p.N + 15) / 16;
-  const long long rows = End::PAIRED ? 2ll * p.M : p.M;
+static int row_gemm_tile(int N, long long rows, int K, bool paired) {
+  const int tiles = (N + 15) / 16;
   // what memory takes for W, in the same unit: 16 rows at 50 GB/s
   const float floor = rows / 2500.f;
   int nt = 0, mt = 0;
@@ -328,12 +385,18 @@ static int row_gemm_pick(const RowGemm<End>& p) {
       // (3, 1) and (4, 1) take in no less; of gate and up, tiles of 8 outputs
       // by eight waves are for what they share (1024 x 128, one row: 3.0 with
       // them, 2.8 with 16; 1024 x 768 3.4, 3.7)
-      if ((n < 3 || m > 1) && (!End::PAIRED || m > 1 || p.K > 256)) look(n, m);
+      if ((n < 3 || m > 1) && (!paired || m > 1 || K > 256)) look(n, m);
     }
+  return nt * 8 + mt;
+}
+
+template <class End>
+static int row_gemm_pick(const RowGemm<End>& p) {
+  const long long rows = End::PAIRED ? 2ll * p.M : p.M;
   // waves that share the depth, and pieces of it on their way, fit LDS
 #define TILE(NT, MT, KW, S) \
   case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S>(p);
-  switch (nt * 8 + mt) {
+  switch (row_gemm_tile(p.N, rows, p.K, End::PAIRED)) {
     TILE(1, 1, 8, 2)
     TILE(1, 2, 4, 3)
     TILE(1, 3, 4, 3)
@@ -360,6 +423,20 @@ static int row_gemm_pick(const RowGemm<End>& p) {
     TILE(4, 7, 3, 2)
   }
 #undef TILE
+  return -2;
+}
+
+// Of a few normed rows, see norm_gains.
+template <class End>
+static int row_gemm_normed(const RowGemm<End>& p, const RowNorm& norm) {
+  const long long rows = End::PAIRED ? 2ll * p.M : p.M;
+  switch (row_gemm_tile(p.N, rows, p.K, End::PAIRED)) {
+    case 9: return row_gemm_normed_launch<1, 8, 2>(p, norm);
+    case 10: return row_gemm_normed_launch<2, 4, 3>(p, norm);
+    case 11: return row_gemm_normed_launch<3, 4, 3>(p, norm);
+    case 12: return row_gemm_normed_launch<4, 4, 3>(p, norm);
+    case 13: return row_gemm_normed_launch<5, 4, 3>(p, norm);
+  }
   return -2;
 }
 
@@ -455,15 +532,63 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
       PlainEnd{act}, (hipStream_t)stream});
 }
 
+// Whether a product norms its rows itself: every workgroup does all of them, so
+// few, and of more than one not where workgroups come in rounds.  us, both
+// launches -> this:
+//   1 row: 1536 x 1024 5.5 -> 4.9, gate and up of 5632 x 1024 6.9 -> 5.8, 32000 x
+//       1024 14.6 -> 13.9, 3072 x 2048 7.0 -> 6.6, gate and up of 11264 x 2048
+//       11.7 -> 11.2, 6144 x 4096 13.0 -> 13.7
+//   2 rows: 5.8 -> 4.9, 7.0 -> 6.2, 14.4 -> 14.7, 6.9 -> 7.3, 11.8 -> 11.6
+//   4 rows: 5.8 -> 5.3, 7.1 -> 6.5, 14.6 -> 15.2; 6: 6.0 -> 5.8, 7.3 -> 7.8
+static bool norm_gains(int N, int rows, int K) {
+  return (N == 1 && K <= 2048) ||
+         (N <= 4 && K <= 1024 && rows <= 512 * 32);
+}
+
+static bool norm_fits(const void* x, const void* residual, const void* sum,
+                      const void* weight, int N, int rows, int K) {
+  return norm_gains(N, rows, K) && K % 64 == 0 && weight &&
+         (uintptr_t)weight % 16 == 0 && (uintptr_t)residual % 16 == 0 &&
+         (uintptr_t)sum % 16 == 0 && !residual == !sum &&
+         (!sum || (sum != residual && sum != x));
+}
+
+// out = act(norm(x) W^T), of x + residual where there is one, which is left in
+// ``sum`` (dense rows both).
+extern "C" int ll_row_gemm_normed(void* out, int ld_out, const void* x,
+                                  const void* w, const void* residual,
+                                  void* sum, const void* norm_weight,
+                                  float eps, int N, int M, int K, int ldx,
+                                  int kind, int up, void* stream) {
+  if (N <= 0 || M <= 0 || K <= 0 || M % 4 || ldx % 8 || ld_out % 4 ||
+      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 8 ||
+      (kind != PLAIN && kind != SWIGLU) ||
+      !norm_fits(x, residual, sum, norm_weight, N,
+                 kind == SWIGLU ? 2 * M : M, K))
+    return -2;
+  const RowNorm norm{(const bf16_t*)residual, (bf16_t*)sum,
+                     (const bf16_t*)norm_weight, eps};
+  const RowAct act{kind, up, 0.f, 0.f};
+  if (kind == SWIGLU)
+    return row_gemm_normed(
+        RowGemm<GatedEnd>{out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N,
+                          M, K, ldx, GatedEnd{act}, (hipStream_t)stream},
+        norm);
+  return row_gemm_normed(
+      RowGemm<PlainEnd>{out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M,
+                        K, ldx, PlainEnd{act}, (hipStream_t)stream},
+      norm);
+}
+
 // Queries, keys and values of N rows, rotated, and with caches appended: see
 // RotaryEnd.  W holds n_q + 2 n_kv heads of D rows, D a power of two, in that
-// order; caches are [page][head][page slot][D].
-extern "C" int ll_row_gemm_rotary(void* out, const void* x, const void* w,
-                                  const void* cos_sin, const void* positions,
-                                  void* kcache, void* vcache,
-                                  const void* slots, int N, int n_q, int n_kv,
-                                  int D, int K, int ldx, int page,
-                                  void* stream) {
+// order; caches are [page][head][page slot][D].  With norm_weight of normed
+// rows, as above.
+extern "C" int ll_row_gemm_rotary(
+    void* out, const void* x, const void* w, const void* cos_sin,
+    const void* positions, void* kcache, void* vcache, const void* slots,
+    const void* residual, void* sum, const void* norm_weight, float eps, int N,
+    int n_q, int n_kv, int D, int K, int ldx, int page, void* stream) {
   if (N <= 0 || N > 128 || n_q <= 0 || n_kv <= 0 || D < 8 || (D & (D - 1)) ||
       n_q > 1 << 16 || n_kv > 1 << 16 || D > 1 << 10 || K <= 0 || K % 8 ||
       ldx % 8 || page <= 0 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
@@ -472,13 +597,19 @@ extern "C" int ll_row_gemm_rotary(void* out, const void* x, const void* w,
       !positions || !kcache != !vcache || (kcache && !slots))
     return -2;
   const int M = (n_q + 2 * n_kv) * D;
-  if (read_twice(N, M, K) || ll_row_gemm_shares(N, M, K) > 1) return -2;
-  return row_gemm_pick(RowGemm<RotaryEnd>{
+  const RowGemm<RotaryEnd> p{
       out, M, (const bf16_t*)x, (const bf16_t*)w, N, M / 2, K, ldx,
       RotaryEnd{(const float*)cos_sin, (const int*)positions,
                 (const int*)slots, (bf16_t*)kcache, (bf16_t*)vcache,
                 __builtin_ctz(D) - 1, n_q, n_kv, page},
-      (hipStream_t)stream});
+      (hipStream_t)stream};
+  if (norm_weight) {
+    if (!norm_fits(x, residual, sum, norm_weight, N, M, K)) return -2;
+    return row_gemm_normed(p, RowNorm{(const bf16_t*)residual, (bf16_t*)sum,
+                                      (const bf16_t*)norm_weight, eps});
+  }
+  if (read_twice(N, M, K) || ll_row_gemm_shares(N, M, K) > 1) return -2;
+  return row_gemm_pick(p);
 }
 
 // The same for H pairs of rows and matrices at once, as latent attention needs

@@ -181,14 +181,25 @@ class ColumnParallelLinear(nn.Module, _Fp8WeightMixin):
                     or getattr(self.forward, "__func__", None)
                     is not ColumnParallelLinear.forward)
 
-    def forward_rotary(self, x: torch.Tensor, *args) -> torch.Tensor | None:
-        """The shard's queries, keys and values with what follows in the
-        product's own launch (``ops.linear_rotary``), or None where that would
-        be something else, or more than 128 rows."""
+    def forward_rotary(self, x: torch.Tensor, *args, norm=None):
+        """The shard's queries, keys and values with what follows, and for a
+        few rows what comes before, in the product's own launch
+        (``ops.linear_rotary``), or None where that would be something else,
+        or more than 128 rows."""
         from .. import ops as _ops
         if x.dim() != 2 or x.shape[0] > 128 or not self._only_product():
             return None
-        return _ops.linear_rotary(x, self.weight, *args)
+        return _ops.linear_rotary(x, self.weight, *args, norm=norm)
+
+    def forward_normed_swiglu(self, x: torch.Tensor, norm: tuple):
+        """``forward_swiglu`` of a few rows' norm in the same launch
+        (``ops.linear_normed``), or None."""
+        from .. import ops as _ops
+        if (not _ops.norms_rows(x) or _ops._FUSED_SWIGLU
+                or not self._only_product()):
+            return None
+        return _ops.linear_normed(x, self.weight, norm, "swiglu",
+                                  self.out_local // 2)
 
     def forward_swiglu(self, x: torch.Tensor) -> torch.Tensor | None:
         """swiglu of the shard's [gate | up] outputs in the product's own
