@@ -8,6 +8,7 @@ one matrix product.
 parallel layers have ``inner`` instead: it writes what the output
 projection reads (``out_width`` columns of a wider row), so that the
 layer applies the projections of mixer and feed-forward as one product.
+``proj``: the mixer's input projection, where the layer has made it.
 Where both also read the same norm, ``inputs`` names the weights of a
 module's input projections, and the layer stacks them into one product,
 whose sections start at the columns given to ``place``.
@@ -22,7 +23,8 @@ import torch.nn.functional as F
 
 from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
-from ..ops import linear_act, linear_decode, linear_heads, linear_rows
+from ..ops import (linear_act, linear_decode, linear_heads, linear_rows,
+                   linear_two)
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
@@ -337,8 +339,9 @@ class DifferentialAttention(nn.Module):
     def cache_spec(self):
         return PageSpec(self.kv_heads * (2 * self.dim + self.vdim))
 
-    def inner(self, x, b, cache, index: int, out) -> None:
-        proj = _linear(x, self.w_in)
+    def inner(self, x, b, cache, index: int, out, proj=None) -> None:
+        if proj is None:
+            proj = _linear(x, self.w_in)
         pages = cache.pages[index]
         hy.pair_append(proj, self.k_off, self.v_off, self.kv_heads,
                        self.dim, self.vdim, b, pages)
@@ -381,8 +384,9 @@ class GatedLinearAttention(nn.Module):
     def cache_spec(self):
         return StateSpec(self.heads, self.vdim, self.dim, 0, 0)
 
-    def inner(self, x, b, cache, index: int, out) -> None:
-        proj = _linear(x, self.w_in)
+    def inner(self, x, b, cache, index: int, out, proj=None) -> None:
+        if proj is None:
+            proj = _linear(x, self.w_in)
         dec = _linear(proj[:, self.a_off:self.a_off + self.decay_rank],
                       self.w_a2)
         hy.gated_linear(out, proj, self.k_off, self.v_off, self.g_off, dec,
@@ -436,8 +440,9 @@ class StateSpaceDuality(nn.Module):
         return StateSpec(self.heads, self.vdim, self.state, self.channels,
                          self.taps)
 
-    def inner(self, x, b, cache, index: int, out) -> None:
-        proj = _linear(x, self.w_in)
+    def inner(self, x, b, cache, index: int, out, proj=None) -> None:
+        if proj is None:
+            proj = _linear(x, self.w_in)
         hy.state_space(out, proj, self.z_off, self.dt_off,
                        cache.state[index], cache.ring[index], b, self.w_conv,
                        self.b_conv, self.per_head, self.w_norm, self.groups,
@@ -463,6 +468,14 @@ class ClampedSwiGLU(nn.Module):
     def load(self, w: dict[str, torch.Tensor]) -> None:
         stacked, (_, self.u_off) = _stack_rows([w["gate"], w["up"]])
         self.w_in = _param(stacked.to(dtype=self.dtype, device=self.device))
+
+    def inner_beside(self, x, out, x_mix, w_mix):
+        """``inner`` in one launch with the product of ``x_mix`` and
+        ``w_mix``, which it returns; None: neither is done."""
+        if x.shape[0] > 128:
+            return None
+        return linear_two(x_mix, w_mix, x, self.w_in, "clamped", out,
+                          self.u_off, self.limit, self.sharpness)
 
     def inner(self, x, out) -> None:
         if linear_act(x, self.w_in, "clamped", out, self.u_off, self.limit,

@@ -160,8 +160,10 @@ class TaletarLayer(nn.Module):
         n = self.mix.out_width
         mid = torch.empty(h1.shape[0], self.w_out.shape[1], dtype=h1.dtype,
                           device=h1.device)
-        self.mix.inner(h1, b, cache, index, mid[:, :n])
-        if self.ff is not None:
+        proj = None if self.ff is None else self.ff.inner_beside(
+            h2, mid[:, n:], h1, self.mix.w_in)
+        self.mix.inner(h1, b, cache, index, mid[:, :n], proj)
+        if self.ff is not None and proj is None:
             self.ff.inner(h2, mid[:, n:])
         return _linear(mid, self.w_out)
 

@@ -961,6 +961,36 @@ def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
     return product(x, weight, act, out, up, a, b)
 
 
+def linear_two(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor,
+               weight2: torch.Tensor, act: str, out2: torch.Tensor, up: int,
+               a: float = 0.0, b: float = 0.0) -> torch.Tensor | None:
+    """x @ W^T, and into ``out2`` linear_act(x2, W2, act), of up to 128 bf16
+    rows in one launch; act "swiglu" or "clamped".  None where row_gemm.hip does
+    not take all of it."""
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or act not in ("swiglu", "clamped")
+            or not _takes_row_gemm(x, weight)
+            or not _takes_row_gemm(x2, weight2) or x.shape != x2.shape
+            or x.device != x2.device):
+        return None
+    second = _product_of(x2, weight2, act, out2, up)
+    first = None if second is None else _product_of(x, weight, "plain", None,
+                                                    0)
+    if first is None:
+        return None
+    (M, out), M2 = first, second[0]
+    rc = _lib.ll_row_gemm_two(
+        _ptr(out), ctypes.c_int(out.stride(0)), _ptr(x),
+        ctypes.c_int(x.stride(0)), _ptr(weight), ctypes.c_int(M), _ptr(out2),
+        ctypes.c_int(out2.stride(0)), _ptr(x2), ctypes.c_int(x2.stride(0)),
+        _ptr(weight2), ctypes.c_int(M2), ctypes.c_int(_ROW_ACTS[act]),
+        ctypes.c_int(up), ctypes.c_float(a), ctypes.c_float(b),
+        ctypes.c_int(x.shape[0]), ctypes.c_int(x.shape[1]), _stream())
+    if rc == -2:
+        return None
+    _check(rc, "ll_row_gemm_two")
+    return out
+
+
 def linear_decode(x: torch.Tensor, weight: torch.Tensor,
                   w8: tuple | None = None) -> torch.Tensor:
     """out = x @ W^T for up to 128 rows.

@@ -150,20 +150,19 @@ struct RotaryEnd {
 
 // The order in which a sum is made differs with the number of rows, as with
 // any product: tiles, waves and shares follow from it.  M outputs, of PAIRED
-// ends pairs.
+// ends pairs; block: of the product's workgroups.
 template <int NT, int MT, int KW, int S, class End>
-__global__ __launch_bounds__(KW * 64, NT * MT > 24 ? 1 : 2)
-void row_gemm_kernel(
-    void* __restrict__ out, int ld_out, const bf16_t* __restrict__ x,
-    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, End end) {
+__device__ __forceinline__ void row_gemm_block(
+    char* lds, int block, void* __restrict__ out, int ld_out,
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int N, int M,
+    int K, int ldx, const End& end) {
   using Tile = RowTile<NT, MT, KW, S>;
   constexpr int OUT = End::PAIRED ? 8 * MT : 16 * MT;  // outputs a tile
   constexpr int ITEMS = 16 * NT * (OUT / 4);
-  extern __shared__ __align__(1024) char lds[];
   // tiles of the same rows of W are 8 apart: on one XCD
   const int across = (N + 16 * NT - 1) / (16 * NT);
-  const int in = blockIdx.x % (8 * across);
-  const int tile = blockIdx.x / (8 * across) * 8 + in % 8;
+  const int in = block % (8 * across);
+  const int tile = block / (8 * across) * 8 + in % 8;
   const int m0 = tile * OUT, n0 = in / 8 * 16 * NT;
   if (m0 >= M) return;
   auto here = [&](int i, int& n, int& m) {
@@ -197,6 +196,37 @@ void row_gemm_kernel(
     const f32x4 u = End::PAIRED ? Tile::sum(lds, n - n0, m - m0 + OUT) : v;
     end.put(out, ld_out, n, m, early, v, u);
   }
+}
+
+template <int NT, int MT, int KW, int S, class End>
+__global__ __launch_bounds__(KW * 64, NT * MT > 24 ? 1 : 2)
+void row_gemm_kernel(
+    void* __restrict__ out, int ld_out, const bf16_t* __restrict__ x,
+    const bf16_t* __restrict__ w, int N, int M, int K, int ldx, End end) {
+  extern __shared__ __align__(1024) char lds[];
+  row_gemm_block<NT, MT, KW, S>(lds, blockIdx.x, out, ld_out, x, w, N, M, K,
+                                ldx, end);
+}
+
+// Two products of equally many rows and equal depth, of which neither needs
+// the other: the first ``blocks`` workgroups do one, the others the other.
+// A launch less, and one beginning, last round and end for both.
+struct RowOperands {
+  void* out;
+  const bf16_t *x, *w;
+  int ld_out, M, ldx;
+};
+template <int NT, int MT, int KW, int S>
+__global__ __launch_bounds__(KW * 64, NT * MT > 24 ? 1 : 2)
+void row_gemm_two_kernel(RowOperands a, PlainEnd a_end, RowOperands b,
+                         GatedEnd b_end, int blocks, int N, int K) {
+  extern __shared__ __align__(1024) char lds[];
+  if ((int)blockIdx.x < blocks)
+    row_gemm_block<NT, MT, KW, S>(lds, blockIdx.x, a.out, a.ld_out, a.x, a.w,
+                                  N, a.M, K, a.ldx, a_end);
+  else
+    row_gemm_block<NT, MT, KW, S>(lds, blockIdx.x - blocks, b.out, b.ld_out,
+                                  b.x, b.w, N, b.M, K, b.ldx, b_end);
 }
 
 // The same of a few normed rows: out = norm(x) W^T
@@ -359,16 +389,19 @@ static int row_gemm_launch(const RowGemm<End>& p) {
 // than whole rounds say: another than 32 outputs has to take in 15% less (one
 // row of 20480 x 1024 11.0 with 48, 10.1 with 32; 16512 x 1024 9.2 with 32, 8.6
 // with 80).
-static int row_gemm_tile(int N, long long rows, int K, bool paired) {
+static int row_gemm_tile(int N, long long rows, int K, bool paired,
+                         long long beside = 0) {
   const int tiles = (N + 15) / 16;
   // what memory takes for W, in the same unit: 16 rows at 50 GB/s
-  const float floor = rows / 2500.f;
+  const float floor = (rows + beside) / 2500.f;
   int nt = 0, mt = 0;
   float least = 0.f;
   auto look = [&](int n, int m) {
     // tiles of the same rows of W are on one of eight XCDs of 32 units
     const long long down = (rows + 16 * m - 1) / (16 * m);
-    const long long count = (down + 7) / 8 * ((tiles + n - 1) / n);
+    const long long other = (beside + 16 * m - 1) / (16 * m);
+    const long long count =
+        ((down + 7) / 8 + (other + 7) / 8) * ((tiles + n - 1) / n);
     const long long rounds = (count + 31) / 32;
     if (m == 7 && rounds > 2) return;  // memory bounds these, of any tile
     const float takes = fmaxf((float)(rounds * (n + m)), floor);
@@ -390,40 +423,74 @@ static int row_gemm_tile(int N, long long rows, int K, bool paired) {
   return nt * 8 + mt;
 }
 
+// all tiles: waves that share the depth, and pieces of it on their way, fit LDS
+#define ROW_GEMM_TILES(GO) \
+  GO(1, 1, 8, 2)           \
+  GO(1, 2, 4, 3)           \
+  GO(1, 3, 4, 3)           \
+  GO(1, 4, 4, 3)           \
+  GO(1, 5, 4, 3)           \
+  GO(2, 1, 4, 3)           \
+  GO(2, 2, 4, 2)           \
+  GO(2, 3, 4, 2)           \
+  GO(2, 4, 4, 2)           \
+  GO(2, 5, 4, 2)           \
+  GO(2, 6, 4, 2)           \
+  GO(2, 7, 4, 2)           \
+  GO(3, 2, 4, 2)           \
+  GO(3, 3, 4, 2)           \
+  GO(3, 4, 4, 2)           \
+  GO(3, 5, 4, 2)           \
+  GO(3, 6, 4, 2)           \
+  GO(3, 7, 4, 2)           \
+  GO(4, 2, 4, 2)           \
+  GO(4, 3, 4, 2)           \
+  GO(4, 4, 4, 2)           \
+  GO(4, 5, 4, 2)           \
+  GO(4, 6, 4, 2)           \
+  GO(4, 7, 3, 2)
+
 template <class End>
 static int row_gemm_pick(const RowGemm<End>& p) {
   const long long rows = End::PAIRED ? 2ll * p.M : p.M;
-  // waves that share the depth, and pieces of it on their way, fit LDS
-#define TILE(NT, MT, KW, S) \
-  case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S>(p);
   switch (row_gemm_tile(p.N, rows, p.K, End::PAIRED)) {
-    TILE(1, 1, 8, 2)
-    TILE(1, 2, 4, 3)
-    TILE(1, 3, 4, 3)
-    TILE(1, 4, 4, 3)
-    TILE(1, 5, 4, 3)
-    TILE(2, 1, 4, 3)
-    TILE(2, 2, 4, 2)
-    TILE(2, 3, 4, 2)
-    TILE(2, 4, 4, 2)
-    TILE(2, 5, 4, 2)
-    TILE(2, 6, 4, 2)
-    TILE(2, 7, 4, 2)
-    TILE(3, 2, 4, 2)
-    TILE(3, 3, 4, 2)
-    TILE(3, 4, 4, 2)
-    TILE(3, 5, 4, 2)
-    TILE(3, 6, 4, 2)
-    TILE(3, 7, 4, 2)
-    TILE(4, 2, 4, 2)
-    TILE(4, 3, 4, 2)
-    TILE(4, 4, 4, 2)
-    TILE(4, 5, 4, 2)
-    TILE(4, 6, 4, 2)
-    TILE(4, 7, 3, 2)
+#define GO(NT, MT, KW, S) \
+  case NT * 8 + MT: return row_gemm_launch<NT, MT, KW, S>(p);
+    ROW_GEMM_TILES(GO)
+#undef GO
   }
-#undef TILE
   return -2;
+}
+
+// The tile is chosen for the tiles of both.  us, a layer's input projection and
+// its gate and up, one after the other -> together (rows: outputs, pairs, depth):
+//   1: 4160, 2176 of 1024 9.0 -> 6.3, 8320, 4352 of 2048 15.8 -> 13.1, 16512,
+//       11904 of 4096 52.4 -> 48.1; 64: 12.0 -> 8.2, 24.1 -> 17.2, 61.6 -> 60.2;
+//       128: 14.5 -> 10.1, 29.5 -> 27.9, 103.4 -> 99.4
+struct RowGemmTwo {
+  RowOperands a, b;
+  PlainEnd a_end;
+  GatedEnd b_end;
+  int N, K;
+  hipStream_t stream;
+};
+template <int NT, int MT, int KW, int S>
+static int row_gemm_two_launch(const RowGemmTwo& p) {
+  auto* kernel = &row_gemm_two_kernel<NT, MT, KW, S>;
+  constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const int across = (p.N + 16 * NT - 1) / (16 * NT);
+  auto blocks = [&](int M, int out) {
+    return ((M + out - 1) / out + 7) / 8 * 8 * across;
+  };
+  const int first = blocks(p.a.M, 16 * MT), second = blocks(p.b.M, 8 * MT);
+  hipLaunchKernelGGL(kernel, dim3(first + second), dim3(KW * 64), lds,
+                     p.stream, p.a, p.a_end, p.b, p.b_end, first, p.N, p.K);
+  HY_CHECK();
+  return 0;
 }
 
 // Of a few normed rows, see norm_gains.
@@ -530,6 +597,43 @@ extern "C" int ll_row_gemm(void* out, int ld_out, const void* x,
   return row_gemm_pick(RowGemm<PlainEnd>{
       out, ld_out, (const bf16_t*)x, (const bf16_t*)w, N, M, K, ldx,
       PlainEnd{act}, (hipStream_t)stream});
+}
+
+// out1 = x1 W1^T and out2 = gated(x2 W2^T) of N rows, both K deep, as
+// ll_row_gemm makes them (kind: SWIGLU or CLAMPED).  0: done, -2: not for this
+// kernel.
+extern "C" int ll_row_gemm_two(void* out1, int ld_out1, const void* x1,
+                               int ldx1, const void* w1, int M1, void* out2,
+                               int ld_out2, const void* x2, int ldx2,
+                               const void* w2, int M2, int kind, int up,
+                               float a, float b, int N, int K, void* stream) {
+  auto fits = [&](const void* out, int ld_out, const void* x, int ldx,
+                  const void* w, int M, int rows) {
+    return M > 0 && M % 4 == 0 && ldx % 8 == 0 && ld_out % 4 == 0 &&
+           (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
+           (uintptr_t)out % 8 == 0 && !read_twice(N, rows, K);
+  };
+  if (N <= 0 || N > 128 || K <= 0 || K % 8 ||
+      (kind != SWIGLU && kind != CLAMPED) ||
+      !fits(out1, ld_out1, x1, ldx1, w1, M1, M1) ||
+      !fits(out2, ld_out2, x2, ldx2, w2, M2, 2 * M2) ||
+      ll_row_gemm_shares(N, M1, K) > 1)
+    return -2;
+  const RowGemmTwo p{
+      {out1, (const bf16_t*)x1, (const bf16_t*)w1, ld_out1, M1, ldx1},
+      {out2, (const bf16_t*)x2, (const bf16_t*)w2, ld_out2, M2, ldx2},
+      PlainEnd{RowAct{PLAIN, 0, 0.f, 0.f}},
+      GatedEnd{RowAct{kind, up, a, b}},
+      N,
+      K,
+      (hipStream_t)stream};
+  switch (row_gemm_tile(N, M1, K, true, 2ll * M2)) {
+#define GO(NT, MT, KW, S) \
+  case NT * 8 + MT: return row_gemm_two_launch<NT, MT, KW, S>(p);
+    ROW_GEMM_TILES(GO)
+#undef GO
+  }
+  return -2;
 }
 
 // Whether a product norms its rows itself: every workgroup does all of them, so
