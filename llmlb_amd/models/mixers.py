@@ -387,11 +387,15 @@ class GatedLinearAttention(nn.Module):
     def inner(self, x, b, cache, index: int, out, proj=None) -> None:
         if proj is None:
             proj = _linear(x, self.w_in)
-        dec = _linear(proj[:, self.a_off:self.a_off + self.decay_rank],
-                      self.w_a2)
+        dec = None
+        if not hy.decays_in_step(proj, self.a_off, self.w_a2, self.dim,
+                                 b):
+            dec = _linear(proj[:, self.a_off:self.a_off + self.decay_rank],
+                          self.w_a2)
         hy.gated_linear(out, proj, self.k_off, self.v_off, self.g_off, dec,
                         self.b_a2, cache.state[index], b, self.w_norm,
-                        self.heads, self.dim, self.vdim, self.tau, self.eps)
+                        self.heads, self.dim, self.vdim, self.tau, self.eps,
+                        (self.a_off, self.w_a2))
 
 
 class StateSpaceDuality(nn.Module):

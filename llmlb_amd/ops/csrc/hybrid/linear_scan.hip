@@ -21,7 +21,8 @@
 #include "memory.h"
 #include "recurrent.h"
 
-enum Kind { CHANNEL, HEAD, MEMORY };  // gated linear, Mamba-2, mLSTM
+// gated linear (LOW: a step with its decays' projection), Mamba-2, mLSTM
+enum Kind { CHANNEL, HEAD, MEMORY, LOW };
 
 // N consecutive elements as they lie in memory, widened on use, so that
 // elements in flight take half the registers and nothing waits for them.
@@ -416,6 +417,11 @@ __global__ __launch_bounds__(256) void ring_store_kernel(
 // sequence); the state's loads are issued first so that everything the
 // token needs is computed behind them.
 //   CHANNEL: gated linear attention, out = silu(gate) norm(o)
+//   LOW: the same, and w_low [H D][rank] times the ``rank`` numbers from
+//     ``low_off`` on of the token's row makes the decays' projection, four
+//     lanes a channel: for small heads that costs less than the gap to a
+//     launch of its own.  A kernel of its own because the mere branch made
+//     CHANNEL 0.6 us slower at 128 x 128.
 //   HEAD: Mamba-2, y = o + skip x (gate and norm span the heads)
 //   MEMORY: mLSTM, out = sigmoid(gate) norm(o); ``dec`` points to the
 //     input gates' projections (the forget gates' follow), per_head [2][H]
@@ -425,6 +431,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
     T* __restrict__ out, int ld_out, float* __restrict__ y,
     float* __restrict__ state, const T* __restrict__ proj, int ld, int q_off,
     int k_off, int v_off, int g_off, const T* __restrict__ dec,
+    const T* __restrict__ w_low, int low_off, int rank,
     const float* __restrict__ dec_bias, const float* __restrict__ w_norm,
     T* __restrict__ ring, const float* __restrict__ wconv,
     const float* __restrict__ conv_bias, const float* __restrict__ per_head,
@@ -504,14 +511,37 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
     for (int i = 0; i < RPL; ++i) N[i] = 0.f;
     if (pos > 0) load_spread<RPL, EXACT>(ex, l16, D, N);
   } else {
+    if constexpr (KIND == LOW) {
+      const int part = tid & 3;
+      for (int d = tid / 4; d < DP; d += 64) {
+        const T* w = w_low + ((size_t)h * D + (d < D ? d : 0)) * rank;
+        float sum = 0.f;
+#pragma unroll 2
+        for (int r = part * 8; r < rank; r += 32) {
+          float a[8], b[8];
+          load8(row + low_off + r, a);
+          load8(w + r, b);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sum += a[i] * b[i];
+        }
+        sum += __shfl_xor(sum, 1, WAVE);
+        sum += __shfl_xor(sum, 2, WAVE);
+        if (part == 0)
+          lg[d] = d < D ? decay_t<T>(-(to_f(from_f<T>(sum)) +
+                                       dec_bias[h * D + d]),
+                                     rate)
+                        : 0.f;
+      }
+    }
     for (int d = tid; d < DP; d += 256) {
       const bool ok = d < D;
       lq[d] = ok ? to_f(row[q_off + h * D + d]) * q_scale : 0.f;
       lk[d] = ok ? to_f(row[k_off + h * D + d]) : 0.f;
-      lg[d] = ok ? decay_t<T>(-(to_f(dec[((size_t)s * H + h) * D + d]) +
-                                dec_bias[h * D + d]),
-                              rate)
-                 : 0.f;
+      if constexpr (KIND == CHANNEL)
+        lg[d] = ok ? decay_t<T>(-(to_f(dec[((size_t)s * H + h) * D + d]) +
+                                  dec_bias[h * D + d]),
+                                rate)
+                   : 0.f;
     }
     for (int j = tid; j < V; j += 256) lv[j] = to_f(row[v_off + h * V + j]);
   }
@@ -522,7 +552,7 @@ __global__ __launch_bounds__(256) void linear_step_kernel(
     const int at = spread_at<RPL, EXACT>(l16, i);
     q[i] = lq[at];
     k[i] = lk[at] * dt;
-    g[i] = KIND == CHANNEL ? lg[at] : gh;
+    g[i] = KIND == CHANNEL || KIND == LOW ? lg[at] : gh;
   }
   if constexpr (KIND == MEMORY) {
     // every 16 lanes make the normaliser; what it was has been read
@@ -586,6 +616,7 @@ template <Kind KIND>
 static int launch_step(void* out, int ld_out, void* y, void* state,
                        const void* proj, int ld, int q_off, int k_off,
                        int v_off, int g_off, const void* dec,
+                       const void* w_low, int low_off, int rank,
                        const void* dec_bias, const void* w_norm, void* ring,
                        const void* wconv, const void* conv_bias,
                        const void* per_head, void* extra, const void* pos,
@@ -600,10 +631,11 @@ static int launch_step(void* out, int ld_out, void* y, void* state,
       (linear_step_kernel<T, RPL, EXACT, KIND>), grid, block, lds,
       (hipStream_t)stream, (T*)out, ld_out, (float*)y, (float*)state,
       (const T*)proj, ld, q_off, k_off, v_off, g_off, (const T*)dec,
-      (const float*)dec_bias, (const float*)w_norm, (T*)ring,
-      (const float*)wconv, (const float*)conv_bias, (const float*)per_head,
-      (float*)extra, (const int*)pos, (const int*)row, G, H, D, V, taps,
-      q_scale, rate, eps)));
+      (const T*)w_low, low_off, rank, (const float*)dec_bias,
+      (const float*)w_norm, (T*)ring, (const float*)wconv,
+      (const float*)conv_bias, (const float*)per_head, (float*)extra,
+      (const int*)pos, (const int*)row, G, H, D, V, taps, q_scale, rate,
+      eps)));
   HY_CHECK();
   return 0;
 }
@@ -695,15 +727,20 @@ int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
 
 int hy_gla_step(void* out, int ld_out, void* state, const void* proj, int ld,
                 int k_off, int v_off, int g_off, const void* dec,
+                const void* w_low, int low_off, int rank,
                 const void* dec_bias, const void* w_norm, const void* pos,
                 const void* row, int n_seq, int H, int D, int V,
                 float q_scale, float rate, float eps, int dtype,
                 void* stream) {
-  return launch_step<CHANNEL>(out, ld_out, nullptr, state, proj, ld, 0,
-                              k_off, v_off, g_off, dec, dec_bias, w_norm,
-                              nullptr, nullptr, nullptr, nullptr, nullptr,
-                              pos, row, n_seq, H, H, D, V, 1, q_scale, rate,
-                              eps, dtype, stream);
+  if (w_low ? rank <= 0 || rank % 8 || low_off % 8 || ld % 8 ||
+                  ((uintptr_t)w_low | (uintptr_t)proj) % 16
+            : !dec)
+    return -2;
+  return (w_low ? launch_step<LOW> : launch_step<CHANNEL>)(
+      out, ld_out, nullptr, state, proj, ld, 0, k_off, v_off, g_off, dec,
+      w_low, low_off, rank, dec_bias, w_norm, nullptr, nullptr, nullptr,
+      nullptr, nullptr, pos, row, n_seq, H, H, D, V, 1, q_scale, rate, eps,
+      dtype, stream);
 }
 
 int hy_memory_step(void* out, int ld_out, void* state, void* extra,
@@ -715,9 +752,9 @@ int hy_memory_step(void* out, int ld_out, void* state, void* extra,
   const size_t esize = dtype == 0 ? 2 : 4;
   return launch_step<MEMORY>(out, ld_out, nullptr, state, proj, ld, 0, k_off,
                              v_off, g_off, (const char*)proj + i_off * esize,
-                             nullptr, w_norm, nullptr, nullptr, nullptr, bias,
-                             extra, pos, row, n_seq, H, H, D, V, 1, q_scale,
-                             cap, eps, dtype, stream);
+                             nullptr, 0, 0, nullptr, w_norm, nullptr, nullptr,
+                             nullptr, bias, extra, pos, row, n_seq, H, H, D,
+                             V, 1, q_scale, cap, eps, dtype, stream);
 }
 
 int hy_memory_gates(void* steps, void* n0, void* extra, const void* proj,
@@ -744,9 +781,10 @@ int hy_ssm_step(void* y, void* state, const void* proj, int ld, int dt_off,
                 void* stream) {
   if (taps <= 0) return -2;
   return launch_step<HEAD>(nullptr, 0, y, state, proj, ld, H * V + G * N,
-                           H * V, 0, dt_off, nullptr, nullptr, nullptr, ring,
-                           wconv, bias, per_head, nullptr, pos, row, n_seq, G,
-                           H, N, V, taps, 1.f, 0.f, 0.f, dtype, stream);
+                           H * V, 0, dt_off, nullptr, nullptr, 0, 0, nullptr,
+                           nullptr, ring, wconv, bias, per_head, nullptr, pos,
+                           row, n_seq, G, H, N, V, taps, 1.f, 0.f, 0.f, dtype,
+                           stream);
 }
 
 int hy_ssm_prep(void* xbc, void* steps, const void* proj, int ld, int dt_off,

@@ -511,25 +511,43 @@ def _gated_norm(out, y, gate, g_off, w, groups, gate_first: bool, eps,
         _dt(out.dtype), _stream()), "hy_gated_norm")
 
 
+def decays_in_step(proj, low_off, w_low, dim, b) -> bool:
+    """Whether a step's kernel makes the decays' projection itself: a
+    token a sequence, loads of eight numbers on 16 bytes, and at most
+    4096 weights a head, which are two loads a lane.  In four layers with
+    heads of 64 channels and rank 64 a step takes less than with a launch
+    of their own (1 token: 206 us to 199; 64: 328 to 320), and with 128
+    and rank 128 more (2 tokens: 789 to 793; 64: 1324 to 1336)."""
+    return b.decode and proj.is_cuda and w_low.dtype == proj.dtype \
+        and w_low.is_contiguous() and proj.stride(1) == 1 \
+        and dim * w_low.shape[1] <= 4096 \
+        and (w_low.shape[1] | low_off | proj.stride(0)) % 8 == 0 \
+        and (w_low.data_ptr() | proj.data_ptr()) % 16 == 0
+
+
 def gated_linear(out, proj, k_off, v_off, g_off, dec, dec_bias, state, b,
-                 w_norm, heads, dim, vdim, tau, eps) -> None:
+                 w_norm, heads, dim, vdim, tau, eps, low=None) -> None:
     """Gated linear attention of a packed batch into ``out``
     [T, H * vdim] (columns of wider rows).  ``proj`` starts with the
-    queries; ``dec`` [T, H * dim] is the decays' projection.  Updates
-    ``state``."""
+    queries; ``dec`` [T, H * dim] is the decays' projection, or None where
+    ``decays_in_step`` allows ``low``, the offset in ``proj`` and the
+    weights that it is the product of.  Updates ``state``."""
     if not proj.is_cuda:
         ref.gated_linear(out, proj, k_off, v_off, g_off, dec, dec_bias,
                          state, b, w_norm, heads, dim, vdim, tau, eps)
         return
     assert proj.stride(1) == 1 and out.stride(1) == 1 \
-        and dec.is_contiguous()
+        and (dec is None or dec.is_contiguous())
     lib, dt, st = native(), _dt(proj.dtype), _stream()
     T, H, D, V = b.n_tok, heads, dim, vdim
     ld, q_scale, rate = _i(proj.stride(0)), _f(D ** -0.5), _f(1.0 / tau)
     if b.decode:
+        low_off, w_low = low if dec is None else (0, None)
         _check(lib.hy_gla_step(
             _ptr(out), _i(out.stride(0)), _ptr(state), _ptr(proj), ld,
-            _i(k_off), _i(v_off), _i(g_off), _ptr(dec), _ptr(dec_bias),
+            _i(k_off), _i(v_off), _i(g_off), _p(dec), _p(w_low),
+            _i(low_off), _i(0 if w_low is None else w_low.shape[1]),
+            _ptr(dec_bias),
             _ptr(w_norm), _ptr(b.pos), _ptr(b.row), _i(T), _i(H), _i(D),
             _i(V), q_scale, rate, _f(eps), dt, st), "hy_gla_step")
         return
