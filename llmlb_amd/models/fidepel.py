@@ -166,9 +166,14 @@ class FidepelLayer(nn.Module):
         index, weight, lists = hy.window_front(
             self.mix.prep(proj, b, cache, run), self.ff.routing(h),
             self.ff.act(proj, mid[:, n:]))
-        self.mix.attend(proj, b, cache, run, mid[:, :n])
-        z = self.ff.routed(h, index, lists)
-        return _linear(mid, self.w_out), (z, weight)
+        window = self.mix.attention(proj, b, cache, run, mid[:, :n])
+        both = hy.few_layer(window, h, index, lists, self.ff.w_up,
+                            self.ff.w_down, mid, self.w_out)
+        if both is None:
+            hy.window_attention(*window)
+            z = self.ff.routed(h, index, lists)
+            both = _linear(mid, self.w_out), z
+        return both[0], (both[1], weight)
 
 
 class FidepelForCausalLM(PackedCausalLM):

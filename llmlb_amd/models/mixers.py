@@ -547,14 +547,14 @@ class WindowedAttention(nn.Module):
                 self.rot, self.k_off, self.v_off, self.w_q, self.w_k,
                 self.eps, self.cos_sin, b, cache.pages[index])
 
-    def attend(self, proj, b, cache, index: int, out) -> None:
-        hy.window_attention(out, proj, self.g_off, self.heads, self.kv_heads,
-                            self.dim, self.vdim, cache.pages[index], b,
-                            self.window)
+    def attention(self, proj, b, cache, index: int, out) -> tuple:
+        """Arguments of ``hybrid.window_attention``."""
+        return (out, proj, self.g_off, self.heads, self.kv_heads, self.dim,
+                self.vdim, cache.pages[index], b, self.window)
 
     def inner(self, proj, b, cache, index: int, out) -> None:
         hy.window_prep(*self.prep(proj, b, cache, index))
-        self.attend(proj, b, cache, index, out)
+        hy.window_attention(*self.attention(proj, b, cache, index, out))
 
 
 class GroupedAttention(nn.Module):

@@ -11,8 +11,7 @@
 //
 // Both compute (w in^T) tiles: a lane holds outputs 4g..4g+3 (g = lane/16)
 // of pair n = lane % 16.
-#include "experts.h"
-#include "row_tile.h"
+#include "few_experts.h"
 #include "tile_product.h"
 
 // LDS rows are P pieces of 16 bytes; piece c of row r lies at
@@ -299,73 +298,12 @@ static int expert_product(const ExpertProduct& p) {
   return 0;
 }
 
-// Few pairs: workgroup (expert, 16 MT outputs), tiles of up to 64 of the
-// expert's pairs as in row_tile.h.  Bound by reading the matrices: both
-// products of 16 experts of 4096 x 1280 took 105 us for 64 tokens with
-// operands loaded straight into registers, 67 (5.0 TB/s) this way; 8 tokens
-// 88 -> 60, 16 experts of 1024 x 256 13.1 -> 10.5.  hy_expert_few_tile
-// has the outputs a tile.
-#define FEW_PAIRS 2048  // most that fit a workgroup's list
-// 16 NT pairs by 16 MT outputs; pieces of the depth on their way so that every
-// NT fits the LDS of the first
-#define FEW_KW 4
-template <int NT, int MT>
-using FewTile =
-    RowTile<NT, MT, FEW_KW, NT == 1 ? 3 : (NT == 2 ? 2 : 1)>;
-template <int MT>
-constexpr int FEW_LDS = FewTile<1, MT>::LDS;
-
 template <int MT>
 __global__ __launch_bounds__(FEW_KW * 64, 2) void expert_few_kernel(
-    bf16_t* __restrict__ out, const bf16_t* __restrict__ in,
-    const bf16_t* __restrict__ w, const int* __restrict__ index, int N, int K,
-    int div, int act, int n_pairs) {
-  static_assert(FewTile<2, MT>::LDS <= FEW_LDS<MT> &&
-                    FewTile<4, MT>::LDS <= FEW_LDS<MT>,
-                "one size of LDS for all tiles");
+    FewExperts a) {
   extern __shared__ __align__(1024) char lds[];
-  __shared__ unsigned short list[FEW_PAIRS];
-  __shared__ int len;
-  const int e = blockIdx.y, n0 = blockIdx.x * 16 * MT;
-  const int tid = threadIdx.x;
-  if (tid == 0) len = 0;
-  __syncthreads();
-  for (int p = tid; p < n_pairs; p += FEW_KW * 64)
-    if (index[p] == e) list[atomicAdd(&len, 1)] = (unsigned short)p;
-  __syncthreads();
-  const int count = len;
-  auto tile = [&](auto t, int first) {
-    using Tile = decltype(t);
-    Tile::run(
-        lds, K, blockIdx.x + e,
-        [&](int r) {
-          const int p = first + r < count ? first + r : count - 1;
-          return in + (size_t)(list[p] / div) * K;
-        },
-        [&](int r) {
-          return w + ((size_t)e * N + (n0 + r < N ? n0 + r : N - 1)) * K;
-        });
-    Tile::each(4 * MT, [&](int r, int c) {
-      f32x4 v = Tile::sum(lds, r, c);
-      if (act) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v[j] = fmaxf(v[j], 0.f);
-          v[j] *= v[j];
-        }
-      }
-      if (first + r < count && n0 + c < N)
-        *reinterpret_cast<uint2*>(out + (size_t)list[first + r] * N + n0 + c) =
-            make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
-    });
-    __syncthreads();
-  };
-  for (int first = 0; first < count; first += 64) {
-    const int left = count - first;
-    if (left <= 16) tile(FewTile<1, MT>{}, first);
-    else if (left <= 32) tile(FewTile<2, MT>{}, first);
-    else tile(FewTile<4, MT>{}, first);
-  }
+  __shared__ FewList list;
+  few_block<MT>(a, blockIdx.x, blockIdx.y, lds, list);
 }
 
 extern "C" {
@@ -450,14 +388,14 @@ int hy_expert_few_tile(int E, int N, int K, int n_pairs) {
 int hy_expert_few(void* out, const void* in, const void* w, const void* index,
                   int E, int N, int K, int div, int act, int n_pairs, int tile,
                   void* stream) {
-  if (E <= 0 || N <= 0 || K <= 0 || N % 8 || K % 8 || div <= 0 ||
-      E > 65535 || n_pairs > FEW_PAIRS)
-    return -2;
+  const FewExperts a{(bf16_t*)out, (const bf16_t*)in, (const bf16_t*)w,
+                     (const int*)index, E, N, K, div, act, n_pairs};
+  if (!few_ok(a)) return -2;
   if (n_pairs <= 0) return 0;
 #define GO(MT)                                                               \
   do {                                                                       \
-    static_assert(FEW_LDS<MT> + sizeof(short) * FEW_PAIRS + 64 <=            \
-                      160 * 1024, "LDS of a compute unit");                  \
+    static_assert(FEW_LDS<MT> + sizeof(FewList) <= 160 * 1024,               \
+                  "LDS of a compute unit");                                  \
     static const hipError_t sized = hipFuncSetAttribute(                     \
         reinterpret_cast<const void*>(expert_few_kernel<MT>),                \
         hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS<MT>);            \
@@ -465,8 +403,7 @@ int hy_expert_few(void* out, const void* in, const void* w, const void* index,
     hipLaunchKernelGGL(expert_few_kernel<MT>,                                \
                        dim3((N + 16 * MT - 1) / (16 * MT), E),               \
                        dim3(FEW_KW * 64), FEW_LDS<MT>, (hipStream_t)stream,  \
-                       (bf16_t*)out, (const bf16_t*)in, (const bf16_t*)w,    \
-                       (const int*)index, N, K, div, act, n_pairs);          \
+                       a);                                                   \
   } while (0)
   switch (tile < 0 ? hy_expert_few_tile(E, N, K, n_pairs) : tile) {
     case 1: GO(1); break;

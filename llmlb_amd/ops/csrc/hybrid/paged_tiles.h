@@ -35,14 +35,20 @@ struct Stage {
       pg[i] = pages[p < last_page ? p : last_page];
     }
   }
-  // row r of the fetched tile; r / 16 is the same for the whole wave
-  __device__ __forceinline__ const bf16_t* row(int r,
-                                               const int (&pg)[4]) const {
-    const int s = __builtin_amdgcn_readfirstlane(r / PAGE);
-    const int p = s == 0 ? pg[0] : (s == 1 ? pg[1] : (s == 2 ? pg[2]
-                                                             : pg[3]));
-    return cache + (size_t)__builtin_amdgcn_readfirstlane(p) * page_size +
-           head_off + (r % PAGE) * width;
+  // where the row of piece ``tid + 256 i`` lies in the cache, rows having PR
+  // pieces; its page is the same for the whole wave
+  template <int PR>
+  __device__ __forceinline__ size_t row(int i, const int (&pg)[4]) const {
+    const int r = (threadIdx.x + i * 256) / PR;
+    int p;
+    if constexpr (PR >= 16 && 256 % PR == 0) {
+      p = pg[i * 256 / PR / PAGE];
+    } else {
+      const int s = __builtin_amdgcn_readfirstlane(r / PAGE);
+      p = s == 0 ? pg[0] : (s == 1 ? pg[1] : (s == 2 ? pg[2] : pg[3]));
+    }
+    return (size_t)__builtin_amdgcn_readfirstlane(p) * page_size + head_off +
+           (r % PAGE) * width;
   }
   // ONCE: nobody reads the tile again, it goes past the caches
   template <bool ONCE = false>
@@ -54,22 +60,39 @@ struct Stage {
   __device__ __forceinline__ void fetch(int j0, const int (&pg)[4],
                                         u32x4 (&pk)[KL],
                                         u32x4 (&pv)[VL]) const {
+    ask<ONCE>(pg, pk, pv, true);
+    hide(j0, pv);
+  }
+  // The same in two parts, for tiles that are asked for long before: one that
+  // is not ``live`` asks for one piece over and over instead, so that the
+  // loads can be waited for by count.
+  template <bool ONCE>
+  __device__ __forceinline__ void ask(const int (&pg)[4], u32x4 (&pk)[KL],
+                                      u32x4 (&pv)[VL], bool live) const {
+    const size_t keep = -(size_t)live;
 #pragma unroll
     for (int i = 0; i < KL; ++i) {
-      const int p = threadIdx.x + i * 256;
-      const int c = p % KR, d = c % (DQ / 8) * 8;
+      const int c = (threadIdx.x + i * 256) % KR, d = c % (DQ / 8) * 8;
       // columns past D meet zeros of the query
-      pk[i] = load<ONCE>(row(p / KR, pg) + c / (DQ / 8) * D +
-                         (d < D ? d : 0));
+      const size_t at = row<KR>(i, pg) + c / (DQ / 8) * D + (d < D ? d : 0);
+      pk[i] = load<ONCE>(cache + (at & keep));
     }
 #pragma unroll
     for (int i = 0; i < VL; ++i) {
+      const int d = (threadIdx.x + i * 256) % VR * 8;
+      const size_t at = row<VR>(i, pg) + MAPS * D + (d < V ? d : 0);
+      pv[i] = load<ONCE>(cache + (at & keep));
+    }
+  }
+  // columns past V are zeros; rows past the last key meet zero weights and
+  // must be finite
+  __device__ __forceinline__ void hide(int j0, u32x4 (&pv)[VL],
+                                       bool live = true) const {
+    const int last = live ? last_key : -1;
+#pragma unroll
+    for (int i = 0; i < VL; ++i) {
       const int p = threadIdx.x + i * 256;
-      const int r = p / VR, d = p % VR * 8;
-      pv[i] = load<ONCE>(row(r, pg) + MAPS * D + (d < V ? d : 0));
-      // columns past V are zeros; rows past the last key meet zero weights
-      // and must be finite
-      if (j0 + r > last_key || d >= V) pv[i] = u32x4{0, 0, 0, 0};
+      if (j0 + p / VR > last || p % VR * 8 >= V) pv[i] = u32x4{0, 0, 0, 0};
     }
   }
   static __device__ __forceinline__ void store(unsigned short* lk,

@@ -12,7 +12,7 @@
 // n = lane % 16, the scores of keys 4g..4g+3 of each 16-key tile
 // (g = lane / 16).
 #include "flash.h"
-#include "paged_tiles.h"
+#include "window_decode.h"
 
 // ---------------------------------------------------------------------------
 // Prompt portions: 32 rows a wave, tiles of 64 keys through LDS, the next
@@ -244,160 +244,16 @@ __global__ __launch_bounds__(256, 2) void window_prompt_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Single tokens.  One workgroup: one query, up to 16 heads of one
-// key/value head, one part of its window.  Each wave scores 16 of a
-// tile's 64 keys, the weights go through LDS, and each wave accumulates a
-// quarter of the value columns.
-//   acc [N][H][parts][V], ml [N][H][parts] (maximum, sum); one part: the
-//   output itself
-// ONCE: no other workgroup reads the head's keys, which then go past the
-// caches and leave them to what the next kernels read: 8 layers of 61
-// sequences from 777 tokens, 32 heads of 128, 1382 -> 1354 us a step of the
-// model, of 64 sequences from 1024, 16 heads of 64, 507 -> 497.
 template <int DQ, int DV, bool ONCE>
 __global__ __launch_bounds__(256, 2)
-void window_decode_kernel(
-    bf16_t* __restrict__ out, int ld_out, float* __restrict__ ws_acc,
-    float* __restrict__ ws_ml, const bf16_t* __restrict__ proj, int ld,
-    int g_off, const bf16_t* __restrict__ cache,
-    const int* __restrict__ pos_, const int* __restrict__ row_,
-    const int* __restrict__ bt, int max_blocks, int H, int G, int D, int V,
-    Mask mask, int parts) {
-  constexpr int KD = DQ / 32, NV = DV / 64, PP = 64 + 8;
-  using St = Stage<1, DQ, DV>;
-  __shared__ unsigned short lk[64 * St::KP];
-  __shared__ unsigned short lv[64 * St::VP];
-  __shared__ unsigned short lp[16 * PP];
-  __shared__ float lmax[16][4], lsum[16][4];
-  const int q = blockIdx.x, part = blockIdx.z;
-  const int R = H / G, ht = (R + 15) / 16;
-  const int kv = blockIdx.y / ht, h0 = blockIdx.y % ht * 16;
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid & 63;
-  const int n = lane & 15, g = lane >> 4;
-  const int pos = pos_[q];
-  const int h = kv * R + h0 + n;  // this lane's head
-  const bool real = h0 + n < R;
-
-  const int span = mask.span(pos);
-  const int lo = mask.first(pos) & ~(PAGE - 1);
-  const int tiles = (pos - lo) / 64 + 1;
-  const int per = (tiles + parts - 1) / parts;
-  const int t_lo = part * per;
-  const int t_hi = t_lo + per < tiles ? t_lo + per : tiles;
-
-  St st(cache, bt + (size_t)row_[q] * max_blocks, G, kv, D, V, pos);
-  u32x4 pk[St::KL], pv[St::VL];
-  int pg[4];
-  if (t_lo < t_hi) {
-    st.fetch_pages(lo + t_lo * 64, pg);
-    st.template fetch<ONCE>(lo + t_lo * 64, pg, pk, pv);
-    if (t_lo + 1 < t_hi) st.fetch_pages(lo + t_lo * 64 + 64, pg);
-  }
-  u32x4 qf[KD];
-#pragma unroll
-  for (int k = 0; k < KD; ++k) {
-    const int d = k * 32 + g * 8;
-    qf[k] = u32x4{0, 0, 0, 0};
-    if (d < D && real)
-      qf[k] = *reinterpret_cast<const u32x4*>(proj + (size_t)q * ld +
-                                              (size_t)h * D + d);
-  }
-  // what the sum is multiplied with to gate
-  float z = 1.f;
-  if (real && g_off >= 0)
-    z += __expf(-to_f(proj[(size_t)q * ld + g_off + h]));
-
-  f32x4 o[NV];
-  float m = -1e30f, l = 0.f;
-#pragma unroll
-  for (int v = 0; v < NV; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int t = t_lo; t < t_hi; ++t) {
-    St::store(lk, lv, pk, pv);
-    __syncthreads();
-    if (t + 1 < t_hi) {
-      st.template fetch<ONCE>(lo + t * 64 + 64, pg, pk, pv);
-      if (t + 2 < t_hi) st.fetch_pages(lo + t * 64 + 128, pg);
-    }
-    const int j = lo + t * 64 + wave * 16 + g * 4;
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < KD; ++k)
-      s = mfma(*reinterpret_cast<const u32x4*>(
-                   &lk[(wave * 16 + n) * St::KP + k * 32 + g * 8]),
-               qf[k], s);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      s[i] = (unsigned)(pos - j - i) <= (unsigned)span ? s[i] : -INFINITY;
-    float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-    if (g == 0) lmax[n][wave] = mx;
-    __syncthreads();
-    mx = m;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, lmax[n][i]);
-    const float keep = __builtin_amdgcn_exp2f(m - mx);
-    m = mx;
-    l *= keep;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[i] = __builtin_amdgcn_exp2f(s[i] - m);
-      l += s[i];
-    }
-    *reinterpret_cast<uint2*>(&lp[n * PP + wave * 16 + g * 4]) =
-        make_uint2(to_bf16x2(s[0], s[1]), to_bf16x2(s[2], s[3]));
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < NV; ++v) o[v] *= keep;
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const u32x4 pf = *reinterpret_cast<const u32x4*>(
-          &lp[n * PP + ks * 32 + g * 8]);
-#pragma unroll
-      for (int v = 0; v < NV; ++v)
-        o[v] = mfma(load_columns(&lv[(ks * 32 + g * 8 + (n >> 2)) * St::VP +
-                                     (wave * NV + v) * 16 + (n & 3) * 4],
-                                 4 * St::VP),
-                    pf, o[v]);
-    }
-    __syncthreads();
-  }
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
-  if (g == 0) lsum[n][wave] = l;
-  __syncthreads();
-  if (!real) return;
-  l = lsum[n][0] + lsum[n][1] + lsum[n][2] + lsum[n][3];
-  if (parts == 1) {
-    const float f = 1.f / (l * z);
-    bf16_t* dst = out + (size_t)q * ld_out + (size_t)h * V;
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int d = (wave * NV + v) * 16 + g * 4;
-      if (d < V)
-        *reinterpret_cast<uint2*>(dst + d) =
-            make_uint2(to_bf16x2(o[v][0] * f, o[v][1] * f),
-                       to_bf16x2(o[v][2] * f, o[v][3] * f));
-    }
-    return;
-  }
-  const size_t at = ((size_t)q * H + h) * parts + part;
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int d = (wave * NV + v) * 16 + g * 4;
-    if (d < V)
-      *reinterpret_cast<float4*>(ws_acc + at * V + d) =
-          make_float4(o[v][0], o[v][1], o[v][2], o[v][3]);
-  }
-  if (wave == 0 && g == 0) {
-    ws_ml[at * 2] = m;
-    ws_ml[at * 2 + 1] = l;
-  }
+void window_decode_kernel(WindowDecode a) {
+  __shared__ WindowLds<DQ, DV> lds;
+  window_decode_block<DQ, DV, ONCE>(a, blockIdx.x, blockIdx.y, blockIdx.z,
+                                    lds);
 }
 
 // Join the parts and gate.  One wave a head; lane p first holds part p's
 // weight.  A part without keys has sum 0 and the lowest maximum.
-#define PARTS_MAX 64
 __global__ __launch_bounds__(256) void window_merge_kernel(
     bf16_t* __restrict__ out, int ld_out, const float* __restrict__ ws_acc,
     const float* __restrict__ ws_ml, const bf16_t* __restrict__ proj, int ld,
@@ -435,13 +291,6 @@ __global__ __launch_bounds__(256) void window_merge_kernel(
   if (c < V) store4(out + (size_t)q * ld_out + (size_t)h * V + c, o);
 }
 
-static bool window_ok(int ld, int ld_out, int H, int G, int D, int V,
-                      int window) {
-  return G > 0 && H > 0 && H % G == 0 && D > 0 && V > 0 && D % 8 == 0 &&
-         V % 8 == 0 && D <= 256 && V <= 256 && ld % 8 == 0 &&
-         ld_out % 8 == 0 && window >= 1;
-}
-
 // GO(DQ, DV) for the smallest tile that holds D and V
 #define WINDOW_SIZES(D, V)                               \
   do {                                                   \
@@ -457,6 +306,15 @@ static bool window_ok(int ld, int ld_out, int H, int G, int D, int V,
     else if (V <= 128) GO(Q, 128);                       \
     else GO(Q, 256);                                     \
   } while (0)
+
+int window_merge(const WindowDecode& a, int n_rows, hipStream_t stream) {
+  if (a.parts == 1) return 0;
+  hipLaunchKernelGGL(window_merge_kernel, dim3(n_rows, (a.H + 3) / 4),
+                     dim3(256), 0, stream, a.out, a.ld_out, a.acc, a.ml,
+                     a.proj, a.ld, a.g_off, a.H, a.V, a.parts);
+  HY_CHECK();
+  return 0;
+}
 
 extern "C" {
 
@@ -496,20 +354,18 @@ int hy_window_decode(void* out, int ld_out, void* acc, void* ml,
                      const void* pos, const void* row, const void* bt,
                      int max_blocks, int H, int G, int D, int V, int window,
                      int chunk, int n_rows, int parts, void* stream) {
-  if (!window_ok(ld, ld_out, H, G, D, V, window) || parts < 1 ||
-      parts > PARTS_MAX || (parts > 1 && (!acc || !ml)))
-    return -2;
+  const WindowDecode a{(bf16_t*)out, ld_out, (float*)acc, (float*)ml,
+                       (const bf16_t*)proj, ld, g_off, (const bf16_t*)cache,
+                       (const int*)pos, (const int*)row, (const int*)bt,
+                       max_blocks, H, G, D, V, Mask{window, chunk != 0},
+                       parts};
+  if (!window_decode_ok(a)) return -2;
   if (n_rows <= 0) return 0;
   const int tiles = (H / G + 15) / 16;
-  if (G * tiles > 65535) return -2;
-  const Mask mask{window, chunk != 0};
-#define RUN(DQ, DV, ONCE)                                                    \
-  hipLaunchKernelGGL((window_decode_kernel<DQ, DV, ONCE>),                   \
-                     dim3(n_rows, G * tiles, parts), dim3(256), 0,           \
-                     (hipStream_t)stream, (bf16_t*)out, ld_out, (float*)acc, \
-                     (float*)ml, (const bf16_t*)proj, ld, g_off,             \
-                     (const bf16_t*)cache, (const int*)pos, (const int*)row, \
-                     (const int*)bt, max_blocks, H, G, D, V, mask, parts)
+#define RUN(DQ, DV, ONCE)                                          \
+  hipLaunchKernelGGL((window_decode_kernel<DQ, DV, ONCE>),         \
+                     dim3(n_rows, G * tiles, parts), dim3(256), 0, \
+                     (hipStream_t)stream, a)
 #define GO(DQ, DV)                     \
   do {                                 \
     if (tiles == 1) RUN(DQ, DV, true); \
@@ -519,13 +375,7 @@ int hy_window_decode(void* out, int ld_out, void* acc, void* ml,
 #undef GO
 #undef RUN
   HY_CHECK();
-  if (parts == 1) return 0;
-  hipLaunchKernelGGL(window_merge_kernel, dim3(n_rows, (H + 3) / 4),
-                     dim3(256), 0, (hipStream_t)stream, (bf16_t*)out, ld_out,
-                     (const float*)acc, (const float*)ml,
-                     (const bf16_t*)proj, ld, g_off, H, V, parts);
-  HY_CHECK();
-  return 0;
+  return window_merge(a, n_rows, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -15,6 +15,8 @@ import math
 
 import torch
 
+import llmlb_amd.ops as ops
+
 from . import NativeKernelsMissing, _check, _ptr, _stream, linear_rows
 from . import reference_hybrid as ref
 from .build import library_path
@@ -837,6 +839,63 @@ def window_attention(out, proj, g_off, heads, kv_heads, dim, vdim, cache, b,
         _check(lib.hy_window_flash(
             *dst, *src, _ptr(items), _i(n_items), *where, *sizes, st),
             "hy_window_flash")
+
+
+def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
+    """``window_attention(*window)``, ``experts`` of ``h`` and the product
+    mid @ w_out^T of a parallel layer's single tokens, independent parts in
+    the same launch: (product, experts' outputs).  None where nothing is
+    done: more tokens, other sizes, what other kernels or the library
+    take."""
+    out, proj, g_off, H, G, D, V, cache, b, size, *chunk = window
+    n, top = index.shape
+    E, F, W = w_up.shape
+    if (not proj.is_cuda or lists is not None or b.n_short != n or n > 128
+            or FEW_TILE >= 0 or ops._USE_CUSTOM_DECODE_GEMM != "auto"
+            or not ops._takes_row_gemm(mid, w_out)
+            or not ops._only_numbers(h, proj, w_up, w_down)
+            or not can_window_mfma(proj.dtype, H // G, D, V)
+            or not can_expert_mfma(h.dtype, W, F)
+            or (proj.stride(0) | out.stride(0) | mid.shape[1]) % 8
+            or w_out.shape[0] % 4 or not mid.is_contiguous()
+            or not w_out.is_contiguous()
+            or (mid.data_ptr() | w_out.data_ptr()) % 16):
+        return None
+    product = ops._product_of(mid, w_out, "plain", None, 0)
+    if product is None:
+        return None
+    assert proj.stride(1) == 1 and out.stride(1) == 1 \
+        and h.is_contiguous() and w_up.is_contiguous() \
+        and w_down.is_contiguous() and w_down.shape == (E, W, F) \
+        and h.shape == (n, W) and cache.shape[0] * G * 16 < 2 ** 31
+    lib, bt, st = native(), b.block_tables, _stream()
+    parts = window_parts(n, G, H // G, min(size, b.max_keys))
+    acc = ml = None
+    if parts > 1:
+        acc = torch.empty(n, H, parts, V, dtype=torch.float32,
+                          device=proj.device)
+        ml = torch.empty(n, H, parts, 2, dtype=torch.float32,
+                         device=proj.device)
+    u = torch.empty(n * top, F, dtype=h.dtype, device=h.device)
+    done = lib.hy_window_up(
+        _ptr(out), _i(out.stride(0)), _p(acc), _p(ml), _ptr(proj),
+        _i(proj.stride(0)), _i(-1 if g_off is None else g_off), _ptr(cache),
+        _ptr(b.pos), _ptr(b.row), _ptr(bt), _i(bt.shape[1]), _i(H), _i(G),
+        _i(D), _i(V), _i(size), _i(bool(chunk and chunk[0])), _i(n),
+        _i(parts), _ptr(u), _ptr(h), _ptr(w_up), _ptr(index), _i(E), _i(F),
+        _i(W), _i(top), st)
+    if done == 0:
+        return None
+    z = torch.empty(n, top, W, dtype=h.dtype, device=h.device)
+    M, y = product
+    if done == 1:
+        done = lib.hy_down_out(
+            _ptr(y), _ptr(mid), _ptr(w_out), _i(n), _i(M), _i(mid.shape[1]),
+            _ptr(z), _ptr(u), _ptr(w_down), _ptr(index), _i(E), _i(W), _i(F),
+            _i(n * top), st)
+    if done != 1:
+        _check(done or -1, "hy_window_up, hy_down_out")
+    return y, z
 
 
 # -- mixture of experts ----------------------------------------------------
