@@ -98,8 +98,13 @@ __global__ __launch_bounds__(256) void post_norm_add_kernel(
 // type.  y null: nothing is added; w2 (and h2) null: one norm; w1 null: the
 // sum alone.  ROUTED: x += mult (y + sum over k of zw[k] z[k]) with ``top``
 // more rows z of the token.  ONE: w1 and w2 are single numbers.  One
-// workgroup per row, kept in registers between the passes where it fits.
-template <typename T, bool ROUTED, bool ONE>
+// workgroup per row, of which KEEP vectors a thread stay in registers between
+// the passes; a few rows' time is a chain of loads, so their weights are asked
+// for with them.  us, weights after the norm and always room for four -> this:
+// 64 rows of 4096, two norms 4.18 -> 3.84, with 4 routed rows 4.66 -> 3.99; of 1024
+// 3.07 -> 2.78, 3.33 -> 2.88; 16384 of 4096 184 -> 181, 249 -> 246.  (post_norm_add
+// and post_pre_norm gained nothing by it.)
+template <typename T, bool ROUTED, bool ONE, int KEEP>
 __global__ __launch_bounds__(256) void add_norms_kernel(
     float* __restrict__ x, const T* __restrict__ y,
     const T* __restrict__ z, const float* __restrict__ zw, int top,
@@ -113,8 +118,18 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
   }
   const bool vec = (width & 7) == 0;
   const int nvec = vec ? width >> 3 : 0;
-  float keep[NORM_KEEP][8];
+  float keep[KEEP][8], w1k[KEEP][8], w2k[KEEP][8];
   float ssq = 0.f;
+  if (!ONE && w1) {
+#pragma unroll
+    for (int n = 0; n < KEEP; ++n) {
+      const int i = threadIdx.x + n * 256;
+      if (i < nvec) {
+        load8(w1 + i * 8, w1k[n]);
+        if (w2) load8(w2 + i * 8, w2k[n]);
+      }
+    }
+  }
   auto sum = [&](int i, float* f) {
     load8(x + base + i * 8, f);
     if (y) {
@@ -138,11 +153,11 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
     for (int j = 0; j < 8; ++j) ssq += f[j] * f[j];
   };
 #pragma unroll
-  for (int n = 0; n < NORM_KEEP; ++n) {
+  for (int n = 0; n < KEEP; ++n) {
     const int i = threadIdx.x + n * 256;
     if (i < nvec) sum(i, keep[n]);
   }
-  for (int i = threadIdx.x + NORM_KEEP * 256; i < nvec; i += 256) {
+  for (int i = threadIdx.x + KEEP * 256; i < nvec; i += 256) {
     float f[8];
     sum(i, f);
   }
@@ -162,28 +177,30 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
   if (!w1) return;
   const float r = 1.f / sqrtf(block_sum_256(ssq, red) / width + eps);
 
-  auto emit = [&](int i, const float* f) {
-    float w[8], o[8];
-    if (!ONE) load8(w1 + i * 8, w);
+  auto emit = [&](int i, const float* f, const float* a, const float* b) {
+    float o[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f[j] * r * (ONE ? w1[0] : w[j]);
+    for (int j = 0; j < 8; ++j) o[j] = f[j] * r * (ONE ? w1[0] : a[j]);
     store8(h1 + base + i * 8, o);
     if (!w2) return;
-    if (!ONE) load8(w2 + i * 8, w);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f[j] * r * (ONE ? w2[0] : w[j]);
+    for (int j = 0; j < 8; ++j) o[j] = f[j] * r * (ONE ? w2[0] : b[j]);
     store8(h2 + base + i * 8, o);
   };
 #pragma unroll
-  for (int n = 0; n < NORM_KEEP; ++n) {
+  for (int n = 0; n < KEEP; ++n) {
     const int i = threadIdx.x + n * 256;
-    if (i < nvec) emit(i, keep[n]);
+    if (i < nvec) emit(i, keep[n], w1k[n], w2k[n]);
   }
   // a thread reads back only what it wrote itself
-  for (int i = threadIdx.x + NORM_KEEP * 256; i < nvec; i += 256) {
-    float f[8];
+  for (int i = threadIdx.x + KEEP * 256; i < nvec; i += 256) {
+    float f[8], a[8], b[8];
     load8(x + base + i * 8, f);
-    emit(i, f);
+    if (!ONE) {
+      load8(w1 + i * 8, a);
+      if (w2) load8(w2 + i * 8, b);
+    }
+    emit(i, f, a, b);
   }
   if (!vec)
     for (int i = threadIdx.x; i < width; i += 256) {
@@ -627,17 +644,24 @@ int hy_add_norms(void* x, const void* y, const void* z, const void* zw,
   if ((w1 && !h1) || (w2 && (!h2 || !w1))) return -2;
   if (z && (!y || !zw || top < 1)) return -2;
   if (n_tok <= 0) return 0;
-#define GO(ROUTED, ONE)                                                      \
+#define RUN(ROUTED, ONE, KEEP)                                               \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                        \
-      (add_norms_kernel<T, ROUTED, ONE>), dim3(n_tok), dim3(256), 0,         \
+      (add_norms_kernel<T, ROUTED, ONE, KEEP>), dim3(n_tok), dim3(256), 0,   \
       (hipStream_t)stream, (float*)x, (const T*)y, (const T*)z,              \
       (const float*)zw, top, mult, (const float*)w1, (const float*)w2,       \
       (T*)h1, (T*)h2, width, eps))
+#define GO(ROUTED, ONE)                            \
+  do {                                             \
+    if (width <= 2048) RUN(ROUTED, ONE, 1);        \
+    else if (width <= 4096) RUN(ROUTED, ONE, 2);   \
+    else RUN(ROUTED, ONE, 4);                      \
+  } while (0)
   if (z && one) GO(true, true);
   else if (z) GO(true, false);
   else if (one) GO(false, true);
   else GO(false, false);
 #undef GO
+#undef RUN
   HY_CHECK();
   return 0;
 }
