@@ -35,8 +35,8 @@ __device__ __forceinline__ int swizzle_w(int r) {
 // other: copies are at one scalar address and a lane's own offset, which
 // takes no vector instruction a step (63 a wave before, a quarter of the
 // time).  16384 tokens with 4 of 16 experts, us: 4096 to 1280 wide 668 ->
-// 612, back 752 -> 687; 2048 to 512 169 -> 153, back 174 -> 166.  What a
-// compute unit takes in bounds it then, 42 GB/s of about 50.
+// 612, back 752 -> 687; 2048 to 512 169 -> 153, back 174 -> 166.  A
+// compute unit takes in 42 GB/s then; copies alone reach 115.
 // Results are stored by way of the caches: the next kernel reads them, and
 // past the caches (nontemporal) they wait for what these write back (2048
 // wide in a model: back 222 -> 193).
