@@ -108,6 +108,7 @@ def test_gradients_and_autocast_keep_the_library():
         assert ops.linear_act(x, w, "gelu") is None
 
 
+@torch.inference_mode()     # as all captures of a process
 def test_captured():
     x, w = _rows(300, 512, 8).contiguous(), _rows(640, 512, 9).contiguous()
     graph = torch.cuda.CUDAGraph()

@@ -120,6 +120,7 @@ def test_other_operands_take_two_launches():
         assert ops.linear_normed(*a) is None
 
 
+@torch.inference_mode()     # as all captures of a process
 def test_captured():
     x, r, w, g = _inputs(1, 2048, 1024)
     ops.linear_normed(x, w, (g, 1e-5, r))

@@ -108,6 +108,7 @@ def test_other_routes():
     assert hy.few_layer(*args) is None
 
 
+@torch.inference_mode()     # as all captures of a process
 def test_captured():
     """Replays with eager work between them."""
     args = operands(20, 256, 4, 2, 64, 64, 64, 32, 8, 2, 300, 64, False)
