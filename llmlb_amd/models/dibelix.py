@@ -212,7 +212,7 @@ class DibelixForCausalLM(PackedCausalLM):
             hy.post_norm_add(x, xb, ly.mix(xb, b, cache, i), ly.norm1, eps,
                              self.norm_offset)
             if ly.ff is not None:
-                hy.post_norm_add(x, xb, ly.ff(xb), ly.norm2, eps,
+                hy.post_norm_add(x, xb, ly.ff(xb, True), ly.norm2, eps,
                                  self.norm_offset)
             if on_layer is not None:
                 on_layer(i, x)

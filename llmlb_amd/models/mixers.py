@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
 from ..ops import (linear_act, linear_decode, linear_heads, linear_rows,
-                   linear_two)
+                   linear_shares, linear_two)
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
@@ -287,10 +287,14 @@ class DenseFF(nn.Module):
         self.w_up = _param(F.pad(w["up"], (0, 0, 0, gap)).to(**to))
         self.w_down = _param(F.pad(w["down"], (0, gap)).to(**to))
 
-    def forward(self, x):
+    def forward(self, x, shares: bool = False):
+        """``shares``: the caller also takes float shares of the product
+        (``linear_shares``) in rows of whole vectors."""
         u = linear_act(x, self.w_up, self.act)
         if u is not None:
-            return _linear(u, self.w_down)
+            y = linear_shares(u, self.w_down) \
+                if shares and self.width % 8 == 0 else None
+            return _linear(u, self.w_down) if y is None else y
         u = _linear(x, self.w_up)
         if self.act == "gelu":
             hy.gelu_tanh_(u)

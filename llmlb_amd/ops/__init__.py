@@ -991,6 +991,31 @@ def linear_two(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor,
     return out
 
 
+def linear_shares(x: torch.Tensor, weight: torch.Tensor
+                  ) -> torch.Tensor | None:
+    """x @ W^T as float shares [n, N, M] of the depth whose sum, rounded once,
+    is what linear_decode returns, for a caller that adds them up itself.  None
+    where it would not take the depth in shares."""
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight)
+            or weight.dtype != x.dtype or x.stride(1) != 1
+            or not weight.is_contiguous()):
+        return None
+    (N, K), M = x.shape, weight.shape[0]
+    sizes = (ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
+    shares = _lib.ll_row_gemm_shares(*sizes)
+    if shares < 2:
+        return None
+    ws = torch.empty(shares, N, M, device=x.device, dtype=torch.float32)
+    parts = _lib.ll_row_gemm_parts(
+        _ptr(x), _ptr(weight), _ptr(ws), ctypes.c_int(shares), *sizes,
+        ctypes.c_int(x.stride(0)), _stream())
+    if parts == -2:
+        return None
+    if parts < 1:
+        _check(parts, "ll_row_gemm_parts")
+    return ws[:parts]
+
+
 def linear_decode(x: torch.Tensor, weight: torch.Tensor,
                   w8: tuple | None = None) -> torch.Tensor:
     """out = x @ W^T for up to 128 rows.

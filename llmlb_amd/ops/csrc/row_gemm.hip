@@ -529,14 +529,14 @@ extern "C" int ll_row_gemm_shares(int N, int M, int K) {
   return shares >= 2 && large * shares >= 176 ? shares : 1;
 }
 
-// The same in shares (see above), ws [shares][N][M] floats.
-extern "C" int ll_row_gemm_split(void* out, int ld_out, const void* x,
-                                 const void* w, void* ws, int shares, int N,
-                                 int M, int K, int ldx, void* stream) {
+// The shares alone, ws [shares][N][M] floats; > 0: as many as there are (with
+// rounding to pieces of 64, up to ``shares``), -2: not for this kernel.
+extern "C" int ll_row_gemm_parts(const void* x, const void* w, void* ws,
+                                 int shares, int N, int M, int K, int ldx,
+                                 void* stream) {
   if (N <= 16 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
-      ld_out % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
-      (uintptr_t)out % 8 || (uintptr_t)ws % 16 || shares < 1 ||
-      shares > 256)
+      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)ws % 16 ||
+      shares < 1 || shares > 256)
     return -2;
   const int tiles = (N + 15) / 16, across = (tiles + 3) / 4;
   const int depth = ((K + shares - 1) / shares + 63) / 64 * 64;
@@ -560,11 +560,21 @@ extern "C" int ll_row_gemm_split(void* out, int ld_out, const void* x,
     default: GO(4); break;
   }
 #undef GO
-  HY_CHECK();
+  return hipGetLastError() == hipSuccess ? parts : -1;
+}
+
+// The same product in shares, which a second kernel adds up.
+extern "C" int ll_row_gemm_split(void* out, int ld_out, const void* x,
+                                 const void* w, void* ws, int shares, int N,
+                                 int M, int K, int ldx, void* stream) {
+  if (ld_out % 4 || (uintptr_t)out % 8) return -2;
+  const int parts =
+      ll_row_gemm_parts(x, w, ws, shares, N, M, K, ldx, stream);
+  if (parts < 0) return parts;
   hipLaunchKernelGGL(row_gemm_join_kernel,
                      dim3((unsigned)(((size_t)N * (M / 4) + 255) / 256)),
-                     dim3(256), 0, st, (bf16_t*)out, ld_out, (const float*)ws,
-                     N, M, parts);
+                     dim3(256), 0, (hipStream_t)stream, (bf16_t*)out, ld_out,
+                     (const float*)ws, N, M, parts);
   HY_CHECK();
   return 0;
 }

@@ -80,11 +80,19 @@ def embed_rows(table, ids, copy: bool = True):
 
 def post_norm_add(x, xb, y, w, eps, w_offset=0.0) -> None:
     """In place: x += rmsnorm(y) * (w_offset + w); xb = x in the storage
-    type (xb may be x itself)."""
+    type (xb may be x itself).  ``y`` may be float shares [n, T, W] of a
+    16-bit product, which are added up first."""
     if not x.is_cuda:
         ref.post_norm_add(x, xb, y, w, eps, w_offset)
         return
-    assert y.is_contiguous() and y.shape == x.shape
+    assert y.is_contiguous() and y.shape[-2:] == x.shape
+    if y.dim() == 3:
+        assert y.dtype == torch.float32 and xb.dtype == torch.bfloat16
+        _check(native().hy_post_norm_join(
+            _ptr(x), _ptr(xb), _ptr(y), _i(y.shape[0]), _ptr(w),
+            _f(w_offset), _i(x.shape[0]), _i(x.shape[1]), _f(eps),
+            _stream()), "hy_post_norm_join")
+        return
     _check(native().hy_post_norm_add(
         _ptr(x), None if xb is x else _ptr(xb), _ptr(y), _ptr(w),
         _f(w_offset), _i(x.shape[0]), _i(x.shape[1]), _f(eps), _dt(y.dtype),
