@@ -239,6 +239,8 @@ static int float_gemm_launch(const FloatGemm& p) {
   auto* kernel = &float_gemm_kernel<NT, MT, KW>;
   constexpr int lds = FloatTile<NT, MT, KW>::LDS;
   static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+  // a lane's copies are at 32-bit offsets in bytes from the tile's first row
+  if (64ll * NT * p.ldx > 1ll << 32 || 64ll * MT * p.K > 1ll << 32) return -2;
   static const hipError_t sized = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -303,10 +305,9 @@ static int float_tile(int N, int M, int K) {
 extern "C" int ll_float_gemm(void* out, int ld_out, const void* x,
                              const void* w, int N, int M, int K, int ldx,
                              int kind, int tile, void* stream) {
-  // copies are at a lane's 32-bit offset in bytes
   if (N <= 0 || M <= 0 || K <= 0 || M % 4 || K % 32 || ldx < K || ldx % 4 ||
-      ld_out < M || ld_out % 4 || K >= 1 << 24 || ldx >= 1 << 24 ||
-      (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16 ||
+      ld_out < M || ld_out % 4 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
+      (uintptr_t)out % 16 ||
       (kind != PLAIN && kind != RELU2 && kind != GELU))
     return -2;
   // a tile's beginning and end are most of a shallow product (us, the library

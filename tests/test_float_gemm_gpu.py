@@ -120,3 +120,14 @@ def test_captured():
         x.copy_(_rows(300, 512, seed))
         graph.replay()
         assert torch.equal(out, ops.linear_rows(x, w))
+
+
+@pytest.mark.parametrize("tile", [-1, 7, 8, 10])
+def test_long_strides(tile):
+    """Rows 14 million numbers apart: past 32 bits in tiles of 80 rows."""
+    x = torch.zeros(97, 14_000_000, device=DEV)[:, :64]
+    x.copy_(_rows(97, 64, 12))
+    w = _rows(4096, 64, 13).contiguous()
+    out = ops._float_gemm(x, w, tile=tile)
+    assert (out is None) if tile >= 8 else (tile < 0 or out is not None)
+    _close(ops.linear_rows(x, w) if out is None else out, x, w)
