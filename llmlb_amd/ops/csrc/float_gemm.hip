@@ -2,13 +2,18 @@
 //
 //   out[N, M] = act(x[N, K] W[M, K]^T)     float, summed in float
 //
-// A float is the sum of three bf16 numbers without a remainder (8 + 8 + 8
-// bits), so a product of two is nine products of those, of which the three
-// smallest are left out: less than 2^-21 of the product, 2^-24 on average.  Six
-// times the work at sixteen times the rate of the float instructions, and the
-// sum is rounded once in 32 of the depth where theirs is in every four: errors
-// of normal numbers 1024 deep are 1.7e-7 to 2.4e-7 of the result (the library's
-// product 2.9e-7 to 5.7e-7), 3328 deep 3.2e-7 to 4.5e-7 (5.2e-7 to 1.0e-6).
+// A float is the sum of three bf16 numbers without a remainder, each the nearest
+// to what the ones before leave (8 bits and a sign each), so a product of two is
+// nine products of those, of which the three smallest are left out: 2^-24 of the
+// product at most, to either side.  Six times the work at sixteen times the rate
+// of the float instructions, and the sum is rounded once in 32 of the depth where
+// theirs is in every four.  Errors against 64 bits, the library's -> here: normal
+// numbers 32 deep 1.0e-7 -> 3.8e-8, 256 2.9e-7 -> 6.4e-8, 1024 5.8e-7 -> 1.6e-7,
+// 3328 1.0e-6 -> 3.1e-7; numbers from 1 to 1.01 256 deep 2.1e-7 -> 5.2e-8, on
+// average 9e-10 to one side.  Only rows with a single number that is not zero,
+// which the library rounds once, are further off: 2.5e-8 -> 3.4e-8.  (Cutting bits
+// off takes as many instructions and a few percent less time, but parts of one
+// sign leave out up to 2^-21, always to the same side: 6.9e-8 of single numbers.)
 //
 // Bound by vector instructions, which take numbers apart (5.5 a number of a
 // tile's edge), beside matrix instructions (a tile of 64 x 64, of 128 of the
@@ -18,27 +23,14 @@
 // one wave a SIMD: 600 rows, 1024 x 1024 16 us, 13.5 this way); larger tiles
 // take less apart (600 rows of 4096 x 2048 74 us with 64 x 64, 61 with 80 x 64).
 // us, the library -> here, weights from HBM:
-//   600 rows: 1024 x 1024 16.5 -> 13.4, 3328 x 1024 38 -> 32, 4128 x 1024 52 ->
-//       39, 1024 x 3328 43 -> 32; 64 rows: 8.3 -> 5.1, 12.5 -> 8.4, 13.7 ->
-//       12.7, 11.5 -> 11.7; 16 rows of 4096 x 2048 12.5 -> 9.5; 1600 rows of
-//       4096 x 2048 245 -> 143 (188 TFLOP/s)
+//   600 rows: 1024 x 1024 16.7 -> 13.9, 3328 x 1024 37 -> 34, 4128 x 1024 53 ->
+//       40, 1024 x 3328 41 -> 34; 64 rows: 8.3 -> 5.3, 12.5 -> 8.6, 13.4 ->
+//       13.0, 11.6 -> 11.6; 16 rows of 4096 x 2048 12.2 -> 9.3; 1600 rows of
+//       4096 x 2048 238 -> 151 (178 TFLOP/s)
 #include <float.h>
 
 #include "hybrid/row_act.h"
 #include "hybrid/lds_copy.h"
-
-// Two floats as sums of three bf16 numbers each, by cutting bits off.
-__device__ __forceinline__ void cut3(unsigned a, unsigned b,
-                                     unsigned (&part)[3]) {
-#pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    part[t] = __builtin_amdgcn_perm(b, a, 0x07060302);
-    a = __float_as_uint(__uint_as_float(a) -
-                        __uint_as_float(a & 0xffff0000u));
-    b = __float_as_uint(__uint_as_float(b) -
-                        __uint_as_float(b & 0xffff0000u));
-  }
-}
 
 // One tile, 16 NT rows of x against 16 MT of W; KW waves share it and split
 // the depth in pieces of 32 (rows of 128 bytes), as RowTile's do.
@@ -107,10 +99,11 @@ struct FloatTile {
         for (int s = 0; s < 2; ++s)
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
-            unsigned cut[3];
-            cut3(raw[f][s][2 * c], raw[f][s][2 * c + 1], cut);
+            unsigned p[3];
+            split3(__uint_as_float(raw[f][s][2 * c]),
+                   __uint_as_float(raw[f][s][2 * c + 1]), p[0], p[1], p[2]);
 #pragma unroll
-            for (int t = 0; t < 3; ++t) part[f][t][2 * s + c] = cut[t];
+            for (int t = 0; t < 3; ++t) part[f][t][2 * s + c] = p[t];
           }
       constexpr int WP[] = {2, 0, 1, 1, 0, 0}, XP[] = {0, 2, 1, 0, 1, 0};
 #pragma unroll

@@ -131,3 +131,30 @@ def test_long_strides(tile):
     out = ops._float_gemm(x, w, tile=tile)
     assert (out is None) if tile >= 8 else (tile < 0 or out is not None)
     _close(ops.linear_rows(x, w) if out is None else out, x, w)
+
+
+@pytest.mark.parametrize("K", [32, 96, 256])
+def test_shallow_errors_are_not_the_librarys(K):
+    g = torch.Generator(device=DEV).manual_seed(K)
+    near = [1 + 0.01 * torch.rand(300, K, generator=g, device=DEV)
+            for _ in range(2)]
+    for x, w in ((_rows(300, K, 1), _rows(256, K, 2).contiguous()),
+                 (near[0], near[1][:256].contiguous())):
+        ref = x.double() @ w.double().T
+        off = [t.double() - ref for t in
+               (ops._float_gemm(x, w), torch.nn.functional.linear(x, w))]
+        assert off[0].norm() <= off[1].norm()
+    # what is left out of these has the sign of the parts: to either side, so
+    # that 76800 sums average far below a float's last bit
+    assert abs((off[0] / ref).mean()) < 2.0 ** -27
+
+
+def test_rows_of_one_number():
+    """2^-24 are left out at most, and the last of the parts' sums may be cut
+    off, not rounded: 2^-23."""
+    x = torch.zeros(256, 128, device=DEV)
+    x[torch.arange(256), torch.arange(256) % 128] = _rows(256, 32, 14)[:, 0]
+    w = _rows(512, 128, 15).contiguous()
+    ref = x.double() @ w.double().T
+    off = ((ops._float_gemm(x, w).double() - ref) / ref).abs()
+    assert off.max() <= 1.5 * 2.0 ** -23
