@@ -15,22 +15,29 @@
 // off takes as many instructions and a few percent less time, but parts of one
 // sign leave out up to 2^-21, always to the same side: 6.9e-8 of single numbers.)
 //
-// Bound by vector instructions, which take numbers apart (5.5 a number of a
-// tile's edge), beside matrix instructions (a tile of 64 x 64, of 128 of the
-// depth: 1630 and 1540 cycles a SIMD, 3060 in all), and by how tiles fill the
+// Bound by vector instructions, which take numbers apart and look for the largest
+// (6 a number of a tile's edge), beside matrix instructions (a tile of 64 x 64, of
+// 128 of the depth: 1780 and 1540 cycles a SIMD), and by how tiles fill the
 // last round.  So waves have one stage and no pipeline of their own, and two to
 // four of them a SIMD cover each other (two stages and a software pipeline at
-// one wave a SIMD: 600 rows, 1024 x 1024 16 us, 13.5 this way); larger tiles
-// take less apart (600 rows of 4096 x 2048 74 us with 64 x 64, 61 with 80 x 64).
+// one wave a SIMD: 600 rows, 1024 x 1024 16 us, 14.2 this way); larger tiles
+// take less apart (600 rows of 4096 x 2048 76 us with 64 x 64, 66 with 80 x 64).
 // us, the library -> here, weights from HBM:
-//   600 rows: 1024 x 1024 16.7 -> 13.9, 3328 x 1024 37 -> 34, 4128 x 1024 53 ->
-//       40, 1024 x 3328 41 -> 34; 64 rows: 8.3 -> 5.3, 12.5 -> 8.6, 13.4 ->
-//       13.0, 11.6 -> 11.6; 16 rows of 4096 x 2048 12.2 -> 9.3; 1600 rows of
-//       4096 x 2048 238 -> 151 (178 TFLOP/s)
+//   600 rows: 1024 x 1024 16.7 -> 14.2, 3328 x 1024 37 -> 34, 4128 x 1024 53 ->
+//       41, 1024 x 3328 41 -> 34; 64 rows: 8.5 -> 5.5, 12.5 -> 8.9, 13.3 ->
+//       13.2, 11.7 -> 11.6; 16 rows of 4096 x 2048 12.3 -> 9.4; 1600 rows of
+//       4096 x 2048 237 -> 156 (172 TFLOP/s)
+// The largest numbers, which tell what may be lost (see the kernel), cost 2 to 5%.
 #include <float.h>
 
 #include "hybrid/row_act.h"
 #include "hybrid/lds_copy.h"
+
+// the larger of ``most`` and the sizes of two numbers, in one instruction
+__device__ __forceinline__ float larger(float most, float a, float b) {
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(a), "v"(b));
+  return most;
+}
 
 // One tile, 16 NT rows of x against 16 MT of W; KW waves share it and split
 // the depth in pieces of 32 (rows of 128 bytes), as RowTile's do.
@@ -40,7 +47,10 @@ struct FloatTile {
   static constexpr int STAGE = F * 2048;  // one piece of all rows
   static constexpr int RP = 16 * MT + 4;  // row of the sums
   static constexpr int STAGES = KW * STAGE, SUMS = KW / 2 * 16 * NT * RP * 4;
-  static constexpr int LDS = STAGES > SUMS ? STAGES : SUMS;
+  // behind the sums: the largest size in every 16th row of x, and of W, and a bit
+  // for every block of 16 x 16 outputs
+  static constexpr int ENDS = SUMS + 33 * 4;
+  static constexpr int LDS = STAGES > ENDS ? STAGES : ENDS;
 
   // x, w: the tile's first rows; last_x, last_w: the last ones there are
   static __device__ __forceinline__ void run(char* lds, int K, int step,
@@ -80,6 +90,7 @@ struct FloatTile {
     for (int a = 0; a < MT; ++a)
 #pragma unroll
       for (int b = 0; b < NT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float most[2] = {0.f, 0.f};  // of the lane's rows of x, of W
     if (count) copy(0);
     for (int i = 0; i < count; ++i) {
       wait_copies<0>();
@@ -99,9 +110,11 @@ struct FloatTile {
         for (int s = 0; s < 2; ++s)
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
+            const float lo = __uint_as_float(raw[f][s][2 * c]);
+            const float hi = __uint_as_float(raw[f][s][2 * c + 1]);
+            most[f >= NT] = larger(most[f >= NT], lo, hi);
             unsigned p[3];
-            split3(__uint_as_float(raw[f][s][2 * c]),
-                   __uint_as_float(raw[f][s][2 * c + 1]), p[0], p[1], p[2]);
+            split3(lo, hi, p[0], p[1], p[2]);
 #pragma unroll
             for (int t = 0; t < 3; ++t) part[f][t][2 * s + c] = p[t];
           }
@@ -124,6 +137,7 @@ struct FloatTile {
           a * 16 + hi * 4);
     };
     __syncthreads();
+    if (tid < 33) ends(lds)[tid] = 0;
     if (wave >= KW / 2) {
 #pragma unroll
       for (int b = 0; b < NT; ++b)
@@ -131,6 +145,9 @@ struct FloatTile {
         for (int a = 0; a < MT; ++a) *at_of(wave - KW / 2, a, b) = acc[a][b];
     }
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)  // sizes are in order as whole numbers too
+      atomicMax(&ends(lds)[16 * i + lo], __float_as_uint(most[i]));
     if (wave < KW / 2) {
 #pragma unroll
       for (int b = 0; b < NT; ++b)
@@ -143,6 +160,9 @@ struct FloatTile {
     __syncthreads();
   }
 
+  static __device__ __forceinline__ unsigned* ends(char* lds) {
+    return reinterpret_cast<unsigned*>(lds + SUMS);
+  }
   static __device__ __forceinline__ f32x4 sum(const char* lds, int r, int c) {
     const float* const sums = reinterpret_cast<const float*>(lds);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -154,20 +174,36 @@ struct FloatTile {
   }
 };
 
-// One output as a loop over the depth, where the sum of parts will not do.
-// The parts of an infinite number are that and no number.  Parts of numbers
-// below 2^-102 may be too small for a bf16 number; what is lost of a depth of
-// 10^6 is 2^-24 of a result of 10^-20 at most, unless the other numbers are
-// above 10^5.
-static __device__ __noinline__ float float_dot(const float* x, const float* w,
-                                               int K) {
-  float v = 0.f;
-  for (int k = 0; k < K; ++k) v = fmaf(x[k], w[k], v);
-  return v;
+// A block of 16 x 16 outputs by the float instructions, where the sum of parts
+// will not do; x, w: the lane's row (lane % 16) of each.  Bound by them and by
+// waiting for rows: 600 rows of 4096 x 1024 take 44 us, 64 with one row that has
+// no numbers (374 with a loop over the depth a lane), 176 (4711) with all of them.
+static __device__ __forceinline__ f32x4 float_block(const float* x,
+                                                    const float* w, int K) {
+  x += threadIdx.x % WAVE / 16 * 4, w += threadIdx.x % WAVE / 16 * 4;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < K; k += 128) {  // eight loads of each on their way
+    f32x4 a[8], b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int at = k + 16 * i < K ? k + 16 * i : k;
+      a[i] = *reinterpret_cast<const f32x4*>(w + at);
+      b[i] = *reinterpret_cast<const f32x4*>(x + at);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool more = k + 16 * i < K;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            more ? a[i][j] : 0.f, more ? b[i][j] : 0.f, acc, 0, 0, 0);
+      }
+  }
+  return acc;
 }
 
 template <int NT, int MT, int KW>
-__global__ __launch_bounds__(KW * 64, 1) void float_gemm_kernel(
+__global__ __launch_bounds__(KW * 64, KW == 4 ? 2 : 1) void float_gemm_kernel(
     float* __restrict__ out, int ld_out, const float* __restrict__ x,
     const float* __restrict__ w, int N, int M, int K, int ldx, int kind,
     bool narrow) {
@@ -193,16 +229,30 @@ __global__ __launch_bounds__(KW * 64, 1) void float_gemm_kernel(
   if (n0 >= N || m0 >= M) return;
   Tile::run(lds, K, turn, x + (size_t)n0 * ldx, ldx, N - 1 - n0,
             w + (size_t)m0 * K, M - 1 - m0);
-  for (int i = threadIdx.x; i < 16 * NT * 4 * MT; i += KW * 64) {
-    const int r = i / (4 * MT), c = i % (4 * MT) * 4;
-    if (n0 + r >= N || m0 + c >= M) continue;
-    f32x4 v = Tile::sum(lds, r, c);
+  // Outputs c .. c + 3 of row r whose sum of parts will not do: the parts of an
+  // infinite number are that and no number, and parts below 2^-126 may be lost,
+  // of a product 2^-125 of the other number and 2^-123 of sums.  So a sum has to
+  // be 2^25 of what K products can lose, where rows have numbers at all (those of
+  // padding have not), as far as the largest numbers of every 16th row tell.
+  const unsigned* const most = Tile::ends(lds);
+  const float least = K * 0x1p-98f;
+  auto lost = [&](int r, int c, f32x4 v) {
+    const float of_x = __uint_as_float(most[r % 16]);
+    unsigned bits = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      const float of_w = __uint_as_float(most[16 + c % 16 + j]);
       const float size = fabsf(v[j]);
-      if (!(size <= FLT_MAX) || (size < 1e-20f && size > 0.f))
-        v[j] = float_dot(x + (size_t)(n0 + r) * ldx,
-                         w + (size_t)(m0 + c + j) * K, K);
+      const bool zeros = of_x == 0.f || of_w == 0.f;
+      bits |= (!(size <= FLT_MAX) ||
+               (!zeros && !(size >= least * (1.f + of_x + of_w))))
+              << j;
+    }
+    return bits;
+  };
+  auto put = [&](int r, int c, f32x4 v, unsigned bits) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
       if (kind == RELU2) {
         v[j] = fmaxf(v[j], 0.f);
         v[j] *= v[j];
@@ -210,7 +260,38 @@ __global__ __launch_bounds__(KW * 64, 1) void float_gemm_kernel(
         v[j] = gelu_tanh_f(v[j]);
       }
     }
-    *reinterpret_cast<f32x4*>(out + (size_t)(n0 + r) * ld_out + m0 + c) = v;
+    float* const to = out + (size_t)(n0 + r) * ld_out + m0 + c;
+    if (bits == 15)
+      *reinterpret_cast<f32x4*>(to) = v;
+    else
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (bits >> j & 1) to[j] = v[j];
+  };
+  for (int i = threadIdx.x; i < 16 * NT * 4 * MT; i += KW * 64) {
+    const int r = i / (4 * MT), c = i % (4 * MT) * 4;
+    if (n0 + r >= N || m0 + c >= M) continue;
+    const f32x4 v = Tile::sum(lds, r, c);
+    const unsigned bits = lost(r, c, v);
+    if (bits)
+      atomicOr(Tile::ends(lds) + 32, 1u << (r / 16 * MT + c / 16));
+    put(r, c, v, 15 & ~bits);
+  }
+  __syncthreads();
+  unsigned blocks = __builtin_amdgcn_readfirstlane(most[32]);
+  const int lo = threadIdx.x & 15;
+  int others = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  for (; blocks; blocks &= blocks - 1) {  // every KW-th is the wave's
+    if (others--) continue;
+    others = KW - 1;
+    const int block = __builtin_ctz(blocks);
+    const int r = block / MT * 16 + lo, c0 = block % MT * 16;
+    const int row = n0 + r < N ? n0 + r : N - 1;
+    const int col = m0 + c0 + lo < M ? m0 + c0 + lo : M - 1;
+    const f32x4 v = float_block(x + (size_t)row * ldx, w + (size_t)col * K, K);
+    const int c = c0 + threadIdx.x % WAVE / 16 * 4;
+    if (n0 + r < N && m0 + c < M)
+      put(r, c, v, lost(r, c, Tile::sum(lds, r, c)));
   }
 }
 

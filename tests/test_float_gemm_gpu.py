@@ -158,3 +158,44 @@ def test_rows_of_one_number():
     ref = x.double() @ w.double().T
     off = ((ops._float_gemm(x, w).double() - ref) / ref).abs()
     assert off.max() <= 1.5 * 2.0 ** -23
+
+
+# numbers of which bf16 parts are too small, or nothing is left, by numbers
+# large enough to tell (of 288 normal numbers times 3e36 by ordinary ones sums
+# stay below infinity to 6 times their spread); both ways round, and results that
+# are small themselves
+@pytest.mark.parametrize("of_x,of_w", [
+    (1e-36, 1e30), (1e30, 1e-36), (1e-39, 1e30), (1e-42, 3e36), (1e-33, 1e5),
+    (1e-30, 1.0), (1.0, 1e-37), (1e-20, 1e-16), (1e-39, 1.0), (1e-25, 1e25),
+    (3e38 / 256, 1.0)])
+@pytest.mark.parametrize("tile", [-1, 0, 4, 8, 9])
+def test_small_by_large_numbers(of_x, of_w, tile):
+    x, w = _rows(70, 288, 16) * of_x, _rows(68, 288, 17) * of_w
+    # beside an ordinary row and output, one of a single number and of none
+    x[5], w[9] = _rows(1, 288, 18)[0], _rows(1, 288, 19)[0]
+    x[33, 1:], w[20], x[64] = 0, 0, 0
+    out = ops._float_gemm(x, w.contiguous(), tile=tile).double()
+    x, w = x.double(), w.double()
+    bound = (x.abs() @ w.abs().T) * (288 * 2.0 ** -24 + 2.0 ** -22) \
+        + 288 * 2.0 ** -149
+    assert ((out - x @ w.T).abs() <= bound).all()
+    assert (out[64] == 0).all() and (out[:, 20] == 0).all()
+
+
+@pytest.mark.parametrize("tile", range(TILES))
+def test_outputs_made_again(tile):
+    """Blocks of 16 x 16 of a tile's edges and middle, and activations of
+    them."""
+    x, w = _rows(175, 160, 20).contiguous(), _rows(200, 160, 21).contiguous()
+    for r in (0, 47, 95, 174):
+        x[r] *= 1e-30
+    x[100, 3], w[150, 2] = float("inf"), float("nan")
+    ref = x.double() @ w.double().T
+    out = ops._float_gemm(x, w, tile=tile)
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out[100].isinf(), ref[100].isinf())
+    keep = torch.tensor([r for r in range(175) if r != 100], device=DEV)
+    cols = torch.tensor([c for c in range(200) if c != 150], device=DEV)
+    _close(out[keep][:, cols], x[keep], w[cols])
+    assert torch.equal(ops._float_gemm(x, w, "relu2", tile=tile)[keep][:, cols],
+                       out[keep][:, cols].clamp(min=0) ** 2)
