@@ -374,6 +374,26 @@ static int float_tile(int N, int M, int K) {
   return best;
 }
 
+// Whether the library's product is the faster.  A tile's beginning and end are
+// most of a shallow product, of which there are many tiles; deep products of fewer
+// outputs than fill the chip it takes in shares of the depth.  The library's time
+// over this one's, means of 7 to 14 sizes each by depth and outputs:
+//   32: to 2^17.5 0.99, 2^18.5 0.93, 2^19 0.88, 2^20 0.65; 64: 1.04, 0.96, 0.86,
+//   0.75; 128: 1.19, 1.21, 1.30, 0.94, then 0.77; 256: 2^19 1.01, then 0.88, 0.91
+//   and to 2^22 0.96; 384: 1.02, 0.92, to 2^21 1.01; 512: 1.22, 0.94, 1.17; 640:
+//   1.01, 0.96, 1.18; more than 512 rows 128 deep 0.72
+//   4096: to 2^17 0.93, to 2^18 1.07; 8192 0.91, 1.08; 14336 0.88, 1.13; 3328 to
+//   2^16 0.97; 18304 1.6
+// The launch and pass of an activation's own kernel are more than that from 256 on.
+static bool library_gains(int N, int M, int K, int kind) {
+  const double outputs = (double)N * M;
+  if (K < 256 && N > 512) return true;
+  if (K >= 256 && kind != PLAIN) return false;
+  if (K >= 4096 && K <= 16384 && outputs < 1 << 17) return true;
+  return outputs > (K < 128 ? 1 << 18 : 1 << 19) &&
+         outputs * K * K <= 0x1p38;
+}
+
 // Rows of x start ldx numbers apart, those of out ld_out.  tile: -1, or the
 // one to take.  0: done, -2: not for this kernel.
 extern "C" int ll_float_gemm(void* out, int ld_out, const void* x,
@@ -384,9 +404,7 @@ extern "C" int ll_float_gemm(void* out, int ld_out, const void* x,
       (uintptr_t)out % 16 ||
       (kind != PLAIN && kind != RELU2 && kind != GELU))
     return -2;
-  // a tile's beginning and end are most of a shallow product (us, the library
-  // and here: 1600 rows, 1024 x 128 8.8 and 12.3, 1024 x 256 12.5 and 13.8)
-  if (tile < 0 && K < 256 && N > 512) return -2;
+  if (tile < 0 && library_gains(N, M, K, kind)) return -2;
   const FloatGemm p{(float*)out, ld_out, (const float*)x, (const float*)w,
                     N, M, K, ldx, kind, (hipStream_t)stream};
   switch (tile < 0 ? float_tile(N, M, K) : tile) {
