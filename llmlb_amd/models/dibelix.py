@@ -212,7 +212,9 @@ class DibelixForCausalLM(PackedCausalLM):
             hy.post_norm_add(x, xb, ly.mix(xb, b, cache, i), ly.norm1, eps,
                              self.norm_offset)
             if ly.ff is not None:
-                hy.post_norm_add(x, xb, ly.ff(xb, True), ly.norm2, eps,
+                # a module in its place is called as any other
+                ff = getattr(ly.ff, "rows_or_shares", ly.ff)
+                hy.post_norm_add(x, xb, ff(xb), ly.norm2, eps,
                                  self.norm_offset)
             if on_layer is not None:
                 on_layer(i, x)

@@ -25,6 +25,7 @@ from ..backend.kv_cache import StateSpec, PageSpec
 from ..ops import hybrid as hy
 from ..ops import (linear_act, linear_decode, linear_heads, linear_rows,
                    linear_shares, linear_two)
+from ..parallel.tp import _watched
 
 FULL_CONTEXT = 2 ** 30     # the window of an unmasked causal layer
 
@@ -287,20 +288,30 @@ class DenseFF(nn.Module):
         self.w_up = _param(F.pad(w["up"], (0, 0, 0, gap)).to(**to))
         self.w_down = _param(F.pad(w["down"], (0, gap)).to(**to))
 
-    def forward(self, x, shares: bool = False):
-        """``shares``: the caller also takes float shares of the product
-        (``linear_shares``) in rows of whole vectors."""
+    def forward(self, x):
         u = linear_act(x, self.w_up, self.act)
         if u is not None:
-            y = linear_shares(u, self.w_down) \
-                if shares and self.width % 8 == 0 else None
-            return _linear(u, self.w_down) if y is None else y
+            return _linear(u, self.w_down)
         u = _linear(x, self.w_up)
         if self.act == "gelu":
             hy.gelu_tanh_(u)
         else:
             hy.squared_relu(u, u)
         return _linear(u, self.w_down)
+
+    def rows_or_shares(self, x):
+        """``self(x)`` or, where calling the module is no more than its
+        products and a row is whole vectors, float shares of it
+        (``linear_shares``) for a caller that adds them up."""
+        if (self.width % 8 or _watched(self)
+                or getattr(self.forward, "__func__", None)
+                is not DenseFF.forward):
+            return self(x)
+        u = linear_act(x, self.w_up, self.act)
+        if u is None:
+            return self(x)
+        y = linear_shares(u, self.w_down)
+        return _linear(u, self.w_down) if y is None else y
 
 
 class DifferentialAttention(nn.Module):

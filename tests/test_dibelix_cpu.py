@@ -331,3 +331,26 @@ def test_heads_are_joined_by_one_copy():
     with Copies() as mode:
         run.step([(0, torch.randn(5, 40).double())])
     assert mode.seen == 1
+
+
+def test_feed_forwards_of_others(plain):
+    """A feed-forward's forward, or all of it, may be replaced by what takes
+    rows and returns rows."""
+    cfg, w, folder = plain
+    toks = U.tokens(19, cfg["vocab"], 6)
+    want = U.run_cuts(U.engine(folder), toks, [7, 8])
+
+    class Other(torch.nn.Module):
+        def __init__(self, ff):
+            super().__init__()
+            self.ff = ff
+
+        def forward(self, x):
+            return self.ff(x)
+
+    eng = U.engine(folder)
+    first, second = [ly.ff for ly in eng.model.layers_]
+    first.forward = lambda x, forward=first.forward: forward(x)
+    eng.model.layers_[1].ff = Other(second)
+    assert torch.equal(torch.as_tensor(U.run_cuts(eng, toks, [7, 8])),
+                       torch.as_tensor(want))

@@ -59,3 +59,22 @@ def test_other_products_are_not_in_shares():
     x = rand(8, 64, 14336).bfloat16()
     assert ops.linear_shares(x.float(), w.float()) is None
     assert ops.linear_shares(x, w.requires_grad_()) is None
+
+
+def test_hooks_see_rows():
+    """A watched or replaced feed-forward returns its rows, as others do."""
+    from llmlb_amd.models.mixers import DenseFF
+    ff = DenseFF(width=2048, ff=8192, dtype=torch.bfloat16, device=DEV)
+    ff.load({"up": rand(10, 8192, 2048) * 2048 ** -0.5,
+             "down": rand(11, 2048, 8192) * 8192 ** -0.5})
+    x = rand(12, 100, 2048).bfloat16()
+    want, shares = ff(x), ff.rows_or_shares(x)
+    assert want.dtype == x.dtype and shares.dim() == 3
+    seen = []
+    hook = ff.register_forward_hook(lambda m, args, out: seen.append(out))
+    assert torch.equal(ff.rows_or_shares(x), want)
+    assert torch.equal(seen[0], want)
+    hook.remove()
+    plain = ff.forward
+    ff.forward = lambda x: plain(x) * 2
+    assert torch.equal(ff.rows_or_shares(x), want * 2)
