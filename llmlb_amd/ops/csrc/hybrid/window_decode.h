@@ -41,15 +41,23 @@ __host__ inline bool window_decode_ok(const WindowDecode& a) {
 // quarter of the value columns.
 //   acc [N][H][parts][V], ml [N][H][parts] (maximum, sum); one part: the
 //   output itself
+// groups: how many workgroups there are
 // ONCE: no other workgroup reads the head's keys, which then go past the
 // caches and leave them to what the next kernels read: 8 layers of 61
 // sequences from 777 tokens, 32 heads of 128, 1382 -> 1354 us a step of the
 // model, of 64 sequences from 1024, 16 heads of 64, 507 -> 497.
 // Two tiles are on their way while one is worked on, which is why tiles come
-// in twos and past the last ones too, of one piece and without weights (loads
-// that come and go are not waited for by count): one tile ahead
+// in twos (loads that come and go are not waited for by count): one tile ahead
 // 8 layers' attention beside their experts' first products, 61 sequences, took
-// 78.8 us a layer, this way 74.9.
+// 78.8 us a layer, this way 74.9.  Heads of up to 64 gain by it only where units
+// have several workgroups of four tiles or more, whose keys nobody else reads;
+// larger ones than 128 have no registers for it.  us, one ahead, two ahead (of one
+// tile, with a second one without weights) and as chosen:
+//   heads     sequences, keys: 1, 64          1, 192         64, 192       64, 778
+//   128 x 128, 4 a key's     4.9, 5.6, 4.4  7.8, 8.0, 6.8  8.7, 8.9, 7.7  18.8, 16.1, 15.4
+//   64 x 64, 4 a key's       3.7, 5.2, 3.7  5.4, 7.0, 5.5  6.5, 7.6, 5.8  19.4, 17.2, 16.5
+//   32 x 32, 1 a key's       3.5, 4.6, 3.5  5.1, 6.2, 5.1  6.3, 7.7, 6.0  18.9, 17.5, 17.1
+//   256 x 256, 4 a key's     5.9, 8.1, 4.8  10.7, 12.1, 8.3  12.0, 14.3, 10.0  29.0, 29.0, 25.7
 template <int DQ, int DV>
 struct __align__(16) WindowLds {
   using St = Stage<1, DQ, DV>;
@@ -60,7 +68,8 @@ struct __align__(16) WindowLds {
 };
 template <int DQ, int DV, bool ONCE>
 __device__ __forceinline__ void window_decode_block(
-    const WindowDecode& a, int q, int y, int part, WindowLds<DQ, DV>& lds) {
+    const WindowDecode& a, int q, int y, int part, int groups,
+    WindowLds<DQ, DV>& lds) {
   constexpr int KD = DQ / 32, NV = DV / 64, PP = 64 + 8;
   using St = Stage<1, DQ, DV>;
   unsigned short *lk = lds.lk, *lv = lds.lv, *lp = lds.lp;
@@ -84,17 +93,27 @@ __device__ __forceinline__ void window_decode_block(
   const int t_hi = t_lo + per < tiles ? t_lo + per : tiles;
 
   St st(a.cache, a.bt + (size_t)a.row[q] * a.max_blocks, G, kv, D, V, pos);
-  // two tiles on their way
   u32x4 pk[2][St::KL], pv[2][St::VL];
   int pg[2][4];
-  auto fetch = [&](int t, int s) {
+  constexpr bool NEVER = DQ > 128 || DV > 128 || (!ONCE && DQ <= 64);
+  constexpr bool WIDE = DQ > 64 && DV > 64;
+  const int some = t_hi - t_lo;
+  const bool two =
+      !NEVER && (WIDE ? ONCE || some > 1 : groups >= 256 && some >= 4);
+  auto ask = [&](int t, int s) {
     st.template ask<ONCE>(pg[s], pk[s], pv[s], t < t_hi);
-    st.fetch_pages(lo + t * 64 + 128, pg[s]);
   };
   st.fetch_pages(lo + t_lo * 64, pg[0]);
-  st.fetch_pages(lo + t_lo * 64 + 64, pg[1]);
-  fetch(t_lo, 0);
-  fetch(t_lo + 1, 1);
+  if (two) {
+    st.fetch_pages(lo + t_lo * 64 + 64, pg[1]);
+    ask(t_lo, 0);
+    ask(t_lo + 1, 1);
+    st.fetch_pages(lo + t_lo * 64 + 128, pg[0]);
+    st.fetch_pages(lo + t_lo * 64 + 192, pg[1]);
+  } else {
+    ask(t_lo, 0);
+    st.fetch_pages(lo + t_lo * 64 + 64, pg[0]);
+  }
   u32x4 qf[KD];
 #pragma unroll
   for (int k = 0; k < KD; ++k) {
@@ -113,14 +132,14 @@ __device__ __forceinline__ void window_decode_block(
   float m = -1e30f, l = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto tile = [&](int t, int set) {
+  auto tile = [&](int t, int set, auto next) {
 #pragma unroll
     for (int i = 0; i < St::VL; ++i)  // hidden here, not where asked for
       asm volatile("" : "+v"(pv[set][i]));
     st.hide(lo + t * 64, pv[set], t < t_hi);
     St::store(lk, lv, pk[set], pv[set]);
     __syncthreads();
-    fetch(t + 2, set);
+    next(t, set);
     const int j = lo + t * 64 + wave * 16 + g * 4;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -165,9 +184,23 @@ __device__ __forceinline__ void window_decode_block(
     }
     __syncthreads();
   };
-  for (int t = t_lo; t < t_hi; t += 2) {
-    tile(t, 0);
-    tile(t + 1, 1);
+  if (two) {
+    auto next = [&](int t, int set) {
+      ask(t + 2, set);
+      st.fetch_pages(lo + t * 64 + 256, pg[set]);
+    };
+    for (int t = t_lo; t < t_hi; t += 2) {
+      tile(t, 0, next);
+      if (t + 1 >= t_hi) break;
+      tile(t + 1, 1, next);
+    }
+  } else {
+    for (int t = t_lo; t < t_hi; ++t)
+      tile(t, 0, [&](int t, int) {
+        if (t + 1 >= t_hi) return;
+        ask(t + 1, 0);
+        st.fetch_pages(lo + t * 64 + 128, pg[0]);
+      });
   }
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);

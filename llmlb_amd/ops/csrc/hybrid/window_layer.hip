@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256, 2) void window_up_kernel(
   if (b < attend) {
     const int q = b % n_rows, rest = b / n_rows;
     window_decode_block<DQ, DV, ONCE>(
-        a, q, rest % heads, rest / heads,
+        a, q, rest % heads, rest / heads, attend,
         *reinterpret_cast<WindowLds<DQ, DV>*>(lds));
     return;
   }

@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256, 2)
 void window_decode_kernel(WindowDecode a) {
   __shared__ WindowLds<DQ, DV> lds;
   window_decode_block<DQ, DV, ONCE>(a, blockIdx.x, blockIdx.y, blockIdx.z,
-                                    lds);
+                                    gridDim.x * gridDim.y * gridDim.z, lds);
 }
 
 // Join the parts and gate.  One wave a head; lane p first holds part p's
