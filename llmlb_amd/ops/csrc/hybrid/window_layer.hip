@@ -18,6 +18,10 @@
 //   64 tokens  64 experts, 8 a token                        92.5 ->  83.1
 //   64 tokens  1024 wide, 4 heads of 64, 256, from 500      27.5 ->  22.0
 //   1 token    the same, 32 experts of 512, from 100        18.5 ->  11.3
+// Tiles are those that both can have, so where a half's own kernel has much
+// better ones the halves stay apart: see apart_is_faster, and hybrid.few_layer.
+// Heads of 33 to 64 and of 97 to 128 (both sides, within their tiles) are those of
+// the models that are served; each further pair of sizes is four more kernels.
 #include "few_experts.h"
 #include "window_decode.h"
 
@@ -83,6 +87,25 @@ __global__ __launch_bounds__(256, 2) void down_out_kernel(FewRows a,
   few_block<OUT_MT>(f, b % down_tiles, b / down_tiles, lds, list);
 }
 
+// Whether the experts' second product and the output product, N x M and K deep,
+// take less in launches of their own.  A tile of 32 x 32 is as many rows of x as
+// of W, and by four waves: many tiles of more than 32 rows, which read W again,
+// lose to larger ones, the deepest to shares of the depth, and few deep ones
+// beside experts that are done long before to 16 x 16 by eight waves.  Both
+// launches' time over the one's (experts x their width, outputs, depth, rows):
+//   16 x 1280: 4096, 4096 deep 16 rows 1.09, 64 1.01, 96 0.95; 5376 1.11, 1.03,
+//       0.93; 8192 1.12, 0.95, 0.86; 6144, 2048 1.08, 1.01, 0.97; 4096 1.08, 0.96,
+//       0.92; 64 x 1280: 4096, 5376 1.08, 1.04, 1.01; 8192 1.08, 1.00, 0.98
+//   8 x 1536: 8192, 1024 1.05, 1.02, 0.97; 2048 1.04, 1.00, 0.95; 4096 1.05, 0.89
+//   16 x 512: 2048, 4096 1.27, 1.18, 1.15; 5376 1.21, 1.09, 1.10; 8192 1.11, 0.99
+//   16 x 256: 1024, 2048 1.32, 1.17, 1.32; 4096 1.08, 0.92; 64 x 256: 1.43, 1.24
+static bool apart_is_faster(int N, int M, int K, int E, int F) {
+  if (K > 3ll * M && (long long)E * F < 3ll * K) return true;
+  if (N <= 32) return false;
+  const long long tiles = (M + 31ll) / 32 * ((N + 31) / 32);
+  return K >= 8192 || tiles >= 768 || tiles * K > 1400000;
+}
+
 extern "C" {
 
 int hy_expert_few_tile(int E, int N, int K, int n_pairs);
@@ -138,7 +161,7 @@ int hy_window_up(void* out, int ld_out, void* acc, void* ml, const void* proj,
   return rc ? rc : 1;
 }
 
-// 1: done; < 0: an error
+// 1: done; 0: sizes that take the separate kernels; < 0: an error
 int hy_down_out(void* out, const void* x, const void* w, int N, int M, int K,
                 void* z, const void* u, const void* w_down, const void* index,
                 int E, int W, int F, int n_pairs, void* stream) {
@@ -148,6 +171,7 @@ int hy_down_out(void* out, const void* x, const void* w, int N, int M, int K,
   if (!few_ok(f) || N <= 0 || M <= 0 || K <= 0 || M % 4 || K % 8 ||
       ((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)out % 8)
     return -2;
+  if (apart_is_faster(N, M, K, E, F)) return 0;
   const int tiles = (W + 16 * OUT_MT - 1) / (16 * OUT_MT);
   const int m_tiles = (M + 16 * OUT_MT - 1) / (16 * OUT_MT);
 #define GO(NT)                                                               \

@@ -852,9 +852,12 @@ def window_attention(out, proj, g_off, heads, kv_heads, dim, vdim, cache, b,
 def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
     """``window_attention(*window)``, ``experts`` of ``h`` and the product
     mid @ w_out^T of a parallel layer's single tokens, independent parts in
-    the same launch: (product, experts' outputs).  None where nothing is
-    done: more tokens, other sizes, what other kernels or the library
-    take."""
+    the same launch where that is faster (window_layer.hip): (product,
+    experts' outputs).  None where nothing is done: more tokens, other
+    sizes, and few keys beside experts with 16 pairs or more each whose own
+    kernel has larger tiles (16 experts of 4096 x 1280, both launches' time
+    over the one's: 64 tokens of up to 60 keys 0.95, 300 1.03; 128 tokens
+    0.85, 0.93, 1000 1.03)."""
     out, proj, g_off, H, G, D, V, cache, b, size, *chunk = window
     n, top = index.shape
     E, F, W = w_up.shape
@@ -869,6 +872,11 @@ def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
             or not w_out.is_contiguous()
             or (mid.data_ptr() | w_out.data_ptr()) % 16):
         return None
+    lib, bt, st = native(), b.block_tables, _stream()
+    keys, each = min(size, b.max_keys), n * top / E
+    if (each >= 16 and keys < (128 if each < 24 else 768)
+            and lib.hy_expert_few_tile(_i(E), _i(F), _i(W), _i(n * top)) > 2):
+        return None
     product = ops._product_of(mid, w_out, "plain", None, 0)
     if product is None:
         return None
@@ -876,8 +884,7 @@ def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
         and h.is_contiguous() and w_up.is_contiguous() \
         and w_down.is_contiguous() and w_down.shape == (E, W, F) \
         and h.shape == (n, W) and cache.shape[0] * G * 16 < 2 ** 31
-    lib, bt, st = native(), b.block_tables, _stream()
-    parts = window_parts(n, G, H // G, min(size, b.max_keys))
+    parts = window_parts(n, G, H // G, keys)
     acc = ml = None
     if parts > 1:
         acc = torch.empty(n, H, parts, V, dtype=torch.float32,
@@ -894,15 +901,22 @@ def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
         _i(W), _i(top), st)
     if done == 0:
         return None
+    if done != 1:
+        _check(done, "hy_window_up")
     z = torch.empty(n, top, W, dtype=h.dtype, device=h.device)
     M, y = product
-    if done == 1:
-        done = lib.hy_down_out(
-            _ptr(y), _ptr(mid), _ptr(w_out), _i(n), _i(M), _i(mid.shape[1]),
-            _ptr(z), _ptr(u), _ptr(w_down), _ptr(index), _i(E), _i(W), _i(F),
-            _i(n * top), st)
+    done = lib.hy_down_out(
+        _ptr(y), _ptr(mid), _ptr(w_out), _i(n), _i(M), _i(mid.shape[1]),
+        _ptr(z), _ptr(u), _ptr(w_down), _ptr(index), _i(E), _i(W), _i(F),
+        _i(n * top), st)
+    if done == 0:
+        _check(lib.hy_expert_few(_ptr(z), _ptr(u), _ptr(w_down), _ptr(index),
+                                 _i(E), _i(W), _i(F), _i(1), _i(0),
+                                 _i(n * top), _i(FEW_TILE), st),
+               "hy_expert_few")
+        return ops.linear_decode(mid, w_out), z
     if done != 1:
-        _check(done or -1, "hy_window_up, hy_down_out")
+        _check(done, "hy_down_out")
     return y, z
 
 

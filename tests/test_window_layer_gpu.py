@@ -125,3 +125,22 @@ def test_captured():
         for a, b in zip(got, want):
             assert torch.equal(a, b)
         ops.linear_decode(args[6], args[7])
+
+
+# output products with launches of their own: deep for their width beside short
+# experts, 8192 deep, and of many tiles
+@pytest.mark.parametrize("W, ff, shared, E, n", [
+    (72, 40, 1000, 4, 5), (128, 64, 8192, 16, 40), (4096, 64, 5632, 4, 70)])
+def test_products_apart(W, ff, shared, E, n):
+    check(operands(n, W, 4, 2, 64, 64, ff, shared, E, 2, 150, 64, False))
+
+
+def test_few_keys_beside_large_tiles_of_experts():
+    """16 pairs an expert, whose own kernel has tiles of 80 outputs."""
+    sizes = (2048, 4, 2, 64, 64, 1040, 0, 16, 4)
+    for n, ctx, size, taken in ((64, 60, 4096, False), (64, 300, 100, False),
+                                (64, 300, 4096, True), (60, 60, 4096, True),
+                                (100, 700, 4096, False),
+                                (100, 800, 4096, True)):
+        args = operands(n, *sizes, ctx, size, False)
+        assert (hy.few_layer(*args) is not None) == taken
