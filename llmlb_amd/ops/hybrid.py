@@ -523,12 +523,18 @@ def _gated_norm(out, y, gate, g_off, w, groups, gate_first: bool, eps,
 
 def decays_in_step(proj, low_off, w_low, dim, b) -> bool:
     """Whether a step's kernel makes the decays' projection itself: a
-    token a sequence, loads of eight numbers on 16 bytes, and at most
-    4096 weights a head, which are two loads a lane.  In four layers with
-    heads of 64 channels and rank 64 a step takes less than with a launch
-    of their own (1 token: 206 us to 199; 64: 328 to 320), and with 128
-    and rank 128 more (2 tokens: 789 to 793; 64: 1324 to 1336)."""
+    token a sequence, loads of eight numbers on 16 bytes, at most 4096
+    weights a head, which are two loads a lane, and products that are not
+    asked of the library.  us, a launch of their own and this, for 1 and 64
+    tokens, 16 heads in 16 bits: 64 channels and rank 32 6.3 and 4.5, 10.5
+    and 8.1; 64 6.3 and 4.6, 10.3 and 8.2; 32 and 128 6.2 and 4.5, 9.9 and
+    8.3; 128 and 32 7.1 and 5.9, 29.0 and 27.1; 256 and 16 8.2 and 8.0, 52.6
+    and 51.7.  Alone 128 and 128 gains as well (29.3 and 27.4), but in a
+    model's step, where the launch is hidden better, it loses 0.9 to 2.8 a
+    layer (2 tokens: 789 to 793 for four; 64: 1324 to 1336); what lies
+    between was not measured there."""
     return b.decode and proj.is_cuda and w_low.dtype == proj.dtype \
+        and ops._USE_CUSTOM_DECODE_GEMM == "auto" \
         and w_low.is_contiguous() and proj.stride(1) == 1 \
         and dim * w_low.shape[1] <= 4096 \
         and (w_low.shape[1] | low_off | proj.stride(0)) % 8 == 0 \

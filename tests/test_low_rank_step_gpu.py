@@ -85,3 +85,13 @@ def test_unfit_operands_keep_their_launch():
     assert not hy.decays_in_step(proj, 16, w, 264, b)
     b.decode = False
     assert not hy.decays_in_step(proj, 16, w, 16, b)
+
+
+@pytest.mark.parametrize("mode", ["0", "off", "1"])
+def test_the_librarys_product_where_it_is_asked_for(mode, monkeypatch):
+    import llmlb_amd.ops as ops
+    proj = torch.zeros(2, 64, dtype=B16, device=DEV)
+    w = torch.zeros(16, 16, dtype=B16, device=DEV)
+    assert hy.decays_in_step(proj, 16, w, 16, batch(2, DEV))
+    monkeypatch.setattr(ops, "_USE_CUSTOM_DECODE_GEMM", mode)
+    assert not hy.decays_in_step(proj, 16, w, 16, batch(2, DEV))
