@@ -182,19 +182,26 @@ def rope_kv_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     _check(rc, "ll_rope_kv_append")
 
 
-def norms_rows(x: torch.Tensor) -> bool:
-    """Whether a product may norm rows of this shape itself
-    (linear_normed)."""
-    return x.dim() == 2 and x.shape[0] <= 4 and x.numel() <= 4096
+def norms_rows(x: torch.Tensor, outputs: int = 1) -> bool:
+    """Whether a product of this many rows of weights, or any, norms rows of
+    this shape itself (linear_normed): the rule of row_gemm.hip."""
+    if x.dim() != 2:
+        return False
+    N, K = x.shape
+    if N == 1:
+        return K <= 512 or (K <= 2048 and outputs <= 48 * 1024)
+    return N <= 4 and K <= 1024 and outputs <= 16 * 1024
 
 
-def _norm_operands(x: torch.Tensor, norm: tuple):
-    """(arguments, x + residual or None) of a product that norms its rows by
-    ``norm`` (weight, eps, residual or None); None where it does not."""
+def _norm_operands(x: torch.Tensor, outputs: int, norm: tuple):
+    """(arguments, x + residual or None) of a product with ``outputs`` rows
+    of weights that norms its rows by ``norm`` (weight, eps, residual or
+    None); None where it does not."""
     weight, eps, residual = norm
     K = x.shape[1]
-    if (not norms_rows(x) or K % 64 or not x.is_contiguous() or weight.shape != (K,)
-            or weight.dtype != x.dtype or weight.device != x.device
+    if (not norms_rows(x, outputs) or K % 64 or not x.is_contiguous()
+            or weight.shape != (K,) or weight.dtype != x.dtype
+            or weight.device != x.device
             or not weight.is_contiguous() or not _only_numbers(weight)):
         return None
     if residual is None:
@@ -242,7 +249,7 @@ def linear_rotary(x: torch.Tensor, weight: torch.Tensor, n_q: int,
             kcache.shape[2]
     total, normed = None, (None, None, None, ctypes.c_float(0.0))
     if norm is not None:
-        found = _norm_operands(x, norm)
+        found = _norm_operands(x, M, norm)
         if found is None:
             return None
         normed, total = found
@@ -265,9 +272,10 @@ def linear_normed(x: torch.Tensor, weight: torch.Tensor, norm: tuple,
     ``norm`` as for linear_rotary, act "plain" or "swiglu" (as for
     linear_act); None where row_gemm.hip does not take it."""
     if (_USE_CUSTOM_DECODE_GEMM != "auto" or act not in ("plain", "swiglu")
-            or not norms_rows(x) or not _takes_row_gemm(x, weight)):
+            or not norms_rows(x, weight.shape[0])
+            or not _takes_row_gemm(x, weight)):
         return None
-    found = _norm_operands(x, norm)
+    found = _norm_operands(x, weight.shape[0], norm)
     if found is None:
         return None
     normed, total = found

@@ -649,16 +649,21 @@ extern "C" int ll_row_gemm_two(void* out1, int ld_out1, const void* x1,
 }
 
 // Whether a product norms its rows itself: every workgroup does all of them, so
-// few, and of more than one not where workgroups come in rounds.  us, both
-// launches -> this:
+// few, and not where workgroups come in rounds (of one row, in several, unless
+// its norm is next to nothing).  us, both launches -> this:
 //   1 row: 1536 x 1024 5.5 -> 4.9, gate and up of 5632 x 1024 6.9 -> 5.8, 32000 x
 //       1024 14.6 -> 13.9, 3072 x 2048 7.0 -> 6.6, gate and up of 11264 x 2048
 //       11.7 -> 11.2, 6144 x 4096 13.0 -> 13.7
+//   1 row of many outputs: 49152 x 1024 20.4 -> 20.1, 98304 34.6 -> 35.4, 152064
+//       49.8 -> 51.0; 49152 x 1536 27.2 -> 27.1, 65536 34.5 -> 35.1, 152064 72.3 ->
+//       74.4; 49152 x 2048 34.3 -> 34.2, 98304 63.2 -> 64.0; 152064 x 512 32.2 ->
+//       31.2; between rounds 22528 x 2048 18.6 -> 19.4
 //   2 rows: 5.8 -> 4.9, 7.0 -> 6.2, 14.4 -> 14.7, 6.9 -> 7.3, 11.8 -> 11.6
 //   4 rows: 5.8 -> 5.3, 7.1 -> 6.5, 14.6 -> 15.2; 6: 6.0 -> 5.8, 7.3 -> 7.8
+// rows: of W.  ops.norms_rows is the same rule.
 static bool norm_gains(int N, int rows, int K) {
-  return (N == 1 && K <= 2048) ||
-         (N <= 4 && K <= 1024 && rows <= 512 * 32);
+  if (N == 1) return K <= 512 || (K <= 2048 && rows <= 48 * 1024);
+  return N <= 4 && K <= 1024 && rows <= 16 * 1024;
 }
 
 static bool norm_fits(const void* x, const void* residual, const void* sum,
