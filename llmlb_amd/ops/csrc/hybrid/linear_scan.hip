@@ -254,14 +254,23 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(
         extra + ((size_t)e_row[e] * H + head) * extra_row(D), r0, D, N);
 }
 
-// The same with one column a lane and whole vectors, for few sequences: half the SIMDs or more
-// have no wave then, and a wave's own instructions bound it, so that whatever
+// The same with one column a lane and whole vectors, for few sequences: fewer
+// than two waves a SIMD, whose own instructions bound them, so that whatever
 // is the same for a column, or one number a token, is done for 16 tokens at
 // once, a token a lane: their values, decays and steps are asked for in one
 // load each and broadcast, their outputs are finished and stored together.
 // That also leaves the 63 loads that a wave can count to the queries and keys.
-// A load of each a token -> this: 2 sequences of 300 tokens, 16 heads of 64 by
-// 64 in 32 bits, matrix memory 56.9 us -> 40.9 (190 ns a token -> 136).
+// Entries of 300 tokens, us, a load of each a token -> this (the same bits):
+//   heads x D x V     waves   gated linear          Mamba-2         matrix memory
+//   16 64 64   bf16    512   40.0 -> 36.4     37.5 -> 30.7     57.2 -> 41.4
+//                     1024   40.1 -> 36.5     38.2 -> 31.4     58.0 -> 41.3
+//                     1792   68.5 -> 63.7     62.4 -> 53.3     81.1 -> 63.1
+//              f32     512   38.7 -> 35.3     35.0 -> 30.5     55.4 -> 40.0
+//                     1792   68.1 -> 64.0     63.1 -> 54.2    112.8 -> 63.3
+//   8 128 128  bf16   1024   49.8 -> 46.3     58.5 -> 41.0     73.0 -> 57.4
+//                     1792   82.0 -> 80.9     72.7 -> 59.9    103.0 -> 84.0
+//              f32    1792  140.7 -> 115      92.4 -> 84.8    104.0 -> 94.4
+//   16 16 16   bf16   1984   44.2 -> 32.8     43.7 -> 31.8     63.5 -> 38.4
 template <class F, int... U>
 __device__ __forceinline__ void for_each(std::integer_sequence<int, U...>,
                                          F f) {

@@ -57,3 +57,43 @@ def test_unequal_lengths_together():
     got = run.step(list(enumerate(hs)))
     for i, h in enumerate(hs):
         check(got[i], oracle(h, w, "", m, 1e-5))
+
+
+# 512, 1024 and 1984 waves of the 2047 at most
+@pytest.mark.parametrize("kind", ["channel", "head", "memory"])
+@pytest.mark.parametrize("E, H, D, V", [(3, 2, 16, 16), (2, 16, 64, 64),
+                                        (4, 8, 128, 128), (31, 16, 32, 16)])
+def test_sixteen_bits(kind, E, H, D, V):
+    """The same numbers in either type: all sums are of floats in the same
+    order, but a product may be rounded before it is added or not, 33 + D
+    times 2^-24 at most, 1e-5."""
+    from llmlb_amd.ops import hybrid as hy
+    from llmlb_amd.ops.hybrid import _f, _i, _p, _ptr, _stream
+    g = torch.Generator(device=DEV).manual_seed(D + E)
+    rand = lambda *s: torch.rand(*s, generator=g, device=DEV)
+    lens = [(1, 15, 16, 17, 33)[i % 5] for i in range(E)]
+    T, ld = sum(lens), 2 * H * D + H * V
+    rows = (2 * rand(T, ld) - 1).bfloat16()
+    decay = 0.9 + 0.1 * rand(T, H * (D if kind == "channel" else 1))
+    dt = None if kind == "channel" else rand(T, H)
+    skip = None if kind == "channel" else 0.5 + rand(T, H)
+    n0 = rand(E, H, D) if kind == "memory" else None
+    ints = lambda l: torch.tensor(l, dtype=torch.int32, device=DEV)
+    runs = (ints([sum(lens[:i]) for i in range(E)]), ints(lens),
+            ints([i % 2 for i in range(E)]), ints(list(range(E))[::-1]))
+    first = rand(E, H, V, D)
+    got = []
+    for x in (rows, rows.float()):
+        o, state = torch.zeros(T, H * V, device=DEV), first.clone()
+        extra = torch.zeros(E, H, hy.memory_extra(D), device=DEV)
+        rc = hy.native().hy_linear_scan(
+            _ptr(o), _ptr(state), _ptr(x), _i(ld), _i(0), _i(H * D),
+            _i(2 * H * D), _ptr(decay), _p(dt), _p(skip), *map(_ptr, runs),
+            _i(E), _i(H), _i(H), _i(D), _i(V), _f(D ** -0.5), _p(n0),
+            _ptr(extra) if kind == "memory" else None, hy._dt(x.dtype),
+            _stream())
+        assert rc == 0
+        got.append((o, state, extra))
+    for a, b in zip(*got):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+    assert got[0][0].abs().max() > 0
