@@ -391,8 +391,9 @@ static int row_gemm_launch(const RowGemm<End>& p) {
 // than whole rounds say: another than 32 outputs has to take in 15% less (one
 // row of 20480 x 1024 11.0 with 48, 10.1 with 32; 16512 x 1024 9.2 with 32, 8.6
 // with 80).
+// takes_in: rows that the busiest unit takes in, in 16s
 static int row_gemm_tile(int N, long long rows, int K, bool paired,
-                         long long beside = 0) {
+                         long long beside = 0, float* takes_in = nullptr) {
   const int tiles = (N + 15) / 16;
   // what memory takes for W, in the same unit: 16 rows at 50 GB/s
   const float floor = (rows + beside) / 2500.f;
@@ -422,6 +423,7 @@ static int row_gemm_tile(int N, long long rows, int K, bool paired,
       // them, 2.8 with 16; 1024 x 768 3.4, 3.7)
       if ((n < 3 || m > 1) && (!paired || m > 1 || K > 256)) look(n, m);
     }
+  if (takes_in) *takes_in = least;
   return nt * 8 + mt;
 }
 
@@ -469,6 +471,12 @@ static int row_gemm_pick(const RowGemm<End>& p) {
 //   1: 4160, 2176 of 1024 9.0 -> 6.3, 8320, 4352 of 2048 15.8 -> 13.1, 16512,
 //       11904 of 4096 52.4 -> 48.1; 64: 12.0 -> 8.2, 24.1 -> 17.2, 61.6 -> 60.2;
 //       128: 14.5 -> 10.1, 29.5 -> 27.9, 103.4 -> 99.4
+// Where one tile for both takes in so much more than each product's own that the
+// launch is not worth it (3 us at 50 GB/s), they stay apart: 72, 100 and 128 rows
+// of 8192, 6144 of 4096 47.1 -> 50.8, 51.3 -> 55.2, 50.6 -> 54.4, of 6144, 4096 of
+// 6144 57.6 -> 60.9, 62.9 -> 65.0, 60.6 -> 62.6; 64 of 1024, 14336 of 4096 46.5 ->
+// 48.2.  Of 150 other sizes three lose in one launch, 0.2 to 2.5%, which all lie
+// beyond this line, as do two that gain 0.1 and 1.7%.
 struct RowGemmTwo {
   RowOperands a, b;
   PlainEnd a_end;
@@ -639,7 +647,12 @@ extern "C" int ll_row_gemm_two(void* out1, int ld_out1, const void* x1,
       N,
       K,
       (hipStream_t)stream};
-  switch (row_gemm_tile(N, M1, K, true, 2ll * M2)) {
+  float both, first, second;
+  const int tile = row_gemm_tile(N, M1, K, true, 2ll * M2, &both);
+  row_gemm_tile(N, M1, K, false, 0, &first);
+  row_gemm_tile(N, 2ll * M2, K, true, 0, &second);
+  if ((both - first - second) * K > 4700.f) return -2;
+  switch (tile) {
 #define GO(NT, MT, KW, S) \
   case NT * 8 + MT: return row_gemm_two_launch<NT, MT, KW, S>(p);
     ROW_GEMM_TILES(GO)
