@@ -173,11 +173,13 @@ __global__ __launch_bounds__(THREADS) void post_norm_join_kernel(
 // sum alone.  ROUTED: x += mult (y + sum over k of zw[k] z[k]) with ``top``
 // more rows z of the token.  ONE: w1 and w2 are single numbers.  One
 // workgroup per row, of which KEEP vectors a thread stay in registers between
-// the passes; a few rows' time is a chain of loads, so their weights are asked
-// for with them.  us, weights after the norm and always room for four -> this:
-// 64 rows of 4096, two norms 4.18 -> 3.84, with 4 routed rows 4.66 -> 3.99; of 1024
-// 3.07 -> 2.78, 3.33 -> 2.88; 16384 of 4096 184 -> 181, 249 -> 246.  (post_norm_add
-// and post_pre_norm gained nothing by it.)
+// the passes; a few rows' time is a chain of loads, so that up to 4096 columns
+// their weights are asked for with them.  (Wider rows have too few registers left:
+// 1000 rows of 5120 with 4 routed rows 20.1 us, 23.8 with their weights early,
+// 19.6 as here; 64 of 5120 7.6, 7.4, 6.4.)  us, weights after the norm and always
+// room for four -> this: 64 rows of 4096, two norms 4.18 -> 3.84, with 4 routed
+// rows 4.66 -> 3.99; of 1024 3.07 -> 2.78, 3.33 -> 2.88; 16384 of 4096 184 -> 181,
+// 249 -> 246.  (post_norm_add and post_pre_norm gained nothing by it.)
 template <typename T, bool ROUTED, bool ONE, int KEEP>
 __global__ __launch_bounds__(256) void add_norms_kernel(
     float* __restrict__ x, const T* __restrict__ y,
@@ -192,9 +194,10 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
   }
   const bool vec = (width & 7) == 0;
   const int nvec = vec ? width >> 3 : 0;
+  constexpr bool WEIGHTS = !ONE && KEEP <= 2;
   float keep[KEEP][8], w1k[KEEP][8], w2k[KEEP][8];
   float ssq = 0.f;
-  if (!ONE && w1) {
+  if (WEIGHTS && w1) {
 #pragma unroll
     for (int n = 0; n < KEEP; ++n) {
       const int i = threadIdx.x + n * 256;
@@ -264,7 +267,12 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
 #pragma unroll
   for (int n = 0; n < KEEP; ++n) {
     const int i = threadIdx.x + n * 256;
-    if (i < nvec) emit(i, keep[n], w1k[n], w2k[n]);
+    if (i >= nvec) continue;
+    if (!ONE && !WEIGHTS) {
+      load8(w1 + i * 8, w1k[n]);
+      if (w2) load8(w2 + i * 8, w2k[n]);
+    }
+    emit(i, keep[n], w1k[n], w2k[n]);
   }
   // a thread reads back only what it wrote itself
   for (int i = threadIdx.x + KEEP * 256; i < nvec; i += 256) {
