@@ -472,11 +472,13 @@ static int row_gemm_pick(const RowGemm<End>& p) {
 //       11904 of 4096 52.4 -> 48.1; 64: 12.0 -> 8.2, 24.1 -> 17.2, 61.6 -> 60.2;
 //       128: 14.5 -> 10.1, 29.5 -> 27.9, 103.4 -> 99.4
 // Where one tile for both takes in so much more than each product's own that the
-// launch is not worth it (3 us at 50 GB/s), they stay apart: 72, 100 and 128 rows
-// of 8192, 6144 of 4096 47.1 -> 50.8, 51.3 -> 55.2, 50.6 -> 54.4, of 6144, 4096 of
-// 6144 57.6 -> 60.9, 62.9 -> 65.0, 60.6 -> 62.6; 64 of 1024, 14336 of 4096 46.5 ->
-// 48.2.  Of 150 other sizes three lose in one launch, 0.2 to 2.5%, which all lie
-// beyond this line, as do two that gain 0.1 and 1.7%.
+// launch is not worth it (3 us at 50 GB/s, of up to 16 rows, which memory bounds,
+// 3.6), they stay apart: 72, 100 and 128 rows of 8192, 6144 of 4096 47.1 -> 50.8,
+// 51.3 -> 55.2, 50.6 -> 54.4, of 6144, 4096 of 6144 57.6 -> 60.9, 62.9 -> 65.0, 60.6
+// -> 62.6; 64 of 1024, 14336 of 4096 46.5 -> 48.2; 1 and 16 of 16384, 5632 of 6144
+// 56.0 -> 56.6, 57.5 -> 59.3, but of 10240, 11904 of 4096, which take in just less,
+// 48.4 -> 47.5, 49.6 -> 49.2.  Of 150 other sizes three lose in one launch, 0.2 to
+// 2.5%, which all lie beyond this line, as do two that gain 0.1 and 1.7%.
 struct RowGemmTwo {
   RowOperands a, b;
   PlainEnd a_end;
@@ -651,7 +653,7 @@ extern "C" int ll_row_gemm_two(void* out1, int ld_out1, const void* x1,
   const int tile = row_gemm_tile(N, M1, K, true, 2ll * M2, &both);
   row_gemm_tile(N, M1, K, false, 0, &first);
   row_gemm_tile(N, 2ll * M2, K, true, 0, &second);
-  if ((both - first - second) * K > 4700.f) return -2;
+  if ((both - first - second) * K > (N <= 16 ? 5700.f : 4700.f)) return -2;
   switch (tile) {
 #define GO(NT, MT, KW, S) \
   case NT * 8 + MT: return row_gemm_two_launch<NT, MT, KW, S>(p);

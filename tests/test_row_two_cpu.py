@@ -15,6 +15,7 @@ import llmlb_amd.ops as ops
     (72, 8192, 6144, 4096, False), (128, 8192, 6144, 4096, False),
     (128, 8192, 6144, 2048, True), (72, 6144, 4096, 6144, False),
     (64, 1024, 14336, 4096, False), (64, 1024, 14336, 1024, True),
+    (16, 10240, 11904, 4096, True), (16, 16384, 5632, 6144, False),
     (64, 4160, 2176, 1024, True), (128, 16512, 11904, 4096, True)])
 def test_one_tile_for_both(N, M1, M2, K, together):
     at, i, f = ctypes.c_void_p(4096), ctypes.c_int, ctypes.c_float
