@@ -860,10 +860,12 @@ def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
     mid @ w_out^T of a parallel layer's single tokens, independent parts in
     the same launch where that is faster (window_layer.hip): (product,
     experts' outputs).  None where nothing is done: more tokens, other
-    sizes, and few keys beside experts with 16 pairs or more each whose own
-    kernel has larger tiles (16 experts of 4096 x 1280, both launches' time
-    over the one's: 64 tokens of up to 60 keys 0.95, 300 1.03; 128 tokens
-    0.85, 0.93, 1000 1.03)."""
+    sizes, and beside experts with 16 pairs or more each whose own kernel
+    has larger tiles, if keys are few or, of 24 pairs on, whatever they are
+    (a captured step does not know them).  16 experts of 4096 x 1280, both
+    launches' time over the one's: 64 tokens of up to 60 keys 0.95, 300
+    1.03; 128 tokens 0.85, 0.93, 1000 1.03; steps of the model with 96
+    tokens after 100 keys 0.96, 500 1.00."""
     out, proj, g_off, H, G, D, V, cache, b, size, *chunk = window
     n, top = index.shape
     E, F, W = w_up.shape
@@ -880,7 +882,7 @@ def few_layer(window, h, index, lists, w_up, w_down, mid, w_out):
         return None
     lib, bt, st = native(), b.block_tables, _stream()
     keys, each = min(size, b.max_keys), n * top / E
-    if (each >= 16 and keys < (128 if each < 24 else 768)
+    if (each >= 16 and (keys < 128 or each >= 24)
             and lib.hy_expert_few_tile(_i(E), _i(F), _i(W), _i(n * top)) > 2):
         return None
     product = ops._product_of(mid, w_out, "plain", None, 0)

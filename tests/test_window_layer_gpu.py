@@ -135,12 +135,13 @@ def test_products_apart(W, ff, shared, E, n):
     check(operands(n, W, 4, 2, 64, 64, ff, shared, E, 2, 150, 64, False))
 
 
-def test_few_keys_beside_large_tiles_of_experts():
-    """16 pairs an expert, whose own kernel has tiles of 80 outputs."""
+def test_large_tiles_of_experts():
+    """16 pairs an expert and few keys, or 24, where their own kernel has
+    tiles of 80 outputs."""
     sizes = (2048, 4, 2, 64, 64, 1040, 0, 16, 4)
     for n, ctx, size, taken in ((64, 60, 4096, False), (64, 300, 100, False),
                                 (64, 300, 4096, True), (60, 60, 4096, True),
-                                (100, 700, 4096, False),
-                                (100, 800, 4096, True)):
+                                (95, 800, 4096, True),
+                                (96, 800, 4096, False)):
         args = operands(n, *sizes, ctx, size, False)
         assert (hy.few_layer(*args) is not None) == taken
