@@ -20,7 +20,7 @@ from ..backend.ragged import RaggedBatch
 from ..ops import hybrid as hy
 from ..ops.reference import build_cos_sin_table
 from ..parallel.tp import TPContext
-from .mixers import ChannelDelta, DenseFF, LatentAttention
+from .mixers import ChannelDelta, DenseFF, LatentAttention, for_norm
 from .packed import PackedCausalLM, read_folder
 
 
@@ -209,12 +209,10 @@ class DibelixForCausalLM(PackedCausalLM):
         eps = self.cfg.eps
         x, xb = hy.embed_rows(self.embed, b.ids)
         for i, ly in enumerate(self.layers_):
-            hy.post_norm_add(x, xb, ly.mix(xb, b, cache, i), ly.norm1, eps,
-                             self.norm_offset)
+            hy.post_norm_add(x, xb, for_norm(ly.mix)(xb, b, cache, i),
+                             ly.norm1, eps, self.norm_offset)
             if ly.ff is not None:
-                # a module in its place is called as any other
-                ff = getattr(ly.ff, "rows_or_shares", ly.ff)
-                hy.post_norm_add(x, xb, ff(xb), ly.norm2, eps,
+                hy.post_norm_add(x, xb, for_norm(ly.ff)(xb), ly.norm2, eps,
                                  self.norm_offset)
             if on_layer is not None:
                 on_layer(i, x)

@@ -393,7 +393,7 @@ class LlamaForCausalLM(nn.Module):
         """o_proj -> +residual -> norm -> mlp.  Returns (h, residual)."""
         layer = self.layers_[layer_idx]
         T = attn_out.shape[0]
-        o = None
+        o = shares = None
         if (quant_ok and ops.w8a8_active() and attn_out.is_cuda
                 and T <= 128 and attn_out.dtype == torch.bfloat16):
             # o_proj joins the quantized path: one standalone row
@@ -406,7 +406,11 @@ class LlamaForCausalLM(nn.Module):
                 if o is not None:
                     # RowParallelLinear: the mixin GEMM is shard-local
                     o = layer.o_proj.tp.all_reduce(o)
-        if o is None:
+        elif not ops.norms_rows(residual):
+            fused = getattr(layer.o_proj, "forward_shares", None)
+            shares = fused(attn_out.reshape(T, -1)) \
+                if fused and residual.is_contiguous() else None
+        if o is None and shares is None:
             o = layer.o_proj(attn_out.reshape(T, -1))
         if (quant_ok and ops.w8a8_active() and o.is_cuda and T <= 128
                 and o.dtype == torch.bfloat16):
@@ -420,13 +424,18 @@ class LlamaForCausalLM(nn.Module):
                     return h, residual
                 # fall back mid-path: finish with bf16 swiglu+down
                 return layer.down.forward(ops.swiglu(gateup)), residual
-        fused = getattr(layer.gate_up, "forward_normed_swiglu", None)
+        fused = getattr(layer.gate_up, "forward_normed_swiglu", None) \
+            if shares is None else None
         found = fused(o, (layer.post_norm_w, self.cfg.norm_eps, residual)) \
             if fused else None
         if found is not None:
             return layer.down.forward(found[0]), found[1]
-        normed, residual = ops.rmsnorm(o, layer.post_norm_w,
-                                       self.cfg.norm_eps, residual)
+        if shares is None:
+            normed, residual = ops.rmsnorm(o, layer.post_norm_w,
+                                           self.cfg.norm_eps, residual)
+        else:
+            normed, residual = ops.rmsnorm_joined(
+                shares, layer.post_norm_w, self.cfg.norm_eps, residual)
         fused = getattr(layer.gate_up, "forward_swiglu", None)
         act = fused(normed) if fused else None
         if act is not None:

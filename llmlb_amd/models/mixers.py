@@ -4,7 +4,8 @@ Each takes its sizes and constants as arguments and reads the layer's
 input [T, width] in the storage type.  Projections of the same input are
 one matrix product.
 
-``forward`` returns the sublayer's output before any norm.  Modules for
+``forward`` returns the sublayer's output before any norm, and
+``rows_or_shares`` (see ``Projected``) the same for a norm.  Modules for
 parallel layers have ``inner`` instead: it writes what the output
 projection reads (``out_width`` columns of a wider row), so that the
 layer applies the projections of mixer and feed-forward as one product.
@@ -64,7 +65,39 @@ def _halves(dim: int, rot: int) -> torch.Tensor:
     return torch.cat([turned[0::2], turned[1::2], order[rot:]])
 
 
-class LatentAttention(nn.Module):
+class Projected(nn.Module):
+    """A sublayer that ends in a product: ``before(...)`` is what the matrix
+    that ``projection`` names reads."""
+
+    projection = "w_o"
+
+    def forward(self, *args, **kwargs):
+        return _linear(self.before(*args, **kwargs),
+                       getattr(self, self.projection))
+
+    def rows_or_shares(self, *args):
+        """``self(*args)`` or, where calling the module is no more than its
+        product and a row is whole vectors, float shares of it
+        (``linear_shares``) for a norm that adds them up."""
+        w = getattr(self, self.projection)
+        if (w.shape[0] % 8 or _watched(self)
+                or getattr(self.forward, "__func__", None)
+                is not Projected.forward):
+            return self(*args)
+        x = self.before(*args)
+        y = linear_shares(x, w, joined=True)
+        return _linear(x, w) if y is None else y
+
+
+def for_norm(module, width: int = 0):
+    """What to call for a norm of ``width`` columns that takes shares
+    (0: of any width).  A module in another's place is called as any other."""
+    if width > hy.JOINED_WIDTH:
+        return module
+    return getattr(module, "rows_or_shares", module)
+
+
+class LatentAttention(Projected):
     """Multi-head attention whose keys and values are linear maps of one
     cached latent per token, plus a rotated key part shared by the
     heads.  ``kv_from`` names the layer whose latents this one reads
@@ -137,7 +170,7 @@ class LatentAttention(nn.Module):
         return PageSpec(self.rank + self.rot) \
             if self.kv_from is None else None
 
-    def forward(self, x, b, cache, index: int):
+    def before(self, x, b, cache, index: int):
         own = self.kv_from is None
         pages = cache.pages[index if own else self.kv_from]
         proj = _linear(x, self.w_in)
@@ -156,7 +189,7 @@ class LatentAttention(nn.Module):
             hy.latent_flash(o, proj, self.heads, self.dim, self.rot,
                             self.w_uk, self.w_uv, pages, b, self.window,
                             self.scale, self.w_sink, self.g_off)
-        return _linear(o, self.w_o)
+        return o
 
     def _absorbed(self, proj, b, pages, n, out=None):
         """The first n tokens of the batch -> [n, heads * vdim]."""
@@ -185,7 +218,7 @@ class LatentAttention(nn.Module):
         return out
 
 
-class ChannelDelta(nn.Module):
+class ChannelDelta(Projected):
     """Gated delta rule with a decay per head and key channel, short
     convolutions on q, k and v, and a gated norm on each head's
     output."""
@@ -235,15 +268,14 @@ class ChannelDelta(nn.Module):
         C = 2 * self.kv_heads * self.dim + self.heads * self.vdim
         return StateSpec(self.heads, self.vdim, self.dim, C, self.taps)
 
-    def forward(self, x, b, cache, index: int):
+    def before(self, x, b, cache, index: int):
         proj = _linear(x, self.w_in)
         dec, gate = self._low_rank(proj)
-        o = hy.gated_delta(
+        return hy.gated_delta(
             proj, self.b_off, dec, gate, cache.state[index],
             cache.ring[index], b, self.w_conv, self.a_log, self.dt_bias,
             self.w_norm, self.kv_heads, self.heads, self.dim, self.vdim,
             self.taps, self.eps)
-        return _linear(o, self.w_o)
 
     def _low_rank(self, proj):
         """The second projections of decays and gates; alike, they are one
@@ -262,9 +294,11 @@ class ChannelDelta(nn.Module):
                         self.w_g2))
 
 
-class DenseFF(nn.Module):
+class DenseFF(Projected):
     """down(act(up x)); ``act``: "gelu" (its tanh form) or "relu2", the
     square of relu."""
+
+    projection = "w_down"
 
     def __init__(self, *, width, ff, dtype, device, act="gelu"):
         super().__init__()
@@ -288,30 +322,15 @@ class DenseFF(nn.Module):
         self.w_up = _param(F.pad(w["up"], (0, 0, 0, gap)).to(**to))
         self.w_down = _param(F.pad(w["down"], (0, gap)).to(**to))
 
-    def forward(self, x):
-        u = linear_act(x, self.w_up, self.act)
-        if u is not None:
-            return _linear(u, self.w_down)
-        u = _linear(x, self.w_up)
-        if self.act == "gelu":
-            hy.gelu_tanh_(u)
-        else:
-            hy.squared_relu(u, u)
-        return _linear(u, self.w_down)
-
-    def rows_or_shares(self, x):
-        """``self(x)`` or, where calling the module is no more than its
-        products and a row is whole vectors, float shares of it
-        (``linear_shares``) for a caller that adds them up."""
-        if (self.width % 8 or _watched(self)
-                or getattr(self.forward, "__func__", None)
-                is not DenseFF.forward):
-            return self(x)
+    def before(self, x):
         u = linear_act(x, self.w_up, self.act)
         if u is None:
-            return self(x)
-        y = linear_shares(u, self.w_down)
-        return _linear(u, self.w_down) if y is None else y
+            u = _linear(x, self.w_up)
+            if self.act == "gelu":
+                hy.gelu_tanh_(u)
+            else:
+                hy.squared_relu(u, u)
+        return u
 
 
 class DifferentialAttention(nn.Module):
@@ -572,7 +591,7 @@ class WindowedAttention(nn.Module):
         hy.window_attention(*self.attention(proj, b, cache, index, out))
 
 
-class GroupedAttention(nn.Module):
+class GroupedAttention(Projected):
     """Causal attention with grouped key/value heads, over the last
     ``window`` tokens or (``chunk``) those of the query's own run of
     ``window`` positions (None: all).  Queries and keys are normed per
@@ -649,7 +668,7 @@ class GroupedAttention(nn.Module):
     def cache_spec(self):
         return PageSpec(self.kv_heads * (self.dim + self.vdim))
 
-    def forward(self, x, b, cache, index: int):
+    def before(self, x, b, cache, index: int):
         H, G, D, V = self.heads, self.kv_heads, self.dim, self.vdim
         proj, pages = _linear(x, self.w_in), cache.pages[index]
         hy.head_prep(proj, H, G, D, V, self.rot, self.k_off, self.v_off,
@@ -658,10 +677,10 @@ class GroupedAttention(nn.Module):
         o = torch.empty(x.shape[0], H * V, dtype=x.dtype, device=x.device)
         hy.window_attention(o, proj, None, H, G, D, V, pages, b, self.window,
                             self.chunk)
-        return _linear(o, self.w_o)
+        return o
 
 
-class MatrixMemory(nn.Module):
+class MatrixMemory(Projected):
     """mLSTM: S <- exp(f) S + exp(i) k v^T with a normaliser n of the same
     gates, o = S^T q / max(|n . q|, 1), kept in range by a running
     maximum of the gates' logarithms; i = cap tanh(. / cap) and
@@ -701,7 +720,7 @@ class MatrixMemory(nn.Module):
         return StateSpec(self.heads, self.vdim, self.dim, 0, 0,
                          hy.memory_extra(self.dim))
 
-    def forward(self, x, b, cache, index: int):
+    def before(self, x, b, cache, index: int):
         proj = _linear(x, self.w_in)
         o = torch.empty(x.shape[0], self.heads * self.vdim, dtype=x.dtype,
                         device=x.device)
@@ -710,7 +729,7 @@ class MatrixMemory(nn.Module):
                          cache.state[index], cache.extra[index], b,
                          self.w_norm, self.heads, self.dim, self.vdim,
                          self.eps)
-        return _linear(o, self.w_o)
+        return o
 
 
 class RoutedExperts(nn.Module):

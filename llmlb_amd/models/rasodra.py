@@ -23,7 +23,7 @@ from ..ops import hybrid as hy
 from ..ops.reference import build_cos_sin_table
 from ..parallel.tp import TPContext
 from .mixers import (DenseFF, GroupedAttention, LatentAttention,
-                     MatrixMemory)
+                     MatrixMemory, for_norm)
 from .packed import PackedCausalLM, read_folder
 
 
@@ -235,9 +235,9 @@ class RasodraForCausalLM(PackedCausalLM):
             h = between(ly.norm1)
             if i and on_layer is not None:
                 on_layer(i - 1, x)
-            y, w_post = ly.mix(h, b, cache, i), ly.norm1b
+            y, w_post = for_norm(ly.mix, self.cfg.width)(h, b, cache, i), ly.norm1b
             if ly.ff is not None:
-                y, w_post = ly.ff(between(ly.norm2)), ly.norm2b
+                y, w_post = for_norm(ly.ff, self.cfg.width)(between(ly.norm2)), ly.norm2b
         if y is not None:
             between(None)
             if on_layer is not None:

@@ -22,8 +22,8 @@ from ..backend.ragged import RaggedBatch
 from ..ops import hybrid as hy
 from ..parallel.tp import TPContext
 from .mixers import (ClampedSwiGLU, DifferentialAttention,
-                     GatedLinearAttention, StateSpaceDuality, _linear,
-                     _param)
+                     GatedLinearAttention, Projected, StateSpaceDuality,
+                     _param, for_norm)
 from .packed import PackedCausalLM, read_folder
 
 
@@ -143,7 +143,11 @@ def _mixer(cfg: TaletarConfig, i: int, dtype, device):
     raise ValueError(f"layer {i}: unknown mixer '{kind}'")
 
 
-class TaletarLayer(nn.Module):
+class TaletarLayer(Projected):
+    """mixer(h1) + feed_forward(h2), one product of what both leave in a row."""
+
+    projection = "w_out"
+
     def __init__(self, cfg: TaletarConfig, i: int, dtype, device):
         super().__init__()
         self.mix = _mixer(cfg, i, dtype, device)
@@ -155,8 +159,7 @@ class TaletarLayer(nn.Module):
             device=device)
         self.norm2 = None
 
-    def forward(self, h1, h2, b, cache, index: int):
-        """mixer(h1) + feed_forward(h2)."""
+    def before(self, h1, h2, b, cache, index: int):
         n = self.mix.out_width
         mid = torch.empty(h1.shape[0], self.w_out.shape[1], dtype=h1.dtype,
                           device=h1.device)
@@ -165,7 +168,7 @@ class TaletarLayer(nn.Module):
         self.mix.inner(h1, b, cache, index, mid[:, :n], proj)
         if self.ff is not None and proj is None:
             self.ff.inner(h2, mid[:, n:])
-        return _linear(mid, self.w_out)
+        return mid
 
 
 class TaletarForCausalLM(PackedCausalLM):
@@ -235,7 +238,7 @@ class TaletarForCausalLM(PackedCausalLM):
             h1, h2 = hy.add_norms(x, y, ly.norm1, ly.norm2, eps, self.dtype)
             if i and on_layer is not None:
                 on_layer(i - 1, x)
-            y = ly(h1, h2, b, cache, i)
+            y = for_norm(ly, self.cfg.width)(h1, h2, b, cache, i)
         if y is not None:
             hy.add_norms(x, y, None, None, eps, self.dtype)
             if on_layer is not None:

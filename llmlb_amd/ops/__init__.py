@@ -125,6 +125,23 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     return out, residual
 
 
+def rmsnorm_joined(shares: torch.Tensor, weight: torch.Tensor, eps: float,
+                   residual: torch.Tensor):
+    """``rmsnorm`` with a residual of a product in float shares [n, T, H]
+    (``linear_shares``), which are added up and rounded to bf16 first."""
+    n, T, H = shares.shape
+    assert (shares.is_contiguous() and shares.dtype == torch.float32
+            and residual.shape == (T, H) and residual.is_contiguous()
+            and weight.shape == (H,) and weight.is_contiguous()
+            and weight.dtype == residual.dtype == torch.bfloat16)
+    out = torch.empty_like(residual)
+    _check(_require_native().ll_rmsnorm_join(
+        _ptr(out), _ptr(shares), ctypes.c_int(n), _ptr(weight),
+        _ptr(residual), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_float(eps),
+        _stream()), "ll_rmsnorm_join")
+    return out, residual
+
+
 def rope_apply(q: torch.Tensor, k: torch.Tensor, cos_sin: torch.Tensor,
                positions: torch.Tensor):
     """In-place rotate-half RoPE on q [T, n_q, D] and k [T, n_kv, D]."""
@@ -999,18 +1016,21 @@ def linear_two(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor,
     return out
 
 
-def linear_shares(x: torch.Tensor, weight: torch.Tensor
-                  ) -> torch.Tensor | None:
+def linear_shares(x: torch.Tensor, weight: torch.Tensor,
+                  joined: bool = False) -> torch.Tensor | None:
     """x @ W^T as float shares [n, N, M] of the depth whose sum, rounded once,
     is what linear_decode returns, for a caller that adds them up itself.  None
-    where it would not take the depth in shares."""
+    where it would not take the depth in shares.  ``joined``: the caller's next
+    launch adds them up for next to nothing, so that more products gain by it;
+    their sums are linear_decode's in another order."""
     if (_USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight)
             or weight.dtype != x.dtype or x.stride(1) != 1
             or not weight.is_contiguous()):
         return None
     (N, K), M = x.shape, weight.shape[0]
     sizes = (ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
-    shares = _lib.ll_row_gemm_shares(*sizes)
+    plan = _lib.ll_row_gemm_joined if joined else _lib.ll_row_gemm_shares
+    shares = plan(*sizes)
     if shares < 2:
         return None
     ws = torch.empty(shares, N, M, device=x.device, dtype=torch.float32)

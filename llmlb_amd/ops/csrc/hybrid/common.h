@@ -94,6 +94,40 @@ __device__ __forceinline__ float block_sum_256(float v, float* red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
+// The same of any whole waves; ``red`` holds a float for each
+template <int THREADS>
+__device__ __forceinline__ float block_sum(float v, float* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = v;
+  __syncthreads();
+  v = 0.f;
+#pragma unroll
+  for (int i = 0; i < THREADS / WAVE; ++i) v += red[i];
+  return v;
+}
+
+// 8 numbers of a product in float shares, ``step`` apart, which are added up in
+// order and rounded to 16 bits, as by a launch of their own.  Four are asked for
+// at a time: one after the other they are a chain of loads.
+__device__ __forceinline__ void join8(const float* ws, int shares, size_t step,
+                                      float* f) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = 0.f;
+  for (int s0 = 0; s0 < shares; s0 += 4) {
+    float part[4][8];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      load8(ws + (s0 + s < shares ? s0 + s : shares - 1) * step, part[s]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (s0 + s < shares)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] += part[s][j];
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = to_f(from_f<bf16_t>(f[j]));
+}
+
 // sum over each group of 16 consecutive lanes, without LDS traffic
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {

@@ -113,23 +113,7 @@ __global__ __launch_bounds__(THREADS) void post_norm_join_kernel(
   float keep[8], xk[8], wk[8];
   const int own = threadIdx.x;
   auto join = [&](int i, float* f) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = 0.f;
-    for (int s0 = 0; s0 < shares; s0 += 4) {
-      float part[4][8];
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        load8(ws + (s0 + s < shares ? s0 + s : shares - 1) * step + base +
-                  i * 8,
-              part[s]);
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        if (s0 + s < shares)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] += part[s][j];
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = to_f(from_f<bf16_t>(f[j]));
+    join8(ws + base + i * 8, shares, step, f);
   };
   float ssq = 0.f;
   if (own < nvec) {
@@ -145,13 +129,7 @@ __global__ __launch_bounds__(THREADS) void post_norm_join_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j) ssq += f[j] * f[j];
   }
-  ssq = wave_sum(ssq);
-  if (own % WAVE == 0) red[own / WAVE] = ssq;
-  __syncthreads();
-  ssq = 0.f;
-#pragma unroll
-  for (int i = 0; i < THREADS / WAVE; ++i) ssq += red[i];
-  const float r = 1.f / sqrtf(ssq / width + eps);
+  const float r = 1.f / sqrtf(block_sum<THREADS>(ssq, red) / width + eps);
   auto emit = [&](int i, const float* f, float* xr, const float* wr) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) xr[j] += f[j] * r * (w_offset + wr[j]);
@@ -290,6 +268,45 @@ __global__ __launch_bounds__(256) void add_norms_kernel(
       h1[base + i] = from_f<T>(v * w1[ONE ? 0 : i]);
       if (w2) h2[base + i] = from_f<T>(v * w2[ONE ? 0 : i]);
     }
+}
+
+// add_norms of a product in float shares [shares][rows][width]: see
+// post_norm_join.  A row has a thread for every vector.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void add_norms_join_kernel(
+    float* __restrict__ x, const float* __restrict__ ws, int shares,
+    float mult, const float* __restrict__ w1, const float* __restrict__ w2,
+    bf16_t* __restrict__ h1, bf16_t* __restrict__ h2, int width, float eps) {
+  __shared__ float red[THREADS / WAVE];
+  const int i = threadIdx.x * 8;
+  const size_t at = (size_t)blockIdx.x * width + i;
+  const bool own = i < width;
+  float f[8], d[8], w1k[8], w2k[8], ssq = 0.f;
+  if (own) {
+    if (w1) load8(w1 + i, w1k);
+    if (w2) load8(w2 + i, w2k);
+    load8(x + at, f);
+    join8(ws + at, shares, (size_t)gridDim.x * width, d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f[j] += mult * d[j];
+      ssq += f[j] * f[j];
+    }
+    store8(x + at, f);
+  }
+  if (!w1) return;
+  const float r = 1.f / sqrtf(block_sum<THREADS>(ssq, red) / width + eps);
+  if (!own) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    f[j] *= r;
+    d[j] = f[j] * w1k[j];
+  }
+  store8(h1 + at, d);
+  if (!w2) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) d[j] = f[j] * w2k[j];
+  store8(h2 + at, d);
 }
 
 // Each of a row's ``groups`` parts of S columns divided by its rms, times
@@ -541,6 +558,56 @@ __global__ __launch_bounds__(256) void post_pre_norm_kernel(
   }
 }
 
+// post_pre_norm of a product in float shares, as add_norms_join.
+template <int THREADS, bool CENTRED>
+__global__ __launch_bounds__(THREADS) void post_pre_norm_join_kernel(
+    float* __restrict__ x, const float* __restrict__ ws, int shares,
+    const float* __restrict__ w_post, const float* __restrict__ w_pre,
+    bf16_t* __restrict__ h, int width, float eps) {
+  __shared__ float red[4][THREADS / WAVE];
+  const int i = threadIdx.x * 8;
+  const size_t at = (size_t)blockIdx.x * width + i;
+  const bool own = i < width;
+  const float inv = 1.f / width;
+  float f[8], d[8], post[8], pre[8];
+  if (own) {
+    load8(w_post + i, post);
+    if (w_pre) load8(w_pre + i, pre);
+    load8(x + at, f);
+    join8(ws + at, shares, (size_t)gridDim.x * width, d);
+  }
+  // v less its mean; what its norm divides by
+  auto norm = [&](float* v, float* sums, float* squares) {
+    float mean = 0.f, s = 0.f;
+    if (CENTRED) {
+      if (own)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += v[j];
+      mean = block_sum<THREADS>(s, sums) * inv;
+    }
+    s = 0.f;
+    if (own)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[j] -= mean;
+        s += v[j] * v[j];
+      }
+    return 1.f / sqrtf(block_sum<THREADS>(s, squares) * inv + eps);
+  };
+  float r = norm(d, red[0], red[1]);
+  if (own) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] += d[j] * r * post[j];
+    store8(x + at, f);
+  }
+  if (!w_pre) return;
+  r = norm(f, red[2], red[3]);
+  if (!own) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = f[j] * r * pre[j];
+  store8(h + at, f);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_tanh_kernel(T* __restrict__ y,
                                                         long long n) {
@@ -763,6 +830,55 @@ int hy_add_norms(void* x, const void* y, const void* z, const void* zw,
   else GO(false, false);
 #undef GO
 #undef RUN
+  HY_CHECK();
+  return 0;
+}
+
+// y: shares of 16-bit results; rows of whole vectors, one a thread
+int hy_add_norms_join(void* x, const void* y, int shares, float mult,
+                      const void* w1, const void* w2, void* h1, void* h2,
+                      int n_tok, int width, float eps, void* stream) {
+  if (shares < 1 || width <= 0 || width % 8 || width > 8192 || (w1 && !h1) ||
+      (w2 && (!h2 || !w1)))
+    return -2;
+  if (n_tok <= 0) return 0;
+#define GO(THREADS)                                                          \
+  hipLaunchKernelGGL(add_norms_join_kernel<THREADS>, dim3(n_tok),            \
+                     dim3(THREADS), 0, (hipStream_t)stream, (float*)x,       \
+                     (const float*)y, shares, mult, (const float*)w1,        \
+                     (const float*)w2, (bf16_t*)h1, (bf16_t*)h2, width, eps)
+  if (width <= 2048) GO(256);
+  else if (width <= 4096) GO(512);
+  else GO(1024);
+#undef GO
+  HY_CHECK();
+  return 0;
+}
+
+int hy_post_pre_norm_join(void* x, const void* y, int shares,
+                          const void* w_post, const void* w_pre, void* h,
+                          int centred, int n_tok, int width, float eps,
+                          void* stream) {
+  if (shares < 1 || width <= 0 || width % 8 || width > 8192 || !w_post ||
+      (w_pre && !h))
+    return -2;
+  if (n_tok <= 0) return 0;
+#define GO(THREADS, CENTRED)                                               \
+  hipLaunchKernelGGL((post_pre_norm_join_kernel<THREADS, CENTRED>),        \
+                     dim3(n_tok), dim3(THREADS), 0, (hipStream_t)stream,   \
+                     (float*)x, (const float*)y, shares,                   \
+                     (const float*)w_post, (const float*)w_pre,            \
+                     (bf16_t*)h, width, eps)
+#define PICK(THREADS)                \
+  do {                               \
+    if (centred) GO(THREADS, true);  \
+    else GO(THREADS, false);         \
+  } while (0)
+  if (width <= 2048) PICK(256);
+  else if (width <= 4096) PICK(512);
+  else PICK(1024);
+#undef PICK
+#undef GO
   HY_CHECK();
   return 0;
 }

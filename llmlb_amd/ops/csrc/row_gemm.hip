@@ -327,6 +327,37 @@ __global__ __launch_bounds__(256) void row_gemm_join_kernel(
       make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
 }
 
+// residual += the sum of the shares, rounded to bf16 first, out = its RMS norm,
+// as rmsnorm (kernels.hip) of the joined product.  A row has a thread for every
+// vector, which asks for all that it needs at once.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_join_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ ws, int shares,
+    const bf16_t* __restrict__ weight, bf16_t* __restrict__ residual, int width,
+    float eps) {
+  __shared__ float red[THREADS / WAVE];
+  const int i = threadIdx.x * 8;
+  const size_t at = (size_t)blockIdx.x * width + i;
+  const bool own = i < width;
+  float f[8], r[8], w[8], ssq = 0.f;
+  if (own) {
+    load8(weight + i, w);
+    load8(residual + at, r);
+    join8(ws + at, shares, (size_t)gridDim.x * width, f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f[j] = to_f(from_f<bf16_t>(f[j] + r[j]));
+      ssq += f[j] * f[j];
+    }
+    store8(residual + at, f);
+  }
+  const float scale = rsqrtf(block_sum<THREADS>(ssq, red) / width + eps);
+  if (!own) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] = f[j] * scale * w[j];
+  store8(out + at, f);
+}
+
 template <class End>
 struct RowGemm {
   void* out;
@@ -539,38 +570,121 @@ extern "C" int ll_row_gemm_shares(int N, int M, int K) {
   return shares >= 2 && large * shares >= 176 ? shares : 1;
 }
 
+// Tiles of rows: of few outputs two from 33 rows on, or their shares would be too
+// few workgroups.
+static int share_across(int N, int M) {
+  return N > 64 || (N > 32 && M <= 1024) ? 2 : 1;
+}
+// Workgroups that shares of tiles of 16 mt outputs make, and the largest tile of
+// which there are enough for most compute units.
+static long long share_blocks(int N, int M, int mt, int shares) {
+  return (M + 16ll * mt - 1) / (16 * mt) * share_across(N, M) * shares;
+}
+static int share_tile(int N, int M, int shares) {
+  if (share_blocks(N, M, 8, shares) >= 176) return 8;
+  return share_blocks(N, M, 4, shares) >= 176 ? 4 : 2;
+}
+
+template <int NT, int MT, int KW, int S>
+static int row_gemm_share_launch(float* ws, const bf16_t* x, const bf16_t* w,
+                                 int shares, int N, int M, int K, int ldx,
+                                 hipStream_t stream) {
+  auto* kernel = &row_gemm_share_kernel<NT, MT, KW, S>;
+  constexpr int lds = RowTile<NT, MT, KW, S>::LDS;
+  static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const int depth = ((K + shares - 1) / shares + 63) / 64 * 64;
+  const int parts = (K + depth - 1) / depth;
+  const int across = (N + 16 * NT - 1) / (16 * NT);
+  const int down = (M + 16 * MT - 1) / (16 * MT);
+  hipLaunchKernelGGL(kernel, dim3((down + 7) / 8 * 8 * across, parts),
+                     dim3(KW * 64), lds, stream, ws, x, w, N, M, K, ldx,
+                     depth);
+  return hipGetLastError() == hipSuccess ? parts : -1;
+}
+
 // The shares alone, ws [shares][N][M] floats; > 0: as many as there are (with
 // rounding to pieces of 64, up to ``shares``), -2: not for this kernel.
 extern "C" int ll_row_gemm_parts(const void* x, const void* w, void* ws,
                                  int shares, int N, int M, int K, int ldx,
                                  void* stream) {
-  if (N <= 16 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
+  if (N <= 0 || N > 128 || M <= 0 || K <= 0 || M % 4 || K % 8 || ldx % 8 ||
       (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)ws % 16 ||
       shares < 1 || shares > 256)
     return -2;
-  const int tiles = (N + 15) / 16, across = (tiles + 3) / 4;
-  const int depth = ((K + shares - 1) / shares + 63) / 64 * 64;
-  const int parts = (K + depth - 1) / depth;
-  hipStream_t st = (hipStream_t)stream;
-#define GO(NT)                                                               \
-  do {                                                                       \
-    constexpr int lds = RowTile<NT, 4, 4, 2>::LDS;                           \
-    static const hipError_t sized = hipFuncSetAttribute(                     \
-        reinterpret_cast<const void*>(row_gemm_share_kernel<NT, 4, 4, 2>),   \
-        hipFuncAttributeMaxDynamicSharedMemorySize, lds);                    \
-    if (sized != hipSuccess) return -1;                                      \
-    hipLaunchKernelGGL((row_gemm_share_kernel<NT, 4, 4, 2>),                 \
-                       dim3(((M + 63) / 64 + 7) / 8 * 8 * across, parts),    \
-                       dim3(256), lds, st, (float*)ws, (const bf16_t*)x,     \
-                       (const bf16_t*)w, N, M, K, ldx, depth);               \
-  } while (0)
-  switch ((tiles + across - 1) / across) {
-    case 2: GO(2); break;
-    case 3: GO(3); break;
-    default: GO(4); break;
-  }
+  const int tiles = (N + 15) / 16, across = share_across(N, M);
+  switch ((tiles + across - 1) / across * 8 +
+          share_tile(N, M, shares) - 1) {
+#define GO(NT, MT, KW, S)                                                  \
+  case NT * 8 + MT - 1:                                                    \
+    return row_gemm_share_launch<NT, MT, KW, S>(                           \
+        (float*)ws, (const bf16_t*)x, (const bf16_t*)w, shares, N, M, K,   \
+        ldx, (hipStream_t)stream);
+    GO(1, 2, 8, 3)
+    GO(1, 4, 4, 4)
+    GO(1, 8, 4, 2)
+    GO(2, 2, 8, 2)
+    GO(2, 4, 4, 2)
+    GO(2, 8, 4, 2)
+    GO(3, 2, 4, 3)
+    GO(3, 4, 4, 2)
+    GO(3, 8, 3, 2)
+    GO(4, 2, 4, 3)
+    GO(4, 4, 4, 2)
+    GO(4, 8, 3, 2)
 #undef GO
-  return hipGetLastError() == hipSuccess ? parts : -1;
+  }
+  return -2;
+}
+
+// In how many shares a product whose shares the norm after it adds up, which
+// reads them in the launch that it needs anyway.  So more gain than of those that
+// need a launch to join: all whose outputs make few tiles, which read x that much
+// more often, or leave compute units idle (up to 16 rows of 2048 outputs are 128
+// workgroups).  us, product and norm one after the other -> in shares that the norm
+// adds up, weights from HBM:
+//   2048 outputs, 2816 deep: 1 row 7.3 -> 7.3, 16 8.4 -> 7.7, 64 9.8 -> 9.8, 96 11.4
+//       -> 10.3; 6400 deep: 10.7 -> 9.6, 13.9 -> 10.1, 15.9 -> 13.1, 19.6 -> 14.7
+//   1024 outputs, 2816 deep: 7.0 -> 6.6, 8.3 -> 7.1, 8.2 -> 7.8, 9.2 -> 8.6
+//   4096 outputs, 4096 deep: 24 rows 12.9 -> 12.2, 32 14.1 -> 12.5, 64 15.4 -> 15.5,
+//       96 (two) 17.5 -> 16.2; 14336 deep: 12 rows 25.8 -> 25.1, 24 30.1 -> 25.7
+// Not gained by it: 1024 x 1024 (64 rows 6.2 -> 7.1), 2048 x 2048 (8.5 -> 9.0), up
+// to 8 rows of 4096 outputs, which memory bounds (1 row, 14336 deep 24.1 -> 24.9), and
+// five shares or more, whose sums are more to write and read (16 rows of 2048 x 4096
+// 8.4 with four, 9.3 with eight; 128 rows 13.2, 16.6, with two 12.7).
+extern "C" int ll_row_gemm_joined(int N, int M, int K) {
+  const int more = ll_row_gemm_shares(N, M, K);
+  if (more > 1 || N <= 0 || N > 128 || M < 768 || M > 4096 || M % 4)
+    return more;
+  if (M <= 2048) {
+    if (K < 2816) return 1;
+    return N > 64 && M > 1536 && K < 4096 ? 2 : 4;
+  }
+  if (N > 64) return K >= 4096 ? 2 : 1;
+  return K >= (N > 16 ? 3072 : (N > 8 ? 6144 : 1 << 30)) ? 4 : 1;
+}
+
+extern "C" int ll_rmsnorm_join(void* out, const void* ws, int shares,
+                               const void* weight, void* residual, int rows,
+                               int width, float eps, void* stream) {
+  if (shares < 1 || rows <= 0 || width <= 0 || width % 8 || width > 8192 ||
+      ((uintptr_t)out | (uintptr_t)ws | (uintptr_t)weight |
+       (uintptr_t)residual) % 16)
+    return -2;
+#define GO(THREADS)                                                         \
+  hipLaunchKernelGGL(rmsnorm_join_kernel<THREADS>, dim3(rows),              \
+                     dim3(THREADS), 0, (hipStream_t)stream, (bf16_t*)out,   \
+                     (const float*)ws, shares, (const bf16_t*)weight,       \
+                     (bf16_t*)residual, width, eps)
+  if (width <= 2048) GO(256);
+  else if (width <= 4096) GO(512);
+  else GO(1024);
+#undef GO
+  HY_CHECK();
+  return 0;
 }
 
 // The same product in shares, which a second kernel adds up.

@@ -99,14 +99,36 @@ def post_norm_add(x, xb, y, w, eps, w_offset=0.0) -> None:
         _stream()), "hy_post_norm_add")
 
 
+JOINED_WIDTH = 8192     # of rows whose shares add_norms and post_pre_norm take
+
+
+def _shares_fit(x, y, dtype) -> None:
+    assert (y.is_contiguous() and y.dtype == torch.float32
+            and y.shape[1:] == x.shape and x.is_contiguous()
+            and dtype == torch.bfloat16)
+
+
 def add_norms(x, y, w1, w2, eps, dtype, mult=1.0, routed=None):
     """In place: x += mult * y (None: nothing to add).  Returns
     rmsnorm(x) * w1 and rmsnorm(x) * w2 in ``dtype``, None for a weight
     that is None (w2 alone may not be given); weights are rows or single
     numbers.  ``routed``: (z [T, n, W], g [T, n]) whose weighted sum
-    over n is added to y first."""
+    over n is added to y first.  Without it and with weights that are rows,
+    ``y`` may be float shares [n, T, W], as for ``post_norm_add``."""
     if not x.is_cuda:
         return ref.add_norms(x, y, w1, w2, eps, dtype, mult, routed)
+    if y is not None and y.dim() == 3:
+        _shares_fit(x, y, dtype)
+        assert routed is None
+        for w in (w1, w2):
+            assert w is None or w.numel() == x.shape[1]
+        h1, h2 = (None if w is None else torch.empty(
+            x.shape, dtype=dtype, device=x.device) for w in (w1, w2))
+        _check(native().hy_add_norms_join(
+            _ptr(x), _ptr(y), _i(y.shape[0]), _f(mult), _p(w1), _p(w2),
+            _p(h1), _p(h2), _i(x.shape[0]), _i(x.shape[1]), _f(eps),
+            _stream()), "hy_add_norms_join")
+        return h1, h2
     assert y is None or (y.is_contiguous() and y.shape == x.shape
                          and y.dtype == dtype)
     z, g = routed or (None, None)
@@ -132,10 +154,22 @@ def add_norms(x, y, w1, w2, eps, dtype, mult=1.0, routed=None):
 def post_pre_norm(x, y, w_post, w_pre, eps, dtype, centred: bool):
     """In place: x += norm(y) * w_post (y None: nothing to add).  Returns
     norm(x) * w_pre in ``dtype`` (w_pre None: nothing).  ``centred``:
-    layer norms, else RMS norms."""
+    layer norms, else RMS norms.  ``y`` may be float shares [n, T, W], as for
+    ``post_norm_add``."""
     if not x.is_cuda:
         return ref.post_pre_norm(x, y, w_post, w_pre, eps, dtype, centred)
     assert x.is_contiguous()
+    if y is not None and y.dim() == 3:
+        _shares_fit(x, y, dtype)
+        assert w_post.numel() == x.shape[1]
+        assert w_pre is None or w_pre.numel() == x.shape[1]
+        h = None if w_pre is None else torch.empty(x.shape, dtype=dtype,
+                                                   device=x.device)
+        _check(native().hy_post_pre_norm_join(
+            _ptr(x), _ptr(y), _i(y.shape[0]), _ptr(w_post), _p(w_pre), _p(h),
+            _i(centred), _i(x.shape[0]), _i(x.shape[1]), _f(eps),
+            _stream()), "hy_post_pre_norm_join")
+        return h
     assert y is None or (y.is_contiguous() and y.shape == x.shape
                          and y.dtype == dtype
                          and w_post.numel() == x.shape[1])

@@ -243,6 +243,18 @@ class RowParallelLinear(nn.Module, _Fp8WeightMixin):
                 y = _ops.linear_rows(x, self.weight)
         return self.tp.all_reduce(y)
 
+    def forward_shares(self, x: torch.Tensor) -> torch.Tensor | None:
+        """Float shares of the module's output for a norm that adds them up
+        (``ops.rmsnorm_joined``), or None where calling the module would be
+        something else or more, or nothing is gained."""
+        from .. import ops as _ops
+        if (x.dim() != 2 or self.tp.world_size > 1 or _ops._FP8_WEIGHTS
+                or self.weight.shape[0] % 8 or self.weight.shape[0] > 8192
+                or _watched(self) or getattr(self.forward, "__func__", None)
+                is not RowParallelLinear.forward):
+            return None
+        return _ops.linear_shares(x, self.weight, joined=True)
+
     def forward_swiglu_w8a8(self, gateup: torch.Tensor):
         """swiglu_q (quantizing activation kernel) + W8A8 down GEMM;
         None when inapplicable."""

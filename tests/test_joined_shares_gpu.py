@@ -1,0 +1,113 @@
+"""Products in shares for the norm after them: the shares against float64, the
+norms that add them up against those of the joined rows."""
+import pytest
+import torch
+
+import llmlb_amd.ops as ops
+from llmlb_amd.ops import hybrid as hy
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rand(seed, *shape):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=DEV)
+
+
+# every tile (16 to 64 rows, one and two of them, 32 to 128 outputs), rows and
+# outputs that are no whole tiles, depths that are no whole pieces
+@pytest.mark.parametrize("N, M, K", [
+    (1, 768, 2816), (16, 1020, 2824), (17, 1024, 3000), (33, 1024, 2816),
+    (48, 772, 3080), (64, 1024, 2816), (65, 1024, 2824), (128, 1000, 3584),
+    (1, 2048, 2816), (16, 2044, 4104), (32, 2048, 2816), (41, 1540, 2816),
+    (64, 2048, 6400), (65, 2048, 2824), (128, 2048, 4096), (100, 2044, 4104),
+    (9, 4096, 6144), (17, 3076, 3072), (40, 4096, 4096), (64, 4092, 4104),
+    (65, 4096, 4096), (128, 4092, 4104)])
+def test_shares(N, M, K):
+    x, w = rand(N, N, K).bfloat16(), rand(M, M, K).bfloat16()
+    parts = ops.linear_shares(x, w, joined=True)
+    assert parts.dtype == torch.float32 and parts.shape[1:] == (N, M)
+    assert 2 <= parts.shape[0] <= 4
+    want = x.double() @ w.double().T
+    # each of K additions is off by 2^-24 of what has been summed up, which is
+    # no more than the sum of absolute products
+    most = x.double().abs() @ w.double().abs().T
+    off = (parts.double().sum(0) - want).abs()
+    assert (off <= K * 2.0 ** -24 * most).all()
+    assert off.norm() <= 1e-6 * want.norm()
+
+
+# rows of one norm's own columns, a thread with no vector, one, and all of
+# 1024; shares in whole fours and not
+@pytest.mark.parametrize("width", [8, 2040, 2048, 2056, 4096, 4104, 8192])
+@pytest.mark.parametrize("shares, T", [(1, 1), (2, 33), (4, 128), (5, 3)])
+def test_norms(width, shares, T):
+    ws, x0 = rand(1, shares, T, width), rand(2, T, width)
+    w1, w2 = rand(3, width), rand(4, width)
+    y = torch.zeros_like(ws[0])
+    for part in ws:
+        y = y + part
+    y, bf = y.bfloat16(), torch.bfloat16
+
+    def both(f):
+        """f(stream, y) with the shares and with their sum."""
+        (a, *ha), (b, *hb) = ((lambda x: (x, *f(x, rows)))(x0.clone())
+                              for rows in (ws, y))
+        # sums of squares in another order: width 2^-24 of them, half of that
+        # in a root; then one rounding to 16 bits
+        assert (a - b).abs().max() <= width * 2.0 ** -23 * b.abs().max()
+        for p, q in zip(ha, hb):
+            assert (p is None) == (q is None)
+            if p is not None:
+                p, q = p.float(), q.float()
+                assert ((p - q).abs() <= 2.0 ** -7 * q.abs() + 1e-5
+                        * q.abs().max()).all()
+
+    for a, b in ((w1, w2), (w1, None), (None, None)):
+        both(lambda x, rows: hy.add_norms(x, rows, a, b, 1e-5, bf, 0.5))
+        both(lambda x, rows: (hy.post_pre_norm(x, rows, w2, a, 1e-5, bf,
+                                               b is None),))
+    weight = w1.bfloat16()
+    residual = x0.bfloat16()
+    got, sums = ops.rmsnorm_joined(ws, weight, 1e-5, residual.clone())
+    want, sums_ = ops.rmsnorm(y, weight, 1e-5, residual.clone())
+    assert torch.equal(sums, sums_)
+    assert ((got - want).float().abs() <= 2.0 ** -7 * want.float().abs()).all()
+
+
+def test_hooks_see_rows():
+    """What is watched or replaced is called, as before."""
+    from llmlb_amd.models.mixers import Projected, for_norm
+    from llmlb_amd.parallel.tp import RowParallelLinear, TPContext
+
+    class Part(Projected):
+        def before(self, x, twice=False):
+            return x + x if twice else x
+
+    part, x = Part(), rand(5, 16, 4096).bfloat16()
+    part.w_o = rand(6, 2048, 4096).bfloat16()
+    want = part(x)
+    assert torch.equal(part(x, twice=True), part(x + x))
+    assert for_norm(part)(x).dim() == 3 and for_norm(part, 8200) is part
+    seen = []
+    hook = part.register_forward_hook(lambda m, args, out: seen.append(out))
+    assert torch.equal(for_norm(part)(x), want) and len(seen) == 1
+    hook.remove()
+    part.forward = lambda x: x
+    assert for_norm(part)(x) is x
+
+    line = RowParallelLinear(4096, 2048, TPContext()).to(DEV)
+    assert line.forward_shares(x).dim() == 3
+    line.register_forward_hook(lambda m, args, out: None)
+    assert line.forward_shares(x) is None
+
+
+def test_other_products_stay_whole():
+    x, w = rand(7, 64, 1024).bfloat16(), rand(8, 1024, 1024).bfloat16()
+    assert ops.linear_shares(x, w, joined=True) is None
+    x, w = rand(7, 8, 4096).bfloat16(), rand(8, 4096, 4096).bfloat16()
+    assert ops.linear_shares(x, w, joined=True) is None
+    x, w = rand(7, 129, 4096).bfloat16(), rand(8, 2048, 4096).bfloat16()
+    assert ops.linear_shares(x, w, joined=True) is None
+    assert ops.linear_shares(x[:64], w.requires_grad_(), joined=True) is None
