@@ -249,6 +249,18 @@ class _DecodeGraph:
         return self.logits[:n]
 
 
+def _token_arrays(runs: list) -> list:
+    """Token ids of every run as int64.  A decode step's runs are lists of one
+    id, which become one array (64 of them: 51 us one by one, 17 this way)."""
+    if all(type(t) is list and len(t) == 1 for t in runs):
+        try:
+            flat = np.array(array.array("q", [t[0] for t in runs]))
+            return list(flat.reshape(-1, 1))
+        except (TypeError, OverflowError):
+            pass
+    return [_token_array(t) for t in runs]
+
+
 def _token_array(toks) -> np.ndarray:
     """Token ids as int64.  (numpy looks at every element of a list for its
     type first: 391 us for 16384 ids, 263 this way.)"""
@@ -258,6 +270,24 @@ def _token_array(toks) -> np.ndarray:
         except (TypeError, OverflowError):
             pass
     return np.asarray(toks, dtype=np.int64)
+
+
+def _in_order(work, vocab: int, cap: int) -> bool:
+    """Whether every run of a batch can be run: its tokens are in the
+    vocabulary, its sequence stays within ``cap`` and its wanted places are
+    among them.  All tokens at once (64 runs of one token one by one: 190 us,
+    22 this way)."""
+    for seq, toks, want in work:
+        n = len(toks)
+        if not n or seq.length + n > cap:
+            return False
+        for i in want:
+            if not 0 <= i < n:
+                return False
+    if not work:
+        return True
+    flat = np.concatenate([toks for _, toks, _ in work])
+    return flat.min() >= 0 and flat.max() < vocab
 
 
 class _RaggedGraph:
@@ -1003,15 +1033,16 @@ class Engine:
         vocab = self.cfg.model.vocab
         cap = min(self.cfg.model.max_pos,
                   self.max_blocks_per_seq * BLOCK_SIZE)
-        work = [(seq, _token_array(toks), want)
-                for seq, toks, want in work]
-        for seq, toks, want in work:
-            if not len(toks) or toks.min() < 0 or toks.max() >= vocab:
-                raise ValueError("token ids must be in [0, vocab)")
-            if seq.length + len(toks) > cap:
-                raise ValueError(f"sequence longer than {cap} tokens")
-            if any(not 0 <= i < len(toks) for i in want):
-                raise ValueError("wanted place outside the tokens")
+        work = [(seq, toks, want) for (seq, _, want), toks in
+                zip(work, _token_arrays([toks for _, toks, _ in work]))]
+        if not _in_order(work, vocab, cap):     # say what is not
+            for seq, toks, want in work:
+                if not len(toks) or toks.min() < 0 or toks.max() >= vocab:
+                    raise ValueError("token ids must be in [0, vocab)")
+                if seq.length + len(toks) > cap:
+                    raise ValueError(f"sequence longer than {cap} tokens")
+                if any(not 0 <= i < len(toks) for i in want):
+                    raise ValueError("wanted place outside the tokens")
         if len({id(seq) for seq, _, _ in work}) != len(work):
             raise ValueError("a sequence may appear once in a batch")
         if not work:

@@ -112,16 +112,16 @@ class RaggedBatch:
     def pack(runs) -> np.ndarray:
         """``runs``: [(row, position, token ids)], short ones first ->
         the flat int32 array that ``over`` splits."""
-        n = np.array([len(t) for _, _, t in runs], dtype=np.int32)
-        row = np.array([r for r, _, _ in runs], dtype=np.int32)
-        pos = np.array([p for _, p, _ in runs], dtype=np.int32)
+        row, pos, n = np.array([(r, p, len(t)) for r, p, t in runs],
+                               dtype=np.int32).T
         end = np.cumsum(n, dtype=np.int32)
         start = end - n
         at = np.arange(end[-1], dtype=np.int32)
+        # (one conversion of all tokens, not one a run)
+        ids = np.concatenate([t for _, _, t in runs]).astype(np.int32)
         return np.concatenate(
-            [np.asarray(t, dtype=np.int32) for _, _, t in runs]
-            + [at + np.repeat(pos - start, n), np.repeat(row, n),
-               np.repeat(start, n), np.repeat(end, n), start, n, pos, row])
+            [ids, at + np.repeat(pos - start, n), np.repeat(row, n),
+             np.repeat(start, n), np.repeat(end, n), start, n, pos, row])
 
     @classmethod
     def over(cls, flat: torch.Tensor, runs, block_tables,
