@@ -1,8 +1,11 @@
 // Products of tokens with their experts' matrices, any sizes and either
 // type: for every pair of an expert's list (experts.h)
 //   out[pair] = act(w[expert] in[pair / div])
-// with act(z) = max(z, 0)^2 or none.  Tiles of 32 pairs x 64 outputs.
+// with act(z) = max(z, 0)^2 or none.
+//  * expert_float_kernel  32 bits by float_tile.h
+//  * expert_rows_kernel   other sizes, tiles of 32 pairs x 64 outputs
 #include "experts.h"
+#include "float_tile.h"
 
 #define BM 32
 #define BN 64
@@ -63,12 +66,103 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(
   }
 }
 
+struct ExpertRows {
+  const void *in, *w;
+  void* out;
+  const int *counts, *pairs;
+  int E, N, K, div, act, n_tok, n_pairs;
+  hipStream_t stream;
+};
+
+// 16 NT pairs of an expert against 16 MT rows of its matrix.
+template <int NT, int MT, int KW>
+__global__ __launch_bounds__(KW * 64, KW == 4 ? 2 : 1)
+void expert_float_kernel(float* __restrict__ out, const float* __restrict__ in,
+                         const float* __restrict__ w,
+                         const int* __restrict__ counts,
+                         const int* __restrict__ pairs, int E, int N, int K,
+                         int div, int act, int n_tok) {
+  using Tile = FloatTile<NT, MT, KW>;
+  extern __shared__ __align__(1024) char lds[];
+  __shared__ ExpertTiles<16 * NT> tiles;
+  if (threadIdx.x < WAVE) tiles.count(counts, E);
+  __syncthreads();
+  const int i = blockIdx.y, whole = tiles.whole[E - 1];
+  if (i >= whole + tiles.rest[E - 1]) return;
+  const ExpertTile t =
+      tiles.get(counts, E, i < whole ? i : i - whole, i >= whole);
+  const int* list = pairs + (size_t)t.expert * n_tok + t.first;
+  const int n0 = blockIdx.x * 16 * MT, last = N - 1 - n0;
+  if (last < 0) return;
+  const float* const we = w + ((size_t)t.expert * N + n0) * K;
+  auto row = [&](int r) { return list[r < t.n ? r : t.n - 1]; };
+  Tile::run(
+      lds, K, blockIdx.x + t.expert, in,
+      [&](int r) { return (unsigned)(row(r) / div) * (unsigned)K; }, we,
+      [&](int r) { return (unsigned)(r < last ? r : last) * (unsigned)K; });
+  Tile::finish(
+      lds, K, act ? RELU2 : PLAIN, t.n, N - n0,
+      [&](int r) { return in + (size_t)(row(r) / div) * K; },
+      [&](int c) { return we + (size_t)c * K; },
+      [&](int r) { return out + (size_t)row(r) * N + n0; });
+}
+
+template <int NT, int MT, int KW>
+static int expert_float(const ExpertRows& p) {
+  auto* kernel = &expert_float_kernel<NT, MT, KW>;
+  constexpr int lds = FloatTile<NT, MT, KW>::LDS;
+  static const hipError_t sized = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(kernel),
+      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (sized != hipSuccess) return -1;
+  const int tiles =
+      p.n_pairs / (16 * NT) + (p.E < p.n_pairs ? p.E : p.n_pairs);
+  hipLaunchKernelGGL(kernel, dim3((p.N + 16 * MT - 1) / (16 * MT), tiles),
+                     dim3(KW * 64), lds, p.stream, (float*)p.out,
+                     (const float*)p.in, (const float*)p.w, p.counts, p.pairs,
+                     p.E, p.N, p.K, p.div, p.act, p.n_tok);
+  HY_CHECK();
+  return 0;
+}
+
+// Sizes that FloatTile's copies take: whole pieces of 32 of the depth, offsets of
+// 32 bits, whole vectors of outputs.
+static bool expert_float_ok(const ExpertRows& p) {
+  const long long rows = (p.n_pairs + p.div - 1ll) / p.div;
+  return p.K % 32 == 0 && p.N % 4 == 0 &&
+         ((uintptr_t)p.in | (uintptr_t)p.w | (uintptr_t)p.out) % 16 == 0 &&
+         4 * rows * p.K <= 1ll << 32 && 256ll * p.K <= 1ll << 32 &&
+         p.n_pairs / 16 + p.E < 65536;
+}
+
+// By the pairs an expert has: few, of deep products, in tiles of 16, whose waves
+// share the depth; larger tiles, which take less apart, where they fill the chip.
+// us, expert_rows -> here, 16 experts, 4 a token, up (256 outputs, 1024 deep) and
+// down (1024, 256 deep): 20 tokens 87 -> 7, 28 -> 6; 100 101 -> 8, 32 -> 7; 300 173 ->
+// 12, 89 -> 12; 1200 377 -> 27, 231 -> 35.  The tiles of 16, 32 and 48 x 32 and of 48
+// and 64 x 64 at 100 tokens 7.6, 8.9, 10.4, 14.0, 16.7 up and 9.6, 7.4, 11.0, 9.0, 9.9
+// down, at 300 14.7, 13.5, 11.8, 15.3, 19.0 and 22, 16.8, 20, 12.2, 14.2, at 600 22.3,
+// 20.4, 21.1, 29.8, 30.8 and 42, 29, 38, 21, 21.
+static int expert_float_pick(const ExpertRows& p) {
+  const int experts = p.E < p.n_pairs ? p.E : p.n_pairs;
+  const int each = p.n_pairs / experts;
+  const bool deep = p.K >= 512;
+  if (((each + 47ll) / 48) * experts * ((p.N + 63) / 64) >= 384)
+    return each < 350 ? expert_float<3, 4, 4>(p) : expert_float<4, 4, 4>(p);
+  if (each <= (deep ? 25 : 8)) return expert_float<1, 2, 8>(p);
+  return each <= 64 || !deep ? expert_float<2, 2, 8>(p)
+                             : expert_float<3, 2, 8>(p);
+}
+
 extern "C" int hy_expert_rows(void* out, const void* in, const void* w,
                               const void* counts, const void* pairs, int E,
                               int N, int K, int div, int act, int n_tok,
                               int n_pairs, int dtype, void* stream) {
   if (E <= 0 || E > EXPERTS_MAX || N <= 0 || K <= 0 || div <= 0 || N > 65535 * BN) return -2;
   if (n_tok <= 0 || n_pairs <= 0) return 0;
+  const ExpertRows p{in, w, out, (const int*)counts, (const int*)pairs, E, N,
+                     K, div, act, n_tok, n_pairs, (hipStream_t)stream};
+  if (dtype == 1 && expert_float_ok(p)) return expert_float_pick(p);
   const int tiles = n_pairs / BM + (E < n_pairs ? E : n_pairs);
   HY_DTYPE(dtype, hipLaunchKernelGGL(
       expert_rows_kernel<T>, dim3(tiles, (N + BN - 1) / BN), dim3(256), 0,
