@@ -9,16 +9,20 @@
 // LDS once for all of them.  Its four or eight waves work on pages of their
 // own, two at a time, without a barrier: pages are whole runs of memory,
 // copied to LDS and waited for by the wave that asked.  What hides the wait is
-// other waves, eight or more to a compute unit; a second stage of LDS in their
-// place was no faster.  Weights and sums stay floats: a weight enters its
-// product as the sum of three bf16 numbers, which are all of its 24 bits.
+// other waves, eight or more to a compute unit (a second stage of LDS in their
+// place was no faster), and the wave's own other half: the next keys are on their
+// way while values are worked on, the next values while keys are (us, both waited
+// for at once -> this: 64 sequences of 900 tokens 40.1 -> 38.5, 32 of 2000 e4m3 27.1
+// -> 26.0, 8 of 1000 12.7 -> 11.3, 10 of 100 6.7 -> 6.4).  Weights and sums stay
+// floats: a weight enters its product as the sum of three bf16 numbers, which are
+// all of its 24 bits.
 //
 // Sequences use as many parts as their length fills (16 pages each), which
 // the host does not know: the rest of the grid ends at once, and where one
 // part is all, it writes the result itself.
 //
 // Against a lane per part of a row, us (sequences, heads, tokens):
-//   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 41 (5.8 TB/s),
+//   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 39 (5.5 TB/s),
 //     64 x 3600 255 -> 156 (6.2 TB/s), 1 x 4000 47 -> 16
 //   e4m3, the same heads: 64 x 900 70 -> 21; 32 x 2048 in two parts 28, in
 //     one of eight waves 25 (5.6 TB/s), 128 x 1500 56.  Values leave LDS as
@@ -114,6 +118,7 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
   auto look_up = [&](int i) {
     const int p = 2 * (first + (i + lane / 2) * W) + (lane & 1);
     ids = row[p < pages ? p : pages - 1];
+    asm volatile("" : "+v"(ids));  // waited for here, and not by every pass
   };
   // source of lane's piece in copy j of a page
   int off[A::CP];
@@ -122,59 +127,56 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
     const int r = j * (1024 / A::ROW) + lane / A::PR;
     off[j] = r * A::ROW + (((lane % A::PR) ^ turn<A::ROW>(r)) * 16);
   }
-  auto copy = [&](int i) {
-    if (i % 32 == 0) look_up(i);
+  // keys and values of pair i, with their scales
+  auto copy = [&](int i, bool values) {
+    const char* const from = values ? vc : kc;
+    const unsigned there = to + (values ? 2 : 0) * A::BYTES;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int page = __builtin_amdgcn_readlane(ids, 2 * (i % 32) + t);
       const size_t at = ((size_t)page * G + kv) * A::BYTES;
 #pragma unroll
-      for (int j = 0; j < A::CP; ++j) {
-        stream_to_lds(reinterpret_cast<const bf16_t*>(kc + at + off[j]),
-                      to + t * A::BYTES + j * 1024);
-        stream_to_lds(reinterpret_cast<const bf16_t*>(
-                          vc + at + (FP8 && t ? off[j] ^ 64 : off[j])),
-                      to + (2 + t) * A::BYTES + j * 1024);
-      }
+      for (int j = 0; j < A::CP; ++j)
+        stream_to_lds(
+            reinterpret_cast<const bf16_t*>(
+                from + at + (FP8 && t && values ? off[j] ^ 64 : off[j])),
+            there + t * A::BYTES + j * 1024);
     }
-    if (FP8) {  // scales: 16 of each page's keys, then of the values
-      const int page =
-          g & 1 ? __builtin_amdgcn_readlane(ids, 2 * (i % 32) + 1)
-                : __builtin_amdgcn_readlane(ids, 2 * (i % 32));
-      const float* s = g < 2 ? k_scale : v_scale;
-      copy4_to_lds(s + ((size_t)page * G + kv) * PAGE + n,
-                   to + 4 * A::BYTES);
+    if (FP8 && lane < 32) {  // scales of 16 keys or values of each page
+      const int page = __builtin_amdgcn_readlane(ids, 2 * (i % 32) + 1);
+      const int page0 = __builtin_amdgcn_readlane(ids, 2 * (i % 32));
+      copy4_to_lds((values ? v_scale : k_scale) +
+                       ((size_t)(g ? page : page0) * G + kv) * PAGE + n,
+                   to + 4 * A::BYTES + (values ? 128 : 0));
     }
   };
 
+  // Queries come with the page numbers: waited for later, they would make every
+  // pass of the loop wait for all copies.  (Columns past the heads are the first
+  // once more.)
+  u32x4 qf[KD];
+#pragma unroll
+  for (int k = 0; k < KD; ++k)
+    qf[k] = *reinterpret_cast<const u32x4*>(
+        q + (size_t)seq * ldq +
+        (size_t)(kv * R + h0 + (n < heads ? n : 0)) * D + k * 32 + g * 8);
   f32x4 o[VT];
   float m = -1e30f, l = 0.f;
 #pragma unroll
   for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (count) copy(0);
-  u32x4 qf[KD];
+  // copies of a pair's keys, or values
+  constexpr int HALF = 2 * A::CP + (FP8 ? 1 : 0);
+  if (count) look_up(0);
 #pragma unroll
-  for (int k = 0; k < KD; ++k) {
-    qf[k] = u32x4{0, 0, 0, 0};
-    if (n < heads)
-      qf[k] = *reinterpret_cast<const u32x4*>(
-          q + (size_t)seq * ldq + (size_t)(kv * R + h0 + n) * D + k * 32 +
-          g * 8);
+  for (int k = 0; k < KD; ++k) asm volatile("" : "+v"(qf[k]));
+  if (count) {
+    copy(0, false);
+    copy(0, true);
   }
-
   for (int i = 0; i < count; ++i) {
-    wait_copies<0>();
+    wait_copies<HALF>();  // the keys are there
     const int j0 = (first + i * W) * 32;  // the pair's first key
-    if (j0 + 32 > len) {
-      // rows past the end: an earlier sequence may have left anything there
-      const int r = lane / 2;
-      if (j0 + r >= len)
-#pragma unroll
-        for (int c = 0; c < A::ROW / 32; ++c)
-          *reinterpret_cast<uint4*>(st + 2 * A::BYTES + r * A::ROW +
-                                    (lane & 1) * (A::ROW / 2) + c * 16) =
-              make_uint4(0, 0, 0, 0);
-    }
+    const bool more = i + 1 < count;
     f32x4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -201,6 +203,12 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
       for (int r = 0; r < 4; ++r)
         s[t][r] = j0 + t * 16 + g * 4 + r < len ? s[t][r] * by[r] : -INFINITY;
     }
+    // all keys have been read before the next ones' copies start
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (more) {
+      if ((i + 1) % 32 == 0) look_up(i + 1);
+      copy(i + 1, false);
+    }
     float mx = m;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -214,6 +222,20 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
       l *= keep;
 #pragma unroll
       for (int v = 0; v < VT; ++v) o[v] *= keep;
+    }
+    if (more)
+      wait_copies<HALF>();
+    else
+      wait_copies<0>();
+    if (j0 + 32 > len) {
+      // rows past the end: an earlier sequence may have left anything there
+      const int r = lane / 2;
+      if (j0 + r >= len)
+#pragma unroll
+        for (int c = 0; c < A::ROW / 32; ++c)
+          *reinterpret_cast<uint4*>(st + 2 * A::BYTES + r * A::ROW +
+                                    (lane & 1) * (A::ROW / 2) + c * 16) =
+              make_uint4(0, 0, 0, 0);
     }
     u32x4 hi, mid, lo;
 #pragma unroll
@@ -263,9 +285,8 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
       o[v] = mfma(vf, mid, o[v]);
       o[v] = mfma(vf, lo, o[v]);
     }
-    // all has been read before the next copy starts
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (i + 1 < count) copy(i + 1);
+    if (more) copy(i + 1, true);
   }
 
   l += __shfl_xor(l, 16, WAVE);
