@@ -28,10 +28,7 @@ __device__ __forceinline__ float dg_bf2f(unsigned short u) {
   return c.f;
 }
 __device__ __forceinline__ unsigned short dg_f2bf(float f) {
-  union { float f; unsigned int i; } c;
-  c.f = f;
-  unsigned int x = c.i + (0x7FFF + ((c.i >> 16) & 1));
-  return (unsigned short)(x >> 16);
+  return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 __device__ __forceinline__ void dg_unpack8(const uint4 v, float* f) {
   f[0] = dg_bf2f(v.x & 0xffff);  f[1] = dg_bf2f(v.x >> 16);

@@ -24,13 +24,25 @@ template <typename T>
 __device__ __forceinline__ T from_f(float f);
 template <>
 __device__ __forceinline__ float from_f<float>(float f) { return f; }
-// round to nearest even
+// Round to nearest even, by the conversion that the hardware has: an instruction
+// for two numbers, where adding up bits by hand takes three for one.  Of all 2^32
+// floats none but NaN gets other bits, and NaN stays NaN.  It counts where nothing
+// hides the instructions, in what ends a product of many rows (tile_gemm.hip).
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+__device__ __forceinline__ unsigned to_bf16x2(float lo, float hi) {
+  const f32x2 v = {lo, hi};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
 template <>
 __device__ __forceinline__ bf16_t from_f<bf16_t>(float f) {
-  unsigned x = __float_as_uint(f);
-  bf16_t r;
-  r.u = (unsigned short)((x + 0x7FFFu + ((x >> 16) & 1u)) >> 16);
-  return r;
+  return bf16_t{__builtin_bit_cast(unsigned short, (__bf16)f)};
+}
+// both numbers as bf16 holds them
+__device__ __forceinline__ void round_bf16x2(float& a, float& b) {
+  const unsigned v = to_bf16x2(a, b);
+  a = __uint_as_float(v << 16);
+  b = __uint_as_float(v & 0xffff0000u);
 }
 
 // 8 consecutive elements; the address is 16-byte aligned
@@ -47,14 +59,10 @@ __device__ __forceinline__ void load8(const float* p, float* f) {
   f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
   f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
 }
-__device__ __forceinline__ unsigned pack2(float lo, float hi) {
-  return (unsigned)from_f<bf16_t>(lo).u |
-         ((unsigned)from_f<bf16_t>(hi).u << 16);
-}
 __device__ __forceinline__ void store8(bf16_t* p, const float* f) {
   uint4 v;
-  v.x = pack2(f[0], f[1]); v.y = pack2(f[2], f[3]);
-  v.z = pack2(f[4], f[5]); v.w = pack2(f[6], f[7]);
+  v.x = to_bf16x2(f[0], f[1]); v.y = to_bf16x2(f[2], f[3]);
+  v.z = to_bf16x2(f[4], f[5]); v.w = to_bf16x2(f[6], f[7]);
   *reinterpret_cast<uint4*>(p) = v;
 }
 __device__ __forceinline__ void store8(float* p, const float* f) {
@@ -73,8 +81,8 @@ __device__ __forceinline__ void load4(const float* p, float* f) {
   f[0] = v.x; f[1] = v.y; f[2] = v.z; f[3] = v.w;
 }
 __device__ __forceinline__ void store4(bf16_t* p, const float* f) {
-  *reinterpret_cast<uint2*>(p) = make_uint2(pack2(f[0], f[1]),
-                                            pack2(f[2], f[3]));
+  *reinterpret_cast<uint2*>(p) = make_uint2(to_bf16x2(f[0], f[1]),
+                                            to_bf16x2(f[2], f[3]));
 }
 __device__ __forceinline__ void store4(float* p, const float* f) {
   *reinterpret_cast<float4*>(p) = make_float4(f[0], f[1], f[2], f[3]);
@@ -125,7 +133,7 @@ __device__ __forceinline__ void join8(const float* ws, int shares, size_t step,
         for (int j = 0; j < 8; ++j) f[j] += part[s][j];
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) f[j] = to_f(from_f<bf16_t>(f[j]));
+  for (int j = 0; j < 8; j += 2) round_bf16x2(f[j], f[j + 1]);
 }
 
 // sum over each group of 16 consecutive lanes, without LDS traffic

@@ -205,10 +205,10 @@ void latent_flash_kernel(
         for (int v = 0; v < VT; ++v) o[a][v] *= keep;
 #pragma unroll
         for (int p = 0; p < 2; ++p)
-          pf[a][p] = u32x4{pack2(s[a][2 * p][0], s[a][2 * p][1]),
-                           pack2(s[a][2 * p][2], s[a][2 * p][3]),
-                           pack2(s[a][2 * p + 1][0], s[a][2 * p + 1][1]),
-                           pack2(s[a][2 * p + 1][2], s[a][2 * p + 1][3])};
+          pf[a][p] = u32x4{to_bf16x2(s[a][2 * p][0], s[a][2 * p][1]),
+                           to_bf16x2(s[a][2 * p][2], s[a][2 * p][3]),
+                           to_bf16x2(s[a][2 * p + 1][0], s[a][2 * p + 1][1]),
+                           to_bf16x2(s[a][2 * p + 1][2], s[a][2 * p + 1][3])};
       }
 #pragma unroll
       for (int v = 0; v < VT; ++v)
@@ -257,8 +257,8 @@ void latent_flash_kernel(
       if ((V & 3) == 0) {
         if (d < V)
           *reinterpret_cast<uint2*>(dst + d) =
-              make_uint2(pack2(o[a][v][0] * inv, o[a][v][1] * inv),
-                         pack2(o[a][v][2] * inv, o[a][v][3] * inv));
+              make_uint2(to_bf16x2(o[a][v][0] * inv, o[a][v][1] * inv),
+                         to_bf16x2(o[a][v][2] * inv, o[a][v][3] * inv));
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(
         if (g_off >= 0) x[i] /= 1.f + __expf(-z[i]);
       }
       *reinterpret_cast<uint2*>(dst + v * 16) =
-          make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
+          make_uint2(to_bf16x2(x[0], x[1]), to_bf16x2(x[2], x[3]));
     }
   }
 }
@@ -548,7 +548,7 @@ void latent_decode_kernel(
     }
     l = l * kmine + sum;
     *reinterpret_cast<uint2*>(&lp[(ht * 16 + n) * PP + kt * 16 + g * 4]) =
-        make_uint2(pack2(s[0], s[1]), pack2(s[2], s[3]));
+        make_uint2(to_bf16x2(s[0], s[1]), to_bf16x2(s[2], s[3]));
     __syncthreads();
 #pragma unroll
     for (int a = 0; a < HT; ++a)
@@ -592,8 +592,8 @@ void latent_decode_kernel(
         const int d = (wave * NT + r) * 16 + g * 4;
         if (d < rank)  // rank is a multiple of 8
           *reinterpret_cast<uint2*>(dst + d) =
-              make_uint2(pack2(o[a][r][0] * inv, o[a][r][1] * inv),
-                         pack2(o[a][r][2] * inv, o[a][r][3] * inv));
+              make_uint2(to_bf16x2(o[a][r][0] * inv, o[a][r][1] * inv),
+                         to_bf16x2(o[a][r][2] * inv, o[a][r][3] * inv));
       }
     } else {
       const size_t at = ((size_t)q * H + h) * parts + part;
@@ -648,7 +648,8 @@ __global__ __launch_bounds__(128) void latent_merge_kernel(
   if (d >= rank) return;
   const float inv = 1.f / sum;
   *reinterpret_cast<uint2*>(out + ((size_t)h * N + q) * rank + d) =
-      make_uint2(pack2(v[0] * inv, v[1] * inv), pack2(v[2] * inv, v[3] * inv));
+      make_uint2(to_bf16x2(v[0] * inv, v[1] * inv),
+                 to_bf16x2(v[2] * inv, v[3] * inv));
 }
 
 template <int NT, int HT>

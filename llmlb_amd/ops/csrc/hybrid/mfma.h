@@ -35,12 +35,11 @@ __device__ __forceinline__ uint2 load_byte_columns(const char* p) {
       uint2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_s32x2*)p));
 }
 
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-// two floats to bf16, nearest even
-__device__ __forceinline__ unsigned to_bf16x2(float lo, float hi) {
-  const f32x2 v = {lo, hi};
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+// what bf16 holds of four numbers
+__device__ __forceinline__ f32x4 rounded(f32x4 v) {
+  const unsigned a = to_bf16x2(v[0], v[1]), b = to_bf16x2(v[2], v[3]);
+  return f32x4{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u),
+               __uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
 }
 
 // two floats as sums of bf16 numbers, hi + lo

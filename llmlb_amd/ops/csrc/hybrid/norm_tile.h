@@ -104,10 +104,10 @@ struct NormTile {
           const u32x4 r = rv[i];
 #pragma unroll
           for (int c = 0; c < 4; ++c)
-            v[j][c] = pack2(__uint_as_float(v[j][c] << 16) +
-                                __uint_as_float(r[c] << 16),
-                            __uint_as_float(v[j][c] & 0xffff0000u) +
-                                __uint_as_float(r[c] & 0xffff0000u));
+            v[j][c] = to_bf16x2(__uint_as_float(v[j][c] << 16) +
+                                    __uint_as_float(r[c] << 16),
+                                __uint_as_float(v[j][c] & 0xffff0000u) +
+                                    __uint_as_float(r[c] & 0xffff0000u));
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -128,10 +128,10 @@ struct NormTile {
         const u32x4 g = gv[i], sum = v[j];
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          v[j][c] = pack2(__uint_as_float(v[j][c] << 16) * scale *
-                              __uint_as_float(g[c] << 16),
-                          __uint_as_float(v[j][c] & 0xffff0000u) * scale *
-                              __uint_as_float(g[c] & 0xffff0000u));
+          v[j][c] = to_bf16x2(__uint_as_float(v[j][c] << 16) * scale *
+                                  __uint_as_float(g[c] << 16),
+                              __uint_as_float(v[j][c] & 0xffff0000u) * scale *
+                                  __uint_as_float(g[c] & 0xffff0000u));
         xv[i] = v[j];
         if (writes && norm.residual)
           *reinterpret_cast<u32x4*>(norm.sum + (size_t)n * K + i * 8) = sum;

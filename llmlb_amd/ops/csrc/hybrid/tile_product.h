@@ -244,17 +244,18 @@ __device__ __forceinline__ void tile_product(const Source& source,
         unsigned p[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float v[2];
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const int e = 2 * i + j;
-            const float sum = acc[a][b + e / 4][e % 4];
-            const float z = ROUND ? to_f(from_f<bf16_t>(sum)) : sum;
-            if constexpr (GATED)
-              v[j] = row_gate(
-                  as, z, to_f(from_f<bf16_t>(acc[a][b + 2 + e / 4][e % 4])));
-            else
-              v[j] = row_act(as, z);
+          const int t = b + i / 2, e = i % 2 * 2;
+          float v[2] = {acc[a][t][e], acc[a][t][e + 1]};
+          // (plain sums are rounded where they are stored)
+          if constexpr (ROUND && KIND != PLAIN) round_bf16x2(v[0], v[1]);
+          if constexpr (GATED) {
+            float u[2] = {acc[a][t + 2][e], acc[a][t + 2][e + 1]};
+            round_bf16x2(u[0], u[1]);
+            v[0] = row_gate(as, v[0], u[0]);
+            v[1] = row_gate(as, v[1], u[1]);
+          } else {
+            v[0] = row_act(as, v[0]);
+            v[1] = row_act(as, v[1]);
           }
           p[i] = to_bf16x2(v[0], v[1]);
         }

@@ -35,14 +35,16 @@ __device__ __forceinline__ float bf2f(unsigned short u) {
   return c.f;
 }
 
-// round-to-nearest-even f32 -> bf16 (matches torch's conversion)
+// round-to-nearest-even f32 -> bf16 (matches torch's conversion), one
+// instruction for two
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+__device__ __forceinline__ unsigned f2bf2(float lo, float hi) {
+  const f32x2 v = {lo, hi};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+}
 __device__ __forceinline__ unsigned short f2bf(float f) {
-  union { float f; unsigned int i; } c;
-  c.f = f;
-  unsigned int x = c.i;
-  unsigned int rounding_bias = 0x7FFF + ((x >> 16) & 1);
-  x += rounding_bias;
-  return (unsigned short)(x >> 16);
+  return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
 
 // unpack a uint4 (8 bf16) into 8 floats
@@ -55,10 +57,10 @@ __device__ __forceinline__ void unpack8(const uint4 v, float* f) {
 
 __device__ __forceinline__ uint4 pack8(const float* f) {
   uint4 v;
-  v.x = (unsigned int)f2bf(f[0]) | ((unsigned int)f2bf(f[1]) << 16);
-  v.y = (unsigned int)f2bf(f[2]) | ((unsigned int)f2bf(f[3]) << 16);
-  v.z = (unsigned int)f2bf(f[4]) | ((unsigned int)f2bf(f[5]) << 16);
-  v.w = (unsigned int)f2bf(f[6]) | ((unsigned int)f2bf(f[7]) << 16);
+  v.x = f2bf2(f[0], f[1]);
+  v.y = f2bf2(f[2], f[3]);
+  v.z = f2bf2(f[4], f[5]);
+  v.w = f2bf2(f[6], f[7]);
   return v;
 }
 

@@ -41,9 +41,9 @@ struct PlainEnd {
   __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
                                       Early, f32x4 v, f32x4) const {
     if (act.kind != PLAIN) {
+      v = rounded(v);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = row_act(act, to_f(from_f<bf16_t>(v[i])));
+      for (int i = 0; i < 4; ++i) v[i] = row_act(act, v[i]);
     }
     const size_t at = (size_t)n * ld_out + m;
     if (act.kind == CAPPED)
@@ -65,10 +65,10 @@ struct GatedEnd {
   __device__ __forceinline__ int second(int m) const { return act.up + m; }
   __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
                                       Early, f32x4 v, f32x4 u) const {
+    v = rounded(v);
+    u = rounded(u);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      v[i] = row_gate(act, to_f(from_f<bf16_t>(v[i])),
-                      to_f(from_f<bf16_t>(u[i])));
+    for (int i = 0; i < 4; ++i) v[i] = row_gate(act, v[i], u[i]);
     *reinterpret_cast<uint2*>(static_cast<bf16_t*>(out) +
                               (size_t)n * ld_out + m) =
         make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
@@ -117,11 +117,8 @@ struct RotaryEnd {
   __device__ __forceinline__ void put(void* out, int ld_out, int n, int m,
                                       const Early& e, f32x4 v, f32x4 u) const {
     const int half = 1 << shift, head = m >> shift, j = m & (half - 1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = to_f(from_f<bf16_t>(v[i]));
-      u[i] = to_f(from_f<bf16_t>(u[i]));
-    }
+    v = rounded(v);
+    u = rounded(u);
     if (head < n_q + n_kv) {
       const float c[4] = {e.c.x, e.c.y, e.c.z, e.c.w};
       const float s[4] = {e.s.x, e.s.y, e.s.z, e.s.w};
@@ -132,8 +129,8 @@ struct RotaryEnd {
         u[i] = fmaf(b, c[i], a * s[i]);
       }
     }
-    const uint2 lo = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
-    const uint2 hi = make_uint2(pack2(u[0], u[1]), pack2(u[2], u[3]));
+    const uint2 lo = make_uint2(to_bf16x2(v[0], v[1]), to_bf16x2(v[2], v[3]));
+    const uint2 hi = make_uint2(to_bf16x2(u[0], u[1]), to_bf16x2(u[2], u[3]));
     bf16_t* to = static_cast<bf16_t*>(out) + (size_t)n * ld_out + first(m);
     *reinterpret_cast<uint2*>(to) = lo;
     *reinterpret_cast<uint2*>(to + half) = hi;
@@ -345,9 +342,12 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_join_kernel(
     load8(residual + at, r);
     join8(ws + at, shares, (size_t)gridDim.x * width, f);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      f[j] = to_f(from_f<bf16_t>(f[j] + r[j]));
+    for (int j = 0; j < 8; ++j) f[j] += r[j];
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      round_bf16x2(f[j], f[j + 1]);
       ssq += f[j] * f[j];
+      ssq += f[j + 1] * f[j + 1];
     }
     store8(residual + at, f);
   }
@@ -907,9 +907,9 @@ __global__ __launch_bounds__(KW * 64, 2) void head_gemm_kernel(
       const float g[4] = {
           __uint_as_float(z.x << 16), __uint_as_float(z.x & 0xffff0000u),
           __uint_as_float(z.y << 16), __uint_as_float(z.y & 0xffff0000u)};
+      v = rounded(v);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = to_f(from_f<bf16_t>(v[i])) * sigmoid_f(g[i]);
+      for (int i = 0; i < 4; ++i) v[i] *= sigmoid_f(g[i]);
     }
     *reinterpret_cast<uint2*>(out + (size_t)h * os +
                               (size_t)(n0 + r) * ld_out + m0 + c) =
