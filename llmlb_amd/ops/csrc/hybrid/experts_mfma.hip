@@ -211,13 +211,18 @@ void expert_tile_kernel(
   }
 }
 
-// The rows of experts' lists, for tile_product
+// The rows of experts' lists, for tile_product.  A tile's part of its list is
+// in LDS before the copies of its rows begin: asked for there, it would have
+// to wait for all copies under way.
 template <int BM, int BN>
 struct ListRows {
+  // of tiles that are fetched, copied, computed and stored at a time
+  static constexpr int PARTS = 8;
   const bf16_t *in, *w_;
   const int *counts, *pairs;
   int E, N, K, div, n_tok, n_blocks;
   const ExpertTiles<BM>* found;
+  int* parts;  // [PARTS][BM]
   struct At {
     ExpertTile t;
     const int* list;
@@ -226,20 +231,34 @@ struct ListRows {
   __device__ __forceinline__ long long tiles() const {
     return (long long)(found->whole[E - 1] + found->rest[E - 1]) * n_blocks;
   }
-  __device__ __forceinline__ At at(int i) const {
-    const int whole = found->whole[E - 1], j = i / n_blocks;
-    At a;
-    a.t = found->get(counts, E, j < whole ? j : j - whole, j >= whole);
-    a.list = pairs + (size_t)a.t.expert * n_tok + a.t.first;
-    a.m0 = i % n_blocks * BN;
-    return a;
+  // a workgroup's tiles are as far apart as an XCD has workgroups
+  __device__ __forceinline__ int* part(int i) const {
+    return parts + i / (int)(gridDim.x >> 3) % PARTS * BM;
   }
+  __device__ __forceinline__ ExpertTile tile(int i) const {
+    const int whole = found->whole[E - 1], j = i / n_blocks;
+    return found->get(counts, E, j < whole ? j : j - whole, j >= whole);
+  }
+  __device__ __forceinline__ At at(int i) const {
+    return At{tile(i), part(i), i % n_blocks * BN};
+  }
+  // 64 numbers a wave; past the end the last one again
+  __device__ __forceinline__ void fetch(int i) const {
+    static_assert(BM % WAVE == 0, "whole waves");
+    const int at = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
+    if (at >= BM) return;
+    const ExpertTile t = tile(i);
+    const int r = threadIdx.x < t.n ? threadIdx.x : t.n - 1;
+    copy_words_to_lds(pairs + (size_t)t.expert * n_tok + t.first + r,
+                      lds_byte(part(i) + at));
+  }
+  __device__ __forceinline__ void fetched() const { wait_barrier<0>(); }
   __device__ __forceinline__ const bf16_t* x(const At&) const { return in; }
   __device__ __forceinline__ const bf16_t* w(const At& a) const {
     return w_ + (size_t)a.t.expert * N * K;
   }
   __device__ __forceinline__ unsigned x_offset(const At& a, int r) const {
-    return (unsigned)(a.list[r < a.t.n ? r : a.t.n - 1] / div) * (unsigned)K;
+    return (unsigned)(a.list[r] / div) * (unsigned)K;
   }
   __device__ __forceinline__ long long row(const At& a, int r) const {
     return r < a.t.n ? a.list[r] : -1;
@@ -251,10 +270,12 @@ struct ListRows {
 
 // Bound by the matrix cores' power and, for shallow products, by what they
 // write: 16384 tokens with 4 of 16 experts, us, the best of the tiles above
-// -> here: 1024 to 256 wide 60 -> 46, back 61 -> 58; 2048 to 512 162 -> 135,
-// back 211 -> 187; 4096 to 1280 629 -> 573 (1200 TFLOP/s), back 720 -> 695.
-// 256 x 256 leaves no LDS for the tiles' numbers; 256 x 128 and 128 x 256
-// read more (2048 to 512: 146, 156).
+// -> here: 1024 to 256 wide 60 -> 43, back 61 -> 50; 2048 to 512 162 -> 122,
+// back 211 -> 169; 12288 tokens, 4096 to 1280 404 -> 390 and back 503 -> 473
+// against lists asked for from memory and results stored at once (2048 to
+// 512 so 134, back 175).  Without any stores the way back of 512 deep takes
+// 116 us; they alone take 41.  256 x 256 leaves no LDS for the tiles' numbers;
+// 256 x 128 and 128 x 256 read more (2048 to 512: 146, 156).
 template <int BM, int BN, int WM, int WN, int D, int KIND>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
 void expert_product_kernel(bf16_t* __restrict__ out,
@@ -262,9 +283,11 @@ void expert_product_kernel(bf16_t* __restrict__ out,
   __shared__ ExpertTiles<BM> tiles;
   if (threadIdx.x < WAVE) tiles.count(rows.counts, rows.E);
   __syncthreads();
+  __shared__ int parts[ListRows<BM, BN>::PARTS * BM];
   rows.found = &tiles;
-  tile_product<BM, BN, WM, WN, D, KIND, false>(rows, out, rows.N, rows.N, rows.K,
-                                        RowAct{KIND, 0, 0.f, 0.f});
+  rows.parts = parts;
+  tile_product<BM, BN, WM, WN, D, KIND, false, true>(
+      rows, out, rows.N, rows.N, rows.K, RowAct{KIND, 0, 0.f, 0.f});
 }
 
 struct ExpertProduct {
@@ -278,7 +301,8 @@ template <int BM, int BN, int WM, int WN, int D, int KIND>
 static int expert_product(const ExpertProduct& p) {
   auto* kernel = &expert_product_kernel<BM, BN, WM, WN, D, KIND>;
   constexpr int lds = ((D + 1) * BM + D * BN) * DEPTH * 2;
-  static_assert(lds + sizeof(ExpertTiles<BM>) <= 160 * 1024,
+  static_assert(lds + sizeof(ExpertTiles<BM>) +
+                        ListRows<BM, BN>::PARTS * BM * 4 <= 160 * 1024,
                 "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
@@ -291,7 +315,7 @@ static int expert_product(const ExpertProduct& p) {
   if (most >= 1ll << 27) return -2;
   const long long per = (most + 7) / 8;
   const ListRows<BM, BN> rows{p.in, p.w, p.counts, p.pairs, p.E, p.N,
-                              p.K,  p.div, p.n_tok, nb, nullptr};
+                              p.K,  p.div, p.n_tok, nb, nullptr, nullptr};
   hipLaunchKernelGGL(kernel, dim3(8 * (unsigned)(per < 32 ? per : 32)),
                      dim3(WM * WN * 64), lds, p.stream, p.out, rows);
   HY_CHECK();
@@ -340,7 +364,8 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
     case 1: GO(256, 256, 4, 4, 64, 2); break;
     case 2: GO(128, 256, 2, 4, 32, 3); break;
     case 3:
-      if (K % DEPTH == 0 && near) {
+      // (a tile's part of its list is under way for a step at least)
+      if (K % DEPTH == 0 && K >= 2 * DEPTH && near) {
         const ExpertProduct p{(bf16_t*)out, (const bf16_t*)in,
                               (const bf16_t*)w, (const int*)counts,
                               (const int*)pairs, E, N, K, div, n_tok,

@@ -27,7 +27,14 @@ __device__ __forceinline__ void copy_to_lds(const bf16_t* base, unsigned at,
                  "s"(wave_base)
                : "memory");
 }
-// the same for data that nobody reads again
+// 64 lanes copy four bytes each to 256 bytes of LDS
+__device__ __forceinline__ void copy_words_to_lds(const int* src,
+                                                  unsigned to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src)
+               : "memory");
+}
+// the same as the first for data that nobody reads again
 __device__ __forceinline__ void stream_to_lds(const bf16_t* src,
                                               unsigned to) {
   asm volatile(

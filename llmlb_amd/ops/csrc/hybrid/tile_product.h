@@ -14,6 +14,18 @@ __device__ __forceinline__ void times(F&& f) {
   }
 }
 
+// f of the number i, FROM <= i < TO, as a constant
+template <int FROM, int TO, class F>
+__device__ __forceinline__ void pick(int i, F&& f) {
+  if constexpr (TO - FROM == 1) {
+    f(std::integral_constant<int, FROM>{});
+  } else {
+    constexpr int MID = (FROM + TO) / 2;
+    if (i < MID) pick<FROM, MID>(i, f);
+    else pick<MID, TO>(i, f);
+  }
+}
+
 constexpr int DEPTH = 64;  // of a step: a row's part is a line of memory
 
 // The tiles of a workgroup, one after the other: BM rows of x against BN rows
@@ -38,8 +50,12 @@ constexpr int DEPTH = 64;  // of a step: a row's part is a line of memory
 // banks.  W's rows enter the matrix cores in an order in which a lane gets 8
 // consecutive outputs of each of its rows.
 // ROUND: sums are rounded to bf16 before the activation.
+// HELD: a tile's results wait in registers, and their stores follow two a step.
+// A store counts as done before a copy behind it does, so that a burst of them
+// holds the copies up.  It is worth the code in products of experts, whose rows
+// lie apart and whose depth is a few steps.
 template <int BM, int BN, int WM, int WN, int D, int KIND, bool ROUND,
-          class Source>
+          bool HELD, class Source>
 __device__ __forceinline__ void tile_product(const Source& source,
                                              bf16_t* __restrict__ out,
                                              int ld_out, int M, int K,
@@ -116,6 +132,7 @@ __device__ __forceinline__ void tile_product(const Source& source,
     xk = 0;
     if (x_tile + slots < end) {
       x_tile += slots;
+      if (x_tile + slots < end) source.fetch(x_tile + slots);
       aim_x();
     }
   };
@@ -128,6 +145,9 @@ __device__ __forceinline__ void tile_product(const Source& source,
       aim_w();
     }
   };
+  source.fetch(tile);
+  if (tile + slots < end) source.fetch(tile + slots);
+  source.fetched();
   aim_x();
   aim_w();
 #pragma unroll
@@ -202,7 +222,45 @@ __device__ __forceinline__ void tile_product(const Source& source,
   constexpr std::integral_constant<int, 0> H0{};
   constexpr std::integral_constant<int, 1> H1{};
 
-  bool stored = false;  // STORES of each wave's may be under way
+  // -- results
+  constexpr int LATER = 2, SENDS = HELD ? (STORES + LATER - 1) / LATER : 0;
+  u32x4 held[HELD ? STORES : 1];
+  int sent = SENDS;     // of the last tile's
+  bool stored = false;  // its stores are of all lanes
+  auto held_at = source.at(tile);
+  auto store = [&](const auto& at, int i, u32x4 v) {
+    int lane_ = lane;
+    // (places of what is held are not to be kept through the steps)
+    if (HELD) asm volatile("" : "+v"(lane_));
+    const long long n = source.row(at, wm + i / GROUPS * 16 + (lane_ & 15));
+    const int m = at.m0 + (GATED ? wn / 2 : wn) + i % GROUPS * 32 +
+                  (lane_ >> 4) * 8;
+    if (n >= 0 && m < M)
+      *reinterpret_cast<u32x4*>(out + n * ld_out + m) = v;
+  };
+  auto send = [&] {
+    if constexpr (HELD)
+      pick<0, SENDS>(sent++, [&](auto IS) {
+        times<LATER>([&](auto IP) {
+          constexpr int i = IS * LATER + IP;
+          if constexpr (i < STORES) store(held_at, i, held[i]);
+        });
+      });
+  };
+  // all but the copies of the steps past the next one, and what has been
+  // stored behind the next one's
+  constexpr int COPIES = (D - 2) * (CX + CW) + CX;
+  auto step = [&](auto&& wait) {
+    half(H0, [] {});
+    step_x();
+    half(H1, [&] {
+      wait();
+      ux = next_x(ux);
+      uw = next_w(uw);
+    });
+    step_w();
+  };
+
   wait_barrier<(D - 1) * (CX + CW)>();
 #pragma unroll
   for (int b = 0; b < TW; ++b) read_w(0, at_w(0), b);
@@ -214,58 +272,64 @@ __device__ __forceinline__ void tile_product(const Source& source,
 #pragma unroll
       for (int b = 0; b < TW; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     int s = 0;
-    do {
-      half(H0, [] {});
-      step_x();
-      half(H1, [&] {
-        // all but the copies of the steps past the next one, and what the
-        // tile before stored behind the next one's
-        constexpr int COPIES = (D - 2) * (CX + CW) + CX;
-        if (s < (D - 1) * DEPTH && stored) wait_barrier<COPIES + STORES>();
-        else wait_barrier<COPIES>();
-        ux = next_x(ux);
-        uw = next_w(uw);
-      });
-      step_w();
-    } while ((s += DEPTH) < K);
+    if constexpr (HELD) {
+      bool last = false;  // the step before has sent LATER
+      while (s < K && sent < SENDS) {
+        step([&] {
+          if (last) wait_barrier<COPIES + LATER>();
+          else wait_barrier<COPIES>();
+        });
+        send();
+        last = stored && sent * LATER <= STORES;
+        s += DEPTH;
+      }
+      for (; s < K; s += DEPTH) step([] { wait_barrier<COPIES>(); });
+      while (sent < SENDS) send();  // what a shallow product has left
+    } else {
+      do {
+        step([&] {
+          if (s < (D - 1) * DEPTH && stored) wait_barrier<COPIES + STORES>();
+          else wait_barrier<COPIES>();
+        });
+      } while ((s += DEPTH) < K);
+    }
 
     const auto at = source.at(tile);
     // edges store less, and the wait is for all of it
     stored = source.whole(at) && at.m0 + OUT <= M;
+    held_at = at;
+    sent = 0;
     RowAct as = act;
     as.kind = KIND;
-    times<TX>([&](auto IA) {
-      constexpr int a = IA;
-      const long long n = source.row(at, wm + a * 16 + l);
-      bf16_t* row = out + n * ld_out;
-      times<GROUPS>([&](auto IB) {
-        constexpr int b = GATED ? 4 * IB : 2 * IB;
-        const int m = at.m0 + (GATED ? wn / 2 : wn) + IB * 32 + g * 8;
-        unsigned p[4];
+    times<STORES>([&](auto II) {
+      constexpr int I = II, a = I / GROUPS;
+      constexpr int b = I % GROUPS * (GATED ? 4 : 2);
+      unsigned p[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = b + i / 2, e = i % 2 * 2;
-          float v[2] = {acc[a][t][e], acc[a][t][e + 1]};
-          // (plain sums are rounded where they are stored)
-          if constexpr (ROUND && KIND != PLAIN) round_bf16x2(v[0], v[1]);
-          if constexpr (GATED) {
-            float u[2] = {acc[a][t + 2][e], acc[a][t + 2][e + 1]};
-            round_bf16x2(u[0], u[1]);
-            v[0] = row_gate(as, v[0], u[0]);
-            v[1] = row_gate(as, v[1], u[1]);
-          } else {
-            v[0] = row_act(as, v[0]);
-            v[1] = row_act(as, v[1]);
-          }
-          p[i] = to_bf16x2(v[0], v[1]);
+      for (int i = 0; i < 4; ++i) {
+        const int t = b + i / 2, e = i % 2 * 2;
+        float v[2] = {acc[a][t][e], acc[a][t][e + 1]};
+        // (plain sums are rounded where they are stored)
+        if constexpr (ROUND && KIND != PLAIN) round_bf16x2(v[0], v[1]);
+        if constexpr (GATED) {
+          float u[2] = {acc[a][t + 2][e], acc[a][t + 2][e + 1]};
+          round_bf16x2(u[0], u[1]);
+          v[0] = row_gate(as, v[0], u[0]);
+          v[1] = row_gate(as, v[1], u[1]);
+        } else {
+          v[0] = row_act(as, v[0]);
+          v[1] = row_act(as, v[1]);
         }
-        if (n >= 0 && m < M)
-          *reinterpret_cast<u32x4*>(row + m) = u32x4{p[0], p[1], p[2], p[3]};
-      });
+        p[i] = to_bf16x2(v[0], v[1]);
+      }
+      const u32x4 v{p[0], p[1], p[2], p[3]};
+      if constexpr (HELD) held[I] = v;
+      else store(at, I, v);
     });
     tile += slots;
     if (tile >= end) break;
   }
+  while (sent < SENDS) send();
   // no copy is under way when the workgroup's LDS is given back
   wait_barrier<0>();
 }

@@ -48,6 +48,8 @@ struct Rows {
     const int rows = down - run * 4 < 4 ? down - run * 4 : 4;
     return At{(run * 4 + in % rows) * BM, in / rows * OUT};
   }
+  __device__ __forceinline__ void fetch(int) const {}
+  __device__ __forceinline__ void fetched() const {}
   __device__ __forceinline__ const bf16_t* x(const At& a) const {
     return x_ + (size_t)a.n0 * ldx;
   }
@@ -68,7 +70,8 @@ template <int BM, int BN, int WM, int WN, int D, int KIND>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
 void tile_gemm_kernel(Rows<BM, BN, KIND> rows, bf16_t* __restrict__ out,
                       int ld_out, int M, int K, RowAct act) {
-  tile_product<BM, BN, WM, WN, D, KIND, true>(rows, out, ld_out, M, K, act);
+  tile_product<BM, BN, WM, WN, D, KIND, true, false>(rows, out, ld_out, M, K,
+                                                     act);
 }
 
 template <int BM, int BN, int WM, int WN, int D, int KIND>
