@@ -104,11 +104,22 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
 }
 
 // delta_prep for at most TAPS_MAX taps and D <= 256: a workgroup walks
-// PREP_TOK tokens.  blockIdx.y ranges: q/k heads (16 lanes a head, 16
-// heads a workgroup), then value channels, then decays (8 channels a
-// thread).  VEC: all sections start on whole vectors.
+// PREP_TOK tokens, in one of the parts that a token's row has: q/k heads (LANES
+// lanes a head), value channels, decays (N channels a thread).  VEC: all
+// sections start on whole vectors.
+//
+// Bound by memory: 16384 tokens of 16 heads of 128 read 270 MB and write 540, and
+// take 178 us, 4.5 TB/s.  What counts is that all of a row is written at about
+// the same time: with the workgroups of one part side by side, 4 KB of every row,
+// it is 207.  Four tokens are asked for at once, for a load behind a store is
+// there only when the store is: one at a time 227 (8 channels a lane, which
+// leave room for fewer waves), four 217.
 #define PREP_TOK 16
-template <typename T, int RPL, bool VEC>
+template <int LANES>
+__device__ __forceinline__ float row_sum(float x) {
+  return LANES == 32 ? half_wave_sum(x) : row16_sum(x);
+}
+template <typename T, int RPL, int LANES, bool VEC>
 __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     float* __restrict__ ws, const T* __restrict__ proj, int ld, int b_off,
     const T* __restrict__ dec, const T* __restrict__ ring,
@@ -116,71 +127,88 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     const float* __restrict__ dt_bias, const int* __restrict__ pos_,
     const int* __restrict__ row_, const int* __restrict__ tstart_, int n_tok,
     int KH, int H, int D, int V, int taps, float q_scale, int qk_blocks,
-    int v_blocks) {
-  const int t0 = blockIdx.x * PREP_TOK;
+    int v_blocks, int parts) {
+  constexpr int N = LANES == 32 ? 4 : 8;
+  const int t0 = blockIdx.x / parts * PREP_TOK;
   const int t1 = t0 + PREP_TOK < n_tok ? t0 + PREP_TOK : n_tok;
   const int C = 2 * KH * D + H * V;
   const WsLayout at(KH, H, D, V);
-  int y = blockIdx.y;
+  int y = blockIdx.x % parts;
   if (y < qk_blocks) {
-    const int unit = y * 16 + threadIdx.x / 16;
-    if (unit >= KH) return;  // whole groups of 16 lanes
-    const int r0 = (threadIdx.x & 15) * RPL;
+    const int unit = y * (256 / LANES) + threadIdx.x / LANES;
+    if (unit >= KH) return;  // whole groups of lanes
+    const int r0 = threadIdx.x % LANES * RPL;
     const int valid = D - r0 < RPL ? (D - r0 > 0 ? D - r0 : 0) : RPL;
     const int cq = unit * D + (valid ? r0 : 0), ck = KH * D + cq;
     ConvRun<T, RPL, VEC> q(proj, ld, ring, wconv, nullptr, C, taps, cq,
                            valid);
     ConvRun<T, RPL, VEC> k(proj, ld, ring, wconv, nullptr, C, taps, ck,
                            valid);
-    for (int t = t0; t < t1; ++t) {
-      const int ts = tstart_[t];
-      if (t == t0 || t == ts) {
-        q.start(t, pos_[t], ts, row_[t]);
-        k.start(t, pos_[t], ts, row_[t]);
-      }
-      float a[RPL], b[RPL], qq = 0.f, kk = 0.f, qk = 0.f;
-      q.step(t, a);
-      k.step(t, b);
+    auto start = [&](int t, int ts) {
+      q.start(t, pos_[t], ts, row_[t]);
+      k.start(t, pos_[t], ts, row_[t]);
+    };
+    walk_tokens<RPL <= 8 ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
+      constexpr int G = decltype(n)::value;
+      float xq[G][RPL], xk[G][RPL];
 #pragma unroll
-      for (int i = 0; i < RPL; ++i) {
-        if (!VEC && i >= valid) a[i] = b[i] = 0.f;
-        qq += a[i] * a[i];
-        kk += b[i] * b[i];
-        qk += a[i] * b[i];
+      for (int j = 0; j < G; ++j) {
+        q.load(t + j, xq[j]);
+        k.load(t + j, xk[j]);
       }
-      const float qs = q_scale / sqrtf(row16_sum(qq) + 1e-6f);
-      const float ks = 1.f / sqrtf(row16_sum(kk) + 1e-6f);
-      qk = row16_sum(qk) * qs * ks;
 #pragma unroll
-      for (int i = 0; i < RPL; ++i) {
-        a[i] *= qs;
-        b[i] *= ks;
+      for (int j = 0; j < G; ++j) {
+        float a[RPL], b[RPL], qq = 0.f, kk = 0.f, qk = 0.f;
+        q.step(xq[j], a);
+        k.step(xk[j], b);
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+          if (!VEC && i >= valid) a[i] = b[i] = 0.f;
+          qq += a[i] * a[i];
+          kk += b[i] * b[i];
+          qk += a[i] * b[i];
+        }
+        const float qs = q_scale / sqrtf(row_sum<LANES>(qq) + 1e-6f);
+        const float ks = 1.f / sqrtf(row_sum<LANES>(kk) + 1e-6f);
+        qk = row_sum<LANES>(qk) * qs * ks;
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+          a[i] *= qs;
+          b[i] *= ks;
+        }
+        float* w = ws + (size_t)(t + j) * at.size;
+        store_some<RPL, VEC>(w + cq, valid, a);
+        store_some<RPL, VEC>(w + ck, valid, b);
+        if (threadIdx.x % LANES == 0) w[at.qk + unit] = qk;
       }
-      float* w = ws + (size_t)t * at.size;
-      store_some<RPL, VEC>(w + cq, valid, a);
-      store_some<RPL, VEC>(w + ck, valid, b);
-      if ((threadIdx.x & 15) == 0) w[at.qk + unit] = qk;
-    }
+    });
     return;
   }
   y -= qk_blocks;
   if (y < v_blocks) {
-    const int j = (y * 256 + threadIdx.x) * 8;
+    const int j = (y * 256 + threadIdx.x) * N;
     if (j >= H * V) return;
-    const int valid = H * V - j < 8 ? H * V - j : 8;
-    ConvRun<T, 8, VEC> v(proj, ld, ring, wconv, nullptr, C, taps,
+    const int valid = H * V - j < N ? H * V - j : N;
+    ConvRun<T, N, VEC> v(proj, ld, ring, wconv, nullptr, C, taps,
                          2 * KH * D + j, valid);
-    for (int t = t0; t < t1; ++t) {
-      const int ts = tstart_[t];
-      if (t == t0 || t == ts) v.start(t, pos_[t], ts, row_[t]);
-      float f[8];
-      v.step(t, f);
-      store_some<8, VEC>(ws + (size_t)t * at.size + at.v + j, valid, f);
-    }
+    auto start = [&](int t, int ts) { v.start(t, pos_[t], ts, row_[t]); };
+    walk_tokens<4>(tstart_, t0, t1, start, [&](int t, auto n) {
+      constexpr int G = decltype(n)::value;
+      float x[G][N];
+#pragma unroll
+      for (int i = 0; i < G; ++i) v.load(t + i, x[i]);
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        float f[N];
+        v.step(x[i], f);
+        store_some<N, VEC>(ws + (size_t)(t + i) * at.size + at.v + j, valid,
+                           f);
+      }
+    });
     return;
   }
   y -= v_blocks;
-  const int j = (y * 256 + threadIdx.x) * 8;
+  const int j = (y * 256 + threadIdx.x) * N;
   if (y == 0)
     for (int i = threadIdx.x; i < (t1 - t0) * H; i += 256) {
       const int t = t0 + i / H, h = i % H;
@@ -188,19 +216,30 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
           sigmoid_t<T>(to_f(proj[(size_t)t * ld + b_off + h]));
     }
   if (j >= H * D) return;
-  const int valid = H * D - j < 8 ? H * D - j : 8;
-  float bias[8], rate[8];
-  load_some<8, VEC>(dt_bias + j, valid, bias);
+  const int valid = H * D - j < N ? H * D - j : N;
+  float bias[N], rate[N];
+  load_some<N, VEC>(dt_bias + j, valid, bias);
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < N; ++i)
     rate[i] = i < valid ? expf(a_log[(j + i) / D]) : 0.f;
-  for (int t = t0; t < t1; ++t) {
-    float f[8];
-    load_some<8, VEC>(dec + (size_t)t * H * D + j, valid, f);
+  auto decays = [&](int t, auto n) {
+    constexpr int G = decltype(n)::value;
+    float f[G][N];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = decay_t<T>(f[i] + bias[i], rate[i]);
-    store_some<8, VEC>(ws + (size_t)t * at.size + at.g + j, valid, f);
-  }
+    for (int k = 0; k < G; ++k)
+      load_some<N, VEC>(dec + (size_t)(t + k) * H * D + j, valid, f[k]);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        f[k][i] = decay_t<T>(f[k][i] + bias[i], rate[i]);
+      store_some<N, VEC>(ws + (size_t)(t + k) * at.size + at.g + j, valid,
+                         f[k]);
+    }
+  };
+  int t = t0;
+  for (; t + 4 <= t1; t += 4) decays(t, std::integral_constant<int, 4>{});
+  for (; t < t1; ++t) decays(t, std::integral_constant<int, 1>{});
 }
 
 // One wave = 4 CPL value columns of one head of one sequence: 16 lanes a
@@ -529,32 +568,39 @@ int hy_delta_prep(void* ws, const void* proj, int ld, int b_off,
   if (!delta_ok(KH, H, D, V, taps)) return -2;
   if (n_tok <= 0) return 0;
   if (taps <= TAPS_MAX && D <= 256) {
-    const int qk_blocks = (KH + 15) / 16;
-    const int v_blocks = (H * V + 2047) / 2048;
-    const int g_blocks = (H * D + 2047) / 2048;
-    const dim3 grid((n_tok + PREP_TOK - 1) / PREP_TOK,
-                    qk_blocks + v_blocks + g_blocks);
     const bool whole = rows_per_lane(D) * 16 == D && D % 8 == 0 &&
                        V % 8 == 0 && ld % 8 == 0;
-#define RUN(RPL, VEC)                                                        \
+    const int lanes = whole && rows_per_lane(D) >= 8 ? 32 : 16;
+    const int n = lanes == 32 ? 1024 : 2048;
+    const int qk_blocks = (KH + 256 / lanes - 1) / (256 / lanes);
+    const int v_blocks = (H * V + n - 1) / n;
+    const int g_blocks = (H * D + n - 1) / n;
+    const int parts = qk_blocks + v_blocks + g_blocks;
+    const dim3 grid((n_tok + PREP_TOK - 1) / PREP_TOK * parts);
+#define RUN(RPL, LANES, VEC)                                                 \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                        \
-      (delta_prep_run_kernel<T, RPL, VEC>), grid, dim3(256), 0,              \
+      (delta_prep_run_kernel<T, RPL, LANES, VEC>), grid, dim3(256), 0,       \
       (hipStream_t)stream, (float*)ws, (const T*)proj, ld, b_off,            \
       (const T*)dec, (const T*)ring, (const float*)wconv,                    \
       (const float*)a_log, (const float*)dt_bias, (const int*)pos,           \
       (const int*)row, (const int*)tstart, n_tok, KH, H, D, V, taps,         \
-      q_scale, qk_blocks, v_blocks))
-#define PICK(RPL)            \
-  do {                       \
-    if (whole) RUN(RPL, true); \
-    else RUN(RPL, false);    \
+      q_scale, qk_blocks, v_blocks, parts))
+#define PICK(RPL)                    \
+  do {                               \
+    if (whole) RUN(RPL, 16, true);   \
+    else RUN(RPL, 16, false);        \
   } while (0)
     switch (rows_per_lane(D)) {
       case 1: PICK(1); break;
       case 2: PICK(2); break;
       case 4: PICK(4); break;
-      case 8: PICK(8); break;
-      default: PICK(16); break;
+      case 8:
+        if (whole) RUN(4, 32, true);
+        else RUN(8, 16, false);
+        break;
+      default:
+        if (whole) RUN(8, 32, true);
+        else RUN(16, 16, false);
     }
 #undef PICK
 #undef RUN

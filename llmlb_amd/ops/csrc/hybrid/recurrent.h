@@ -7,7 +7,7 @@
 // position p in entry p % taps: the entry of the current token is never
 // one that its own taps read.
 #pragma once
-#include "common.h"
+#include "row_act.h"
 
 // silu(conv + bias) of channel c at packed token t (bias null: none)
 template <typename T>
@@ -97,7 +97,7 @@ __device__ __forceinline__ void store_some(T* p, int valid, const float* f) {
   }
 }
 
-// 16-bit results take the hardware's exponential and logarithm
+// 16-bit models take the hardware's exponential and logarithm
 template <typename T>
 __device__ __forceinline__ float sigmoid_t(float x) {
   return sizeof(T) == 2 ? 1.f / (1.f + __expf(-x)) : sigmoid_f(x);
@@ -105,9 +105,12 @@ __device__ __forceinline__ float sigmoid_t(float x) {
 template <typename T>
 __device__ __forceinline__ float decay_t(float z, float rate) {
   if (sizeof(T) == 2) {
-    const float e = __expf(-fabsf(z));
-    // log(1 + e) by its series where 1 + e would lose e
-    const float lp = e < 1e-3f ? e * (1.f - 0.5f * e) : __logf(1.f + e);
+    const float e = __builtin_amdgcn_exp2f(-LOG2E * fabsf(z));
+    // log(1 + e) by its series where 1 + e would lose e; both are made, which
+    // is less than a branch for every number
+    constexpr float LN2 = 0.6931471805599453f;
+    const float l = LN2 * __builtin_amdgcn_logf(1.f + e);
+    const float lp = e < 1e-3f ? e * (1.f - 0.5f * e) : l;
     return __expf(-rate * (fmaxf(z, 0.f) + lp));
   }
   return expf(-rate * softplus_f(z));
@@ -152,9 +155,11 @@ struct ConvRun {
             valid, hist[b - 1]);
     }
   }
-  __device__ __forceinline__ void step(int t, float* y) {
-    float x[N];
+  __device__ __forceinline__ void load(int t, float* x) const {
     load_some<N, VEC>(proj + (size_t)t * ld + c, valid, x);
+  }
+  // the next token, whose inputs are x
+  __device__ __forceinline__ void step(const float* x, float* y) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       float acc = x[i] * w[0][i] + b0[i];
@@ -164,10 +169,30 @@ struct ConvRun {
 #pragma unroll
       for (int b = TAPS_MAX - 1; b > 1; --b) hist[b - 1][i] = hist[b - 2][i];
       hist[0][i] = x[i];
-      y[i] = acc * sigmoid_t<T>(acc);
+      y[i] = sizeof(T) == 2 ? row_ratio(acc, __expf(-acc))
+                            : acc * sigmoid_f(acc);
     }
   }
 };
+
+// Tokens t0 .. t1 - 1 in order, some at a time: start(t, its sequence's first)
+// where the tokens before t have not been walked, go(t, n) for the next n.  n,
+// a constant, is GROUP where all of these are of one sequence, else 1.
+template <int GROUP, class Start, class Go>
+__device__ __forceinline__ void walk_tokens(const int* tstart, int t0, int t1,
+                                            Start start, Go go) {
+  for (int t = t0; t < t1;) {
+    const int first = tstart[t];
+    if (t == t0 || t == first) start(t, first);
+    if (t + GROUP <= t1 && tstart[t + GROUP - 1] <= t) {
+      go(t, std::integral_constant<int, GROUP>{});
+      t += GROUP;
+    } else {
+      go(t, std::integral_constant<int, 1>{});
+      ++t;
+    }
+  }
+}
 
 template <int RPL, bool EXACT>
 __device__ __forceinline__ void load_rows(const float* __restrict__ p, int r0,

@@ -1,0 +1,88 @@
+"""What the delta rule takes of a packed batch (convolutions, unit norms,
+decays), whose tokens are walked four at a time, against float64."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from llmlb_amd.ops import _ptr, _stream
+from llmlb_amd.ops import hybrid as hy
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# lengths of sequences that begin before, at and behind a group of four and
+# the 16 tokens of a workgroup; positions within and past the taps
+SEQUENCES = [(1, 0), (2, 7), (3, 0), (4, 1), (5, 2), (16, 3), (17, 0), (31, 4),
+             (1, 2), (7, 0)]
+
+
+def _wants(proj, b_off, dec, ring, w, a_log, bias, KH, H, D, V, taps):
+    """q, k, decays, v, beta of every token."""
+    C, rows = 2 * KH * D + H * V, []
+    t = 0
+    for slot, (n, pos) in enumerate(SEQUENCES):
+        past = [ring[slot, (pos - b) % taps] if pos - b >= 0
+                else torch.zeros(C, dtype=torch.float64)
+                for b in range(taps - 1, 0, -1)]
+        x = torch.cat([torch.stack(past), proj[t:t + n, :C]])
+        rows.append(sum(x[b:b + n] * w[b] for b in range(taps)))
+        t += n
+    y = torch.cat(rows)
+    y = y * torch.sigmoid(y)
+    q, k = (y[:, i * KH * D:][:, :KH * D].reshape(t, KH, D) for i in (0, 1))
+    q, k = (z / (z.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+            for z in (q, k))
+    rate = a_log.exp().repeat_interleave(D)
+    return (q * D ** -0.5, k, (-rate * F.softplus(dec + bias)).exp(),
+            y[:, 2 * KH * D:], torch.sigmoid(proj[:, b_off:b_off + H]))
+
+
+# 32 lanes a head (128, 256) and 16, whole vectors and not, fewer taps; the
+# last heads of a workgroup are not there
+@pytest.mark.parametrize("KH, H, D, V", [(3, 6, 128, 72), (9, 9, 256, 128),
+                                         (3, 3, 64, 64), (17, 17, 24, 20),
+                                         (2, 4, 100, 36), (1, 1, 200, 8)])
+@pytest.mark.parametrize("taps", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32],
+                         ids=["bf16", "fp32"])
+def test_delta_prep(KH, H, D, V, taps, dtype):
+    g = torch.Generator().manual_seed(D + taps)
+    T, C = sum(n for n, _ in SEQUENCES), 2 * KH * D + H * V
+    b_off = C + -C % 8
+    ld = b_off + H + -H % 8
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g).to(dtype)
+
+    proj, dec = rand(T, ld), rand(T, H * D) * 4
+    ring, w = rand(len(SEQUENCES), taps, C), rand(taps, C).float()
+    a_log, bias = rand(H).float(), rand(H * D).float()
+    pos, row, start, t = [], [], [], 0
+    for slot, (n, first) in enumerate(SEQUENCES):
+        pos += range(first, first + n)
+        row += [slot] * n
+        start += [t] * n
+        t += n
+    wants = _wants(*(z.double() if torch.is_tensor(z) else z for z in (
+        proj, b_off, dec, ring, w, a_log, bias)), KH, H, D, V, taps)
+    on = [z.to(DEV) for z in (proj, dec, ring, w, a_log, bias)]
+    at = [torch.tensor(z, dtype=torch.int32, device=DEV)
+          for z in (pos, row, start)]
+    lib, sizes = hy.native(), [hy._i(n) for n in (KH, H, D, V)]
+    ws = torch.full((T, int(lib.hy_delta_ws_floats(*sizes))), 7.0, device=DEV)
+    assert lib.hy_delta_prep(
+        _ptr(ws), _ptr(on[0]), hy._i(ld), hy._i(b_off), *map(_ptr, on[1:]),
+        *map(_ptr, at), hy._i(T), *sizes, hy._i(taps), hy._f(D ** -0.5),
+        hy._dt(dtype), _stream()) == 0
+    ws = ws.double().cpu()
+    q, k, decay, v, beta = wants
+    first = 0
+    for want in (q.flatten(1), k.flatten(1), decay, v,
+                 (q * k).sum(-1), beta):
+        got = ws[:, first:first + want.shape[1]]
+        first += want.shape[1]
+        # a few roundings to 24 bits each, of terms no larger than 30; the
+        # hardware's exponential and logarithm are off by 2^-22 of themselves,
+        # an exponent of up to 90 by 90 * 2^-23
+        assert (got - want).abs().max() <= 2.0 ** -16 * max(
+            1.0, want.abs().max())
+        assert (got - want).norm() <= 1e-6 * want.norm()
