@@ -18,13 +18,14 @@
 // Bound by vector instructions, which take numbers apart and look for the largest
 // (6 a number of a tile's edge), beside matrix instructions (a tile of 64 x 64, of
 // 128 of the depth: 1780 and 1540 cycles a SIMD), and by how tiles fill the
-// last round.  So waves have one stage and no pipeline of their own, and two to
-// four of them a SIMD cover each other (two stages and a software pipeline at
-// one wave a SIMD: 600 rows, 1024 x 1024 16 us, 14.2 this way); larger tiles
-// take less apart (600 rows of 4096 x 2048 76 us with 64 x 64, 66 with 80 x 64).
-// us, the library -> here, weights from HBM:
-//   600 rows: 1024 x 1024 16.7 -> 14.2, 3328 x 1024 37 -> 34, 4128 x 1024 53 ->
-//       41, 1024 x 3328 41 -> 34; 64 rows: 8.5 -> 5.5, 12.5 -> 8.9, 13.3 ->
+// last round.  So waves have one stage in LDS, and two to four of them a SIMD cover
+// each other (two stages at one wave a SIMD: 600 rows, 1024 x 1024 16 us, 14.2
+// this way); a wave takes numbers apart between matrix instructions, each of which
+// leaves room for two (3328 x 1024 35 -> 32.3, 4128 x 1024 40.3 -> 37.7); larger
+// tiles take less apart (600 rows of 4096 x 2048 76 us with 64 x 64, 66 with 80 x
+// 64).  us, the library -> here, weights from HBM:
+//   600 rows: 1024 x 1024 16.7 -> 13.9, 3328 x 1024 37 -> 32, 4128 x 1024 53 ->
+//       38, 1024 x 3328 41 -> 34; 64 rows: 8.5 -> 5.5, 12.5 -> 8.9, 13.3 ->
 //       13.2, 11.7 -> 11.6; 16 rows of 4096 x 2048 12.3 -> 9.4; 1600 rows of
 //       4096 x 2048 237 -> 156 (172 TFLOP/s)
 // The largest numbers, which tell what may be lost (see the kernel), cost 2 to 5%.

@@ -5,7 +5,8 @@
 // W is read once and nothing else is large, so the bound is memory for big
 // matrices and latency for small ones; hybrid/row_tile.h says how a tile is
 // computed.  Deep matrices of more than 31 rows take the depth in shares, and
-// a second kernel that adds them up.
+// a second kernel that adds them up, or the norm that follows does, for which
+// matrices of few tiles are taken in shares too.
 //
 // Sizes of a tile are ll_row_gemm's choice.  Against the library's
 // products, us, weights from HBM (N rows: M x K, before -> now):
