@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+import dibelix_util as U
 from llmlb_amd.backend.engine import (_in_order, _token_array, _token_arrays)
 from llmlb_amd.backend.ragged import RaggedBatch
 
@@ -47,3 +48,21 @@ def test_pack():
     assert flat.tolist() == [
         7, 5, 1, 2, 3, 9, 0, 3, 4, 5, 4, 0, 2, 2, 2, 0, 1, 2, 2, 2,
         1, 2, 5, 5, 5, 0, 1, 2, 1, 1, 3, 9, 0, 3, 4, 0, 2]
+
+
+def test_batches_that_can_be_read_once(tmp_path):
+    """A batch and its wanted places may be any iterables."""
+    cfg = U.PLAIN
+    eng = U.engine(U.write_model(tmp_path / "m", cfg, U.weights(cfg)),
+                   blocks=20, rows=4)
+    a, b, c, d = (eng.open_sequence() for _ in range(4))
+    want = eng.run_batch([(a, [1, 2, 3], [0, 2]), (b, [4], [0])])
+    got = eng.run_batch(iter([(c, [1, 2, 3], iter([0, 2])),
+                              (d, [4], iter([0]))]))
+    assert got.shape == (3, cfg["vocab"]) and torch.equal(got, want)
+    assert c.length == 3 and d.length == 1
+    for bad, why in (((a, [5], iter([1])), "wanted place"),
+                     ((a, [cfg["vocab"]], iter([0])), "vocab")):
+        with pytest.raises(ValueError, match=why):
+            eng.run_batch(iter([bad]))
+    assert a.length == 3
