@@ -22,7 +22,10 @@ __global__ __launch_bounds__(256) void route_rows_kernel(Routing a) {
   const int lane = threadIdx.x & (WAVE - 1);
   const T* x = (const T*)a.h + (size_t)t * a.width;
   // four experts of a wave at a time: their rows fly together (300 tokens of 1024
-  // columns, 16 experts, 32 bits, one by one 30.5 us, 11 this way)
+  // columns, 16 experts, 32 bits, one by one 30.5 us, 11 this way); by vectors of
+  // four where all of them lie on whole ones
+  const bool whole = a.width % 4 == 0 &&
+                     ((uintptr_t)a.h | (uintptr_t)a.w) % (4 * sizeof(T)) == 0;
   for (int e0 = wave; e0 < E; e0 += 16) {
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     const T* r[4];
@@ -30,7 +33,7 @@ __global__ __launch_bounds__(256) void route_rows_kernel(Routing a) {
     for (int j = 0; j < 4; ++j)
       r[j] = (const T*)a.w +
              (size_t)(e0 + 4 * j < E ? e0 + 4 * j : e0) * a.width;
-    if (a.width % 4 == 0) {
+    if (whole) {
 #pragma unroll 2
       for (int i = lane * 4; i < a.width; i += 4 * WAVE) {
         float f[4], g[4][4];

@@ -85,3 +85,26 @@ def test_numbers_that_do_not_come_apart():
         e = int(flat[p])
         want = act(odd[9].double() @ up[e].double().T) @ down[e].double().T
         assert (z[p].double() - want).norm() <= 1e-5 * want.norm()
+
+
+# rows that are whole vectors of four and not, at addresses that are and are not
+@pytest.mark.parametrize("W, dtype", [
+    (64, torch.float32), (1024, torch.float32), (1026, torch.float32),
+    (1028, torch.bfloat16), (1026, torch.bfloat16)])
+@pytest.mark.parametrize("at_h, at_w", [(0, 0), (1, 0), (0, 1), (2, 4)])
+def test_router_at_any_address(W, dtype, at_h, at_w):
+    g = torch.Generator(device=DEV).manual_seed(W)
+    T, E = 21, 13
+    flat_h = torch.randn(T * W + 8, generator=g, device=DEV).to(dtype)
+    flat_w = (torch.randn(E * W + 8, generator=g, device=DEV)
+              * 3.0 * W ** -0.5).to(dtype)
+    h = flat_h[at_h:at_h + T * W].view(T, W)
+    w = flat_w[at_w:at_w + E * W].view(E, W)
+    index, weight, _ = hy.route(h, w, E, 1, 1, 1.0, False)
+    want = (h.double() @ w.double().T).softmax(1)
+    got = torch.zeros(T, E, dtype=torch.float64, device=DEV)
+    got.scatter_(1, index.long(), weight.double())
+    # a logit is off by W 2^-24 of its products' sizes at most, and so is the
+    # logarithm of a share of all by twice that and a few roundings more
+    off = W * 2.0 ** -24 * (h.double().abs() @ w.double().abs().T).max()
+    assert (got - want).abs().max() <= 2 * off + 2.0 ** -20
