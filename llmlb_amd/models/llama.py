@@ -406,10 +406,10 @@ class LlamaForCausalLM(nn.Module):
                 if o is not None:
                     # RowParallelLinear: the mixin GEMM is shard-local
                     o = layer.o_proj.tp.all_reduce(o)
-        elif not ops.norms_rows(residual):
+        elif (residual is not None and not ops.norms_rows(residual)
+                and ops.joins_rows(T, layer.post_norm_w, residual)):
             fused = getattr(layer.o_proj, "forward_shares", None)
-            shares = fused(attn_out.reshape(T, -1)) \
-                if fused and residual.is_contiguous() else None
+            shares = fused(attn_out.reshape(T, -1)) if fused else None
         if o is None and shares is None:
             o = layer.o_proj(attn_out.reshape(T, -1))
         if (quant_ok and ops.w8a8_active() and o.is_cuda and T <= 128

@@ -125,15 +125,28 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     return out, residual
 
 
+def _on_vectors(*tensors: torch.Tensor | None) -> bool:
+    """Whether all that there are begin where a load of 16 bytes may."""
+    return not any(t is not None and t.data_ptr() % 16 for t in tensors)
+
+
+def joins_rows(T: int, weight: torch.Tensor, residual: torch.Tensor) -> bool:
+    """Whether ``rmsnorm_joined`` takes T rows with these; ``rmsnorm`` takes
+    more."""
+    H = residual.shape[-1]
+    return (residual.shape == (T, H) and residual.is_contiguous()
+            and weight.shape == (H,) and weight.is_contiguous()
+            and weight.dtype == residual.dtype == torch.bfloat16
+            and _on_vectors(weight, residual))
+
+
 def rmsnorm_joined(shares: torch.Tensor, weight: torch.Tensor, eps: float,
                    residual: torch.Tensor):
     """``rmsnorm`` with a residual of a product in float shares [n, T, H]
     (``linear_shares``), which are added up and rounded to bf16 first."""
     n, T, H = shares.shape
     assert (shares.is_contiguous() and shares.dtype == torch.float32
-            and residual.shape == (T, H) and residual.is_contiguous()
-            and weight.shape == (H,) and weight.is_contiguous()
-            and weight.dtype == residual.dtype == torch.bfloat16)
+            and residual.shape[-1] == H and joins_rows(T, weight, residual))
     out = torch.empty_like(residual)
     _check(_require_native().ll_rmsnorm_join(
         _ptr(out), _ptr(shares), ctypes.c_int(n), _ptr(weight),

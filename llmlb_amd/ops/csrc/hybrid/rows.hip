@@ -714,6 +714,12 @@ __global__ __launch_bounds__(256) void soft_cap_kernel(
   }
 }
 
+// whether every address that there is may be read by loads of 16 bytes
+template <class... P>
+static bool on_vectors(P... p) {
+  return (((uintptr_t)p % 16 == 0) && ...);
+}
+
 extern "C" {
 
 int hy_embed_rows(void* x, void* xb, const void* table, const void* ids,
@@ -742,7 +748,8 @@ int hy_post_norm_add(void* x, void* xb, const void* y, const void* w,
 int hy_post_norm_join(void* x, void* xb, const void* y, int shares,
                       const void* w, float w_offset, int n_tok, int width,
                       float eps, void* stream) {
-  if (shares < 1 || width <= 0 || width % 8) return -2;
+  if (shares < 1 || width <= 0 || width % 8 || !on_vectors(x, xb, y, w))
+    return -2;
   if (n_tok <= 0) return 0;
 #define GO(THREADS)                                                         \
   hipLaunchKernelGGL(post_norm_join_kernel<THREADS>, dim3(n_tok),           \
@@ -839,7 +846,7 @@ int hy_add_norms_join(void* x, const void* y, int shares, float mult,
                       const void* w1, const void* w2, void* h1, void* h2,
                       int n_tok, int width, float eps, void* stream) {
   if (shares < 1 || width <= 0 || width % 8 || width > 8192 || (w1 && !h1) ||
-      (w2 && (!h2 || !w1)))
+      (w2 && (!h2 || !w1)) || !on_vectors(x, y, w1, w2, h1, h2))
     return -2;
   if (n_tok <= 0) return 0;
 #define GO(THREADS)                                                          \
@@ -860,7 +867,7 @@ int hy_post_pre_norm_join(void* x, const void* y, int shares,
                           int centred, int n_tok, int width, float eps,
                           void* stream) {
   if (shares < 1 || width <= 0 || width % 8 || width > 8192 || !w_post ||
-      (w_pre && !h))
+      (w_pre && !h) || !on_vectors(x, y, w_post, w_pre, h))
     return -2;
   if (n_tok <= 0) return 0;
 #define GO(THREADS, CENTRED)                                               \

@@ -17,7 +17,8 @@ import torch
 
 import llmlb_amd.ops as ops
 
-from . import NativeKernelsMissing, _check, _ptr, _stream, linear_rows
+from . import (NativeKernelsMissing, _check, _on_vectors, _ptr, _stream,
+               linear_rows)
 from . import reference_hybrid as ref
 from .build import library_path
 
@@ -87,7 +88,9 @@ def post_norm_add(x, xb, y, w, eps, w_offset=0.0) -> None:
         return
     assert y.is_contiguous() and y.shape[-2:] == x.shape
     if y.dim() == 3:
-        assert y.dtype == torch.float32 and xb.dtype == torch.bfloat16
+        assert xb.dtype == torch.bfloat16
+        if not (_joinable(x, y, (w,)) and _on_vectors(xb)):
+            return post_norm_add(x, xb, _joined(y), w, eps, w_offset)
         _check(native().hy_post_norm_join(
             _ptr(x), _ptr(xb), _ptr(y), _i(y.shape[0]), _ptr(w),
             _f(w_offset), _i(x.shape[0]), _i(x.shape[1]), _f(eps),
@@ -102,10 +105,21 @@ def post_norm_add(x, xb, y, w, eps, w_offset=0.0) -> None:
 JOINED_WIDTH = 8192     # of rows whose shares add_norms and post_pre_norm take
 
 
-def _shares_fit(x, y, dtype) -> None:
+def _joinable(x, y, weights) -> bool:
+    """Whether the kernels that add up shares take these, and weights that
+    are rows.  Their loads are of 16 bytes."""
     assert (y.is_contiguous() and y.dtype == torch.float32
-            and y.shape[1:] == x.shape and x.is_contiguous()
-            and dtype == torch.bfloat16)
+            and y.shape[1:] == x.shape and x.is_contiguous())
+    return _on_vectors(x, y, *weights) and all(
+        w is None or w.numel() == x.shape[1] for w in weights)
+
+
+def _joined(shares):
+    """Their sum, in order and rounded once, as the kernels make it."""
+    y = shares[0]
+    for part in shares[1:]:
+        y = y + part
+    return y.to(torch.bfloat16)
 
 
 def add_norms(x, y, w1, w2, eps, dtype, mult=1.0, routed=None):
@@ -113,15 +127,14 @@ def add_norms(x, y, w1, w2, eps, dtype, mult=1.0, routed=None):
     rmsnorm(x) * w1 and rmsnorm(x) * w2 in ``dtype``, None for a weight
     that is None (w2 alone may not be given); weights are rows or single
     numbers.  ``routed``: (z [T, n, W], g [T, n]) whose weighted sum
-    over n is added to y first.  Without it and with weights that are rows,
-    ``y`` may be float shares [n, T, W], as for ``post_norm_add``."""
+    over n is added to y first.  Without it ``y`` may be float shares
+    [n, T, W], as for ``post_norm_add``."""
     if not x.is_cuda:
         return ref.add_norms(x, y, w1, w2, eps, dtype, mult, routed)
     if y is not None and y.dim() == 3:
-        _shares_fit(x, y, dtype)
-        assert routed is None
-        for w in (w1, w2):
-            assert w is None or w.numel() == x.shape[1]
+        assert routed is None and dtype == torch.bfloat16
+        if not _joinable(x, y, (w1, w2)):
+            return add_norms(x, _joined(y), w1, w2, eps, dtype, mult)
         h1, h2 = (None if w is None else torch.empty(
             x.shape, dtype=dtype, device=x.device) for w in (w1, w2))
         _check(native().hy_add_norms_join(
@@ -160,9 +173,10 @@ def post_pre_norm(x, y, w_post, w_pre, eps, dtype, centred: bool):
         return ref.post_pre_norm(x, y, w_post, w_pre, eps, dtype, centred)
     assert x.is_contiguous()
     if y is not None and y.dim() == 3:
-        _shares_fit(x, y, dtype)
-        assert w_post.numel() == x.shape[1]
-        assert w_pre is None or w_pre.numel() == x.shape[1]
+        assert dtype == torch.bfloat16
+        if not _joinable(x, y, (w_post, w_pre)):
+            return post_pre_norm(x, _joined(y), w_post, w_pre, eps, dtype,
+                                 centred)
         h = None if w_pre is None else torch.empty(x.shape, dtype=dtype,
                                                    device=x.device)
         _check(native().hy_post_pre_norm_join(

@@ -111,3 +111,66 @@ def test_other_products_stay_whole():
     x, w = rand(7, 129, 4096).bfloat16(), rand(8, 2048, 4096).bfloat16()
     assert ops.linear_shares(x, w, joined=True) is None
     assert ops.linear_shares(x[:64], w.requires_grad_(), joined=True) is None
+
+
+# what the norms of whole rows take, those of shares take too: weights and streams
+# in the middle of others, weights that are one number
+@pytest.mark.parametrize("at", [0, 1, 4, 8])
+def test_norms_at_any_address(at):
+    T, W = 5, 1024
+    ws = rand(1, 3, T, W)
+    y = (ws[0] + ws[1] + ws[2]).bfloat16()
+    bf = torch.bfloat16
+
+    def within(seed, *shape, dtype=torch.float32):
+        n = torch.Size(shape).numel()
+        return rand(seed, n + 8).to(dtype)[at:at + n].view(shape)
+
+    w1, w2 = within(2, W), within(3, W)
+    one = within(4, 1)
+
+    def both(f):
+        # as in test_norms
+        for rows in (ws, y):
+            x = within(5, T, W)
+            yield x, f(x, rows)
+
+    for f in (lambda x, r: hy.add_norms(x, r, w1, w2, 1e-5, bf, 0.5),
+              lambda x, r: hy.add_norms(x, r, one, one, 1e-5, bf),
+              lambda x, r: (hy.post_pre_norm(x, r, w1, w2, 1e-5, bf, True),)):
+        (a, ha), (b, hb) = both(f)
+        assert (a - b).abs().max() <= W * 2.0 ** -23 * b.abs().max()
+        for p, q in zip(ha, hb):
+            off = (p.float() - q.float()).abs()
+            assert (off <= 2.0 ** -7 * q.float().abs()
+                    + 1e-5 * q.float().abs().max()).all()
+    sums = []
+    for rows in (ws, y):
+        x, xb = within(5, T, W), within(6, T, W, dtype=bf)
+        hy.post_norm_add(x, xb, rows, w1, 1e-5)
+        assert torch.equal(xb, x.bfloat16())
+        sums.append(x)
+    assert (sums[0] - sums[1]).abs().max() <= (
+        W * 2.0 ** -23 * sums[1].abs().max())
+
+
+@pytest.mark.parametrize("at", [0, 1, 8])
+def test_llama_layer_with_a_weight_at_any_address(at):
+    """Attention's product in shares and the norm after it, with a norm weight
+    that is part of another tensor."""
+    from llmlb_amd.models.llama import LlamaConfig, LlamaForCausalLM
+
+    cfg = LlamaConfig(hidden=1024, layers=1, q_heads=32, kv_heads=8,
+                      head_dim=128, inter=2816, vocab=64, max_pos=64)
+    model = LlamaForCausalLM(cfg, dtype=torch.bfloat16, device=DEV)
+    layer = model.layers_[0]
+    attn, residual = rand(1, 8, 4096).bfloat16(), rand(2, 8, 1024).bfloat16()
+    assert layer.o_proj.forward_shares(attn) is not None
+    want = model.layer_attn_epilogue(0, attn, residual.clone())
+    flat = layer.post_norm_w.data.new_ones(1024 + 8)
+    layer.post_norm_w.data = flat[at:at + 1024]
+    got = model.layer_attn_epilogue(0, attn, residual.clone())
+    for a, b in zip(got, want):
+        a, b = a.double(), b.double()
+        # sums in another order, and a rounding to 16 bits of what they make
+        assert (a - b).norm() <= 2.0 ** -8 * b.norm()
