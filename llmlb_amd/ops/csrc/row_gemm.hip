@@ -571,18 +571,17 @@ extern "C" int ll_row_gemm_shares(int N, int M, int K) {
   return shares >= 2 && large * shares >= 176 ? shares : 1;
 }
 
-// Tiles of rows: of few outputs two from 33 rows on, or their shares would be too
-// few workgroups.
-static int share_across(int N, int M) {
-  return N > 64 || (N > 32 && M <= 1024) ? 2 : 1;
+// Tiles of rows: from 33 rows on two where the shares of both are still no more
+// workgroups than compute units.
+static int share_across(int N, int M, int shares) {
+  return N > 64 || (N > 32 && (M + 31ll) / 32 * 2 * shares <= 256) ? 2 : 1;
 }
-// Workgroups that shares of tiles of 16 mt outputs make, and the largest tile of
-// which there are enough for most compute units.
+// Workgroups that shares of tiles of 16 mt outputs make, and the tile: the larger
+// where there are enough of it for most compute units.
 static long long share_blocks(int N, int M, int mt, int shares) {
-  return (M + 16ll * mt - 1) / (16 * mt) * share_across(N, M) * shares;
+  return (M + 16ll * mt - 1) / (16 * mt) * share_across(N, M, shares) * shares;
 }
 static int share_tile(int N, int M, int shares) {
-  if (share_blocks(N, M, 8, shares) >= 176) return 8;
   return share_blocks(N, M, 4, shares) >= 176 ? 4 : 2;
 }
 
@@ -616,7 +615,7 @@ extern "C" int ll_row_gemm_parts(const void* x, const void* w, void* ws,
       (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)ws % 16 ||
       shares < 1 || shares > 256)
     return -2;
-  const int tiles = (N + 15) / 16, across = share_across(N, M);
+  const int tiles = (N + 15) / 16, across = share_across(N, M, shares);
   switch ((tiles + across - 1) / across * 8 +
           share_tile(N, M, shares) - 1) {
 #define GO(NT, MT, KW, S)                                                  \
@@ -626,16 +625,12 @@ extern "C" int ll_row_gemm_parts(const void* x, const void* w, void* ws,
         ldx, (hipStream_t)stream);
     GO(1, 2, 8, 3)
     GO(1, 4, 4, 4)
-    GO(1, 8, 4, 2)
     GO(2, 2, 8, 2)
     GO(2, 4, 4, 2)
-    GO(2, 8, 4, 2)
     GO(3, 2, 4, 3)
     GO(3, 4, 4, 2)
-    GO(3, 8, 3, 2)
     GO(4, 2, 4, 3)
     GO(4, 4, 4, 2)
-    GO(4, 8, 3, 2)
 #undef GO
   }
   return -2;

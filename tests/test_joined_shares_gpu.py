@@ -1,5 +1,7 @@
 """Products in shares for the norm after them: the shares against float64, the
 norms that add them up against those of the joined rows."""
+import ctypes
+
 import pytest
 import torch
 
@@ -15,20 +17,9 @@ def rand(seed, *shape):
     return torch.randn(*shape, generator=g, device=DEV)
 
 
-# every tile (16 to 64 rows, one and two of them, 32 to 128 outputs), rows and
-# outputs that are no whole tiles, depths that are no whole pieces
-@pytest.mark.parametrize("N, M, K", [
-    (1, 768, 2816), (16, 1020, 2824), (17, 1024, 3000), (33, 1024, 2816),
-    (48, 772, 3080), (64, 1024, 2816), (65, 1024, 2824), (128, 1000, 3584),
-    (1, 2048, 2816), (16, 2044, 4104), (32, 2048, 2816), (41, 1540, 2816),
-    (64, 2048, 6400), (65, 2048, 2824), (128, 2048, 4096), (100, 2044, 4104),
-    (9, 4096, 6144), (17, 3076, 3072), (40, 4096, 4096), (64, 4092, 4104),
-    (65, 4096, 4096), (128, 4092, 4104)])
-def test_shares(N, M, K):
-    x, w = rand(N, N, K).bfloat16(), rand(M, M, K).bfloat16()
-    parts = ops.linear_shares(x, w, joined=True)
-    assert parts.dtype == torch.float32 and parts.shape[1:] == (N, M)
-    assert 2 <= parts.shape[0] <= 4
+def check(parts, x, w):
+    """Float shares of x w^T against its 64-bit product."""
+    K = x.shape[1]
     want = x.double() @ w.double().T
     # each of K additions is off by 2^-24 of what has been summed up, which is
     # no more than the sum of absolute products
@@ -36,6 +27,43 @@ def test_shares(N, M, K):
     off = (parts.double().sum(0) - want).abs()
     assert (off <= K * 2.0 ** -24 * most).all()
     assert off.norm() <= 1e-6 * want.norm()
+
+
+# the eight tiles, of 16 to 64 rows (one of them and two) and 32 (few outputs or
+# shares) or 64 outputs (many): each at its first and last rows, outputs that are
+# no whole tiles, depths that are no whole pieces
+@pytest.mark.parametrize("N, M, K, shares", [
+    (1, 768, 2816, 4), (16, 1020, 2824, 4), (16, 4092, 264, 2),   # 16 x 32
+    (1, 2816, 520, 4), (16, 4092, 6152, 4),                       # 16 x 64
+    (17, 1024, 3000, 4), (32, 2048, 2816, 4), (33, 1024, 2816, 4),
+    (64, 1020, 2824, 4),                                          # 32 x 32
+    (17, 2812, 520, 4), (32, 4096, 3080, 4), (32, 3076, 64, 4),   # 32 x 64
+    (33, 1540, 2816, 4), (48, 4092, 3072, 2), (65, 772, 3080, 2),
+    (96, 2048, 2824, 2),                                          # 48 x 32
+    (33, 2816, 6144, 4), (48, 1024, 24576, 11), (65, 4096, 4096, 2),
+    (96, 2044, 4104, 4),                                          # 48 x 64
+    (49, 2048, 6400, 4), (64, 4092, 4104, 2), (97, 1000, 3584, 4),
+    (128, 2048, 4096, 2),                                         # 64 x 32
+    (49, 4096, 6144, 4), (64, 1024, 24584, 11), (97, 2816, 4104, 2),
+    (128, 4092, 4104, 2), (128, 2044, 4104, 4)])                  # 64 x 64
+def test_shares(N, M, K, shares):
+    x, w = rand(N, N, K).bfloat16(), rand(M, M, K).bfloat16()
+    ws = torch.full((shares, N, M), float("nan"), device=DEV)
+    sizes = [ctypes.c_int(n) for n in (shares, N, M, K, K)]
+    parts = ops._require_native().ll_row_gemm_parts(
+        ops._ptr(x), ops._ptr(w), ops._ptr(ws), *sizes, ops._stream())
+    assert 1 <= parts <= shares
+    check(ws[:parts], x, w)
+    assert ws[parts:].isnan().all()
+
+
+@pytest.mark.parametrize("N, M, K", [(1, 1024, 2816), (128, 2048, 4096),
+                                     (24, 4096, 6152), (48, 1024, 24576)])
+def test_shares_of_the_rule(N, M, K):
+    x, w = rand(N, N, K).bfloat16(), rand(M, M, K).bfloat16()
+    parts = ops.linear_shares(x, w, joined=True)
+    assert parts.dtype == torch.float32 and parts.shape[1:] == (N, M)
+    check(parts, x, w)
 
 
 # rows of one norm's own columns, a thread with no vector, one, and all of
