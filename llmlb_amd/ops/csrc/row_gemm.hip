@@ -638,29 +638,54 @@ extern "C" int ll_row_gemm_parts(const void* x, const void* w, void* ws,
 
 // In how many shares a product whose shares the norm after it adds up, which
 // reads them in the launch that it needs anyway.  So more gain than of those that
-// need a launch to join: all whose outputs make few tiles, which read x that much
-// more often, or leave compute units idle (up to 16 rows of 2048 outputs are 128
-// workgroups).  us, product and norm one after the other -> in shares that the norm
-// adds up, weights from HBM:
-//   2048 outputs, 2816 deep: 1 row 7.3 -> 7.3, 16 8.4 -> 7.7, 64 9.8 -> 9.8, 96 11.4
-//       -> 10.3; 6400 deep: 10.7 -> 9.6, 13.9 -> 10.1, 15.9 -> 13.1, 19.6 -> 14.7
-//   1024 outputs, 2816 deep: 7.0 -> 6.6, 8.3 -> 7.1, 8.2 -> 7.8, 9.2 -> 8.6
-//   4096 outputs, 4096 deep: 24 rows 12.9 -> 12.2, 32 14.1 -> 12.5, 64 15.4 -> 15.5,
-//       96 (two) 17.5 -> 16.2; 14336 deep: 12 rows 25.8 -> 25.1, 24 30.1 -> 25.7
-// Not gained by it: 1024 x 1024 (64 rows 6.2 -> 7.1), 2048 x 2048 (8.5 -> 9.0), up
-// to 8 rows of 4096 outputs, which memory bounds (1 row, 14336 deep 24.1 -> 24.9), and
-// five shares or more, whose sums are more to write and read (16 rows of 2048 x 4096
-// 8.4 with four, 9.3 with eight; 128 rows 13.2, 16.6, with two 12.7).
+// need a launch to join: all whose outputs make few tiles, which leave compute units
+// idle (up to 16 rows of 2048 outputs are 128 workgroups) or read x that much more
+// often.  What bounds it: a second round of workgroups costs more than shares gain
+// (48 rows of 2560 x 4096 in two shares, 160 workgroups, 3% faster, in four, 320,
+// 13% slower), so there is at most one for every compute unit; and sums are more to
+// write and read, so that each share needs some depth, more of it the more sums
+// there are.  Product and norm, whole -> shares, us, weights from HBM (by
+// post_norm_add; add_norms and the Llama norm are alike to 3%):
+//   1024 outputs, 2816 deep, four: 1 row 7.0 -> 6.6, 16 8.3 -> 7.3, 64 8.4 -> 7.9,
+//       128 9.5 -> 9.4; 2048 deep: 6.4 -> 6.2, 7.1 -> 6.7, 7.3 -> 7.4, 8.5 -> 8.6
+//   2048 outputs, 3584 deep, four: 1 row 8.1 -> 7.8, 16 9.6 -> 8.2, 64 11.2 -> 10.5;
+//       2816 deep: 7.3 -> 7.5, 8.7 -> 7.8, 10.0 -> 9.9 (Llama's norm 9.7 -> 9.7);
+//       96 rows, two: 2816 deep 11.7 -> 10.5, 4096 14.0 -> 11.8 (four 11.9), 6400
+//       19.6 -> 15.5, four 14.6
+//   4096 outputs, two: 32 rows, 3584 deep 12.8 -> 11.8, 64 15.0 -> 14.1; 4096 deep
+//       14.1 -> 12.4, 15.6 -> 14.8 (four 12.7, 15.3), 96 rows 17.5 -> 16.2; 2816 deep
+//       11.5 -> 10.9, 13.1 -> 12.8; 24 rows, 6144 deep two and four alike (-9%),
+//       14336 30.4 -> 27.3, four 25.4
+//   4096 outputs, up to 16 rows, which memory bounds: 8 rows gain 3% at most,
+//       16 with two 4096 deep 1%, 6144 6%, 14336 5%, with four 3 and 8%
+//   1280 outputs, whose own tiles of 48 and 80 rows are one round of workgroups:
+//       36 rows, 3136 deep 8.2 -> 8.7, 4608 9.7 -> 9.5, 70 and 90 rows 1 to 4% and
+//       0 to 2% slower to 6016 deep; 60 and 110 rows gain as beside it
+// Five shares or more of 2048 x 4096 lose (16 rows 8.4 with four, 9.3 with eight).
+// Of 2900 products of 1 to 128 rows, 768 to 5120 outputs and 2048 to 19456 deep
+// three are more than 2% slower by it, 4% at most (70 rows of 768 x 3136).
 extern "C" int ll_row_gemm_joined(int N, int M, int K) {
   const int more = ll_row_gemm_shares(N, M, K);
   if (more > 1 || N <= 0 || N > 128 || M < 768 || M > 4096 || M % 4)
     return more;
+  int shares = 1;
   if (M <= 2048) {
-    if (K < 2816) return 1;
-    return N > 64 && M > 1536 && K < 4096 ? 2 : 4;
+    if (K >= (M > 1536 && N <= 64 ? 3072 : 2816))
+      shares = N > 64 && M > 1024 && K <= 4096 ? 2 : 4;
+  } else if (N > 64) {
+    shares = K >= 4096 ? 2 : 1;
+  } else if (N > 16) {
+    shares = K >= 6144 ? 4 : (K >= 3072 ? 2 : 1);
+  } else if (N >= 12) {
+    shares = K >= 12288 ? 4 : (K >= 6144 ? 2 : 1);
   }
-  if (N > 64) return K >= 4096 ? 2 : 1;
-  return K >= (N > 16 ? 3072 : (N > 8 ? 6144 : 1 << 30)) ? 4 : 1;
+  if (M > 1024 && M < 1408 &&
+      ((N > 32 && N <= 48 && K < 4608) || (N > 64 && N <= 96)))
+    shares = 1;
+  while (shares > 1 &&
+         share_blocks(N, M, share_tile(N, M, shares), shares) > 256)
+    shares /= 2;
+  return shares;
 }
 
 extern "C" int ll_rmsnorm_join(void* out, const void* ws, int shares,
