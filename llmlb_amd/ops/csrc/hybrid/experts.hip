@@ -4,6 +4,8 @@
 // with act(z) = max(z, 0)^2 or none.
 //  * expert_float_kernel  32 bits by float_tile.h
 //  * expert_rows_kernel   other sizes, tiles of 32 pairs x 64 outputs
+#include <math.h>
+
 #include "experts.h"
 #include "float_tile.h"
 
@@ -135,23 +137,58 @@ static bool expert_float_ok(const ExpertRows& p) {
          p.n_pairs / 16 + p.E < 65536;
 }
 
-// By the pairs an expert has: few, of deep products, in tiles of 16, whose waves
-// share the depth; larger tiles, which take less apart, where they fill the chip.
-// us, expert_rows -> here, 16 experts, 4 a token, up (256 outputs, 1024 deep) and
-// down (1024, 256 deep): 20 tokens 87 -> 7, 28 -> 6; 100 101 -> 8, 32 -> 7; 300 173 ->
-// 12, 89 -> 12; 1200 377 -> 27, 231 -> 35.  The tiles of 16, 32 and 48 x 32 and of 48
-// and 64 x 64 at 100 tokens 7.6, 8.9, 10.4, 14.0, 16.7 up and 9.6, 7.4, 11.0, 9.0, 9.9
-// down, at 300 14.7, 13.5, 11.8, 15.3, 19.0 and 22, 16.8, 20, 12.2, 14.2, at 600 22.3,
-// 20.4, 21.1, 29.8, 30.8 and 42, 29, 38, 21, 21.
-static int expert_float_pick(const ExpertRows& p) {
+// Tiles that there are: how many a compute unit is taken to have at once, us of
+// one 1024 deep where each unit has one and where each has all of them, of the
+// beginning and end, and of every full round more.  Fitted to 328 products: 4 to 256
+// experts, 1 to 8 a token, 1 to 4096 tokens, 96 to 4096 outputs and as deep, weights
+// from HBM.  Of 234 others the tile taken is 2.2% slower than the fastest on average
+// and 20 are more than 10% slower, 28% at most (by pairs an expert and the depth
+// alone, from 16 experts of 1024 x 256, 5.4%, 47 and 46%).  us, expert_rows_kernel ->
+// these, 16 experts, 4 a token, up (256 outputs, 1024 deep) and down (1024, 256 deep):
+// 20 tokens 138 -> 8.4, 38 -> 7.9; 100 155 -> 10.9, 46 -> 10.4; 300 172 -> 20, 90 ->
+// 17.5; 1200 376 -> 27, 231 -> 37.
+struct ExpertTileTime {
+  int rows, cols, at_once;
+  float one, all, ends, more;
+};
+static const ExpertTileTime EXPERT_TILES[] = {
+    {16, 32, 3, 2.3f, 6.5f, 6.8f, 1.f},  {32, 32, 2, 3.2f, 6.4f, 6.8f, 3.3f},
+    {48, 32, 2, 4.3f, 10.4f, 7.f, 1.f},  {48, 64, 2, 6.9f, 13.5f, 6.9f, 0.f},
+    {64, 64, 2, 6.5f, 13.5f, 8.2f, 0.f}};
+
+// The tile that is estimated to take least.  An expert has its share of the pairs
+// and as many more as their root, by which shares differ.
+static int expert_float_tile(const ExpertRows& p) {
   const int experts = p.E < p.n_pairs ? p.E : p.n_pairs;
-  const int each = p.n_pairs / experts;
-  const bool deep = p.K >= 512;
-  if (((each + 47ll) / 48) * experts * ((p.N + 63) / 64) >= 384)
-    return each < 350 ? expert_float<3, 4, 4>(p) : expert_float<4, 4, 4>(p);
-  if (each <= (deep ? 25 : 8)) return expert_float<1, 2, 8>(p);
-  return each <= 64 || !deep ? expert_float<2, 2, 8>(p)
-                             : expert_float<3, 2, 8>(p);
+  const float each = (float)p.n_pairs / experts, most = each + sqrtf(each);
+  int best = 0;
+  float least = 0.f;
+  for (int t = 0; t < 5; ++t) {
+    const ExpertTileTime& at = EXPERT_TILES[t];
+    const float tiles = each < 4.f * at.rows ? ceilf(most / at.rows)
+                                             : each / at.rows + 0.5f;
+    const long long n =
+        (long long)(experts * tiles) * ((p.N + at.cols - 1ll) / at.cols);
+    const int round = 256 * at.at_once, rest = (int)(n % round);
+    const float full = (float)(n / round);
+    float us = full * at.all;
+    if (rest)
+      us += at.one + (at.all - at.one) * (float)((rest - 1) / 256) /
+                         (float)(at.at_once - 1);
+    us = us * ((float)p.K / 1024.f) + at.ends + full * at.more;
+    if (t == 0 || us < least) least = us, best = t;
+  }
+  return best;
+}
+
+static int expert_float_pick(const ExpertRows& p) {
+  switch (expert_float_tile(p)) {
+    case 0: return expert_float<1, 2, 8>(p);
+    case 1: return expert_float<2, 2, 8>(p);
+    case 2: return expert_float<3, 2, 8>(p);
+    case 3: return expert_float<3, 4, 4>(p);
+    default: return expert_float<4, 4, 4>(p);
+  }
 }
 
 extern "C" int hy_expert_rows(void* out, const void* in, const void* w,
