@@ -157,3 +157,49 @@ def test_two_parts(kv, D):
     assert ((out.double() - ref).abs() <= bound).all()
     if D == 128:
         test_page_attention_fp8(2 * kv, kv, 2)
+
+
+# A wave looks up the pages of 32 pairs at a time: tokens just before, at and behind
+# its second and third look, 4096 apart for four waves and 8192 for eight (144
+# workgroups that would be two parts); the first waves look, and the others do not
+@pytest.mark.parametrize("D,fp8", [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("kv,parts,lens", [
+    (1, 1, [4096, 4097, 4129, 4225, 4240, 8190, 8193, 8400, 40]),
+    (2, 1, [12289, 3, 5000]), (16, 2, [8192, 8193, 8450, 70, 1, 16385, 300, 33,
+                                       9000]),
+    (1, 3, [12288, 12289, 12400, 24577])])
+def test_pages_of_long_sequences(D, fp8, kv, parts, lens):
+    heads = 2 * kv
+    g = torch.Generator(device=DEV).manual_seed(D + kv)
+    per = [-(-n // 16) for n in lens]
+    ids = torch.randperm(sum(per), generator=g, device=DEV).int() + 1
+    bt = torch.zeros(len(lens), max(per) + 3, dtype=torch.int32, device=DEV)
+    for s, part in enumerate(ids.split(per)):
+        bt[s, :per[s]] = part
+    shape = (sum(per) + 1, kv, 16, D)
+    q = torch.randn(len(lens), heads, D, generator=g, device=DEV).bfloat16()
+    caches, scales, wide = [], [], []
+    for _ in range(2):
+        t = torch.randn(shape, generator=g, device=DEV)
+        if fp8:
+            s = torch.rand(shape[:3], generator=g, device=DEV) * 0.01 + 0.001
+            t = (t / s[..., None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+            wide.append(t.float() * s[..., None])
+            caches.append(t.view(torch.uint8))
+            scales.append(s)
+        else:
+            caches.append(t.bfloat16())
+            wide.append(caches[-1])
+    n = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    ref, bound = _exact(q, *wide, bt, n, D ** -0.5)
+    for s, tokens in enumerate(lens):           # nothing behind the end is read
+        if tokens % 16:
+            page = bt[s, per[s] - 1].long()
+            for c in caches:
+                c[page, :, tokens % 16:] = 0x7F if fp8 else float("nan")
+            for c in scales:
+                c[page, :, tokens % 16:] = float("nan")
+    more = dict(k_scale=scales[0], v_scale=scales[1]) if fp8 else {}
+    out = ops.paged_attn_decode(q, *caches, bt, n, D ** -0.5, n_parts=parts,
+                                **more)
+    assert ((out.double() - ref).abs() <= bound).all()
