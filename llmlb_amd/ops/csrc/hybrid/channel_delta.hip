@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     for (int k = 0; k < G; ++k) {
 #pragma unroll
       for (int i = 0; i < N; ++i)
-        f[k][i] = decay_t<T>(f[k][i] + bias[i], rate[i]);
+        f[k][i] = decay_t<T, true>(f[k][i] + bias[i], rate[i]);
       store_some<N, VEC>(ws + (size_t)(t + k) * at.size + at.g + j, valid,
                          f[k]);
     }

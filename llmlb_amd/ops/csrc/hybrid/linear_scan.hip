@@ -487,13 +487,11 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(
     float* __restrict__ g, const T* __restrict__ dec,
     const float* __restrict__ bias, int n_tok, int C, float rate) {
   constexpr int N = VEC ? 8 : 1;
-  const int across = (C + 256 * N - 1) / (256 * N);
-  const int c = (blockIdx.x % across * 256 + threadIdx.x) * N;
+  const int c = (blockIdx.y * 256 + threadIdx.x) * N;
   if (c >= C) return;
   float b[N];
   load_run<N, VEC>(bias + c, b);
-  const int step = gridDim.x / across;
-  for (int t = blockIdx.x / across; t < n_tok; t += step) {
+  for (int t = blockIdx.x; t < n_tok; t += gridDim.x) {
     float f[N];
     load_run<N, VEC>(dec + (size_t)t * C + c, f);
 #pragma unroll
@@ -899,7 +897,7 @@ int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
   if (n_tok <= 0 || C <= 0) return 0;
   const bool vec = C % 8 == 0;
   const int cols = vec ? 2048 : 256;
-  const dim3 grid((n_tok < 2048 ? n_tok : 2048) * ((C + cols - 1) / cols));
+  const dim3 grid(n_tok < 2048 ? n_tok : 2048, (C + cols - 1) / cols);
 #define GO(VEC)                                                          \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                    \
       (gla_decay_kernel<T, VEC>), grid, dim3(256), 0,                    \

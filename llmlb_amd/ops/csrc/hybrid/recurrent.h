@@ -102,15 +102,21 @@ template <typename T>
 __device__ __forceinline__ float sigmoid_t(float x) {
   return sizeof(T) == 2 ? 1.f / (1.f + __expf(-x)) : sigmoid_f(x);
 }
-template <typename T>
+// (BOTH: log(1 + e) and its series are made and one is taken, which is less than
+// a branch where nothing else hides it, and more where many numbers do.)
+template <typename T, bool BOTH = false>
 __device__ __forceinline__ float decay_t(float z, float rate) {
   if (sizeof(T) == 2) {
-    const float e = __builtin_amdgcn_exp2f(-LOG2E * fabsf(z));
-    // log(1 + e) by its series where 1 + e would lose e; both are made, which
-    // is less than a branch for every number
-    constexpr float LN2 = 0.6931471805599453f;
-    const float l = LN2 * __builtin_amdgcn_logf(1.f + e);
-    const float lp = e < 1e-3f ? e * (1.f - 0.5f * e) : l;
+    const float e = __expf(-fabsf(z));
+    // log(1 + e) by its series where 1 + e would lose e
+    float lp;
+    if (BOTH) {
+      constexpr float LN2 = 0.6931471805599453f;
+      const float l = LN2 * __builtin_amdgcn_logf(1.f + e);
+      lp = e < 1e-3f ? e * (1.f - 0.5f * e) : l;
+    } else {
+      lp = e < 1e-3f ? e * (1.f - 0.5f * e) : __logf(1.f + e);
+    }
     return __expf(-rate * (fmaxf(z, 0.f) + lp));
   }
   return expf(-rate * softplus_f(z));
