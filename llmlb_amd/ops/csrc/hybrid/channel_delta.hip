@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
       q.start(t, pos_[t], ts, row_[t]);
       k.start(t, pos_[t], ts, row_[t]);
     };
-    walk_tokens<RPL <= 8 ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
+    walk_tokens<VEC && RPL <= 8 ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
       constexpr int G = decltype(n)::value;
       float xq[G][RPL], xk[G][RPL];
 #pragma unroll
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     ConvRun<T, N, VEC> v(proj, ld, ring, wconv, nullptr, C, taps,
                          2 * KH * D + j, valid);
     auto start = [&](int t, int ts) { v.start(t, pos_[t], ts, row_[t]); };
-    walk_tokens<4>(tstart_, t0, t1, start, [&](int t, auto n) {
+    walk_tokens<VEC ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
       constexpr int G = decltype(n)::value;
       float x[G][N];
 #pragma unroll
@@ -238,7 +238,8 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     }
   };
   int t = t0;
-  for (; t + 4 <= t1; t += 4) decays(t, std::integral_constant<int, 4>{});
+  if (VEC)
+    for (; t + 4 <= t1; t += 4) decays(t, std::integral_constant<int, 4>{});
   for (; t < t1; ++t) decays(t, std::integral_constant<int, 1>{});
 }
 

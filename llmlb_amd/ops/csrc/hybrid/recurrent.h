@@ -187,16 +187,18 @@ struct ConvRun {
 template <int GROUP, class Start, class Go>
 __device__ __forceinline__ void walk_tokens(const int* tstart, int t0, int t1,
                                             Start start, Go go) {
+  constexpr std::integral_constant<int, 1> ONE{};
   for (int t = t0; t < t1;) {
     const int first = tstart[t];
     if (t == t0 || t == first) start(t, first);
-    if (t + GROUP <= t1 && tstart[t + GROUP - 1] <= t) {
-      go(t, std::integral_constant<int, GROUP>{});
-      t += GROUP;
-    } else {
-      go(t, std::integral_constant<int, 1>{});
-      ++t;
+    if constexpr (GROUP > 1) {
+      if (t + GROUP <= t1 && tstart[t + GROUP - 1] <= t) {
+        go(t, std::integral_constant<int, GROUP>{});
+        t += GROUP;
+        continue;
+      }
     }
+    go(t++, ONE);
   }
 }
 
