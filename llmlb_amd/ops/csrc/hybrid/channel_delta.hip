@@ -109,11 +109,16 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
 // sections start on whole vectors.
 //
 // Bound by memory: 16384 tokens of 16 heads of 128 read 270 MB and write 540, and
-// take 178 us, 4.5 TB/s.  What counts is that all of a row is written at about
-// the same time: with the workgroups of one part side by side, 4 KB of every row,
-// it is 207.  Four tokens are asked for at once, for a load behind a store is
-// there only when the store is: one at a time 227 (8 channels a lane, which
-// leave room for fewer waves), four 217.
+// take 175 us, 4.6 TB/s.  What counts where more is written than the last cache
+// holds, 256 MB, is that all of a row is written at about the same time: with the
+// workgroups of one part side by side, 4 KB of every row, it is 217.  What it holds
+// is better written part by part, where no XCD gets more of the heavier parts than
+// another (together -> apart, us: 16 heads of 128, 6000 tokens, 197 MB 74 -> 69; 32
+// heads, 2048, 134 MB 46 -> 36; 4 of 256, 16384, 235 MB 123 -> 109).  Whole vectors
+// are asked for four tokens at once, for a load behind a store is there only when
+// the store is: one at a time 227 (8 channels a lane, which leave room for fewer
+// waves).  Single numbers are not: four tokens of them leave room for two waves in
+// the place of three (2 heads of 100 and 36, 16384 tokens 136 us, one at a time 75).
 #define PREP_TOK 16
 template <int LANES>
 __device__ __forceinline__ float row_sum(float x) {
@@ -129,11 +134,12 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
     int KH, int H, int D, int V, int taps, float q_scale, int qk_blocks,
     int v_blocks, int parts) {
   constexpr int N = LANES == 32 ? 4 : 8;
-  const int t0 = blockIdx.x / parts * PREP_TOK;
+  const RunPart own = run_part(parts);
+  const int t0 = own.run * PREP_TOK;
   const int t1 = t0 + PREP_TOK < n_tok ? t0 + PREP_TOK : n_tok;
   const int C = 2 * KH * D + H * V;
   const WsLayout at(KH, H, D, V);
-  int y = blockIdx.x % parts;
+  int y = own.part;
   if (y < qk_blocks) {
     const int unit = y * (256 / LANES) + threadIdx.x / LANES;
     if (unit >= KH) return;  // whole groups of lanes
@@ -577,7 +583,13 @@ int hy_delta_prep(void* ws, const void* proj, int ld, int b_off,
     const int v_blocks = (H * V + n - 1) / n;
     const int g_blocks = (H * D + n - 1) / n;
     const int parts = qk_blocks + v_blocks + g_blocks;
-    const dim3 grid((n_tok + PREP_TOK - 1) / PREP_TOK * parts);
+    // 32 bits read twice as much, 16 us, apart -> together, 5 and 12 parts: 150 MB
+    // 95.8 -> 91.5, 134 MB 86 -> 79; but three, 235 MB 138 -> 182
+    const long long writes = 4ll * n_tok * WsLayout(KH, H, D, V).size;
+    const bool large =
+        whole && writes > (dtype == 1 && parts > 4 ? 128ll : 256ll) << 20;
+    const dim3 grid =
+        run_parts((n_tok + PREP_TOK - 1) / PREP_TOK, parts, large);
 #define RUN(RPL, LANES, VEC)                                                 \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                        \
       (delta_prep_run_kernel<T, RPL, LANES, VEC>), grid, dim3(256), 0,       \

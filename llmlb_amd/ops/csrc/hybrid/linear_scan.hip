@@ -523,9 +523,14 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(
 }
 
 // The same for at most TAPS_MAX taps: 8 channels a thread, each input of
-// PREP_TOK successive tokens read once, and four of them at once: a load behind
-// a store is there only when the store is.  16384 tokens of 12288 channels 106 ->
-// 81 us.
+// PREP_TOK successive tokens read once, and four of them at once where they are
+// vectors of 16 bits: a load behind a store is there only when the store is.  (Not
+// of 32 bits, 16384 tokens of 2048 channels 59 -> 63 us.)  What the last cache does
+// not hold, 256 MB read and written, a row's workgroups go through side by side, and
+// what it holds one part after the other: of 2304 channels every other workgroup has
+// an eighth of the work, which side by side is every other XCD's.  us, one token at
+// a time and parts apart -> this, 16384 tokens: 6144 channels 103 -> 82, 12288 200 ->
+// 162, 2304 46 -> 35 (side by side 41); 2048 tokens of 6144 21.3 -> 16.5.
 #define PREP_TOK 16
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void ssm_conv_run_kernel(
@@ -535,9 +540,10 @@ __global__ __launch_bounds__(256) void ssm_conv_run_kernel(
     const int* __restrict__ row_, const int* __restrict__ tstart_, int n_tok,
     int C, int taps) {
   const int across = (C + 2047) / 2048;
-  const int t0 = blockIdx.x / across * PREP_TOK;
+  const RunPart own = run_part(across);
+  const int t0 = own.run * PREP_TOK;
   const int t1 = t0 + PREP_TOK < n_tok ? t0 + PREP_TOK : n_tok;
-  const int c = (blockIdx.x % across * 256 + threadIdx.x) * 8;
+  const int c = (own.part * 256 + threadIdx.x) * 8;
   if (c >= C) return;
   const int valid = C - c < 8 ? C - c : 8;
   ConvRun<T, 8, VEC> run(proj, ld, ring, wconv, bias, C, taps, c, valid);
@@ -982,14 +988,17 @@ int hy_ssm_prep(void* xbc, void* steps, const void* proj, int ld, int dt_off,
   if ((long long)n_tok * H >= (1ll << 30)) return -2;
   hipStream_t st = (hipStream_t)stream;
   if (taps <= TAPS_MAX) {
-    const dim3 grid((n_tok + PREP_TOK - 1) / PREP_TOK * ((C + 2047) / 2048));
+    const bool vec = C % 8 == 0 && ld % 8 == 0;
+    const bool large = vec && dtype == 0 && 4ll * n_tok * C > 256ll << 20;
+    const dim3 grid = run_parts((n_tok + PREP_TOK - 1) / PREP_TOK,
+                                (C + 2047) / 2048, large);
 #define GO(VEC)                                                              \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                        \
       (ssm_conv_run_kernel<T, VEC>), grid, dim3(256), 0, st, (T*)xbc,        \
       (const T*)proj, ld, (const T*)ring, (const float*)wconv,               \
       (const float*)bias, (const int*)pos, (const int*)row,                  \
       (const int*)tstart, n_tok, C, taps))
-    if (C % 8 == 0 && ld % 8 == 0) GO(true);
+    if (vec) GO(true);
     else GO(false);
 #undef GO
   } else {

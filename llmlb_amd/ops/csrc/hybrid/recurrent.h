@@ -181,6 +181,20 @@ struct ConvRun {
   }
 };
 
+// A row's parts, a workgroup each, of runs of rows: side by side where
+// ``together``, else a part of all runs after the other.
+struct RunPart {
+  int run, part;
+};
+__host__ inline dim3 run_parts(int runs, int parts, bool together) {
+  return together ? dim3((unsigned)runs * (unsigned)parts)
+                  : dim3((unsigned)runs, (unsigned)parts);
+}
+__device__ __forceinline__ RunPart run_part(int parts) {
+  if (gridDim.y > 1) return RunPart{(int)blockIdx.x, (int)blockIdx.y};
+  return RunPart{(int)blockIdx.x / parts, (int)blockIdx.x % parts};
+}
+
 // Tokens t0 .. t1 - 1 in order, some at a time: start(t, its sequence's first)
 // where the tokens before t have not been walked, go(t, n) for the next n.  n,
 // a constant, is GROUP where all of these are of one sequence, else 1.

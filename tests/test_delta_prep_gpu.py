@@ -86,3 +86,79 @@ def test_delta_prep(KH, H, D, V, taps, dtype):
         assert (got - want).abs().max() <= 2.0 ** -16 * max(
             1.0, want.abs().max())
         assert (got - want).norm() <= 1e-6 * want.norm()
+
+
+def _place(tokens, sequences):
+    """pos, row and first token of each, of equal sequences."""
+    at = torch.arange(tokens, dtype=torch.int32, device=DEV)
+    row = at // (tokens // sequences)
+    first = row * (tokens // sequences)
+    return at - first, row, first
+
+
+def _prep(proj, dec, ring, where, w, a_log, bias, size, taps):
+    ws = torch.full((len(proj), int(hy.native().hy_delta_ws_floats(
+        *map(hy._i, size)))), float("nan"), device=DEV)
+    pos, row, first = where
+    assert hy.native().hy_delta_prep(
+        _ptr(ws), _ptr(proj), hy._i(proj.stride(0)),
+        hy._i(2 * size[0] * size[2] + size[1] * size[3]), _ptr(dec),
+        _ptr(ring), _ptr(w), _ptr(a_log), _ptr(bias), _ptr(pos), _ptr(row),
+        _ptr(first), hy._i(len(proj)), *map(hy._i, size), hy._i(taps),
+        hy._f(0.1), hy._dt(proj.dtype), _stream()) == 0
+    return ws
+
+
+# 4100 tokens of 16 and 32 heads of 128 write more than 128 and 256 MB, whose
+# workgroups are in another order than those of the sequences one by one
+@pytest.mark.parametrize("heads, dtype", [(32, torch.bfloat16),
+                                          (16, torch.float32)])
+def test_many_tokens(heads, dtype):
+    T, n, taps, size = 4100, 4, 4, (heads, heads, 128, 128)
+    g = torch.Generator(device=DEV).manual_seed(heads)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device=DEV)
+
+    C = 3 * heads * 128
+    proj, dec = rand(T, C + heads).to(dtype), rand(T, heads * 128).to(dtype)
+    ring = rand(n, taps, C).to(dtype)
+    rest = rand(taps, C), rand(heads), rand(heads * 128), size, taps
+    got = _prep(proj, dec, ring, _place(T, n), *rest)
+    each = T // n
+    for s in range(n):
+        part = slice(s * each, (s + 1) * each)
+        want = _prep(proj[part], dec[part], ring[s:s + 1], _place(each, 1),
+                     *rest)
+        used = 3 * heads * 128 + heads * 128 + 2 * heads
+        assert torch.equal(got[part, :used], want[:, :used])
+        assert not want[:, :used].isnan().any()
+
+
+# 11000 tokens of 6144 channels are more than 256 MB read and written
+@pytest.mark.parametrize("T", [11000, 1000])
+def test_state_space_convolution(T):
+    C, H, n, taps, dtype = 6144, 8, 4, 4, torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(T)
+    proj = torch.randn(T, C + H, generator=g, device=DEV).to(dtype)
+    ring = torch.randn(n, taps, C, generator=g, device=DEV).to(dtype)
+    w = torch.randn(taps, C, generator=g, device=DEV)
+    b = torch.randn(C, generator=g, device=DEV)
+    heads = torch.randn(3, H, generator=g, device=DEV)
+
+    def prep(proj, ring, where):
+        out = torch.full((len(proj), C), float("nan"), dtype=dtype,
+                         device=DEV)
+        assert hy.native().hy_ssm_prep(
+            _ptr(out), None, _ptr(proj), hy._i(C + H), hy._i(C), _ptr(ring),
+            _ptr(w), _ptr(b), _ptr(heads), *map(_ptr, where),
+            hy._i(len(proj)), hy._i(C), hy._i(H), hy._i(taps), hy._i(0),
+            _stream()) == 0
+        return out
+
+    got, each = prep(proj, ring, _place(T, n)), T // n
+    for s in range(n):
+        part = slice(s * each, (s + 1) * each)
+        want = prep(proj[part], ring[s:s + 1], _place(each, 1))
+        assert torch.equal(got[part], want)
+        assert not want.isnan().any()
