@@ -211,10 +211,11 @@ void expert_tile_kernel(
   }
 }
 
-// The rows of experts' lists, for tile_product.  A tile's part of its list is
-// in LDS before the copies of its rows begin: asked for there, it would have
-// to wait for all copies under way.
-template <int BM, int BN>
+// The rows of experts' lists, for tile_product.  AHEAD: a tile's part of its
+// list is in LDS before the copies of its rows begin; asked for there, it would
+// have to wait for all copies under way.  It is on its way for a step at least,
+// so tiles have two or more.
+template <int BM, int BN, bool AHEAD>
 struct ListRows {
   // of tiles that are fetched, copied, computed and stored at a time
   static constexpr int PARTS = 8;
@@ -240,11 +241,15 @@ struct ListRows {
     return found->get(counts, E, j < whole ? j : j - whole, j >= whole);
   }
   __device__ __forceinline__ At at(int i) const {
-    return At{tile(i), part(i), i % n_blocks * BN};
+    const ExpertTile t = tile(i);
+    return At{t,
+              AHEAD ? part(i) : pairs + (size_t)t.expert * n_tok + t.first,
+              i % n_blocks * BN};
   }
   // 64 numbers a wave; past the end the last one again
   __device__ __forceinline__ void fetch(int i) const {
     static_assert(BM % WAVE == 0, "whole waves");
+    if (!AHEAD) return;
     const int at = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
     if (at >= BM) return;
     const ExpertTile t = tile(i);
@@ -252,13 +257,16 @@ struct ListRows {
     copy_words_to_lds(pairs + (size_t)t.expert * n_tok + t.first + r,
                       lds_byte(part(i) + at));
   }
-  __device__ __forceinline__ void fetched() const { wait_barrier<0>(); }
+  __device__ __forceinline__ void fetched() const {
+    if (AHEAD) wait_barrier<0>();
+  }
   __device__ __forceinline__ const bf16_t* x(const At&) const { return in; }
   __device__ __forceinline__ const bf16_t* w(const At& a) const {
     return w_ + (size_t)a.t.expert * N * K;
   }
   __device__ __forceinline__ unsigned x_offset(const At& a, int r) const {
-    return (unsigned)(a.list[r] / div) * (unsigned)K;
+    const int i = AHEAD || r < a.t.n ? r : a.t.n - 1;
+    return (unsigned)(a.list[i] / div) * (unsigned)K;
   }
   __device__ __forceinline__ long long row(const At& a, int r) const {
     return r < a.t.n ? a.list[r] : -1;
@@ -270,23 +278,26 @@ struct ListRows {
 
 // Bound by the matrix cores' power and, for shallow products, by what they
 // write: 16384 tokens with 4 of 16 experts, us, the best of the tiles above
-// -> here: 1024 to 256 wide 60 -> 43, back 61 -> 50; 2048 to 512 162 -> 122,
-// back 211 -> 169; 12288 tokens, 4096 to 1280 404 -> 390 and back 503 -> 473
-// against lists asked for from memory and results stored at once (2048 to
-// 512 so 134, back 175).  Without any stores the way back of 512 deep takes
-// 116 us; they alone take 41.  256 x 256 leaves no LDS for the tiles' numbers;
-// 256 x 128 and 128 x 256 read more (2048 to 512: 146, 156).
-template <int BM, int BN, int WM, int WN, int D, int KIND>
+// -> here: 1024 to 256 wide 60 -> 46, back 61 -> 52; 2048 to 512 162 -> 117,
+// back 211 -> 176.  Of that, lists asked for from memory and results stored at
+// once -> lists in LDS -> results held, sides in turn: 2048 to 512 120 -> 118 ->
+// 117, back 178 -> 180 -> 175; 4096 to 1280 555 -> 545 -> 538, back 677 -> 666 ->
+// 645; 1024 to 256 46 -> 45 -> 46, back 54 -> 52 -> 52; back 128 deep to 2048 61.7 ->
+// 57 -> 59; 4096 tokens back 2048 to 512 46 -> 46 -> 43.  One step deep both lose:
+// 64 to 2048 73 -> 81.  Without any stores the way back of 512 deep takes 116 us;
+// they alone take 41.  256 x 256 leaves no LDS for the tiles' numbers; 256 x 128 and
+// 128 x 256 read more (2048 to 512: 146, 156).
+template <int BM, int BN, int WM, int WN, int D, int KIND, bool DEEP>
 __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4)
 void expert_product_kernel(bf16_t* __restrict__ out,
-                           ListRows<BM, BN> rows) {
+                           ListRows<BM, BN, DEEP> rows) {
   __shared__ ExpertTiles<BM> tiles;
   if (threadIdx.x < WAVE) tiles.count(rows.counts, rows.E);
   __syncthreads();
-  __shared__ int parts[ListRows<BM, BN>::PARTS * BM];
+  __shared__ int parts[DEEP ? rows.PARTS * BM : 1];
   rows.found = &tiles;
   rows.parts = parts;
-  tile_product<BM, BN, WM, WN, D, KIND, false, true>(
+  tile_product<BM, BN, WM, WN, D, KIND, false, DEEP>(
       rows, out, rows.N, rows.N, rows.K, RowAct{KIND, 0, 0.f, 0.f});
 }
 
@@ -297,12 +308,12 @@ struct ExpertProduct {
   int E, N, K, div, n_tok, n_pairs;
   hipStream_t stream;
 };
-template <int BM, int BN, int WM, int WN, int D, int KIND>
+template <int BM, int BN, int WM, int WN, int D, int KIND, bool DEEP>
 static int expert_product(const ExpertProduct& p) {
-  auto* kernel = &expert_product_kernel<BM, BN, WM, WN, D, KIND>;
+  auto* kernel = &expert_product_kernel<BM, BN, WM, WN, D, KIND, DEEP>;
   constexpr int lds = ((D + 1) * BM + D * BN) * DEPTH * 2;
   static_assert(lds + sizeof(ExpertTiles<BM>) +
-                        ListRows<BM, BN>::PARTS * BM * 4 <= 160 * 1024,
+                        ListRows<BM, BN, DEEP>::PARTS * BM * 4 <= 160 * 1024,
                 "LDS of a compute unit");
   static const hipError_t sized = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
@@ -314,7 +325,7 @@ static int expert_product(const ExpertProduct& p) {
       ((long long)p.n_pairs / BM + (p.E < p.n_pairs ? p.E : p.n_pairs)) * nb;
   if (most >= 1ll << 27) return -2;
   const long long per = (most + 7) / 8;
-  const ListRows<BM, BN> rows{p.in, p.w, p.counts, p.pairs, p.E, p.N,
+  const ListRows<BM, BN, DEEP> rows{p.in, p.w, p.counts, p.pairs, p.E, p.N,
                               p.K,  p.div, p.n_tok, nb, nullptr, nullptr};
   hipLaunchKernelGGL(kernel, dim3(8 * (unsigned)(per < 32 ? per : 32)),
                      dim3(WM * WN * 64), lds, p.stream, p.out, rows);
@@ -364,14 +375,17 @@ int hy_expert_tiles(void* out, const void* in, const void* w,
     case 1: GO(256, 256, 4, 4, 64, 2); break;
     case 2: GO(128, 256, 2, 4, 32, 3); break;
     case 3:
-      // (a tile's part of its list is under way for a step at least)
-      if (K % DEPTH == 0 && K >= 2 * DEPTH && near) {
+      if (K % DEPTH == 0 && near) {
         const ExpertProduct p{(bf16_t*)out, (const bf16_t*)in,
                               (const bf16_t*)w, (const int*)counts,
                               (const int*)pairs, E, N, K, div, n_tok,
                               n_pairs, (hipStream_t)stream};
-        return act ? expert_product<192, 256, 2, 4, 2, RELU2>(p)
-                   : expert_product<192, 256, 2, 4, 2, PLAIN>(p);
+        // a tile of one step has none to fetch and to store in
+        if (K == DEPTH)
+          return act ? expert_product<192, 256, 2, 4, 2, RELU2, false>(p)
+                     : expert_product<192, 256, 2, 4, 2, PLAIN, false>(p);
+        return act ? expert_product<192, 256, 2, 4, 2, RELU2, true>(p)
+                   : expert_product<192, 256, 2, 4, 2, PLAIN, true>(p);
       }
       GO(256, 256, 4, 4, 64, 2);
       break;

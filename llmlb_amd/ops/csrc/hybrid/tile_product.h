@@ -228,11 +228,8 @@ __device__ __forceinline__ void tile_product(const Source& source,
   int sent = SENDS;     // of the last tile's
   bool stored = false;  // its stores are of all lanes
   auto held_at = source.at(tile);
-  auto store = [&](const auto& at, int i, u32x4 v) {
-    int lane_ = lane;
-    // (places of what is held are not to be kept through the steps)
-    if (HELD) asm volatile("" : "+v"(lane_));
-    const long long n = source.row(at, wm + i / GROUPS * 16 + (lane_ & 15));
+  // group i of the tile's row n of results
+  auto store = [&](const auto& at, long long n, int i, int lane_, u32x4 v) {
     const int m = at.m0 + (GATED ? wn / 2 : wn) + i % GROUPS * 32 +
                   (lane_ >> 4) * 8;
     if (n >= 0 && m < M)
@@ -243,7 +240,14 @@ __device__ __forceinline__ void tile_product(const Source& source,
       pick<0, SENDS>(sent++, [&](auto IS) {
         times<LATER>([&](auto IP) {
           constexpr int i = IS * LATER + IP;
-          if constexpr (i < STORES) store(held_at, i, held[i]);
+          if constexpr (i < STORES) {
+            int lane_ = lane;
+            // (places of what is held are not to be kept through the steps)
+            asm volatile("" : "+v"(lane_));
+            store(held_at,
+                  source.row(held_at, wm + i / GROUPS * 16 + (lane_ & 15)), i,
+                  lane_, held[i]);
+          }
         });
       });
   };
@@ -301,8 +305,11 @@ __device__ __forceinline__ void tile_product(const Source& source,
     sent = 0;
     RowAct as = act;
     as.kind = KIND;
+    long long n = 0;  // a row's place is looked up once
     times<STORES>([&](auto II) {
       constexpr int I = II, a = I / GROUPS;
+      if constexpr (!HELD && I % GROUPS == 0)
+        n = source.row(at, wm + a * 16 + (lane & 15));
       constexpr int b = I % GROUPS * (GATED ? 4 : 2);
       unsigned p[4];
 #pragma unroll
@@ -324,7 +331,7 @@ __device__ __forceinline__ void tile_product(const Source& source,
       }
       const u32x4 v{p[0], p[1], p[2], p[3]};
       if constexpr (HELD) held[I] = v;
-      else store(at, I, v);
+      else store(at, n, I, lane, v);
     });
     tile += slots;
     if (tile >= end) break;

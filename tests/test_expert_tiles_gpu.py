@@ -26,8 +26,8 @@ def _lists(T):
     return torch.tensor(sizes, dtype=torch.int32).to(DEV), pairs.to(DEV)
 
 
-# depths of two steps (the least; one step takes other tiles), of fewer steps
-# than a tile's stores take, as many and more; outputs that are no whole tiles
+# depths of one step, whose results are stored at once, of fewer steps than a
+# tile's held stores take, as many and more; outputs that are no whole tiles
 @pytest.mark.parametrize("act, div", [(1, TOP), (0, 1)])
 @pytest.mark.parametrize("N", [1024, 1544])
 @pytest.mark.parametrize("K", [64, 128, 192, 320, 384, 448, 1024])
@@ -61,3 +61,23 @@ def test_tiles(K, N, act, div):
             want, off = want ** 2, 2 * want * off + off ** 2
         bound = off + 2.0 ** -8 * (want.abs() + off)
         assert ((out[rows].double() - want).abs() <= bound).all()
+
+
+# ten tiles a workgroup: more than the lists in LDS have places
+@pytest.mark.parametrize("K", [64, 128, 192, 256])
+def test_many_tiles(K):
+    T, N, act, div = 16384, 1544, 1, TOP
+    counts, pairs = _lists(T)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randn(T, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(E, N, K, generator=g, device=DEV).mul_(
+        K ** -0.5).bfloat16()
+    outs = []
+    for tile in (3, 0):
+        out = torch.full((T * TOP, N), 7.0, device=DEV, dtype=torch.bfloat16)
+        assert hy.native().hy_expert_tiles(
+            _ptr(out), _ptr(x), _ptr(w), _ptr(counts), _ptr(pairs), hy._i(E),
+            hy._i(N), hy._i(K), hy._i(div), hy._i(act), hy._i(T),
+            hy._i(T * TOP), hy._i(tile), _stream()) == 0
+        outs.append(out)
+    assert torch.equal(*outs)
