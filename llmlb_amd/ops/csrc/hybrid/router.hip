@@ -9,7 +9,11 @@ __global__ __launch_bounds__(256) void route_kernel(Routing a) {
   route_block<NT>(a, blockIdx.x, lds);
 }
 
-template <typename T>
+// J experts of a wave at a time: their rows fly together (300 tokens of 1024
+// columns, 16 experts, 32 bits, one by one 30.5 us, four 11), as many as a wave
+// has, for each place is worked on (2000 tokens of 4100 columns, 4 experts, 16 bits,
+// one by one 18 us, four 28).
+template <typename T, int J>
 __global__ __launch_bounds__(256) void route_rows_kernel(Routing a) {
   extern __shared__ float lds[];
   const int E = a.E, top = a.top;
@@ -21,37 +25,35 @@ __global__ __launch_bounds__(256) void route_rows_kernel(Routing a) {
   const int t = blockIdx.x, wave = threadIdx.x / WAVE;
   const int lane = threadIdx.x & (WAVE - 1);
   const T* x = (const T*)a.h + (size_t)t * a.width;
-  // four experts of a wave at a time: their rows fly together (300 tokens of 1024
-  // columns, 16 experts, 32 bits, one by one 30.5 us, 11 this way); by vectors of
-  // four where all of them lie on whole ones
+  // by vectors of four where all rows lie on whole ones
   const bool whole = a.width % 4 == 0 &&
                      ((uintptr_t)a.h | (uintptr_t)a.w) % (4 * sizeof(T)) == 0;
-  for (int e0 = wave; e0 < E; e0 += 16) {
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    const T* r[4];
+  for (int e0 = wave; e0 < E; e0 += 4 * J) {
+    float acc[J] = {};
+    const T* r[J];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < J; ++j)
       r[j] = (const T*)a.w +
              (size_t)(e0 + 4 * j < E ? e0 + 4 * j : e0) * a.width;
     if (whole) {
 #pragma unroll 2
       for (int i = lane * 4; i < a.width; i += 4 * WAVE) {
-        float f[4], g[4][4];
+        float f[4], g[J][4];
         load4(x + i, f);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) load4(r[j] + i, g[j]);
+        for (int j = 0; j < J; ++j) load4(r[j] + i, g[j]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < J; ++j)
 #pragma unroll
           for (int c = 0; c < 4; ++c) acc[j] += f[c] * g[j][c];
       }
     } else {
       for (int i = lane; i < a.width; i += WAVE)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] += to_f(x[i]) * to_f(r[j][i]);
+        for (int j = 0; j < J; ++j) acc[j] += to_f(x[i]) * to_f(r[j][i]);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < J; ++j) {
       acc[j] = wave_sum(acc[j]);
       if (lane == 0 && e0 + 4 * j < E) s[e0 + 4 * j] = acc[j];
     }
@@ -88,9 +90,14 @@ extern "C" int hy_route(void* index, void* weight, void* counts, void* pairs,
     else GO(4);
 #undef GO
   } else {
-    HY_DTYPE(dtype, hipLaunchKernelGGL(
-        route_rows_kernel<T>, dim3(n_tok), dim3(256),
-        4 * (E + 2 * groups + 2 * top), st, a));
+#define GO(J)                                            \
+  HY_DTYPE(dtype, hipLaunchKernelGGL(                    \
+      (route_rows_kernel<T, J>), dim3(n_tok), dim3(256), \
+      4 * (E + 2 * groups + 2 * top), st, a))
+    if (E <= 4) GO(1);
+    else if (E <= 8) GO(2);
+    else GO(4);
+#undef GO
   }
   HY_CHECK();
   return 0;
