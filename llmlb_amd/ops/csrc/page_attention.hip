@@ -12,8 +12,8 @@
 // other waves, eight or more to a compute unit (a second stage of LDS in their
 // place was no faster), and the wave's own other half: the next keys are on their
 // way while values are worked on, the next values while keys are (us, both waited
-// for at once -> this: 64 sequences of 900 tokens 40.1 -> 38.5, 32 of 2000 e4m3 27.1
-// -> 26.0, 8 of 1000 12.7 -> 11.3, 10 of 100 6.7 -> 6.4).  Weights and sums stay
+// for at once -> this: 64 sequences of 675 to 900 tokens 40.1 -> 38.6, 32 of 1500 to
+// 2000 e4m3 25.5 -> 24.2, 8 of 1000 12.7 -> 11.2, 10 of 100 6.6 -> 6.4).  Weights and sums stay
 // floats: a weight enters its product as the sum of three bf16 numbers, which are
 // all of its 24 bits.
 //
@@ -22,7 +22,7 @@
 // part is all, it writes the result itself.
 //
 // Against a lane per part of a row, us (sequences, heads, tokens):
-//   bf16, 32 on 8 heads of 128: 64 x about 900 76 -> 39 (5.5 TB/s),
+//   bf16, 32 on 8 heads of 128: 64 x 675 to 900 76 -> 39 (5.5 TB/s),
 //     64 x 3600 255 -> 156 (6.2 TB/s), 1 x 4000 47 -> 16
 //   e4m3, the same heads: 64 x 900 70 -> 21; 32 x 2048 in two parts 28, in
 //     one of eight waves 25 (5.6 TB/s), 128 x 1500 56.  Values leave LDS as
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
     const int r = j * (1024 / A::ROW) + lane / A::PR;
     off[j] = r * A::ROW + (((lane % A::PR) ^ turn<A::ROW>(r)) * 16);
   }
-  // keys and values of pair i, with their scales
+  // keys of pair i, with the scales of both, and values
   auto copy = [&](int i, bool values) {
     const char* const from = values ? vc : kc;
     const unsigned there = to + (values ? 2 : 0) * A::BYTES;
@@ -142,12 +142,13 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
                 from + at + (FP8 && t && values ? off[j] ^ 64 : off[j])),
             there + t * A::BYTES + j * 1024);
     }
-    if (FP8 && lane < 32) {  // scales of 16 keys or values of each page
-      const int page = __builtin_amdgcn_readlane(ids, 2 * (i % 32) + 1);
-      const int page0 = __builtin_amdgcn_readlane(ids, 2 * (i % 32));
-      copy4_to_lds((values ? v_scale : k_scale) +
-                       ((size_t)(g ? page : page0) * G + kv) * PAGE + n,
-                   to + 4 * A::BYTES + (values ? 128 : 0));
+    if (FP8 && !values) {  // 16 of each page's keys, then of the values
+      const int page =
+          g & 1 ? __builtin_amdgcn_readlane(ids, 2 * (i % 32) + 1)
+                : __builtin_amdgcn_readlane(ids, 2 * (i % 32));
+      const float* s = g < 2 ? k_scale : v_scale;
+      copy4_to_lds(s + ((size_t)page * G + kv) * PAGE + n,
+                   to + 4 * A::BYTES);
     }
   };
 
@@ -164,8 +165,8 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
   float m = -1e30f, l = 0.f;
 #pragma unroll
   for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // copies of a pair's keys, or values
-  constexpr int HALF = 2 * A::CP + (FP8 ? 1 : 0);
+  // copies of a pair's values, and of its keys
+  constexpr int VALUES = 2 * A::CP, KEYS = VALUES + (FP8 ? 1 : 0);
   if (count) look_up(0);
 #pragma unroll
   for (int k = 0; k < KD; ++k) asm volatile("" : "+v"(qf[k]));
@@ -174,10 +175,10 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
     copy(0, true);
   }
   for (int i = 0; i < count; ++i) {
-    wait_copies<HALF>();  // the keys are there
+    wait_copies<VALUES>();  // the keys are there
     const int j0 = (first + i * W) * 32;  // the pair's first key
     const bool more = i + 1 < count;
-    f32x4 s[2];
+    f32x4 s[2], v_by[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -196,9 +197,11 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
         s[t] = mfma(kf, qf[k], s[t]);
       }
       f32x4 by = {scale, scale, scale, scale};
-      if (FP8)
-        by *= *reinterpret_cast<const f32x4*>(st + 4 * A::BYTES + t * 64 +
-                                              g * 16);
+      if (FP8) {
+        const char* const scales = st + 4 * A::BYTES + t * 64 + g * 16;
+        by *= *reinterpret_cast<const f32x4*>(scales);
+        v_by[t] = *reinterpret_cast<const f32x4*>(scales + 128);
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         s[t][r] = j0 + t * 16 + g * 4 + r < len ? s[t][r] * by[r] : -INFINITY;
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
       for (int v = 0; v < VT; ++v) o[v] *= keep;
     }
     if (more)
-      wait_copies<HALF>();
+      wait_copies<KEYS>();
     else
       wait_copies<0>();
     if (j0 + 32 > len) {
@@ -247,11 +250,9 @@ __global__ __launch_bounds__(W * 64, 3) void page_attn_kernel(
         l += p[r];
       }
       if (FP8) {
-        const f32x4 by = *reinterpret_cast<const f32x4*>(
-            st + 4 * A::BYTES + 128 + t * 64 + g * 16);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          p[r] = j0 + t * 16 + g * 4 + r < len ? p[r] * by[r] : 0.f;
+          p[r] = j0 + t * 16 + g * 4 + r < len ? p[r] * v_by[t][r] : 0.f;
       }
 #pragma unroll
       for (int r = 0; r < 4; r += 2) {
