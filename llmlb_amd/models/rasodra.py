@@ -235,9 +235,12 @@ class RasodraForCausalLM(PackedCausalLM):
             h = between(ly.norm1)
             if i and on_layer is not None:
                 on_layer(i - 1, x)
-            y, w_post = for_norm(ly.mix, self.cfg.width)(h, b, cache, i), ly.norm1b
+            y = for_norm(ly.mix, self.cfg.width)(h, b, cache, i)
+            w_post = ly.norm1b
             if ly.ff is not None:
-                y, w_post = for_norm(ly.ff, self.cfg.width)(between(ly.norm2)), ly.norm2b
+                h = between(ly.norm2)
+                y = for_norm(ly.ff, self.cfg.width)(h)
+                w_post = ly.norm2b
         if y is not None:
             between(None)
             if on_layer is not None:

@@ -144,7 +144,7 @@ def _mixer(cfg: TaletarConfig, i: int, dtype, device):
 
 
 class TaletarLayer(Projected):
-    """mixer(h1) + feed_forward(h2), one product of what both leave in a row."""
+    """mixer(h1) + feed_forward(h2), one product of a row that both leave."""
 
     projection = "w_out"
 

@@ -13,9 +13,9 @@
 // place was no faster), and the wave's own other half: the next keys are on their
 // way while values are worked on, the next values while keys are (us, both waited
 // for at once -> this: 64 sequences of 675 to 900 tokens 40.1 -> 38.6, 32 of 1500 to
-// 2000 e4m3 25.5 -> 24.2, 8 of 1000 12.7 -> 11.2, 10 of 100 6.6 -> 6.4).  Weights and sums stay
-// floats: a weight enters its product as the sum of three bf16 numbers, which are
-// all of its 24 bits.
+// 2000 e4m3 25.5 -> 24.2, 8 of 1000 12.7 -> 11.2, 10 of 100 6.6 -> 6.4).  Weights and
+// sums stay floats: a weight enters its product as the sum of three bf16 numbers,
+// which are all of its 24 bits.
 //
 // Sequences use as many parts as their length fills (16 pages each), which
 // the host does not know: the rest of the grid ends at once, and where one

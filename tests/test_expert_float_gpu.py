@@ -47,13 +47,13 @@ def test_experts(E, top, T, W, F, used):
         p = (flat == e).nonzero().flatten()
         x, a, b = h[p // top].double(), up[e].double(), down[e].double()
         s = x @ a.T
-        # of every product 2^-21 is left out at most, and a sum of n is rounded
+        # of every product 2^-24 is left out at most, and a sum of n is rounded
         # less than n times; the square doubles what the first has lost
-        off = (x.abs() @ a.abs().T) * (2.0 ** -21 + W * 2.0 ** -24)
+        off = (x.abs() @ a.abs().T) * (W + 1) * 2.0 ** -24
         u = act(s)
         lost = 2 * off * (s.clamp(min=0.0) + off) + 2.0 ** -23 * u
         bound = lost @ b.abs().T + (u + lost) @ b.abs().T * (
-            2.0 ** -21 + F * 2.0 ** -24)
+            (F + 1) * 2.0 ** -24)
         assert ((z[p].double() - u @ b.T).abs() <= bound).all()
         # and on the whole no more than sums in 32 bits are
         assert (z[p].double() - u @ b.T).norm() <= 2e-6 * (u @ b.T).norm()
