@@ -481,17 +481,23 @@ __global__ __launch_bounds__(64) void memory_gates_kernel(
   if (lane == 0) ex[extra_row(D) - 4] = m;
 }
 
-// g = sigmoid(dec + bias)^rate per channel
-template <typename T, bool VEC>
+// g = sigmoid(dec + bias)^rate per channel.  Bound by memory; a row's workgroups
+// go side by side, see ssm_conv_run, where all of them have as much to do: 16384
+// tokens of 4096 channels apart 100 us, side by side 93, 12288 270, 257; but 3072
+// channels 75, 87, and 2048 tokens of 4096 11.3, 12.2.
+template <typename T, bool VEC, bool TOGETHER>
 __global__ __launch_bounds__(256) void gla_decay_kernel(
     float* __restrict__ g, const T* __restrict__ dec,
     const float* __restrict__ bias, int n_tok, int C, float rate) {
   constexpr int N = VEC ? 8 : 1;
-  const int c = (blockIdx.y * 256 + threadIdx.x) * N;
+  const int across = TOGETHER ? C / (256 * N) : 1;
+  const int part = TOGETHER ? blockIdx.x % across : blockIdx.y;
+  const int c = (part * 256 + threadIdx.x) * N;
   if (c >= C) return;
   float b[N];
   load_run<N, VEC>(bias + c, b);
-  for (int t = blockIdx.x; t < n_tok; t += gridDim.x) {
+  const int step = gridDim.x / across;
+  for (int t = blockIdx.x / across; t < n_tok; t += step) {
     float f[N];
     load_run<N, VEC>(dec + (size_t)t * C + c, f);
 #pragma unroll
@@ -903,14 +909,18 @@ int hy_gla_decay(void* g, const void* dec, const void* bias, int n_tok, int C,
   if (n_tok <= 0 || C <= 0) return 0;
   const bool vec = C % 8 == 0;
   const int cols = vec ? 2048 : 256;
-  const dim3 grid(n_tok < 2048 ? n_tok : 2048, (C + cols - 1) / cols);
-#define GO(VEC)                                                          \
+  const bool large =
+      dtype == 0 && C % 2048 == 0 && 6ll * n_tok * C > 256ll << 20;
+  const dim3 grid =
+      run_parts(n_tok < 2048 ? n_tok : 2048, (C + cols - 1) / cols, large);
+#define GO(VEC, TOGETHER)                                                \
   HY_DTYPE(dtype, hipLaunchKernelGGL(                                    \
-      (gla_decay_kernel<T, VEC>), grid, dim3(256), 0,                    \
+      (gla_decay_kernel<T, VEC, TOGETHER>), grid, dim3(256), 0,          \
       (hipStream_t)stream, (float*)g, (const T*)dec, (const float*)bias, \
       n_tok, C, rate))
-  if (vec) GO(true);
-  else GO(false);
+  if (large) GO(true, true);
+  else if (vec) GO(true, false);
+  else GO(false, false);
 #undef GO
   HY_CHECK();
   return 0;

@@ -162,3 +162,21 @@ def test_state_space_convolution(T):
         want = prep(proj[part], ring[s:s + 1], _place(each, 1))
         assert torch.equal(got[part], want)
         assert not want.isnan().any()
+
+
+# more than 256 MB read and written, in whole parts of rows and not, and less
+@pytest.mark.parametrize("T, C", [(11000, 4096), (11000, 4104), (9000, 6144),
+                                  (300, 4096), (70, 2050)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gated_linear_decays(T, C, dtype):
+    g = torch.Generator(device=DEV).manual_seed(C)
+    dec = torch.randn(T, C, generator=g, device=DEV).to(dtype) * 3
+    bias = torch.randn(C, generator=g, device=DEV)
+    out = torch.full((T, C), float("nan"), device=DEV)
+    assert hy.native().hy_gla_decay(
+        _ptr(out), _ptr(dec), _ptr(bias), hy._i(T), hy._i(C),
+        hy._f(1 / 16), hy._dt(dtype), _stream()) == 0
+    want = torch.sigmoid(dec.double() + bias.double()) ** (1 / 16)
+    # the sum, a logarithm and an exponential in 24 bits; the hardware's are off
+    # by 2^-22 of themselves, and a sixteenth of the logarithm is at most one
+    assert (out.double() - want).abs().max() <= 2.0 ** -20
