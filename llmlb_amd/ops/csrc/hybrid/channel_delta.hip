@@ -583,11 +583,14 @@ int hy_delta_prep(void* ws, const void* proj, int ld, int b_off,
     const int v_blocks = (H * V + n - 1) / n;
     const int g_blocks = (H * D + n - 1) / n;
     const int parts = qk_blocks + v_blocks + g_blocks;
-    // 32 bits read twice as much, 16 us, apart -> together, 5 and 12 parts: 150 MB
-    // 95.8 -> 91.5, 134 MB 86 -> 79; but three, 235 MB 138 -> 182
+    // 32 bits read twice as much, us, apart -> together, 5 and 12 parts: 150 MB
+    // 95.8 -> 91.5, 134 MB 86 -> 79; but three, 235 MB 138 -> 182.  Where the last
+    // q/k workgroup has heads missing, together loses: 20 heads of 64, 16384
+    // tokens 132 -> 157.
     const long long writes = 4ll * n_tok * WsLayout(KH, H, D, V).size;
     const bool large =
-        whole && writes > (dtype == 1 && parts > 4 ? 128ll : 256ll) << 20;
+        whole && KH % (256 / lanes) == 0 &&
+        writes > (dtype == 1 && parts > 4 ? 128ll : 256ll) << 20;
     const dim3 grid =
         run_parts((n_tok + PREP_TOK - 1) / PREP_TOK, parts, large);
 #define RUN(RPL, LANES, VEC)                                                 \
