@@ -1033,9 +1033,9 @@ class Engine:
         vocab = self.cfg.model.vocab
         cap = min(self.cfg.model.max_pos,
                   self.max_blocks_per_seq * BLOCK_SIZE)
-        # (work and wanted places may be iterables, which are read once)
-        work = [(seq, toks, list(want)) for seq, toks, want in work]
-        work = [(seq, toks, want) for (seq, _, want), toks in
+        work = list(work)       # (it and wanted places may be read only once)
+        work = [(seq, toks, want if type(want) is list else list(want))
+                for (seq, _, want), toks in
                 zip(work, _token_arrays([toks for _, toks, _ in work]))]
         if not _in_order(work, vocab, cap):     # say what is not
             for seq, toks, want in work:
