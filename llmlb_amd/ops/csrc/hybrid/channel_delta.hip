@@ -154,7 +154,8 @@ __global__ __launch_bounds__(256) void delta_prep_run_kernel(
       q.start(t, pos_[t], ts, row_[t]);
       k.start(t, pos_[t], ts, row_[t]);
     };
-    walk_tokens<VEC && RPL <= 8 ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
+    constexpr int AT_ONCE = VEC && RPL <= 8 ? 4 : 1;
+    walk_tokens<AT_ONCE>(tstart_, t0, t1, start, [&](int t, auto n) {
       constexpr int G = decltype(n)::value;
       float xq[G][RPL], xk[G][RPL];
 #pragma unroll

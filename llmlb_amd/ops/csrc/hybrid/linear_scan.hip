@@ -554,7 +554,8 @@ __global__ __launch_bounds__(256) void ssm_conv_run_kernel(
   const int valid = C - c < 8 ? C - c : 8;
   ConvRun<T, 8, VEC> run(proj, ld, ring, wconv, bias, C, taps, c, valid);
   auto start = [&](int t, int ts) { run.start(t, pos_[t], ts, row_[t]); };
-  walk_tokens<VEC && sizeof(T) == 2 ? 4 : 1>(tstart_, t0, t1, start, [&](int t, auto n) {
+  constexpr int AT_ONCE = VEC && sizeof(T) == 2 ? 4 : 1;
+  walk_tokens<AT_ONCE>(tstart_, t0, t1, start, [&](int t, auto n) {
     constexpr int G = decltype(n)::value;
     float x[G][8];
 #pragma unroll

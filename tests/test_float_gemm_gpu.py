@@ -11,10 +11,10 @@ TILES = 11
 
 
 def _close(out, x, w):
-    """Of every product 2^-21 is left out at most, and a sum of K is rounded
+    """Of every product 2^-24 is left out at most, and a sum of K is rounded
     less than K times."""
     x, w = x.double(), w.double()
-    bound = (x.abs() @ w.abs().T) * (2.0 ** -21 + x.shape[1] * 2.0 ** -24)
+    bound = (x.abs() @ w.abs().T) * (x.shape[1] + 1) * 2.0 ** -24
     assert ((out.double() - x @ w.T).abs() <= bound).all()
 
 
