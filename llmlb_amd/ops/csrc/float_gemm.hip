@@ -7,9 +7,11 @@
 // nine products of those, of which the three smallest are left out: 2^-24 of the
 // product at most, to either side.  Six times the work at sixteen times the rate
 // of the float instructions, and the sum is rounded once in 32 of the depth where
-// theirs is in every four.  Errors against 64 bits, the library's -> here: normal
-// numbers 32 deep 1.0e-7 -> 3.8e-8, 256 2.9e-7 -> 6.4e-8, 1024 5.8e-7 -> 1.6e-7,
-// 3328 1.0e-6 -> 3.1e-7; numbers from 1 to 1.01 256 deep 2.1e-7 -> 5.2e-8, on
+// theirs is in every four.  Errors against 64 bits, the library's -> here in tiles
+// of eight waves, of four, which sum twice the depth each: normal numbers 32 deep
+// 1.0e-7 -> 3.8e-8, 256 2.9e-7 -> 6.4e-8, 1.0e-7, 1024 5.8e-7 -> 1.6e-7, 2.3e-7, 3328
+// 1.0e-6 -> 3.1e-7, 4.4e-7 (a piece's six products summed by themselves and added once
+// would be 8.5e-8 and 1.3e-7 there, in 4 to 20% more time); numbers from 1 to 1.01 256 deep 2.1e-7 -> 5.2e-8, on
 // average 9e-10 to one side.  Only rows with a single number that is not zero,
 // which the library rounds once, are further off: 2.5e-8 -> 3.4e-8.  (Cutting bits
 // off takes as many instructions and a few percent less time, but parts of one
