@@ -977,7 +977,8 @@ def _takes_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def _takes_row_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return _takes_product(x, weight) and x.shape[0] <= 128
+    # (prompts ask before every norm: the number of rows first)
+    return x.dim() == 2 and x.shape[0] <= 128 and _takes_product(x, weight)
 
 
 def linear_act(x: torch.Tensor, weight: torch.Tensor, act: str,
