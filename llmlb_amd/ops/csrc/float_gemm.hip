@@ -10,12 +10,13 @@
 // theirs is in every four.  Errors against 64 bits, the library's -> here in tiles
 // of eight waves, of four, which sum twice the depth each: normal numbers 32 deep
 // 1.0e-7 -> 3.8e-8, 256 2.9e-7 -> 6.4e-8, 1.0e-7, 1024 5.8e-7 -> 1.6e-7, 2.3e-7, 3328
-// 1.0e-6 -> 3.1e-7, 4.4e-7 (a piece's six products summed by themselves and added once
-// would be 8.5e-8 and 1.3e-7 there, in 4 to 20% more time); numbers from 1 to 1.01 256 deep 2.1e-7 -> 5.2e-8, on
-// average 9e-10 to one side.  Only rows with a single number that is not zero,
-// which the library rounds once, are further off: 2.5e-8 -> 3.4e-8.  (Cutting bits
-// off takes as many instructions and a few percent less time, but parts of one
-// sign leave out up to 2^-21, always to the same side: 6.9e-8 of single numbers.)
+// 1.0e-6 -> 3.1e-7, 4.4e-7 (a piece's six products summed by themselves and added
+// once would be 8.5e-8 and 1.3e-7 there, in 4 to 20% more time); numbers from 1 to
+// 1.01 256 deep 2.1e-7 -> 5.2e-8, on average 9e-10 to one side.  Only rows with a
+// single number that is not zero, which the library rounds once, are further off:
+// 2.5e-8 -> 3.4e-8.  (Cutting bits off takes as many instructions and a few percent
+// less time, but parts of one sign leave out up to 2^-21, always to the same side:
+// 6.9e-8 of single numbers.)
 //
 // Bound by vector instructions, which take numbers apart and look for the largest
 // (6 a number of a tile's edge), beside matrix instructions (a tile of 64 x 64, of
