@@ -20,7 +20,8 @@ from ..backend.ragged import RaggedBatch
 from ..ops import hybrid as hy
 from ..ops.reference import build_cos_sin_table
 from ..parallel.tp import TPContext
-from .mixers import ChannelDelta, DenseFF, LatentAttention, for_norm
+from .mixers import (ChannelDelta, DenseFF, LatentAttention, few_rows,
+                     for_norm)
 from .packed import PackedCausalLM, read_folder
 
 
@@ -208,11 +209,14 @@ class DibelixForCausalLM(PackedCausalLM):
         ``on_layer(i, x)`` sees it after each layer."""
         eps = self.cfg.eps
         x, xb = hy.embed_rows(self.embed, b.ids)
+        few = few_rows(x.shape[0], xb.dtype)
         for i, ly in enumerate(self.layers_):
-            hy.post_norm_add(x, xb, for_norm(ly.mix)(xb, b, cache, i),
-                             ly.norm1, eps, self.norm_offset)
+            mix = for_norm(ly.mix) if few else ly.mix
+            hy.post_norm_add(x, xb, mix(xb, b, cache, i), ly.norm1, eps,
+                             self.norm_offset)
             if ly.ff is not None:
-                hy.post_norm_add(x, xb, for_norm(ly.ff)(xb), ly.norm2, eps,
+                ff = for_norm(ly.ff) if few else ly.ff
+                hy.post_norm_add(x, xb, ff(xb), ly.norm2, eps,
                                  self.norm_offset)
             if on_layer is not None:
                 on_layer(i, x)

@@ -406,7 +406,8 @@ class LlamaForCausalLM(nn.Module):
                 if o is not None:
                     # RowParallelLinear: the mixin GEMM is shard-local
                     o = layer.o_proj.tp.all_reduce(o)
-        elif (residual is not None and not ops.norms_rows(residual)
+        elif (T <= 128 and residual is not None
+                and not ops.norms_rows(residual)
                 and ops.joins_rows(T, layer.post_norm_w, residual)):
             fused = getattr(layer.o_proj, "forward_shares", None)
             shares = fused(attn_out.reshape(T, -1)) if fused else None

@@ -89,6 +89,13 @@ class Projected(nn.Module):
         return _linear(x, w) if y is None else y
 
 
+def few_rows(n_tok: int, dtype) -> bool:
+    """Whether products of n_tok rows may be taken in shares at all.  Asked
+    once a step: prompts and floats, for which the host is what a short step
+    waits for, call the modules themselves."""
+    return n_tok <= 128 and dtype == torch.bfloat16
+
+
 def for_norm(module, width: int = 0):
     """What to call for a norm of ``width`` columns that takes shares
     (0: of any width).  A module in another's place is called as any other."""

@@ -23,7 +23,7 @@ from ..ops import hybrid as hy
 from ..ops.reference import build_cos_sin_table
 from ..parallel.tp import TPContext
 from .mixers import (DenseFF, GroupedAttention, LatentAttention,
-                     MatrixMemory, for_norm)
+                     MatrixMemory, few_rows, for_norm)
 from .packed import PackedCausalLM, read_folder
 
 
@@ -225,6 +225,7 @@ class RasodraForCausalLM(PackedCausalLM):
         """Residual stream [T, width] in 32-bit after the last layer.
         ``on_layer(i, x)`` sees it after each layer."""
         x, _ = hy.embed_rows(self.embed, b.ids, copy=False)
+        few = few_rows(x.shape[0], self.dtype)
         y = w_post = None
 
         def between(w_pre):
@@ -235,11 +236,12 @@ class RasodraForCausalLM(PackedCausalLM):
             h = between(ly.norm1)
             if i and on_layer is not None:
                 on_layer(i - 1, x)
-            y = for_norm(ly.mix, self.cfg.width)(h, b, cache, i)
+            mix = for_norm(ly.mix, self.cfg.width) if few else ly.mix
+            y = mix(h, b, cache, i)
             w_post = ly.norm1b
             if ly.ff is not None:
                 h = between(ly.norm2)
-                y = for_norm(ly.ff, self.cfg.width)(h)
+                y = (for_norm(ly.ff, self.cfg.width) if few else ly.ff)(h)
                 w_post = ly.norm2b
         if y is not None:
             between(None)

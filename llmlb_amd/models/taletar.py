@@ -23,7 +23,7 @@ from ..ops import hybrid as hy
 from ..parallel.tp import TPContext
 from .mixers import (ClampedSwiGLU, DifferentialAttention,
                      GatedLinearAttention, Projected, StateSpaceDuality,
-                     _param, for_norm)
+                     _param, few_rows, for_norm)
 from .packed import PackedCausalLM, read_folder
 
 
@@ -233,12 +233,14 @@ class TaletarForCausalLM(PackedCausalLM):
         ``on_layer(i, x)`` sees it after each layer."""
         eps = self.cfg.eps
         x, _ = hy.embed_rows(self.embed, b.ids, copy=False)
+        few = few_rows(x.shape[0], self.dtype)
         y = None
         for i, ly in enumerate(self.layers_):
             h1, h2 = hy.add_norms(x, y, ly.norm1, ly.norm2, eps, self.dtype)
             if i and on_layer is not None:
                 on_layer(i - 1, x)
-            y = for_norm(ly, self.cfg.width)(h1, h2, b, cache, i)
+            y = (for_norm(ly, self.cfg.width) if few else ly)(
+                h1, h2, b, cache, i)
         if y is not None:
             hy.add_norms(x, y, None, None, eps, self.dtype)
             if on_layer is not None:

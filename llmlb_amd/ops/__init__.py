@@ -12,6 +12,7 @@ always use the fp32 reference implementations (tests, CI without GPU).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -127,7 +128,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
 
 def _on_vectors(*tensors: torch.Tensor | None) -> bool:
     """Whether all that there are begin where a load of 16 bytes may."""
-    return not any(t is not None and t.data_ptr() % 16 for t in tensors)
+    for t in tensors:
+        if t is not None and t.data_ptr() % 16:
+            return False
+    return True
 
 
 def joins_rows(T: int, weight: torch.Tensor, residual: torch.Tensor) -> bool:
@@ -1030,6 +1034,14 @@ def linear_two(x: torch.Tensor, weight: torch.Tensor, x2: torch.Tensor,
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _share_count(N: int, M: int, K: int, joined: bool) -> int:
+    """The kernels' rule, of sizes alone.  (Asked for every sublayer it takes 0.7 us
+    of the host's time each, kept 0.1.)"""
+    rule = _lib.ll_row_gemm_joined if joined else _lib.ll_row_gemm_shares
+    return rule(ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
+
+
 def linear_shares(x: torch.Tensor, weight: torch.Tensor,
                   joined: bool = False) -> torch.Tensor | None:
     """x @ W^T as float shares [n, N, M] of the depth whose sum, rounded once,
@@ -1037,19 +1049,20 @@ def linear_shares(x: torch.Tensor, weight: torch.Tensor,
     where it would not take the depth in shares.  ``joined``: the caller's next
     launch adds them up for next to nothing, so that more products gain by it;
     their sums are linear_decode's in another order."""
-    if (_USE_CUSTOM_DECODE_GEMM != "auto" or not _takes_row_gemm(x, weight)
+    if (_USE_CUSTOM_DECODE_GEMM != "auto" or _lib is None or x.dim() != 2
+            or weight.dim() != 2 or x.dtype != torch.bfloat16):
+        return None
+    (N, K), M = x.shape, weight.shape[0]
+    # (most that ask have too many rows or too little depth)
+    shares = _share_count(N, M, K, joined) if N <= 128 else 1
+    if (shares < 2 or not _takes_row_gemm(x, weight)
             or weight.dtype != x.dtype or x.stride(1) != 1
             or not weight.is_contiguous()):
         return None
-    (N, K), M = x.shape, weight.shape[0]
-    sizes = (ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K))
-    plan = _lib.ll_row_gemm_joined if joined else _lib.ll_row_gemm_shares
-    shares = plan(*sizes)
-    if shares < 2:
-        return None
     ws = torch.empty(shares, N, M, device=x.device, dtype=torch.float32)
     parts = _lib.ll_row_gemm_parts(
-        _ptr(x), _ptr(weight), _ptr(ws), ctypes.c_int(shares), *sizes,
+        _ptr(x), _ptr(weight), _ptr(ws), ctypes.c_int(shares),
+        ctypes.c_int(N), ctypes.c_int(M), ctypes.c_int(K),
         ctypes.c_int(x.stride(0)), _stream())
     if parts == -2:
         return None

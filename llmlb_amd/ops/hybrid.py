@@ -110,8 +110,10 @@ def _joinable(x, y, weights) -> bool:
     are rows.  Their loads are of 16 bytes."""
     assert (y.is_contiguous() and y.dtype == torch.float32
             and y.shape[1:] == x.shape and x.is_contiguous())
-    return _on_vectors(x, y, *weights) and all(
-        w is None or w.numel() == x.shape[1] for w in weights)
+    for w in weights:
+        if w is not None and w.numel() != x.shape[1]:
+            return False
+    return _on_vectors(x, y, *weights)
 
 
 def _joined(shares):

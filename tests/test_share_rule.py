@@ -3,6 +3,7 @@ the host's, and needs no GPU."""
 import ctypes
 
 import pytest
+import torch
 
 import llmlb_amd.ops as ops
 
@@ -51,3 +52,37 @@ def test_one_round_of_workgroups(K):
     (64, 2046, 4096, 1), (129, 2048, 4096, 1), (0, 2048, 4096, 1)])
 def test_lines(N, M, K, n):
     assert shares(N, M, K) == n
+
+
+@pytest.mark.parametrize("K", [64, 2816, 4104, 24576])
+@pytest.mark.parametrize("joined", [True, False])
+def test_kept_counts_are_the_rule(K, joined):
+    for N in (1, 16, 33, 64, 128):
+        for M in (764, 1024, 2048, 4096):
+            want = shares(N, M, K, "joined" if joined else "shares")
+            for _ in range(2):
+                assert ops._share_count(N, M, K, joined) == want
+
+
+@pytest.mark.parametrize("rows, dtype, asked", [
+    (128, torch.bfloat16, True), (129, torch.bfloat16, False),
+    (5, torch.float32, False)])
+def test_prompts_and_floats_are_not_asked(monkeypatch, rows, dtype, asked):
+    """Their products never come in shares, and asking each sublayer costs a
+    step that waits for the host 3% of its time."""
+    from llmlb_amd.models import mixers
+
+    class Part(mixers.Projected):
+        def __init__(self):
+            super().__init__()
+            self.w_o = mixers._param(torch.ones(8, 8, dtype=dtype))
+
+        def before(self, x):
+            return x
+
+    seen = []
+    monkeypatch.setattr(mixers, "linear_shares",
+                        lambda *a, **k: seen.append(1))
+    part, x = Part(), torch.ones(rows, 8, dtype=dtype)
+    call = mixers.for_norm(part) if mixers.few_rows(rows, dtype) else part
+    assert torch.equal(call(x), x * 8) and len(seen) == asked
